@@ -34,12 +34,12 @@ struct DecodeItems {
     const int32_t *item_seq, *item_range, *seq_active, *seq_chunk;
     int batch;
     int max_ranges;
+    const int32_t* order;      // uniform grid: the sequence that blockIdx.z stands for (null: itself)
 };
 
 // FUSED: `q` is the raw fused qkv row of the step's single new token per sequence.  The kernel applies the
-// q/k epilogue itself (per-head RMSNorm + RoPE, qknorm_rope_head), uses the new token's K/V straight from
-// registers for its own dot product and writes them to their cache slot (token ctx-1 of the sequence), so
-// the separate norm/rope/store launch disappears from a decode step.
+// q/k epilogue itself (per-head RMSNorm + RoPE, qknorm_rope_head) and writes the new token's K/V to their cache slot
+// (token ctx-1 of the sequence) before it walks the keys, so the separate norm/rope/store launch disappears from a decode step.
 struct FusedQkv {
     const bf16* q_norm_w;
     const bf16* k_norm_w;
@@ -52,7 +52,7 @@ __device__ __forceinline__ void merge_row_wave(const float* __restrict__ ws_acc,
                                                int num_splits, int64_t bh, int active, int lane);
 
 template <int G, bool FUSED>
-__global__ __launch_bounds__(256) void attn_decode_kernel(
+__global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     const bf16* __restrict__ q, int64_t q_stride, bf16* __restrict__ kc, bf16* __restrict__ vc,
     const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ tables, int64_t table_stride, int hkv,
     float scale_log2, bf16* __restrict__ out, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int min_range, DecodeItems items, FusedQkv fz,
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         // transposed order - the 8 heads of a sequence side by side on one XCD, whole 2-KB token rows per XCD - measured
         // 6.49 ms against 6.29 ms per step of 256 sequences: not taken)
         split = blockIdx.x;
-        b = blockIdx.z;
+        b = items.order ? items.order[blockIdx.z] : blockIdx.z;
         num_splits = gridDim.x;
         ctx = ctx_lens[b];
         chunk = decode_range_keys(ctx, num_splits, min_range);
@@ -93,20 +93,28 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
     const int end = min(ctx, start + chunk);
 
     bf16x8 qv[G];
+    if (start < end) {
 #pragma unroll
-    for (int g = 0; g < G; ++g)
-        qv[g] = *reinterpret_cast<const bf16x8*>(q + (int64_t)b * q_stride + (int64_t)(kvh * G + g) * 128 + c * 8);
-    bf16x8 k_new = {0, 0, 0, 0, 0, 0, 0, 0}, v_new = k_new;
-    if constexpr (FUSED) {
-        if (ctx > 0) {                                       // block-uniform
+        for (int g = 0; g < G; ++g)
+            qv[g] = *reinterpret_cast<const bf16x8*>(q + (int64_t)b * q_stride + (int64_t)(kvh * G + g) * 128 + c * 8);
+        if constexpr (FUSED) {
             const float* cs_row = fz.cos_sin + fz.positions[b] * 128;
             const bf16x8 qw = *reinterpret_cast<const bf16x8*>(fz.q_norm_w + c * 8);
-            const bf16x8 kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
 #pragma unroll
             for (int g = 0; g < G; ++g) qv[g] = qknorm_rope_head(qv[g], qw, cs_row, c, fz.eps);
-            const bf16* row = q + (int64_t)b * q_stride;
-            k_new = qknorm_rope_head(*reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8), kw, cs_row, c, fz.eps);
-            v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
+            if (end == ctx) {                                // (uniform)
+                // the new token's keys and values go to the cache first; the loop's loads of them are the same lanes' (in order behind the
+                // stores)
+                const bf16x8 kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
+                const bf16* row = q + (int64_t)b * q_stride;
+                const bf16x8 k_new = qknorm_rope_head(*reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8), kw, cs_row, c, fz.eps);
+                const bf16x8 v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
+                if (((ctx - 1) & 15) == rowid) {
+                    const int64_t off = (((int64_t)tables[(int64_t)b * table_stride + ((ctx - 1) >> 8)] * NVH_KV_PAGE + ((ctx - 1) & 255)) * hkv + kvh) * 128 + c * 8;
+                    *reinterpret_cast<bf16x8*>(kc + off) = k_new;
+                    *reinterpret_cast<bf16x8*>(vc + off) = v_new;
+                }
+            }
         }
     }
 
@@ -119,65 +127,86 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(
         for (int j = 0; j < 8; ++j) acc[g][j] = 0.f;
     }
 
+    // The keys and values of a trip (64 tokens) are requested a trip ahead into a second register set, so the work on one trip hides
+    // the loads of the next; the page after the one at hand is looked up a trip ahead.  With one workgroup a CU a trip takes 1.2 us (one set,
+    // every trip's loads waited for before its work: 1.6 us), about the 64 KB in flight over the memory's latency.  Measured beside it, a
+    // launch of 24 sequences of 100..2047 keys at 38.0 us: three and four sets 36.1 and 35.7 us, but 100 short sequences 8 and 25 % slower for
+    // the registers; two teams of four waves that split a sequence's trips 32.6 us, but a sequence's sums would then depend on the launch.
     const int32_t* table = tables + (int64_t)b * table_stride;
-    for (int base = start; base < end; base += 64) {
-        const int64_t slot0 = (int64_t)table[base >> 8] * NVH_KV_PAGE + (base & 255);
-        bf16x8 kf[4], vf[4];
-        bool valid[4];
+    u32x4 ka[4], va[4], kb[4], vb[4];                        // (whole words: as 16-bit elements every one would take a register across the loop)
+    const int last_page = (end - 1) >> 8;
+    int page = start < end ? table[start >> 8] : 0;
+    auto fetch = [&](int base, u32x4 (&kf)[4], u32x4 (&vf)[4]) {
+        // (scalar base of the trip + a 32-bit lane offset: one register per address)
+        const int64_t slot0 = (((int64_t)page * NVH_KV_PAGE + (base & 255)) * hkv + kvh) * 128;
+        const bf16 *kp = kc + slot0, *vp = vc + slot0;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int toff = u * 16 + rowid;
-            valid[u] = base + toff < end;
-            const int64_t off = ((slot0 + (valid[u] ? toff : 0)) * hkv + kvh) * 128 + c * 8;
-            kf[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kc + off));   // streamed once
-            vf[u] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vc + off));
-            if constexpr (FUSED) {
-                if (base + toff == ctx - 1) {                // the new token: not in the cache yet
-                    kf[u] = k_new;
-                    vf[u] = v_new;
-                    *reinterpret_cast<bf16x8*>(kc + off) = k_new;
-                    *reinterpret_cast<bf16x8*>(vc + off) = v_new;
-                }
-            }
+            const unsigned off = (unsigned)((base + toff < end ? toff : 0) * hkv * 128 + c * 8);
+            kf[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kp + off));   // streamed once
+            vf[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vp + off));
         }
+        page = table[min((base + 64) >> 8, last_page)];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto consume = [&](int base, const u32x4 (&kw)[4], const u32x4 (&vw)[4]) {
         float s[G][4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
+            const int tok = base + u * 16 + rowid;
+            const bf16x8 kf = __builtin_bit_cast(bf16x8, kw[u]);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 float d = 0.f;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     bf16x2 a = {qv[g][2 * j], qv[g][2 * j + 1]};
-                    bf16x2 k2 = {kf[u][2 * j], kf[u][2 * j + 1]};
+                    bf16x2 k2 = {kf[2 * j], kf[2 * j + 1]};
                     d = __builtin_amdgcn_fdot2_f32_bf16(a, k2, d, false);
                 }
                 d = row16_sum(d) * scale_log2;
-                s[g][u] = valid[u] ? d : -INFINITY;
+                s[g][u] = tok < end ? d : -INFINITY;
             }
         }
+        float alpha[G];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
+        for (int g = 0; g < G; ++g) {                        // s becomes the weights
             const float mn = fmaxf(fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3])), m[g]);
             const float mu = (mn == -INFINITY) ? 0.f : mn;
-            const float alpha = __builtin_amdgcn_exp2f(m[g] - mu);
-            float p[4];
+            alpha[g] = __builtin_amdgcn_exp2f(m[g] - mu);
             float ps = 0.f;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                p[u] = __builtin_amdgcn_exp2f(s[g][u] - mu);
-                ps += p[u];
+                s[g][u] = __builtin_amdgcn_exp2f(s[g][u] - mu);
+                ps += s[g][u];
             }
-            l[g] = l[g] * alpha + ps;
+            l[g] = l[g] * alpha[g] + ps;
             m[g] = mn;
+        }
+        // (column by column, so that only four widened values are alive at a time)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                float a = acc[g][j] * alpha;
+        for (int j = 0; j < 8; ++j) {
+            float v[4];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) a += p[u] * bf2f(vf[u][j]);
+            for (int u = 0; u < 4; ++u) v[u] = __builtin_bit_cast(float, j & 1 ? vw[u][j >> 1] & 0xffff0000u : vw[u][j >> 1] << 16);
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                float a = acc[g][j] * alpha[g];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) a += s[g][u] * v[u];
                 acc[g][j] = a;
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (start < end) fetch(start, ka, va);
+    for (int base = start; base < end; base += 128) {
+        if (base + 64 < end) fetch(base + 64, kb, vb);
+        consume(base, ka, va);
+        if (base + 64 >= end) break;
+        if (base + 128 < end) fetch(base + 128, ka, va);
+        consume(base + 64, kb, vb);
     }
 
     // merge the 4 rows of the wave (lanes l, l^16, l^32 hold the same output columns)
@@ -641,8 +670,23 @@ extern "C" int32_t nvh_attn_decode_items(const void* q, int64_t q_token_stride, 
     NVH_REQUIRE(item_seq, NVH_EINVAL, "nvh_attn_decode_items: null work list");
     DecodeArgs a{q, q_token_stride, const_cast<void*>(k_cache), const_cast<void*>(v_cache), context_lens, block_tables,
                  table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace,
-                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges}, num_items};
+                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
     return launch_decode<false>("nvh_attn_decode_items", a, FusedQkv{});
+}
+
+int32_t nvh_attn_decode_fused_qkv_ordered(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
+                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                          int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys, void* workspace,
+                                          const int32_t* order, hipStream_t stream) {
+    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
+    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
+                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
+    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
+                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, stream, DecodeItems{}, 0};
+    a.items.order = order;
+    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
+                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }
 
 extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stride, const void* q_norm_weight,
@@ -652,13 +696,9 @@ extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stri
                                              int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
                                              float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys,
                                              void* workspace, nvh_stream_t stream) {
-    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
-    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
-                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
-    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
-                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, (hipStream_t)stream, DecodeItems{}, 0};
-    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
-                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
+    return nvh_attn_decode_fused_qkv_ordered(qkv, token_stride, q_norm_weight, k_norm_weight, eps, positions, cos_sin, k_cache, v_cache, context_lens,
+                                             block_tables, table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, num_splits,
+                                             min_range_keys, workspace, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int32_t nvh_attn_decode_fused_qkv_items(const void* qkv, int64_t token_stride, const void* q_norm_weight,
@@ -674,7 +714,7 @@ extern "C" int32_t nvh_attn_decode_fused_qkv_items(const void* qkv, int64_t toke
                 "nvh_attn_decode_fused_qkv_items: 16-byte alignment required");
     DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
                  num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace, (hipStream_t)stream,
-                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges}, num_items};
+                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
     return launch_decode<true>("nvh_attn_decode_fused_qkv_items", a,
                                FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }

@@ -48,6 +48,16 @@ int32_t nvh_noalloc_scratch(float** out);
 // Device address, on the current GPU, of the arrival counters the decode attention uses to merge key ranges in its own
 // launch (resolved on first use, or by nvh_device_check before a graph capture).
 int32_t nvh_decode_arrivals(unsigned** out);
+// nvh_attn_decode_fused_qkv whose sequences are dispatched in the given order (attention_decode.hip; null: as they lie), and nvh_embedding with
+// one workgroup more that leaves that order, the longest context first (elementwise.hip).
+#define NVH_ORDER_MAX 1024
+int32_t nvh_attn_decode_fused_qkv_ordered(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
+                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                          int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys, void* workspace,
+                                          const int32_t* order, hipStream_t stream);
+int32_t nvh_embedding_order(const int64_t* ids, const void* table, void* out, int64_t num_tokens, int64_t dim, int64_t vocab_start, int64_t vocab_rows,
+                            const int32_t* context_lens, int32_t* order, int64_t batch, hipStream_t st);
 
 // Routing and measurement switches.  Every kernel choice in this library is a pure function of the call's shapes; the
 // switches below exist for A/B measurements and for tests that compare two routes.  They are read from the environment
