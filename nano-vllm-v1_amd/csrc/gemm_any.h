@@ -22,7 +22,7 @@ __device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + expf(-
 // y[M, N] = x[M, K] w[N, K]^T (+ bias[N]) (times sigmoid(gate[m, n]) when a gate is given; squared relu with `relu2`) for ANY M, N, K (ragged
 // edges are zero-filled on the way into LDS and masked on the way out).  The order in which an output element sums over k depends on
 // (N, K) only, never on M or on the row's place in the batch.  bf16: 64 x 64 tile per workgroup, four waves of 2 x 2 MFMA 16x16x32
-// tiles, fp32 accumulation.  fp32: the same tile with 4 x 4 outputs per lane on the vector ALU (true fp32 products and sums).
+// tiles, fp32 accumulation.  fp32: see gemm_any_f32_tile_body.
 constexpr int GT = 64, GK = 64, GLD = GK + 8;
 
 // What happens to a sum on its way out.
@@ -195,48 +195,114 @@ __device__ __forceinline__ void gemm_any_bf16_few_rows(const bf16* __restrict__ 
     }
 }
 
-__device__ __forceinline__ void gemm_any_f32_tile(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
-                                                  const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap rm, int n0, int N, int K,
-                                                  const float* __restrict__ gate = nullptr, int64_t ldg = 0, int relu2 = 0) {
-    constexpr int BK = 16;
-    __shared__ float xs[BK][GT + 4];
-    __shared__ float ws[BK][GT + 4];
-    const int tid = threadIdx.x;
-    const int tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
-    float acc[4][4] = {};
-    const int lr = tid >> 2, lc = (tid & 3) * 4;             // 64 rows x 16 columns per stage: 4 consecutive k per thread
-    const int64_t xrow = lr < rm.rows ? rm.src(lr) : 0;
-    for (int k0 = 0; k0 < K; k0 += BK) {
+// fp32: rows r0 .. r0 + 16 MR - 1 of the rows `rm` covers and columns n0 .. n0 + 16 NC - 1, on the matrix cores (16x16x4, products and sums in
+// fp32).  The four waves of the workgroup split k: wave w takes the chunks of 32 numbered w, w + 4, ..., straight from memory (whole 128-byte
+// lines a row, DEPTH chunks ahead, no barrier), and the four partial tiles meet in LDS as (p0 + p1) + (p2 + p3) - an order that depends on K alone.
+// Bound by the matrix cores (124 TFLOP/s measured on independent products of this form) and the L1 in front of them once the grid covers the
+// chip, below that by the chain of a wave's chunks.  Rows x columns x k, us a launch, before (64 x 64 tiles on the vector ALU, one LDS stage) and
+// now: 1 x 1024 x 1024 97 -> 6.3, 64 x 4096 x 1024 115 -> 12.7, 301 x 1024 x 1024 108 -> 21, 301 x 6144 x 1024 162 -> 72 (53 TFLOP/s),
+// 1000 x 32768 x 1024 1797 -> 1142 (59 TFLOP/s).
+constexpr int F32_CHUNK = 32;
+template <int MR, int NC, bool VEC>
+__device__ __forceinline__ void gemm_any_f32_tile_body(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
+                                                       const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap rm, int r0, int n0, int N,
+                                                       int K, const float* __restrict__ gate, int64_t ldg, int relu2, f32x4* lds) {
+    constexpr int DEPTH = MR * NC == 1 ? 4 : 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
+    const float *xp[MR], *wp[NC];
+    f32x4 acc[NC][MR];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = k0 + lc + e;
-            xs[lc + e][lr] = (lr < rm.rows && k < K) ? x[xrow * ldx + k] : 0.f;
-            ws[lc + e][lr] = (n0 + lr < N && k < K) ? w[(int64_t)(n0 + lr) * ldw + k] : 0.f;
+    for (int j = 0; j < MR; ++j) xp[j] = x + rm.src(min(r0 + 16 * j + fr, rm.rows - 1)) * ldx;      // (rows beyond the tile's repeat its last: not written)
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+        wp[i] = w + (int64_t)min(n0 + 16 * i + fr, N - 1) * ldw;
+#pragma unroll
+        for (int j = 0; j < MR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int chunks = (K + F32_CHUNK - 1) / F32_CHUNK;
+    f32x4 xf[DEPTH][2][MR], wf[DEPTH][2][NC];
+    auto load4 = [&](const float* row, int k) {
+        if constexpr (VEC) {
+            return *reinterpret_cast<const f32x4*>(row + min(k, K - 4));                             // (K a multiple of 4)
+        } else {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = row[min(k + e, K - 1)];
+            return v;
         }
-        __syncthreads();
+    };
+    auto load = [&](int c, f32x4 (&xs)[2][MR], f32x4 (&ws)[2][NC]) {
+        const int k = min(c, chunks - 1) * F32_CHUNK + 4 * fq;
 #pragma unroll
-        for (int k = 0; k < BK; ++k) {
-            float a[4], b[4];
+        for (int half = 0; half < 2; ++half) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                a[e] = xs[k][tm + e];
-                b[e] = ws[k][tn + e];
-            }
+            for (int j = 0; j < MR; ++j) xs[half][j] = load4(xp[j], k + 16 * half);
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+            for (int i = 0; i < NC; ++i) ws[half][i] = load4(wp[i], k + 16 * half);
         }
-        __syncthreads();
+    };
+    auto multiply = [&](const f32x4 (&xs)[2][MR], const f32x4 (&ws)[2][NC]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+#pragma unroll
+                    for (int j = 0; j < MR; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ws[h][i][e], xs[h][j][e], acc[i][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load(wave + 4 * d, xf[d], wf[d]);
+    // (no branch inside: the loads of a set go back to the registers it was read from, and only their age is waited for)
+    int c0 = wave;
+    for (; c0 + 4 * (DEPTH - 1) < K / F32_CHUNK; c0 += 4 * DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            multiply(xf[d], wf[d]);
+            load(c0 + 4 * (d + DEPTH), xf[d], wf[d]);
+            __builtin_amdgcn_sched_barrier(0);               // (left alone, all the loads sink to the end of the loop)
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int d = 0; d < DEPTH; ++d) {
+        const int c = c0 + 4 * d;
+        if (c >= chunks) break;
+        if ((c + 1) * F32_CHUNK > K) {                       // the last chunk: what lies beyond K counts as zero on both sides
+            const int k = c * F32_CHUNK + 4 * fq;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tn + j;
-            if (tm + i < rm.rows && n < N) {
-                const int64_t m = rm.dst(tm + i);
-                float v = acc[i][j] + (bias ? bias[n] : 0.f);
+            for (int e = 0; e < 8; ++e) {
+                const int h = e >> 2;
+                const bool in = k + 16 * h + (e & 3) < K;
+#pragma unroll
+                for (int j = 0; j < MR; ++j) xf[d][h][j][e & 3] = in ? xf[d][h][j][e & 3] : 0.f;
+#pragma unroll
+                for (int i = 0; i < NC; ++i) wf[d][h][i][e & 3] = in ? wf[d][h][i][e & 3] : 0.f;
+            }
+        }
+        multiply(xf[d], wf[d]);
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < MR; ++j) lds[(wave * NC * MR + i * MR + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    // fragment (i, j) is finished by one wave: row r0 + 16 j + fr, columns n0 + 16 i + 4 fq + e
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < MR; ++j) {
+            constexpr int F = NC * MR;
+            const int f = i * MR + j;
+            if (f % 4 != wave) continue;
+            const f32x4 sum = (lds[f * 64 + lane] + lds[(F + f) * 64 + lane]) + (lds[(2 * F + f) * 64 + lane] + lds[(3 * F + f) * 64 + lane]);
+            const int r = r0 + 16 * j + fr;
+            if (r >= rm.rows) continue;
+            const int64_t m = rm.dst(r);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = n0 + 16 * i + 4 * fq + e;
+                if (n >= N) continue;
+                float v = sum[e] + (bias ? bias[n] : 0.f);
                 if (gate) v *= sigmoid(gate[m * ldg + n]);
                 if (relu2) {
                     v = fmaxf(v, 0.f);
@@ -245,6 +311,21 @@ __device__ __forceinline__ void gemm_any_f32_tile(const float* __restrict__ x, i
                 y[m * ldy + n] = v;
             }
         }
+}
+
+template <int MR, int NC>
+__device__ __forceinline__ void gemm_any_f32_tile(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
+                                                  const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap rm, int r0, int n0, int N, int K,
+                                                  int vec_ok, const float* __restrict__ gate = nullptr, int64_t ldg = 0, int relu2 = 0) {
+    __shared__ f32x4 lds[4 * MR * NC * 64];
+    __syncthreads();                                         // (a tile before this one may still be read)
+    if (vec_ok) gemm_any_f32_tile_body<MR, NC, true>(x, ldx, w, ldw, bias, y, ldy, rm, r0, n0, N, K, gate, ldg, relu2, lds);
+    else gemm_any_f32_tile_body<MR, NC, false>(x, ldx, w, ldw, bias, y, ldy, rm, r0, n0, N, K, gate, ldg, relu2, lds);
+}
+
+// Whether rows of fp32 operands can be read 16 bytes at a time.
+__host__ __forceinline__ int f32_vec_ok(const void* x, int64_t ldx, const void* w, int64_t K) {
+    return K % 4 == 0 && ldx % 4 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
 }
 
 }  // namespace nvh_any

@@ -16,6 +16,7 @@
 //   nvh_latent_q_rotary  rotary of every head's rotated query part into its place behind the absorbed part
 // The attention itself is nvh_attn_paged_any (attention_any.hip).
 #include "common.h"
+#include <algorithm>
 #include "gemm_any.h"
 
 namespace {
@@ -139,10 +140,11 @@ __global__ __launch_bounds__(256) void gemm_heads_bf16_kernel(HeadsArgs a) {
 }
 
 __global__ __launch_bounds__(256) void gemm_heads_f32_kernel(HeadsArgs a) {
-    const int h = blockIdx.z, m0 = blockIdx.y * nvh_any::GT;
-    nvh_any::gemm_any_f32_tile((const float*)a.x + h * a.x_head, a.ldx, (const float*)a.w + (int64_t)h * a.N * a.K, a.K, nullptr, (float*)a.y + h * a.y_head, a.ldy,
-                               nvh_any::RowMap{nullptr, m0, min(nvh_any::GT, a.M - m0)}, blockIdx.x * nvh_any::GT, a.N, a.K,
-                               a.gate ? (const float*)a.gate + (int64_t)h * a.N : nullptr, a.ldg);
+    const int h = blockIdx.z;
+    for (int m0 = blockIdx.y * 32; m0 < a.M; m0 += gridDim.y * 32)      // (once, but for more rows than a grid has tiles)
+        nvh_any::gemm_any_f32_tile<2, 2>((const float*)a.x + h * a.x_head, a.ldx, (const float*)a.w + (int64_t)h * a.N * a.K, a.K, nullptr, (float*)a.y + h * a.y_head, a.ldy,
+                                         nvh_any::RowMap{nullptr, m0, min(32, a.M - m0)}, 0, blockIdx.x * 32, a.N, a.K, a.vec_ok,
+                                         a.gate ? (const float*)a.gate + (int64_t)h * a.N : nullptr, a.ldg);
 }
 
 }  // namespace
@@ -190,11 +192,12 @@ extern "C" int32_t nvh_gemm_heads_nt(const void* x, int64_t x_row_stride, int64_
                     x_row_stride >= (heads - 1) * x_head_stride + K && y_row_stride >= (heads - 1) * y_head_stride + N,
                 NVH_EINVAL, "nvh_gemm_heads_nt: bad sizes");
     if (M == 0) return NVH_OK;
-    const int vec_ok = !act_f32 && K % 8 == 0 && x_row_stride % 8 == 0 && x_head_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
+    const int vec_ok = act_f32 ? nvh_any::f32_vec_ok(x, x_row_stride, w, K) && x_head_stride % 4 == 0
+                               : K % 8 == 0 && x_row_stride % 8 == 0 && x_head_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
     const HeadsArgs a{x, x_row_stride, x_head_stride, w, y, y_row_stride, y_head_stride, (int)M, (int)N, (int)K, vec_ok, gate, gate_row_stride};
     const dim3 grid((unsigned)nvh_cdiv(N, nvh_any::GT), (unsigned)nvh_cdiv(M, nvh_any::GT), (unsigned)heads);
     hipStream_t st = (hipStream_t)stream;
-    if (act_f32) gemm_heads_f32_kernel<<<grid, 256, 0, st>>>(a);
+    if (act_f32) gemm_heads_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)std::min<int64_t>(nvh_cdiv(M, 32), 65535), (unsigned)heads), 256, 0, st>>>(a);
     else gemm_heads_bf16_kernel<<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_heads_nt");
     return NVH_OK;

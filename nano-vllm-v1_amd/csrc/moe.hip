@@ -394,12 +394,16 @@ __global__ __launch_bounds__(256) void gemm_grouped_bf16_kernel(GroupedArgs a) {
     nvh_any::gemm_any_bf16_tile<OUT_F32>((const bf16*)a.x, a.ldx, w, a.K, nullptr, a.y, a.ldy, rm, n0, a.N, a.K, a.vec_ok, nullptr, 0, a.relu2);
 }
 
+// (a tile of the list is 64 rows: blockIdx.z is its upper or lower half)
 __global__ __launch_bounds__(256) void gemm_grouped_f32_kernel(GroupedArgs a) {
-    const int rows = a.tile_rows[blockIdx.y];
-    if (rows <= 0) return;
+    const int rows = a.tile_rows[blockIdx.y], r0 = blockIdx.z * 32;
+    if (rows <= r0) return;                                  // (uniform)
     const float* w = (const float*)a.w + (int64_t)a.tile_expert[blockIdx.y] * a.N * a.K;
-    nvh_any::gemm_any_f32_tile((const float*)a.x, a.ldx, w, a.K, nullptr, (float*)a.y, a.ldy, nvh_any::RowMap{a.gather, a.tile_row0[blockIdx.y], rows},
-                               blockIdx.x * nvh_any::GT, a.N, a.K, nullptr, 0, a.relu2);
+    const nvh_any::RowMap rm{a.gather, a.tile_row0[blockIdx.y], rows};
+    if (rows - r0 <= 16)
+        nvh_any::gemm_any_f32_tile<1, 2>((const float*)a.x, a.ldx, w, a.K, nullptr, (float*)a.y, a.ldy, rm, r0, blockIdx.x * 32, a.N, a.K, a.vec_ok, nullptr, 0, a.relu2);
+    else
+        nvh_any::gemm_any_f32_tile<2, 2>((const float*)a.x, a.ldx, w, a.K, nullptr, (float*)a.y, a.ldy, rm, r0, blockIdx.x * 32, a.N, a.K, a.vec_ok, nullptr, 0, a.relu2);
 }
 
 template <typename A>
@@ -521,11 +525,11 @@ extern "C" int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, 
                 "nvh_gemm_grouped_any_nt: bad sizes");
     NVH_REQUIRE(!in_f32 || out_f32, NVH_ENOSYS, "nvh_gemm_grouped_any_nt: fp32 operands give an fp32 product");
     if (max_tiles == 0) return NVH_OK;
-    const int vec_ok = !in_f32 && K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
+    const int vec_ok = in_f32 ? nvh_any::f32_vec_ok(x, x_row_stride, w, K) : K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
     const GroupedArgs a{x, x_row_stride, gather, w, y, y_row_stride, tile_expert, tile_row0, tile_rows, (int)N, (int)K, vec_ok, relu2};
     const dim3 grid((unsigned)nvh_cdiv(N, nvh_any::GT), (unsigned)max_tiles);
     hipStream_t st = (hipStream_t)stream;
-    if (in_f32) gemm_grouped_f32_kernel<<<grid, 256, 0, st>>>(a);
+    if (in_f32) gemm_grouped_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)max_tiles, 2), 256, 0, st>>>(a);
     else if (out_f32) gemm_grouped_bf16_kernel<true><<<grid, 256, 0, st>>>(a);
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");

@@ -4,6 +4,7 @@
 //   tanh-GELU gate, [stream | first embedding] concatenation for a looped stack, row gather, logit softcap.
 // Every kernel is one workgroup per row (or a flat element grid) with 16-byte accesses where the row allows.
 #include "common.h"
+#include <algorithm>
 #include "gemm_any.h"
 
 namespace {
@@ -489,10 +490,11 @@ __global__ __launch_bounds__(256) void gemm_any_bf16_kernel(const bf16* __restri
     nvh_any::gemm_any_bf16_tile<OUT_F32>(x, ldx, w, ldw, bias, yv, ldy, nvh_any::RowMap{nullptr, m0, min(nvh_any::GT, M - m0)}, blockIdx.x * nvh_any::GT, N, K, vec_ok);
 }
 
+template <int MR, int NC>
 __global__ __launch_bounds__(256) void gemm_any_f32_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
-                                                           const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, int M, int N, int K) {
-    const int m0 = blockIdx.y * nvh_any::GT;
-    nvh_any::gemm_any_f32_tile(x, ldx, w, ldw, bias, y, ldy, nvh_any::RowMap{nullptr, m0, min(nvh_any::GT, M - m0)}, blockIdx.x * nvh_any::GT, N, K);
+                                                           const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, int M, int N, int K, int vec_ok) {
+    for (int64_t m0 = blockIdx.y * 16 * MR; m0 < M; m0 += (int64_t)gridDim.y * 16 * MR)      // (once, but for more rows than a grid has tiles)
+        nvh_any::gemm_any_f32_tile<MR, NC>(x, ldx, w, ldw, bias, y, ldy, nvh_any::RowMap{nullptr, (int)m0, (int)min((int64_t)16 * MR, M - m0)}, 0, blockIdx.x * 16 * NC, N, K, vec_ok);
 }
 
 }  // namespace
@@ -585,7 +587,10 @@ extern "C" int32_t nvh_gemm_any_nt(const void* x, int64_t x_row_stride, const vo
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)nvh_cdiv(N, nvh_any::GT), (unsigned)nvh_cdiv(M, nvh_any::GT));
     if (in_f32) {
-        gemm_any_f32_kernel<<<grid, 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K);
+        // (16 rows or fewer: small tiles, so that more workgroups share the weights' stream; the same sums either way)
+        const int vec_ok = nvh_any::f32_vec_ok(x, x_row_stride, w, K);
+        if (M <= 16) gemm_any_f32_kernel<1, 1><<<dim3((unsigned)nvh_cdiv(N, 16), 1), 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
+        else gemm_any_f32_kernel<2, 2><<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)std::min<int64_t>(nvh_cdiv(M, 32), 65535)), 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
     } else {
         const int vec_ok = K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
         if (out_f32) gemm_any_bf16_kernel<true><<<grid, 256, 0, st>>>((const bf16*)x, x_row_stride, (const bf16*)w, K, (const bf16*)bias, y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
