@@ -604,6 +604,13 @@ int32_t nvh_delta_prep(const void* r, int64_t r_stride, const void* k, int64_t k
                        int64_t rank, float decay_scale, int32_t act_f32, nvh_stream_t stream);
 int32_t nvh_delta_scan(const float* pack, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
                        const int32_t* context_lens, float* out, int64_t batch, int64_t heads, int64_t dk, int64_t dv, nvh_stream_t stream);
+/* nvh_delta_scan whose portions of at least min_tokens tokens go through chunks of 16 tokens (the others as in nvh_delta_scan): results within
+ * rounding of the token-by-token ones.  num_tokens = cu_seqlens_q[batch]; cu_seqlens_q is required, pack and workspace are 16-byte aligned;
+ * workspace: nvh_delta_chunk_workspace_bytes (0: these head sizes have no chunked form). */
+int64_t nvh_delta_chunk_workspace_bytes(int64_t num_tokens, int64_t batch, int64_t heads, int64_t dk, int64_t dv);
+int32_t nvh_delta_scan_chunked(const float* pack, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                               const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens, int64_t heads, int64_t dk, int64_t dv,
+                               int64_t min_tokens, float* workspace, nvh_stream_t stream);
 int32_t nvh_delta_post(const float* o, const void* norm_weight, const void* gate, int64_t gate_stride, void* y, int64_t y_stride,
                        int64_t rows, int64_t heads, int64_t dv, float eps, int32_t act_f32, nvh_stream_t stream);
 

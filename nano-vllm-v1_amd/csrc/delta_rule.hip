@@ -8,8 +8,10 @@
 //   nvh_delta_scan   walks a sequence's tokens in order from the state its slot holds (or from zero when the sequence
 //                    starts) and leaves the state there.  Columns of S are independent of each other, so the work is
 //                    spread over (sequence, head, column); each column is held by 16 lanes (4 when dk is no multiple
-//                    of 16), each with every 16th (4th) row, which meet twice per token in a cross-lane sum.  The order of every sum is fixed by the sizes alone: decoding
-//                    token by token, in portions or in one piece gives the same bits.
+//                    of 16), each with every 16th (4th) row, which meet twice per token in a cross-lane sum.  The order of
+//                    every sum is fixed by the sizes alone: decoding token by token, or cut into other portions, gives the
+//                    same bits.
+//   nvh_delta_scan_chunked   the same, portions of many tokens in chunks of 16 (see there).
 //   nvh_delta_post   per head: o / rms(o), times the norm weight and the sigmoid output gate, to the activation type.
 //   nvh_gated_delta_prep   the gated delta rule, S <- g S; d = beta (v - S^T k); S <- S + k d^T; o = S^T q, with one decay g per head
 //                    and a write strength beta per head, is the recurrence above with w = g on every channel, u = k (a unit
@@ -160,6 +162,7 @@ struct DeltaScanArgs {
     const int32_t* context_lens;    // [B]: tokens of the sequence including this step's (a step that holds them all starts from zero)
     float* out;                // [T, H*dv]
     int H, dk, dv;
+    int skip_from;             // portions of this many tokens and more are left to the chunked form (0: none)
 };
 
 // Lanes per state column (SUBS: 16 when dk is a multiple of 16, else 4), rows i = SUBS * ii + sub held by lane `sub`; a
@@ -179,6 +182,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
     const int lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : seq, hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : seq + 1;
     const int slot = p.slots[seq];
     if (slot < 0 || hi <= lo) return;                        // a padded row (uniform over the workgroup)
+    if (p.skip_from > 0 && hi - lo >= p.skip_from) return;
     const bool fresh = p.context_lens[seq] == hi - lo;
     float* sp = p.state + (((int64_t)slot * p.H + head) * dk) * dv;
     float S[DKQ];
@@ -303,6 +307,470 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
     }
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// The chunked form, for portions of many tokens (token by token every token costs the chain S -> u^T S -> S, 0.25 - 0.33 us, whatever the chip
+// has idle).  Within a chunk of 16 tokens the recurrence is linear in the chunk's first state S0.  With P_t the product of the decays of tokens
+// 0 .. t, the removals d_t = u_t^T S_(t-1) satisfy
+//   d_t + sum_(s<t) A_ts d_s = (u_t P_(t-1)) S0 + sum_(s<t) K_ts v_s,    A_ts = u_t . (w_(s+1) .. w_(t-1) a_s),  K_ts the same with k_s,
+// a unit lower triangular system, so D = W S0 + Y and, with the outputs' own pair products, O = Q S0 + Z, and the state behind the chunk is
+//   S = P_15 S0 + K'^T V - A'^T D,      K'_s = w_(s+1) .. w_15 k_s,  A' likewise.
+// W, Q, Y, Z, K', A' and P need no state: one launch forms them for all chunks at once.  The second launch walks the chunks: per chunk products of
+// 16 x 16 a wave on the matrix cores and one meeting of the waves.  Results differ from the token-by-token form within rounding.  What is summed over
+// a chunk's pairs of tokens, the triangular inverse and K'^T V are held in double (against float64, in the 2-norm over 1024 tokens: outputs 4.8e-8,
+// states 5.0e-8; token by token 8.3e-8 and 4.9e-8; with K'^T V in fp32 7.2e-8 for the states).
+// us at one sequence of 1024 tokens, token by token and in chunks (both launches): 16 heads of 64 x 64: 271, 27 + 47; 8 heads of 128 x 128: 331,
+// 28 + 75.  The first launch is bound by its chain when the chip is not full (11 us at 256 tokens), and else by the double products (172 us at 8448
+// records of 64 x 64); the second by the chain of a chunk, 0.74 us.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+constexpr int CT = 16;                                       // tokens of a chunk
+constexpr int MLD = CT + 1;                                  // doubles a row of a 16 x 16 matrix takes in LDS (its columns then lie in different banks)
+
+// What the first launch keeps in LDS: r | k | w | u | au, 16 rows of dk + 4 floats each, and in doubles the decays and their reciprocals (16 rows of
+// dk + 2 each), which later give their place to four matrices.
+__host__ __device__ constexpr int chunk_rows_floats(int dk) { return 5 * CT * (dk + 4); }
+__host__ __device__ constexpr int chunk_doubles(int dk) { return 2 * CT * (dk + 2) > 4 * CT * MLD ? 2 * CT * (dk + 2) : 4 * CT * MLD; }
+
+struct DeltaChunkArgs {
+    DeltaScanArgs s;
+    float* ws;                 // a record per (chunk slot, head), see chunk_record
+    int batch;
+};
+
+// Floats of a record: W | Q | A'^T | K'^T (16 dk each, as the lanes of the second launch read them) | P (dk) | Y | Z | V (16 dv each, likewise).
+__host__ __device__ __forceinline__ int64_t chunk_record(int dk, int dv) { return 65 * (int64_t)dk + 48 * (int64_t)dv; }
+// First chunk slot of a sequence whose tokens start at row `lo`: sequences never overlap, and all fit num_tokens / 16 + batch slots.
+__device__ __forceinline__ int chunk_base(int lo, int seq) { return lo / CT + seq; }
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const u32x2 v = __builtin_bit_cast(u32x2, x);
+    const u32x2 r = {(uint32_t)__builtin_amdgcn_mov_dpp((int)v[0], CTRL, 0xf, 0xf, true), (uint32_t)__builtin_amdgcn_mov_dpp((int)v[1], CTRL, 0xf, 0xf, true)};
+    return __builtin_bit_cast(double, r);
+}
+// The sums of four values over the 16 lanes of a row; lane g is left with that of value g & 3.
+__device__ __forceinline__ double row16_sum4(double v0, double v1, double v2, double v3, int g) {
+    const bool odd = g & 1, high = g & 2;
+    const double lo = (odd ? v1 : v0) + dpp_f64<0xB1>(odd ? v0 : v1), hi = (odd ? v3 : v2) + dpp_f64<0xB1>(odd ? v2 : v3);     // neighbours
+    double x = (high ? hi : lo) + dpp_f64<0x4E>(high ? lo : hi);         // pairs
+    x += dpp_f64<0x124>(x);                                              // rotations by 4 and 8 within the row
+    return x + dpp_f64<0x128>(x);
+}
+
+// Lower triangular 16 x 16 matrices in double on the matrix cores.  Index i of an operand or of a result's column (lane & 15) stands for token
+// chunk_tok(i): element e of a lane in quarter q of the wave is then token 4 q + e, in a result's rows as in the contraction's steps.  So a result is
+// the next product's right operand as it stands, and its transpose's left operand; what is needed as a left operand is carried transposed too.
+__device__ __forceinline__ int chunk_tok(int i) { return 4 * (i & 3) + (i >> 2); }
+
+struct Tri {
+    f64x4 n, t;                // X and its transpose
+};
+
+__device__ __forceinline__ f64x4 mfma_f64(const f64x4& l, const f64x4& r, f64x4 c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f64_16x16x4f64(l[e], r[e], c, 0, 0, 0);
+    return c;
+}
+// c + l r where only l's tokens up to a result's own row (T: column) enter, and nothing above the diagonal: what is not finite in a token then
+// leaves the tokens before it alone.  W: r's columns are channels and not tokens.
+template <bool T, bool W>
+__device__ __forceinline__ f64x4 mfma_f64_below(const f64x4& l, const f64x4& r, const f64x4& c, int q, int own) {
+    f64x4 res = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int t = 0; t < CT; ++t) {
+        f64x4 lm, rm;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const bool in = 4 * q + e <= t;
+            lm[e] = in ? l[e] : 0.0;
+            rm[e] = in ? r[e] : 0.0;
+        }
+        const f64x4 x = mfma_f64(lm, rm, c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (T ? own == t && (W || 4 * q + e <= t) : 4 * q + e == t && (W || own <= t)) res[e] = x[e];
+    }
+    return res;
+}
+template <bool SAFE>
+__device__ __forceinline__ f64x4 tri_mul_n(const f64x4& l, const f64x4& r, const f64x4& c, int q, int own) {      // l: the left matrix transposed
+    if constexpr (SAFE) return mfma_f64_below<false, false>(l, r, c, q, own);
+    else return mfma_f64(l, r, c);
+}
+template <bool SAFE>
+__device__ __forceinline__ f64x4 tri_mul_t(const f64x4& l, const f64x4& r, const f64x4& c, int q, int own) {      // the transposed product
+    if constexpr (SAFE) return mfma_f64_below<true, false>(l, r, c, q, own);
+    else return mfma_f64(l, r, c);
+}
+
+// From a chunk's pair products A, K, Rk, Ra to what its columns are multiplied with, as left operands (that is, transposed):
+//   T = (I + A)^-1 = (I - A)(I + A^2)(I + A^4)(I + A^8)   (A^16 = 0; in double, since powers may be large),
+//   G = Ra T,   M = T K,   N = Rk - Ra M,      so that   W = T U',  Q = R' - G U',  Y = M V,  Z = N V.
+struct ChunkFactors {
+    f64x4 T, G, M, N;
+};
+template <bool SAFE>
+__device__ __forceinline__ ChunkFactors chunk_factors(const double* mats, int q, int own) {
+    const f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+    auto load = [&](int which, bool strict) {
+        Tri x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * q + e;
+            x.n[e] = mats[(which * CT + t) * MLD + own];
+            x.t[e] = mats[(which * CT + own) * MLD + t];
+            if (SAFE && (strict ? own >= t : own > t)) x.n[e] = 0.0;
+            if (SAFE && (strict ? t >= own : t > own)) x.t[e] = 0.0;
+        }
+        return x;
+    };
+    const Tri A = load(0, true), K = load(1, true), Rk = load(2, false), Ra = load(3, false);
+    auto square = [&](const Tri& x) { return Tri{tri_mul_n<SAFE>(x.t, x.n, zero, q, own), tri_mul_t<SAFE>(x.n, x.t, zero, q, own)}; };
+    auto grow = [&](const Tri& x, const f64x4& pn) { return Tri{tri_mul_n<SAFE>(x.t, pn, x.n, q, own), tri_mul_t<SAFE>(pn, x.t, x.t, q, own)}; };
+    const Tri P2 = square(A), P4 = square(P2);
+    const f64x4 P8 = tri_mul_n<SAFE>(P4.t, P4.n, zero, q, own);
+    Tri T;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const double one = 4 * q + e == own ? 1.0 : 0.0;
+        T.n[e] = one - A.n[e];
+        T.t[e] = one - A.t[e];
+    }
+    T = grow(T, P2.n);
+    T = grow(T, P4.n);
+    T = grow(T, P8);
+    ChunkFactors f;
+    f.T = T.t;
+    f.G = tri_mul_t<SAFE>(T.n, Ra.t, zero, q, own);
+    const f64x4 Mn = tri_mul_n<SAFE>(T.t, K.n, zero, q, own);
+    f.M = tri_mul_t<SAFE>(K.n, T.t, zero, q, own);
+    f.N = Rk.t - tri_mul_t<SAFE>(Mn, Ra.t, zero, q, own);
+    return f;
+}
+
+// CPL: key channels a lane of the pair products holds (dk = 16 CPL).
+template <int CPL>
+__global__ __launch_bounds__(256, CPL <= 4 ? 4 : 2) void delta_chunk_prep_kernel(DeltaChunkArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];       // (chunk_rows_floats, chunk_doubles)
+    const DeltaScanArgs& p = a.s;
+    constexpr int dk = 16 * CPL, LD = dk + 4, DLD = dk + 2;
+    const int dv = p.dv, head = blockIdx.x, cslot = blockIdx.y, tid = threadIdx.x;
+    int first = 0, end = a.batch;                            // the last sequence whose chunk slots begin at or before this one
+    while (end - first > 1) {
+        const int mid = (first + end) >> 1;
+        if (chunk_base(p.cu_seqlens_q[mid], mid) <= cslot) first = mid;
+        else end = mid;
+    }
+    const int lo = p.cu_seqlens_q[first], hi = p.cu_seqlens_q[first + 1];
+    const int t0 = lo + CT * (cslot - chunk_base(lo, first)), nt = min(CT, hi - t0);
+    if (hi - lo < p.skip_from || nt <= 0 || p.slots[first] < 0) return;      // (uniform)
+    const int64_t prow = 5 * dk + dv, tok_stride = (int64_t)p.H * prow;
+    const float* base = p.pack + (int64_t)t0 * tok_stride + (int64_t)head * prow;
+    float* rec = a.ws + ((int64_t)cslot * p.H + head) * chunk_record(dk, dv);
+    auto row = [&](int which, int t) { return sm + (which * CT + t) * LD; };
+    double *mats = reinterpret_cast<double*>(sm + chunk_rows_floats(dk)), *cums = mats, *rcums = mats + CT * DLD;
+    // Everything the workgroup reads is requested at once, on every path (a load under a condition would be waited for on its own).  Tokens beyond
+    // the portion's end change nothing: decay 1, everything else 0.
+    constexpr int PIECES = CT * 5 * dk / 4, ROUNDS = (PIECES + 255) / 256;
+    f32x4 piece[ROUNDS];
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const int e = min(tid + 256 * i, PIECES - 1), t = e / (5 * dk / 4), c4 = (e - t * (5 * dk / 4)) * 4;
+        piece[i] = *reinterpret_cast<const f32x4*>(base + min(t, nt - 1) * tok_stride + c4);
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, q = lane >> 4, vtiles = dv >> 4;
+    constexpr int VAHEAD = 2;                                // tiles of v that a wave requests up front
+    f32x4 vt[VAHEAD];
+    auto load_v = [&](int tile) {                            // (this lane's four tokens of a column)
+        const float* vp = base + 5 * dk + 16 * min(tile, vtiles - 1) + col;
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = vp[min(4 * q + e, nt - 1) * tok_stride];
+        return x;
+    };
+#pragma unroll
+    for (int i = 0; i < VAHEAD; ++i) vt[i] = load_v(wave + 4 * i);
+    bool odd = false;                                        // does r, k, w, u or au hold a value that is not finite
+#pragma unroll
+    for (int i = 0; i < ROUNDS; ++i) {
+        const int e = tid + 256 * i, t = e / (5 * dk / 4), c4 = (e - t * (5 * dk / 4)) * 4, which = c4 / dk;
+        const float fill = which == 2 ? 1.f : 0.f;
+        if (PIECES % 256 == 0 || e < PIECES) *reinterpret_cast<f32x4*>(row(which, t) + (c4 - which * dk)) = t < nt ? piece[i] : f32x4{fill, fill, fill, fill};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) odd |= !(fabsf(piece[i][c]) <= 3.402823466e+38f);
+    }
+    odd = __syncthreads_or(odd);
+    const int s = tid >> 4, g = tid & 15, ch = g * CPL, own = chunk_tok(col);
+    const f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+    double cum[CPL], before[CPL];                            // the decay up to token s, with and without its own
+    bool far = odd;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) before[i] = 1.0;
+#pragma unroll 4
+    for (int t = 0; t < CT - 1; ++t) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const double w = row(2, t)[ch + i];
+            before[i] *= t < s ? w : 1.0;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+        cum[i] = before[i] * row(2, s)[ch + i];
+        far |= !(cum[i] >= 1e-80 && cum[i] <= 1e80);
+        cums[s * DLD + ch + i] = cum[i];
+        rcums[s * DLD + ch + i] = 1.0 / cum[i];
+    }
+    far = __syncthreads_or(far);
+    float ap[CPL], kp[CPL];                                  // a and k of token s, decayed to the chunk's end
+    f64x4 pairs = zero;
+    if (!far) {
+        // A, K, Rk, Ra = U' (a / cum)^T, U' (k / cum)^T, R' (k / cum)^T, R' (a / cum)^T, a matrix a wave; a lane's channels of a step are those
+        // of quarter q.  All in double, where the quotients neither over- nor underflow within the limits checked above.
+        const bool r_left = wave >= 2, k_right = wave == 1 || wave == 2;
+        const float *lrow = row(r_left ? 0 : 3, own) + q * (dk / 4), *rrow = row(k_right ? 1 : 4, own) + q * (dk / 4);
+        const double *lcum = cums + (r_left ? own : max(own - 1, 0)) * DLD + q * (dk / 4), *rcum = rcums + own * DLD + q * (dk / 4);
+        const bool first_u = !r_left && own == 0;
+        f64x4 other = zero;
+#pragma unroll
+        for (int j = 0; j < dk / 4; j += 2) {
+            const double l0 = lrow[j] * (first_u ? 1.0 : lcum[j]), l1 = lrow[j + 1] * (first_u ? 1.0 : lcum[j + 1]);
+            pairs = __builtin_amdgcn_mfma_f64_16x16x4f64(l0, rrow[j] * rcum[j], pairs, 0, 0, 0);
+            other = __builtin_amdgcn_mfma_f64_16x16x4f64(l1, rrow[j + 1] * rcum[j + 1], other, 0, 0, 0);
+        }
+        pairs += other;
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const double rest = cums[(CT - 1) * DLD + ch + i] * rcums[s * DLD + ch + i];
+            ap[i] = (float)(row(4, s)[ch + i] * rest);
+            kp[i] = (float)(row(1, s)[ch + i] * rest);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 4 * q + e;
+            mats[(wave * CT + t) * MLD + own] = (r_left ? own <= t : own < t) ? pairs[e] : 0.0;
+        }
+    } else {                                                 // 16 lanes share token s, each with CPL channels, and walk t = 0 .. 15
+        double xa[CPL], xk[CPL];
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) xa[i] = xk[i] = 0.0;
+#pragma unroll 1
+        for (int t = 0; t < CT; ++t) {
+            double dA = 0.0, dK = 0.0, dRk = 0.0, dRa = 0.0;
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                const double u = row(3, t)[ch + i], w = row(2, t)[ch + i], r = row(0, t)[ch + i];
+                dA = __builtin_fma(u, xa[i], dA);
+                dK = __builtin_fma(u, xk[i], dK);
+                xa[i] = t == s ? row(4, t)[ch + i] : xa[i] * w;
+                xk[i] = t == s ? row(1, t)[ch + i] : xk[i] * w;
+                dRk = __builtin_fma(r, xk[i], dRk);
+                dRa = __builtin_fma(r, xa[i], dRa);
+            }
+            const double sum = row16_sum4(dA, dK, dRk, dRa, g);
+            if (g < 4) mats[(g * CT + t) * MLD + s] = sum;
+        }
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            ap[i] = (float)xa[i];
+            kp[i] = (float)xk[i];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {                          // A', K', U', R' in place
+        row(4, s)[ch + i] = ap[i];
+        row(1, s)[ch + i] = kp[i];
+        row(3, s)[ch + i] = (float)(row(3, s)[ch + i] * before[i]);
+        row(0, s)[ch + i] = (float)(row(0, s)[ch + i] * cum[i]);
+        if (s == CT - 1) rec[64 * dk + ch + i] = (float)cum[i];
+    }
+    __syncthreads();
+    ChunkFactors f;                                          // computed by one wave, not always on the same SIMD
+    const bool elected = wave == (int)((blockIdx.x / 8 + blockIdx.y) & 3);
+    if (elected) {
+        f = odd ? chunk_factors<true>(mats, q, own) : chunk_factors<false>(mats, q, own);
+        f64x4* out = reinterpret_cast<f64x4*>(mats) + lane;
+        out[0] = f.T;
+        out[64] = f.G;
+        out[128] = f.M;
+        out[192] = f.N;
+    }
+    __syncthreads();
+    {
+        const f64x4* in = reinterpret_cast<const f64x4*>(mats) + lane;
+        f.T = in[0];
+        f.G = in[64];
+        f.M = in[128];
+        f.N = in[192];
+    }
+#pragma unroll
+    for (int i = 0; i < (CPL + 3) / 4; ++i) {                // 16 key channels a wave: W and Q with the channels as rows, as the second launch reads them
+        const int tile = wave + 4 * i;
+        if (CPL % 4 && tile >= CPL) break;
+        const int c0 = 16 * tile;
+        f64x4 u, Q;
+        const f32x4 rp = *reinterpret_cast<const f32x4*>(row(0, own) + c0 + 4 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            u[e] = row(3, 4 * q + e)[c0 + own];
+            Q[e] = rp[e];
+        }
+        f64x4 W;
+        if (odd) {
+            W = mfma_f64_below<true, true>(u, f.T, zero, q, own);
+            Q -= mfma_f64_below<true, true>(u, f.G, zero, q, own);
+        } else {
+            W = mfma_f64(u, f.T, zero);
+            Q -= mfma_f64(u, f.G, zero);
+        }
+        float* out = rec + (tile * 64 + q * 16 + own) * 4;
+        *reinterpret_cast<f32x4*>(out) = f32x4{(float)W[0], (float)W[1], (float)W[2], (float)W[3]};
+        *reinterpret_cast<f32x4*>(out + 16 * dk) = f32x4{(float)Q[0], (float)Q[1], (float)Q[2], (float)Q[3]};
+        f32x4 A, K;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            A[e] = row(4, 4 * q + e)[c0 + col];
+            K[e] = row(1, 4 * q + e)[c0 + own];              // (for a product in double, whose rows lie otherwise)
+        }
+        float* at = rec + 32 * dk + (tile * 64 + lane) * 4;
+        *reinterpret_cast<f32x4*>(at) = A;
+        *reinterpret_cast<f32x4*>(at + 16 * dk) = K;
+    }
+    auto values = [&](int tile, f32x4 v) {                   // 16 columns of v: Y and Z
+        f64x4 x;
+        bool vodd = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (4 * q + e >= nt) v[e] = 0.f;
+            vodd |= !(fabsf(v[e]) <= 3.402823466e+38f);
+            x[e] = v[e];
+        }
+        f64x4 Y, Z;
+        if (odd || __any(vodd)) {
+            Y = mfma_f64_below<false, true>(f.M, x, zero, q, own);
+            Z = mfma_f64_below<false, true>(f.N, x, zero, q, own);
+        } else {
+            Y = mfma_f64(f.M, x, zero);
+            Z = mfma_f64(f.N, x, zero);
+        }
+        float* out = rec + 65 * dk + (tile * 64 + lane) * 4;
+        *reinterpret_cast<f32x4*>(out) = f32x4{(float)Y[0], (float)Y[1], (float)Y[2], (float)Y[3]};
+        *reinterpret_cast<f32x4*>(out + 16 * dv) = f32x4{(float)Z[0], (float)Z[1], (float)Z[2], (float)Z[3]};
+        *reinterpret_cast<f32x4*>(out + 32 * dv) = v;
+    };
+#pragma unroll
+    for (int i = 0; i < VAHEAD; ++i)
+        if (wave + 4 * i < vtiles) values(wave + 4 * i, vt[i]);
+    for (int tile = wave + 4 * VAHEAD; tile < vtiles; tile += 4) values(tile, load_v(tile));
+}
+
+// NW waves of 16 key channels each hold 16 columns of a head's state, in the layout in which a product leaves its result (row 4 q + e of lane
+// (q, column) in element e) - which is also the layout in which it takes its right operand, so a state never moves between lanes.  One wave
+// more sums the waves' parts of the outputs, a chunk behind, and writes them.
+template <int NW>
+__global__ __launch_bounds__(64 * NW + 64) void delta_chunk_scan_kernel(DeltaChunkArgs a) {
+    __shared__ f32x4 meet_d[2][NW][64], meet_o[2][NW][64];   // [chunk parity][wave][lane]
+    const DeltaScanArgs& p = a.s;
+    constexpr int dk = 16 * NW;
+    const int seq = blockIdx.x, head = blockIdx.y, dv = p.dv, cb = blockIdx.z;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int lo = p.cu_seqlens_q[seq], hi = p.cu_seqlens_q[seq + 1], slot = p.slots[seq];
+    if (slot < 0 || hi <= lo || hi - lo < p.skip_from) return;       // (uniform)
+    const int64_t record = chunk_record(dk, dv), step = (int64_t)p.H * record;
+    const float* rec = a.ws + ((int64_t)chunk_base(lo, seq) * p.H + head) * record;
+    const int chunks = (hi - lo + CT - 1) / CT;
+    if (wave == NW) {                                        // the outputs: the parts of chunk j are written before the barrier of chunk j + 1
+        float* out = p.out + (int64_t)lo * p.H * dv + head * dv + 16 * cb + col;
+        const float* zp = rec + 65 * dk + 16 * dv + (cb * 64 + lane) * 4;
+        f32x4 z = *reinterpret_cast<const f32x4*>(zp);
+        __syncthreads();
+        for (int j = 0; j < chunks; ++j) {
+            const f32x4 after = *reinterpret_cast<const f32x4*>(zp + min(j + 1, chunks - 1) * step);
+            __syncthreads();
+            f32x4 res = meet_o[j & 1][0][lane];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) res += meet_o[j & 1][w][lane];
+            res += z;
+            z = after;
+            const int t = CT * j + 4 * q;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (lo + t + e < hi) out[(int64_t)(t + e) * p.H * dv] = res[e];
+        }
+        return;
+    }
+    const bool fresh = p.context_lens[seq] == hi - lo;
+    float* sp = p.state + (((int64_t)slot * p.H + head) * dk + 16 * wave + 4 * q) * dv + 16 * cb + col;
+    f32x4 S = {0.f, 0.f, 0.f, 0.f};
+    if (!fresh) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = sp[(int64_t)e * dv];
+    }
+    struct Operands {
+        f32x4 W, Q, A, K, P, Y, V;
+    };
+    auto fetch = [&](int j, Operands& x) {
+        const float* r = rec + min(j, chunks - 1) * step;
+        const float* m = r + (wave * 64 + lane) * 4;
+        const float* n = r + 65 * dk + (cb * 64 + lane) * 4;
+        x.W = *reinterpret_cast<const f32x4*>(m);
+        x.Q = *reinterpret_cast<const f32x4*>(m + 16 * dk);
+        x.A = *reinterpret_cast<const f32x4*>(m + 32 * dk);
+        x.K = *reinterpret_cast<const f32x4*>(m + 48 * dk);
+        x.P = *reinterpret_cast<const f32x4*>(r + 64 * dk + 16 * wave + 4 * q);
+        x.Y = *reinterpret_cast<const f32x4*>(n);
+        x.V = *reinterpret_cast<const f32x4*>(n + 32 * dv);
+    };
+    // The chain of a chunk is D's product, the meeting and A's product; what does not depend on the meeting runs in its shadow.
+    auto chunk = [&](int j, const Operands& x) {
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        f32x4 d = zero, o = zero, ad = zero;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[e], S[e], d, 0, 0, 0);
+        meet_d[j & 1][wave][lane] = d;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[e], S[e], o, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();                                     // (the buffers of the other parity: every wave has left them before it came here)
+        f32x4 part[NW];
+#pragma unroll
+        for (int w = 0; w < NW; ++w) part[w] = meet_d[j & 1][w][lane];
+        meet_o[j & 1][wave][lane] = o;
+        __builtin_amdgcn_sched_barrier(0);
+        f64x4 kv = {0.0, 0.0, 0.0, 0.0};                     // (most of what a state is off by came from this sum, in fp32)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)x.V[e], kv, 0, 0, 0);
+        f32x4 sum = x.Y;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += part[w];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ad = __builtin_amdgcn_mfma_f32_16x16x4f32(x.A[e], sum[e], ad, 0, 0, 0);
+        #pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = x.P[e] * S[e] + ((float)kv[e] - ad[e]);
+    };
+    constexpr int AHEAD = NW <= 4 ? 4 : 3;                   // records in flight
+    Operands x[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) fetch(i, x[i]);
+    int j = 0;
+    for (; j + AHEAD <= chunks; j += AHEAD) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            chunk(j + i, x[i]);
+            fetch(j + i + AHEAD, x[i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD - 1; ++i)
+        if (j + i < chunks) chunk(j + i, x[i]);
+    __syncthreads();                                         // (the last chunk's outputs)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sp[(int64_t)e * dv] = S[e];
+}
+
 template <typename A>
 __global__ __launch_bounds__(256) void delta_post_kernel(const float* __restrict__ o, const A* __restrict__ norm_w, const A* __restrict__ gate,
                                                          int64_t gate_stride, A* __restrict__ y, int64_t y_stride, int64_t rows, int H, int dv, float eps) {
@@ -407,8 +875,53 @@ extern "C" int32_t nvh_delta_scan(const float* pack, float* state, const int32_t
     NVH_REQUIRE(batch >= 0 && heads > 0 && dk > 0 && dv > 0, NVH_EINVAL, "nvh_delta_scan: bad sizes");
     NVH_REQUIRE(dk <= 256, NVH_ENOSYS, "nvh_delta_scan: key size %ld above 256", (long)dk);
     if (batch == 0) return NVH_OK;
-    DeltaScanArgs p{pack, state, slots, cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv};
+    DeltaScanArgs p{pack, state, slots, cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 0};
     return launch_delta_scan(p, batch, (hipStream_t)stream);
+}
+
+// Head sizes that the chunked form is built for: whole 16-wide tiles, at most eight waves of key channels.
+static bool delta_chunkable(int64_t dk, int64_t dv) {
+    return dv % 16 == 0 && dv <= 16 * 65535 && (dk == 16 || dk == 32 || dk == 48 || dk == 64 || dk == 96 || dk == 128);
+}
+
+extern "C" int64_t nvh_delta_chunk_workspace_bytes(int64_t num_tokens, int64_t batch, int64_t heads, int64_t dk, int64_t dv) {
+    if (!delta_chunkable(dk, dv) || num_tokens < 0 || batch < 0 || heads <= 0 || heads > 65535 || num_tokens / CT + batch > 65535) return 0;
+    return (num_tokens / CT + batch) * heads * chunk_record((int)dk, (int)dv) * (int64_t)sizeof(float);
+}
+
+template <int CPL>
+static void launch_delta_chunks(const DeltaChunkArgs& a, int64_t slots, int64_t batch, hipStream_t st) {
+    const size_t lds = sizeof(float) * (size_t)chunk_rows_floats(16 * CPL) + sizeof(double) * (size_t)chunk_doubles(16 * CPL);
+    if (lds > 60 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prep_kernel<CPL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // (heads fastest: with a multiple of eight heads a head's records are written and read by the same XCD, through its L2)
+    delta_chunk_prep_kernel<CPL><<<dim3((unsigned)a.s.H, (unsigned)slots), 256, lds, st>>>(a);
+    delta_chunk_scan_kernel<CPL><<<dim3((unsigned)batch, (unsigned)a.s.H, (unsigned)(a.s.dv / 16)), 64 * CPL + 64, 0, st>>>(a);
+}
+
+extern "C" int32_t nvh_delta_scan_chunked(const float* pack, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                          const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens, int64_t heads, int64_t dk,
+                                          int64_t dv, int64_t min_tokens, float* workspace, nvh_stream_t stream) {
+    NVH_REQUIRE(pack && state && slots && cu_seqlens_q && context_lens && out && workspace, NVH_EINVAL, "nvh_delta_scan_chunked: null pointer");
+    NVH_REQUIRE(batch >= 0 && num_tokens >= 0 && num_tokens < (1 << 30) && heads > 0 && heads <= 65535 && num_tokens / CT + batch <= 65535 && min_tokens >= 1 && min_tokens < (1 << 30), NVH_EINVAL,
+                "nvh_delta_scan_chunked: bad sizes");
+    NVH_REQUIRE(delta_chunkable(dk, dv), NVH_ENOSYS, "nvh_delta_scan_chunked: head size %ld x %ld", (long)dk, (long)dv);
+    NVH_REQUIRE(nvh_aligned16(pack) && nvh_aligned16(workspace), NVH_EINVAL, "nvh_delta_scan_chunked: 16-byte alignment required");
+    if (batch == 0 || num_tokens == 0) return NVH_OK;
+    hipStream_t st = (hipStream_t)stream;
+    const DeltaScanArgs p{pack, state, slots, cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, (int)min_tokens};
+    const DeltaChunkArgs a{p, workspace, (int)batch};
+    const int64_t cslots = num_tokens / CT + batch;
+    switch (dk / 16) {
+        case 1: launch_delta_chunks<1>(a, cslots, batch, st); break;
+        case 2: launch_delta_chunks<2>(a, cslots, batch, st); break;
+        case 3: launch_delta_chunks<3>(a, cslots, batch, st); break;
+        case 4: launch_delta_chunks<4>(a, cslots, batch, st); break;
+        case 6: launch_delta_chunks<6>(a, cslots, batch, st); break;
+        default: launch_delta_chunks<8>(a, cslots, batch, st);
+    }
+    NVH_CHECK_LAUNCH("nvh_delta_scan_chunked");
+    if (batch == 1 && num_tokens >= min_tokens) return NVH_OK;
+    return launch_delta_scan(p, batch, st);                  // the portions below min_tokens
 }
 
 extern "C" int32_t nvh_delta_post(const float* o, const void* norm_weight, const void* gate, int64_t gate_stride, void* y, int64_t y_stride,

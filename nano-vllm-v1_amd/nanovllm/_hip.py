@@ -104,6 +104,8 @@ SIGNATURES = {
     "nvh_attn_conv_prep": (i32, [vp, i64, vp, i64, vp, vp, vp, vp, vp, i32, f32, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i32, i32, vp]),
     "nvh_attn_paged_any_parts_bytes": (i64, [i64, i64, i64, i64, i64, i64, i64, i32, i32]),
     "nvh_delta_prep": (i32, [vp, i64, vp, i64, vp, i64, vp, i64, vp, i64, vp, vp, vp, vp, i64, i64, i64, i64, f32, i32, vp]),
+    "nvh_delta_chunk_workspace_bytes": (i64, [i64, i64, i64, i64, i64]),
+    "nvh_delta_scan_chunked": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, vp]),
     "nvh_delta_scan": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, vp]),
     "nvh_gated_delta_prep": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i32, vp]),
     "nvh_delta_post": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i64, f32, i32, vp]),

@@ -50,7 +50,7 @@ class GeneralizedDeltaRule(nn.Module):
         if state is None or ctx.state_slots is None:
             raise RuntimeError("the delta rule needs a bound state pool and a state slot per sequence")
         o = ops.delta_rule(r, k, v, a_raw, lowrank, self.w2.data, self.w0.data, self.a_bias.data, state, ctx.state_slots,
-                           ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.head_dim, self.decay_scale)
+                           ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.head_dim, self.decay_scale, max_seqlen_q=ctx.max_seqlen_q or 0)
         return ops.delta_post(o, self.norm.data, g, self.num_heads, self.head_dim, self.eps)
 
 
@@ -104,7 +104,7 @@ class GatedDeltaRule(nn.Module):
         if state is None or ctx.state_slots is None:
             raise RuntimeError("the delta rule needs a bound state pool and a state slot per sequence")
         o = ops.gated_delta_rule(qkv, b, a, self.conv_weight.data, self.dt_bias.data, self.A_log.data, self.conv_inputs.pool(run), state, ctx.state_slots,
-                                 ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.qk_heads, self.key_dim, self.value_dim)
+                                 ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.qk_heads, self.key_dim, self.value_dim, max_seqlen_q=ctx.max_seqlen_q or 0)
         return ops.group_rmsnorm_gate(o, self.norm.data, self.value_dim, self.eps, gate, "silu", gate_first=False)
 
 

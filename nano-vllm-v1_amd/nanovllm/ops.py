@@ -795,14 +795,38 @@ def attn_pool_blocks(k_cache, v_cache, cu_seqlens_q, context_lens, block_tables,
               int(pool), pk.shape[1], pk.data_ptr(), pv.data_ptr(), f, _stream())
 
 
+# Portions of at least DELTA_CHUNK_MIN tokens take the delta rule's chunked form, unless so many heads of about the longest portion's length run
+# side by side that they fill the chip token by token (the chunked form reads and writes more: it is for the chain's sake).  us token by token / in
+# chunks, 16 heads of 64 x 64: 96 tokens 28.6 / 22.8, 128 tokens 36.8 / 19.2, 1024 tokens 271 / 75, four of 192 tokens 56 / 43, eight of 128 tokens
+# 42.9 / 47.4; 32 heads: four of 128 tokens 43.5 / 47.2, eight of 512 tokens 242 / 310; eight heads of 128 x 128: 96 tokens 34.4 / 35.2, 128 tokens
+# 44 / 28, 1024 tokens 331 / 104, eight of 128 tokens 67.6 / 56.8.
+DELTA_CHUNK_MIN = 128
+DELTA_CHUNK_HEADS = 96                                       # of 64 key channels
+
+
+def _delta_scan(pack, state, slots, cu_seqlens_q, context_lens, heads: int, dk: int, dv: int, max_seqlen_q: int) -> torch.Tensor:
+    t, batch = pack.shape[0], context_lens.numel()
+    out = torch.empty(t, heads * dv, dtype=F32, device=pack.device)
+    if cu_seqlens_q is not None and max_seqlen_q >= DELTA_CHUNK_MIN and 64 * t * heads <= DELTA_CHUNK_HEADS * dk * max_seqlen_q:
+        nbytes = int(_hip.lib().nvh_delta_chunk_workspace_bytes(t, batch, heads, dk, dv))
+        if nbytes:
+            ws = torch.empty(nbytes // 4, dtype=F32, device=pack.device)
+            _hip.call("nvh_delta_scan_chunked", pack.data_ptr(), state.data_ptr(), slots.data_ptr(), cu_seqlens_q.data_ptr(), context_lens.data_ptr(),
+                      out.data_ptr(), batch, t, heads, dk, dv, DELTA_CHUNK_MIN, ws.data_ptr(), _stream())
+            return out
+    _hip.call("nvh_delta_scan", pack.data_ptr(), state.data_ptr(), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(),
+              out.data_ptr(), batch, heads, dk, dv, _stream())
+    return out
+
+
 def delta_rule(r, k, v, a_raw, lowrank, w2, w0, a_bias, state, slots, cu_seqlens_q, context_lens, heads: int, dk: int,
-               decay_scale: float) -> torch.Tensor:
+               decay_scale: float, max_seqlen_q: int = 0) -> torch.Tensor:
     """One step of the generalized delta rule over the packed tokens: fp32 outputs [T, H*dk]; `state` [slots, H, dk, dk] fp32 is
     read (unless the sequence starts in this step) and left updated.  r, k, v, a_raw, lowrank: column views of the fused
-    projection output (row stride free)."""
+    projection output (row stride free).  `max_seqlen_q`: the most tokens a sequence brings (0: unknown; portions of DELTA_CHUNK_MIN and
+    more then still go token by token)."""
     f = _act_flag(r, k, v, a_raw, lowrank, w2, w0, a_bias)
     t = r.shape[0]
-    batch = context_lens.numel()
     for x in (r, k, v, a_raw, lowrank):
         assert x.stride(1) == 1 and x.shape[0] == t
     assert state.dtype == F32 and state.is_contiguous() and tuple(state.shape[1:]) == (heads, dk, dk) and slots.dtype == torch.int32
@@ -812,19 +836,16 @@ def delta_rule(r, k, v, a_raw, lowrank, w2, w0, a_bias, state, slots, cu_seqlens
     _hip.call("nvh_delta_prep", r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), a_raw.data_ptr(),
               a_raw.stride(0), lowrank.data_ptr(), lowrank.stride(0), w2.data_ptr(), w0.data_ptr(), a_bias.data_ptr(), pack.data_ptr(),
               t, heads, dk, rank, float(decay_scale), f, _stream())
-    out = torch.empty(t, heads * dk, dtype=F32, device=r.device)
-    _hip.call("nvh_delta_scan", pack.data_ptr(), state.data_ptr(), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(),
-              out.data_ptr(), batch, heads, dk, dk, _stream())
-    return out
+    return _delta_scan(pack, state, slots, cu_seqlens_q, context_lens, heads, dk, dk, max_seqlen_q)
 
 
 def gated_delta_rule(qkv, b, a, conv_w, dt_bias, a_log, conv_state, state, slots, cu_seqlens_q, context_lens, heads: int, qk_heads: int,
-                     dk: int, dv: int) -> torch.Tensor:
+                     dk: int, dv: int, max_seqlen_q: int = 0) -> torch.Tensor:
     """One step of the gated delta rule over the packed tokens: fp32 outputs [T, H*dv].  `qkv`: the column view q | k | v of the
     projection rows (qk_heads*dk, qk_heads*dk, heads*dv channels), convolved over time with `conv_w` [C, taps] (continued from
     `conv_state` [slots, taps - 1, C] fp32, then brought up to date) and passed through silu; `b`, `a`: column views [T, H] of the
     write-strength and decay logits.  `state` [slots, H, dk, dv] fp32 is read (unless the sequence starts in this step) and left
-    updated."""
+    updated.  `max_seqlen_q` as in delta_rule."""
     f = _act_flag(qkv, b, a, conv_w, dt_bias, a_log)
     t, c = qkv.shape[0], 2 * qk_heads * dk + heads * dv
     taps = conv_w.shape[1]
@@ -840,10 +861,7 @@ def gated_delta_rule(qkv, b, a, conv_w, dt_bias, a_log, conv_state, state, slots
               batch, t, taps, heads, qk_heads, dk, dv, f, _stream())
     _hip.call("nvh_conv_state_update", qkv.data_ptr(), qkv.stride(0), _p(conv_state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch,
               taps, c, f, _stream())
-    out = torch.empty(t, heads * dv, dtype=F32, device=qkv.device)
-    _hip.call("nvh_delta_scan", pack.data_ptr(), state.data_ptr(), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(),
-              out.data_ptr(), batch, heads, dk, dv, _stream())
-    return out
+    return _delta_scan(pack, state, slots, cu_seqlens_q, context_lens, heads, dk, dv, max_seqlen_q)
 
 
 def delta_post(o: torch.Tensor, norm_weight: torch.Tensor, gate: torch.Tensor | None, heads: int, dv: int, eps: float) -> torch.Tensor:
