@@ -420,6 +420,244 @@ __global__ __launch_bounds__(256) void attn_paged_any_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// The same attention for fp32 caches on the matrix cores (16x16x4, fp32 in and out), dim = 16 NKS and vdim = 16 NVT, pages of whole 16-key blocks.
+// A workgroup is 16 rows - consecutive queries of one head or, where every sequence brings one query (`grouped`), the heads of a KV group - and its
+// four waves take every fourth block of 16 keys: S^T = K Q^T leaves a lane the scores of query lane % 16 and keys 4 (lane / 16) + e, which is how
+// O^T = V^T P^T takes them, so nothing is exchanged but a maximum.  A value is used once per workgroup: keys and values go from the cache to the
+// registers, the next block's while this one's products run, and LDS holds only the waves' results for the merge.  Which wave a key falls to depends
+// on its position alone and a row's results on no other row, so neither the cut nor the batch changes a bit.
+// us, the form above (two scalar LDS reads for two multiply-adds) and this one, 16 heads of 128 x 128 over 8: 301 queries 168 and 26, 1024 queries 897
+// and 127, 1024 at the end of 4096 keys 4468 and 464, one query over 1500 keys 778 and 58, 64 x one over 700 keys 1134 and 72; 16 heads of 256 x 192
+// over one, 1024 queries: 1673 and 210.  A short prompt is bound by the chain of its longest tile (load, product, exponentials, product per 64 keys),
+// a long one by the fp32 products (124 TFLOP/s at most).
+template <int NKS, int NVT>
+__global__ __launch_bounds__(256) void attn_paged_f32_kernel(AttnArgs a, int grouped) {
+    extern __shared__ __attribute__((aligned(16))) float smem[];     // [4 waves][16 rows][vdim + 4] outputs, then [4][16] maxima and sums
+    constexpr int dim = 16 * NKS, vdim = 16 * NVT, OLD = vdim + 4, BLOCK = 16, TILE = 64;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, row = lane & 15, quarter = lane >> 4;
+    const int group = a.H / a.G;
+    int seq = -1, q0 = 0, qlen = 1, qbase = 0, head0, nq;
+    if (grouped) {
+        const int parts = (group + 15) / 16, part = blockIdx.y % parts;
+        if ((int)blockIdx.x < a.batch) seq = qbase = blockIdx.x;
+        head0 = (blockIdx.y / parts) * group + 16 * part;
+        nq = min(16, group - 16 * part);
+    } else {
+        int tile = blockIdx.x;
+        for (int b = 0; b < a.batch; ++b) {
+            const int lo = a.cu_seqlens_q ? a.cu_seqlens_q[b] : b, hi = a.cu_seqlens_q ? a.cu_seqlens_q[b + 1] : b + 1;
+            const int tiles = (hi - lo + AQ - 1) / AQ;
+            if (tile < tiles) {
+                seq = b;
+                q0 = tile * AQ;
+                qlen = hi - lo;
+                qbase = lo;
+                break;
+            }
+            tile -= tiles;
+        }
+        head0 = blockIdx.y;
+        nq = min(AQ, qlen - q0);
+    }
+    if (seq < 0) return;                                     // (uniform over the workgroup)
+    const int kvh = head0 / group;
+    const int past = a.context_lens[seq] - qlen;             // keys before this step's first query
+    const int myrow = min(row, nq - 1), head = grouped ? head0 + myrow : head0, qtok = grouped ? 0 : q0 + myrow;      // (rows past nq repeat the last)
+    const int qpos = past + qtok, last_key = past + q0 + (grouped ? 0 : nq - 1);
+    const int32_t* table = a.block_tables + (int64_t)seq * a.table_stride;
+    const int nblocks = a.pool > 0 ? blocks_seen(last_key, a.window, a.pool) : 0, my_blocks = a.pool > 0 ? blocks_seen(qpos, a.window, a.pool) : 0;
+    const TileOrder order(TileWalk(a.window, a.keep_first, a.chunk, past + q0, TILE), nblocks);
+    const float *kc = (const float*)a.k_cache, *vc = (const float*)a.v_cache;
+    f32x4 k[NKS], v[NVT], acc[NVT], qr[NKS];
+    // The block of the tile at k0 that is this wave's.  Blocks past the last key repeat the one that holds it: nobody sees them.
+    auto fetch_k = [&](int k0) {
+        const float* src;
+        if (k0 < 0) {
+            int pi, at;
+            block_place(min(order.block_of(k0) + BLOCK * wave + row, nblocks - 1), a.pool, a.page, pi, at);
+            src = (const float*)a.pk + (((int64_t)table[pi] * a.pool_rows + at) * a.G + kvh) * dim;
+        } else {
+            const int kb = min(k0 + BLOCK * wave, last_key / BLOCK * BLOCK), page = kb / a.page;
+            src = kc + (((int64_t)table[page] * a.page + (min(kb + row, last_key) - page * a.page)) * a.G + kvh) * dim;
+        }
+#pragma unroll
+        for (int j = 0; j < NKS; ++j) k[j] = *reinterpret_cast<const f32x4*>(src + 16 * j + 4 * quarter);
+    };
+    auto fetch_v = [&](int k0) {
+        if (k0 < 0) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                int pi, at;
+                block_place(min(order.block_of(k0) + BLOCK * wave + 4 * quarter + e, nblocks - 1), a.pool, a.page, pi, at);
+                const float* src = (const float*)a.pv + (((int64_t)table[pi] * a.pool_rows + at) * a.G + kvh) * vdim + row;
+#pragma unroll
+                for (int c = 0; c < NVT; ++c) v[c][e] = src[16 * c];
+            }
+        } else {
+            const int kb = min(k0 + BLOCK * wave, last_key / BLOCK * BLOCK), page = kb / a.page;
+            const float* src = vc + (((int64_t)table[page] * a.G + kvh) * vdim + row) * a.page + (kb - page * a.page) + 4 * quarter;
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) v[c] = *reinterpret_cast<const f32x4*>(src + (int64_t)16 * c * a.page);
+        }
+    };
+    int k0 = order.first();
+    if (k0 <= last_key) {                                    // (a sequence without keys has no pages)
+        fetch_k(k0);
+        fetch_v(k0);
+    }
+    {
+        const float* src = (const float*)a.q + (int64_t)(qbase + qtok) * a.ldq + head * dim + 4 * quarter;
+        const float sc = a.scale * query_temperature(qpos, a.temp_coef, a.temp_every);
+#pragma unroll
+        for (int j = 0; j < NKS; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qr[j][e] = src[16 * j + e] * sc;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NVT; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // (a sink is what the row starts from: it has been seen with score sink, weight 1 and no value - by the first wave)
+    const bool sunk = a.sinks && wave == 0;
+    float m_run = sunk ? a.sinks[head] : -INFINITY, l_run = sunk && quarter == 0 ? 1.f : 0.f;     // (a lane sums its own keys' weights)
+    const float slope = a.slopes ? a.slopes[head] : 0.f;
+    const float* bias = a.bias ? a.bias + (int64_t)head * a.bias_len : nullptr;
+    while (k0 <= last_key) {
+        const bool pooled = k0 < 0;                          // (uniform) a tile of block means
+        const int next = order.next(k0), kb = k0 + BLOCK * wave, key0 = kb + 4 * quarter, block0 = pooled ? order.block_of(k0) + BLOCK * wave + 4 * quarter : 0;
+        float biases[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) biases[e] = bias[min(max(qpos - (key0 + e), 0), a.bias_len - 1)];
+        }
+        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
+#pragma unroll
+        for (int j = 0; j < NKS; ++j) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (j & 1) s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j][e], qr[j][e], s1, 0, 0, 0);
+                else s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[j][e], qr[j][e], s0, 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_k(next);                                       // (past the end: a block that was read before)
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 s = s0 + s1;
+        bool ok[4];
+        float top = m_run;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (a.softcap > 0.f) s[e] = a.softcap * tanhf(s[e] / a.softcap);
+            ok[e] = pooled ? block0 + e < my_blocks : key_visible(key0 + e, qpos, a.window, a.keep_first, a.chunk);
+            s[e] = ok[e] ? s[e] - slope * (float)(qpos - (key0 + e)) + biases[e] : -INFINITY;
+            top = fmaxf(top, s[e]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        // (a row that sees nothing yet keeps m = -inf)
+        const float alpha = top == -INFINITY ? 1.f : expf(m_run - top);
+        f32x4 p;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) p[e] = ok[e] ? expf(s[e] - top) : 0.f;
+        l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+        m_run = top;
+        if (!pooled && kb + BLOCK - 1 > last_key) {          // what the page holds past the last key may be anything
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[c][e] = key0 + e <= last_key ? v[c][e] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NVT; ++c) acc[c] *= alpha;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int c = 0; c < NVT; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c][e], p[e], acc[c], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_v(next);
+        __builtin_amdgcn_sched_barrier(0);
+        k0 = next;
+    }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    float* ml = smem + 4 * 16 * OLD;                         // [4][16][2]
+    {
+        float* out = smem + (wave * 16 + row) * OLD + 4 * quarter;
+#pragma unroll
+        for (int c = 0; c < NVT; ++c) *reinterpret_cast<f32x4*>(out + 16 * c) = acc[c];
+        if (quarter == 0) {
+            ml[(wave * 16 + row) * 2] = m_run;
+            ml[(wave * 16 + row) * 2 + 1] = l_run;
+        }
+    }
+    __syncthreads();
+    // epilogue, 16 lanes a row: merge the waves, normalise, turn back by the query's position, gate
+    const int qi = tid >> 4, sub = tid & 15;
+    float weight[4], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = fmaxf(m, ml[(w * 16 + qi) * 2]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float mw = ml[(w * 16 + qi) * 2];
+        weight[w] = mw == -INFINITY ? 0.f : expf(mw - m);
+        l += weight[w] * ml[(w * 16 + qi) * 2 + 1];
+    }
+    float* os = smem + qi * OLD;                             // (the first wave's rows: every lane replaces the elements that it has read)
+#pragma unroll
+    for (int c = 0; c < NVT; ++c) {
+        const int col = sub + 16 * c;
+        float o = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) o += weight[w] * smem[(w * 16 + qi) * OLD + col];
+        os[col] = l > 0.f ? o / l : 0.f;
+    }
+    __syncthreads();
+    if (qi < nq) {
+        const int64_t tok = qbase + (grouped ? 0 : q0 + qi);
+        const int h = grouped ? head0 + qi : head0;
+        const float g = a.gate ? a.gate[tok * a.H + h] : 1.0f, pos = (float)(past + (grouped ? 0 : q0 + qi));
+#pragma unroll
+        for (int c = 0; c < NVT; ++c) {
+            const int col = sub + 16 * c;
+            float x = os[col];
+            if (a.v_freq) {
+                int partner, pair;
+                bool first;
+                pair_of(col, vdim, a.v_interleaved, partner, pair, first);
+                float sn, cs;
+                rot_sincos<float>(pos * a.v_freq[pair], sn, cs);
+                x = first ? x * cs + os[partner] * sn : x * cs - os[partner] * sn;      // the rotation by -pos
+            }
+            if (a.gate_elems) x *= elem_gate<float>(((const float*)a.gate_elems)[tok * a.ld_elems + h * vdim + col]);
+            ((float*)a.out)[(tok * a.H + h) * vdim + col] = x * g;
+        }
+    }
+}
+
+template <int NKS, int NVT>
+static void launch_attn_f32(const AttnArgs& a, int64_t total_q, hipStream_t st) {
+    const size_t lds = sizeof(float) * (size_t)(4 * 16 * (16 * NVT + 4) + 4 * 16 * 2);
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_paged_f32_kernel<NKS, NVT>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    const bool grouped = !a.cu_seqlens_q;
+    const dim3 grid(grouped ? (unsigned)a.batch : (unsigned)(total_q / AQ + a.batch), (unsigned)(grouped ? a.G * ((a.H / a.G + 15) / 16) : a.H));
+    attn_paged_f32_kernel<NKS, NVT><<<grid, 256, lds, st>>>(a, grouped);
+}
+
+// Head sizes (dim / 16, vdim / 16) that the fp32 matrix-core form is built for; false: another one.
+static bool dispatch_attn_f32(const AttnArgs& a, int64_t total_q, hipStream_t st) {
+    if (a.dim % 16 || a.vdim % 16) return false;
+#define NVH_ATTN_F32(K, V)                       \
+    if (a.dim == 16 * K && a.vdim == 16 * V) {   \
+        launch_attn_f32<K, V>(a, total_q, st);   \
+        return true;                             \
+    }
+    NVH_ATTN_F32(1, 1) NVH_ATTN_F32(2, 2) NVH_ATTN_F32(4, 4) NVH_ATTN_F32(6, 6) NVH_ATTN_F32(8, 8) NVH_ATTN_F32(4, 8) NVH_ATTN_F32(8, 4) NVH_ATTN_F32(16, 12) NVH_ATTN_F32(16, 16)
+#undef NVH_ATTN_F32
+    return false;
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // The same attention on the matrix cores, for bf16 caches with dim and vdim multiples of 16.  A workgroup is 64
 // consecutive queries of one (sequence, head): four waves of 16 queries, all walking the same 64-key tiles (K rows and
 // V transposed in LDS).  Per tile a wave forms S^T = K Q^T (lane: query lane%16, keys 4 (lane/16) + r of each 16-key
@@ -1220,6 +1458,8 @@ extern "C" int32_t nvh_attn_paged_any(const void* q, int64_t q_row_stride, const
         if (bias) dispatch_attn_mfma<VAR_BIAS>(a, total_q, st);
         else if (pool > 0 || softcap > 0.f || temp_every > 0) dispatch_attn_mfma<VAR_EXT>(a, total_q, st);
         else dispatch_attn_mfma<VAR_PLAIN>(a, total_q, st);
+    } else if (act_f32 && page % 16 == 0 && nvh_aligned16(k_cache) && nvh_aligned16(v_cache) && (pool == 0 || nvh_aligned16(pooled_k)) &&
+               !nvh_switch_on(SW_ATTN_ANY_NO_MFMA) && dispatch_attn_f32(a, total_q, st)) {      // (launched)
     } else if (vdim <= 256) {                                // (16 value columns a lane; the choice depends on the size alone)
         if (act_f32) attn_paged_any_kernel<float, 16><<<grid, 256, lds, st>>>(a);
         else attn_paged_any_kernel<bf16, 16><<<grid, 256, lds, st>>>(a);
