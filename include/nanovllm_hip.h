@@ -702,6 +702,15 @@ int32_t nvh_gated_linear_scan(const float* q, int64_t q_stride, const float* k, 
                               const int32_t* context_lens, float* out, int64_t batch, int64_t heads, int64_t dk, int64_t dv,
                               int64_t segments, int64_t segment_min_tokens, float* ws_states, float* ws_decays, int32_t read_first,
                               const float* bonus, nvh_stream_t stream);
+/* nvh_gated_linear_scan whose portions of at least min_tokens tokens go through chunks of 16 tokens (the others as without segments): results within
+ * rounding of the token-by-token ones.  num_tokens = cu_seqlens_q[batch]; cu_seqlens_q is required; q, k, w [T, H, dk], state and workspace are 16-byte
+ * aligned, their strides multiples of four; workspace: nvh_scan_chunk_workspace_bytes (0: these head sizes have no chunked form). */
+int64_t nvh_scan_chunk_workspace_bytes(int64_t num_tokens, int64_t batch, int64_t heads, int64_t dk, int64_t dv);
+int32_t nvh_gated_linear_scan_chunked(const float* q, int64_t q_stride, const float* k, int64_t k_stride, int64_t qk_groups, const float* w,
+                                      int64_t w_stride, int32_t w_scalar, const float* kscale, int64_t kscale_stride, const float* v,
+                                      int64_t v_stride, const float* skip, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                      const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens, int64_t heads, int64_t dk,
+                                      int64_t dv, int64_t min_tokens, float* workspace, int32_t read_first, const float* bonus, nvh_stream_t stream);
 /* Whether key size dk has the segmented form of the scan. */
 int32_t nvh_scan_segmentable(int64_t dk);
 int32_t nvh_hgrn2_prep(const void* q, int64_t q_stride, const void* f, int64_t f_stride, const void* v, int64_t v_stride,

@@ -21,6 +21,7 @@
 //                    g = exp(-exp(A_log) softplus(a + dt_bias)), all in fp32, and leaves the scan's rows; q and k heads
 //                    may be shared by groups of value heads, and the value size is free.
 #include "common.h"
+#include "scan_chunk.h"
 
 namespace {
 
@@ -321,10 +322,6 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
 // us at one sequence of 1024 tokens, token by token and in chunks (both launches): 16 heads of 64 x 64: 271, 27 + 47; 8 heads of 128 x 128: 331,
 // 28 + 75.  The first launch is bound by its chain when the chip is not full (11 us at 256 tokens), and else by the double products (172 us at 8448
 // records of 64 x 64); the second by the chain of a chunk, 0.74 us.
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-constexpr int CT = 16;                                       // tokens of a chunk
-constexpr int MLD = CT + 1;                                  // doubles a row of a 16 x 16 matrix takes in LDS (its columns then lie in different banks)
-
 // What the first launch keeps in LDS: r | k | w | u | au, 16 rows of dk + 4 floats each, and in doubles the decays and their reciprocals (16 rows of
 // dk + 2 each), which later give their place to four matrices.
 __host__ __device__ constexpr int chunk_rows_floats(int dk) { return 5 * CT * (dk + 4); }
@@ -338,59 +335,10 @@ struct DeltaChunkArgs {
 
 // Floats of a record: W | Q | A'^T | K'^T (16 dk each, as the lanes of the second launch read them) | P (dk) | Y | Z | V (16 dv each, likewise).
 __host__ __device__ __forceinline__ int64_t chunk_record(int dk, int dv) { return 65 * (int64_t)dk + 48 * (int64_t)dv; }
-// First chunk slot of a sequence whose tokens start at row `lo`: sequences never overlap, and all fit num_tokens / 16 + batch slots.
-__device__ __forceinline__ int chunk_base(int lo, int seq) { return lo / CT + seq; }
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double x) {
-    const u32x2 v = __builtin_bit_cast(u32x2, x);
-    const u32x2 r = {(uint32_t)__builtin_amdgcn_mov_dpp((int)v[0], CTRL, 0xf, 0xf, true), (uint32_t)__builtin_amdgcn_mov_dpp((int)v[1], CTRL, 0xf, 0xf, true)};
-    return __builtin_bit_cast(double, r);
-}
-// The sums of four values over the 16 lanes of a row; lane g is left with that of value g & 3.
-__device__ __forceinline__ double row16_sum4(double v0, double v1, double v2, double v3, int g) {
-    const bool odd = g & 1, high = g & 2;
-    const double lo = (odd ? v1 : v0) + dpp_f64<0xB1>(odd ? v0 : v1), hi = (odd ? v3 : v2) + dpp_f64<0xB1>(odd ? v2 : v3);     // neighbours
-    double x = (high ? hi : lo) + dpp_f64<0x4E>(high ? lo : hi);         // pairs
-    x += dpp_f64<0x124>(x);                                              // rotations by 4 and 8 within the row
-    return x + dpp_f64<0x128>(x);
-}
-
-// Lower triangular 16 x 16 matrices in double on the matrix cores.  Index i of an operand or of a result's column (lane & 15) stands for token
-// chunk_tok(i): element e of a lane in quarter q of the wave is then token 4 q + e, in a result's rows as in the contraction's steps.  So a result is
-// the next product's right operand as it stands, and its transpose's left operand; what is needed as a left operand is carried transposed too.
-__device__ __forceinline__ int chunk_tok(int i) { return 4 * (i & 3) + (i >> 2); }
-
 struct Tri {
     f64x4 n, t;                // X and its transpose
 };
 
-__device__ __forceinline__ f64x4 mfma_f64(const f64x4& l, const f64x4& r, f64x4 c) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f64_16x16x4f64(l[e], r[e], c, 0, 0, 0);
-    return c;
-}
-// c + l r where only l's tokens up to a result's own row (T: column) enter, and nothing above the diagonal: what is not finite in a token then
-// leaves the tokens before it alone.  W: r's columns are channels and not tokens.
-template <bool T, bool W>
-__device__ __forceinline__ f64x4 mfma_f64_below(const f64x4& l, const f64x4& r, const f64x4& c, int q, int own) {
-    f64x4 res = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
-    for (int t = 0; t < CT; ++t) {
-        f64x4 lm, rm;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const bool in = 4 * q + e <= t;
-            lm[e] = in ? l[e] : 0.0;
-            rm[e] = in ? r[e] : 0.0;
-        }
-        const f64x4 x = mfma_f64(lm, rm, c);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (T ? own == t && (W || 4 * q + e <= t) : 4 * q + e == t && (W || own <= t)) res[e] = x[e];
-    }
-    return res;
-}
 template <bool SAFE>
 __device__ __forceinline__ f64x4 tri_mul_n(const f64x4& l, const f64x4& r, const f64x4& c, int q, int own) {      // l: the left matrix transposed
     if constexpr (SAFE) return mfma_f64_below<false, false>(l, r, c, q, own);

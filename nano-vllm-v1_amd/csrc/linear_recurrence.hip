@@ -15,6 +15,7 @@
 // Everything that enters the recurrence is fp32; A (bf16 or fp32) is the type of projections, weights and results.
 #include <algorithm>
 #include "common.h"
+#include "scan_chunk.h"
 
 namespace {
 
@@ -398,6 +399,7 @@ struct ScanArgs {
     int nseg, seg_min;         // segments per long portion (1: none) and the fewest tokens that are cut
     float *ws_l, *ws_d;        // records of the segments: end states [batch, H, nseg, dv, dk] and decay products [batch, H, nseg, dk]
     const float* bonus;        // PRE only: [H, dk] or null (0)
+    int skip_from;             // > 0, MODE 0: portions of at least this many tokens are left to the chunked form
 };
 
 // Lanes per state column (SUBS), rows held per lane (DKQ), EXACT: dk == DKQ * SUBS (no loop carries a run-time bound; rows
@@ -430,6 +432,7 @@ __global__ __launch_bounds__(256) void gated_linear_scan_kernel(ScanArgs p) {
     const int seq_lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : seq, seq_hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : seq + 1;
     const int slot = p.slots[seq];
     if (slot < 0 || seq_hi <= seq_lo) return;                // a padded row (uniform over the workgroup)
+    if (MODE == 0 && p.skip_from > 0 && seq_hi - seq_lo >= p.skip_from) return;
     const int nseg = (MODE != 0 && seq_hi - seq_lo >= p.seg_min) ? p.nseg : 1;
     if (seg >= nseg || (MODE == 2 && seg == 0)) return;      // (uniform)
     const int seg_len = (seq_hi - seq_lo + nseg - 1) / nseg;
@@ -617,6 +620,278 @@ __global__ __launch_bounds__(256) void gated_linear_scan_kernel(ScanArgs p) {
         for (int ii = 0; ii < DKQ; ++ii)
             if (row_ok(ii)) sp[(int64_t)col * dk + row_of(ii)] = S[ii];
     }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// The chunked form, for portions of many tokens.  Within a chunk of 16 tokens, with P_t the product of the decays of tokens 0 .. t,
+//   o_t = (P_t q_t) S0 + sum_(s<=t) N_ts v_s,   N_ts = q_t . (w_(s+1) .. w_t c_s k_s)  (+ skip on the diagonal),
+//   S = P_15 S0 + K'^T V,                       K'_s = w_(s+1) .. w_15 c_s k_s
+// (PRE: P_(t-1) for P_t, and on the diagonal the bonus).  One launch forms P_t q_t, N V and K' for all chunks at once, the second walks the chunks.
+// N and the sums over a chunk are held in double, as in the delta rule's chunked form (against float64, in the 2-norm over 1024 tokens of slow decay:
+// outputs 1.1e-7, states 7.3e-8; token by token 1.9e-7 and 1.8e-7).
+// A prompt of 1024 tokens, in segments and in chunks, us: 16 heads of 64 x 64 72 and 51; 4 heads of 128 x 256 108 and 71; three prompts of 1008
+// tokens together 81 and 39, 160 and 49; 128 tokens, token by token and in chunks: 29 and 14, 41 and 20.  The first launch is bound by its loads and
+// its chain where the chip is not full, the second by the records' way through L2 (0.6 us a chunk).
+struct ScanChunkArgs {
+    ScanArgs s;
+    float* ws;                 // a record per (chunk slot, head): P q | K' (16 dk each) | P_15 (dk) | N V (16 dv), as the second launch's lanes read them
+    int batch;
+};
+__host__ __device__ __forceinline__ int64_t scan_chunk_record(int dk, int dv) { return 33 * (int64_t)dk + 16 * (int64_t)dv; }
+__host__ __device__ constexpr int scan_chunk_rows(int dk) { return 3 * CT * (dk + 4); }
+__host__ __device__ constexpr int scan_chunk_doubles(int dk) { return (2 * CT * (dk + 2) > 4 * CT * MLD ? 2 * CT * (dk + 2) : 4 * CT * MLD) + CT; }
+
+// CPL: key channels of a lane where 16 lanes share a token (dk = 16 CPL).
+template <int CPL, bool PRE>
+__global__ __launch_bounds__(256) void scan_chunk_prep_kernel(ScanChunkArgs a) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];       // q | k | w, 16 rows of dk + 4 each; decays and reciprocals in double, then N's parts
+    const ScanArgs& p = a.s;
+    constexpr int dk = 16 * CPL, LD = dk + 4, DLD = dk + 2;
+    const int dv = p.dv, head = blockIdx.x, cslot = blockIdx.y, tid = threadIdx.x;
+    int first = 0, end = a.batch;                            // the last sequence whose chunk slots begin at or before this one
+    while (end - first > 1) {
+        const int mid = (first + end) >> 1;
+        if (chunk_base(p.cu_seqlens_q[mid], mid) <= cslot) first = mid;
+        else end = mid;
+    }
+    const int lo = p.cu_seqlens_q[first], hi = p.cu_seqlens_q[first + 1];
+    const int t0 = lo + CT * (cslot - chunk_base(lo, first)), nt = min(CT, hi - t0);
+    if (hi - lo < p.skip_from || nt <= 0 || p.slots[first] < 0) return;      // (uniform)
+    const int group = head / (p.H / p.qk_groups);
+    float* rec = a.ws + ((int64_t)cslot * p.H + head) * scan_chunk_record(dk, dv);
+    auto row = [&](int which, int t) { return sm + (which * CT + t) * LD; };
+    double *mats = reinterpret_cast<double*>(sm + scan_chunk_rows(dk)), *cums = mats, *rcums = mats + CT * DLD, *diag = mats + scan_chunk_doubles(dk) - CT;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, q = lane >> 4, vtiles = dv >> 4;
+    const int s = tid >> 4, g = tid & 15, ch = g * CPL, own = chunk_tok(col);
+    // Tokens beyond the portion's end change nothing: decay 1, everything else 0.
+    {
+        constexpr int PIECES = CT * dk / 4, ROUNDS = (PIECES + 255) / 256;
+        f32x4 xq[ROUNDS], xk[ROUNDS], xw[ROUNDS];
+        float xc[ROUNDS];
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int e = min(tid + 256 * i, PIECES - 1), t = e / (dk / 4), c4 = (e - t * (dk / 4)) * 4;
+            const int64_t tok = t0 + min(t, nt - 1);
+            xq[i] = *reinterpret_cast<const f32x4*>(p.q + tok * p.q_stride + group * dk + c4);
+            xk[i] = *reinterpret_cast<const f32x4*>(p.k + tok * p.k_stride + group * dk + c4);
+            if (p.w_scalar) {
+                const float w = p.w[tok * p.w_stride + head];
+                xw[i] = f32x4{w, w, w, w};
+            } else {
+                xw[i] = *reinterpret_cast<const f32x4*>(p.w + tok * p.w_stride + (int64_t)head * dk + c4);
+            }
+            xc[i] = p.kscale ? p.kscale[tok * p.ks_stride + head] : 1.f;
+        }
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) {
+            const int e = tid + 256 * i, t = e / (dk / 4), c4 = (e - t * (dk / 4)) * 4;
+            if (PIECES % 256 == 0 || e < PIECES) {
+                const bool in = t < nt;
+                *reinterpret_cast<f32x4*>(row(0, t) + c4) = in ? xq[i] : f32x4{0.f, 0.f, 0.f, 0.f};
+                *reinterpret_cast<f32x4*>(row(1, t) + c4) = in ? xk[i] * xc[i] : f32x4{0.f, 0.f, 0.f, 0.f};
+                *reinterpret_cast<f32x4*>(row(2, t) + c4) = in ? xw[i] : f32x4{1.f, 1.f, 1.f, 1.f};
+            }
+        }
+    }
+    __syncthreads();
+    double cum[CPL], before[CPL], own_sum = 0.0;             // the decay up to token s, with and without its own; q (bonus) k of the token itself
+    bool far = false;
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) before[i] = 1.0;
+#pragma unroll 4
+    for (int t = 0; t < CT - 1; ++t) {
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) {
+            const double w = row(2, t)[ch + i];
+            before[i] *= t < s ? w : 1.0;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {
+        cum[i] = before[i] * row(2, s)[ch + i];
+        far |= !(cum[i] >= 1e-80 && cum[i] <= 1e80);
+        cums[s * DLD + ch + i] = cum[i];
+        rcums[s * DLD + ch + i] = 1.0 / cum[i];
+        if (PRE) own_sum = __builtin_fma((double)row(0, s)[ch + i] * (p.bonus ? p.bonus[(int64_t)head * dk + ch + i] : 0.f), (double)row(1, s)[ch + i], own_sum);
+    }
+    if (PRE) {
+        own_sum = row16_sum4(own_sum, 0.0, 0.0, 0.0, g);
+        if (g == 0) diag[s] = own_sum;
+    }
+    far = __syncthreads_or(far);
+    float kp[CPL];                                           // k of token s, decayed to the chunk's end
+    if (!far) {
+        // N = (P q) (k / P)^T, a quarter of the channels a wave; in double, where the quotients neither over- nor underflow within the limits above
+        constexpr int PER = dk / 4;
+        const int c0 = wave * PER + q * (PER / 4);
+        const float *lrow = row(0, own) + c0, *rrow = row(1, own) + c0;
+        const double *lcum = cums + (PRE ? max(own - 1, 0) : own) * DLD + c0, *rcum = rcums + own * DLD + c0;
+        const bool one = PRE && own == 0;
+        f64x4 n = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < PER / 4; ++j) n = __builtin_amdgcn_mfma_f64_16x16x4f64(lrow[j] * (one ? 1.0 : lcum[j]), rrow[j] * rcum[j], n, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) kp[i] = (float)(row(1, s)[ch + i] * (cums[(CT - 1) * DLD + ch + i] * rcums[s * DLD + ch + i]));
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mats[(wave * CT + 4 * q + e) * MLD + own] = n[e];
+    } else {                                                 // decays as products of those in between, 16 lanes walk token s to the chunk's end
+        double xk[CPL];
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) xk[i] = 0.0;
+#pragma unroll 1
+        for (int t = 0; t < CT; ++t) {
+            double d = 0.0;
+#pragma unroll
+            for (int i = 0; i < CPL; ++i) {
+                if (PRE) d = __builtin_fma((double)row(0, t)[ch + i], xk[i], d);
+                xk[i] = t == s ? row(1, t)[ch + i] : xk[i] * row(2, t)[ch + i];
+                if (!PRE) d = __builtin_fma((double)row(0, t)[ch + i], xk[i], d);
+            }
+            d = row16_sum4(d, 0.0, 0.0, 0.0, g);
+            if (g < 4) mats[(g * CT + t) * MLD + s] = g == 0 ? d : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < CPL; ++i) kp[i] = (float)xk[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < CPL; ++i) {                          // K' and P q in place
+        row(1, s)[ch + i] = kp[i];
+        row(0, s)[ch + i] = (float)(row(0, s)[ch + i] * (PRE ? before[i] : cum[i]));
+        if (s == CT - 1) rec[32 * dk + ch + i] = (float)cum[i];
+    }
+    f64x4 N;                                                 // (as a left operand: lane's token own, columns 4 q + e)
+    const double skip = p.skip ? p.skip[head] : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = 4 * q + e;
+        const double* at = mats + own * MLD + t;
+        const double n = (at[0] + at[CT * MLD]) + (at[2 * CT * MLD] + at[3 * CT * MLD]);
+        N[e] = t < own ? n : t > own ? 0.0 : skip + (PRE ? diag[own] : n);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (CPL + 3) / 4; ++i) {
+        const int tile = wave + 4 * i;
+        if (CPL % 4 && tile >= CPL) break;
+        const int c0 = 16 * tile;
+        float* at = rec + (tile * 64 + lane) * 4;
+        *reinterpret_cast<f32x4*>(at) = *reinterpret_cast<const f32x4*>(row(0, col) + c0 + 4 * q);
+        f32x4 K;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) K[e] = row(1, 4 * q + e)[c0 + own];
+        *reinterpret_cast<f32x4*>(at + 16 * dk) = K;
+    }
+    for (int tile = wave; tile < vtiles; tile += 4) {        // 16 columns of v
+        const float* vp = p.v + (int64_t)head * dv + 16 * tile + col;
+        f64x4 x;
+        bool vodd = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float v = vp[(int64_t)(t0 + min(4 * q + e, nt - 1)) * p.v_stride];
+            x[e] = 4 * q + e < nt ? v : 0.f;
+            vodd |= !(fabsf(v) <= 3.402823466e+38f);
+        }
+        const f64x4 zero = {0.0, 0.0, 0.0, 0.0};
+        const f64x4 Z = __any(vodd) ? mfma_f64_below<false, true>(N, x, zero, q, own) : mfma_f64(N, x, zero);
+        *reinterpret_cast<f32x4*>(rec + 33 * dk + (tile * 64 + lane) * 4) = f32x4{(float)Z[0], (float)Z[1], (float)Z[2], (float)Z[3]};
+    }
+}
+
+// NW waves of 16 key channels each hold 16 columns of a head's state, row 4 q + e of lane (q, column) in element e, as a product leaves its result and
+// takes its right operand.  One wave more sums the waves' parts of the outputs, a chunk behind, and writes them.
+template <int NW>
+__global__ __launch_bounds__(64 * NW + 64) void scan_chunk_walk_kernel(ScanChunkArgs a) {
+    __shared__ f32x4 meet[2][NW][64];                        // [chunk parity][wave][lane]
+    const ScanArgs& p = a.s;
+    constexpr int dk = 16 * NW;
+    const int seq = blockIdx.x, head = blockIdx.y, dv = p.dv, cb = blockIdx.z;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int lo = p.cu_seqlens_q[seq], hi = p.cu_seqlens_q[seq + 1], slot = p.slots[seq];
+    if (slot < 0 || hi <= lo || hi - lo < p.skip_from) return;       // (uniform)
+    const int64_t record = scan_chunk_record(dk, dv), step = (int64_t)p.H * record;
+    const float* rec = a.ws + ((int64_t)chunk_base(lo, seq) * p.H + head) * record;
+    const int chunks = (hi - lo + CT - 1) / CT;
+    if (wave == NW) {                                        // the outputs: the parts of chunk j are written after the barrier of chunk j
+        float* out = p.out + (int64_t)lo * p.H * dv + head * dv + 16 * cb + col;
+        const float* zp = rec + 33 * dk + (cb * 64 + lane) * 4;
+        f32x4 z = *reinterpret_cast<const f32x4*>(zp);
+        for (int j = 0; j < chunks; ++j) {
+            const f32x4 after = *reinterpret_cast<const f32x4*>(zp + min(j + 1, chunks - 1) * step);
+            __syncthreads();
+            f32x4 res = meet[j & 1][0][lane];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) res += meet[j & 1][w][lane];
+            res += z;
+            z = after;
+            const int t = CT * j + 4 * q;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (lo + t + e < hi) out[(int64_t)(t + e) * p.H * dv] = res[e];
+        }
+        return;
+    }
+    float* sp = p.state + (((int64_t)slot * p.H + head) * dv + 16 * cb + col) * dk + 16 * wave + 4 * q;
+    f32x4 S = {0.f, 0.f, 0.f, 0.f};
+    if (p.context_lens[seq] != hi - lo) S = *reinterpret_cast<const f32x4*>(sp);
+    struct Operands {
+        f32x4 Q, K, P;
+        float v[4];
+    };
+    const float* vp = p.v + (int64_t)head * dv + 16 * cb + col;
+    auto fetch = [&](int j, Operands& x) {
+        j = min(j, chunks - 1);
+        const float* r = rec + j * step;
+        x.Q = *reinterpret_cast<const f32x4*>(r + (wave * 64 + lane) * 4);
+        x.K = *reinterpret_cast<const f32x4*>(r + 16 * dk + (wave * 64 + lane) * 4);
+        x.P = *reinterpret_cast<const f32x4*>(r + 32 * dk + 16 * wave + 4 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.v[e] = vp[(int64_t)min(lo + CT * j + 4 * q + e, hi - 1) * p.v_stride];      // (K' is zero past the end)
+    };
+    auto chunk = [&](int j, const Operands& x) {
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[e], S[e], o, 0, 0, 0);
+        f64x4 kv = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)x.v[e], kv, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = __builtin_fmaf(x.P[e], S[e], (float)kv[e]);
+        meet[j & 1][wave][lane] = o;
+        __syncthreads();                                     // (of the other parity: the outputs' wave has left it before it came here)
+    };
+    constexpr int AHEAD = 4;                                 // records in flight
+    Operands x[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) fetch(i, x[i]);
+    int j = 0;
+    for (; j + AHEAD <= chunks; j += AHEAD) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            chunk(j + i, x[i]);
+            fetch(j + i + AHEAD, x[i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD - 1; ++i)
+        if (j + i < chunks) chunk(j + i, x[i]);
+    *reinterpret_cast<f32x4*>(sp) = S;
+}
+
+template <int CPL>
+void launch_scan_chunks(const ScanChunkArgs& a, int64_t cslots, int64_t batch, int read_first, hipStream_t st) {
+    const size_t lds = sizeof(float) * (size_t)scan_chunk_rows(16 * CPL) + sizeof(double) * (size_t)scan_chunk_doubles(16 * CPL);
+    const dim3 grid((unsigned)a.s.H, (unsigned)cslots);
+    if (read_first) scan_chunk_prep_kernel<CPL, true><<<grid, 256, lds, st>>>(a);
+    else scan_chunk_prep_kernel<CPL, false><<<grid, 256, lds, st>>>(a);
+    scan_chunk_walk_kernel<CPL><<<dim3((unsigned)batch, (unsigned)a.s.H, (unsigned)(a.s.dv / 16)), 64 * CPL + 64, 0, st>>>(a);
+}
+
+// Head sizes that the chunked form is built for: whole 16-wide tiles, at most eight waves of key channels.
+bool scan_chunkable(int64_t dk, int64_t dv) {
+    return dv % 16 == 0 && dv <= 16 * 65535 && (dk == 16 || dk == 32 || dk == 48 || dk == 64 || dk == 96 || dk == 128);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -877,25 +1152,8 @@ extern "C" int32_t nvh_scan_segmentable(int64_t dk) {
     return dk % 16 == 0 && (dk / 16 <= 4 || dk / 16 == 6 || dk / 16 == 8 || dk / 16 == 16);
 }
 
-extern "C" int32_t nvh_gated_linear_scan(const float* q, int64_t q_stride, const float* k, int64_t k_stride, int64_t qk_groups, const float* w,
-                                         int64_t w_stride, int32_t w_scalar, const float* kscale, int64_t kscale_stride, const float* v,
-                                         int64_t v_stride, const float* skip, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
-                                         const int32_t* context_lens, float* out, int64_t batch, int64_t heads, int64_t dk, int64_t dv,
-                                         int64_t segments, int64_t segment_min_tokens, float* ws_states, float* ws_decays, int32_t read_first,
-                                         const float* bonus, nvh_stream_t stream) {
-    NVH_REQUIRE(q && k && w && v && state && slots && context_lens && out, NVH_EINVAL, "nvh_gated_linear_scan: null pointer");
-    NVH_REQUIRE(batch >= 0 && heads > 0 && dk > 0 && dv > 0 && qk_groups > 0 && heads % qk_groups == 0, NVH_EINVAL, "nvh_gated_linear_scan: bad sizes");
-    NVH_REQUIRE(dk <= 512, NVH_ENOSYS, "nvh_gated_linear_scan: key size %ld above 512", (long)dk);
-    if (batch == 0) return NVH_OK;
-    ScanArgs p{q, k, q_stride, k_stride, (int)qk_groups, w, w_stride, w_scalar, kscale, kscale_stride, v, v_stride, skip, state, slots,
-                     cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1, 1 << 30, ws_states, ws_decays, bonus};
-    NVH_REQUIRE(read_first || !bonus, NVH_EINVAL, "nvh_gated_linear_scan: a bonus needs read_first");
-    if (segments > 1 && nvh_scan_segmentable(dk)) {
-        NVH_REQUIRE(segments <= 64 && segment_min_tokens >= 2 * segments && ws_states && ws_decays && cu_seqlens_q, NVH_EINVAL, "nvh_gated_linear_scan: bad segments");
-        p.nseg = (int)segments;
-        p.seg_min = (int)segment_min_tokens;
-    }
-    hipStream_t st = (hipStream_t)stream;
+static void launch_scan(const ScanArgs& p, int64_t batch, int read_first, hipStream_t st) {
+    const int dk = p.dk;
     // (the choice depends on dk alone, so a sequence sees one summation order whatever the batch or the cut)
     if (dk % 16 == 0) {
         switch (dk / 16) {
@@ -912,14 +1170,77 @@ extern "C" int32_t nvh_gated_linear_scan(const float* q, int64_t q_stride, const
                 else launch_scan_as<32, 16, false>(p, batch, read_first, st);
         }
     } else {
-        const int dkq = (int)(dk + 3) / 4;
+        const int dkq = (dk + 3) / 4;
         if (dkq <= 8) launch_scan_as<8, 4, false>(p, batch, read_first, st);
         else if (dkq <= 16) launch_scan_as<16, 4, false>(p, batch, read_first, st);
         else if (dkq <= 32) launch_scan_as<32, 4, false>(p, batch, read_first, st);
         else if (dkq <= 64) launch_scan_as<64, 4, false>(p, batch, read_first, st);
         else launch_scan_as<32, 16, false>(p, batch, read_first, st);
     }
+}
+
+extern "C" int32_t nvh_gated_linear_scan(const float* q, int64_t q_stride, const float* k, int64_t k_stride, int64_t qk_groups, const float* w,
+                                         int64_t w_stride, int32_t w_scalar, const float* kscale, int64_t kscale_stride, const float* v,
+                                         int64_t v_stride, const float* skip, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                         const int32_t* context_lens, float* out, int64_t batch, int64_t heads, int64_t dk, int64_t dv,
+                                         int64_t segments, int64_t segment_min_tokens, float* ws_states, float* ws_decays, int32_t read_first,
+                                         const float* bonus, nvh_stream_t stream) {
+    NVH_REQUIRE(q && k && w && v && state && slots && context_lens && out, NVH_EINVAL, "nvh_gated_linear_scan: null pointer");
+    NVH_REQUIRE(batch >= 0 && heads > 0 && dk > 0 && dv > 0 && qk_groups > 0 && heads % qk_groups == 0, NVH_EINVAL, "nvh_gated_linear_scan: bad sizes");
+    NVH_REQUIRE(dk <= 512, NVH_ENOSYS, "nvh_gated_linear_scan: key size %ld above 512", (long)dk);
+    if (batch == 0) return NVH_OK;
+    ScanArgs p{q, k, q_stride, k_stride, (int)qk_groups, w, w_stride, w_scalar, kscale, kscale_stride, v, v_stride, skip, state, slots,
+                     cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1, 1 << 30, ws_states, ws_decays, bonus, 0};
+    NVH_REQUIRE(read_first || !bonus, NVH_EINVAL, "nvh_gated_linear_scan: a bonus needs read_first");
+    if (segments > 1 && nvh_scan_segmentable(dk)) {
+        NVH_REQUIRE(segments <= 64 && segment_min_tokens >= 2 * segments && ws_states && ws_decays && cu_seqlens_q, NVH_EINVAL, "nvh_gated_linear_scan: bad segments");
+        p.nseg = (int)segments;
+        p.seg_min = (int)segment_min_tokens;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    launch_scan(p, batch, read_first, st);
     NVH_CHECK_LAUNCH("nvh_gated_linear_scan");
+    return NVH_OK;
+}
+
+extern "C" int64_t nvh_scan_chunk_workspace_bytes(int64_t num_tokens, int64_t batch, int64_t heads, int64_t dk, int64_t dv) {
+    if (!scan_chunkable(dk, dv) || num_tokens < 0 || batch < 0 || heads <= 0 || heads > 65535 || num_tokens / CT + batch > 65535) return 0;
+    return (num_tokens / CT + batch) * heads * scan_chunk_record((int)dk, (int)dv) * (int64_t)sizeof(float);
+}
+
+extern "C" int32_t nvh_gated_linear_scan_chunked(const float* q, int64_t q_stride, const float* k, int64_t k_stride, int64_t qk_groups, const float* w,
+                                                 int64_t w_stride, int32_t w_scalar, const float* kscale, int64_t kscale_stride, const float* v,
+                                                 int64_t v_stride, const float* skip, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                                 const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens, int64_t heads, int64_t dk,
+                                                 int64_t dv, int64_t min_tokens, float* workspace, int32_t read_first, const float* bonus,
+                                                 nvh_stream_t stream) {
+    NVH_REQUIRE(q && k && w && v && state && slots && cu_seqlens_q && context_lens && out && workspace, NVH_EINVAL, "nvh_gated_linear_scan_chunked: null pointer");
+    NVH_REQUIRE(batch >= 0 && num_tokens >= 0 && num_tokens < (1 << 30) && heads > 0 && heads <= 65535 && qk_groups > 0 && heads % qk_groups == 0 &&
+                    num_tokens / CT + batch <= 65535 && min_tokens >= 1 && min_tokens < (1 << 30),
+                NVH_EINVAL, "nvh_gated_linear_scan_chunked: bad sizes");
+    NVH_REQUIRE(scan_chunkable(dk, dv), NVH_ENOSYS, "nvh_gated_linear_scan_chunked: head size %ld x %ld", (long)dk, (long)dv);
+    NVH_REQUIRE(nvh_aligned16(q) && nvh_aligned16(k) && (w_scalar || nvh_aligned16(w)) && nvh_aligned16(state) && nvh_aligned16(workspace) && q_stride % 4 == 0 &&
+                    k_stride % 4 == 0 && (w_scalar || w_stride % 4 == 0),
+                NVH_EINVAL, "nvh_gated_linear_scan_chunked: 16-byte alignment required");
+    NVH_REQUIRE(read_first || !bonus, NVH_EINVAL, "nvh_gated_linear_scan_chunked: a bonus needs read_first");
+    if (batch == 0 || num_tokens == 0) return NVH_OK;
+    const ScanArgs p{q, k, q_stride, k_stride, (int)qk_groups, w, w_stride, w_scalar, kscale, kscale_stride, v, v_stride, skip, state, slots,
+                     cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1, 1 << 30, nullptr, nullptr, bonus, (int)min_tokens};
+    const ScanChunkArgs a{p, workspace, (int)batch};
+    const int64_t cslots = num_tokens / CT + batch;
+    hipStream_t st = (hipStream_t)stream;
+    switch (dk / 16) {
+        case 1: launch_scan_chunks<1>(a, cslots, batch, read_first, st); break;
+        case 2: launch_scan_chunks<2>(a, cslots, batch, read_first, st); break;
+        case 3: launch_scan_chunks<3>(a, cslots, batch, read_first, st); break;
+        case 4: launch_scan_chunks<4>(a, cslots, batch, read_first, st); break;
+        case 6: launch_scan_chunks<6>(a, cslots, batch, read_first, st); break;
+        default: launch_scan_chunks<8>(a, cslots, batch, read_first, st);
+    }
+    NVH_CHECK_LAUNCH("nvh_gated_linear_scan_chunked");
+    if (batch == 1 && num_tokens >= min_tokens) return NVH_OK;
+    launch_scan(p, batch, read_first, st);                   // the portions below min_tokens
+    NVH_CHECK_LAUNCH("nvh_gated_linear_scan_chunked");
     return NVH_OK;
 }
 

@@ -122,6 +122,8 @@ SIGNATURES = {
     "nvh_hyper_norm": (i32, [vp, i64, vp, vp, vp, vp, i64, vp, i64, vp, i64, vp, vp, i64, i32, vp, vp, f32, vp, i64, i64, i64, i32, vp]),
     # linear recurrences with a diagonal decay (csrc/linear_recurrence.hip)
     "nvh_gated_linear_scan": (i32, [vp, i64, vp, i64, i64, vp, i64, i32, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, vp, i32, vp, vp]),
+    "nvh_scan_chunk_workspace_bytes": (i64, [i64, i64, i64, i64, i64]),
+    "nvh_gated_linear_scan_chunked": (i32, [vp, i64, vp, i64, i64, vp, i64, i32, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, i32, vp, vp]),
     "nvh_scan_segmentable": (i32, [i64]),
     "nvh_hgrn2_prep": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, i64, i64, i64, i32, vp]),
     "nvh_gla_prep": (i32, [vp, i64, vp, i64, vp, i64, vp, i64, f32, f32, vp, vp, vp, vp, i64, i64, i64, i32, vp]),

@@ -1054,6 +1054,13 @@ def _f32_rows(t, *tensors):
         assert x.dtype == F32 and x.is_cuda and x.stride(-1) == 1 and x.shape[0] == t
 
 
+# Portions of at least SCAN_CHUNK_MIN tokens take the scan's chunked form, unless so many heads of about the longest portion's length run side by side
+# that they fill the chip token by token.  us before (token by token, or in segments) / in chunks: 16 heads of 64 x 64, 64 tokens 18.3 / 11.7, 1024
+# tokens 72 / 51, three prompts of 1008 tokens 81 / 39, twelve of 64 tokens 25.2 / 26.1; four heads of 128 x 256, 64 tokens 23.2 / 15.8, 1024 tokens
+# 108 / 71, three prompts 160 / 49; 32 heads of 128 x 64, four of 64 tokens 28.6 / 29.9, 16 of 512 tokens 577 / 611.
+SCAN_CHUNK_MIN = 64
+SCAN_CHUNK_HEADS = 192                                       # of 64 key channels
+# What has no chunked form:
 SCAN_SEGMENT_MIN_TOKENS = 256      # a sequence that brings at least this many tokens to a step is scanned in segments ...
 SCAN_SEGMENT_MAX_BATCH = 8         # ... in steps of at most this many sequences (the segments' records are scratch per sequence)
 
@@ -1078,6 +1085,16 @@ def gated_linear_scan(q, k, w, v, state, slots, cu_seqlens_q, context_lens, head
     batch = context_lens.numel()
     assert cu_seqlens_q is not None or t == batch
     out = torch.empty(t, heads * dv, dtype=F32, device=v.device)
+    if cu_seqlens_q is not None and max_seqlen_q >= SCAN_CHUNK_MIN and 64 * t * heads <= SCAN_CHUNK_HEADS * dk * max_seqlen_q:
+        nbytes = int(_hip.lib().nvh_scan_chunk_workspace_bytes(t, batch, heads, dk, dv))
+        lined_up = all(x.data_ptr() % 16 == 0 and x.stride(0) % 4 == 0 for x in (q, k) + (() if w_scalar else (w,))) and state.data_ptr() % 16 == 0
+        if nbytes and lined_up:
+            ws = torch.empty(nbytes // 4, dtype=F32, device=v.device)
+            _hip.call("nvh_gated_linear_scan_chunked", q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), g, w.data_ptr(), w.stride(0), int(w_scalar),
+                      _p(kscale), kscale.stride(0) if kscale is not None else 0, v.data_ptr(), v.stride(0), _p(skip), state.data_ptr(), slots.data_ptr(),
+                      cu_seqlens_q.data_ptr(), context_lens.data_ptr(), out.data_ptr(), batch, t, heads, dk, dv, SCAN_CHUNK_MIN, ws.data_ptr(),
+                      int(read_first), _p(bonus), _stream())
+            return out
     # Long portions (prompt chunks) in small batches: segments walked side by side, joined in a second launch.  The choice
     # depends on the step's longest portion, so a position's result may differ between schedules - within fp32 rounding.
     segments, ws_l, ws_d = 1, None, None
