@@ -542,13 +542,12 @@ __global__ __launch_bounds__(256) void attn_paged_f32_kernel(AttnArgs a, int gro
         fetch_k(next);                                       // (past the end: a block that was read before)
         __builtin_amdgcn_sched_barrier(0);
         f32x4 s = s0 + s1;
-        bool ok[4];
         float top = m_run;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if (a.softcap > 0.f) s[e] = a.softcap * tanhf(s[e] / a.softcap);
-            ok[e] = pooled ? block0 + e < my_blocks : key_visible(key0 + e, qpos, a.window, a.keep_first, a.chunk);
-            s[e] = ok[e] ? s[e] - slope * (float)(qpos - (key0 + e)) + biases[e] : -INFINITY;
+            const bool ok = pooled ? block0 + e < my_blocks : key_visible(key0 + e, qpos, a.window, a.keep_first, a.chunk);
+            s[e] = ok ? s[e] - slope * (float)(qpos - (key0 + e)) + biases[e] : -INFINITY;
             top = fmaxf(top, s[e]);
         }
         top = fmaxf(top, __shfl_xor(top, 16, 64));
@@ -557,7 +556,7 @@ __global__ __launch_bounds__(256) void attn_paged_f32_kernel(AttnArgs a, int gro
         const float alpha = top == -INFINITY ? 1.f : expf(m_run - top);
         f32x4 p;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) p[e] = ok[e] ? expf(s[e] - top) : 0.f;
+        for (int e = 0; e < 4; ++e) p[e] = s[e] == -INFINITY ? 0.f : expf(s[e] - top);       // (unseen, or a bias that masks)
         l_run = l_run * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
         m_run = top;
         if (!pooled && kb + BLOCK - 1 > last_key) {          // what the page holds past the last key may be anything
