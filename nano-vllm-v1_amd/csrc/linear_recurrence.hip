@@ -11,6 +11,7 @@
 //                    16 lanes (4 when dk is no multiple of 16) in registers, operands staged through LDS a stage ahead.
 //                    The order of every sum is fixed by the sizes alone: one piece, portions or single tokens give the
 //                    same bits.
+//   nvh_gated_linear_scan_chunked   the same, portions of many tokens in chunks of 16 (see there).
 //   nvh_group_rmsnorm_gate  read-out: RMS norm over groups of columns, weight, and a silu / sigmoid gate before or after.
 // Everything that enters the recurrence is fp32; A (bf16 or fp32) is the type of projections, weights and results.
 #include <algorithm>
