@@ -195,7 +195,7 @@ struct DeltaScanArgs {
     const int32_t* context_lens;    // [B]: tokens of the sequence including this step's (a step that holds them all starts from zero)
     float* out;                // [T, H*dv]
     int H, dk, dv;
-    int skip_from;             // portions of this many tokens and more are left to the chunked form (0: none)
+    int skip_from;             // portions of this many tokens and more are left to the chunked form (1 << 30: none)
 };
 
 // Lanes per state column (SUBS: 16 when dk is a multiple of 16, else 4), rows i = SUBS * ii + sub held by lane `sub`; a
@@ -214,8 +214,8 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
     const bool live = col < dv;
     const int lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : seq, hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : seq + 1;
     const int slot = p.slots[seq];
-    if (slot < 0 || hi <= lo) return;                        // a padded row (uniform over the workgroup)
-    if (p.skip_from > 0 && hi - lo >= p.skip_from) return;
+    // a padded row, or left to the chunked form (uniform over the workgroup; in one test)
+    if (slot < 0 || (unsigned)(hi - lo - 1) >= (unsigned)(p.skip_from - 1)) return;
     const bool fresh = p.context_lens[seq] == hi - lo;
     float* sp = p.state + (((int64_t)slot * p.H + head) * dk) * dv;
     float S[DKQ];
@@ -864,7 +864,7 @@ extern "C" int32_t nvh_delta_scan(const float* pack, float* state, const int32_t
     NVH_REQUIRE(batch >= 0 && heads > 0 && dk > 0 && dv > 0, NVH_EINVAL, "nvh_delta_scan: bad sizes");
     NVH_REQUIRE(dk <= 256, NVH_ENOSYS, "nvh_delta_scan: key size %ld above 256", (long)dk);
     if (batch == 0) return NVH_OK;
-    DeltaScanArgs p{pack, state, slots, cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 0};
+    DeltaScanArgs p{pack, state, slots, cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1 << 30};
     return launch_delta_scan(p, batch, (hipStream_t)stream);
 }
 

@@ -400,7 +400,7 @@ struct ScanArgs {
     int nseg, seg_min;         // segments per long portion (1: none) and the fewest tokens that are cut
     float *ws_l, *ws_d;        // records of the segments: end states [batch, H, nseg, dv, dk] and decay products [batch, H, nseg, dk]
     const float* bonus;        // PRE only: [H, dk] or null (0)
-    int skip_from;             // > 0, MODE 0: portions of at least this many tokens are left to the chunked form
+    int skip_from;             // WALK 3: portions of at least this many tokens are left to the chunked form (1 << 30: no chunked form)
 };
 
 // Lanes per state column (SUBS), rows held per lane (DKQ), EXACT: dk == DKQ * SUBS (no loop carries a run-time bound; rows
@@ -419,8 +419,11 @@ struct ScanArgs {
 // PRE: the token is read out BEFORE it is written and decayed, with a bonus u per key channel for the token itself,
 //   o = (S + diag(u) (c k) v^T)^T q (+ d v),   S <- diag(w) S + (c k) v^T,
 // the form of the RWKV time mix.  The joining launch then weighs a segment's start state by the decays BEFORE the token.
-template <int DKQ, int SUBS, bool EXACT, int MODE, bool PRE>
+//
+// WALK: the mode; 3: mode 0 without the portions that the chunked form takes (a test that costs a step of single tokens 0.7 us of 21).
+template <int DKQ, int SUBS, bool EXACT, int WALK, bool PRE>
 __global__ __launch_bounds__(256) void gated_linear_scan_kernel(ScanArgs p) {
+    constexpr int MODE = WALK == 3 ? 0 : WALK;
     constexpr int COLS = 256 / SUBS;
     constexpr int CH = (3 * DKQ * SUBS + COLS + 4 + 255) / 256;     // loads per lane and token
     constexpr int TOK = (32 / CH) < 2 ? 2 : (32 / CH);
@@ -433,7 +436,7 @@ __global__ __launch_bounds__(256) void gated_linear_scan_kernel(ScanArgs p) {
     const int seq_lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : seq, seq_hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : seq + 1;
     const int slot = p.slots[seq];
     if (slot < 0 || seq_hi <= seq_lo) return;                // a padded row (uniform over the workgroup)
-    if (MODE == 0 && p.skip_from > 0 && seq_hi - seq_lo >= p.skip_from) return;
+    if (WALK == 3 && seq_hi - seq_lo >= p.skip_from) return;
     const int nseg = (MODE != 0 && seq_hi - seq_lo >= p.seg_min) ? p.nseg : 1;
     if (seg >= nseg || (MODE == 2 && seg == 0)) return;      // (uniform)
     const int seg_len = (seq_hi - seq_lo + nseg - 1) / nseg;
@@ -981,6 +984,12 @@ void launch_scan_pre(const ScanArgs& p, int64_t batch, hipStream_t st) {
             gated_linear_scan_kernel<DKQ, SUBS, EXACT, 2, PRE><<<grid, 256, lds, st>>>(p);
             return;
         }
+        if constexpr (SUBS == 16 && DKQ <= 8) {
+            if (p.skip_from < 1 << 30) {                     // (beside the chunked form, whose key sizes are among these)
+                gated_linear_scan_kernel<DKQ, SUBS, EXACT, 3, PRE><<<dim3((unsigned)batch, (unsigned)p.H, colblocks), 256, lds, st>>>(p);
+                return;
+            }
+        }
     }
     gated_linear_scan_kernel<DKQ, SUBS, EXACT, 0, PRE><<<dim3((unsigned)batch, (unsigned)p.H, colblocks), 256, lds, st>>>(p);
 }
@@ -1191,7 +1200,7 @@ extern "C" int32_t nvh_gated_linear_scan(const float* q, int64_t q_stride, const
     NVH_REQUIRE(dk <= 512, NVH_ENOSYS, "nvh_gated_linear_scan: key size %ld above 512", (long)dk);
     if (batch == 0) return NVH_OK;
     ScanArgs p{q, k, q_stride, k_stride, (int)qk_groups, w, w_stride, w_scalar, kscale, kscale_stride, v, v_stride, skip, state, slots,
-                     cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1, 1 << 30, ws_states, ws_decays, bonus, 0};
+                     cu_seqlens_q, context_lens, out, (int)heads, (int)dk, (int)dv, 1, 1 << 30, ws_states, ws_decays, bonus, 1 << 30};
     NVH_REQUIRE(read_first || !bonus, NVH_EINVAL, "nvh_gated_linear_scan: a bonus needs read_first");
     if (segments > 1 && nvh_scan_segmentable(dk)) {
         NVH_REQUIRE(segments <= 64 && segment_min_tokens >= 2 * segments && ws_states && ws_decays && cu_seqlens_q, NVH_EINVAL, "nvh_gated_linear_scan: bad segments");
