@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
 #pragma unroll
             for (int g = 0; g < G; ++g) qv[g] = qknorm_rope_head(qv[g], qw, cs_row, c, fz.eps);
             if (end == ctx) {                                // (uniform)
-                // the new token's keys and values go to the cache first; the loop's loads of them are the same lanes' (in order behind the
-                // stores)
+                // the new token's keys and values go to the cache first; its lanes load them from there, in order behind their own stores (other lanes
+                // may see what was there before: settle)
                 const bf16x8 kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
                 const bf16* row = q + (int64_t)b * q_stride;
                 const bf16x8 k_new = qknorm_rope_head(*reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8), kw, cs_row, c, fz.eps);
@@ -149,6 +149,15 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         }
         page = table[min((base + 64) >> 8, last_page)];
         __builtin_amdgcn_sched_barrier(0);
+    };
+    // The last trip of a range that holds the new token.  Lanes past the end read the trip's first place; where the new token opens the trip that is
+    // the place another wave is writing, and a weight of 0 times what a reused page held there need not be 0.  They take no value at all.
+    auto settle = [&](int base, u32x4 (&vf)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t keep = base + u * 16 + rowid < end ? 0xffffffffu : 0u;
+            vf[u] &= u32x4{keep, keep, keep, keep};
+        }
     };
     auto consume = [&](int base, const u32x4 (&kw)[4], const u32x4 (&vw)[4]) {
         float s[G][4];
@@ -203,9 +212,11 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     if (start < end) fetch(start, ka, va);
     for (int base = start; base < end; base += 128) {
         if (base + 64 < end) fetch(base + 64, kb, vb);
+        else if constexpr (FUSED) settle(base, va);
         consume(base, ka, va);
         if (base + 64 >= end) break;
         if (base + 128 < end) fetch(base + 128, ka, va);
+        else if constexpr (FUSED) settle(base + 64, vb);
         consume(base + 64, kb, vb);
     }
 

@@ -589,6 +589,41 @@ def test_attn_decode_fused_qkv_equals_sequence(ops, hq, hkv, splits):
     assert float(got[6].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("hq,hkv", [(16, 8), (4, 4), (10, 2), (8, 1)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_attn_decode_fused_qkv_on_pages_that_held_other_things(ops, hq, hkv, splits):
+    """The places from the new token's on hold NaN and infinities, as pages that another request left may: the launch writes the new token's
+    key and value there and reads nothing else of them, also where the new token is the first of 64 keys (its place is then the one that lanes
+    without a key read).  The same bits as on clean pages."""
+    d, lens_k = 128, [1, 2, 64, 65, 66, 128, 129, 192, 193, 256, 257, 513, 577]
+    b = len(lens_k)
+    _, kc, vc, bt, _, _ = _paged_case(90 + hq, [1] * b, lens_k, hq, hkv)
+    qkv = rnd(b, (hq + 2 * hkv) * d, seed=91, scale=1.5)
+    qw, kw = (rnd(d, seed=92).float() * 0.2 + 1).to(BF), (rnd(d, seed=93).float() * 0.2 + 1).to(BF)
+    ctx = torch.tensor(lens_k, dtype=torch.int32)
+    table = dev(R.rope_table(128, 4096, 1e6).squeeze(1).contiguous())
+
+    def run(kcache, vcache):
+        k, v = dev(kcache), dev(vcache)
+        return ops.attn_decode_fused_qkv(dev(qkv), hq, hkv, dev(qw), dev(kw), 1e-6, dev(ctx.long() - 1), table, k, v, dev(ctx), dev(bt), d ** -0.5,
+                                         num_splits=splits), k, v
+
+    ref, kref, vref = run(kc, vc)
+    for bad in (float("nan"), float("inf")):
+        kb, vb = kc.clone(), vc.clone()
+        for i, n in enumerate(lens_k):
+            page, at = int(bt[i, (n - 1) // 256]), (n - 1) % 256
+            kb[page, at:] = bad
+            vb[page, at:] = bad
+        got, kgot, vgot = run(kb, vb)
+        assert torch.isfinite(got.float()).all()
+        assert_exact(got, ref)
+        for i, n in enumerate(lens_k):
+            page, at = int(bt[i, (n - 1) // 256]), (n - 1) % 256
+            assert_exact(kgot[page, at], kref[page, at])
+            assert_exact(vgot[page, at], vref[page, at])
+
+
 def test_attn_decode_merge_kernels_agree(ops):
     """The range merge has a few-rows and a many-rows kernel (more than 2048 output rows); they must give the same
     bits for the same sequence: 8 sequences alone vs the same 8 at the front of a batch of 160."""
