@@ -103,8 +103,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
 #pragma unroll
             for (int g = 0; g < G; ++g) qv[g] = qknorm_rope_head(qv[g], qw, cs_row, c, fz.eps);
             if (end == ctx) {                                // (uniform)
-                // the new token's keys and values go to the cache first; its lanes load them from there, in order behind their own stores (other lanes
-                // may see what was there before: settle)
+                // the new token's keys and values go to the cache first; its lanes load them from there, in order behind their own stores (others may
+                // see what was there before: settle)
                 const bf16x8 kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
                 const bf16* row = q + (int64_t)b * q_stride;
                 const bf16x8 k_new = qknorm_rope_head(*reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8), kw, cs_row, c, fz.eps);
@@ -128,10 +128,11 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     }
 
     // The keys and values of a trip (64 tokens) are requested a trip ahead into a second register set, so the work on one trip hides
-    // the loads of the next; the page after the one at hand is looked up a trip ahead.  With one workgroup a CU a trip takes 1.2 us (one set,
-    // every trip's loads waited for before its work: 1.6 us), about the 64 KB in flight over the memory's latency.  Measured beside it, a
-    // launch of 24 sequences of 100..2047 keys at 38.0 us: three and four sets 36.1 and 35.7 us, but 100 short sequences 8 and 25 % slower for
-    // the registers; two teams of four waves that split a sequence's trips 32.6 us, but a sequence's sums would then depend on the launch.
+    // the loads of the next; the page after the one at hand is looked up a trip ahead.  With one workgroup a CU a trip takes 1.0 us (one set,
+    // every trip's loads waited for before its work: 1.6 us), about the 64 KB in flight over the memory's latency.  Every trip but the last is
+    // worked on behind a request that is made in any case: behind a branch around it the waits would cover the new loads too (a launch of 24
+    // sequences of 100..2047 keys 39.1 us, as it is 31.7; 60 of 64..300 15.7 and 14.5; contexts of one trip 0.2 us longer, for the way past
+    // the loop).  Measured beside it, from 38.0 us: three and four sets 36.1 and 35.7 us, but 100 short sequences 8 and 25 % slower for the registers.
     const int32_t* table = tables + (int64_t)b * table_stride;
     u32x4 ka[4], va[4], kb[4], vb[4];                        // (whole words: as 16-bit elements every one would take a register across the loop)
     const int last_page = (end - 1) >> 8;
@@ -150,8 +151,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         page = table[min((base + 64) >> 8, last_page)];
         __builtin_amdgcn_sched_barrier(0);
     };
-    // The last trip of a range that holds the new token.  Lanes past the end read the trip's first place; where the new token opens the trip that is
-    // the place another wave is writing, and a weight of 0 times what a reused page held there need not be 0.  They take no value at all.
+    // A last trip that the new token opens: lanes past the end have read its place, which another wave is writing, and a weight of 0 times what a reused
+    // page held there need not be 0.  They take no value at all.  (Any other trip has older keys in its first place.)
     auto settle = [&](int base, u32x4 (&vf)[4]) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -209,15 +210,24 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    if (start < end) fetch(start, ka, va);
-    for (int base = start; base < end; base += 128) {
-        if (base + 64 < end) fetch(base + 64, kb, vb);
-        else if constexpr (FUSED) settle(base, va);
+    if (start < end) {
+        int base = start;
+        if (((end - start - 1) >> 6) & 1) {                  // an even number of trips
+            fetch(base, kb, vb);
+            fetch(base + 64, ka, va);
+            consume(base, kb, vb);
+            base += 64;
+        } else {
+            fetch(base, ka, va);
+        }
+        for (; base + 64 < end; base += 128) {
+            fetch(base + 64, kb, vb);
+            consume(base, ka, va);
+            fetch(base + 128, ka, va);
+            consume(base + 64, kb, vb);
+        }
+        if (FUSED && base == ctx - 1) settle(base, va);
         consume(base, ka, va);
-        if (base + 64 >= end) break;
-        if (base + 128 < end) fetch(base + 128, ka, va);
-        else if constexpr (FUSED) settle(base + 64, vb);
-        consume(base + 64, kb, vb);
     }
 
     // merge the 4 rows of the wave (lanes l, l^16, l^32 hold the same output columns)
