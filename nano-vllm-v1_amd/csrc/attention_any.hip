@@ -366,8 +366,8 @@ __global__ __launch_bounds__(256) void attn_paged_any_kernel(AttnArgs a) {
             if (ok1) s1 += bias[min(qpos - (k0 + sub + 16), a.bias_len - 1)];
         }
         const float m_new = fmaxf(m_run, row16_max(fmaxf(s0, s1)));
-        // a row that sees nothing yet keeps m = -inf (only rows past nq: every real query sees key 0)
-        const float p0 = ok0 ? expf(s0 - m_new) : 0.f, p1 = ok1 ? expf(s1 - m_new) : 0.f;
+        // (unseen keys and those that a bias masks weigh nothing; a row that has seen nothing else yet keeps m = -inf)
+        const float p0 = s0 == -INFINITY ? 0.f : expf(s0 - m_new), p1 = s1 == -INFINITY ? 0.f : expf(s1 - m_new);
         const float alpha = m_new == -INFINITY ? 1.f : expf(m_run - m_new);
         l_run = l_run * alpha + row16_sum(p0 + p1);
         m_run = m_new;

@@ -101,8 +101,6 @@ def oracle(x, kw, H, G, d, dv, ends, takes, scale):
 @pytest.mark.parametrize("option", OPTIONS)
 @pytest.mark.parametrize("H,G,d,dv,page", [(4, 2, 128, 128, 256), (2, 2, 64, 128, 48), (3, 1, 16, 16, 16), (2, 1, 128, 64, 64), (2, 1, 256, 192, 64), (2, 2, 80, 80, 48)])
 def test_prompts(H, G, d, dv, page, option):
-    if option == "masking bias" and d == 80:
-        pytest.skip("the general form takes no tile whose every score is -inf")
     ends, takes = [1, 16, 17, 63, 65, 150, 0, 129], [1, 16, 17, 40, 1, 33, 0, 129]
     x, kw = draw(H, G, d, dv, ends, takes, page, OPTIONS[option], d + len(option))
     scale = d ** -0.5
