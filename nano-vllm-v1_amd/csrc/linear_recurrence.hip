@@ -851,7 +851,7 @@ __global__ __launch_bounds__(64 * NW + 64) void scan_chunk_walk_kernel(ScanChunk
         x.K = *reinterpret_cast<const f32x4*>(r + 16 * dk + (wave * 64 + lane) * 4);
         x.P = *reinterpret_cast<const f32x4*>(r + 32 * dk + 16 * wave + 4 * q);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x.v[e] = vp[(int64_t)min(lo + CT * j + 4 * q + e, hi - 1) * p.v_stride];      // (K' is zero past the end)
+        for (int e = 0; e < 4; ++e) x.v[e] = vp[(int64_t)min(lo + CT * j + 4 * q + e, hi - 1) * p.v_stride];
     };
     auto chunk = [&](int j, const Operands& x) {
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -859,7 +859,10 @@ __global__ __launch_bounds__(64 * NW + 64) void scan_chunk_walk_kernel(ScanChunk
         for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[e], S[e], o, 0, 0, 0);
         f64x4 kv = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)x.v[e], kv, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) {
+            const float v = lo + CT * j + 4 * q + e < hi ? x.v[e] : 0.f;      // (past the end a value stands twice: K' is zero there, but 0 times infinity is not)
+            kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)v, kv, 0, 0, 0);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) S[e] = __builtin_fmaf(x.P[e], S[e], (float)kv[e]);
         meet[j & 1][wave][lane] = o;

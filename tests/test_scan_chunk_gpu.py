@@ -118,3 +118,20 @@ def test_values_that_are_not_finite(field, value):
     if field == "v":
         keep = [c for c in range(dv) if c != 5]
         torch.testing.assert_close(got[:, 1][:, keep], want[:, 1][:, keep], **close)
+
+
+@pytest.mark.parametrize("extra", [1, 9, 15])
+def test_infinite_values_in_the_last_chunk(extra):
+    """Infinite values at the last token of a portion that ends within a chunk: the state becomes infinite or not finite exactly where it does token by
+    token, and with the same signs; everything else stays as it is."""
+    H, dk, dv, T = 2, 64, 32, MIN + extra
+    g = torch.Generator().manual_seed(extra)
+    x = operands(T, H, H, dk, dv, g, "mild", False)
+    cu, ctx, slots, state = torch.tensor([0, T]).int(), torch.tensor([T]).int(), torch.tensor([0]).int(), torch.zeros(1, H, dv, dk)
+    x["v"][T - 1, 1, 5], x["v"][T - 1, 0, 7] = float("inf"), float("-inf")
+    want, want_state = scan(x, state, slots, cu, ctx, H, H, dk, dv, 0, False)
+    got, got_state = scan(x, state, slots, cu, ctx, H, H, dk, dv, T, False)
+    assert want_state.isinf().sum() == 2 * dk and not want_state.isnan().any()
+    torch.testing.assert_close(got_state, want_state, rtol=1e-5, atol=1e-5 * want_state[want_state.isfinite()].abs().max().item())
+    assert torch.equal(got.isfinite(), want.isfinite())
+    torch.testing.assert_close(got[want.isfinite()], want[want.isfinite()], rtol=1e-5, atol=1e-5 * want[want.isfinite()].abs().max().item())
