@@ -349,8 +349,8 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
 //   S = P_15 S0 + K'^T V - A'^T D,      K'_s = w_(s+1) .. w_15 k_s,  A' likewise.
 // W, Q, Y, Z, K', A' and P need no state: one launch forms them for all chunks at once.  The second launch walks the chunks: per chunk products of
 // 16 x 16 a wave on the matrix cores and one meeting of the waves.  Results differ from the token-by-token form within rounding.  What is summed over
-// a chunk's pairs of tokens, the triangular inverse and K'^T V are held in double (against float64, in the 2-norm over 1024 tokens: outputs 4.8e-8,
-// states 5.0e-8; token by token 8.3e-8 and 4.9e-8; with K'^T V in fp32 7.2e-8 for the states).
+// a chunk's pairs of tokens, the triangular inverse and P_15 S0 + K'^T V are held in double (against float64, in the 2-norm over 1024 tokens: outputs
+// 4.6e-8, states 3.4e-8; token by token 8.3e-8 and 4.9e-8; with K'^T V alone in double 5.0e-8 for the states, with nothing there 7.2e-8).
 // us at one sequence of 1024 tokens, token by token and in chunks (both launches): 16 heads of 64 x 64: 271, 27 + 47; 8 heads of 128 x 128: 331,
 // 28 + 75.  The first launch is bound by its chain when the chip is not full (11 us at 256 tokens), and else by the double products (172 us at 8448
 // records of 64 x 64); the second by the chain of a chunk, 0.74 us.
@@ -719,16 +719,20 @@ __global__ __launch_bounds__(64 * NW + 64) void delta_chunk_scan_kernel(DeltaChu
         for (int w = 0; w < NW; ++w) part[w] = meet_d[j & 1][w][lane];
         meet_o[j & 1][wave][lane] = o;
         __builtin_amdgcn_sched_barrier(0);
-        f64x4 kv = {0.0, 0.0, 0.0, 0.0};                     // (most of what a state is off by came from this sum, in fp32)
+        f64x4 kv = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int e = 0; e < 4; ++e) kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)x.V[e], kv, 0, 0, 0);
+        // (with the decayed state on it in double too, a state is rounded once a chunk: 3.4e-8 off instead of 5.0e-8, at no cost for 64 key channels
+        // and 101 -> 106 us for 8 heads of 128 x 128, 1024 tokens)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kv[e] = __builtin_fma((double)x.P[e], (double)S[e], kv[e]);
         f32x4 sum = x.Y;
 #pragma unroll
         for (int w = 0; w < NW; ++w) sum += part[w];
 #pragma unroll
         for (int e = 0; e < 4; ++e) ad = __builtin_amdgcn_mfma_f32_16x16x4f32(x.A[e], sum[e], ad, 0, 0, 0);
-        #pragma unroll
-        for (int e = 0; e < 4; ++e) S[e] = x.P[e] * S[e] + ((float)kv[e] - ad[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[e] = (float)(kv[e] - ad[e]);
     };
     constexpr int AHEAD = NW <= 4 ? 4 : 3;                   // records in flight
     Operands x[AHEAD];

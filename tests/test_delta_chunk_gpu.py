@@ -67,8 +67,7 @@ def test_portions_of_every_kind(H, dk, dv, decay):
 
 
 def test_error_against_64_bits():
-    """1024 tokens at the served sizes, in the 2-norm: the outputs are nearer to float64 than token by token, the states as near (each is off by
-    thousands of independent roundings: 5 % is more than their spread)."""
+    """1024 tokens at the served sizes, in the 2-norm: outputs and states are nearer to float64 than token by token."""
     for H, dk, dv in ((16, 64, 64), (8, 128, 128)):
         g = torch.Generator().manual_seed(3)
         rows = pack(1024, H, dk, dv, g, "mild")
@@ -80,7 +79,7 @@ def test_error_against_64_bits():
             out, st = scan(rows, state, slots, cu, ctx, H, dk, dv, longest)
             off.append([(out.double() - want.cpu()).norm(), (st[0].double() - end.cpu()).norm()])
         (out_serial, state_serial), (out_chunks, state_chunks) = off
-        assert out_chunks <= out_serial and state_chunks <= 1.05 * state_serial, (H, off)
+        assert out_chunks < out_serial and state_chunks < state_serial, (H, off)
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
