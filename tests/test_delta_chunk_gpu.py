@@ -83,23 +83,31 @@ def test_error_against_64_bits():
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("at", [37, MIN + 9])
 @pytest.mark.parametrize("field", range(6))
-def test_values_that_are_not_finite(field, value):
-    """One such value at token 37 of 100 leaves the tokens before it, and other heads, as they are; a value of v leaves the other columns as well."""
-    H, dk, dv, T, at = 2, 64, 32, 100, 37
+def test_values_that_are_not_finite(field, at, value):
+    """One such value of r, k, w, u, au or v, with whole chunks before and behind it or in the partial last chunk of a portion that is chunked: the tokens
+    before it, and other heads, stay as they are (of v: other columns as well), and what is not finite token by token is not finite in chunks."""
+    H, dk, dv, T = 2, 64, 32, MIN + 12
     g = torch.Generator().manual_seed(11)
     rows = pack(T, H, dk, dv, g, "mild")
     cu, ctx, slots, state = torch.tensor([0, T]).int(), torch.tensor([T]).int(), torch.tensor([0]).int(), torch.zeros(1, H, dk, dv)
-    want, want_state = scan(rows, state, slots, cu, ctx, H, dk, dv, 128)
+    want, want_state = scan(rows, state, slots, cu, ctx, H, dk, dv, T)
+    plain, _ = scan(rows, state, slots, cu, ctx, H, dk, dv, 0)
+    assert not torch.equal(want, plain)                      # (the two forms round differently: the chunked one ran)
     rows[at, 1, field * dk + 5] = value
-    got, got_state = scan(rows, state, slots, cu, ctx, H, dk, dv, 128)
+    serial, serial_state = scan(rows, state, slots, cu, ctx, H, dk, dv, 0)
+    got, got_state = scan(rows, state, slots, cu, ctx, H, dk, dv, T)
     close = dict(rtol=1e-5, atol=1e-5 * want.abs().max().item())
     torch.testing.assert_close(got[:at], want[:at], **close)
     torch.testing.assert_close(got[:, 0], want[:, 0], **close)
     torch.testing.assert_close(got_state[0, 0], want_state[0, 0], **close)
     assert not got[at, 1].isfinite().all()
+    assert not (got.isfinite() & ~serial.isfinite()).any() and not (got_state.isfinite() & ~serial_state.isfinite()).any()
+    if field == 0:                                           # a read-out alone
+        torch.testing.assert_close(got[at + 1:], want[at + 1:], **close)
+        torch.testing.assert_close(got_state, want_state, **close)
     if field == 5:
         keep = [c for c in range(dv) if c != 5]
         torch.testing.assert_close(got[:, 1][:, keep], want[:, 1][:, keep], **close)
-    else:
-        assert not got[at:, 1].isfinite().any() or value == float("inf") or field == 0
+        torch.testing.assert_close(got_state[0, 1][:, keep], want_state[0, 1][:, keep], **close)
