@@ -1062,7 +1062,8 @@ def _f32_rows(t, *tensors):
 # 108 / 71, three prompts 160 / 49; 32 heads of 128 x 64, four of 64 tokens 28.6 / 29.9, 16 of 512 tokens 577 / 611.
 SCAN_CHUNK_MIN = 64
 SCAN_CHUNK_HEADS = 192                                       # of 64 key channels
-# What has no chunked form:
+# What has no chunked form (key sizes above 128, value sizes that are no multiple of 16, operands that 16-byte loads may not be used on) or is left by
+# the rule above:
 SCAN_SEGMENT_MIN_TOKENS = 256      # a sequence that brings at least this many tokens to a step is scanned in segments ...
 SCAN_SEGMENT_MAX_BATCH = 8         # ... in steps of at most this many sequences (the segments' records are scratch per sequence)
 

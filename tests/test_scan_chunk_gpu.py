@@ -82,8 +82,7 @@ def test_portions_of_every_kind(H, G, dk, dv, scalar, decay, read_first):
 
 @pytest.mark.parametrize("decay", ["mild", "slow"])
 def test_error_against_64_bits(decay):
-    """1024 tokens at the served sizes, in the 2-norm, no further from float64 than token by token (each is off by thousands of independent
-    roundings: 5 % is more than their spread)."""
+    """1024 tokens at the served sizes, in the 2-norm: outputs and states are no further from float64 than token by token."""
     for H, G, dk, dv, read_first in ((16, 16, 64, 64, True), (4, 4, 128, 256, False)):
         g = torch.Generator().manual_seed(3)
         x = operands(1024, H, G, dk, dv, g, decay, False)
@@ -94,15 +93,14 @@ def test_error_against_64_bits(decay):
         for longest in (0, 1024):
             out, st = scan(x, state, slots, cu, ctx, H, G, dk, dv, longest, read_first)
             off.append([((out.double() - want.cpu()).norm() / want.cpu().norm()).item(), ((st[0].double() - end.cpu()).norm() / end.cpu().norm()).item()])
-        print("OFF", decay, [["%.2e" % y for y in z] for z in off])
         (out_serial, state_serial), (out_chunks, state_chunks) = off
-        assert out_chunks <= 1.05 * out_serial and state_chunks <= 1.05 * state_serial, (H, off)
+        assert out_chunks <= out_serial and state_chunks <= state_serial, (H, off)
 
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 @pytest.mark.parametrize("field", ["q", "k", "w", "v"])
 def test_values_that_are_not_finite(field, value):
-    """One such value at token 37 of 140 leaves the tokens before it, and other heads, as they are; a value of v leaves the other columns as well."""
+    """One such value at token 37 of 76 leaves the tokens before it, and other heads, as they are; a value of v leaves the other columns as well."""
     H, dk, dv, T, at = 2, 64, 32, MIN + 12, 37
     g = torch.Generator().manual_seed(11)
     x = operands(T, H, H, dk, dv, g, "mild", False)
@@ -118,6 +116,37 @@ def test_values_that_are_not_finite(field, value):
     if field == "v":
         keep = [c for c in range(dv) if c != 5]
         torch.testing.assert_close(got[:, 1][:, keep], want[:, 1][:, keep], **close)
+
+
+@pytest.mark.parametrize("read_first", [False, True])
+@pytest.mark.parametrize("H,G,dk,dv,scalar,lens", [(2, 2, 64, 24, False, [1, 555]), (2, 1, 128, 40, True, [513, 2]), (1, 1, 256, 64, False, [600, 3]),
+                                                   (2, 2, 48, 40, False, [300, 70, 512]), (2, 1, 256, 32, True, [9, 300]),
+                                                   (16, 16, 16, 16, False, [512, 256, 600, 9, 512, 512, 255, 512])])
+def test_segments(H, G, dk, dv, scalar, lens, read_first):
+    """Head sizes without a chunked form, and one with it whose heads fill the chip: portions of 256 tokens and more in four segments, in eight where the
+    longest has 512, beside shorter ones; fresh and carried.  The bound is eight times what the token-by-token form is off, and 1e-6 of the largest
+    value."""
+    from nanovllm import _hip, ops
+    assert _hip.lib().nvh_scan_segmentable(dk)
+    crowded = 64 * sum(lens) * H > ops.SCAN_CHUNK_HEADS * dk * max(lens)
+    assert crowded or not _hip.lib().nvh_scan_chunk_workspace_bytes(sum(lens), len(lens), H, dk, dv)
+    assert max(lens) >= ops.SCAN_SEGMENT_MIN_TOKENS and len(lens) <= ops.SCAN_SEGMENT_MAX_BATCH
+    g = torch.Generator().manual_seed(dk + dv)
+    T, B, plain = sum(lens), len(lens), dk == 48
+    x = operands(T, H, G, dk, dv, g, "slow", scalar)
+    state = torch.randn(B + 1, H, dv, dk, generator=g)
+    slots, cu, carried = torch.randperm(B + 1, generator=g)[:B].int(), torch.tensor([0] + lens).cumsum(0).int(), [4 * (b % 2 == 0) for b in range(B)]
+    ctx = torch.tensor([n + c for n, c in zip(lens, carried)]).int()
+    serial, serial_state = scan(x, state, slots, cu, ctx, H, G, dk, dv, 0, read_first, plain)
+    got, got_state = scan(x, state, slots, cu, ctx, H, G, dk, dv, max(lens), read_first, plain)
+    y = full(x, H, G, dk, plain)
+    for b, n in enumerate(lens):
+        at, s = int(cu[b]), int(slots[b])
+        want, end = recurrence({m: t if m in ("skip", "bonus") else t[at:at + n] for m, t in y.items()},
+                               state[s].double() if carried[b] else torch.zeros(H, dv, dk, dtype=torch.float64), read_first)
+        for a, c, z in ((got[at:at + n], serial[at:at + n], want), (got_state[s], serial_state[s], end)):
+            assert torch.equal(a, c) == (n < ops.SCAN_SEGMENT_MIN_TOKENS), (b, n)      # (long ones round differently: they were cut)
+            assert (a.double() - z).abs().max() <= 8 * (c.double() - z).abs().max() + 1e-6 * z.abs().max(), (b, n)
 
 
 @pytest.mark.parametrize("extra", [1, 9, 15])
