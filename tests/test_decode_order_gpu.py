@@ -65,3 +65,34 @@ def test_order_of_dispatch_changes_no_bit(count, eager):
         assert (few - one[[0, count - 1, 7]].float()).abs().max() < 5e-2
     finally:
         runner.exit()
+
+
+@pytest.mark.parametrize("count", [129, 140])
+def test_order_in_a_mixed_step(count):
+    """Decoding sequences in front of a portion of a prompt, enough for the dispatch by length: handed over in two orders every sequence, the portion's
+    last token too, gets the same logits bit for bit."""
+    from nanovllm.config import Config
+    from nanovllm.engine.model_runner import ModelRunner
+    from nanovllm.engine.sequence import Sequence
+    g = torch.Generator().manual_seed(count)
+    lens = torch.randint(1, 520, (count,), generator=g).tolist() + [300]
+    lens[0], lens[count - 1] = 1, 519
+    pages = [-(-n // 256) for n in lens]
+    runner = ModelRunner(Config(TINY, max_num_batched_tokens=1024, max_num_seqs=160, max_model_len=1024, num_kvcache_blocks=sum(pages), chunked_prefill=True), 0, [])
+    try:
+        seqs, at = [], 0
+        for i, (n, p) in enumerate(zip(lens, pages)):
+            s = Sequence(torch.randint(0, 1024, (n,), generator=g).tolist())
+            s.block_table, at = list(range(at, at + p)), at + p
+            behind = n - 1 if i < count else 70              # (the portion: 230 tokens behind 70)
+            s.num_new_tokens = behind
+            if behind:
+                runner.run([s])
+            s.num_cached_tokens, s.num_new_tokens = behind, n - behind
+            seqs.append(s)
+        *running, prompt = seqs
+        one = runner.forward_logits(running + [prompt])[0].clone()
+        two = runner.forward_logits(running[::-1] + [prompt])[0].clone()
+        assert torch.equal(one[:count], two[:count].flip(0)) and torch.equal(one[count], two[count])
+    finally:
+        runner.exit()
