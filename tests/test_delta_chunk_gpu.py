@@ -111,3 +111,15 @@ def test_values_that_are_not_finite(field, at, value):
         keep = [c for c in range(dv) if c != 5]
         torch.testing.assert_close(got[:, 1][:, keep], want[:, 1][:, keep], **close)
         torch.testing.assert_close(got_state[0, 1][:, keep], want_state[0, 1][:, keep], **close)
+
+
+def test_cuts_at_whole_chunks():
+    """A portion cut at a multiple of 16 tokens into two that are chunked: the same bits."""
+    H, dk, dv, T, cut = 2, 64, 64, 3 * MIN + 5, MIN + 16
+    g = torch.Generator().manual_seed(5)
+    rows, state = pack(T, H, dk, dv, g, "mild"), torch.randn(1, H, dk, dv, generator=g)
+    slots, at = torch.tensor([0]).int(), lambda *n: torch.tensor(n).int()
+    whole, whole_state = scan(rows, state, slots, at(0, T), at(T + 1), H, dk, dv, T)
+    one, mid = scan(rows[:cut].contiguous(), state, slots, at(0, cut), at(cut + 1), H, dk, dv, cut)
+    two, end = scan(rows[cut:].contiguous(), mid, slots, at(0, T - cut), at(T + 1), H, dk, dv, T - cut)
+    assert torch.equal(torch.cat([one, two]), whole) and torch.equal(end, whole_state)

@@ -164,3 +164,16 @@ def test_infinite_values_in_the_last_chunk(extra):
     torch.testing.assert_close(got_state, want_state, rtol=1e-5, atol=1e-5 * want_state[want_state.isfinite()].abs().max().item())
     assert torch.equal(got.isfinite(), want.isfinite())
     torch.testing.assert_close(got[want.isfinite()], want[want.isfinite()], rtol=1e-5, atol=1e-5 * want[want.isfinite()].abs().max().item())
+
+
+def test_cuts_at_whole_chunks():
+    """A portion cut at a multiple of 16 tokens into two that are chunked: the same bits."""
+    H, dk, dv, T, cut = 2, 64, 64, 3 * MIN + 5, MIN + 16
+    g = torch.Generator().manual_seed(5)
+    x, state = operands(T, H, H, dk, dv, g, "mild", False), torch.randn(1, H, dv, dk, generator=g)
+    part = lambda lo, hi: {m: t if m in ("skip", "bonus") else t[lo:hi] for m, t in x.items()}
+    slots, at = torch.tensor([0]).int(), lambda *n: torch.tensor(n).int()
+    whole, whole_state = scan(x, state, slots, at(0, T), at(T + 1), H, H, dk, dv, T, False)
+    one, mid = scan(part(0, cut), state, slots, at(0, cut), at(cut + 1), H, H, dk, dv, cut, False)
+    two, end = scan(part(cut, T), mid, slots, at(0, T - cut), at(T + 1), H, H, dk, dv, T - cut, False)
+    assert torch.equal(torch.cat([one, two]), whole) and torch.equal(end, whole_state)
