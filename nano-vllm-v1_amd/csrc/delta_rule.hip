@@ -352,7 +352,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
 // a chunk's pairs of tokens, the triangular inverse and P_15 S0 + K'^T V are held in double (against float64, in the 2-norm over 1024 tokens: outputs
 // 4.6e-8, states 3.4e-8; token by token 8.3e-8 and 4.9e-8; with K'^T V alone in double 5.0e-8 for the states, with nothing there 7.2e-8).
 // us at one sequence of 1024 tokens, token by token and in chunks (both launches): 16 heads of 64 x 64: 271, 27 + 47; 8 heads of 128 x 128: 331,
-// 28 + 75.  The first launch is bound by its chain when the chip is not full (11 us at 256 tokens), and else by the double products (172 us at 8448
+// 28 + 78.  The first launch is bound by its chain when the chip is not full (11 us at 256 tokens), and else by the double products (172 us at 8448
 // records of 64 x 64); the second by the chain of a chunk, 0.74 us.
 // What the first launch keeps in LDS: r | k | w | u | au, 16 rows of dk + 4 floats each, and in doubles the decays and their reciprocals (16 rows of
 // dk + 2 each), which later give their place to four matrices.

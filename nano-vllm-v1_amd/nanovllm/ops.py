@@ -801,7 +801,7 @@ def attn_pool_blocks(k_cache, v_cache, cu_seqlens_q, context_lens, block_tables,
 # side by side that they fill the chip token by token (the chunked form reads and writes more: it is for the chain's sake).  us token by token / in
 # chunks, 16 heads of 64 x 64: 96 tokens 28.6 / 22.8, 128 tokens 36.8 / 19.2, 1024 tokens 271 / 75, four of 192 tokens 56 / 43, eight of 128 tokens
 # 42.9 / 47.4; 32 heads: four of 128 tokens 43.5 / 47.2, eight of 512 tokens 242 / 310; eight heads of 128 x 128: 96 tokens 34.4 / 35.2, 128 tokens
-# 44 / 28, 1024 tokens 331 / 104, eight of 128 tokens 67.6 / 56.8.
+# 44 / 28, 1024 tokens 331 / 106, eight of 128 tokens 67.6 / 56.8.
 DELTA_CHUNK_MIN = 128
 DELTA_CHUNK_HEADS = 96                                       # of 64 key channels
 
