@@ -973,6 +973,96 @@ __global__ __launch_bounds__(256) void group_rmsnorm_gate_block_kernel(const flo
     }
 }
 
+// One token per sequence (a decode step): no staging, no barrier.  A lane holds its rows of NC columns, requests all of them and its rows of
+// q, k and w (the same for every column) at once, and writes the new ones back; rows, order of the sums and so every bit are those of the form above.
+// Bound by the state's way from and to memory, and below about two workgroups a CU by that memory's latency.  us, the form above and this one: 64
+// sequences with 8 heads of 128 x 128 25.9 and 17.7 (3.8 TB/s both ways), 32 heads of 128 x 64 51.9 and 32.9, 16 heads of 64 x 64 read first
+// 16.5 and 8.7; 16 sequences with 8 heads of 128 x 128 8.5 and 5.1; one 4.1 and 2.4.
+template <int DKQ, bool PRE, int NC>
+__global__ __launch_bounds__(256) void gated_linear_token_kernel(ScanArgs p) {
+    static_assert(DKQ % 4 == 0 && NC <= 16, "rows in groups of four, a lane of a column's sixteen per column block");
+    constexpr int R4 = DKQ / 4;
+    const int seq = blockIdx.x, head = blockIdx.y, dk = 16 * DKQ, dv = p.dv;
+    const int sub = threadIdx.x & 15, lcol = threadIdx.x >> 4, col0 = blockIdx.z * (16 * NC) + lcol;
+    const int slot = p.slots[seq];
+    if (slot < 0) return;                                    // a padded row (uniform)
+    const bool fresh = p.context_lens[seq] == 1;
+    const int group = head / (p.H / p.qk_groups);
+    f32x4* sp = reinterpret_cast<f32x4*>(p.state + (((int64_t)slot * p.H + head) * dv) * dk) + sub;
+    f32x4 S[NC][R4], q[R4], k[R4], w[R4];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const int col = min(col0 + 16 * j, dv - 1);          // (columns past the last repeat it and are not written)
+#pragma unroll
+        for (int c = 0; c < R4; ++c) S[j][c] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : sp[(int64_t)col * (dk / 4) + 16 * c];
+    }
+    const f32x4* qp = reinterpret_cast<const f32x4*>(p.q + (int64_t)seq * p.q_stride + group * dk) + sub;
+    const f32x4* kp = reinterpret_cast<const f32x4*>(p.k + (int64_t)seq * p.k_stride + group * dk) + sub;
+    const float* wrow = p.w + (int64_t)seq * p.w_stride + (p.w_scalar ? head : (int64_t)head * dk);
+#pragma unroll
+    for (int c = 0; c < R4; ++c) {
+        q[c] = qp[16 * c];
+        k[c] = kp[16 * c];
+        if (p.w_scalar) w[c] = f32x4{wrow[0], wrow[0], wrow[0], wrow[0]};
+        else w[c] = reinterpret_cast<const f32x4*>(wrow)[sub + 16 * c];
+    }
+    f32x4 u[PRE ? R4 : 1];
+    if constexpr (PRE) {
+#pragma unroll
+        for (int c = 0; c < R4; ++c) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[c][e] = p.bonus ? p.bonus[(int64_t)head * dk + 64 * c + 4 * sub + e] : 0.f;
+        }
+    }
+    const float strength = p.kscale ? p.kscale[(int64_t)seq * p.ks_stride + head] : 1.0f, skip = p.skip ? p.skip[head] : 0.f;
+    const float* vrow = p.v + (int64_t)seq * p.v_stride + (int64_t)head * dv;
+    float v[NC], mine = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) v[j] = vrow[min(col0 + 16 * j, dv - 1)];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        const float sv = strength * v[j];
+        float o = 0.f;
+#pragma unroll
+        for (int c = 0; c < R4; ++c) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (PRE) {
+                    const float kv = k[c][e] * sv;
+                    o = __builtin_fmaf(__builtin_fmaf(u[c][e], kv, S[j][c][e]), q[c][e], o);
+                    S[j][c][e] = __builtin_fmaf(w[c][e], S[j][c][e], kv);
+                } else {
+                    S[j][c][e] = __builtin_fmaf(w[c][e], S[j][c][e], k[c][e] * sv);
+                    o = __builtin_fmaf(S[j][c][e], q[c][e], o);
+                }
+            }
+        }
+        o = __builtin_fmaf(skip, v[j], row16_sum(o));
+        if (sub == j) mine = o;                              // (a column's sixteen lanes all hold its sum: lane j writes column block j's)
+        if (col0 + 16 * j < dv) {
+#pragma unroll
+            for (int c = 0; c < R4; ++c) sp[(int64_t)(col0 + 16 * j) * (dk / 4) + 16 * c] = S[j][c];
+        }
+    }
+    if (sub < NC && col0 + 16 * sub < dv) p.out[(int64_t)seq * p.H * dv + head * dv + col0 + 16 * sub] = mine;
+}
+
+// Whether a step of one token per sequence takes gated_linear_token_kernel: its lanes read 16 bytes at a time.
+static bool scan_token_ok(const ScanArgs& p) {
+    return !p.cu_seqlens_q && p.nseg == 1 && p.q_stride % 4 == 0 && p.k_stride % 4 == 0 && (p.w_scalar || (p.w_stride % 4 == 0 && nvh_aligned16(p.w))) &&
+           nvh_aligned16(p.q) && nvh_aligned16(p.k) && nvh_aligned16(p.state);
+}
+
+template <int DKQ, bool PRE>
+void launch_scan_token(const ScanArgs& p, int64_t batch, hipStream_t st) {
+    // Columns of a lane: as many as leave the chip two workgroups a CU.
+    constexpr int MOST = DKQ <= 8 ? 4 : 2;
+    if (batch * p.H * nvh_cdiv(p.dv, 16 * MOST) >= 512)
+        gated_linear_token_kernel<DKQ, PRE, MOST><<<dim3((unsigned)batch, (unsigned)p.H, (unsigned)nvh_cdiv(p.dv, 16 * MOST)), 256, 0, st>>>(p);
+    else
+        gated_linear_token_kernel<DKQ, PRE, 1><<<dim3((unsigned)batch, (unsigned)p.H, (unsigned)nvh_cdiv(p.dv, 16)), 256, 0, st>>>(p);
+}
+
 template <int DKQ, int SUBS, bool EXACT, bool PRE>
 void launch_scan_pre(const ScanArgs& p, int64_t batch, hipStream_t st) {
     constexpr int COLS = 256 / SUBS;
@@ -980,6 +1070,12 @@ void launch_scan_pre(const ScanArgs& p, int64_t batch, hipStream_t st) {
     constexpr int TOK = (32 / CH) < 2 ? 2 : (32 / CH);
     const unsigned colblocks = (unsigned)nvh_cdiv(p.dv, COLS);
     const size_t lds = sizeof(float) * (size_t)TOK * (((3 * p.dk + COLS + 4) & ~3) + COLS);
+    if constexpr (EXACT && SUBS == 16 && DKQ % 4 == 0) {
+        if (scan_token_ok(p)) {
+            launch_scan_token<DKQ, PRE>(p, batch, st);
+            return;
+        }
+    }
     if constexpr (EXACT) {
         if (p.nseg > 1) {
             const dim3 grid((unsigned)batch, (unsigned)p.H, colblocks * (unsigned)p.nseg);
