@@ -340,6 +340,94 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaScanArgs p) {
     }
 }
 
+// One token per sequence (a decode step), dk = 16 DKQ: a workgroup holds 4 NC4 columns of a head's state, a lane R consecutive rows of four of them,
+// so that a row's columns are read and written as they lie - the form above reads 16 bytes of a row at a time.  The rows' sums are formed in its
+// order: DKQ rows one after the other, then pairs, fours, eights and the sixteen (row16_sum), the pairs in a lane and the rest through LDS, so
+// every bit is the same.  Bound by the state's way from and to memory.
+// us, the form above and this one: 64 sequences with 8 heads of 128 x 128 40.8 and 17.7 (3.8 TB/s both ways), 16 heads of 64 x 64 23.0 and 8.3; 16 with
+// 8 heads of 128 x 128 11.7 and 5.5; one 4.5 and 3.5.
+template <int DKQ, int NC4>
+__global__ __launch_bounds__(256) void delta_token_kernel(DeltaScanArgs p) {
+    constexpr int dk = 16 * DKQ, GROUPS = 256 / NC4, SUBS = 16 / GROUPS, R = SUBS * DKQ;      // row groups; runs of DKQ rows and rows of a lane
+    static_assert(GROUPS * SUBS == 16 && GROUPS >= 4, "the sixteen runs of rows, at least four to be summed through LDS");
+    __shared__ __attribute__((aligned(16))) float ops[5 * dk];        // r | k | w | u | au
+    __shared__ f32x4 part[2][GROUPS][NC4];
+    const int seq = blockIdx.x, head = blockIdx.y, dv = p.dv, tid = threadIdx.x;
+    const int slot = p.slots[seq];
+    if (slot < 0) return;                                    // a padded row (uniform)
+    const bool fresh = p.context_lens[seq] == 1;
+    const int c4 = tid % NC4, grp = tid / NC4, col = (blockIdx.z * NC4 + c4) * 4, row0 = grp * R;
+    const bool live = col < dv;                              // (dv a multiple of 4)
+    float* sp = p.state + (((int64_t)slot * p.H + head) * dk + row0) * dv + min(col, dv - 4);
+    const float* pack = p.pack + ((int64_t)seq * p.H + head) * (5 * dk + dv);
+    f32x4 S[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) S[i] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const f32x4*>(sp + (int64_t)i * dv);
+    for (int i = tid; i < 5 * dk; i += 256) ops[i] = pack[i];
+    const f32x4 v = *reinterpret_cast<const f32x4*>(pack + 5 * dk + min(col, dv - 4));
+    __syncthreads();
+    const float *r = ops + row0, *k = r + dk, *w = k + dk, *u = w + dk, *au = u + dk;
+    // the sum over all rows of four columns, of which a lane brings its runs' sums
+    auto total = [&](const f32x4 (&run)[SUBS], int which) {
+        f32x4 mine = run[0];
+        if constexpr (SUBS == 2) mine = run[0] + run[1];
+        if constexpr (SUBS == 4) mine = (run[0] + run[1]) + (run[2] + run[3]);
+        part[which][grp][c4] = mine;
+        __syncthreads();
+        f32x4 x[GROUPS];
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) x[g] = part[which][g][c4];
+#pragma unroll
+        for (int n = GROUPS / 2; n >= 1; n /= 2)
+#pragma unroll
+            for (int g = 0; g < n; ++g) x[g] = x[2 * g] + x[2 * g + 1];
+        return x[0];
+    };
+    f32x4 run[SUBS];
+#pragma unroll
+    for (int s = 0; s < SUBS; ++s) {
+        run[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DKQ; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) run[s][e] = __builtin_fmaf(u[s * DKQ + i], S[s * DKQ + i][e], run[s][e]);
+    }
+    const f32x4 dot = total(run, 0);
+#pragma unroll
+    for (int s = 0; s < SUBS; ++s) {
+        run[s] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DKQ; ++i) {
+            const int at = s * DKQ + i;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                S[at][e] = __builtin_fmaf(w[at], S[at][e], __builtin_fmaf(k[at], v[e], -(au[at] * dot[e])));
+                run[s][e] = __builtin_fmaf(S[at][e], r[at], run[s][e]);
+            }
+        }
+    }
+    if (live) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) *reinterpret_cast<f32x4*>(sp + (int64_t)i * dv) = S[i];
+    }
+    const f32x4 o = total(run, 1);
+    if (live && grp == 0) *reinterpret_cast<f32x4*>(p.out + ((int64_t)seq * p.H + head) * dv + col) = o;
+}
+
+// Whether a step of one token per sequence takes delta_token_kernel: rows of whole aligned groups of four columns.
+static bool delta_token_ok(const DeltaScanArgs& p) {
+    return !p.cu_seqlens_q && p.dv % 4 == 0 && nvh_aligned16(p.pack) && nvh_aligned16(p.state) && nvh_aligned16(p.out);
+}
+
+template <int DKQ>
+static void launch_delta_token(const DeltaScanArgs& p, int64_t batch, hipStream_t st) {
+    // 128 columns a workgroup as long as every CU gets two, else 64 (the results are the same)
+    if (DKQ <= 8 && batch * p.H * nvh_cdiv(p.dv, 128) >= 512 && p.dv > 64)
+        delta_token_kernel<DKQ, DKQ <= 8 ? 32 : 16><<<dim3((unsigned)batch, (unsigned)p.H, (unsigned)nvh_cdiv(p.dv, 128)), 256, 0, st>>>(p);
+    else
+        delta_token_kernel<DKQ, 16><<<dim3((unsigned)batch, (unsigned)p.H, (unsigned)nvh_cdiv(p.dv, 64)), 256, 0, st>>>(p);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // The chunked form, for portions of many tokens (token by token every token costs the chain S -> u^T S -> S, 0.25 - 0.33 us, whatever the chip
 // has idle).  Within a chunk of 16 tokens the recurrence is linear in the chunk's first state S0.  With P_t the product of the decays of tokens
@@ -814,6 +902,13 @@ static void launch_delta_scan_as(const DeltaScanArgs& p, int64_t batch, hipStrea
 
 static int32_t launch_delta_scan(const DeltaScanArgs& p, int64_t batch, hipStream_t st) {
     // (the choice depends on dk alone, so a sequence sees one summation order whatever the batch or the cut)
+    if (delta_token_ok(p)) {                                 // (the bits of the form below)
+        switch (p.dk) {
+            case 64: launch_delta_token<4>(p, batch, st); NVH_CHECK_LAUNCH("nvh_delta_scan"); return NVH_OK;
+            case 128: launch_delta_token<8>(p, batch, st); NVH_CHECK_LAUNCH("nvh_delta_scan"); return NVH_OK;
+            case 256: launch_delta_token<16>(p, batch, st); NVH_CHECK_LAUNCH("nvh_delta_scan"); return NVH_OK;
+        }
+    }
     if (p.dk % 16 == 0) {
         switch (p.dk / 16) {
             case 1: launch_delta_scan_as<1, 16, true>(p, batch, st); break;

@@ -34,3 +34,19 @@ def test_gated_linear_scan(B, H, G, dk, dv, read_first, scalar):
     wide[:, :G * dk] = q
     again = state.clone()
     assert torch.equal(ops.gated_linear_scan(wide[:, :G * dk], k, w, v, again, slots, None, ctx, H, dk, dv, **kw)[real], a[real])
+
+
+@pytest.mark.parametrize("B,H,dk,dv", [(1, 1, 64, 4), (3, 2, 64, 36), (5, 3, 128, 72), (3, 2, 256, 64), (40, 16, 64, 64), (33, 16, 128, 128), (70, 8, 128, 100), (5, 3, 64, 30)])
+def test_delta_rule(B, H, dk, dv):
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(B + dk + dv)
+    slots, ctx, cu = _slots(B, g)
+    rows = torch.randn(B, H, 5 * dk + dv, generator=g).cuda() * 0.3
+    state = torch.randn(B + 2, H, dk, dv, generator=g).cuda()
+    if B > 2:
+        state[slots[2]] = float("nan")
+    one, many = state.clone(), state.clone()
+    a = ops._delta_scan(rows, one, slots, None, ctx, H, dk, dv, 1)
+    b = ops._delta_scan(rows, many, slots, cu, ctx, H, dk, dv, 1)
+    real = slots >= 0
+    assert torch.equal(a[real], b[real]) and torch.equal(one.view(torch.int32), many.view(torch.int32))
