@@ -65,34 +65,82 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
         for (int r = 0; r < top; ++r) weights[t * top + r] = weights[t * top + r] / denom;
 }
 
-// The same with the router's product inside: z[e] = x . w[e] + bias[e] in fp32, every expert's dot product spread over the
-// wave's lanes (lane l takes elements l, l + 64, ... of the row) and summed across it.
-// One workgroup per token: its four waves take the experts four at a time in turn, every dot product spread over a wave's
-// lanes (a lane takes 8 consecutive elements of every 512) and summed across it; the logits meet in LDS and the first wave picks.
-template <typename A>
+// (Routing over 16 experts of 1024 columns, us a launch, 64 and 1000 tokens: 12.3 and 12.7 with a piece of 512 at a time, a chain of lane exchanges for
+// every comparison of the argmax and the weights read back to be divided; now 4.8 and 6.3.)
+// Dot products of a token's row with up to EG rows of K, row(g) for g < n, in fp32: a lane takes 8 consecutive elements of every 512, in order.
+// Whole pieces of 512 go two at a time, all their loads ahead of the sums: the rows come from L2, and its latency is what a token waits for.
+template <int EG, typename A, typename Row>
+__device__ __forceinline__ void route_dots(const A* __restrict__ xr, Row row, int n, int K, int vec, int lane, float (&acc)[EG]) {
+#pragma unroll
+    for (int g = 0; g < EG; ++g) acc[g] = 0.f;
+    int k0 = lane * 8;
+    if (vec) {                                               // (uniform)
+        for (int left = K; left >= 1024; left -= 1024, k0 += 1024) {
+            float xv[2][8], wv[2][EG][8];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                nvh_load8(xr, k0 + 512 * u, 8, true, xv[u]);
+#pragma unroll
+                for (int g = 0; g < EG; ++g)
+                    if (g < n) nvh_load8(row(g), k0 + 512 * u, 8, true, wv[u][g]);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int g = 0; g < EG; ++g)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (g < n) acc[g] = __builtin_fmaf(xv[u][i], wv[u][g][i], acc[g]);
+        }
+    }
+    for (; k0 < K; k0 += 512) {
+        float xv[8];
+        nvh_load8(xr, k0, K - k0, vec, xv);
+#pragma unroll
+        for (int g = 0; g < EG; ++g)
+            if (g < n) {
+                float wv[8];
+                nvh_load8(row(g), k0, K - k0, vec, wv);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[i], wv[i], acc[g]);
+            }
+    }
+}
+
+// The largest of a wave's values z[j] of lane l, number l + 64 j (ties: the lowest number); 0x7fffffff and -inf where none is above -inf.
+template <int PL>
+__device__ __forceinline__ int pick_largest(const float (&z)[PL], float& best) {
+    float m = z[0];
+#pragma unroll
+    for (int j = 1; j < PL; ++j) m = fmaxf(m, z[j]);
+    m = wave_max(m);
+    best = m;
+    if (m > -INFINITY) {
+#pragma unroll
+        for (int j = 0; j < PL; ++j) {
+            const unsigned long long at = __ballot(z[j] == m);
+            if (at) return 64 * j + __builtin_ctzll(at);
+        }
+    }
+    best = -INFINITY;
+    return 0x7fffffff;
+}
+
+// The same with the router's product inside: z[e] = x . w[e] + bias[e] in fp32.  One workgroup per token: its four waves take the experts four at
+// a time in turn, every dot product spread over a wave's lanes and summed across it; the logits meet in LDS and the first wave picks.
+// PL: experts a lane of the picking wave holds: experts <= 64 PL.
+template <typename A, int PL>
 __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restrict__ x, int64_t ldx, const A* __restrict__ w, const A* __restrict__ bias,
                                                                int32_t* __restrict__ ids, float* __restrict__ weights, float* __restrict__ logits_out,
                                                                int experts, int K, int top, int vec, int sigmoid_scores) {
-    __shared__ float zs[64 * ROUTE_MAX_PER_LANE];
+    __shared__ float zs[64 * PL];
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const A* xr = x + t * ldx;
     constexpr int EG = 4;
     for (int e0 = wave * EG; e0 < experts; e0 += 4 * EG) {
         float acc[EG];
-#pragma unroll
-        for (int g = 0; g < EG; ++g) acc[g] = 0.f;
-        for (int k0 = lane * 8; k0 < K; k0 += 512) {
-            float xv[8];
-            nvh_load8(xr, k0, K - k0, vec, xv);
-#pragma unroll
-            for (int g = 0; g < EG; ++g) {
-                float wv[8];
-                nvh_load8(w + (int64_t)min(e0 + g, experts - 1) * K, k0, K - k0, vec, wv);
-#pragma unroll
-                for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[i], wv[i], acc[g]);
-            }
-        }
+        route_dots<EG>(xr, [&](int g) { return w + (int64_t)min(e0 + g, experts - 1) * K; }, EG, K, vec, lane, acc);
 #pragma unroll
         for (int g = 0; g < EG; ++g) {
             const int e = e0 + g;
@@ -105,44 +153,31 @@ __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restri
     }
     __syncthreads();
     if (wave != 0) return;
-    float z[ROUTE_MAX_PER_LANE];
+    float z[PL];
 #pragma unroll
-    for (int j = 0; j < ROUTE_MAX_PER_LANE; ++j) z[j] = lane + 64 * j < experts ? zs[lane + 64 * j] : -INFINITY;
-    float first = 0.f, denom = 0.f;
+    for (int j = 0; j < PL; ++j) z[j] = lane + 64 * j < experts ? zs[lane + 64 * j] : -INFINITY;
+    float first = 0.f, denom = 0.f, mine = 0.f;
     for (int r = 0; r < top; ++r) {
-        float bv = -INFINITY;
-        int be = 0x7fffffff;
-#pragma unroll
-        for (int j = 0; j < ROUTE_MAX_PER_LANE; ++j) {
-            const int e = lane + 64 * j;
-            if (z[j] > bv || (z[j] == bv && e < be && z[j] != -INFINITY)) {
-                bv = z[j];
-                be = e;
-            }
-        }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float ov = __shfl_xor(bv, off, 64);
-            const int oe = __shfl_xor(be, off, 64);
-            if (ov > bv || (ov == bv && oe < be)) {
-                bv = ov;
-                be = oe;
-            }
-        }
+        float bv;
+        const int be = pick_largest<PL>(z, bv);
         if (r == 0) first = bv;
         // (sigmoid scores: an expert's weight is its own score, whatever the others'; the order by logit is the order by score)
         const float wgt = sigmoid_scores ? 1.0f / (1.0f + expf(-bv)) : expf(bv - first);
         denom += wgt;
+        if (lane == (r & 63)) mine = wgt;                    // (kept until the sum is known; 64 of them at most)
         if (lane == 0) {
             ids[t * top + r] = be;
-            weights[t * top + r] = wgt;
+            if (top > 64) weights[t * top + r] = wgt;
         }
 #pragma unroll
-        for (int j = 0; j < ROUTE_MAX_PER_LANE; ++j)
+        for (int j = 0; j < PL; ++j)
             if (lane + 64 * j == be) z[j] = -INFINITY;
     }
-    if (lane == 0 && !sigmoid_scores)
+    if (top <= 64) {
+        if (lane < top) weights[t * top + lane] = sigmoid_scores ? mine : mine / denom;
+    } else if (lane == 0 && !sigmoid_scores) {
         for (int r = 0; r < top; ++r) weights[t * top + r] = weights[t * top + r] / denom;
+    }
 }
 
 // Routing by scores: s = softmax(x W^T) over ALL experts; the choice goes by s + correction (a per-expert offset that
@@ -169,22 +204,10 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restri
     const int eg = min(EG, (rows + 3) / 4);
     for (int e0 = wave * eg; e0 < rows; e0 += 4 * eg) {
         float acc[EG];
-#pragma unroll
-        for (int g = 0; g < EG; ++g) acc[g] = 0.f;
-        for (int k0 = lane * 8; k0 < K; k0 += 512) {
-            float xv[8];
-            nvh_load8(xr, k0, K - k0, vec, xv);
-#pragma unroll
-            for (int g = 0; g < EG; ++g)
-                if (g < eg) {                                // (uniform)
-                    const int e = min(e0 + g, rows - 1);
-                    const A* wr = e < experts ? w + (int64_t)e * K : aux + (int64_t)(e - experts) * K;
-                    float wv[8];
-                    nvh_load8(wr, k0, K - k0, vec, wv);
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[i], wv[i], acc[g]);
-                }
-        }
+        route_dots<EG>(xr, [&](int g) {
+            const int e = min(e0 + g, rows - 1);
+            return e < experts ? w + (int64_t)e * K : aux + (int64_t)(e - experts) * K;
+        }, eg, K, vec, lane, acc);
 #pragma unroll
         for (int g = 0; g < EG; ++g)
             if (g < eg) {
@@ -283,38 +306,36 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restri
     bool taken[PL];
 #pragma unroll
     for (int j = 0; j < PL; ++j) taken[j] = lane + 64 * j >= experts;
-    float total = 0.f;
+    float total = 0.f, mine = 0.f;
     for (int r = 0; r < top; ++r) {
-        float bv = -INFINITY;
-        int be = 0x7fffffff;
+        // the largest that is left, the lowest number among equals (nothing above -inf left, or nothing that compares: the lowest number left)
+        float bv, open[PL];
 #pragma unroll
-        for (int j = 0; j < PL; ++j) {
-            const int e = lane + 64 * j;
-            if (!taken[j] && (z[j] > bv || be == 0x7fffffff)) {
-                bv = z[j];
-                be = e;
+        for (int j = 0; j < PL; ++j) open[j] = taken[j] ? -INFINITY : z[j];
+        int be = pick_largest<PL>(open, bv);
+        if (be == 0x7fffffff) {
+#pragma unroll
+            for (int j = PL - 1; j >= 0; --j) {
+                const unsigned long long at = __ballot(!taken[j]);
+                if (at) be = 64 * j + __builtin_ctzll(at);
             }
         }
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const float ov = __shfl_xor(bv, off, 64);
-            const int oe = __shfl_xor(be, off, 64);
-            if (oe != 0x7fffffff && (be == 0x7fffffff || ov > bv || (ov == bv && oe < be))) {
-                bv = ov;
-                be = oe;
-            }
-        }
+        const float wgt = zs[be] * scale;
+        if (lane == (r & 63)) mine = wgt;                    // (kept until the sum is known; 64 of them at most)
         if (lane == 0) {
             ids[t * top + r] = be;
-            weights[t * top + r] = zs[be] * scale;
+            if (top > 64) weights[t * top + r] = wgt;
         }
         total += zs[be];
 #pragma unroll
         for (int j = 0; j < PL; ++j)
             if (lane + 64 * j == be) taken[j] = true;
     }
-    if (renorm && lane == 0)
+    if (top <= 64) {
+        if (lane < top) weights[t * top + lane] = renorm ? mine / (total + 1e-20f) : mine;
+    } else if (renorm && lane == 0) {
         for (int r = 0; r < top; ++r) weights[t * top + r] = weights[t * top + r] / (total + 1e-20f);
+    }
 }
 
 // One workgroup: counts per expert, block starts, then every pair takes the next free position of its expert's block.
@@ -467,8 +488,18 @@ extern "C" int32_t nvh_moe_route_linear(const void* x, int64_t x_row_stride, con
     const dim3 grid((unsigned)num_tokens);
     hipStream_t st = (hipStream_t)stream;
     const int vec = K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
-    if (act_f32) moe_route_linear_kernel<float><<<grid, 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, (const float*)bias, ids, weights, logits_out, (int)experts, (int)K, (int)top, vec, sigmoid_scores);
-    else moe_route_linear_kernel<bf16><<<grid, 256, 0, st>>>((const bf16*)x, x_row_stride, (const bf16*)w, (const bf16*)bias, ids, weights, logits_out, (int)experts, (int)K, (int)top, vec, sigmoid_scores);
+#define NVH_ROUTE_LINEAR(A, PL) moe_route_linear_kernel<A, PL><<<grid, 256, 0, st>>>((const A*)x, x_row_stride, (const A*)w, (const A*)bias, ids, weights, logits_out, (int)experts, (int)K, (int)top, vec, sigmoid_scores)
+    if (experts <= 64) {
+        if (act_f32) NVH_ROUTE_LINEAR(float, 1);
+        else NVH_ROUTE_LINEAR(bf16, 1);
+    } else if (experts <= 256) {
+        if (act_f32) NVH_ROUTE_LINEAR(float, 4);
+        else NVH_ROUTE_LINEAR(bf16, 4);
+    } else {
+        if (act_f32) NVH_ROUTE_LINEAR(float, ROUTE_MAX_PER_LANE);
+        else NVH_ROUTE_LINEAR(bf16, ROUTE_MAX_PER_LANE);
+    }
+#undef NVH_ROUTE_LINEAR
     NVH_CHECK_LAUNCH("nvh_moe_route_linear");
     return NVH_OK;
 }
