@@ -415,6 +415,226 @@ __global__ __launch_bounds__(256) void gemm_grouped_bf16_kernel(GroupedArgs a) {
     nvh_any::gemm_any_bf16_tile<OUT_F32>((const bf16*)a.x, a.ldx, w, a.K, nullptr, a.y, a.ldy, rm, n0, a.N, a.K, a.vec_ok, nullptr, 0, a.relu2);
 }
 
+// Wait until at most `ahead` steps (PW loads of this wave each) are still on their way.
+template <int PW, int MOST>
+__device__ __forceinline__ void wait_steps_in_flight(int ahead) {
+    if constexpr (MOST == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+        static_assert(PW * MOST < 64, "vmcnt is six bits");
+        if (ahead >= MOST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PW * MOST) : "memory");
+        else wait_steps_in_flight<PW, MOST - 1>(ahead);
+    }
+}
+
+// The same product where experts have many rows (bf16, K a multiple of 64): tiles of 128 rows - two neighbouring tiles of the list - by 128 columns,
+// four waves of 64 x 64, two workgroups a CU, operands brought to LDS by 16-byte LDS-DMA a k-step ahead.  What bounds both forms is the operands' way from L2 to LDS, and a 128 x 128 tile needs half of what four 64 x 64 tiles take; sums in the
+// same order, bit for bit the same results.
+// us at 16 experts, the general 64 x 64 tiles, the tiles for few rows below and this one, rows an expert x N x K: 126 x 1536 x 1024 35.0, 24.2,
+// 25.3; 250 x 1536 x 1024 51.5, 38.4, 35.1 (360 TFLOP/s); 250 x 1024 x 768 32.9, 21.5, 19.0; 500 x 1536 x 1024 85, 65, 49; 126 x 1024 x 384
+// 17.2, 9.4, 12.3.  Tried and slower at these sizes: eight waves and three stages with one workgroup a CU (a grid is seldom whole rounds),
+// stages of 32 k four ahead.
+constexpr int TALL = 128;
+
+// Whether tile `t` of the list goes on where tile t - 1, a full one, of the same expert ends.
+__device__ __forceinline__ bool tile_goes_on(const GroupedArgs& a, int t) {
+    return a.tile_expert[t] == a.tile_expert[t - 1] && a.tile_rows[t - 1] == nvh_any::GT && a.tile_row0[t] == a.tile_row0[t - 1] + nvh_any::GT;
+}
+
+// Four consecutive columns of an output row, finished.
+template <bool OUT_F32>
+__device__ __forceinline__ void store_grouped(const GroupedArgs& a, int64_t m, int n, f32x4 v) {
+    if (a.relu2) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = fmaxf(v[e], 0.f);
+            v[e] *= v[e];
+        }
+    }
+    if constexpr (OUT_F32) {
+        *reinterpret_cast<f32x4*>((float*)a.y + m * a.ldy + n) = v;
+    } else {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)v[e];
+        *reinterpret_cast<bf16x4*>((bf16*)a.y + m * a.ldy + n) = o;
+    }
+}
+
+template <bool OUT_F32>
+__global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedArgs a, int max_tiles, int tiles_n) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    // Workgroup ids go round the XCDs: two neighbouring list tiles with all their columns fall to one, so a row is fetched into one L2.
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int t = 2 * ((slot / (2 * tiles_n)) * 8 + xcd) + (slot / tiles_n & 1), n0 = slot % tiles_n * TALL;
+    if (t >= max_tiles) return;
+    int rows = a.tile_rows[t];
+    if (rows <= 0) return;                                   // (uniform: a tile beyond the list's end)
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // How many tiles before this one belong to the same run of rows: an odd one was taken by its predecessor.
+    int before = 0;
+    for (int base = t; base > 0; base -= 64) {
+        const int at = base - lane;
+        const unsigned long long run = __ballot(at > 0 && tile_goes_on(a, max(at, 1)));
+        const int n = run == ~0ull ? 64 : __builtin_ctzll(~run);
+        before += n;
+        if (n < 64) break;
+    }
+    if (before & 1) return;
+    const int expert = a.tile_expert[t], row0 = a.tile_row0[t];
+    if (t + 1 < max_tiles && a.tile_rows[t + 1] > 0 && tile_goes_on(a, t + 1)) rows += a.tile_rows[t + 1];
+    const int N = a.N, K = a.K;
+    const bf16 *x = (const bf16*)a.x, *w = (const bf16*)a.w + (int64_t)expert * N * K;
+    // LDS per stage: 128 rows of w, then 128 of x, 64 k (128 bytes) each; 16-byte piece c of row r lies at place c ^ ((r >> 1) & 7), which spreads a
+    // fragment read over all banks.  A DMA instruction brings 8 rows: a wave's are pieces wave, wave + 4, ...
+    constexpr int STAGE = 2 * TALL * 128, PW = 2 * TALL / 8 / 4;
+    const bf16* src[PW];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int p = wave + 4 * i, r = (p & 15) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
+        if (p < 16) {
+            src[i] = w + (int64_t)min(n0 + r, N - 1) * K + chunk * 8;
+        } else {                                             // (rows beyond the tile's repeat its last: not written)
+            const int at = row0 + min(r, rows - 1);
+            src[i] = x + (int64_t)(a.gather ? a.gather[at] : at) * a.ldx + chunk * 8;
+        }
+    }
+    const int steps = K / 64;
+    auto stage = [&](int step) {
+        char* base = smem + (step & 1) * STAGE;
+#pragma unroll
+        for (int i = 0; i < PW; ++i)
+            __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)(src[i] + step * 64), (LDS_AS void*)(base + (wave + 4 * i) * 1024), 16, 0, 0);
+    };
+    const int wn = (wave & 1) * 64, wm = (wave >> 1) * 64, fr = lane & 15, fq = lane >> 4;
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    stage(0);
+    for (int step = 0; step < steps; ++step) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's pieces of the step
+        __builtin_amdgcn_s_barrier();                        // everybody's; and everybody has left the stage that is filled next
+        asm volatile("" ::: "memory");
+        if (step + 1 < steps) stage(step + 1);
+        const char *ws = smem + (step & 1) * STAGE, *xs = ws + TALL * 128;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            bf16x8 wf[4], xf[4];
+            const int kc = ks * 4 + fq;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = wn + 16 * i + fr;
+                wf[i] = *reinterpret_cast<const bf16x8*>(ws + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = wm + 16 * j + fr;
+                xf[j] = *reinterpret_cast<const bf16x8*>(xs + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // a lane holds, for weight tile i and row tile j: row wm + 16 j + fr, columns wn + 16 i + 4 fq + e (N a multiple of 4)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int r = wm + 16 * j + fr;
+        if (r >= rows) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = n0 + wn + 16 * i + 4 * fq;
+            if (n < N) store_grouped<OUT_F32>(a, row0 + r, n, acc[i][j]);
+        }
+    }
+}
+
+template <bool OUT_F32>
+static bool launch_grouped_tall(const GroupedArgs& a, int64_t max_tiles, hipStream_t st) {
+    const int64_t tiles_n = nvh_cdiv(a.N, TALL), slots = nvh_cdiv(max_tiles, 16) * 16 * tiles_n;
+    constexpr int lds = 2 * 2 * TALL * 128;
+    if (slots >= (1ll << 31)) return false;
+    gemm_grouped_tall_bf16_kernel<OUT_F32><<<dim3((unsigned)slots), 256, lds, st>>>(a, (int)max_tiles, (int)tiles_n);
+    return true;
+}
+
+// A list tile of at most 16 MT rows by 64 columns (K a multiple of 64, N of 4): a wave's 16 columns and all rows, operands through a ring of LDS
+// stages of 64 k each, filled by 16-byte LDS-DMA all stages but one ahead.  What it waits for is the weights' stream.  us at 16 experts, the general
+// tiles (operands through registers, or straight from memory for few rows) and this one, rows an expert x N x K: 1 x 1536 x 1024 10.2 and 7.4,
+// 16 x 1536 x 1024 23.8 and 13.6 (3.7 TB/s), 8 x 768 x 1024 11.2 and 7.1, 16 x 1024 x 768 11.7 and 6.7, 64 x 1536 x 1024 26.4 and 18.2.
+constexpr int SHORT_N = 64, SHORT_LDS = 64 * 1024;
+template <bool OUT_F32, int MT>
+__device__ __forceinline__ void gemm_grouped_short_tile(const GroupedArgs& a, int expert, int row0, int rows, int n0, char* smem) {
+    constexpr int STAGE = (SHORT_N + 16 * MT) * 128, STAGES = SHORT_LDS / STAGE, AHEAD = STAGES - 1;
+    constexpr int PIECES = SHORT_N / 8 + 2 * MT, PW = (PIECES + 3) / 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int N = a.N, K = a.K;
+    const bf16 *x = (const bf16*)a.x, *w = (const bf16*)a.w + (int64_t)expert * N * K;
+    // (LDS rows and places as in the tall form; pieces 0 .. 7 are w's, then x's; a wave without a last piece of its own brings the first ones once more)
+    const bf16* src[PW];
+    int off[PW];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+        const int p = (wave + 4 * i) % PIECES, r = (p < 8 ? p : p - 8) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
+        if (p < 8) {
+            src[i] = w + (int64_t)min(n0 + r, N - 1) * K + chunk * 8;
+        } else {
+            const int at = row0 + min(r, rows - 1);
+            src[i] = x + (int64_t)(a.gather ? a.gather[at] : at) * a.ldx + chunk * 8;
+        }
+        off[i] = p * 1024;
+    }
+    const int steps = K / 64, fr = lane & 15, fq = lane >> 4;
+    auto stage = [&](int step) {
+        char* base = smem + step % STAGES * STAGE;
+#pragma unroll
+        for (int i = 0; i < PW; ++i)
+            __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)(src[i] + step * 64), (LDS_AS void*)(base + off[i]), 16, 0, 0);
+    };
+    f32x4 acc[MT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int step = 0; step < AHEAD && step < steps; ++step) stage(step);
+    for (int step = 0; step < steps; ++step) {
+        wait_steps_in_flight<PW, AHEAD - 1>(min(AHEAD - 1, steps - 1 - step));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (step + AHEAD < steps) stage(step + AHEAD);       // (into the stage that everybody left before this barrier)
+        const char *ws = smem + step % STAGES * STAGE, *xs = ws + SHORT_N * 128;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int kc = ks * 4 + fq, rw = wave * 16 + fr;
+            const bf16x8 wf = *reinterpret_cast<const bf16x8*>(ws + rw * 128 + ((kc ^ ((rw >> 1) & 7)) << 4));
+#pragma unroll
+            for (int j = 0; j < MT; ++j) {
+                const int r = 16 * j + fr;
+                const bf16x8 xf = *reinterpret_cast<const bf16x8*>(xs + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf, acc[j], 0, 0, 0);
+            }
+        }
+    }
+    const int n = n0 + wave * 16 + 4 * fq;
+    if (n >= N) return;
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+        if (16 * j + fr < rows) store_grouped<OUT_F32>(a, row0 + 16 * j + fr, n, acc[j]);
+}
+
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void gemm_grouped_short_bf16_kernel(GroupedArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int rows = a.tile_rows[blockIdx.y];
+    if (rows <= 0) return;                                   // (uniform: a tile beyond the list's end)
+    const int expert = a.tile_expert[blockIdx.y], row0 = a.tile_row0[blockIdx.y], n0 = blockIdx.x * SHORT_N;
+    if (rows <= 16) gemm_grouped_short_tile<OUT_F32, 1>(a, expert, row0, rows, n0, smem);
+    else if (rows <= 32) gemm_grouped_short_tile<OUT_F32, 2>(a, expert, row0, rows, n0, smem);
+    else gemm_grouped_short_tile<OUT_F32, 4>(a, expert, row0, rows, n0, smem);
+}
+
 // (a tile of the list is 64 rows: blockIdx.z is its upper or lower half)
 __global__ __launch_bounds__(256) void gemm_grouped_f32_kernel(GroupedArgs a) {
     const int rows = a.tile_rows[blockIdx.y], r0 = blockIdx.z * 32;
@@ -548,9 +768,9 @@ extern "C" int32_t nvh_moe_align(const int32_t* ids, int64_t num_tokens, int64_t
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
-                                           const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
-                                           int64_t N, int64_t K, int32_t relu2, int32_t in_f32, int32_t out_f32, nvh_stream_t stream) {
+static int32_t grouped_product(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
+                               const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
+                               int64_t N, int64_t K, int32_t relu2, int32_t in_f32, int32_t out_f32, int32_t tall, nvh_stream_t stream) {
     NVH_REQUIRE(x && w && y && tile_expert && tile_row0 && tile_rows, NVH_EINVAL, "nvh_gemm_grouped_any_nt: null pointer");
     NVH_REQUIRE(max_tiles >= 0 && max_tiles < 65536 && N > 0 && K > 0 && N < (1 << 30) && K < (1 << 30) && x_row_stride >= K && y_row_stride >= N, NVH_EINVAL,
                 "nvh_gemm_grouped_any_nt: bad sizes");
@@ -560,11 +780,31 @@ extern "C" int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, 
     const GroupedArgs a{x, x_row_stride, gather, w, y, y_row_stride, tile_expert, tile_row0, tile_rows, (int)N, (int)K, vec_ok, relu2};
     const dim3 grid((unsigned)nvh_cdiv(N, nvh_any::GT), (unsigned)max_tiles);
     hipStream_t st = (hipStream_t)stream;
+    if (!in_f32 && vec_ok && K % 64 == 0 && N % 4 == 0 && y_row_stride % 4 == 0 && nvh_aligned16(y)) {
+        if (!(tall && (out_f32 ? launch_grouped_tall<true>(a, max_tiles, st) : launch_grouped_tall<false>(a, max_tiles, st)))) {
+            if (out_f32) gemm_grouped_short_bf16_kernel<true><<<grid, 256, SHORT_LDS, st>>>(a);
+            else gemm_grouped_short_bf16_kernel<false><<<grid, 256, SHORT_LDS, st>>>(a);
+        }
+        NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");
+        return NVH_OK;
+    }
     if (in_f32) gemm_grouped_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)max_tiles, 2), 256, 0, st>>>(a);
     else if (out_f32) gemm_grouped_bf16_kernel<true><<<grid, 256, 0, st>>>(a);
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");
     return NVH_OK;
+}
+
+extern "C" int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
+                                           const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
+                                           int64_t N, int64_t K, int32_t relu2, int32_t in_f32, int32_t out_f32, nvh_stream_t stream) {
+    return grouped_product(x, x_row_stride, gather, w, y, y_row_stride, tile_expert, tile_row0, tile_rows, max_tiles, N, K, relu2, in_f32, out_f32, 0, stream);
+}
+
+extern "C" int32_t nvh_gemm_grouped_many_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
+                                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
+                                            int64_t N, int64_t K, int32_t relu2, int32_t in_f32, int32_t out_f32, nvh_stream_t stream) {
+    return grouped_product(x, x_row_stride, gather, w, y, y_row_stride, tile_expert, tile_row0, tile_rows, max_tiles, N, K, relu2, in_f32, out_f32, 1, stream);
 }
 
 extern "C" int32_t nvh_glu_clamp_pairs(const void* gate_up, int64_t row_stride, const int32_t* pos_of_pair, const float* weights, void* y, int64_t y_stride,

@@ -5,6 +5,34 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("out_f32,act", [(False, None), (True, None), (False, "relu2")])
+@pytest.mark.parametrize("n,k", [(4, 64), (60, 128), (64, 192), (132, 448), (200, 1024)])
+def test_blocks_of_every_size(n, k, out_f32, act):
+    """Experts without a row, with one, around 16, 32, 64, 128 and 192 rows and more than 64 tiles' worth: tiles of few rows, pairs of tiles, a pair's
+    odd last tile.  The reference reads rows that no 16-byte load may be used on, which takes the general form."""
+    from nanovllm import ops
+    sizes = [0, 1, 15, 16, 17, 32, 33, 64, 65, 127, 128, 129, 192, 0, 4200]
+    g = torch.Generator().manual_seed(n + k)
+    ids = torch.repeat_interleave(torch.arange(len(sizes)), torch.tensor(sizes))[torch.randperm(sum(sizes), generator=g)].int()[:, None].cuda()
+    T = ids.shape[0]
+    x = torch.randn(T, k, generator=g).bfloat16().cuda()
+    w = (torch.randn(len(sizes), n, k, generator=g) * 0.1).bfloat16().cuda()
+    plan = ops.moe_align(ids, len(sizes))
+    at = plan["pos_of_pair"].long()
+    odd = torch.empty(T, k + 1, dtype=x.dtype, device=x.device)
+    odd[:, :k] = x
+    want = ops.linear_grouped(odd[:, :k], w, plan, True, out_f32, act)[at]
+    default = ops.GROUPED_MANY_ROWS
+    try:
+        for few in (1 << 30, 0):                             # the tiles for few rows an expert, and those for many
+            ops.GROUPED_MANY_ROWS = few
+            assert torch.equal(ops.linear_grouped(x, w, plan, True, out_f32, act)[at], want)
+            rows = x[plan["src_token"].long()]
+            assert torch.equal(ops.linear_grouped(rows, w, plan, False, out_f32, act)[at], want)
+    finally:
+        ops.GROUPED_MANY_ROWS = default
+
+
 @pytest.mark.parametrize("experts,top,k", [(1, 1, 8), (3, 2, 1000), (16, 4, 1024), (64, 64, 1536), (65, 7, 520), (300, 80, 2048)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_routing(experts, top, k, dtype):
