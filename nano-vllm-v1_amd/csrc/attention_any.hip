@@ -161,6 +161,188 @@ __global__ __launch_bounds__(256) void attn_rotary_prep_kernel(PrepArgs a) {
         for (int h = threadIdx.x; h < a.H; h += 256) a.gate_out[t * a.H + h] = 1.0f / (1.0f + expf(-ldf(vr + nv, h)));
 }
 
+// The same with eight consecutive elements per lane and 16-byte accesses (head sizes and rotated dimensions that keep a piece of eight on one side
+// of a rotation, aligned rows).  A token's workgroup requests everything it reads at once - its pieces, their rotation partners, the weights of
+// both - and the sines and cosines of a position are formed once for all heads.  Values: piece by piece beside q and k (`v_tiles` 0), or, for many
+// tokens, by workgroups of their own behind the tokens' (64 tokens by 64 columns, turned in LDS, so that tokens that lie side by side in a page leave
+// as one cache line).
+// us, the form above and this one, 16 + 8 heads of 128 x 128: 1000 tokens 24.6 and 9.3, 64 tokens 17.1 and 8.1.
+constexpr int PREP_PAIRS = 128;                              // rotation pairs of a head at most
+constexpr int PREP_TILE_TOKENS = 128;                       // tokens from which values go by tiles
+constexpr int VT = 64;                                       // tokens and columns of a value tile
+template <typename A, int J>
+__global__ __launch_bounds__(256) void attn_rotary_prep_vec_kernel(PrepArgs a, int64_t tokens, int v_tiles) {
+    __shared__ float smem[VT * (VT + 1)];                    // a value tile, or: sums per piece (256 J), cosines, sines, partial sums of the rows
+    const int nq = a.H * a.dim, nk = a.G * a.dim, nv = a.G * a.vdim, tid = threadIdx.x;
+    // v: eight values of a row from column c on, turned by the token's position
+    auto turned = [&](const A* vr, int c, float pos, float (&x)[8]) {
+        nvh_load8(vr, c, 8, 1, x);
+        if (!a.v_freq) return;
+        const int d = c % a.vdim, half = a.vdim >> 1;
+        float o[8];
+        if (!a.v_interleaved) nvh_load8(vr, d < half ? c + half : c - half, 8, 1, o);
+        float y[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            int partner, pair;
+            bool first;
+            pair_of(d + e, a.vdim, a.v_interleaved, partner, pair, first);
+            const float other = a.v_interleaved ? x[e ^ 1] : o[e];
+            float sn, cs;
+            rot_sincos<A>(pos * a.v_freq[pair], sn, cs);
+            y[e] = first ? x[e] * cs - other * sn : x[e] * cs + other * sn;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = y[e];
+    };
+    if ((int64_t)blockIdx.x >= tokens) {                     // (uniform) a value tile
+        const int tile = (int)(blockIdx.x - tokens), c0 = tile % v_tiles * VT;
+        const int64_t t0 = (int64_t)(tile / v_tiles) * VT;
+#pragma unroll
+        for (int j = 0; j < VT * VT / 8 / 256; ++j) {
+            const int i = tid + 256 * j, r = i >> 3, c = c0 + ((i & 7) << 3);
+            const int64_t t = min(t0 + r, tokens - 1);
+            if (c < nv) {
+                float x[8];
+                turned((const A*)a.proj + t * a.ld + nq + nk, c, (float)a.positions[t], x);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) smem[r * (VT + 1) + c - c0 + e] = x[e];
+            }
+        }
+        __syncthreads();
+        const int r = tid & (VT - 1);
+        const int64_t slot = t0 + r < tokens ? a.slot_mapping[t0 + r] : -1;
+        if (slot < 0) return;
+        A* dst = (A*)a.v_cache + (slot / a.page) * a.page * nv + slot % a.page;
+#pragma unroll
+        for (int j = 0; j < VT / 4; ++j) {
+            const int c = (tid >> 6) + 4 * j;
+            if (c0 + c < nv) dst[(int64_t)(c0 + c) * a.page] = (A)smem[r * (VT + 1) + c];
+        }
+        return;
+    }
+    const int64_t t = blockIdx.x;
+    const A* row = (const A*)a.proj + t * a.ld;
+    const int64_t slot = a.slot_mapping ? a.slot_mapping[t] : -1;
+    const float pos = (float)a.positions[t];
+    const int pieces = (nq + nk) >> 3, half = a.rot_dims >> 1, per_head = a.dim >> 3;
+    float *sums = smem, *cosines = smem + 256 * J, *sines = cosines + PREP_PAIRS, *red = sines + PREP_PAIRS;
+    const bool normed = a.q_norm != nullptr;
+    float x[J][8], o[J][8], w[J][8], wo[J][8];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int c = min(tid + 256 * j, pieces - 1) << 3, d = c % a.dim;          // (q and k adjoin; pieces past the last repeat it)
+        const int to = d >= a.rot_dims || a.qk_interleaved ? 0 : (d < half ? half : -half);
+        nvh_load8(row, c, 8, 1, x[j]);
+        if (!a.qk_interleaved) nvh_load8(row, c + to, 8, 1, o[j]);
+        if (normed) {
+            const A* wn = (const A*)(c < nq ? a.q_norm : a.k_norm);
+            const int at = a.norm_per_head ? d : (c < nq ? c : c - nq);
+            nvh_load8(wn, at, 8, 1, w[j]);
+            if (!a.qk_interleaved) nvh_load8(wn, at + to, 8, 1, wo[j]);
+        }
+    }
+    for (int i = tid; i < half; i += 256) {
+        float sn, cs;
+        rot_sincos<A>(pos * a.qk_freq[i], sn, cs);
+        cosines[i] = cs * a.qk_mag;
+        sines[i] = sn * a.qk_mag;
+    }
+    float sq = 0.f, sk = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int i = tid + 256 * j;
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += x[j][e] * x[j][e];
+        sums[i] = ss;
+        if (i < pieces) (i << 3 < nq ? sq : sk) += ss;
+    }
+    if (normed && !a.norm_per_head) {                        // (uniform)
+        sq = wave_sum(sq);
+        sk = wave_sum(sk);
+        if ((tid & 63) == 0) {
+            red[tid >> 6] = sq;
+            red[4 + (tid >> 6)] = sk;
+        }
+    }
+    __syncthreads();
+    const float inv_q = normed && !a.norm_per_head ? 1.0f / sqrtf((red[0] + red[1] + red[2] + red[3]) / (float)nq + a.eps) : 1.f;
+    const float inv_k = normed && !a.norm_per_head ? 1.0f / sqrtf((red[4] + red[5] + red[6] + red[7]) / (float)nk + a.eps) : 1.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int i = tid + 256 * j, c = i << 3, d = c % a.dim;
+        if (i >= pieces) break;
+        const bool is_k = c >= nq;
+        if (normed) {
+            float rinv = is_k ? inv_k : inv_q;
+            if (a.norm_per_head) {
+                const float* hs = sums + i / per_head * per_head;
+                float ss = 0.f;
+                for (int p = 0; p < per_head; ++p) ss += hs[p];
+                rinv = 1.0f / sqrtf(ss / (float)a.dim + a.eps);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                x[j][e] = x[j][e] * rinv * w[j][e];
+                if (!a.qk_interleaved) o[j][e] = o[j][e] * rinv * wo[j][e];
+            }
+        }
+        A out[8];
+        if (d < a.rot_dims) {
+            const bool first = d < half;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int pair = a.qk_interleaved ? (d + e) >> 1 : (first ? d + e : d + e - half);
+                const float cs = cosines[pair], sn = sines[pair];
+                if (a.qk_interleaved) out[e] = (A)(e & 1 ? x[j][e] * cs + x[j][e ^ 1] * sn : x[j][e] * cs - x[j][e ^ 1] * sn);
+                else out[e] = (A)(first ? x[j][e] * cs - o[j][e] * sn : x[j][e] * cs + o[j][e] * sn);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out[e] = (A)x[j][e];
+        }
+        if (!is_k) __builtin_memcpy(__builtin_assume_aligned((A*)a.q_out + t * nq + c, 16), out, sizeof(out));
+        else if (slot >= 0 && a.k_cache) __builtin_memcpy(__builtin_assume_aligned((A*)a.k_cache + slot * nk + (c - nq), 16), out, sizeof(out));
+    }
+    const A* vr = row + nq + nk;
+    if (v_tiles == 0 && slot >= 0 && a.v_cache) {
+        A* dst = (A*)a.v_cache + (slot / a.page) * a.page * nv + slot % a.page;      // element i of the row goes to dst[i * page]
+        for (int i = 255 - tid; i < nv >> 3; i += 256) {     // (from the last lane down: the first ones have more pieces of q and k)
+            float v[8];
+            turned(vr, i << 3, pos, v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dst[(int64_t)((i << 3) + e) * a.page] = (A)v[e];
+        }
+    }
+    if (a.gate_out)
+        for (int h = tid; h < a.H; h += 256) a.gate_out[t * a.H + h] = 1.0f / (1.0f + expf(-ldf(vr + nv, h)));
+}
+
+// Whether attn_rotary_prep_vec_kernel takes the call: pieces of eight that lie on one side of every rotation, and aligned.
+template <typename A>
+static bool prep_vec_ok(const PrepArgs& a) {
+    const int per16 = 16 / (int)sizeof(A);
+    const auto rotates = [](int n, int interleaved) { return n % (interleaved ? 8 : 16) == 0; };
+    return a.dim % 8 == 0 && a.vdim % 8 == 0 && rotates(a.rot_dims, a.qk_interleaved) && a.rot_dims <= 2 * PREP_PAIRS &&
+           (!a.v_freq || rotates(a.vdim, a.v_interleaved)) && (a.H + a.G) * a.dim <= 8 * 256 * 4 && a.ld % per16 == 0 && nvh_aligned16(a.proj) &&
+           nvh_aligned16(a.q_out) && (!a.k_cache || nvh_aligned16(a.k_cache)) && (!a.q_norm || (nvh_aligned16(a.q_norm) && nvh_aligned16(a.k_norm)));
+}
+
+template <typename A>
+static void launch_rotary_prep(const PrepArgs& a, int64_t tokens, size_t lds, hipStream_t st) {
+    if (!prep_vec_ok<A>(a)) {
+        attn_rotary_prep_kernel<A><<<dim3((unsigned)tokens), 256, lds, st>>>(a);
+        return;
+    }
+    const int nv = a.G * a.vdim, pieces = (a.H + a.G) * a.dim / 8;
+    const int v_tiles = tokens >= PREP_TILE_TOKENS && a.v_cache && a.slot_mapping ? (int)nvh_cdiv(nv, VT) : 0;
+    const dim3 grid((unsigned)(tokens + nvh_cdiv(tokens, VT) * v_tiles));
+    if (pieces <= 256) attn_rotary_prep_vec_kernel<A, 1><<<grid, 256, 0, st>>>(a, tokens, v_tiles);
+    else if (pieces <= 512) attn_rotary_prep_vec_kernel<A, 2><<<grid, 256, 0, st>>>(a, tokens, v_tiles);
+    else attn_rotary_prep_vec_kernel<A, 4><<<grid, 256, 0, st>>>(a, tokens, v_tiles);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int AQ = 16;        // queries per workgroup (one 16-lane row of a wave per query)
 constexpr int AK = 32;        // keys per tile
@@ -1403,8 +1585,8 @@ extern "C" int32_t nvh_attn_rotary_prep(const void* proj, int64_t proj_row_strid
     hipStream_t st = (hipStream_t)stream;
     const size_t lds = norm_per_head ? sizeof(float) * (size_t)(num_q_heads + num_kv_heads) : 0;
     NVH_REQUIRE(lds <= 32 * 1024, NVH_ENOSYS, "nvh_attn_rotary_prep: %ld heads above the per-head norm's limit", (long)(num_q_heads + num_kv_heads));
-    if (act_f32) attn_rotary_prep_kernel<float><<<dim3((unsigned)num_tokens), 256, lds, st>>>(a);
-    else attn_rotary_prep_kernel<bf16><<<dim3((unsigned)num_tokens), 256, lds, st>>>(a);
+    if (act_f32) launch_rotary_prep<float>(a, num_tokens, lds, st);
+    else launch_rotary_prep<bf16>(a, num_tokens, lds, st);
     NVH_CHECK_LAUNCH("nvh_attn_rotary_prep");
     return NVH_OK;
 }
