@@ -382,6 +382,7 @@ struct AttnArgs {
     int kv_split;              // one-query form: workgroups per (sequence, KV head), each with H / (G kv_split) of the group's heads
     int key_parts;             // one-query form: workgroups that share a sequence's key tiles (tile j goes to part j % key_parts); > 1: the
     float* parts;              // parts leave [batch, G kv_split, key_parts, 16, vdim + 2] (unnormalised rows, then max and sum) here
+    int balance;               // one-query form: sequences are dealt out by their length (balanced_place)
 };
 
 // The key tiles (of `tile` keys, starting at multiples of it) that a workgroup whose first query sits at position qlo has to
@@ -859,6 +860,39 @@ constexpr int MQ = 64, MK = 64;
 // VAR: the plain variant, the one with pooled blocks, softcap and query temperature, or the one with a learned distance bias (none
 // carries code of the others).
 enum AttnVariant { VAR_PLAIN, VAR_EXT, VAR_BIAS };
+// One query per sequence: which sequence and group of heads a workgroup takes.  All workgroups of a step fit the chip a few to a CU, the ones numbered
+// L and L + 256 beside each other, and as they lie that gives a CU the same long sequence twice.  So the work is dealt out by length: the
+// longest sequences to the first 256 workgroups, the next ones to the next 256 in the opposite order, and so on.  Every workgroup ranks the
+// sequences (at most 256) for itself; a result does not depend on where it is computed.
+// us, as they lay and dealt out, 64 sequences of 512 .. 1535 keys, 8 KV heads: 128 x 128 51.2 and 46.3 in one model, 75.3 and 67.7 in another, with a
+// query temperature or pooled blocks 54.5 and 49.2; 128 x 64 58.0 and 52.2; 64 x 128 72.8 and 69.7.
+constexpr int BALANCE_MAX = 256;
+__device__ __forceinline__ void balanced_place(const AttnArgs& a, int* keys, int& seq, int& by) {
+    const int tid = threadIdx.x, total = gridDim.x * gridDim.y, L = blockIdx.x + gridDim.x * blockIdx.y;
+    const int round = L >> 8, in_round = min(256, total - 256 * round), at = L & 255;
+    const int item = 256 * round + (round & 1 ? in_round - 1 - at : at), want = item / (int)gridDim.y;
+    int len = 0;                                             // keys that the sequence's query sees (roughly: what counts is the order)
+    if (tid < a.batch) {
+        len = a.context_lens[tid];
+        if (a.chunk > 0) len = len > 0 ? (len - 1) % a.chunk + 1 : 0;
+        if (a.window > 0) len = min(len, a.window + a.keep_first);
+    }
+    const int key = tid < a.batch ? (len << 8 | (255 - tid)) : -1;
+    keys[tid] = key;
+    __syncthreads();
+    int rank = 0;
+    for (int j = 0; j < a.batch; j += 4) {                   // (four at a time: behind the batch lie the -1 of the lanes without a sequence)
+        const int4 other = *reinterpret_cast<const int4*>(keys + j);
+        rank += (other.x > key) + (other.y > key) + (other.z > key) + (other.w > key);
+    }
+    __syncthreads();
+    if (tid < a.batch && rank == want) keys[0] = tid;
+    __syncthreads();
+    seq = __builtin_amdgcn_readfirstlane(keys[0]);
+    by = item - want * (int)gridDim.y;
+    __syncthreads();                                         // (the place is used for other things from here on)
+}
+
 template <int NKS, int NVT, bool EXACT, int MODE, int VAR>
 __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     constexpr bool GROUPED = MODE == 1;                      // rows are the heads of a KV group (one query per sequence)
@@ -866,8 +900,12 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     constexpr bool SPLIT = MODE != 0;                        // the waves share 16 rows and split the keys
     constexpr int ROWS_Q = MQ;                               // queries per workgroup
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    int seq = -1, q0 = 0, qlen = 0, qbase = 0;
-    if (!a.cu_seqlens_q) {                                   // one query per sequence
+    int seq = -1, q0 = 0, qlen = 0, qbase = 0, by = blockIdx.y;
+    if (GROUPED && a.balance) {                              // (uniform)
+        balanced_place(a, reinterpret_cast<int*>(smem_raw), seq, by);
+        qbase = seq;
+        qlen = 1;
+    } else if (!a.cu_seqlens_q) {                            // one query per sequence
         if ((int)blockIdx.x < a.batch) {
             seq = qbase = blockIdx.x;
             qlen = 1;
@@ -889,10 +927,10 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     }
     if (seq < 0) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fr = lane & 15, fq = lane >> 4;
-    // GROUPED: blockIdx.y counts (KV head, part of its group of heads); the parts of one KV head read the same keys and values
+    // GROUPED: `by` counts (KV head, part of its group of heads); the parts of one KV head read the same keys and values
     const int group = GROUPED ? a.H / (a.G * a.kv_split) : a.H / a.G;
-    const int kvh = GROUPED ? blockIdx.y / a.kv_split : blockIdx.y / group;
-    const int head = GROUPED ? blockIdx.y * group + min(fr, group - 1) : blockIdx.y;       // (GROUPED: this lane's row is a head)
+    const int kvh = GROUPED ? by / a.kv_split : by / group;
+    const int head = GROUPED ? by * group + min(fr, group - 1) : by;       // (GROUPED: this lane's row is a head)
     const int dim = EXACT ? 16 * NKS : a.dim, vdim = EXACT ? 16 * NVT : a.vdim, nks = dim >> 4, nvt = vdim >> 4;
     const int klen = a.context_lens[seq], past = klen - qlen;
     const int nq = GROUPED ? 1 : min(ROWS_Q, qlen - q0);
@@ -909,7 +947,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     const int last_key = past + q0 + nq - 1;
     const int part = GROUPED ? (int)blockIdx.z : 0, nparts = GROUPED ? a.key_parts : 1;
     float* prow = nullptr;                                   // this workgroup's record among the parts
-    if (GROUPED && nparts > 1) prow = a.parts + (((int64_t)seq * gridDim.y + blockIdx.y) * nparts + part) * 16 * (vdim + 2);
+    if (GROUPED && nparts > 1) prow = a.parts + (((int64_t)seq * gridDim.y + by) * nparts + part) * 16 * (vdim + 2);
     if (last_key < 0 && prow) {                              // a padded row: every part records "no keys", the merge then writes zeros
         if (tid < 16) {
             prow[tid * (vdim + 2) + vdim] = -INFINITY;
@@ -921,7 +959,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         for (int i = tid; i < nrows * vdim; i += 256) {
             const int r = i / vdim;
             const int64_t tok = GROUPED ? qbase : qbase + q0 + r;
-            const int hd = GROUPED ? (int)blockIdx.y * group + r : (int)blockIdx.y;
+            const int hd = GROUPED ? by * group + r : by;
             ((bf16*)a.out)[(tok * a.H + hd) * vdim + (i - r * vdim)] = (bf16)0.f;
         }
         return;
@@ -976,7 +1014,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     if constexpr (BIAS) {
         float* bias_s = reinterpret_cast<float*>(smem_raw + a.bias_offset);
         const int heads_here = GROUPED ? group : 1;
-        const float* src = a.bias + (int64_t)(GROUPED ? (int)blockIdx.y * group : head) * a.bias_len;
+        const float* src = a.bias + (int64_t)(GROUPED ? by * group : head) * a.bias_len;
         for (int i = tid; i < heads_here * a.bias_ld; i += 256) {
             const int r = i / a.bias_ld, d = i - r * a.bias_ld - 3;
             bias_s[i] = src[(int64_t)r * a.bias_len + min(max(d, 0), a.bias_len - 1)];
@@ -1244,7 +1282,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         for (int i = tid; i < nrows * pieces; i += 256) {
             const int r = i / pieces, c = (i - r * pieces) << 3;
             const int64_t tok = GROUPED ? qbase : qbase + q0 + r;
-            const int hd = GROUPED ? (int)blockIdx.y * group + r : (int)blockIdx.y;
+            const int hd = GROUPED ? by * group + r : by;
             const float g = a.gate ? a.gate[tok * a.H + hd] : 1.0f;
             bf16x8 ge, out;
             if (a.gate_elems) ge = *reinterpret_cast<const bf16x8*>((const bf16*)a.gate_elems + tok * a.ld_elems + hd * vdim + c);
@@ -1264,7 +1302,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         const int r = i / half, pair = i - r * half;
         const int c1 = a.v_interleaved ? 2 * pair : pair, c2 = a.v_interleaved ? 2 * pair + 1 : pair + half;
         const int64_t tok = GROUPED ? qbase : qbase + q0 + r;
-        const int hd = GROUPED ? (int)blockIdx.y * group + r : (int)blockIdx.y;
+        const int hd = GROUPED ? by * group + r : by;
         float u = os[r * vdim + c1], v = os[r * vdim + c2];
         if (a.v_freq) {
             float sn, cs;
@@ -1362,6 +1400,8 @@ static void launch_attn_mfma(const AttnArgs& a, int64_t total_q, hipStream_t st)
     if (grouped) {
         b.kv_split = pl.split;
         b.key_parts = pl.key_parts;
+        // (one workgroup a CU or less: nothing to pair; lengths of 2^23 and more do not fit the keys)
+        b.balance = pl.key_parts == 1 && a.batch <= BALANCE_MAX && (int64_t)a.batch * a.G * pl.split > 256 && a.table_stride * a.page < (1 << 23);
         attn_paged_mfma_kernel<NKS, NVT, EXACT, 1, VAR><<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)pl.key_parts), 256, lds, st>>>(b);
         if (pl.key_parts > 1)
             attn_merge_parts_kernel<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)(group / pl.split)), 256, 0, st>>>(a.parts, pl.key_parts, group / pl.split, a.vdim, a.H, a.gate,
@@ -1623,7 +1663,7 @@ extern "C" int32_t nvh_attn_paged_any(const void* q, int64_t q_row_stride, const
     NVH_REQUIRE(q_row_stride >= num_q_heads * dim, NVH_EINVAL, "nvh_attn_paged_any: query row too short");
     AttnArgs a{q, q_row_stride, k_cache, v_cache, cu_seqlens_q, context_lens, block_tables, table_stride, (int)batch, (int)page, (int)num_q_heads,
                (int)num_kv_heads, (int)dim, (int)vdim, scale, gate, v_freq, v_interleaved, out, gate_elems, gate_elems_stride, slopes, bias, (int)bias_len, (int)window, (int)keep_first, (int)chunk, sinks, softcap, temp_coef, (int)temp_every, (int)pool, (int)pool_rows,
-               pooled_k, pooled_v, 0, 0, 0, 0, 1, 1, nullptr};
+               pooled_k, pooled_v, 0, 0, 0, 0, 1, 1, nullptr, 0};
     // at most ceil(len / AQ) tiles per sequence: total_q / AQ + batch bounds their number (surplus workgroups exit)
     const dim3 grid((unsigned)(total_q / AQ + batch), (unsigned)num_q_heads);
     hipStream_t st = (hipStream_t)stream;

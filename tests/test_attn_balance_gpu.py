@@ -1,0 +1,69 @@
+"""bf16 paged attention of any head size: one-token steps whose sequences are dealt out by length."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+PAGE = 256
+
+
+def caches(g, ctx, G, dim, vdim):
+    pages = [-(-c // PAGE) for c in ctx]
+    order, table, at = torch.randperm(sum(pages) + 1, generator=g).int(), torch.full((len(ctx), max(max(pages), 1)), -1, dtype=torch.int32), 0
+    for b, n in enumerate(pages):
+        table[b, :n] = order[at:at + n]
+        at += n
+    k, v = torch.randn(at + 1, PAGE, G, dim, generator=g).bfloat16(), torch.randn(at + 1, G, vdim, PAGE, generator=g).bfloat16()
+    return k, v, table
+
+
+def reference(q, k, v, table, ctx, past, H, G, dim, vdim, window, keep, chunk, sinks):
+    """q [n, H dim] of one sequence behind `past` tokens, float64 on the CPU."""
+    rows = table[:-(-ctx // PAGE)].long()
+    K = k[rows].reshape(-1, G, dim)[:ctx].double()
+    V = v[rows].permute(0, 3, 1, 2).reshape(-1, G, vdim)[:ctx].double()
+    n = q.shape[0]
+    i, j = torch.arange(past, past + n)[:, None], torch.arange(ctx)[None, :]
+    seen = (j <= i)
+    if window:
+        seen &= (i - j < window) | (j < keep)
+    if chunk:
+        seen &= j >= i // chunk * chunk
+    out = torch.empty(n, H, vdim, dtype=torch.float64)
+    for h in range(H):
+        s = (q.double().view(n, H, dim)[:, h] @ K[:, h // (H // G)].t().contiguous()) * dim ** -0.5
+        s = s.masked_fill(~seen, -torch.inf)
+        if sinks is not None:
+            s = torch.cat([s, sinks[h].double().expand(n, 1)], 1)
+        out[:, h] = torch.softmax(s, 1)[:, :ctx] @ V[:, h // (H // G)].contiguous()
+    return out.view(n, H * vdim)
+
+
+def close_to(got, want):
+    """Weights enter with 16 bits, sums are fp32: 2^-14 of the largest value, and the result's own rounding to bf16."""
+    want = want.to(got.device)
+    return ((got.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -13 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (200, 5, 0), (0, 0, 128)])
+@pytest.mark.parametrize("B", [33, 100, 256, 257])
+def test_a_step_of_many_sequences(B, window, keep, chunk):
+    """The sequences of a large batch, dealt out by length, give the bits that they give in small batches; equal lengths, one key, none."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(B + window)
+    H, G, dim, vdim = 16, 8, 64, 64
+    ctx = torch.randint(1, 700, (B,), generator=g).tolist()
+    ctx[3], ctx[7:12], ctx[20] = 0, [511] * 5, 1
+    k, v, table = caches(g, ctx, G, dim, vdim)
+    q = torch.randn(B, H * dim, generator=g).bfloat16().cuda()
+    k, v, table, lens = k.cuda(), v.cuda(), table.cuda(), torch.tensor(ctx).int().cuda()
+    kw = dict(window=window, keep_first=keep, chunk=chunk)
+    got = ops.attn_paged_any(q, k, v, None, lens, table, dim ** -0.5, H, G, dim, vdim, **kw)
+    n = 24                                                   # (too few to be dealt out, too many for key parts)
+    for lo in range(0, B - n, n):
+        assert torch.equal(ops.attn_paged_any(q[lo:lo + n].contiguous(), k, v, None, lens[lo:lo + n].contiguous(), table[lo:lo + n].contiguous(), dim ** -0.5, H, G, dim, vdim, **kw),
+                           got[lo:lo + n])
+    for b in (3, 20, B - 1):
+        if ctx[b]:
+            assert close_to(got[b:b + 1], reference(q[b:b + 1].cpu(), k.cpu(), v.cpu(), table[b].cpu(), ctx[b], ctx[b] - 1, H, G, dim, vdim, window, keep, chunk, None))
+        else:
+            assert (got[b] == 0).all()
