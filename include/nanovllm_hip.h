@@ -656,6 +656,28 @@ int32_t nvh_hyper_norm(float* x, int64_t streams, const float* mix, const float*
 int32_t nvh_residual_subnorm(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale, const float* c32,
                              int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps, float* x, void* h,
                              int64_t h_stride, int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream);
+/* The three closes above with a mixture of experts' result among the terms (in the place of c32 / y32, which is then NULL): sum over r < top, in
+ * order, of moe_weights[t, r] moe_y[pos_of_pair[t, r]] (weights NULL: 1; positions < 0 are skipped), plus shared[t] (type A, may be NULL) times
+ * sigmoid(shared_gate[t shared_gate_stride]) when given - the fp32 rows that nvh_moe_combine writes. */
+int32_t nvh_residual_norm_moe(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride,
+                              const void* b_weight, float branch_scale, float branch_eps, const void* c, int64_t c_stride,
+                              const float* c32, int64_t c32_stride, float* x, int32_t norm_kind, const void* norm_weight,
+                              const void* norm_bias, float eps, void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y,
+                              int64_t moe_y_stride, const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                              int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                              nvh_stream_t stream);
+int32_t nvh_residual_postnorm_moe(const void* y, int64_t y_stride, const float* y32, int64_t y32_stride, const void* layer_scale,
+                                  float alpha, float* x, int32_t write_x, const void* norm_weight, float weight_offset, float eps,
+                                  void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y, int64_t moe_y_stride,
+                                  const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                                  int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                                  nvh_stream_t stream);
+int32_t nvh_residual_subnorm_moe(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale,
+                                 const float* c32, int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps,
+                                 float* x, void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y, int64_t moe_y_stride,
+                                 const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                                 int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                                 nvh_stream_t stream);
 /* y[rows, inter] = act(x[:, :inter]) (* x[:, inter:2 inter] when gated), evaluated in fp32.  act 0: silu, 1: gelu (tanh form),
  * 2: squared relu. */
 int32_t nvh_act_mul(const void* x, int64_t row_stride, void* y, int64_t y_stride, int64_t rows, int64_t inter, int32_t act, int32_t gated,
@@ -751,7 +773,8 @@ int32_t nvh_group_rmsnorm_gate(const float* o, const void* weight, int32_t weigh
  * (tile_expert, tile_row0, tile_rows; unused tiles have 0 rows); max_tiles >= nvh_moe_max_tiles(T top, E).
  * nvh_gemm_grouped_any_nt: y[pos] = x[gather ? gather[pos] : pos] w[expert]^T over the tiles, w [E, N, K]; types as
  * nvh_gemm_any_nt; relu2: the squared relu of the result.  nvh_moe_combine: out fp32 [T, dim] = sum_r weights[t, r] y[pos_of_pair[t, r]] (+ shared[t], type A,
- * times sigmoid(shared_gate[t shared_gate_stride]) when a gate logit per token is given; weights NULL: all 1). */
+ * times sigmoid(shared_gate[t shared_gate_stride]) when a gate logit per token is given; weights NULL: all 1).
+ * nvh_gemm_grouped_many_nt: nvh_gemm_grouped_any_nt for callers whose experts have many rows on average; the same results bit for bit. */
 int32_t nvh_moe_route(const float* logits, int64_t row_stride, int32_t* ids, float* weights, int64_t num_tokens, int64_t experts,
                       int64_t top, nvh_stream_t stream);
 /* nvh_moe_route with the router's product inside: logits = x w^T + bias (x [T, K], w [E, K], bias [E] or NULL, type A;

@@ -177,8 +177,6 @@ struct CloseArgs {
     int dim;
 };
 
-// The close with one branch and no statistics but mean squares (a with or without its norm, norm 0 or 2), four columns a lane and
-// access: the row stays in registers, everything is on its way before the first sum needs it.  R: pieces of 1024 columns.
 template <typename A>
 __device__ __forceinline__ f32x4 load4(const A* p) {
     if constexpr (sizeof(A) == 4) {
@@ -188,79 +186,185 @@ __device__ __forceinline__ f32x4 load4(const A* p) {
         return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
     }
 }
+template <typename A>
+__device__ __forceinline__ void store4(A* p, const f32x4& v) {
+    if constexpr (sizeof(A) == 4) *reinterpret_cast<f32x4*>(p) = v;
+    else *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+}
 
-template <typename A, int R>
-__global__ __launch_bounds__(256) void residual_norm_branch_kernel(CloseArgs p) {
-    __shared__ float red[8];
+// A mixture of experts' result as terms of a close: sum over a token's `top` choices, in choice order, of weight * y[position] (positions < 0 are
+// skipped, null weights are 1), plus the shared expert's row, times sigmoid of the token's gate logit where there is one - what nvh_moe_combine writes.
+struct MoeTerms {
+    const void* y;             // rows of the chosen experts by position (null: no such terms)
+    int64_t ldy;
+    const int32_t* pos;        // [T, top]
+    const float* weights;      // [T, top] or null
+    int top;
+    const void* shared;        // [T, ld] or null
+    int64_t shared_stride;
+    const float* gate;
+    int64_t gate_stride;
+};
+// ... of row t at N consecutive columns from c on: the positions and rows of four choices are on their way together.
+template <typename A, int N>
+__device__ __forceinline__ void moe_sum(const MoeTerms& m, int64_t t, int c, float (&s)[N]) {
+    auto load = [](const A* p, float (&v)[N]) {
+        if constexpr (N == 4) {
+            const f32x4 x = load4(p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = x[e];
+        } else {
+            v[0] = (float)p[0];
+        }
+    };
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = 0.f;
+    const float sg = m.gate ? 1.0f / (1.0f + expf(-m.gate[t * m.gate_stride])) : 1.0f;
+    float sh[N];
+    if (m.shared) load((const A*)m.shared + t * m.shared_stride + c, sh);
+    for (int r0 = 0; r0 < m.top; r0 += 4) {
+        int pos[4];
+        float w[4], v[4][N];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t at = t * m.top + min(r0 + u, m.top - 1);
+            pos[u] = m.pos[at];
+            w[u] = m.weights ? m.weights[at] : 1.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load((const A*)m.y + (int64_t)max(pos[u], 0) * m.ldy + c, v[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (r0 + u < m.top && pos[u] >= 0)
+#pragma unroll
+                for (int e = 0; e < N; ++e) s[e] = __builtin_fmaf(w[u], v[u][e], s[e]);
+    }
+    if (m.shared)
+#pragma unroll
+        for (int e = 0; e < N; ++e) s[e] += sg * sh[e];
+}
+
+// The closes with four columns a lane and access: the row stays in registers, and everything is on its way before the first sum needs it.  A row is
+// a chain of a load, one or two sums across the workgroup and a store, whose latencies are the launch at any number of rows that a step brings
+// (column by column through LDS every pass over the row waits for its own loads).  R: pieces of 1024 columns.  MOE: with a mixture's terms.
+// us for 64 rows of 1024, column by column and this: residual norm with two terms 9.1 and 4.4; a mixture's launch and a close after it 7.8 + 5.0 and 4.5.
+template <typename A, int R, bool MOE>
+__global__ __launch_bounds__(256) void residual_norm_vec_kernel(CloseArgs p, MoeTerms m) {
+    __shared__ float red[16];
     const int64_t row = blockIdx.x;
     const int dim = p.dim;
-    const A* a = (const A*)p.a + row * p.a_stride;
+    const A* a = p.a ? (const A*)p.a + row * p.a_stride : nullptr;
+    const A* b = p.b ? (const A*)p.b + row * p.b_stride : nullptr;
+    const A* c = p.c ? (const A*)p.c + row * p.c_stride : nullptr;
+    const float* c32 = p.c32 ? p.c32 + row * p.c32_stride : nullptr;
     float* xr = p.x + row * dim;
-    f32x4 v[R], x[R], wa[R], nw[R];
-    float s = 0.f;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 va[R], vb[R], x[R], wa[R], wb[R], vc[R], vc32[R], nw[R], nb[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int c = (threadIdx.x + 256 * j) * 4;
-        v[j] = x[j] = wa[j] = nw[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (c < dim) {
-            v[j] = load4(a + c);
-            x[j] = *reinterpret_cast<const f32x4*>(xr + c);
-            if (p.wa) wa[j] = load4((const A*)p.wa + c);
-            if (p.norm) nw[j] = load4((const A*)p.nw + c);
+        const int col = (threadIdx.x + 256 * j) * 4;
+        va[j] = vb[j] = x[j] = wa[j] = wb[j] = vc[j] = vc32[j] = nw[j] = nb[j] = zero;
+        if (col < dim) {
+            if (a) va[j] = load4(a + col);
+            if (b) vb[j] = load4(b + col);
+            if (c) vc[j] = load4(c + col);
+            if (c32) vc32[j] = load4(c32 + col);
+            x[j] = load4(xr + col);
+            if (p.wa) wa[j] = load4((const A*)p.wa + col);
+            if (p.wb) wb[j] = load4((const A*)p.wb + col);
+            if (p.norm) nw[j] = load4((const A*)p.nw + col);
+            if (p.norm && p.nb) nb[j] = load4((const A*)p.nb + col);
+            if constexpr (MOE) {
+                float s[4];
+                moe_sum<A, 4>(m, row, col, s);
+                vc32[j] = f32x4{s[0], s[1], s[2], s[3]};
+            }
         }
     }
+    float ia = 1.f, ib = 1.f, sa = 0.f, sb = 0.f;
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s += v[j][e] * v[j][e];
-    const float ia = p.wa ? 1.0f / sqrtf(block_sum4(s, red) / (float)dim + p.branch_eps) : 1.0f;
-    s = 0.f;
+        for (int e = 0; e < 4; ++e) {
+            sa += va[j][e] * va[j][e];
+            sb += vb[j][e] * vb[j][e];
+        }
+    if (p.wa) ia = 1.0f / sqrtf(block_sum4(sa, red) / (float)dim + p.branch_eps);
+    if (p.wb) ib = 1.0f / sqrtf(block_sum4(sb, red + 4) / (float)dim + p.branch_eps);
+    float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int c = (threadIdx.x + 256 * j) * 4;
+        const int col = (threadIdx.x + 256 * j) * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            x[j][e] += p.branch_scale * (p.wa ? v[j][e] * ia * wa[j][e] : v[j][e]);
-            s += x[j][e] * x[j][e];
+            float s = 0.f;
+            if (a) s += p.wa ? va[j][e] * ia * wa[j][e] : va[j][e];
+            if (b) s += p.wb ? vb[j][e] * ib * wb[j][e] : vb[j][e];
+            s *= p.branch_scale;
+            if (c) s += vc[j][e];
+            if (MOE || c32) s += vc32[j][e];
+            x[j][e] += s;
+            sum += x[j][e];
         }
-        if (c < dim) *reinterpret_cast<f32x4*>(xr + c) = x[j];
+        if (col < dim && (MOE || a || b || c || c32)) *reinterpret_cast<f32x4*>(xr + col) = x[j];
     }
     if (p.norm == 0) return;
-    const float inv = 1.0f / sqrtf(block_sum4(s, red + 4) / (float)dim + p.eps);
+    const float mean = p.norm == 1 ? block_sum4(sum, red + 8) / (float)dim : 0.f;
+    float sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const bool in = (threadIdx.x + 256 * j) * 4 < dim;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            x[j][e] = in ? x[j][e] - mean : 0.f;
+            sq += x[j][e] * x[j][e];
+        }
+    }
+    const float inv = 1.0f / sqrtf(block_sum4(sq, red + 12) / (float)dim + p.eps);
     A* h = (A*)p.h + row * p.h_stride;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int c = (threadIdx.x + 256 * j) * 4;
-        if (c >= dim) continue;
-        if constexpr (sizeof(A) == 4) {
-            *reinterpret_cast<f32x4*>(h + c) = x[j] * inv * nw[j];
-        } else {
-            bf16x4 out;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) out[e] = (bf16)(x[j][e] * inv * nw[j][e]);
-            *reinterpret_cast<bf16x4*>(h + c) = out;
-        }
+        const int col = (threadIdx.x + 256 * j) * 4;
+        if (col < dim) store4(h + col, p.nb ? x[j] * inv * nw[j] + nb[j] : x[j] * inv * nw[j]);
     }
 }
 
+// R for rows of `dim` columns, or 0 where the vector form does not serve them.
+static int close_pieces(int dim) { return dim % 4 || dim > 8192 ? 0 : dim <= 1024 ? 1 : dim <= 2048 ? 2 : dim <= 4096 ? 4 : 8; }
 template <typename A>
-static bool launch_residual_norm_branch(const CloseArgs& p, int64_t rows, hipStream_t st) {
-    auto al = [](const void* q, int bytes) { return q == nullptr || ((uintptr_t)q % bytes) == 0; };
-    constexpr int B = 4 * (int)sizeof(A);
-    if (!p.a || p.b || p.c || p.c32 || p.norm == 1 || p.nb || p.dim % 4 || p.dim > 8192 || p.a_stride % 4 || (p.norm && p.h_stride % 4) || !al(p.a, B) || !al(p.wa, B) ||
-        !al(p.nw, B) || !al(p.h, B) || !al(p.x, 16))
+static bool rows_of_fours(const void* p, int64_t stride) {   // (absent rows do)
+    return !p || (stride % 4 == 0 && ((uintptr_t)p % (4 * sizeof(A))) == 0);
+}
+template <typename A>
+static bool moe_of_fours(const MoeTerms& m) {
+    return rows_of_fours<A>(m.y, m.ldy) && rows_of_fours<A>(m.shared, m.shared_stride);
+}
+#define NVH_CLOSE_CASES(KERNEL, ...)                                                             \
+    switch (pieces * (m.y ? -1 : 1)) {                                                           \
+        case 1: KERNEL<A, 1, false><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case 2: KERNEL<A, 2, false><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case 4: KERNEL<A, 4, false><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case 8: KERNEL<A, 8, false><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case -1: KERNEL<A, 1, true><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case -2: KERNEL<A, 2, true><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        case -4: KERNEL<A, 4, true><<<grid, 256, 0, st>>>(__VA_ARGS__); break;                   \
+        default: KERNEL<A, 8, true><<<grid, 256, 0, st>>>(__VA_ARGS__);                          \
+    }
+
+template <typename A>
+static bool launch_residual_norm_vec(const CloseArgs& p, const MoeTerms& m, int64_t rows, hipStream_t st) {
+    const int pieces = close_pieces(p.dim);
+    if (!pieces || !rows_of_fours<A>(p.a, p.a_stride) || !rows_of_fours<A>(p.b, p.b_stride) || !rows_of_fours<A>(p.c, p.c_stride) ||
+        !rows_of_fours<float>(p.c32, p.c32_stride) || !rows_of_fours<A>(p.wa, 0) || !rows_of_fours<A>(p.wb, 0) || !rows_of_fours<A>(p.nw, 0) ||
+        !rows_of_fours<A>(p.nb, 0) || (p.norm && !rows_of_fours<A>(p.h, p.h_stride)) || !nvh_aligned16(p.x) || !moe_of_fours<A>(m))
         return false;
-    const int pieces = (p.dim + 1023) / 1024;
     const dim3 grid((unsigned)rows);
-    if (pieces <= 1) residual_norm_branch_kernel<A, 1><<<grid, 256, 0, st>>>(p);
-    else if (pieces <= 2) residual_norm_branch_kernel<A, 2><<<grid, 256, 0, st>>>(p);
-    else if (pieces <= 4) residual_norm_branch_kernel<A, 4><<<grid, 256, 0, st>>>(p);
-    else residual_norm_branch_kernel<A, 8><<<grid, 256, 0, st>>>(p);
+    NVH_CLOSE_CASES(residual_norm_vec_kernel, p, m)
     return true;
 }
 
 template <typename A>
-__global__ __launch_bounds__(256) void residual_norm_kernel(CloseArgs p) {
+__global__ __launch_bounds__(256) void residual_norm_kernel(CloseArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
     const int64_t row = blockIdx.x;
@@ -295,8 +399,13 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(CloseArgs p) {
         s *= p.branch_scale;
         if (c) s += (float)c[i];
         if (c32) s += c32[i];
+        if (m.y) {
+            float e[1];
+            moe_sum<A, 1>(m, row, i, e);
+            s += e[0];
+        }
         const float v = xr[i] + s;
-        if (a || b || c || c32) xr[i] = v;
+        if (a || b || c || c32 || m.y) xr[i] = v;
         rowbuf[i] = v;
         sum += v;
     }
@@ -339,7 +448,7 @@ struct PostNormArgs {
 };
 
 template <typename A>
-__global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p) {
+__global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
     const int64_t row = blockIdx.x;
@@ -351,9 +460,14 @@ __global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p) 
     float sq = 0.f;
     for (int i = threadIdx.x; i < dim; i += 256) {
         float v = p.alpha * xr[i];
-        if (y || y32) {
+        if (y || y32 || m.y) {
             float s = y ? (float)y[i] : 0.f;
             if (y32) s += y32[i];
+            if (m.y) {
+                float e[1];
+                moe_sum<A, 1>(m, row, i, e);
+                s += e[0];
+            }
             if (ls) s *= (float)ls[i];
             v += s;
         }
@@ -367,6 +481,72 @@ __global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p) 
         if (p.write_x) xr[i] = v;
         if (h) h[i] = (A)v;
     }
+}
+
+template <typename A, int R, bool MOE>
+__global__ __launch_bounds__(256) void residual_postnorm_vec_kernel(PostNormArgs p, MoeTerms m) {
+    __shared__ float red[4];
+    const int64_t row = blockIdx.x;
+    const int dim = p.dim;
+    float* xr = p.x + row * dim;
+    const bool any = MOE || p.y || p.y32;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
+    f32x4 x[R], y[R], y32[R], ls[R], nw[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int col = (threadIdx.x + 256 * j) * 4;
+        x[j] = y[j] = y32[j] = nw[j] = zero;
+        ls[j] = one;
+        if (col < dim) {
+            x[j] = load4(xr + col);
+            if (p.y) y[j] = load4((const A*)p.y + row * p.y_stride + col);
+            if (p.y32) y32[j] = load4(p.y32 + row * p.y32_stride + col);
+            if (p.ls) ls[j] = load4((const A*)p.ls + col);
+            nw[j] = load4((const A*)p.nw + col);
+            if constexpr (MOE) {
+                float s[4];
+                moe_sum<A, 4>(m, row, col, s);
+                y32[j] = f32x4{s[0], s[1], s[2], s[3]};
+            }
+        }
+    }
+    float sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v = p.alpha * x[j][e];
+            if (any) {
+                float s = y[j][e];
+                if (MOE || p.y32) s += y32[j][e];
+                if (p.ls) s *= ls[j][e];
+                v += s;
+            }
+            x[j][e] = v;
+            sq += v * v;
+        }
+    const float inv = 1.0f / sqrtf(block_sum4(sq, red) / (float)dim + p.eps);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int col = (threadIdx.x + 256 * j) * 4;
+        if (col >= dim) continue;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = x[j][e] * inv * (p.offset + nw[j][e]);
+        if (p.write_x) *reinterpret_cast<f32x4*>(xr + col) = v;
+        if (p.h) store4((A*)p.h + row * p.h_stride + col, v);
+    }
+}
+
+template <typename A>
+static bool launch_residual_postnorm_vec(const PostNormArgs& p, const MoeTerms& m, int64_t rows, hipStream_t st) {
+    const int pieces = close_pieces(p.dim);
+    if (!pieces || !rows_of_fours<A>(p.y, p.y_stride) || !rows_of_fours<float>(p.y32, p.y32_stride) || !rows_of_fours<A>(p.ls, 0) || !rows_of_fours<A>(p.nw, 0) ||
+        !rows_of_fours<A>(p.h, p.h_stride) || !nvh_aligned16(p.x) || !moe_of_fours<A>(m))
+        return false;
+    const dim3 grid((unsigned)rows);
+    NVH_CLOSE_CASES(residual_postnorm_vec_kernel, p, m)
+    return true;
 }
 
 // The close of a sublayer whose RESULT is normed before it joins the stream (the sublayer itself read the stream as it is), per row:
@@ -387,7 +567,7 @@ struct SubNormArgs {
 };
 
 template <typename A>
-__global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p) {
+__global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
     const int64_t row = blockIdx.x;
@@ -401,6 +581,11 @@ __global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p) {
         if (a) y = p.sa * (float)a[i];
         if (b) y = __builtin_fmaf(p.sb, (float)b[i], y);
         if (c32) y += c32[i];
+        if (m.y) {
+            float e[1];
+            moe_sum<A, 1>(m, row, i, e);
+            y += e[0];
+        }
         rowbuf[i] = y;
         sq += y * y;
     }
@@ -413,6 +598,68 @@ __global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p) {
         xr[i] = v;
         if (h) h[i] = (A)v;
     }
+}
+
+template <typename A, int R, bool MOE>
+__global__ __launch_bounds__(256) void residual_subnorm_vec_kernel(SubNormArgs p, MoeTerms m) {
+    __shared__ float red[4];
+    const int64_t row = blockIdx.x;
+    const int dim = p.dim;
+    float* xr = p.x + row * dim;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const float w1 = p.w_elems == 1 ? (float)((const A*)p.w)[0] : 0.f;
+    f32x4 x[R], y[R], b[R], c[R], w[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int col = (threadIdx.x + 256 * j) * 4;
+        x[j] = y[j] = b[j] = c[j] = zero;
+        w[j] = f32x4{w1, w1, w1, w1};
+        if (col < dim) {
+            if (p.a) y[j] = load4((const A*)p.a + row * p.a_stride + col);
+            if (p.b) b[j] = load4((const A*)p.b + row * p.b_stride + col);
+            if (p.c32) c[j] = load4(p.c32 + row * p.c32_stride + col);
+            x[j] = load4(xr + col);
+            if (p.w_elems != 1) w[j] = load4((const A*)p.w + col);
+            if constexpr (MOE) {
+                float s[4];
+                moe_sum<A, 4>(m, row, col, s);
+                c[j] = f32x4{s[0], s[1], s[2], s[3]};
+            }
+        }
+    }
+    float sq = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float v = p.a ? p.sa * y[j][e] : 0.f;
+            if (p.b) v = __builtin_fmaf(p.sb, b[j][e], v);
+            if (MOE || p.c32) v += c[j][e];
+            y[j][e] = v;
+            sq += v * v;
+        }
+    const float inv = p.mult / sqrtf(block_sum4(sq, red) / (float)dim + p.eps);
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        const int col = (threadIdx.x + 256 * j) * 4;
+        if (col >= dim) continue;
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = x[j][e] + y[j][e] * inv * w[j][e];
+        *reinterpret_cast<f32x4*>(xr + col) = v;
+        if (p.h) store4((A*)p.h + row * p.h_stride + col, v);
+    }
+}
+
+template <typename A>
+static bool launch_residual_subnorm_vec(const SubNormArgs& p, const MoeTerms& m, int64_t rows, hipStream_t st) {
+    const int pieces = close_pieces(p.dim);
+    if (!pieces || !rows_of_fours<A>(p.a, p.a_stride) || !rows_of_fours<A>(p.b, p.b_stride) || !rows_of_fours<float>(p.c32, p.c32_stride) ||
+        (p.w_elems != 1 && !rows_of_fours<A>(p.w, 0)) || !rows_of_fours<A>(p.h, p.h_stride) || !nvh_aligned16(p.x) || !moe_of_fours<A>(m))
+        return false;
+    const dim3 grid((unsigned)rows);
+    NVH_CLOSE_CASES(residual_subnorm_vec_kernel, p, m)
+    return true;
 }
 
 // y = act(g) (* u when gated): g = columns [0, inter) and u = columns [inter, 2 inter) of the row.
@@ -612,17 +859,17 @@ extern "C" int32_t nvh_embedding_pos_stream(const int64_t* ids, const int64_t* p
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_residual_norm(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride, const void* b_weight,
-                                     float branch_scale, float branch_eps, const void* c, int64_t c_stride, const float* c32, int64_t c32_stride,
-                                     float* x, int32_t norm_kind, const void* norm_weight, const void* norm_bias, float eps, void* h, int64_t h_stride,
-                                     int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+static int32_t residual_norm(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride, const void* b_weight,
+                             float branch_scale, float branch_eps, const void* c, int64_t c_stride, const float* c32, int64_t c32_stride, float* x,
+                             int32_t norm_kind, const void* norm_weight, const void* norm_bias, float eps, void* h, int64_t h_stride, int64_t rows,
+                             int64_t dim, const MoeTerms& m, int32_t act_f32, nvh_stream_t stream) {
     NVH_STREAM_ARGS_OK("nvh_residual_norm", x && rows >= 0 && dim > 0 && dim <= 32768 && norm_kind >= 0 && norm_kind <= 2 && (norm_kind == 0 || (norm_weight && h)) &&
                                                 (!a_weight || a) && (!b_weight || b));
     if (rows == 0) return NVH_OK;
     const CloseArgs p{a, a_weight, b, b_weight, c, c32, a_stride, b_stride, c_stride, c32_stride, branch_scale, branch_eps, x, norm_kind,
                       norm_weight, norm_bias, eps, h, h_stride, (int)dim};
     hipStream_t st = (hipStream_t)stream;
-    if (act_f32 ? launch_residual_norm_branch<float>(p, rows, st) : launch_residual_norm_branch<bf16>(p, rows, st)) {
+    if (act_f32 ? launch_residual_norm_vec<float>(p, m, rows, st) : launch_residual_norm_vec<bf16>(p, m, rows, st)) {
         NVH_CHECK_LAUNCH("nvh_residual_norm");
         return NVH_OK;
     }
@@ -632,49 +879,116 @@ extern "C" int32_t nvh_residual_norm(const void* a, int64_t a_stride, const void
         const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_norm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_norm: %zu bytes of LDS refused", lds);
     }
-    if (act_f32) residual_norm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p);
-    else residual_norm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p);
+    if (act_f32) residual_norm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    else residual_norm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
     NVH_CHECK_LAUNCH("nvh_residual_norm");
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_residual_postnorm(const void* y, int64_t y_stride, const float* y32, int64_t y32_stride, const void* layer_scale, float alpha,
-                                         float* x, int32_t write_x, const void* norm_weight, float weight_offset, float eps, void* h, int64_t h_stride,
-                                         int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+extern "C" int32_t nvh_residual_norm(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride, const void* b_weight,
+                                     float branch_scale, float branch_eps, const void* c, int64_t c_stride, const float* c32, int64_t c32_stride,
+                                     float* x, int32_t norm_kind, const void* norm_weight, const void* norm_bias, float eps, void* h,
+                                     int64_t h_stride, int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+    return residual_norm(a, a_stride, a_weight, b, b_stride, b_weight, branch_scale, branch_eps, c, c_stride, c32, c32_stride, x, norm_kind, norm_weight, norm_bias, eps, h, h_stride, rows, dim,
+                        MoeTerms{}, act_f32, stream);
+}
+
+extern "C" int32_t nvh_residual_norm_moe(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride,
+                                         const void* b_weight, float branch_scale, float branch_eps, const void* c, int64_t c_stride,
+                                         const float* c32, int64_t c32_stride, float* x, int32_t norm_kind, const void* norm_weight,
+                                         const void* norm_bias, float eps, void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y,
+                                         int64_t moe_y_stride, const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                                         int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                                         nvh_stream_t stream) {
+    NVH_REQUIRE(moe_y && pos_of_pair && top > 0 && top <= 4096 && moe_y_stride >= dim && (!shared || shared_stride >= dim) && (shared || !shared_gate) &&
+                    !c32, NVH_EINVAL, "nvh_residual_norm_moe: bad argument");
+    const MoeTerms m{moe_y, moe_y_stride, pos_of_pair, moe_weights, (int)top, shared, shared_stride, shared_gate, shared_gate_stride};
+    return residual_norm(a, a_stride, a_weight, b, b_stride, b_weight, branch_scale, branch_eps, c, c_stride, c32, c32_stride, x, norm_kind, norm_weight, norm_bias, eps, h, h_stride, rows, dim, m, act_f32, stream);
+}
+
+static int32_t residual_postnorm(const void* y, int64_t y_stride, const float* y32, int64_t y32_stride, const void* layer_scale, float alpha,
+                                 float* x, int32_t write_x, const void* norm_weight, float weight_offset, float eps, void* h, int64_t h_stride,
+                                 int64_t rows, int64_t dim, const MoeTerms& m, int32_t act_f32, nvh_stream_t stream) {
     NVH_STREAM_ARGS_OK("nvh_residual_postnorm", x && norm_weight && rows >= 0 && dim > 0 && dim <= 32768 && (!y || y_stride >= dim) && (!y32 || y32_stride >= dim) &&
                                                     (!h || h_stride >= dim));
     if (rows == 0) return NVH_OK;
     const PostNormArgs p{y, y_stride, y32, y32_stride, layer_scale, alpha, x, norm_weight, weight_offset, eps, h, h_stride, (int)dim, write_x};
     hipStream_t st = (hipStream_t)stream;
+    if (act_f32 ? launch_residual_postnorm_vec<float>(p, m, rows, st) : launch_residual_postnorm_vec<bf16>(p, m, rows, st)) {
+        NVH_CHECK_LAUNCH("nvh_residual_postnorm");
+        return NVH_OK;
+    }
     const size_t lds = sizeof(float) * (size_t)dim;
     if (lds > 48 * 1024) {
         const hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_postnorm_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_postnorm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_postnorm: %zu bytes of LDS refused", lds);
     }
-    if (act_f32) residual_postnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p);
-    else residual_postnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p);
+    if (act_f32) residual_postnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    else residual_postnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
     NVH_CHECK_LAUNCH("nvh_residual_postnorm");
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_residual_subnorm(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale, const float* c32,
-                                        int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps, float* x, void* h,
-                                        int64_t h_stride, int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
-    NVH_STREAM_ARGS_OK("nvh_residual_subnorm", x && weight && (a || b || c32) && rows >= 0 && dim > 0 && dim <= 32768 && (weight_elems == 1 || weight_elems == dim));
+extern "C" int32_t nvh_residual_postnorm(const void* y, int64_t y_stride, const float* y32, int64_t y32_stride, const void* layer_scale, float alpha,
+                                         float* x, int32_t write_x, const void* norm_weight, float weight_offset, float eps, void* h,
+                                         int64_t h_stride, int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+    return residual_postnorm(y, y_stride, y32, y32_stride, layer_scale, alpha, x, write_x, norm_weight, weight_offset, eps, h, h_stride, rows, dim,
+                            MoeTerms{}, act_f32, stream);
+}
+
+extern "C" int32_t nvh_residual_postnorm_moe(const void* y, int64_t y_stride, const float* y32, int64_t y32_stride, const void* layer_scale,
+                                             float alpha, float* x, int32_t write_x, const void* norm_weight, float weight_offset, float eps,
+                                             void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y, int64_t moe_y_stride,
+                                             const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                                             int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                                             nvh_stream_t stream) {
+    NVH_REQUIRE(moe_y && pos_of_pair && top > 0 && top <= 4096 && moe_y_stride >= dim && (!shared || shared_stride >= dim) && (shared || !shared_gate) &&
+                    !y32, NVH_EINVAL, "nvh_residual_postnorm_moe: bad argument");
+    const MoeTerms m{moe_y, moe_y_stride, pos_of_pair, moe_weights, (int)top, shared, shared_stride, shared_gate, shared_gate_stride};
+    return residual_postnorm(y, y_stride, y32, y32_stride, layer_scale, alpha, x, write_x, norm_weight, weight_offset, eps, h, h_stride, rows, dim, m, act_f32, stream);
+}
+
+static int32_t residual_subnorm(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale, const float* c32,
+                                int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps, float* x, void* h,
+                                int64_t h_stride, int64_t rows, int64_t dim, const MoeTerms& m, int32_t act_f32, nvh_stream_t stream) {
+    NVH_STREAM_ARGS_OK("nvh_residual_subnorm", x && weight && (a || b || c32 || m.y) && rows >= 0 && dim > 0 && dim <= 32768 && (weight_elems == 1 || weight_elems == dim));
     if (rows == 0) return NVH_OK;
     const SubNormArgs p{a, b, c32, a_stride, b_stride, c32_stride, a_scale, b_scale, mult, eps, weight, (int)weight_elems, x, h, h_stride, (int)dim};
     hipStream_t st = (hipStream_t)stream;
+    if (act_f32 ? launch_residual_subnorm_vec<float>(p, m, rows, st) : launch_residual_subnorm_vec<bf16>(p, m, rows, st)) {
+        NVH_CHECK_LAUNCH("nvh_residual_subnorm");
+        return NVH_OK;
+    }
     const size_t lds = sizeof(float) * (size_t)dim;
     if (lds > 48 * 1024) {
         const hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_subnorm_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_subnorm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_subnorm: %zu bytes of LDS refused", lds);
     }
-    if (act_f32) residual_subnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p);
-    else residual_subnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p);
+    if (act_f32) residual_subnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    else residual_subnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
     NVH_CHECK_LAUNCH("nvh_residual_subnorm");
     return NVH_OK;
+}
+
+extern "C" int32_t nvh_residual_subnorm(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale,
+                                        const float* c32, int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps,
+                                        float* x, void* h, int64_t h_stride, int64_t rows, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+    return residual_subnorm(a, a_stride, a_scale, b, b_stride, b_scale, c32, c32_stride, mult, weight, weight_elems, eps, x, h, h_stride, rows, dim,
+                           MoeTerms{}, act_f32, stream);
+}
+
+extern "C" int32_t nvh_residual_subnorm_moe(const void* a, int64_t a_stride, float a_scale, const void* b, int64_t b_stride, float b_scale,
+                                            const float* c32, int64_t c32_stride, float mult, const void* weight, int64_t weight_elems, float eps,
+                                            float* x, void* h, int64_t h_stride, int64_t rows, int64_t dim, const void* moe_y, int64_t moe_y_stride,
+                                            const int32_t* pos_of_pair, const float* moe_weights, int64_t top, const void* shared,
+                                            int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, int32_t act_f32,
+                                            nvh_stream_t stream) {
+    NVH_REQUIRE(moe_y && pos_of_pair && top > 0 && top <= 4096 && moe_y_stride >= dim && (!shared || shared_stride >= dim) && (shared || !shared_gate) &&
+                    !c32, NVH_EINVAL, "nvh_residual_subnorm_moe: bad argument");
+    const MoeTerms m{moe_y, moe_y_stride, pos_of_pair, moe_weights, (int)top, shared, shared_stride, shared_gate, shared_gate_stride};
+    return residual_subnorm(a, a_stride, a_scale, b, b_stride, b_scale, c32, c32_stride, mult, weight, weight_elems, eps, x, h, h_stride, rows, dim, m, act_f32, stream);
 }
 
 extern "C" int32_t nvh_act_mul(const void* x, int64_t row_stride, void* y, int64_t y_stride, int64_t rows, int64_t inter, int32_t act, int32_t gated,

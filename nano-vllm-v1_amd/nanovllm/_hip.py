@@ -112,8 +112,11 @@ SIGNATURES = {
     # layer norm / RMS norm around the fp32 stream, plain activations (csrc/stream_f32.hip)
     "nvh_embedding_pos_stream": (i32, [vp, vp, vp, vp, f32, vp, i64, i64, i64, i64, i32, vp]),
     "nvh_residual_norm": (i32, [vp, i64, vp, vp, i64, vp, f32, f32, vp, i64, vp, i64, vp, i32, vp, vp, f32, vp, i64, i64, i64, i32, vp]),
+    "nvh_residual_norm_moe": (i32, [vp, i64, vp, vp, i64, vp, f32, f32, vp, i64, vp, i64, vp, i32, vp, vp, f32, vp, i64, i64, i64, vp, i64, vp, vp, i64, vp, i64, vp, i64, i32, vp]),
     "nvh_residual_postnorm": (i32, [vp, i64, vp, i64, vp, f32, vp, i32, vp, f32, f32, vp, i64, i64, i64, i32, vp]),
+    "nvh_residual_postnorm_moe": (i32, [vp, i64, vp, i64, vp, f32, vp, i32, vp, f32, f32, vp, i64, i64, i64, vp, i64, vp, vp, i64, vp, i64, vp, i64, i32, vp]),
     "nvh_residual_subnorm": (i32, [vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, vp, i64, i64, i64, i32, vp]),
+    "nvh_residual_subnorm_moe": (i32, [vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, vp, i64, i64, i64, vp, i64, vp, vp, i64, vp, i64, vp, i64, i32, vp]),
     "nvh_act_mul": (i32, [vp, i64, vp, i64, i64, i64, i32, i32, i32, vp]),
     "nvh_xielu": (i32, [vp, i64, vp, i64, i64, i64, vp, i32, vp]),
     "nvh_logits_scale": (i32, [vp, i64, vp, i64, i64, f32, f32, i32, vp]),

@@ -98,10 +98,10 @@ class PostSumRMSNorm(nn.Module):
         else:
             self.register_parameter("scale", None)
 
-    def close(self, x: torch.Tensor, y: torch.Tensor | None = None, y32: torch.Tensor | None = None, want_h: bool = True):
-        """y: the sublayer's result in the activation type, y32: in fp32 (either, both or none)."""
+    def close(self, x: torch.Tensor, y: torch.Tensor | None = None, y32: torch.Tensor | None = None, want_h: bool = True, moe: dict | None = None):
+        """y: the sublayer's result in the activation type, y32: in fp32 (either, both or none); moe: as the parts of a mixture's sum."""
         return ops.residual_postnorm(x, self.weight.data, self.eps, y, y32, None if self.scale is None else self.scale.data, self.alpha,
-                                     self.weight_offset, want_h)
+                                     self.weight_offset, want_h, moe=moe)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """The norm alone (no sum, the stream taken once): x fp32 [rows, dim] -> normed rows in the activation type (x is left as it is)."""
@@ -122,6 +122,6 @@ class SublayerOutputNorm(nn.Module):
         self.weight = nn.Parameter(torch.ones(hidden_size or 1), requires_grad=False)
         self.weight.weight_loader = lambda param, t: param.data.copy_(t.reshape(param.shape))
 
-    def close(self, x: torch.Tensor, a=None, a_scale: float = 1.0, b=None, b_scale: float = 1.0, c32=None, want_h: bool = True):
-        """a, b: terms of the result in the activation type (with their factors), c32: a term in fp32."""
-        return ops.residual_subnorm(x, self.weight.data, self.eps, self.mult, a, a_scale, b, b_scale, c32, want_h)
+    def close(self, x: torch.Tensor, a=None, a_scale: float = 1.0, b=None, b_scale: float = 1.0, c32=None, want_h: bool = True, moe: dict | None = None):
+        """a, b: terms of the result in the activation type (with their factors), c32: a term in fp32, moe: the parts of a mixture's sum."""
+        return ops.residual_subnorm(x, self.weight.data, self.eps, self.mult, a, a_scale, b, b_scale, c32, want_h, moe)

@@ -134,6 +134,13 @@ class SparseMoE(nn.Module):
         y, plan, weights, gate = self._experts(x)
         return ops.moe_combine(y, plan, None if self.weight_on_input else weights, self.shared(x) if self.shared is not None else None, gate, top=self.top)
 
+    def parts(self, x: torch.Tensor) -> dict:
+        """What forward() sums, for a close that does so itself (ops.residual_norm, residual_postnorm, residual_subnorm): the experts' rows by
+        position, the plan, the choices' weights and the shared expert's rows with their gate logits."""
+        y, plan, weights, gate = self._experts(x)
+        return dict(y=y, plan=plan, weights=None if self.weight_on_input else weights, shared=self.shared(x) if self.shared is not None else None, gate=gate,
+                    top=self.top)
+
     def terms(self, x: torch.Tensor) -> dict:
         """The result as the terms of a sum that a layer's close forms (ops.hyper_norm): the experts' rows under their weights and the
         shared expert's rows."""

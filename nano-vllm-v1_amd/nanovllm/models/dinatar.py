@@ -137,7 +137,7 @@ class DinatarMoE(nn.Module):
                              shared_ff=int(_get(shared, "ff")) if shared else None, act="silu", router_bias=True)
 
     def forward(self, x: torch.Tensor) -> dict:
-        return dict(c32=self.moe(x))
+        return dict(moe=self.moe.parts(x))
 
 
 class DinatarLayer(nn.Module):

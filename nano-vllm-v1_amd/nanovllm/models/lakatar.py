@@ -111,8 +111,8 @@ class LakatarMoE(nn.Module):
                              groups=int(_get(groups, "count", 1)) if groups else 1, keep_groups=int(_get(groups, "keep", 1)) if groups else 1,
                              route_scale=float(_get(router, "scale", 1.0)), shared_gate=bool(shared))
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.moe(x)
+    def forward(self, x: torch.Tensor) -> dict:
+        return self.moe.parts(x)
 
 
 class LakatarLayer(nn.Module):
@@ -304,7 +304,7 @@ class LakatarForCausalLM(nn.Module):
         for layer in self.layers:
             h = layer.norm1.close(x, y=layer.mixer(h, positions))
             if layer.mlp is not None:
-                h = layer.norm2.close(x, y32=layer.mlp(h))
+                h = layer.norm2.close(x, moe=layer.mlp(h))
             if self.collect is not None:
                 self.collect.append(x.clone())
         return x

@@ -893,13 +893,25 @@ def embedding_pos_stream(ids: torch.Tensor, positions: torch.Tensor, table: torc
     return x
 
 
+def _moe_args(moe: dict, rows: int, dim: int, other: torch.Tensor | None) -> tuple:
+    """A mixture's result as arguments of a close (SparseMoE.parts): what moe_combine of the same parts would have written."""
+    y, plan, weights, shared, gate, top = moe["y"], moe["plan"], moe["weights"], moe["shared"], moe["gate"], moe["top"]
+    assert other is None and y.shape == (rows * top, dim) and y.stride(1) == 1 and plan["pairs"] == rows * top
+    assert weights is None or (weights.dtype == F32 and weights.is_contiguous() and weights.numel() == rows * top)
+    assert shared is None or (shared.dtype == y.dtype and shared.shape == (rows, dim) and shared.stride(1) == 1)
+    assert gate is None or (shared is not None and gate.dtype == F32 and gate.shape == (rows, 1))
+    return (y.data_ptr(), y.stride(0), plan["pos_of_pair"].data_ptr(), _p(weights), top, _p(shared), shared.stride(0) if shared is not None else 0,
+            _p(gate), gate.stride(0) if gate is not None else 0)
+
+
 def residual_norm(x: torch.Tensor, a=None, a_weight=None, b=None, b_weight=None, branch_scale: float = 1.0, branch_eps: float = 0.0, c=None, c32=None,
-                  norm: str | None = None, weight=None, bias=None, eps: float = 0.0) -> torch.Tensor | None:
+                  norm: str | None = None, weight=None, bias=None, eps: float = 0.0, moe: dict | None = None) -> torch.Tensor | None:
     """x <- x + branch_scale * (unit(a) a_weight + unit(b) b_weight) + c + c32 in place (fp32 rows; a branch without a weight
-    is added as it is, absent terms are skipped); returns norm(x) in the activation type, or None without `norm`."""
+    is added as it is, absent terms are skipped); returns norm(x) in the activation type, or None without `norm`.  `moe`
+    (SparseMoE.parts) stands for c32 = the mixture's result."""
     assert x.dtype == F32 and x.is_contiguous() and x.dim() == 2
     rows, dim = x.shape
-    typed = [t for t in (a, a_weight, b, b_weight, c, weight, bias) if t is not None]
+    typed = [t for t in (a, a_weight, b, b_weight, c, weight, bias, moe and moe["y"]) if t is not None]
     assert typed, "nothing to add and nothing to normalise"
     f = _act_flag(*typed)
     for t in (a, b, c):
@@ -908,47 +920,50 @@ def residual_norm(x: torch.Tensor, a=None, a_weight=None, b=None, b_weight=None,
         assert t is None or (t.numel() == dim and t.is_contiguous())
     assert c32 is None or (c32.dtype == F32 and c32.shape == (rows, dim) and c32.stride(1) == 1)
     h = torch.empty(rows, dim, dtype=weight.dtype, device=x.device) if norm is not None else None
-    _hip.call("nvh_residual_norm", _p(a), a.stride(0) if a is not None else 0, _p(a_weight), _p(b), b.stride(0) if b is not None else 0, _p(b_weight),
+    _hip.call("nvh_residual_norm_moe" if moe else "nvh_residual_norm", _p(a), a.stride(0) if a is not None else 0, _p(a_weight), _p(b), b.stride(0) if b is not None else 0, _p(b_weight),
               float(branch_scale), float(branch_eps), _p(c), c.stride(0) if c is not None else 0, _p(c32), c32.stride(0) if c32 is not None else 0,
-              x.data_ptr(), NORM_KINDS[norm], _p(weight), _p(bias), float(eps), _p(h), dim, rows, dim, f, _stream())
+              x.data_ptr(), NORM_KINDS[norm], _p(weight), _p(bias), float(eps), _p(h), dim, rows, dim, *(_moe_args(moe, rows, dim, c32) if moe else ()), f,
+              _stream())
     return h
 
 
 def residual_postnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, y=None, y32=None, layer_scale=None, alpha: float = 1.0,
-                      weight_offset: float = 0.0, want_h: bool = True, in_place: bool = True) -> torch.Tensor | None:
+                      weight_offset: float = 0.0, want_h: bool = True, in_place: bool = True, moe: dict | None = None) -> torch.Tensor | None:
     """x <- rms_norm(alpha x + layer_scale (y + y32)) * (weight_offset + weight) in place (fp32 rows; y of the activation type and
     y32 fp32 may each be absent); returns the new x in the activation type (the input of the next sublayer).  `in_place` False:
-    x is only read."""
+    x is only read.  `moe` (SparseMoE.parts) stands for y32 = the mixture's result."""
     assert x.dtype == F32 and x.is_contiguous() and x.dim() == 2
     rows, dim = x.shape
-    typed = [t for t in (weight, y, layer_scale) if t is not None]
+    typed = [t for t in (weight, y, layer_scale, moe and moe["y"]) if t is not None]
     f = _act_flag(*typed)
     assert weight.numel() == dim and weight.is_contiguous() and (layer_scale is None or (layer_scale.numel() == dim and layer_scale.is_contiguous()))
     assert y is None or (y.shape == (rows, dim) and y.stride(1) == 1)
     assert y32 is None or (y32.dtype == F32 and y32.shape == (rows, dim) and y32.stride(1) == 1)
     h = torch.empty(rows, dim, dtype=weight.dtype, device=x.device) if want_h else None
-    _hip.call("nvh_residual_postnorm", _p(y), y.stride(0) if y is not None else 0, _p(y32), y32.stride(0) if y32 is not None else 0, _p(layer_scale),
-              float(alpha), x.data_ptr(), int(in_place), weight.data_ptr(), float(weight_offset), float(eps), _p(h), dim, rows, dim, f, _stream())
+    _hip.call("nvh_residual_postnorm_moe" if moe else "nvh_residual_postnorm", _p(y), y.stride(0) if y is not None else 0, _p(y32), y32.stride(0) if y32 is not None else 0, _p(layer_scale),
+              float(alpha), x.data_ptr(), int(in_place), weight.data_ptr(), float(weight_offset), float(eps), _p(h), dim, rows, dim,
+              *(_moe_args(moe, rows, dim, y32) if moe else ()), f, _stream())
     return h
 
 
 def residual_subnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, mult: float = 1.0, a=None, a_scale: float = 1.0, b=None, b_scale: float = 1.0,
-                     c32=None, want_h: bool = True):
+                     c32=None, want_h: bool = True, moe: dict | None = None):
     """x <- x + mult * weight * y / sqrt(mean(y^2) + eps) in place (fp32 rows), y = a_scale a + b_scale b + c32: a sublayer's result is
     normed before it joins the stream.  a, b: rows of the activation type, c32: fp32 rows (any may be absent); weight: one number or
-    one per column.  Returns the new x in the activation type (the next sublayer's input), or None."""
-    assert x.dtype == F32 and x.is_contiguous() and x.dim() == 2 and (a is not None or b is not None or c32 is not None)
+    one per column.  Returns the new x in the activation type (the next sublayer's input), or None.  `moe` (SparseMoE.parts) stands for
+    c32 = the mixture's result."""
+    assert x.dtype == F32 and x.is_contiguous() and x.dim() == 2 and (a is not None or b is not None or c32 is not None or moe is not None)
     rows, dim = x.shape
-    typed = [t for t in (a, b, weight) if t is not None]
+    typed = [t for t in (a, b, weight, moe and moe["y"]) if t is not None]
     f = _act_flag(*typed)
     for t in (a, b, c32):
         assert t is None or (t.shape == (rows, dim) and t.stride(1) == 1)
     assert c32 is None or (c32.dtype == F32 and c32.is_cuda)
     assert weight.numel() in (1, dim) and weight.is_contiguous()
     h = torch.empty(rows, dim, dtype=weight.dtype, device=x.device) if want_h else None
-    _hip.call("nvh_residual_subnorm", _p(a), a.stride(0) if a is not None else 0, float(a_scale), _p(b), b.stride(0) if b is not None else 0, float(b_scale),
+    _hip.call("nvh_residual_subnorm_moe" if moe else "nvh_residual_subnorm", _p(a), a.stride(0) if a is not None else 0, float(a_scale), _p(b), b.stride(0) if b is not None else 0, float(b_scale),
               _p(c32), c32.stride(0) if c32 is not None else 0, float(mult), weight.data_ptr(), weight.numel(), float(eps), x.data_ptr(), _p(h), dim, rows, dim,
-              f, _stream())
+              *(_moe_args(moe, rows, dim, c32) if moe else ()), f, _stream())
     return h
 
 
