@@ -203,6 +203,23 @@ __device__ __forceinline__ void gemm_any_bf16_few_rows(const bf16* __restrict__ 
 // now: 1 x 1024 x 1024 97 -> 6.3, 64 x 4096 x 1024 115 -> 12.7, 301 x 1024 x 1024 108 -> 21, 301 x 6144 x 1024 162 -> 72 (53 TFLOP/s),
 // 1000 x 32768 x 1024 1797 -> 1142 (59 TFLOP/s).
 constexpr int F32_CHUNK = 32;
+// Four consecutive sums of row r of the tile, from column n on, on their way out.
+__device__ __forceinline__ void f32_finish(const f32x4& sum, const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap& rm, int r, int n, int N,
+                                           const float* __restrict__ gate, int64_t ldg, int relu2) {
+    if (r >= rm.rows) return;
+    const int64_t m = rm.dst(r);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        float v = sum[e] + (bias ? bias[n + e] : 0.f);
+        if (gate) v *= sigmoid(gate[m * ldg + n + e]);
+        if (relu2) {
+            v = fmaxf(v, 0.f);
+            v *= v;
+        }
+        y[m * ldy + n + e] = v;
+    }
+}
 template <int MR, int NC, bool VEC>
 __device__ __forceinline__ void gemm_any_f32_tile_body(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
                                                        const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap rm, int r0, int n0, int N,
@@ -295,21 +312,100 @@ __device__ __forceinline__ void gemm_any_f32_tile_body(const float* __restrict__
             const int f = i * MR + j;
             if (f % 4 != wave) continue;
             const f32x4 sum = (lds[f * 64 + lane] + lds[(F + f) * 64 + lane]) + (lds[(2 * F + f) * 64 + lane] + lds[(3 * F + f) * 64 + lane]);
-            const int r = r0 + 16 * j + fr;
-            if (r >= rm.rows) continue;
-            const int64_t m = rm.dst(r);
+            f32_finish(sum, bias, y, ldy, rm, r0 + 16 * j + fr, n0 + 16 * i + 4 * fq, N, gate, ldg, relu2);
+        }
+}
+
+// The same product through LDS (K a multiple of 32, 16-byte rows): every wave has a ring of STAGES chunks of its own there, filled by 16-byte LDS-DMA
+// STAGES chunks ahead, so that neither registers nor barriers bound how much is on its way, and tiles can be larger: what bounds the form above is
+// the operands' way to the CUs, which a 64 x 64 tile has half as much of as four 32 x 32 ones.  Chunks, products and sums as above: bit for bit the
+// same results.
+// us, the form above and this, rows x columns x k: 1 x 1024 x 1024 5.9 and 4.7, 64 x 1024 x 1024 11.6 and 5.2, 64 x 4096 x 1024 13.0 and 9.6,
+// 301 x 1024 x 1024 21.2 and 13.9, 301 x 6144 x 1024 74 and 48 (79 TFLOP/s of the 124 that independent products reach), 512 x 6144 x 1024 111 and 70.
+template <int MR, int NC, int STAGES>
+constexpr int f32_ring_bytes() {
+    return 4 * STAGES * 16 * (MR + NC) * 128;                // (at least the four waves' partial tiles, 1 KB a fragment: STAGES 2 (MR + NC) >= MR NC)
+}
+template <int MR, int NC, int STAGES>
+__device__ __forceinline__ void gemm_any_f32_ring(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, int64_t ldw,
+                                                  const float* __restrict__ bias, float* __restrict__ y, int64_t ldy, const RowMap rm, int r0, int n0, int N,
+                                                  int K, const float* __restrict__ gate, int64_t ldg, int relu2, char* lds) {
+    constexpr int STAGE = 16 * (MR + NC) * 128, PIECES = 2 * (MR + NC);
+    static_assert(STAGES * 2 * (MR + NC) >= MR * NC && PIECES * (STAGES - 1) < 64, "the partial tile fits the ring; vmcnt is six bits");
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, fr = lane & 15, fq = lane >> 4;
+    char* ring = lds + wave * STAGES * STAGE;
+    // A stage: 16 NC rows of w, then 16 MR of x, 32 k (128 bytes) each; 16-byte piece c of row r lies at place c ^ ((r >> 1) & 7), which spreads a
+    // fragment read over all banks.  A DMA instruction brings 8 rows.
+    const float* src[PIECES];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int n = n0 + 16 * i + 4 * fq + e;
-                if (n >= N) continue;
-                float v = sum[e] + (bias ? bias[n] : 0.f);
-                if (gate) v *= sigmoid(gate[m * ldg + n]);
-                if (relu2) {
-                    v = fmaxf(v, 0.f);
-                    v *= v;
-                }
-                y[m * ldy + n] = v;
+    for (int i = 0; i < PIECES; ++i) {
+        const bool of_w = i < 2 * NC;
+        const int r = 8 * (of_w ? i : i - 2 * NC) + (lane >> 3), piece = (lane & 7) ^ ((r >> 1) & 7);
+        const float* row = of_w ? w + (int64_t)min(n0 + r, N - 1) * ldw : x + rm.src(min(r0 + r, rm.rows - 1)) * ldx;      // (repeated rows are not written)
+        src[i] = row + 4 * piece + F32_CHUNK * wave;
+    }
+    const int chunks = K / F32_CHUNK, mine = (chunks - wave + 3) / 4;
+    auto stage = [&](int j) {
+        char* base = ring + j % STAGES * STAGE;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+            __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)(src[i] + 4 * F32_CHUNK * j), (LDS_AS void*)(base + 1024 * i), 16, 0, 0);
+    };
+    f32x4 acc[NC][MR];
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < MR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < STAGES && j < mine; ++j) stage(j);
+    for (int j = 0; j < mine; ++j) {
+        const int ahead = min(STAGES - 1, mine - 1 - j);     // chunks behind this one that may still be on their way
+        if (STAGES > 3 && ahead >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 3 ? 3 * PIECES : 0) : "memory");
+        else if (STAGES > 2 && ahead >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(STAGES > 2 ? 2 * PIECES : 0) : "memory");
+        else if (STAGES > 1 && ahead >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const char *ws = ring + j % STAGES * STAGE, *xs = ws + 16 * NC * 128;
+        f32x4 xf[2][MR], wf[2][NC];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int r = 16 * i + fr;
+                wf[h][i] = *reinterpret_cast<const f32x4*>(ws + r * 128 + (((4 * h + fq) ^ ((r >> 1) & 7)) << 4));
             }
+#pragma unroll
+            for (int i = 0; i < MR; ++i) {
+                const int r = 16 * i + fr;
+                xf[h][i] = *reinterpret_cast<const f32x4*>(xs + r * 128 + (((4 * h + fq) ^ ((r >> 1) & 7)) << 4));
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the chunk is in registers: its stage is free
+        __builtin_amdgcn_sched_barrier(0);
+        if (j + STAGES < mine) stage(j + STAGES);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+#pragma unroll
+                    for (int m = 0; m < MR; ++m) acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[h][i][e], xf[h][m][e], acc[i][m], 0, 0, 0);
+    }
+    f32x4* part = reinterpret_cast<f32x4*>(ring);            // (this wave's ring: nobody else's DMA is under way in it)
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < MR; ++j) part[(i * MR + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    constexpr int RING = STAGES * STAGE / 16;                // (in f32x4)
+    const f32x4* parts = reinterpret_cast<const f32x4*>(lds);
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+        for (int j = 0; j < MR; ++j) {
+            const int f = i * MR + j;
+            if (f % 4 != wave) continue;
+            const f32x4* p = parts + f * 64 + lane;
+            f32_finish((p[0] + p[RING]) + (p[2 * RING] + p[3 * RING]), bias, y, ldy, rm, r0 + 16 * j + fr, n0 + 16 * i + 4 * fq, N, gate, ldg, relu2);
         }
 }
 

@@ -744,6 +744,25 @@ __global__ __launch_bounds__(256) void gemm_any_f32_kernel(const float* __restri
         nvh_any::gemm_any_f32_tile<MR, NC>(x, ldx, w, ldw, bias, y, ldy, nvh_any::RowMap{nullptr, (int)m0, (int)min((int64_t)16 * MR, M - m0)}, 0, blockIdx.x * 16 * NC, N, K, vec_ok);
 }
 
+template <int MR, int NC, int STAGES>
+__global__ __launch_bounds__(256) void gemm_any_f32_ring_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ w, const float* __restrict__ bias,
+                                                                float* __restrict__ y, int64_t ldy, int M, int N, int K) {
+    extern __shared__ __attribute__((aligned(16))) char ring_lds[];
+    for (int64_t m0 = blockIdx.y * 16 * MR; m0 < M; m0 += (int64_t)gridDim.y * 16 * MR) {    // (once, but for more rows than a grid has tiles)
+        nvh_any::gemm_any_f32_ring<MR, NC, STAGES>(x, ldx, w, K, bias, y, ldy, nvh_any::RowMap{nullptr, (int)m0, (int)min((int64_t)16 * MR, M - m0)}, 0,
+                                                   blockIdx.x * 16 * NC, N, K, nullptr, 0, 0, ring_lds);
+        __syncthreads();
+    }
+}
+
+template <int MR, int NC, int STAGES>
+void launch_f32_ring(const float* x, int64_t ldx, const float* w, const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+    constexpr int lds = nvh_any::f32_ring_bytes<MR, NC, STAGES>();
+    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_any_f32_ring_kernel<MR, NC, STAGES>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    gemm_any_f32_ring_kernel<MR, NC, STAGES><<<dim3((unsigned)nvh_cdiv(N, 16 * NC), (unsigned)std::min<int64_t>(nvh_cdiv(M, 16 * MR), 65535)), 256, lds, st>>>(
+        x, ldx, w, bias, y, ldy, (int)M, (int)N, (int)K);
+}
+
 }  // namespace
 
 #define NVH_STREAM_ARGS_OK(name, cond) NVH_REQUIRE(cond, NVH_EINVAL, name ": bad argument")
@@ -836,6 +855,19 @@ extern "C" int32_t nvh_gemm_any_nt(const void* x, int64_t x_row_stride, const vo
     if (in_f32) {
         // (16 rows or fewer: small tiles, so that more workgroups share the weights' stream; the same sums either way)
         const int vec_ok = nvh_any::f32_vec_ok(x, x_row_stride, w, K);
+        if (vec_ok && K % nvh_any::F32_CHUNK == 0) {
+            // The tile whose rounds over the CUs take least.  16 x 16 (two workgroups a CU) and 32 x 32 tiles while they fill at most a round;
+            // then 32 x 64 or 64 x 64 ones, a workgroup a CU, a round of which takes 13 and 22 us for K = 1024.
+            auto tiles = [&](int rows, int cols) { return nvh_cdiv(M, rows) * nvh_cdiv(N, cols); };
+#define NVH_F32_RING(MR, NC, STAGES) launch_f32_ring<MR, NC, STAGES>((const float*)x, x_row_stride, (const float*)w, (const float*)bias, (float*)y, y_row_stride, M, N, K, st)
+            if (tiles(16, 16) <= 512) NVH_F32_RING(1, 1, 4);
+            else if (tiles(32, 32) <= 256) NVH_F32_RING(2, 2, 2);
+            else if (nvh_cdiv(tiles(64, 64), 256) * 22 < nvh_cdiv(tiles(32, 64), 256) * 13) NVH_F32_RING(4, 4, 2);
+            else NVH_F32_RING(2, 4, 2);
+#undef NVH_F32_RING
+            NVH_CHECK_LAUNCH("nvh_gemm_any_nt");
+            return NVH_OK;
+        }
         if (M <= 16) gemm_any_f32_kernel<1, 1><<<dim3((unsigned)nvh_cdiv(N, 16), 1), 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
         else gemm_any_f32_kernel<2, 2><<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)std::min<int64_t>(nvh_cdiv(M, 32), 65535)), 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
     } else {

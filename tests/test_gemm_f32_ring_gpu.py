@@ -1,0 +1,23 @@
+"""fp32 products through the waves' LDS rings: the bits of the form that reads any row, at the edges of tiles and of a wave's chunks."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def odd_rows(t):
+    wide = torch.empty(t.shape[0], t.shape[1] + 1, device=t.device)
+    wide[:, :-1] = t
+    return wide[:, :-1]
+
+
+@pytest.mark.parametrize("k", [32, 96, 128, 160, 256, 416, 1024])
+@pytest.mark.parametrize("m,n", [(1, 1), (16, 16), (17, 63), (32, 64), (33, 65), (64, 100), (65, 128), (130, 1030), (300, 2050)])
+def test_plain(m, n, k):
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(m * n + k)
+    x, w, b = torch.randn(m, k, generator=g).cuda(), torch.randn(n, k, generator=g).cuda(), torch.randn(n, generator=g).cuda()
+    want = ops.linear_any(odd_rows(x), w, b)
+    assert torch.equal(ops.linear_any(x, w, b), want)
+    for r in {0, m // 2, m - 1}:
+        assert torch.equal(ops.linear_any(x[r:r + 1].contiguous(), w, b)[0], want[r])
