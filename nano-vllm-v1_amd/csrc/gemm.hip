@@ -1482,6 +1482,14 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
         case T32x128: launch_gemm<32, 128, 4, 1, 4>(a); break;
         case T64x128: launch_gemm<64, 128, 2, 2, 4>(a); break;
         case T64x64: {
+            // 33 .. 64 rows: 64-column tiles leave most CUs without one, and what a workgroup waits for is its stages; 16 columns (32 where 16 would be
+            // more than a workgroup a CU) with six stages.  64 rows x N x 1024, us before and now: 1024 7.7 and 6.5, 2048 7.9 and 6.7, 4096 8.0 and 7.1,
+            // 6144 8.3 and 7.7, 8192 8.6 and 8.4.  The same sums in the same order.
+            if (a.M <= 64 && a.split_k == 1 && !a.swiglu && !a.qkv && !a.sample && a.N <= 32 * 256) {
+                if (a.N <= 16 * 256) launch_gemm<64, 16, 1, 4, 6>(a);
+                else launch_gemm<64, 32, 2, 2, 6>(a);
+                break;
+            }
             if (!a.swiglu && a.qkv == nullptr && a.sample == nullptr && a.split_k == 1 && a.partials == nullptr &&
                 (a.y != nullptr || a.residual != nullptr) && takes_kgroups(a.M, a.N, a.K))
                 launch_gemm_kgroups(a);
