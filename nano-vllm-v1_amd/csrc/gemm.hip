@@ -1496,7 +1496,13 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
             else launch_gemm<64, 64, 2, 2, 4>(a);
             break;
         }
-        case T128x64: launch_gemm<128, 64, 2, 2, 4>(a); break;
+        case T128x64:
+            // One workgroup fits a CU, so a grid a little over 256 takes two rounds: then 128 x 128 tiles, fewer than 200 of them, in one round, eight
+            // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 14.9, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
+            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4; one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  The same sums.
+            if (a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
+            else launch_gemm<128, 64, 2, 2, 4>(a);
+            break;
         case T128x128: {
             // up to one workgroup per CU: nothing shares the CU's LDS, so a third stage (96 KB) keeps two tiles in
             // flight instead of one (1024 x 4096 x 1024: 19.1 -> 17.2 us); larger grids want two residents of 64 KB
