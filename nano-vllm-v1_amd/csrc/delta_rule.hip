@@ -121,6 +121,118 @@ __global__ __launch_bounds__(256) void gated_delta_prep_kernel(GatedDeltaPrepArg
     for (int i = threadIdx.x; i < dv; i += 256) out[5 * dk + i] = sh[2 * dk + i];
 }
 
+// The same for TT consecutive tokens a workgroup: a lane has a channel's weights and its inputs of all of them on the way at once and reads an input
+// once instead of once per tap.  Same sums in the same order.
+// us, one token a workgroup and two or four, heads of 128 x 128: 1000 tokens of 8 heads 33.5 and 17.4 (25 MB written), of 4 15.7 and 11.2, 2000 of 8 61.6 and
+// 28.8, 300 of 8 11.4 and 8.3; eight tokens a workgroup 19.2, 15.7, 30.2, 11.5.
+template <typename A, int TT, int TAPS>
+__global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPrepArgs p, int64_t num_tokens, int vec) {
+    extern __shared__ __attribute__((aligned(16))) float sh[];                            // [TT][n] q (dk) | k (dk) | v (dv) of this head, then the numbers of the tokens
+    __shared__ int first_of[TT], state_of[TT];               // the first row of the token's sequence in this step; its slot, or -1: nothing carried
+    const int64_t t0 = (int64_t)blockIdx.x * TT;
+    const int nt = (int)min((int64_t)TT, num_tokens - t0), tid = threadIdx.x;
+    const int h = blockIdx.y, dk = p.dk, dv = p.dv, g = h / (p.H / p.G);
+    const int nqk = p.G * dk, C = 2 * nqk + p.H * dv, n = 2 * dk + dv;
+    float *inv = sh + TT * n, *beta = inv + 2 * TT, *dec = beta + TT;
+    if (tid < TT) {
+        const int64_t t = t0 + min(tid, nt - 1);
+        int seq = (int)t, lo = (int)t, hi = (int)t + 1;
+        if (p.cu_seqlens_q) {
+            int lo_b = 0, hi_b = p.batch;                    // the sequence whose rows hold token t
+            while (hi_b - lo_b > 1) {
+                const int mid = (lo_b + hi_b) >> 1;
+                if (p.cu_seqlens_q[mid] <= t) lo_b = mid;
+                else hi_b = mid;
+            }
+            seq = lo_b;
+            lo = p.cu_seqlens_q[seq];
+            hi = p.cu_seqlens_q[seq + 1];
+        }
+        const int slot = p.slots[seq];
+        first_of[tid] = lo;
+        state_of[tid] = slot >= 0 && p.context_lens[seq] != hi - lo ? slot : -1;
+        beta[tid] = sigmoidf_(ldf((const A*)p.b, t * p.b_stride + h));
+        dec[tid] = expf(-expf(ldf((const A*)p.a_log, h)) * softplusf_(ldf((const A*)p.a, t * p.a_stride + h) + ldf((const A*)p.dt_bias, h)));
+    }
+    __syncthreads();
+    for (int e = tid; e < n; e += 256) {
+        const int c = e < dk ? g * dk + e : (e < 2 * dk ? nqk + g * dk + (e - dk) : 2 * nqk + h * dv + (e - 2 * dk));      // the channel of the row
+        float w[TAPS], in[TT + TAPS - 1];                    // in[u]: the input of token t0 - (TAPS - 1) + u (rows outside the step: any, not used)
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) w[k] = ldf((const A*)p.conv_w, (int64_t)c * TAPS + k);
+#pragma unroll
+        for (int u = 0; u < TT + TAPS - 1; ++u) in[u] = ldf((const A*)p.qkv, min(max(t0 - (TAPS - 1) + u, (int64_t)0), num_tokens - 1) * p.qkv_stride + c);
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            const int j = (int)(t0 + tt) - first_of[tt];     // tokens of the sequence before this one in the step
+            const float* st = state_of[tt] >= 0 ? p.conv_state + (int64_t)state_of[tt] * (TAPS - 1) * C + c : nullptr;
+            float acc = 0.f;
+#pragma unroll
+            for (int k = 0; k < TAPS; ++k) {                 // tap k multiplies the input TAPS - 1 - k tokens back
+                const int src = j - (TAPS - 1 - k);
+                float x = in[tt + k];
+                if (src < 0) x = st ? st[(int64_t)(TAPS - 1 + src) * C] : 0.f;
+                acc = __builtin_fmaf(w[k], x, acc);
+            }
+            if (tt < nt) sh[tt * n + e] = acc / (1.0f + expf(-acc));
+        }
+    }
+    __syncthreads();
+    const int wave = tid >> 6, lane = tid & 63;
+    for (int i = wave; i < 2 * nt; i += 4) {                 // q, k of every token
+        const float* x = sh + (i >> 1) * n + (i & 1) * dk;
+        float ss = 0.f;
+        for (int c = lane; c < dk; c += 64) ss += x[c] * x[c];
+        ss = wave_sum(ss);
+        if (lane == 0) inv[i] = 1.0f / sqrtf(ss + 1e-6f);
+    }
+    __syncthreads();
+    const int row = 5 * dk + dv;
+    float* out = p.out + (t0 * p.H + h) * (int64_t)row;
+    const float scale = sqrtf((float)dk);
+    auto rows_out = [&](auto piece) {                        // (a piece: one number, or four where every part of a row is a multiple of four)
+        using V = decltype(piece);
+        constexpr int W = sizeof(V) / sizeof(float);
+        for (int i = tid; i < nt * dk / W; i += 256) {
+            const int tt = i * W / dk, c = i * W - tt * dk;
+            float* o = out + (int64_t)tt * p.H * row + c;
+            const float* x = sh + tt * n + c;
+            const float qs = inv[2 * tt] / scale, ks = inv[2 * tt + 1], b = beta[tt], d = dec[tt];
+            V q = *reinterpret_cast<const V*>(x), k = *reinterpret_cast<const V*>(x + dk), bk, bdk, dd;
+#pragma unroll
+            for (int e = 0; e < W; ++e) {
+                float *qe = reinterpret_cast<float*>(&q) + e, *ke = reinterpret_cast<float*>(&k) + e;
+                *qe *= qs;
+                *ke *= ks;
+                reinterpret_cast<float*>(&bk)[e] = b * *ke;
+                reinterpret_cast<float*>(&bdk)[e] = b * d * *ke;
+                reinterpret_cast<float*>(&dd)[e] = d;
+            }
+            *reinterpret_cast<V*>(o) = q;
+            *reinterpret_cast<V*>(o + dk) = bk;
+            *reinterpret_cast<V*>(o + 2 * dk) = dd;
+            *reinterpret_cast<V*>(o + 3 * dk) = k;
+            *reinterpret_cast<V*>(o + 4 * dk) = bdk;
+        }
+        for (int i = tid; i < nt * dv / W; i += 256) {
+            const int tt = i * W / dv, c = i * W - tt * dv;
+            *reinterpret_cast<V*>(out + (int64_t)tt * p.H * row + 5 * dk + c) = *reinterpret_cast<const V*>(sh + tt * n + 2 * dk + c);
+        }
+    };
+    if (vec) rows_out(f32x4{});                              // (uniform)
+    else rows_out(0.f);
+}
+
+template <int TT>
+void launch_gated_delta_prep_run(const GatedDeltaPrepArgs& p, int64_t num_tokens, bool act_f32, hipStream_t st) {
+    const dim3 grid((unsigned)nvh_cdiv(num_tokens, TT), (unsigned)p.H);
+    const size_t lds = sizeof(float) * (size_t)(TT * (2 * p.dk + p.dv) + 4 * TT);
+    const int vec = p.dk % 4 == 0 && p.dv % 4 == 0 && nvh_aligned16(p.out);
+    auto launch = [&](auto kernel) { kernel<<<grid, 256, lds, st>>>(p, num_tokens, vec); };
+    if (act_f32) launch(p.taps == 2 ? &gated_delta_prep_run_kernel<float, TT, 2> : p.taps == 3 ? &gated_delta_prep_run_kernel<float, TT, 3> : &gated_delta_prep_run_kernel<float, TT, 4>);
+    else launch(p.taps == 2 ? &gated_delta_prep_run_kernel<bf16, TT, 2> : p.taps == 3 ? &gated_delta_prep_run_kernel<bf16, TT, 3> : &gated_delta_prep_run_kernel<bf16, TT, 4>);
+}
+
 // TT tokens a workgroup share every row of W2, which a lane reads for its channel (VEC: 16 bytes at a time); the order of a logit's sum is the same
 // for any TT.  Read once per token, two bytes at a time, those rows bound the launch: 1024 tokens, 16 heads of 64, rank 64, 36.7 us; four tokens a
 // workgroup 13.0 us, of which the 25 MB that it writes cannot do without 5.
@@ -950,9 +1062,15 @@ extern "C" int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, con
     GatedDeltaPrepArgs p{qkv, qkv_stride, b, a, b_stride, a_stride, conv_w, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens, out,
                          (int)batch, (int)taps, (int)heads, (int)qk_heads, (int)dk, (int)dv};
     hipStream_t st = (hipStream_t)stream;
-    const dim3 grid((unsigned)num_tokens, (unsigned)heads);
-    if (act_f32) gated_delta_prep_kernel<float><<<grid, 256, lds, st>>>(p);
-    else gated_delta_prep_kernel<bf16><<<grid, 256, lds, st>>>(p);
+    // Tokens a workgroup: four, or two where four leave the chip fewer than four workgroups a CU; below two a CU one token each, as ever.
+    const bool run = taps >= 2 && taps <= 4 && (2 * dk + dv + 4) * 4 * (int64_t)sizeof(float) <= 32 * 1024;
+    if (run && num_tokens * heads >= 4096) launch_gated_delta_prep_run<4>(p, num_tokens, act_f32, st);
+    else if (run && num_tokens * heads >= 1024) launch_gated_delta_prep_run<2>(p, num_tokens, act_f32, st);
+    else {
+        const dim3 grid((unsigned)num_tokens, (unsigned)heads);
+        if (act_f32) gated_delta_prep_kernel<float><<<grid, 256, lds, st>>>(p);
+        else gated_delta_prep_kernel<bf16><<<grid, 256, lds, st>>>(p);
+    }
     NVH_CHECK_LAUNCH("nvh_gated_delta_prep");
     return NVH_OK;
 }
