@@ -763,6 +763,13 @@ int32_t nvh_conv_state_update(const void* xbc, int64_t xbc_stride, float* conv_s
 int32_t nvh_stream_conv(const float* x, const void* w, const float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
                         const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
                         int32_t act_f32, nvh_stream_t stream);
+/* One token per sequence (no cu_seqlens_q): nvh_ssd_conv_prep / nvh_stream_conv with the nvh_conv_state_update that follows them. */
+int32_t nvh_ssd_conv_prep_step(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
+                               const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* context_lens,
+                               int64_t batch, int64_t taps, int64_t heads, int64_t inner, int64_t gn, float* out_x, float* out_b, float* out_c,
+                               float* out_dt, float* out_decay, int32_t act_f32, nvh_stream_t stream);
+int32_t nvh_stream_conv_step(const float* x, const void* w, float* state, const int32_t* slots, const int32_t* context_lens, void* h,
+                             int64_t h_stride, int64_t batch, int64_t taps, int64_t dim, int32_t act_f32, nvh_stream_t stream);
 int32_t nvh_group_rmsnorm_gate(const float* o, const void* weight, int32_t weight_full, const void* gate, int64_t gate_stride,
                                int32_t gate_act, int32_t gate_first, void* y, int64_t y_stride, int64_t rows, int64_t groups,
                                int64_t group_size, float eps, int32_t act_f32, nvh_stream_t stream);

@@ -226,6 +226,7 @@ struct SsdPrepArgs {
     const int32_t *slots, *cu_seqlens_q, *context_lens;
     int batch, taps, H, inner, gn;  // inner = H dv, gn = G N; C = inner + 2 gn
     float *ov, *ok, *oq, *oc, *ow;  // fp32 [T, inner], [T, gn] (B), [T, gn] (C), [T, H] (dt), [T, H] (decay)
+    int step;                  // one token per sequence whose slots are brought up to date on the way (the vector form alone)
 };
 
 template <typename A>
@@ -273,6 +274,7 @@ __global__ __launch_bounds__(256) void ssd_conv_prep_vec_kernel(SsdPrepArgs p) {
     const int C = p.inner + 2 * p.gn;
     const float* st = carried ? p.conv_state + (int64_t)slot * (TAPS - 1) * C : nullptr;
     for (int c = (blockIdx.y * 256 + threadIdx.x) * 8; c < C; c += 256 * 8 * gridDim.y) {
+        float keep[TAPS - 1][8];                             // step: what the slot holds next, this lane's channels being nobody else's
         float acc[8], wf[8 * TAPS];                          // wf[i * TAPS + k]: channel c + i, tap k (as the weights lie)
         if (p.conv_b) {
             nvh_load8((const A*)p.conv_b, c, 8, true, acc);
@@ -300,7 +302,18 @@ __global__ __launch_bounds__(256) void ssd_conv_prep_vec_kernel(SsdPrepArgs p) {
                 for (int i = 0; i < 8; ++i) in[i] = 0.f;
             }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) acc[i] = __builtin_fmaf(wf[i * TAPS + k], in[i], acc[i]);
+            for (int i = 0; i < 8; ++i) {
+                acc[i] = __builtin_fmaf(wf[i * TAPS + k], in[i], acc[i]);
+                if (k > 0) keep[k - 1][i] = in[i];
+            }
+        }
+        if (p.step && slot >= 0) {                           // (uniform)
+            float* out = p.conv_state + (int64_t)slot * (TAPS - 1) * C + c;
+#pragma unroll
+            for (int k = 0; k < TAPS - 1; ++k) {
+                *reinterpret_cast<f32x4*>(out + (int64_t)k * C) = f32x4{keep[k][0], keep[k][1], keep[k][2], keep[k][3]};
+                *reinterpret_cast<f32x4*>(out + (int64_t)k * C + 4) = f32x4{keep[k][4], keep[k][5], keep[k][6], keep[k][7]};
+            }
         }
         float* dst = c < p.inner ? p.ov + t * p.inner + c : (c < p.inner + p.gn ? p.ok + t * p.gn + (c - p.inner) : p.oq + t * p.gn + (c - p.inner - p.gn));
         f32x4 lo4, hi4;
@@ -378,6 +391,77 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(StreamConvArgs p) {
         }
         h[c] = (A)(cur + acc);
     }
+}
+
+// The same for TT consecutive tokens a workgroup, four columns a lane: everything a lane reads is on its way at once, an input once instead of once
+// per tap.  STEP (TT 1, one token per sequence): the slot is brought up to date as well - the lane that reads a column's carried inputs is the only
+// one that does.
+// us, four taps over 1024 columns, with the state's update: 1000 tokens 8.2 (one workgroup a token) and 6.2, 2000 13.8 and 6.8; one token of 64 sequences, where
+// the update is inside, 4.7 and 2.5.
+template <typename A, int TT, int TAPS, bool STEP>
+__global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, int64_t num_tokens, float* carried_out) {
+    static_assert(!STEP || TT == 1, "a step brings one token per sequence");
+    const int64_t t0 = (int64_t)blockIdx.x * TT;
+    const int dim = p.dim, col = (blockIdx.y * 256 + threadIdx.x) * 4;
+    if (col >= dim) return;
+    f32x4 in[TT + TAPS - 1], w[TAPS];                        // in[u]: token t0 - (TAPS - 1) + u (rows outside the step: any, not used); w[k]: tap k
+#pragma unroll
+    for (int u = 0; u < TT + TAPS - 1; ++u)
+        if (!STEP || u == TAPS - 1) in[u] = *reinterpret_cast<const f32x4*>(p.x + min(max(t0 - (TAPS - 1) + u, (int64_t)0), num_tokens - 1) * dim + col);
+    {
+        float wf[4 * TAPS];
+#pragma unroll
+        for (int i = 0; i < 4 * TAPS; ++i) wf[i] = ldf((const A*)p.w, (int64_t)col * TAPS + i);
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) w[k] = f32x4{wf[k], wf[TAPS + k], wf[2 * TAPS + k], wf[3 * TAPS + k]};
+    }
+    int seq = seq_of_token(p.cu_seqlens_q, p.batch, t0);
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) {
+        const int64_t t = t0 + tt;
+        if (t >= num_tokens) break;                          // (uniform, as what follows up to the columns)
+        if (p.cu_seqlens_q)
+            while (seq + 1 < p.batch && p.cu_seqlens_q[seq + 1] <= t) ++seq;
+        const int lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : (int)t, hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : (int)t + 1;
+        if (!p.cu_seqlens_q) seq = (int)t;
+        const int j = (int)t - lo, slot = p.slots[seq];
+        const bool carried = slot >= 0 && p.context_lens[seq] != hi - lo;
+        const float* st = carried ? p.state + (int64_t)slot * (TAPS - 1) * dim + col : nullptr;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, kept[TAPS];
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) {
+            const int src = j - (TAPS - 1 - k);
+            f32x4 x = in[STEP ? TAPS - 1 : tt + k];
+            if (src < 0) x = st ? *reinterpret_cast<const f32x4*>(st + (int64_t)(TAPS - 1 + src) * dim) : f32x4{0.f, 0.f, 0.f, 0.f};
+            kept[k] = x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w[k][e], x[e], acc[e]);
+        }
+        if (STEP && slot >= 0)
+#pragma unroll
+            for (int k = 0; k < TAPS - 1; ++k) *reinterpret_cast<f32x4*>(carried_out + ((int64_t)slot * (TAPS - 1) + k) * dim + col) = kept[k + 1];
+        const f32x4 h = in[tt + TAPS - 1] + acc;
+        A* dst = (A*)p.h + t * p.h_stride + col;
+        if constexpr (sizeof(A) == 4) *reinterpret_cast<f32x4*>(dst) = h;
+        else *reinterpret_cast<bf16x4*>(dst) = bf16x4{(bf16)h[0], (bf16)h[1], (bf16)h[2], (bf16)h[3]};
+    }
+}
+
+// (false: taps, columns or alignment that the form above does not serve)
+template <typename A>
+static bool launch_stream_conv_run(const StreamConvArgs& p, int64_t num_tokens, int taps, float* carried_out, hipStream_t st) {
+    if (taps < 2 || taps > 4 || p.dim % 4 || p.h_stride % 4 || !nvh_aligned16(p.x) || !nvh_aligned16(p.state) || ((uintptr_t)p.h % (4 * sizeof(A)))) return false;
+    constexpr int TT = 4;
+    const unsigned cols = (unsigned)nvh_cdiv(p.dim, 1024);
+#define NVH_CONV_RUN(TAPS)                                                                                                                                   \
+    if (carried_out) stream_conv_run_kernel<A, 1, TAPS, true><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, carried_out);               \
+    else if (num_tokens >= 256 * TT / 2) stream_conv_run_kernel<A, TT, TAPS, false><<<dim3((unsigned)nvh_cdiv(num_tokens, TT), cols), 256, 0, st>>>(p, num_tokens, nullptr); \
+    else stream_conv_run_kernel<A, 1, TAPS, false><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, nullptr)
+    if (taps == 2) { NVH_CONV_RUN(2); }
+    else if (taps == 3) { NVH_CONV_RUN(3); }
+    else { NVH_CONV_RUN(4); }
+#undef NVH_CONV_RUN
+    return true;
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1183,15 +1267,14 @@ static int32_t ssd_args(SsdPrepArgs& p, const void* xbc, int64_t xbc_stride, con
     NVH_REQUIRE(xbc && conv_w && slots && context_lens && (taps == 1 || conv_state), NVH_EINVAL, "ssd convolution: null pointer");
     NVH_REQUIRE(batch >= 0 && taps >= 1 && taps <= 64 && heads > 0 && inner > 0 && gn > 0 && xbc_stride >= inner + 2 * gn, NVH_EINVAL, "ssd convolution: bad sizes");
     p = SsdPrepArgs{xbc, xbc_stride, dt, dt_stride, conv_w, conv_b, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens,
-                    (int)batch, (int)taps, (int)heads, (int)inner, (int)gn, nullptr, nullptr, nullptr, nullptr, nullptr};
+                    (int)batch, (int)taps, (int)heads, (int)inner, (int)gn, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_ssd_conv_prep(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
-                                     const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* cu_seqlens_q,
-                                     const int32_t* context_lens, int64_t batch, int64_t num_tokens, int64_t taps, int64_t heads, int64_t inner,
-                                     int64_t gn, float* out_x, float* out_b, float* out_c, float* out_dt, float* out_decay, int32_t act_f32,
-                                     nvh_stream_t stream) {
+static int32_t ssd_conv_prep(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
+                             const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                             const int32_t* context_lens, int64_t batch, int64_t num_tokens, int64_t taps, int64_t heads, int64_t inner, int64_t gn,
+                             float* out_x, float* out_b, float* out_c, float* out_dt, float* out_decay, int step, int32_t act_f32, nvh_stream_t stream) {
     SsdPrepArgs p;
     const int32_t rc = ssd_args(p, xbc, xbc_stride, dt, dt_stride, conv_w, conv_b, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens, batch, taps, heads, inner, gn);
     if (rc != NVH_OK) return rc;
@@ -1206,6 +1289,7 @@ extern "C" int32_t nvh_ssd_conv_prep(const void* xbc, int64_t xbc_stride, const 
                      (!conv_b || nvh_aligned16(conv_b)) && nvh_aligned16(conv_state) && nvh_aligned16(out_x) && nvh_aligned16(out_b) && nvh_aligned16(out_c);
     const int64_t lanes = vec ? (inner + 2 * gn) / 8 : inner + 2 * gn;
     const dim3 grid((unsigned)num_tokens, (unsigned)(num_tokens >= 512 ? 1 : std::min<int64_t>(nvh_cdiv(lanes, 256), 16)));
+    p.step = step;
     if (vec) {
 #define NVH_CONV_VEC(TAPS)                                                        \
     if (act_f32) ssd_conv_prep_vec_kernel<float, TAPS><<<grid, 256, 0, st>>>(p); \
@@ -1220,7 +1304,25 @@ extern "C" int32_t nvh_ssd_conv_prep(const void* xbc, int64_t xbc_stride, const 
         ssd_conv_prep_kernel<bf16><<<grid, 256, 0, st>>>(p);
     }
     NVH_CHECK_LAUNCH("nvh_ssd_conv_prep");
+    if (step && !vec) return nvh_conv_state_update(xbc, xbc_stride, conv_state, slots, nullptr, context_lens, batch, taps, inner + 2 * gn, act_f32, stream);
     return NVH_OK;
+}
+
+extern "C" int32_t nvh_ssd_conv_prep(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
+                                     const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                     const int32_t* context_lens, int64_t batch, int64_t num_tokens, int64_t taps, int64_t heads, int64_t inner,
+                                     int64_t gn, float* out_x, float* out_b, float* out_c, float* out_dt, float* out_decay, int32_t act_f32,
+                                     nvh_stream_t stream) {
+    return ssd_conv_prep(xbc, xbc_stride, dt, dt_stride, conv_w, conv_b, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens, batch, num_tokens,
+                         taps, heads, inner, gn, out_x, out_b, out_c, out_dt, out_decay, 0, act_f32, stream);
+}
+
+extern "C" int32_t nvh_ssd_conv_prep_step(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
+                                          const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* context_lens,
+                                          int64_t batch, int64_t taps, int64_t heads, int64_t inner, int64_t gn, float* out_x, float* out_b,
+                                          float* out_c, float* out_dt, float* out_decay, int32_t act_f32, nvh_stream_t stream) {
+    return ssd_conv_prep(xbc, xbc_stride, dt, dt_stride, conv_w, conv_b, dt_bias, a_log, conv_state, slots, nullptr, context_lens, batch, batch, taps, heads,
+                         inner, gn, out_x, out_b, out_c, out_dt, out_decay, taps > 1, act_f32, stream);
 }
 
 extern "C" int32_t nvh_conv_state_update(const void* xbc, int64_t xbc_stride, float* conv_state, const int32_t* slots, const int32_t* cu_seqlens_q,
@@ -1239,9 +1341,9 @@ extern "C" int32_t nvh_conv_state_update(const void* xbc, int64_t xbc_stride, fl
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_stream_conv(const float* x, const void* w, const float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
-                                   const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
-                                   int32_t act_f32, nvh_stream_t stream) {
+static int32_t stream_conv(const float* x, const void* w, const float* state, float* state_out, const int32_t* slots, const int32_t* cu_seqlens_q,
+                           const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim, int32_t act_f32,
+                           nvh_stream_t stream) {
     NVH_REQUIRE(x && w && slots && context_lens && h && batch >= 0 && num_tokens >= 0 && taps >= 1 && dim > 0 && h_stride >= dim, NVH_EINVAL,
                 "nvh_stream_conv: bad argument");
     NVH_REQUIRE(taps == 1 || state, NVH_EINVAL, "nvh_stream_conv: null state");
@@ -1249,11 +1351,26 @@ extern "C" int32_t nvh_stream_conv(const float* x, const void* w, const float* s
     if (num_tokens == 0 || batch == 0) return NVH_OK;
     const StreamConvArgs p{x, w, state, slots, cu_seqlens_q, context_lens, h, h_stride, (int)batch, (int)taps, (int)dim};
     hipStream_t st = (hipStream_t)stream;
+    if (act_f32 ? launch_stream_conv_run<float>(p, num_tokens, (int)taps, state_out, st) : launch_stream_conv_run<bf16>(p, num_tokens, (int)taps, state_out, st)) {
+        NVH_CHECK_LAUNCH("nvh_stream_conv");
+        return NVH_OK;
+    }
     const dim3 grid((unsigned)num_tokens, (unsigned)(num_tokens >= 512 ? 1 : std::min<int64_t>(nvh_cdiv(dim, 256), 16)));
     if (act_f32) stream_conv_kernel<float><<<grid, 256, 0, st>>>(p);
     else stream_conv_kernel<bf16><<<grid, 256, 0, st>>>(p);
     NVH_CHECK_LAUNCH("nvh_stream_conv");
-    return NVH_OK;
+    return state_out ? nvh_conv_state_update(x, dim, state_out, slots, nullptr, context_lens, batch, taps, dim, 1, stream) : NVH_OK;
+}
+
+extern "C" int32_t nvh_stream_conv(const float* x, const void* w, const float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                   const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
+                                   int32_t act_f32, nvh_stream_t stream) {
+    return stream_conv(x, w, state, nullptr, slots, cu_seqlens_q, context_lens, h, h_stride, batch, num_tokens, taps, dim, act_f32, stream);
+}
+
+extern "C" int32_t nvh_stream_conv_step(const float* x, const void* w, float* state, const int32_t* slots, const int32_t* context_lens, void* h,
+                                        int64_t h_stride, int64_t batch, int64_t taps, int64_t dim, int32_t act_f32, nvh_stream_t stream) {
+    return stream_conv(x, w, state, taps > 1 ? state : nullptr, slots, nullptr, context_lens, h, h_stride, batch, batch, taps, dim, act_f32, stream);
 }
 
 // Key sizes whose scan has the segmented form (the exact instantiations below).

@@ -979,6 +979,11 @@ def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor | Non
     assert taps == 1 or (state.dtype == F32 and state.is_contiguous() and tuple(state.shape[1:]) == (taps - 1, dim))
     assert slots.dtype == torch.int32 and context_lens.dtype == torch.int32 and (cu_seqlens_q is None or cu_seqlens_q.dtype == torch.int32)
     h = torch.empty(t, dim, dtype=weight.dtype, device=x.device)
+    if cu_seqlens_q is None:                                  # one token per sequence: one launch does both
+        assert t == batch
+        _hip.call("nvh_stream_conv_step", x.data_ptr(), weight.data_ptr(), _p(state), slots.data_ptr(), context_lens.data_ptr(), h.data_ptr(), dim, batch, taps,
+                  dim, f, _stream())
+        return h
     _hip.call("nvh_stream_conv", x.data_ptr(), weight.data_ptr(), _p(state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), h.data_ptr(), dim,
               batch, t, taps, dim, f, _stream())
     _hip.call("nvh_conv_state_update", x.data_ptr(), dim, _p(state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch, taps, dim, 1, _stream())
@@ -1218,6 +1223,12 @@ def ssd_conv_prep(xbc, dt, conv_w, conv_b, dt_bias, a_log, conv_state, slots, cu
     ox = torch.empty(t, inner, dtype=F32, device=xbc.device)
     ob, oc = (torch.empty(t, gn, dtype=F32, device=xbc.device) for _ in range(2))
     odt, odecay = (torch.empty(t, heads, dtype=F32, device=xbc.device) for _ in range(2))
+    if cu_seqlens_q is None:                                  # one token per sequence: one launch does both
+        assert t == batch
+        _hip.call("nvh_ssd_conv_prep_step", xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0), conv_w.data_ptr(), _p(conv_b), dt_bias.data_ptr(),
+                  a_log.data_ptr(), _p(conv_state), slots.data_ptr(), context_lens.data_ptr(), batch, taps, heads, inner, gn, ox.data_ptr(), ob.data_ptr(),
+                  oc.data_ptr(), odt.data_ptr(), odecay.data_ptr(), fl, _stream())
+        return ox, ob, oc, odt, odecay
     _hip.call("nvh_ssd_conv_prep", xbc.data_ptr(), xbc.stride(0), dt.data_ptr(), dt.stride(0), conv_w.data_ptr(), _p(conv_b), dt_bias.data_ptr(),
               a_log.data_ptr(), _p(conv_state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch, t, taps, heads, inner, gn,
               ox.data_ptr(), ob.data_ptr(), oc.data_ptr(), odt.data_ptr(), odecay.data_ptr(), fl, _stream())
