@@ -182,8 +182,30 @@ def check(code: int, what: str) -> None:
         raise HipError(f"{what} failed ({code}): {lib().nvh_last_error().decode()}")
 
 
-def call(name: str, *args) -> None:
+def _ctypes_call(name: str, *args) -> None:
     check(getattr(lib(), name)(*args), name)
+
+
+def native_caller(handle, signatures, check_fn):
+    """call(name, *args) in C (csrc/host/hostpath.c) for the functions of `handle` that return an int32, or None where that module is not built."""
+    try:
+        from ._hostpath import Caller
+    except ImportError:
+        return None
+    table = {}
+    for name, (res, args) in signatures.items():
+        fn = getattr(handle, name)
+        kinds = "".join("f" if a is f32 else "i" for a in args)
+        plain = res is i32 and all(a in (vp, i64, u64, i32, f32) for a in args) and kinds.count("f") <= 8 and kinds.count("i") <= 46
+        table[name] = (C.cast(fn, C.c_void_p).value if plain else 0, kinds, fn)
+    return Caller(table, check_fn)
+
+
+def call(name: str, *args) -> None:
+    """The function's int32 result is an error code: anything but 0 raises.  (Replaced by the native caller with the first call, where there is one.)"""
+    global call
+    call = native_caller(lib(), SIGNATURES, check) or _ctypes_call
+    call(name, *args)
 
 
 class switch:
