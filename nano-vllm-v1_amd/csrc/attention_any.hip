@@ -893,8 +893,10 @@ __device__ __forceinline__ void balanced_place(const AttnArgs& a, int* keys, int
     __syncthreads();                                         // (the place is used for other things from here on)
 }
 
+// (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
+constexpr int attn_waves(int nks, int nvt, int mode, int var) { return nks + nvt <= 4 ? 4 : nks + nvt <= (mode == 1 && nvt <= 4 && var != VAR_EXT ? 12 : 8) ? 3 : nks + nvt <= 16 ? 2 : 1; }
 template <int NKS, int NVT, bool EXACT, int MODE, int VAR>
-__global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_paged_mfma_kernel(AttnArgs a) {
     constexpr bool GROUPED = MODE == 1;                      // rows are the heads of a KV group (one query per sequence)
     constexpr bool EXT = VAR == VAR_EXT, BIAS = VAR == VAR_BIAS;
     constexpr bool SPLIT = MODE != 0;                        // the waves share 16 rows and split the keys
@@ -1054,9 +1056,16 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
     const int nblocks = EXT && a.pool > 0 ? blocks_seen(last_key, a.window, a.pool) : 0, my_blocks = EXT && a.pool > 0 ? blocks_seen(qpos, a.window, a.pool) : 0;
     // keys a row sees: lo_window (or one of the first keep_first) and lo_chunk at least, qpos at most
     const int lo_window = a.window > 0 ? qpos - a.window + 1 : 0, lo_chunk = a.chunk > 0 ? qpos / a.chunk * a.chunk : 0;
+    // A tile between these two is seen whole by every row of the wave (uniform): nothing to mask.  Most of a long context is, and the work per
+    // score bounds the loop.
+    // us, every tile masked and so: 16 heads of 128 x 128 over 8, prompts of 1024 tokens 57.3 and 45.6, 32 of 1000 727 and 577, 1024 behind 3072 204 and 156, 8 of
+    // 100 14.6 and 13.4; 64 single tokens behind 1024 57.8 and 55.2.
+    const int wave_first = __builtin_amdgcn_readfirstlane(SPLIT ? qpos : past + q0 + wave * 16), wave_lastq = __builtin_amdgcn_readfirstlane(wave_last);
+    const int whole_from = max(a.window > 0 ? wave_lastq - a.window + 1 : 0, a.chunk > 0 ? wave_lastq / a.chunk * a.chunk : 0);
+    const int whole_to = a.slopes ? -1 : wave_first - MK + 1;                // (first keys from .. to, both included)
     // The tile in LDS, its first key k0 (pooled_tile: its first block) against this wave's queries.
-    auto compute = [&](auto pooled_tile, int k0) {
-        constexpr bool POOLED = decltype(pooled_tile)::value;
+    auto compute = [&](auto pooled_tile, auto whole_tile, int k0) {
+        constexpr bool POOLED = decltype(pooled_tile)::value, WHOLE = decltype(whole_tile)::value;
         // (wave-uniform; no barrier below)
         if (wave_idle || (POOLED ? k0 >= blocks_seen(wave_last, a.window, a.pool) : k0 > wave_last)) return;
         f32x4 sc[NKT];
@@ -1086,12 +1095,20 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int key = k0 + (SPLIT ? wave : t) * 16 + fq * 4 + r;
-                const bool seen = POOLED ? key < my_blocks : (key <= qpos) & ((key >= lo_window) | (key < a.keep_first)) & (key >= lo_chunk);
-                const bool ok = qok & seen;
-                float s = sc[t][r] * row_scale;
-                if (EXT && cap_in > 0.f) s = a.softcap - 2.0f * a.softcap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(s * cap_in) + 1.0f);
-                if constexpr (BIAS) sc[t][r] = ok ? s + brow[3 - r] : -INFINITY;
-                else sc[t][r] = ok ? (POOLED ? s : s - slope * (float)(qpos - key)) : -INFINITY;
+                float v;
+                if constexpr (BIAS) {
+                    v = __builtin_fmaf(sc[t][r], row_scale, brow[3 - r]);
+                } else {
+#pragma clang fp contract(off)                               // (one rounding in either form: a row's bits do not depend on where its wave begins)
+                    v = sc[t][r] * row_scale;
+                }
+                if (EXT && cap_in > 0.f) v = a.softcap - 2.0f * a.softcap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap_in) + 1.0f);
+                if constexpr (!WHOLE) {
+                    const bool seen = POOLED ? key < my_blocks : (key <= qpos) & ((key >= lo_window) | (key < a.keep_first)) & (key >= lo_chunk);
+                    if (!BIAS && !POOLED) v = __builtin_fmaf(-slope, (float)(qpos - key), v);
+                    v = qok & seen ? v : -INFINITY;
+                }
+                sc[t][r] = v;
                 mx = fmaxf(mx, sc[t][r]);
             }
         }
@@ -1100,6 +1117,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         const float m_new = fmaxf(m_run, mx);
         // e^x as the hardware's 2^(x log2 e): fp32 throughout, about 1 ulp
         const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * 1.4426950408889634f);
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;                // (a row that has seen nothing: its scores are -inf, their weights 0)
         float sum = 0.f;
         // The weights as the B operand of products over 32 rows: of two 16-key blocks, once with hi and once with lo - or, where a wave
         // has one block only, of that block's keys twice, with hi and with lo
@@ -1109,7 +1127,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         for (int t = 0; t < NKT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float pv = sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_new) * 1.4426950408889634f);
+                const float pv = __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * 1.4426950408889634f);
                 sum += pv;
                 const bf16 hi = (bf16)pv;
                 const bf16 lo = (bf16)(pv - (float)hi);
@@ -1160,7 +1178,8 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
         }
         __syncthreads();
         fetch(k_after, kpre, vpre);
-        compute(std::false_type{}, k0);
+        if (k0 >= whole_from && k0 <= whole_to) compute(std::false_type{}, std::true_type{}, k0);
+        else compute(std::false_type{}, std::false_type{}, k0);
     };
     // Two register sets, two tiles ahead: the loads of the tile after next are issued when a tile has been handed to LDS.
     bf16x8 kA[KCH], vA[VCH], kB[KCH], vB[VCH];
@@ -1214,7 +1233,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_kernel(AttnArgs a) {
             }
             __syncthreads();
             fetch_pooled(b0 + bstep);                        // (past the end: the last block's row once more)
-            compute(std::true_type{}, b0);
+            compute(std::true_type{}, std::false_type{}, b0);
         }
         __builtin_amdgcn_sched_barrier(0);
     }

@@ -67,3 +67,30 @@ def test_a_step_of_many_sequences(B, window, keep, chunk):
             assert close_to(got[b:b + 1], reference(q[b:b + 1].cpu(), k.cpu(), v.cpu(), table[b].cpu(), ctx[b], ctx[b] - 1, H, G, dim, vdim, window, keep, chunk, None))
         else:
             assert (got[b] == 0).all()
+
+
+@pytest.mark.parametrize("H,G,dim,vdim", [(2, 1, 128, 128), (2, 2, 64, 128), (1, 1, 256, 192), (2, 2, 48, 80)])
+@pytest.mark.parametrize("window,keep,chunk,sink", [(0, 0, 0, False), (100, 0, 0, True), (200, 70, 0, False), (0, 0, 192, True)])
+def test_tiles_seen_whole(H, G, dim, vdim, window, keep, chunk, sink):
+    """Prompts against float64; a portion behind cached tokens gives the bits of the whole prompt, whichever tiles its waves see whole."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(dim + window + chunk)
+    ctx = [1, 63, 64, 65, 130, 450]
+    k, v, table = caches(g, ctx, G, dim, vdim)
+    q = torch.randn(sum(ctx), H * dim, generator=g).bfloat16()
+    sinks = torch.randn(H, generator=g) if sink else None
+    kc, vc, tab = k.cuda(), v.cuda(), table.cuda()
+    kw = dict(window=window, keep_first=keep, chunk=chunk, sinks=None if sinks is None else sinks.cuda())
+
+    def run(rows, lens, ctx_lens, tables):
+        cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
+        return ops.attn_paged_any(rows.cuda(), kc, vc, cu, torch.tensor(ctx_lens).int().cuda(), tables.contiguous(), dim ** -0.5, H, G, dim, vdim, **kw)
+
+    got = run(q, ctx, ctx, tab)
+    lo = 0
+    for b, n in enumerate(ctx):
+        assert close_to(got[lo:lo + n], reference(q[lo:lo + n], k, v, table[b], n, 0, H, G, dim, vdim, window, keep, chunk, sinks)), b
+        for cut in (1, 15, 16, 40, 64, 100, 127, 200, 333):
+            if cut < n - 1:                                  # (one query left would be a step of another form)
+                assert torch.equal(run(q[lo + cut:lo + n], [n - cut], [n], tab[b:b + 1]), got[lo + cut:lo + n]), (b, cut)
+        lo += n
