@@ -67,43 +67,41 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict_
 
 // (Routing over 16 experts of 1024 columns, us a launch, 64 and 1000 tokens: 12.3 and 12.7 with a piece of 512 at a time, a chain of lane exchanges for
 // every comparison of the argmax and the weights read back to be divided; now 4.8 and 6.3.)
-// Dot products of a token's row with up to EG rows of K, row(g) for g < n, in fp32: a lane takes 8 consecutive elements of every 512, in order.
-// Whole pieces of 512 go two at a time, all their loads ahead of the sums: the rows come from L2, and its latency is what a token waits for.
-template <int EG, typename A, typename Row>
-__device__ __forceinline__ void route_dots(const A* __restrict__ xr, Row row, int n, int K, int vec, int lane, float (&acc)[EG]) {
+// Dot products of a token's row with EG rows of K, row(g) for g < EG, in fp32: a lane takes 8 consecutive elements of every 512, in order.
+// Whole pieces of 512 go PIECES at a time, all their loads ahead of the sums: the rows come from L2, and its latency is what a token waits for.
+// (The order of a sum does not depend on EG and PIECES.)
+template <int EG, int PIECES, typename A, typename Row>
+__device__ __forceinline__ void route_dots(const A* __restrict__ xr, Row row, int K, int vec, int lane, float (&acc)[EG]) {
 #pragma unroll
     for (int g = 0; g < EG; ++g) acc[g] = 0.f;
     int k0 = lane * 8;
     if (vec) {                                               // (uniform)
-        for (int left = K; left >= 1024; left -= 1024, k0 += 1024) {
-            float xv[2][8], wv[2][EG][8];
+        for (int left = K; left >= 512 * PIECES; left -= 512 * PIECES, k0 += 512 * PIECES) {
+            float xv[PIECES][8], wv[PIECES][EG][8];
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
+            for (int u = 0; u < PIECES; ++u) {
                 nvh_load8(xr, k0 + 512 * u, 8, true, xv[u]);
 #pragma unroll
-                for (int g = 0; g < EG; ++g)
-                    if (g < n) nvh_load8(row(g), k0 + 512 * u, 8, true, wv[u][g]);
+                for (int g = 0; g < EG; ++g) nvh_load8(row(g), k0 + 512 * u, 8, true, wv[u][g]);
             }
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+            for (int u = 0; u < PIECES; ++u)
 #pragma unroll
                 for (int g = 0; g < EG; ++g)
 #pragma unroll
-                    for (int i = 0; i < 8; ++i)
-                        if (g < n) acc[g] = __builtin_fmaf(xv[u][i], wv[u][g][i], acc[g]);
+                    for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[u][i], wv[u][g][i], acc[g]);
         }
     }
     for (; k0 < K; k0 += 512) {
         float xv[8];
         nvh_load8(xr, k0, K - k0, vec, xv);
 #pragma unroll
-        for (int g = 0; g < EG; ++g)
-            if (g < n) {
-                float wv[8];
-                nvh_load8(row(g), k0, K - k0, vec, wv);
+        for (int g = 0; g < EG; ++g) {
+            float wv[8];
+            nvh_load8(row(g), k0, K - k0, vec, wv);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[i], wv[i], acc[g]);
-            }
+            for (int i = 0; i < 8; ++i) acc[g] = __builtin_fmaf(xv[i], wv[i], acc[g]);
+        }
     }
 }
 
@@ -137,10 +135,11 @@ __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restri
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const A* xr = x + t * ldx;
-    constexpr int EG = 4;
+    // fp32 rows of many experts come at L2's rate: one piece at a time then, for more waves a CU
+    constexpr int EG = 4, PIECES = sizeof(A) == 4 && PL > 1 ? 1 : 2;
     for (int e0 = wave * EG; e0 < experts; e0 += 4 * EG) {
         float acc[EG];
-        route_dots<EG>(xr, [&](int g) { return w + (int64_t)min(e0 + g, experts - 1) * K; }, EG, K, vec, lane, acc);
+        route_dots<EG, PIECES>(xr, [&](int g) { return w + (int64_t)min(e0 + g, experts - 1) * K; }, K, vec, lane, acc);
 #pragma unroll
         for (int g = 0; g < EG; ++g) {
             const int e = e0 + g;
@@ -187,7 +186,9 @@ __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restri
 // rows that read the same input; their fp32 products go to aux_out [T, n_aux] (a gate of the layer, say).
 // One workgroup per token, products as in moe_route_linear_kernel; the first wave picks.
 // PL: experts (and groups) a lane of the picking wave holds: experts <= 64 PL.
-template <typename A, int PL>
+// us, one wave's rows a piece at a time (eight at once) and now, 16 experts and one more row of 1024, bf16: 64 tokens 6.8 and 4.7, 1008 tokens 7.8 and
+// 5.8; 64 + 1 16.6 and 8.2, 18.8 and 11.9; fp32, 16 + 1: 6.2 and 4.8, 8.0 and 7.2.
+template <typename A, int PL, int EG, int PIECES>
 __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restrict__ x, int64_t ldx, const A* __restrict__ w, const A* __restrict__ correction,
                                                                const A* __restrict__ aux, float* __restrict__ aux_out, int n_aux, int32_t* __restrict__ ids,
                                                                float* __restrict__ weights, float* __restrict__ scores_out, int experts, int K, int top,
@@ -198,24 +199,21 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restri
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const A* xr = x + t * ldx;
-    // every wave takes `eg` rows at a time (up to EG: 17 rows are one pass of five a wave, not two passes of four)
-    constexpr int EG = 8;
+    // every wave takes EG rows at a time; past the last row: that one again
     const int rows = experts + n_aux;
-    const int eg = min(EG, (rows + 3) / 4);
-    for (int e0 = wave * eg; e0 < rows; e0 += 4 * eg) {
+    for (int e0 = wave * EG; e0 < rows; e0 += 4 * EG) {
         float acc[EG];
-        route_dots<EG>(xr, [&](int g) {
+        route_dots<EG, PIECES>(xr, [&](int g) {
             const int e = min(e0 + g, rows - 1);
             return e < experts ? w + (int64_t)e * K : aux + (int64_t)(e - experts) * K;
-        }, eg, K, vec, lane, acc);
+        }, K, vec, lane, acc);
 #pragma unroll
-        for (int g = 0; g < EG; ++g)
-            if (g < eg) {
-                const int e = e0 + g;
-                const float sum = wave_sum(acc[g]);
-                if (lane == 0 && e < experts) zs[e] = sum;
-                else if (lane == 0 && e < rows) aux_out[t * n_aux + (e - experts)] = sum;
-            }
+        for (int g = 0; g < EG; ++g) {
+            const int e = e0 + g;
+            const float sum = wave_sum(acc[g]);
+            if (lane == 0 && e < experts) zs[e] = sum;
+            else if (lane == 0 && e < rows) aux_out[t * n_aux + (e - experts)] = sum;
+        }
     }
     __syncthreads();
     const bool picker = wave == 0;                           // the first wave picks; the others only keep the barriers company
@@ -737,16 +735,20 @@ extern "C" int32_t nvh_moe_route_scored(const void* x, int64_t x_row_stride, con
     const dim3 grid((unsigned)num_tokens);
     hipStream_t st = (hipStream_t)stream;
     const int vec = K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w) && (!aux || nvh_aligned16(aux));
-#define NVH_ROUTE_SCORED(A, PL) moe_route_scored_kernel<A, PL><<<grid, 256, 0, st>>>((const A*)x, x_row_stride, (const A*)w, (const A*)correction, (const A*)aux, aux_out, (int)num_aux, ids, weights, scores_out, (int)experts, (int)K, (int)top, (int)groups, (int)keep, scale, renorm, vec)
+#define NVH_ROUTE_SCORED(A, PL, EG, PIECES) moe_route_scored_kernel<A, PL, EG, PIECES><<<grid, 256, 0, st>>>((const A*)x, x_row_stride, (const A*)w, (const A*)correction, (const A*)aux, aux_out, (int)num_aux, ids, weights, scores_out, (int)experts, (int)K, (int)top, (int)groups, (int)keep, scale, renorm, vec)
+    const int64_t rows = experts + num_aux;
+    // Rows a wave: four, or three where that is as many passes (17 .. 24 rows), or in fp32; the fp32 rows of many experts come at L2's rate, and more
+    // waves a CU are worth more than two pieces at once (128 experts, 1008 tokens: 28.7 us as it was, 31.4 with two rows of two pieces, 26.7 so).
     if (experts <= 64) {
-        if (act_f32) NVH_ROUTE_SCORED(float, 1);
-        else NVH_ROUTE_SCORED(bf16, 1);
+        if (act_f32) NVH_ROUTE_SCORED(float, 1, 3, 2);
+        else if (rows > 16 && rows <= 24) NVH_ROUTE_SCORED(bf16, 1, 3, 2);
+        else NVH_ROUTE_SCORED(bf16, 1, 4, 2);
     } else if (experts <= 256) {
-        if (act_f32) NVH_ROUTE_SCORED(float, 4);
-        else NVH_ROUTE_SCORED(bf16, 4);
+        if (act_f32) NVH_ROUTE_SCORED(float, 4, 4, 1);
+        else NVH_ROUTE_SCORED(bf16, 4, 4, 2);
     } else {
-        if (act_f32) NVH_ROUTE_SCORED(float, ROUTE_MAX_PER_LANE);
-        else NVH_ROUTE_SCORED(bf16, ROUTE_MAX_PER_LANE);
+        if (act_f32) NVH_ROUTE_SCORED(float, ROUTE_MAX_PER_LANE, 4, 1);
+        else NVH_ROUTE_SCORED(bf16, ROUTE_MAX_PER_LANE, 4, 2);
     }
 #undef NVH_ROUTE_SCORED
     NVH_CHECK_LAUNCH("nvh_moe_route_scored");
