@@ -10,6 +10,7 @@
 //                     (gemm_any.h) with a weight matrix per tile and rows gathered through an index, bf16 on the matrix
 //                     cores or true fp32.  A row's result does not depend on where in its expert's block it lies.
 //   nvh_moe_combine   out fp32 [T, dim] = sum over a token's choices, in choice order, of weight * y[pos] (+ shared[t])
+#include <algorithm>
 #include "common.h"
 #include "gemm_any.h"
 
@@ -633,6 +634,43 @@ __global__ __launch_bounds__(256) void gemm_grouped_short_bf16_kernel(GroupedArg
     else gemm_grouped_short_tile<OUT_F32, 4>(a, expert, row0, rows, n0, smem);
 }
 
+// fp32 (K a multiple of 32) through the waves' LDS rings: a list tile by 64 columns, a workgroup a CU, for callers whose experts have many rows, or by 32
+// columns, two workgroups a CU, 49 rows and more in two halves.  Bit for bit the results of the form below.
+// us, the form below, by 32 and by 64 columns, rows an expert x N x K over 16 experts: 8 x 576 x 1024 19.2, 14.5, 13.8; 38 x 576 x 1024 31.8, 27.8, 21.0;
+// 38 x 1536 x 1024 58.6, 48.1, 40.8; 125 x 1536 x 1024 126, 102, 91; 19 x 576 x 1024 (64 experts) 53.7, 43.0, 45.9; 2.5 x 1536 x 1024 25.9, 22.0, 25.6.
+template <int NC>
+__global__ __launch_bounds__(256, NC == 2 ? 2 : 1) void gemm_grouped_f32_ring_kernel(GroupedArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int rows = a.tile_rows[blockIdx.y];
+    if (rows <= 0) return;                                   // (uniform: a tile beyond the list's end)
+    const float *x = (const float*)a.x, *w = (const float*)a.w + (int64_t)a.tile_expert[blockIdx.y] * a.N * a.K;
+    const nvh_any::RowMap rm{a.gather, a.tile_row0[blockIdx.y], rows};
+    const int n0 = blockIdx.x * 16 * NC;
+#define NVH_RING(MR, STAGES, R0) nvh_any::gemm_any_f32_ring<MR, NC, STAGES>(x, a.ldx, w, a.K, nullptr, (float*)a.y, a.ldy, rm, R0, n0, a.N, a.K, nullptr, 0, a.relu2, smem)
+    if (rows <= 16) {
+        NVH_RING(1, 3, 0);
+    } else if (NC == 4 && rows <= 32) {
+        NVH_RING(2, 3, 0);
+    } else if (rows > 32 && rows <= 48) {
+        NVH_RING(3, 2, 0);
+    } else if constexpr (NC == 4) {
+        NVH_RING(4, 2, 0);
+    } else {
+        for (int r0 = 0; r0 < rows; r0 += 32) {
+            if (r0) __syncthreads();                         // (the first half's sums have been read)
+            NVH_RING(2, 2, r0);
+        }
+    }
+#undef NVH_RING
+}
+template <int NC>
+void launch_grouped_f32(const GroupedArgs& a, int64_t max_tiles, hipStream_t st) {
+    constexpr int lds = std::max({nvh_any::f32_ring_bytes<1, NC, 3>(), nvh_any::f32_ring_bytes<2, NC, NC == 4 ? 3 : 2>(), nvh_any::f32_ring_bytes<3, NC, 2>(), NC == 4 ? nvh_any::f32_ring_bytes<4, NC, 2>() : 0});
+    static_assert(lds <= (NC == 4 ? 160 : 80) * 1024);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_f32_ring_kernel<NC>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    gemm_grouped_f32_ring_kernel<NC><<<dim3((unsigned)nvh_cdiv(a.N, 16 * NC), (unsigned)max_tiles), 256, lds, st>>>(a);
+}
+
 // (a tile of the list is 64 rows: blockIdx.z is its upper or lower half)
 __global__ __launch_bounds__(256) void gemm_grouped_f32_kernel(GroupedArgs a) {
     const int rows = a.tile_rows[blockIdx.y], r0 = blockIdx.z * 32;
@@ -790,7 +828,10 @@ static int32_t grouped_product(const void* x, int64_t x_row_stride, const int32_
         NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");
         return NVH_OK;
     }
-    if (in_f32) gemm_grouped_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)max_tiles, 2), 256, 0, st>>>(a);
+    if (in_f32 && vec_ok && K % nvh_any::F32_CHUNK == 0) {
+        if (tall) launch_grouped_f32<4>(a, max_tiles, st);
+        else launch_grouped_f32<2>(a, max_tiles, st);
+    } else if (in_f32) gemm_grouped_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)max_tiles, 2), 256, 0, st>>>(a);
     else if (out_f32) gemm_grouped_bf16_kernel<true><<<grid, 256, 0, st>>>(a);
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");

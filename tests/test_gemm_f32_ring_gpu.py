@@ -21,3 +21,19 @@ def test_plain(m, n, k):
     assert torch.equal(ops.linear_any(x, w, b), want)
     for r in {0, m // 2, m - 1}:
         assert torch.equal(ops.linear_any(x[r:r + 1].contiguous(), w, b)[0], want[r])
+
+
+@pytest.mark.parametrize("relu2", [False, True])
+@pytest.mark.parametrize("n,k", [(16, 32), (33, 96), (100, 576), (576, 1024)])
+def test_grouped(n, k, relu2):
+    from nanovllm import ops
+    sizes = [0, 1, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 130]
+    g = torch.Generator().manual_seed(n + k)
+    ids = torch.repeat_interleave(torch.arange(len(sizes)), torch.tensor(sizes))[torch.randperm(sum(sizes), generator=g)].int()[:, None].cuda()
+    x, w = torch.randn(ids.shape[0], k, generator=g).cuda(), torch.randn(len(sizes), n, k, generator=g).cuda()
+    plan = ops.moe_align(ids, len(sizes))
+    act = "relu2" if relu2 else None
+    at = plan["pos_of_pair"].long()
+    want = ops.linear_grouped(odd_rows(x), w, plan, True, act=act)[at]
+    assert torch.equal(ops.linear_grouped(x, w, plan, True, act=act)[at], want)
+    assert torch.equal(ops.linear_grouped(x[plan["src_token"].long()], w, plan, False, act=act)[at], want)
