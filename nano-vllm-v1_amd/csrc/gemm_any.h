@@ -424,4 +424,7 @@ __host__ __forceinline__ int f32_vec_ok(const void* x, int64_t ldx, const void* 
     return K % 4 == 0 && ldx % 4 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
 }
 
+// y = x w^T in bf16 through LDS rings (moe.hip), without a bias; false: a shape, stride or alignment that it does not take.
+bool launch_short_product(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, bool out_f32, hipStream_t st);
+
 }  // namespace nvh_any

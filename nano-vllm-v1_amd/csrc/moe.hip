@@ -634,6 +634,17 @@ __global__ __launch_bounds__(256) void gemm_grouped_short_bf16_kernel(GroupedArg
     else gemm_grouped_short_tile<OUT_F32, 4>(a, expert, row0, rows, n0, smem);
 }
 
+// One weight matrix, 64 rows a tile.  us, the general form and this, fp32 results: 1 x 32768 x 1024 14.6 and 13.0 (5.2 TB/s), 64 x 32768 x 1024 20.2 and 16.8,
+// 64 x 152064 x 1024 94 and 76, 256 x 32768 x 1024 62 and 51, 1 x 512 x 1024 8.4 and 5.3, 16 x 1024 x 4096 29.1 and 14.9.
+template <bool OUT_F32>
+__global__ __launch_bounds__(256) void gemm_short_bf16_kernel(GroupedArgs a, int M) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int row0 = blockIdx.y * nvh_any::GT, rows = min(nvh_any::GT, M - row0), n0 = blockIdx.x * SHORT_N;
+    if (rows <= 16) gemm_grouped_short_tile<OUT_F32, 1>(a, 0, row0, rows, n0, smem);
+    else if (rows <= 32) gemm_grouped_short_tile<OUT_F32, 2>(a, 0, row0, rows, n0, smem);
+    else gemm_grouped_short_tile<OUT_F32, 4>(a, 0, row0, rows, n0, smem);
+}
+
 // fp32 (K a multiple of 32) through the waves' LDS rings: a list tile by 64 columns, a workgroup a CU, for callers whose experts have many rows, or by 32
 // columns, two workgroups a CU, 49 rows and more in two halves.  Bit for bit the results of the form below.
 // us, the form below, by 32 and by 64 columns, rows an expert x N x K over 16 experts: 8 x 576 x 1024 19.2, 14.5, 13.8; 38 x 576 x 1024 31.8, 27.8, 21.0;
@@ -836,6 +847,15 @@ static int32_t grouped_product(const void* x, int64_t x_row_stride, const int32_
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");
     return NVH_OK;
+}
+
+bool nvh_any::launch_short_product(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, bool out_f32, hipStream_t st) {
+    if (K % 64 != 0 || N % 4 != 0 || ldx % 8 != 0 || ldy % 4 != 0 || !nvh_aligned16(x) || !nvh_aligned16(w) || !nvh_aligned16(y)) return false;
+    const GroupedArgs a{x, ldx, nullptr, w, y, ldy, nullptr, nullptr, nullptr, (int)N, (int)K, 1, 0};
+    const dim3 grid((unsigned)nvh_cdiv(N, SHORT_N), (unsigned)nvh_cdiv(M, nvh_any::GT));
+    if (out_f32) gemm_short_bf16_kernel<true><<<grid, 256, SHORT_LDS, st>>>(a, (int)M);
+    else gemm_short_bf16_kernel<false><<<grid, 256, SHORT_LDS, st>>>(a, (int)M);
+    return true;
 }
 
 extern "C" int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,

@@ -872,6 +872,11 @@ extern "C" int32_t nvh_gemm_any_nt(const void* x, int64_t x_row_stride, const vo
         else gemm_any_f32_kernel<2, 2><<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)std::min<int64_t>(nvh_cdiv(M, 32), 65535)), 256, 0, st>>>((const float*)x, x_row_stride, (const float*)w, K, (const float*)bias, (float*)y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
     } else {
         const int vec_ok = K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
+        // (the same bits: this form's rows of columns through LDS, whole k-tiles ahead; the other takes any shape, stride and bias)
+        if (!bias && nvh_any::launch_short_product(x, x_row_stride, w, y, y_row_stride, M, N, K, out_f32 != 0, st)) {
+            NVH_CHECK_LAUNCH("nvh_gemm_any_nt");
+            return NVH_OK;
+        }
         if (out_f32) gemm_any_bf16_kernel<true><<<grid, 256, 0, st>>>((const bf16*)x, x_row_stride, (const bf16*)w, K, (const bf16*)bias, y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
         else gemm_any_bf16_kernel<false><<<grid, 256, 0, st>>>((const bf16*)x, x_row_stride, (const bf16*)w, K, (const bf16*)bias, y, y_row_stride, (int)M, (int)N, (int)K, vec_ok);
     }
