@@ -110,30 +110,35 @@ __global__ __launch_bounds__(256) void stream_cast_kernel(const float* __restric
     for (int c = threadIdx.x; c < dim; c += 256) out[row * out_stride + c] = (A)x[row * dim + c];
 }
 
-template <typename A>
-__global__ __launch_bounds__(256) void gelu_tanh_mul_kernel(const A* __restrict__ gu, int64_t gu_stride, A* __restrict__ y, int64_t rows, int inter) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * inter) return;
-    const int64_t row = i / inter;
-    const int c = (int)(i - row * inter);
-    const float g = ldf(gu, row * gu_stride + c), u = ldf(gu, row * gu_stride + inter + c);
-    const float act = 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-    y[i] = (A)(act * u);
-}
-
 __global__ __launch_bounds__(256) void gather_rows_f32_kernel(const float* __restrict__ x, const int32_t* __restrict__ index, float* __restrict__ out, int dim) {
     const int64_t row = blockIdx.x;
     const int64_t src = index[row];
     for (int c = threadIdx.x; c < dim; c += 256) out[row * dim + c] = x[src * dim + c];
 }
 
-template <typename A>
-__global__ __launch_bounds__(256) void softcap_kernel(const A* __restrict__ z, int64_t z_stride, float* __restrict__ out, int64_t rows, int vocab, float cap) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * vocab) return;
-    const int64_t row = i / vocab;
-    const float v = ldf(z, row * z_stride + (i - row * vocab));
-    out[i] = cap > 0.f ? cap * tanhf(v / cap) : v;
+// out = cap tanh(z scale / cap), or z scale without a cap.  E: elements a lane, 8 where rows and strides allow 16-byte accesses.
+// us, 256 x 32768 with a cap: 19.5 and 13.5 (67 MB), 64 x 32768 6.2 and 5.3.
+template <typename A, int E>
+__global__ __launch_bounds__(256) void logits_scale_kernel(const A* __restrict__ z, int64_t z_stride, float* __restrict__ out, int64_t rows, int vocab, float scale,
+                                                           float cap) {
+    int64_t row;
+    int c;
+    if (!nvh_piece<E>(rows, vocab, row, c)) return;
+    float v[E];
+    nvh_load_piece<A, E>(z + row * z_stride + c, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const float x = v[e] * scale;
+        v[e] = cap > 0.f ? cap * tanhf(x / cap) : x;
+    }
+    nvh_store_piece<float, E>(out + row * vocab + c, v);
+}
+static void launch_logits_scale(const void* z, int64_t z_stride, float* out, int64_t rows, int64_t vocab, float scale, float cap, bool act_f32, hipStream_t st) {
+    const bool vec = rows * vocab >= NVH_PIECES && vocab % 8 == 0 && z_stride % 8 == 0 && nvh_aligned16(z) && nvh_aligned16(out);
+    const dim3 grid((unsigned)nvh_cdiv(rows * vocab, vec ? 2048 : 256));
+    auto launch = [&](auto kernel, auto type) { kernel<<<grid, 256, 0, st>>>((const decltype(type)*)z, z_stride, out, rows, (int)vocab, scale, cap); };
+    if (act_f32) launch(vec ? &logits_scale_kernel<float, 8> : &logits_scale_kernel<float, 1>, 0.f);
+    else launch(vec ? &logits_scale_kernel<bf16, 8> : &logits_scale_kernel<bf16, 1>, (bf16)0.f);
 }
 
 // x[row] = table[id] * scale + pos_table[position] (fp32); ids or positions outside their tables give zeros for that term.
@@ -664,20 +669,37 @@ static bool launch_residual_subnorm_vec(const SubNormArgs& p, const MoeTerms& m,
 
 // y = act(g) (* u when gated): g = columns [0, inter) and u = columns [inter, 2 inter) of the row.
 // act: 0 silu, 1 gelu (tanh form), 2 squared relu.
-template <typename A>
+// E: elements a lane, 8 where rows and strides allow 16-byte accesses.
+// us, one element a lane behind a division in 64 bits and so: silu 1024 x 3072 10.0 and 6.0 (19 MB), gelu 8.5 and 6.6; 4000 x 768 10.0 and 6.1.
+template <typename A, int E>
 __global__ __launch_bounds__(256) void act_mul_kernel(const A* __restrict__ gu, int64_t gu_stride, A* __restrict__ y, int64_t y_stride, int64_t rows, int inter,
                                                       int act, int gated) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * inter) return;
-    const int64_t row = i / inter;
-    const int c = (int)(i - row * inter);
-    const float g = ldf(gu, row * gu_stride + c);
-    float v;
-    if (act == 0) v = g / (1.0f + expf(-g));
-    else if (act == 1) v = 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-    else v = g > 0.f ? g * g : 0.f;
-    if (gated) v *= ldf(gu, row * gu_stride + inter + c);
-    y[row * y_stride + c] = (A)v;
+    int64_t row;
+    int c;
+    if (!nvh_piece<E>(rows, inter, row, c)) return;
+    const A* src = gu + row * gu_stride + c;
+    float v[E], u[E];
+    nvh_load_piece<A, E>(src, v);
+    if (gated) nvh_load_piece<A, E>(src + inter, u);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const float g = v[e];
+        if (act == 0) v[e] = g / (1.0f + expf(-g));
+        else if (act == 1) v[e] = 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+        else v[e] = g > 0.f ? g * g : 0.f;
+        if (gated) v[e] *= u[e];
+    }
+    nvh_store_piece<A, E>(y + row * y_stride + c, v);
+}
+static void launch_act_mul(const void* x, int64_t row_stride, void* y, int64_t y_stride, int64_t rows, int64_t inter, int act, int gated, bool act_f32, hipStream_t st) {
+    const bool vec = rows * inter >= NVH_PIECES && inter % 8 == 0 && row_stride % 8 == 0 && y_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(y);
+    const dim3 grid((unsigned)nvh_cdiv(rows * inter, vec ? 2048 : 256));
+    auto launch = [&](auto kernel, auto type) {
+        typedef decltype(type) A;
+        kernel<<<grid, 256, 0, st>>>((const A*)x, row_stride, (A*)y, y_stride, rows, (int)inter, act, gated);
+    };
+    if (act_f32) launch(vec ? &act_mul_kernel<float, 8> : &act_mul_kernel<float, 1>, 0.f);
+    else launch(vec ? &act_mul_kernel<bf16, 8> : &act_mul_kernel<bf16, 1>, (bf16)0.f);
 }
 
 // xIELU with the two numbers (p, q) of `params`, in fp32:  z > 0: softplus(p) z^2 + z / 2;  else (1/2 + softplus(q)) (e^z - 1 - z) + z / 2.
@@ -713,16 +735,6 @@ __global__ __launch_bounds__(256) void xielu_kernel(const A* __restrict__ x, int
     }
     if constexpr (VEC) __builtin_memcpy(__builtin_assume_aligned(dst, 16), out, sizeof(out));
     else dst[0] = out[0];
-}
-
-template <typename A>
-__global__ __launch_bounds__(256) void logits_scale_kernel(const A* __restrict__ z, int64_t z_stride, float* __restrict__ out, int64_t rows, int vocab, float scale,
-                                                           float cap) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= rows * vocab) return;
-    const int64_t row = i / vocab;
-    const float v = ldf(z, row * z_stride + (i - row * vocab)) * scale;
-    out[i] = cap > 0.f ? cap * tanhf(v / cap) : v;
 }
 
 
@@ -817,9 +829,7 @@ extern "C" int32_t nvh_gelu_tanh_mul(const void* gate_up, int64_t row_stride, vo
     NVH_STREAM_ARGS_OK("nvh_gelu_tanh_mul", gate_up && y && rows >= 0 && inter > 0 && row_stride >= 2 * inter);
     if (rows == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)nvh_cdiv(rows * inter, 256);
-    if (act_f32) gelu_tanh_mul_kernel<float><<<dim3(blocks), 256, 0, st>>>((const float*)gate_up, row_stride, (float*)y, rows, (int)inter);
-    else gelu_tanh_mul_kernel<bf16><<<dim3(blocks), 256, 0, st>>>((const bf16*)gate_up, row_stride, (bf16*)y, rows, (int)inter);
+    launch_act_mul(gate_up, row_stride, y, inter, rows, inter, 1, 1, act_f32, st);
     NVH_CHECK_LAUNCH("nvh_gelu_tanh_mul");
     return NVH_OK;
 }
@@ -837,9 +847,7 @@ extern "C" int32_t nvh_logit_softcap(const void* logits, int64_t row_stride, flo
     NVH_STREAM_ARGS_OK("nvh_logit_softcap", logits && out && rows >= 0 && vocab > 0 && row_stride >= vocab);
     if (rows == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)nvh_cdiv(rows * vocab, 256);
-    if (act_f32) softcap_kernel<float><<<dim3(blocks), 256, 0, st>>>((const float*)logits, row_stride, out, rows, (int)vocab, cap);
-    else softcap_kernel<bf16><<<dim3(blocks), 256, 0, st>>>((const bf16*)logits, row_stride, out, rows, (int)vocab, cap);
+    launch_logits_scale(logits, row_stride, out, rows, vocab, 1.0f, cap, act_f32, st);
     NVH_CHECK_LAUNCH("nvh_logit_softcap");
     return NVH_OK;
 }
@@ -1033,9 +1041,7 @@ extern "C" int32_t nvh_act_mul(const void* x, int64_t row_stride, void* y, int64
     NVH_STREAM_ARGS_OK("nvh_act_mul", x && y && rows >= 0 && inter > 0 && act >= 0 && act <= 2 && row_stride >= (gated ? 2 : 1) * inter && y_stride >= inter);
     if (rows == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)nvh_cdiv(rows * inter, 256);
-    if (act_f32) act_mul_kernel<float><<<dim3(blocks), 256, 0, st>>>((const float*)x, row_stride, (float*)y, y_stride, rows, (int)inter, act, gated);
-    else act_mul_kernel<bf16><<<dim3(blocks), 256, 0, st>>>((const bf16*)x, row_stride, (bf16*)y, y_stride, rows, (int)inter, act, gated);
+    launch_act_mul(x, row_stride, y, y_stride, rows, inter, act, gated, act_f32, st);
     NVH_CHECK_LAUNCH("nvh_act_mul");
     return NVH_OK;
 }
@@ -1063,9 +1069,7 @@ extern "C" int32_t nvh_logits_scale(const void* logits, int64_t row_stride, floa
     NVH_STREAM_ARGS_OK("nvh_logits_scale", logits && out && rows >= 0 && vocab > 0 && row_stride >= vocab);
     if (rows == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
-    const unsigned blocks = (unsigned)nvh_cdiv(rows * vocab, 256);
-    if (act_f32) logits_scale_kernel<float><<<dim3(blocks), 256, 0, st>>>((const float*)logits, row_stride, out, rows, (int)vocab, scale, cap);
-    else logits_scale_kernel<bf16><<<dim3(blocks), 256, 0, st>>>((const bf16*)logits, row_stride, out, rows, (int)vocab, scale, cap);
+    launch_logits_scale(logits, row_stride, out, rows, vocab, scale, cap, act_f32, st);
     NVH_CHECK_LAUNCH("nvh_logits_scale");
     return NVH_OK;
 }
