@@ -845,34 +845,43 @@ __global__ __launch_bounds__(256, CPL <= 4 ? 4 : 2) void delta_chunk_prep_kernel
     for (int tile = wave + 4 * VAHEAD; tile < vtiles; tile += 4) values(tile, load_v(tile));
 }
 
-// NW waves of 16 key channels each hold 16 columns of a head's state, in the layout in which a product leaves its result (row 4 q + e of lane
-// (q, column) in element e) - which is also the layout in which it takes its right operand, so a state never moves between lanes.  One wave
-// more sums the waves' parts of the outputs, a chunk behind, and writes them.
-template <int NW>
-__global__ __launch_bounds__(64 * NW + 64) void delta_chunk_scan_kernel(DeltaChunkArgs a) {
-    __shared__ f32x4 meet_d[2][NW][64], meet_o[2][NW][64];   // [chunk parity][wave][lane]
+// NW waves of 16 TPW key channels each hold 16 columns of a head's state, in the layout in which a product leaves its result (row 4 q + e of lane
+// (q, column) in element e) - which is also the layout in which it takes its right operand, so a state never moves between lanes.  What bounds the
+// launch is the chain of a chunk in these waves: D's product, the meeting, A's product, the new state.  So as much as can be is done beside them: NW
+// helpers form K'^T V in double a chunk ahead, and one wave more sums the waves' parts of
+// the outputs, a chunk behind, and writes them; it loads nothing, since a load's turn to be waited for lies behind the stores of the chunk before.
+// us of both launches, eight waves (four for 64 channels) with all of it in them and so: 1024 tokens of 16 heads of 64 x 64 73.6 and 66.0, 1000 of 8 heads of
+// 128 x 128 105 and 97, of 4 heads 97 and 89; errors against float64 5.4e-8 and 5.4e-8, 5.7e-8 and 5.6e-8.  At 128 channels eight parts in place of the four
+// sums of two: 114.
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+template <int NW, int TPW>
+struct ScanMeet {                                            // by chunk parity; a lane's own place
+    f32x4 d[2][NW][64], o[2][NW][64], z[2][64];
+    f64x2 kv[2][NW * TPW][2][64];
+};
+template <int NW, int TPW>
+__global__ __launch_bounds__(64 * (2 * NW + 1)) void delta_chunk_scan_kernel(DeltaChunkArgs a) {
+    constexpr int dk = 16 * NW * TPW;
+    __shared__ ScanMeet<NW, TPW> meet;
     const DeltaScanArgs& p = a.s;
-    constexpr int dk = 16 * NW;
     const int seq = blockIdx.x, head = blockIdx.y, dv = p.dv, cb = blockIdx.z;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63, col = lane & 15, q = lane >> 4;
     const int lo = p.cu_seqlens_q[seq], hi = p.cu_seqlens_q[seq + 1], slot = p.slots[seq];
     if (slot < 0 || hi <= lo || hi - lo < p.skip_from) return;       // (uniform)
     const int64_t record = chunk_record(dk, dv), step = (int64_t)p.H * record;
     const float* rec = a.ws + ((int64_t)chunk_base(lo, seq) * p.H + head) * record;
     const int chunks = (hi - lo + CT - 1) / CT;
-    if (wave == NW) {                                        // the outputs: the parts of chunk j are written before the barrier of chunk j + 1
+    // Every wave comes to chunks + 1 barriers: one per chunk, and one behind the last.
+    if (wave == 2 * NW) {                                    // the outputs: the parts of chunk j are written before the barrier of chunk j + 1
         float* out = p.out + (int64_t)lo * p.H * dv + head * dv + 16 * cb + col;
-        const float* zp = rec + 65 * dk + 16 * dv + (cb * 64 + lane) * 4;
-        f32x4 z = *reinterpret_cast<const f32x4*>(zp);
         __syncthreads();
         for (int j = 0; j < chunks; ++j) {
-            const f32x4 after = *reinterpret_cast<const f32x4*>(zp + min(j + 1, chunks - 1) * step);
             __syncthreads();
-            f32x4 res = meet_o[j & 1][0][lane];
+            f32x4 res = meet.o[j & 1][0][lane];
 #pragma unroll
-            for (int w = 1; w < NW; ++w) res += meet_o[j & 1][w][lane];
-            res += z;
-            z = after;
+            for (int w = 1; w < NW; ++w) res += meet.o[j & 1][w][lane];
+            res += meet.z[j & 1][lane];
             const int t = CT * j + 4 * q;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -880,79 +889,137 @@ __global__ __launch_bounds__(64 * NW + 64) void delta_chunk_scan_kernel(DeltaChu
         }
         return;
     }
-    const bool fresh = p.context_lens[seq] == hi - lo;
-    float* sp = p.state + (((int64_t)slot * p.H + head) * dk + 16 * wave + 4 * q) * dv + 16 * cb + col;
-    f32x4 S = {0.f, 0.f, 0.f, 0.f};
-    if (!fresh) {
+    constexpr int AHEAD = TPW == 1 ? 4 : 3;                  // records in flight
+    // body(j, x): chunk j with its operands; fetch(record, x) requests a chunk's
+    auto walk = [&](auto& x, auto fetch, auto body) {
+        auto request = [&](int j, auto& to) { fetch(rec + (int64_t)min(j, chunks - 1) * step, to); };
 #pragma unroll
-        for (int e = 0; e < 4; ++e) S[e] = sp[(int64_t)e * dv];
+        for (int i = 0; i < AHEAD; ++i) request(i, x[i]);
+        int j = 0;
+        for (; j + AHEAD <= chunks; j += AHEAD) {
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                body(j + i, x[i]);
+                request(j + i + AHEAD, x[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD - 1; ++i)
+            if (j + i < chunks) body(j + i, x[i]);
+        __syncthreads();                                     // (the last chunk's outputs)
+    };
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    if (wave >= NW) {
+        const int w = wave - NW;
+        struct Operands {
+            f32x4 K[TPW], V, Z;
+        } x[AHEAD];
+        walk(
+            x,
+            [&](const float* r, Operands& to) {
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) to.K[i] = *reinterpret_cast<const f32x4*>(r + 48 * dk + (TPW * w + i) * 256 + 4 * lane);
+                to.Z = *reinterpret_cast<const f32x4*>(r + 65 * dk + 16 * dv + cb * 256 + 4 * lane);
+                to.V = *reinterpret_cast<const f32x4*>(r + 65 * dk + 32 * dv + cb * 256 + 4 * lane);
+            },
+            [&](int j, const Operands& y) {
+                f64x4 kv[TPW];
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) kv[i] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int i = 0; i < TPW; ++i) kv[i] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)y.K[i][e], (double)y.V[e], kv[i], 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) {
+                    meet.kv[j & 1][TPW * w + i][0][lane] = f64x2{kv[i][0], kv[i][1]};
+                    meet.kv[j & 1][TPW * w + i][1][lane] = f64x2{kv[i][2], kv[i][3]};
+                }
+                __syncthreads();                             // (of the other parity: the state's waves have read it before they came to this barrier)
+                if (w == 0) meet.z[j & 1][lane] = y.Z;
+            });
+        return;
     }
-    struct Operands {
-        f32x4 W, Q, A, K, P, Y, V;
-    };
-    auto fetch = [&](int j, Operands& x) {
-        const float* r = rec + min(j, chunks - 1) * step;
-        const float* m = r + (wave * 64 + lane) * 4;
-        const float* n = r + 65 * dk + (cb * 64 + lane) * 4;
-        x.W = *reinterpret_cast<const f32x4*>(m);
-        x.Q = *reinterpret_cast<const f32x4*>(m + 16 * dk);
-        x.A = *reinterpret_cast<const f32x4*>(m + 32 * dk);
-        x.K = *reinterpret_cast<const f32x4*>(m + 48 * dk);
-        x.P = *reinterpret_cast<const f32x4*>(r + 64 * dk + 16 * wave + 4 * q);
-        x.Y = *reinterpret_cast<const f32x4*>(n);
-        x.V = *reinterpret_cast<const f32x4*>(n + 32 * dv);
-    };
-    // The chain of a chunk is D's product, the meeting and A's product; what does not depend on the meeting runs in its shadow.
-    auto chunk = [&](int j, const Operands& x) {
-        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-        f32x4 d = zero, o = zero, ad = zero;
+    __builtin_amdgcn_s_setprio(3);                           // (ahead of the helpers at the matrix pipe)
+    const bool fresh = p.context_lens[seq] == hi - lo;
+    float* sp = p.state + (((int64_t)slot * p.H + head) * dk + 16 * TPW * wave + 4 * q) * dv + 16 * cb + col;
+    f32x4 S[TPW];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[e], S[e], d, 0, 0, 0);
-        meet_d[j & 1][wave][lane] = d;
-        __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < TPW; ++i) {
+        S[i] = zero;
+        if (!fresh) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[e], S[e], o, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        __syncthreads();                                     // (the buffers of the other parity: every wave has left them before it came here)
-        f32x4 part[NW];
-#pragma unroll
-        for (int w = 0; w < NW; ++w) part[w] = meet_d[j & 1][w][lane];
-        meet_o[j & 1][wave][lane] = o;
-        __builtin_amdgcn_sched_barrier(0);
-        f64x4 kv = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kv = __builtin_amdgcn_mfma_f64_16x16x4f64((double)x.K[e], (double)x.V[e], kv, 0, 0, 0);
-        // (with the decayed state on it in double too, a state is rounded once a chunk: 3.4e-8 off instead of 5.0e-8, at no cost for 64 key channels
-        // and 101 -> 106 us for 8 heads of 128 x 128, 1024 tokens)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kv[e] = __builtin_fma((double)x.P[e], (double)S[e], kv[e]);
-        f32x4 sum = x.Y;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sum += part[w];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) ad = __builtin_amdgcn_mfma_f32_16x16x4f32(x.A[e], sum[e], ad, 0, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[e] = (float)(kv[e] - ad[e]);
-    };
-    constexpr int AHEAD = NW <= 4 ? 4 : 3;                   // records in flight
-    Operands x[AHEAD];
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) fetch(i, x[i]);
-    int j = 0;
-    for (; j + AHEAD <= chunks; j += AHEAD) {
-#pragma unroll
-        for (int i = 0; i < AHEAD; ++i) {
-            chunk(j + i, x[i]);
-            fetch(j + i + AHEAD, x[i]);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int e = 0; e < 4; ++e) S[i][e] = sp[(int64_t)(16 * i + e) * dv];
         }
     }
+    struct Operands {
+        f32x4 W[TPW], Q[TPW], A[TPW], P[TPW], Y;
+    } x[AHEAD];
+    walk(
+        x,
+        [&](const float* r, Operands& to) {
 #pragma unroll
-    for (int i = 0; i < AHEAD - 1; ++i)
-        if (j + i < chunks) chunk(j + i, x[i]);
-    __syncthreads();                                         // (the last chunk's outputs)
+            for (int i = 0; i < TPW; ++i) {
+                const float* m = r + (TPW * wave + i) * 256 + 4 * lane;
+                to.W[i] = *reinterpret_cast<const f32x4*>(m);
+                to.Q[i] = *reinterpret_cast<const f32x4*>(m + 16 * dk);
+                to.A[i] = *reinterpret_cast<const f32x4*>(m + 32 * dk);
+                to.P[i] = *reinterpret_cast<const f32x4*>(r + 64 * dk + 16 * (TPW * wave + i) + 4 * q);
+            }
+            to.Y = *reinterpret_cast<const f32x4*>(r + 65 * dk + cb * 256 + 4 * lane);
+        },
+        [&](int j, const Operands& y) {
+            f32x4 d[TPW], o[TPW], ad[TPW];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sp[(int64_t)e * dv] = S[e];
+            for (int i = 0; i < TPW; ++i) d[i] = o[i] = ad[i] = zero;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) d[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y.W[i][e], S[i][e], d[i], 0, 0, 0);
+            if constexpr (TPW == 2) d[0] += d[1];             // (two short chains and their sum: a chain over both tiles rounds more)
+            meet.d[j & 1][wave][lane] = d[0];
+            __syncthreads();                                 // (the buffers of the other parity: every wave has left them before it came here)
+            f32x4 part[NW];
+            f64x4 kv[TPW];
+#pragma unroll
+            for (int w = 0; w < NW; ++w) part[w] = meet.d[j & 1][w][lane];
+#pragma unroll
+            for (int i = 0; i < TPW; ++i) {
+                const f64x2 a01 = meet.kv[j & 1][TPW * wave + i][0][lane], a23 = meet.kv[j & 1][TPW * wave + i][1][lane];
+                kv[i] = f64x4{a01[0], a01[1], a23[0], a23[1]};
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            // (while the parts come)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) o[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y.Q[i][e], S[i][e], o[i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 sum = y.Y;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sum += part[w];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TPW; ++i) ad[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(y.A[i][e], sum[e], ad[i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (TPW == 2) o[0] += o[1];
+            meet.o[j & 1][wave][lane] = o[0];
+            // (with the decayed state on it in double too, a state is rounded once a chunk: 3.4e-8 off instead of 5.0e-8)
+#pragma unroll
+            for (int i = 0; i < TPW; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) kv[i][e] = __builtin_fma((double)y.P[i][e], (double)S[i][e], kv[i][e]);
+#pragma unroll
+            for (int i = 0; i < TPW; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S[i][e] = (float)(kv[i][e] - ad[i][e]);
+        });
+#pragma unroll
+    for (int i = 0; i < TPW; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sp[(int64_t)(16 * i + e) * dv] = S[i][e];
 }
 
 template <typename A>
@@ -1101,7 +1168,9 @@ static void launch_delta_chunks(const DeltaChunkArgs& a, int64_t slots, int64_t 
     if (lds > 60 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&delta_chunk_prep_kernel<CPL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // (heads fastest: with a multiple of eight heads a head's records are written and read by the same XCD, through its L2)
     delta_chunk_prep_kernel<CPL><<<dim3((unsigned)a.s.H, (unsigned)slots), 256, lds, st>>>(a);
-    delta_chunk_scan_kernel<CPL><<<dim3((unsigned)batch, (unsigned)a.s.H, (unsigned)(a.s.dv / 16)), 64 * CPL + 64, 0, st>>>(a);
+    // (at most four waves of key channels, one a SIMD: more of them would share a SIMD's matrix pipe and have more parts to exchange)
+    constexpr int TPW = CPL > 4 ? 2 : 1, NW = CPL / TPW;
+    delta_chunk_scan_kernel<NW, TPW><<<dim3((unsigned)batch, (unsigned)a.s.H, (unsigned)(a.s.dv / 16)), 64 * (2 * NW + 1), 0, st>>>(a);
 }
 
 extern "C" int32_t nvh_delta_scan_chunked(const float* pack, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
