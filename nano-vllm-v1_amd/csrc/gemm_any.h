@@ -427,4 +427,8 @@ __host__ __forceinline__ int f32_vec_ok(const void* x, int64_t ldx, const void* 
 // y = x w^T in bf16 through LDS rings (moe.hip), without a bias; false: a shape, stride or alignment that it does not take.
 bool launch_short_product(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M, int64_t N, int64_t K, bool out_f32, hipStream_t st);
 
+// The same for a product per head (nvh_gemm_heads_nt), with its gate.
+bool launch_short_heads(const void* x, int64_t ldx, int64_t x_head, const void* w, void* y, int64_t ldy, int64_t y_head, int64_t M, int64_t heads, int64_t N, int64_t K,
+                        const void* gate, int64_t ldg, hipStream_t st);
+
 }  // namespace nvh_any

@@ -198,7 +198,8 @@ extern "C" int32_t nvh_gemm_heads_nt(const void* x, int64_t x_row_stride, int64_
     const dim3 grid((unsigned)nvh_cdiv(N, nvh_any::GT), (unsigned)nvh_cdiv(M, nvh_any::GT), (unsigned)heads);
     hipStream_t st = (hipStream_t)stream;
     if (act_f32) gemm_heads_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)std::min<int64_t>(nvh_cdiv(M, 32), 65535), (unsigned)heads), 256, 0, st>>>(a);
-    else gemm_heads_bf16_kernel<<<grid, 256, 0, st>>>(a);
+    else if (!nvh_any::launch_short_heads(x, x_row_stride, x_head_stride, w, y, y_row_stride, y_head_stride, M, heads, N, K, gate, gate_row_stride, st))
+        gemm_heads_bf16_kernel<<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_heads_nt");
     return NVH_OK;
 }
