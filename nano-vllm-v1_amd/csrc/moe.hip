@@ -337,36 +337,60 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restri
     }
 }
 
-// One workgroup: counts per expert, block starts, then every pair takes the next free position of its expert's block.
+// One workgroup: every pair counts itself with its expert, which is its rank there; the sums over the experts before are a scan by one wave; a pair's position is
+// the two together.  What bounds it is the chain of launch, load, barriers and stores.  us, before (counts, starts by one lane, a second count for the
+// positions; 1024 threads always) and so, tokens x choices of experts: 64 x 2 of 16 2.8 and 2.6, 1000 x 4 of 16 4.9 and 3.9, 1000 x 4 of 64 7.4 and 4.0,
+// 301 x 8 of 128 9.6 and 3.8, 1000 x 8 of 256 20.1 and 9.1.
 // (Which position a pair gets within its block depends on the order the lanes arrive in; nothing downstream depends on it.)
+constexpr int ALIGN_KEPT = 4;                                // pairs whose expert and place a thread keeps in registers
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restrict__ ids, int64_t pairs, int experts, int top, int32_t* __restrict__ src_token,
                                                          int32_t* __restrict__ pos_of_pair, int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_row0,
                                                          int32_t* __restrict__ tile_rows, int max_tiles) {
-    extern __shared__ int sh[];                              // [experts] counts, [experts] starts / cursors, [experts] first tile
+    extern __shared__ int sh[];                              // [experts] counts, [experts] starts, [experts + 1] first tiles
     int* count = sh;
     int* start = sh + experts;
     int* tile0 = sh + 2 * experts;
-    for (int e = threadIdx.x; e < experts; e += 1024) count[e] = 0;
+    const int tid = threadIdx.x, threads = blockDim.x;
+    int kept_e[ALIGN_KEPT], kept_rank[ALIGN_KEPT];
+#pragma unroll
+    for (int u = 0; u < ALIGN_KEPT; ++u) {
+        const int64_t i = tid + (int64_t)u * threads;
+        kept_e[u] = i < pairs ? ids[i] : -1;
+    }
+    for (int e = tid; e < experts; e += threads) count[e] = 0;
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < pairs; i += 1024) {
+    // a pair's rank among its expert's is what the count was when it came
+#pragma unroll
+    for (int u = 0; u < ALIGN_KEPT; ++u)
+        if (kept_e[u] >= 0 && kept_e[u] < experts) kept_rank[u] = atomicAdd(&count[kept_e[u]], 1);
+    for (int64_t i = tid + (int64_t)ALIGN_KEPT * threads; i < pairs; i += threads) {
         const int e = ids[i];
-        if (e >= 0 && e < experts) atomicAdd(&count[e], 1);
+        pos_of_pair[i] = e >= 0 && e < experts ? atomicAdd(&count[e], 1) : -1;       // (the rank for now: read back below by this thread)
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int row = 0, tile = 0;
-        for (int e = 0; e < experts; ++e) {
-            start[e] = row;
-            tile0[e] = tile;
-            row += count[e];
-            tile += (count[e] + nvh_any::GT - 1) / nvh_any::GT;
+    if (tid < 64) {                                          // sums over the experts before, 64 of them at a time
+        int rows = 0, tiles = 0;
+        for (int e0 = 0; e0 < experts; e0 += 64) {
+            const int e = e0 + tid, n = e < experts ? count[e] : 0, nt = (n + nvh_any::GT - 1) / nvh_any::GT;
+            int r = n, t = nt;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int ro = __shfl_up(r, d, 64), to = __shfl_up(t, d, 64);
+                r += tid >= d ? ro : 0;
+                t += tid >= d ? to : 0;
+            }
+            if (e < experts) {
+                start[e] = rows + r - n;
+                tile0[e] = tiles + t - nt;
+            }
+            rows += __shfl(r, 63, 64);
+            tiles += __shfl(t, 63, 64);
         }
-        tile0[experts] = tile;
+        if (tid == 0) tile0[experts] = tiles;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < max_tiles; i += 1024) tile_rows[i] = 0;
-    __syncthreads();
-    for (int e = threadIdx.x; e < experts; e += 1024) {
+    for (int i = tile0[experts] + tid; i < max_tiles; i += threads) tile_rows[i] = 0;
+    for (int e = tid; e < experts; e += threads) {
         const int n = count[e];
         for (int k = 0, t = tile0[e]; k < n && t < max_tiles; k += nvh_any::GT, ++t) {
             tile_expert[t] = e;
@@ -374,14 +398,19 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
             tile_rows[t] = min(nvh_any::GT, n - k);
         }
     }
-    __syncthreads();
-    for (int64_t i = threadIdx.x; i < pairs; i += 1024) {
-        const int e = ids[i];
-        if (e < 0 || e >= experts) {
-            pos_of_pair[i] = -1;
-            continue;
-        }
-        const int pos = atomicAdd(&start[e], 1);
+#pragma unroll
+    for (int u = 0; u < ALIGN_KEPT; ++u) {
+        const int64_t i = tid + (int64_t)u * threads;
+        if (i >= pairs) continue;
+        const bool ok = kept_e[u] >= 0 && kept_e[u] < experts;
+        const int pos = ok ? start[kept_e[u]] + kept_rank[u] : -1;
+        if (ok) src_token[pos] = (int32_t)(i / top);
+        pos_of_pair[i] = pos;
+    }
+    for (int64_t i = tid + (int64_t)ALIGN_KEPT * threads; i < pairs; i += threads) {
+        const int rank = pos_of_pair[i];
+        if (rank < 0) continue;
+        const int pos = start[ids[i]] + rank;
         src_token[pos] = (int32_t)(i / top);
         pos_of_pair[i] = pos;
     }
@@ -848,7 +877,7 @@ extern "C" int32_t nvh_moe_align(const int32_t* ids, int64_t num_tokens, int64_t
                 NVH_EINVAL, "nvh_moe_align: bad sizes");
     if (num_tokens == 0) return NVH_OK;
     const size_t lds = sizeof(int) * (size_t)(3 * experts + 1);
-    moe_align_kernel<<<dim3(1), 1024, lds, (hipStream_t)stream>>>(ids, num_tokens * top, (int)experts, (int)top, src_token, pos_of_pair, tile_expert, tile_row0,
+    moe_align_kernel<<<dim3(1), num_tokens * top <= 256 * ALIGN_KEPT ? 256 : 1024, lds, (hipStream_t)stream>>>(ids, num_tokens * top, (int)experts, (int)top, src_token, pos_of_pair, tile_expert, tile_row0,
                                                                   tile_rows, (int)max_tiles);
     NVH_CHECK_LAUNCH("nvh_moe_align");
     return NVH_OK;

@@ -60,3 +60,23 @@ def test_routing(experts, top, k, dtype):
     x[0] = float("nan")                                      # whatever is chosen then are different experts of the list
     ids = ops.moe_route_scored(x, w, top)[0]
     assert ids[0].min() >= 0 and ids[0].max() < experts and ids[0].unique().numel() == top
+
+
+@pytest.mark.parametrize("experts,top,tokens", [(1, 1, 1), (16, 2, 64), (63, 3, 341), (64, 4, 1000), (65, 5, 1025), (200, 8, 700), (4096, 2, 300)])
+def test_align(experts, top, tokens):
+    """The order by expert: every pair has a place of its own in its expert's run, the tiles cover the runs; pairs that one pass of the threads holds and more."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(experts + tokens)
+    ids = torch.randint(-1, experts, (tokens, top), generator=g).int()
+    plan = {k: v.cpu() if torch.is_tensor(v) else v for k, v in ops.moe_align(ids.cuda(), experts).items()}
+    flat, pos = ids.flatten().long(), plan["pos_of_pair"].long()
+    kept = flat >= 0
+    assert (pos[~kept] == -1).all() and torch.equal(pos[kept].sort().values, torch.arange(int(kept.sum())))
+    by_pos = torch.empty(int(kept.sum()), dtype=torch.long)
+    by_pos[pos[kept]] = flat[kept]
+    assert torch.equal(by_pos, flat[kept].sort().values)
+    assert torch.equal(plan["src_token"].long()[pos[kept]], torch.arange(tokens * top)[kept] // top)
+    tiles = [(int(e), int(r), int(n)) for e, r, n in zip(plan["tile_expert"], plan["tile_row0"], plan["tile_rows"]) if n > 0]
+    count = torch.bincount(flat[kept], minlength=experts)
+    starts = count.cumsum(0) - count
+    assert tiles == [(e, int(starts[e]) + r, min(64, int(count[e]) - r)) for e in range(experts) for r in range(0, int(count[e]), 64)]
