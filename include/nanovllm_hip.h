@@ -781,7 +781,10 @@ int32_t nvh_group_rmsnorm_gate(const float* o, const void* weight, int32_t weigh
  * nvh_gemm_grouped_any_nt: y[pos] = x[gather ? gather[pos] : pos] w[expert]^T over the tiles, w [E, N, K]; types as
  * nvh_gemm_any_nt; relu2: the squared relu of the result.  nvh_moe_combine: out fp32 [T, dim] = sum_r weights[t, r] y[pos_of_pair[t, r]] (+ shared[t], type A,
  * times sigmoid(shared_gate[t shared_gate_stride]) when a gate logit per token is given; weights NULL: all 1).
- * nvh_gemm_grouped_many_nt: nvh_gemm_grouped_any_nt for callers whose experts have many rows on average; the same results bit for bit. */
+ * nvh_gemm_grouped_many_nt: nvh_gemm_grouped_any_nt for callers whose experts have many rows on average; the same results bit for bit.
+ * nvh_gemm_grouped_gated_nt: the product over w [E, 2 inter, K] = [gate | up] and what nvh_act_mul (act 0 .. 2) or nvh_glu_clamp_pairs (act 3; weights
+ * [T, top] or NULL, gather and pos_of_pair of the same plan) make of it, y [pos, inter], bit for bit, in one launch.  bf16, K a multiple of 64, inter
+ * even, rows of x 16-byte aligned (others: NVH_ENOSYS); many: the experts have many rows on average. */
 int32_t nvh_moe_route(const float* logits, int64_t row_stride, int32_t* ids, float* weights, int64_t num_tokens, int64_t experts,
                       int64_t top, nvh_stream_t stream);
 /* nvh_moe_route with the router's product inside: logits = x w^T + bias (x [T, K], w [E, K], bias [E] or NULL, type A;
@@ -804,6 +807,10 @@ int32_t nvh_gemm_grouped_any_nt(const void* x, int64_t x_row_stride, const int32
 int32_t nvh_gemm_grouped_many_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
                                  const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
                                  int64_t N, int64_t K, int32_t relu2, int32_t in_f32, int32_t out_f32, nvh_stream_t stream);
+int32_t nvh_gemm_grouped_gated_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
+                                  const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles,
+                                  int64_t inter, int64_t K, int32_t act, const int32_t* pos_of_pair, const float* weights, int64_t top, float limit,
+                                  float alpha, int32_t many, nvh_stream_t stream);
 int32_t nvh_moe_combine(const void* y, int64_t y_row_stride, const int32_t* pos_of_pair, const float* weights, const void* shared,
                         int64_t shared_stride, const float* shared_gate, int64_t shared_gate_stride, float* out, int64_t num_tokens, int64_t dim,
                         int64_t top, int32_t act_f32, nvh_stream_t stream);

@@ -182,6 +182,13 @@ __device__ __forceinline__ void nvh_load8(const A* p, int64_t off, int valid, bo
 
 // From this many elements on an elementwise launch takes eight a lane (two workgroups a CU); fewer are faster one a lane (gelu, 64 x 3072: 3.1 and 2.2 us).
 constexpr int64_t NVH_PIECES = 1 << 20;
+// 0 silu, 1 gelu (tanh form), 2 squared relu.
+__device__ __forceinline__ float nvh_activation(float g, int act) {
+    if (act == 0) return g / (1.0f + expf(-g));
+    if (act == 1) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
+    return g > 0.f ? g * g : 0.f;
+}
+
 // Elementwise launches over rows of `cols` columns: a lane (256 a workgroup) takes E consecutive columns, cols a multiple of E.  False: past the end.
 template <int E>
 __device__ __forceinline__ bool nvh_piece(int64_t rows, int cols, int64_t& row, int& c) {

@@ -425,7 +425,46 @@ struct GroupedArgs {
     int64_t ldy;
     const int32_t *tile_expert, *tile_row0, *tile_rows;
     int N, K, vec_ok, relu2;
+    // gated products (w's rows are [gate | up] of N / 2 each, y the activation's N / 2 columns): what gated_pair() needs beside the sums
+    int act;                   // 0 .. 2: activation() of the gate times the other half; 3: glu_clamp()
+    const int32_t* pos_of_pair;       // with `weights` (a choice's weight times the expert's input): the row of a token's choice, [tokens, top]
+    const float* weights;
+    int top;
+    float limit, alpha;
 };
+
+// What glu_clamp_pairs_kernel does to a pair of sums.
+__device__ __forceinline__ float glu_clamp(float gate, float up, float w, float limit, float alpha) {
+    const float g = fminf(gate * w, limit), u = fminf(fmaxf(up * w, -limit), limit);
+    return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
+}
+
+// The weight row at place r of a gated tile that starts at place n0: of every sixteen places 4 q + {0, 1} are gate rows and 4 q + {2, 3} the up rows
+// of the same two columns, so the four sums of a lane are two finished pairs.  BLOCKS: sixteens that a wave multiplies; a lane's pairs in them are neighbours.
+template <int BLOCKS>
+__device__ __forceinline__ int gated_row(int n0, int r, int inter) {
+    const int block = (r >> 4) % BLOCKS, q = (r >> 2) & 3;
+    return min(n0 / 2 + r / (16 * BLOCKS) * 8 * BLOCKS + q * 2 * BLOCKS + block * 2 + (r & 1), inter - 1) + (r & 2 ? inter : 0);
+}
+
+// The weight of the choice of token `tok` whose row is m.
+__device__ __forceinline__ float choice_weight(const GroupedArgs& a, int tok, int m) {
+    const int64_t first = (int64_t)tok * a.top;
+    float w = 1.0f;
+    for (int j0 = 0; j0 < a.top; j0 += 4) {
+        int pos[4];
+        float wj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = min(j0 + u, a.top - 1);
+            pos[u] = a.pos_of_pair[first + j];
+            wj[u] = a.weights[first + j];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) w = pos[u] == m ? wj[u] : w;
+    }
+    return w;
+}
 
 template <bool OUT_F32>
 __global__ __launch_bounds__(256) void gemm_grouped_bf16_kernel(GroupedArgs a) {
@@ -469,6 +508,17 @@ __device__ __forceinline__ bool tile_goes_on(const GroupedArgs& a, int t) {
     return a.tile_expert[t] == a.tile_expert[t - 1] && a.tile_rows[t - 1] == nvh_any::GT && a.tile_row0[t] == a.tile_row0[t - 1] + nvh_any::GT;
 }
 
+// Two pairs of sums, rounded as the product alone leaves them, and what becomes of them.
+__device__ __forceinline__ bf16x2 gated_pair(const GroupedArgs& a, f32x4 v, float weight) {
+    bf16x2 o;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float g = (float)(bf16)v[e], u = (float)(bf16)v[2 + e];
+        o[e] = (bf16)(a.act == 3 ? glu_clamp(g, u, weight, a.limit, a.alpha) : nvh_activation(g, a.act) * u);
+    }
+    return o;
+}
+
 // Four consecutive columns of an output row, finished.
 template <bool OUT_F32>
 __device__ __forceinline__ void store_grouped(const GroupedArgs& a, int64_t m, int n, f32x4 v) {
@@ -489,7 +539,7 @@ __device__ __forceinline__ void store_grouped(const GroupedArgs& a, int64_t m, i
     }
 }
 
-template <bool OUT_F32>
+template <bool OUT_F32, bool GATED = false>
 __global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedArgs a, int max_tiles, int tiles_n) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // Workgroup ids go round the XCDs: two neighbouring list tiles with all their columns fall to one, so a row is fetched into one L2.
@@ -521,7 +571,7 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedA
     for (int i = 0; i < PW; ++i) {
         const int p = wave + 4 * i, r = (p & 15) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
         if (p < 16) {
-            src[i] = w + (int64_t)min(n0 + r, N - 1) * K + chunk * 8;
+            src[i] = w + (int64_t)(GATED ? gated_row<4>(n0, r, N / 2) : min(n0 + r, N - 1)) * K + chunk * 8;
         } else {                                             // (rows beyond the tile's repeat its last: not written)
             const int at = row0 + min(r, rows - 1);
             src[i] = x + (int64_t)(a.gather ? a.gather[at] : at) * a.ldx + chunk * 8;
@@ -540,7 +590,12 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedA
     for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __shared__ float row_weight[GATED ? TALL : 1];           // (looked up by a thread a row while the first step is on its way)
+    const bool weighs = GATED && a.weights && tid < rows;
+    const int tok = weighs ? a.gather[row0 + tid] : 0;
     stage(0);
+    if (weighs) row_weight[tid] = choice_weight(a, tok, row0 + tid);
+    if constexpr (GATED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");          // (before the barriers below)
     for (int step = 0; step < steps; ++step) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's pieces of the step
         __builtin_amdgcn_s_barrier();                        // everybody's; and everybody has left the stage that is filled next
@@ -572,6 +627,26 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedA
     for (int j = 0; j < 4; ++j) {
         const int r = wm + 16 * j + fr;
         if (r >= rows) continue;
+        if constexpr (GATED) {                               // eight neighbouring columns
+            const float weight = a.weights ? row_weight[r] : 1.0f;
+            const int c = (n0 + wn) / 2 + 8 * fq, inter = N / 2;
+            bf16* out = (bf16*)a.y + (int64_t)(row0 + r) * a.ldy + c;
+            bf16x8 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bf16x2 pair = gated_pair(a, acc[i][j], weight);
+                o[2 * i] = pair[0];
+                o[2 * i + 1] = pair[1];
+            }
+            if (inter % 8 == 0 && a.ldy % 8 == 0) {
+                if (c < inter) *reinterpret_cast<bf16x8*>(out) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (c + e < inter) out[e] = o[e];
+            }
+            continue;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int n = n0 + wn + 16 * i + 4 * fq;
@@ -580,12 +655,12 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_tall_bf16_kernel(GroupedA
     }
 }
 
-template <bool OUT_F32>
+template <bool OUT_F32, bool GATED = false>
 static bool launch_grouped_tall(const GroupedArgs& a, int64_t max_tiles, hipStream_t st) {
     const int64_t tiles_n = nvh_cdiv(a.N, TALL), slots = nvh_cdiv(max_tiles, 16) * 16 * tiles_n;
     constexpr int lds = 2 * 2 * TALL * 128;
     if (slots >= (1ll << 31)) return false;
-    gemm_grouped_tall_bf16_kernel<OUT_F32><<<dim3((unsigned)slots), 256, lds, st>>>(a, (int)max_tiles, (int)tiles_n);
+    gemm_grouped_tall_bf16_kernel<OUT_F32, GATED><<<dim3((unsigned)slots), 256, lds, st>>>(a, (int)max_tiles, (int)tiles_n);
     return true;
 }
 
@@ -594,7 +669,7 @@ static bool launch_grouped_tall(const GroupedArgs& a, int64_t max_tiles, hipStre
 // tiles (operands through registers, or straight from memory for few rows) and this one, rows an expert x N x K: 1 x 1536 x 1024 10.2 and 7.4,
 // 16 x 1536 x 1024 23.8 and 13.6 (3.7 TB/s), 8 x 768 x 1024 11.2 and 7.1, 16 x 1024 x 768 11.7 and 6.7, 64 x 1536 x 1024 26.4 and 18.2.
 constexpr int SHORT_N = 64, SHORT_LDS = 64 * 1024;
-template <bool OUT_F32, int MT, bool GATE = false>
+template <bool OUT_F32, int MT, bool GATE = false, bool GATED = false>
 __device__ __forceinline__ void gemm_grouped_short_tile(const GroupedArgs& a, int expert, int row0, int rows, int n0, char* smem, const bf16* gate = nullptr, int64_t ldg = 0) {
     constexpr int STAGE = (SHORT_N + 16 * MT) * 128, STAGES = SHORT_LDS / STAGE, AHEAD = STAGES - 1;
     constexpr int PIECES = SHORT_N / 8 + 2 * MT, PW = (PIECES + 3) / 4;
@@ -608,7 +683,7 @@ __device__ __forceinline__ void gemm_grouped_short_tile(const GroupedArgs& a, in
     for (int i = 0; i < PW; ++i) {
         const int p = (wave + 4 * i) % PIECES, r = (p < 8 ? p : p - 8) * 8 + (lane >> 3), chunk = (lane & 7) ^ ((r >> 1) & 7);
         if (p < 8) {
-            src[i] = w + (int64_t)min(n0 + r, N - 1) * K + chunk * 8;
+            src[i] = w + (int64_t)(GATED ? gated_row<1>(n0, r, N / 2) : min(n0 + r, N - 1)) * K + chunk * 8;
         } else {
             const int at = row0 + min(r, rows - 1);
             src[i] = x + (int64_t)(a.gather ? a.gather[at] : at) * a.ldx + chunk * 8;
@@ -631,7 +706,12 @@ __device__ __forceinline__ void gemm_grouped_short_tile(const GroupedArgs& a, in
 #pragma unroll
         for (int j = 0; j < MT; ++j) gates[j] = *reinterpret_cast<const bf16x4*>(gate + (int64_t)(row0 + min(16 * j + fr, rows - 1)) * ldg + min(n, N - 4));
     }
+    __shared__ float row_weight[GATED ? nvh_any::GT : 1];    // (as in the tall form)
+    const bool weighs = GATED && a.weights && tid < rows;
+    const int tok = weighs ? a.gather[row0 + tid] : 0;
     for (int step = 0; step < AHEAD && step < steps; ++step) stage(step);
+    if (weighs) row_weight[tid] = choice_weight(a, tok, row0 + tid);
+    if constexpr (GATED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     for (int step = 0; step < steps; ++step) {
         wait_steps_in_flight<PW, AHEAD - 1>(min(AHEAD - 1, steps - 1 - step));
         asm volatile("" ::: "memory");
@@ -659,19 +739,22 @@ __device__ __forceinline__ void gemm_grouped_short_tile(const GroupedArgs& a, in
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[j][e] *= nvh_any::sigmoid((float)gates[j][e]);
         }
-        store_grouped<OUT_F32>(a, row0 + 16 * j + fr, n, acc[j]);
+        if constexpr (GATED)
+            *reinterpret_cast<bf16x2*>((bf16*)a.y + (int64_t)(row0 + 16 * j + fr) * a.ldy + n / 2) = gated_pair(a, acc[j], a.weights ? row_weight[16 * j + fr] : 1.0f);
+        else
+            store_grouped<OUT_F32>(a, row0 + 16 * j + fr, n, acc[j]);
     }
 }
 
-template <bool OUT_F32>
+template <bool OUT_F32, bool GATED = false>
 __global__ __launch_bounds__(256) void gemm_grouped_short_bf16_kernel(GroupedArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int rows = a.tile_rows[blockIdx.y];
     if (rows <= 0) return;                                   // (uniform: a tile beyond the list's end)
     const int expert = a.tile_expert[blockIdx.y], row0 = a.tile_row0[blockIdx.y], n0 = blockIdx.x * SHORT_N;
-    if (rows <= 16) gemm_grouped_short_tile<OUT_F32, 1>(a, expert, row0, rows, n0, smem);
-    else if (rows <= 32) gemm_grouped_short_tile<OUT_F32, 2>(a, expert, row0, rows, n0, smem);
-    else gemm_grouped_short_tile<OUT_F32, 4>(a, expert, row0, rows, n0, smem);
+    if (rows <= 16) gemm_grouped_short_tile<OUT_F32, 1, false, GATED>(a, expert, row0, rows, n0, smem);
+    else if (rows <= 32) gemm_grouped_short_tile<OUT_F32, 2, false, GATED>(a, expert, row0, rows, n0, smem);
+    else gemm_grouped_short_tile<OUT_F32, 4, false, GATED>(a, expert, row0, rows, n0, smem);
 }
 
 // One weight matrix, 64 rows a tile.  us, the general form and this, fp32 results: 1 x 32768 x 1024 14.6 and 13.0 (5.2 TB/s), 64 x 32768 x 1024 20.2 and 16.8,
@@ -788,11 +871,7 @@ __global__ __launch_bounds__(256) void glu_clamp_pairs_kernel(const A* __restric
     nvh_load_piece<A, E>(row, v);
     nvh_load_piece<A, E>(row + inter, up);
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const float g = fminf(v[e] * w, limit);
-        const float u = fminf(fmaxf(up[e] * w, -limit), limit);
-        v[e] = g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
-    }
+    for (int e = 0; e < E; ++e) v[e] = glu_clamp(v[e], up[e], w, limit, alpha);
     nvh_store_piece<A, E>(y + (int64_t)pos * y_stride + c, v);
 }
 
@@ -910,6 +989,30 @@ static int32_t grouped_product(const void* x, int64_t x_row_stride, const int32_
     else if (out_f32) gemm_grouped_bf16_kernel<true><<<grid, 256, 0, st>>>(a);
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);
     NVH_CHECK_LAUNCH("nvh_gemm_grouped_any_nt");
+    return NVH_OK;
+}
+
+// The experts' gated first half in one launch: the activation has its gate and up sums side by side in a lane, so rows of 2 inter are neither written nor read.
+// Sums, their rounding and the activation's formulas are those of two launches.  us, two launches and one, 16 experts, K 1024, tokens x choices, inter:
+// 1 x 2, 768 7.5 and 6.4; 64 x 2, 384 8.3 and 6.3; 64 x 2, 768 12.3 and 10.1; 1000 x 2, 768 23.6 and 21.6; 1000 x 4, 768 39.0 and 36.4; 1000 x 4, 2048
+// 75 and 70.  What the exponentials cost is now in the product, where they are computed while the other workgroup of a CU multiplies.
+extern "C" int32_t nvh_gemm_grouped_gated_nt(const void* x, int64_t x_row_stride, const int32_t* gather, const void* w, void* y, int64_t y_row_stride,
+                                             const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* tile_rows, int64_t max_tiles, int64_t inter,
+                                             int64_t K, int32_t act, const int32_t* pos_of_pair, const float* weights, int64_t top, float limit, float alpha,
+                                             int32_t many, nvh_stream_t stream) {
+    NVH_REQUIRE(x && w && y && tile_expert && tile_row0 && tile_rows, NVH_EINVAL, "nvh_gemm_grouped_gated_nt: null pointer");
+    NVH_REQUIRE(max_tiles >= 0 && max_tiles < 65536 && inter > 0 && K > 0 && inter < (1 << 29) && K < (1 << 30) && x_row_stride >= K && y_row_stride >= inter && act >= 0 && act <= 3,
+                NVH_EINVAL, "nvh_gemm_grouped_gated_nt: bad sizes");
+    NVH_REQUIRE(!weights || (act == 3 && gather && pos_of_pair && top > 0 && top < (1 << 20)), NVH_EINVAL, "nvh_gemm_grouped_gated_nt: weights go with act 3 and the rows of the choices");
+    NVH_REQUIRE(K % 64 == 0 && inter % 2 == 0 && x_row_stride % 8 == 0 && y_row_stride % 2 == 0 && nvh_aligned16(x) && nvh_aligned16(w) && nvh_aligned16(y), NVH_ENOSYS,
+                "nvh_gemm_grouped_gated_nt: whole k-tiles, pairs of columns and aligned rows only");
+    if (max_tiles == 0) return NVH_OK;
+    const GroupedArgs a{x, x_row_stride, gather, w, y, y_row_stride, tile_expert, tile_row0, tile_rows, (int)(2 * inter), (int)K, 1, 0,
+                        act, pos_of_pair, weights, (int)top, limit, alpha};
+    hipStream_t st = (hipStream_t)stream;
+    if (!(many && launch_grouped_tall<false, true>(a, max_tiles, st)))
+        gemm_grouped_short_bf16_kernel<false, true><<<dim3((unsigned)nvh_cdiv(a.N, SHORT_N), (unsigned)max_tiles), 256, SHORT_LDS, st>>>(a);
+    NVH_CHECK_LAUNCH("nvh_gemm_grouped_gated_nt");
     return NVH_OK;
 }
 

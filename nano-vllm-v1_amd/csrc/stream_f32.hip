@@ -683,10 +683,7 @@ __global__ __launch_bounds__(256) void act_mul_kernel(const A* __restrict__ gu, 
     if (gated) nvh_load_piece<A, E>(src + inter, u);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const float g = v[e];
-        if (act == 0) v[e] = g / (1.0f + expf(-g));
-        else if (act == 1) v[e] = 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g)));
-        else v[e] = g > 0.f ? g * g : 0.f;
+        v[e] = nvh_activation(v[e], act);
         if (gated) v[e] *= u[e];
     }
     nvh_store_piece<A, E>(y + row * y_stride + c, v);

@@ -119,14 +119,13 @@ class SparseMoE(nn.Module):
             if self.shared_gate is not None:
                 gate = self.shared_gate(x, out_f32=True)
         plan = ops.moe_align(ids, self.experts)
-        fused = not self.gated and self.act == "relu2"       # (inside the product's epilogue)
-        first = ops.linear_grouped(x, self.gate_up.data, plan, gather=True, act="relu2" if fused else None)
-        if fused:
-            hidden = first
-        elif self.act == "glu_clamp":
-            hidden = ops.glu_clamp_pairs(first, plan, weights if self.weight_on_input else None, self.limit, self.alpha)
+        if self.gated:
+            hidden = ops.linear_grouped_gated(x, self.gate_up.data, plan, self.act, weights if self.weight_on_input else None, self.limit or 0.0, self.alpha)
         else:
-            hidden = ops.act_mul(first, self.act, self.gated)
+            fused = self.act == "relu2"                      # (inside the product's epilogue)
+            hidden = ops.linear_grouped(x, self.gate_up.data, plan, gather=True, act="relu2" if fused else None)
+            if not fused:
+                hidden = ops.act_mul(hidden, self.act, False)
         return ops.linear_grouped(hidden, self.down.data, plan, gather=False), plan, weights, gate
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

@@ -1326,6 +1326,24 @@ def glu_clamp_pairs(gate_up: torch.Tensor, plan: dict, weights: torch.Tensor | N
     return y
 
 
+def linear_grouped_gated(x: torch.Tensor, weight: torch.Tensor, plan: dict, act: str, weights: torch.Tensor | None = None, limit: float = 0.0, alpha: float = 1.702) -> torch.Tensor:
+    """The experts' gated first half: linear_grouped(x, weight, plan, gather=True) over weight [E, 2 I, K] = [gate | up], then act_mul, or for act
+    "glu_clamp" glu_clamp_pairs with the choices' `weights`.  bf16 rows with whole k-tiles: one launch, the same bits."""
+    e, n, k = weight.shape
+    if x.dtype != BF16 or k % 64 or n % 4 or x.stride(0) % 8 or (x.data_ptr() | weight.data_ptr()) % 16:
+        first = linear_grouped(x, weight, plan, gather=True)
+        return glu_clamp_pairs(first, plan, weights, limit, alpha) if act == "glu_clamp" else act_mul(first, act, True)
+    _act_flag(x, weight)
+    assert weight.is_contiguous() and x.dim() == 2 and x.shape[1] == k and x.stride(1) == 1
+    assert weights is None or (act == "glu_clamp" and weights.dtype == F32 and weights.is_contiguous() and weights.numel() == plan["pairs"])
+    y = torch.empty(plan["pairs"], n // 2, dtype=BF16, device=x.device)
+    _hip.call("nvh_gemm_grouped_gated_nt", x.data_ptr(), x.stride(0), plan["src_token"].data_ptr(), weight.data_ptr(), y.data_ptr(), n // 2,
+              plan["tile_expert"].data_ptr(), plan["tile_row0"].data_ptr(), plan["tile_rows"].data_ptr(), plan["max_tiles"], n // 2, k,
+              3 if act == "glu_clamp" else ACTS[act], plan["pos_of_pair"].data_ptr(), _p(weights), weights.shape[1] if weights is not None else 1,
+              float(limit), float(alpha), int(plan["pairs"] >= GROUPED_MANY_ROWS * e), _stream())
+    return y
+
+
 def moe_combine(y: torch.Tensor, plan: dict, weights: torch.Tensor | None, shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None,
                 top: int | None = None) -> torch.Tensor:
     """fp32 [T, dim]: every token's weighted sum of its choices' rows of y (in choice order), plus `shared` [T, dim], which is

@@ -62,6 +62,38 @@ def test_routing(experts, top, k, dtype):
     assert ids[0].min() >= 0 and ids[0].max() < experts and ids[0].unique().numel() == top
 
 
+@pytest.mark.parametrize("act,weighted", [("silu", False), ("gelu_tanh", False), ("relu2", False), ("glu_clamp", False), ("glu_clamp", True)])
+@pytest.mark.parametrize("inter,k", [(2, 64), (30, 128), (32, 192), (66, 448), (384, 1024)])
+def test_gated(inter, k, act, weighted):
+    """The activation in the product's epilogue against the product and the activation as launches of their own, bit for bit: experts of every size,
+    two and three choices a token, the tiles for few rows an expert and those for many; rows that no 16-byte load may be used on."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(inter + k)
+    T, E, top = 900, 9, 3
+    chance = torch.tensor([0.0, 0.01, 0.02, 0.1, 0.2, 0.5, 1.0, 2.0, 6.0])
+    ids = torch.multinomial(chance.expand(T, E) + 1e-6, top, generator=g).int().cuda()
+    ids[5] = -1                                              # a row of padding: no expert
+    x = torch.randn(T, k, generator=g).bfloat16().cuda()
+    w = (torch.randn(E, 2 * inter, k, generator=g) * 0.2).bfloat16().cuda()
+    weights = torch.rand(T, top, generator=g).cuda() if weighted else None
+    plan = ops.moe_align(ids, E)
+    first = ops.linear_grouped(x, w, plan, gather=True)
+    want = ops.glu_clamp_pairs(first, plan, weights, 1.5, 1.702) if act == "glu_clamp" else ops.act_mul(first, act, True)
+    odd = torch.empty(T, k + 1, dtype=x.dtype, device=x.device)
+    odd[:, :k] = x
+    at = plan["pos_of_pair"].long()
+    at = at[at >= 0]
+    assert at.numel() == (T - 1) * top and torch.equal(plan["src_token"].long()[at], torch.arange(T, device="cuda").repeat_interleave(top)[plan["pos_of_pair"] >= 0])
+    default = ops.GROUPED_MANY_ROWS
+    try:
+        for few in (1 << 30, 0):
+            ops.GROUPED_MANY_ROWS = few
+            for rows in (x, odd[:, :k]):
+                assert torch.equal(ops.linear_grouped_gated(rows, w, plan, act, weights, 1.5, 1.702)[at], want[at])
+    finally:
+        ops.GROUPED_MANY_ROWS = default
+
+
 @pytest.mark.parametrize("experts,top,tokens", [(1, 1, 1), (16, 2, 64), (63, 3, 341), (64, 4, 1000), (65, 5, 1025), (200, 8, 700), (4096, 2, 300)])
 def test_align(experts, top, tokens):
     """The order by expert: every pair has a place of its own in its expert's run, the tiles cover the runs; pairs that one pass of the threads holds and more."""
