@@ -10,8 +10,8 @@
 //                        once more, transposed within a page as the paged attention wants them); sigmoid of the head gates.
 //                        Where the query has no latent of its own the row is [q | dkv | ...]: q is not normed, and its heads'
 //                        rotated parts go to their places in the attention's query rows in the same launch
-//   nvh_gemm_heads_nt    y[t, h, :] = x[t, h, :] W[h]^T for every head (the any-shape product's tile, gemm_any.h, with a
-//                        weight matrix per head): the absorption of W_uk into the query and of W_uv into the output, the
+//   nvh_gemm_heads_nt    y[t, h, :] = x[t, h, :] W[h]^T for every head (the any-shape product's tile, gemm_any.h, or for whole bf16
+//                        k-tiles the ring tiles of moe.hip, with a weight matrix per head): the absorption of W_uk into the query and of W_uv into the output, the
 //                        latter optionally times a sigmoid gate per element
 //   nvh_latent_q_rotary  rotary of every head's rotated query part into its place behind the absorbed part
 // The attention itself is nvh_attn_paged_any (attention_any.hip).
