@@ -9,7 +9,7 @@
  *   block_tables          int32 [B, W] (-1 padded) or None             max_seqlen_q, max_seqlen_k  int
  *
  * Caller(table, check): calls into the kernel library without ctypes' per-argument objects.  table: name -> (address, kinds, fallback) with one
- * letter an argument, "i" for integers and pointers (int or None), "f" for fp32; caller(name, *args) calls the function with the GIL released and, when
+ * letter an argument, "p" for pointers (int or None), "i" for integers (int), "f" for fp32; caller(name, *args) calls the function with the GIL released and, when
  * it returns anything but 0, check(code, name).  Arguments of other types, and functions that the table marks with address 0, go to fallback(*args).
  * A call with 32 arguments took 6.0 us through ctypes, half of what a launch from Python costs, and takes 1.3 here.
  */
@@ -218,13 +218,16 @@ static PyObject* caller_call(PyObject* self, PyObject* const* args, size_t nargs
         if (kinds[k] == 'f') {
             if (!PyFloat_Check(a) && !PyLong_Check(a)) return fall_back(entry, args, n, args[0], c->check);
             const double d = PyFloat_AsDouble(a);
-            if (d == -1.0 && PyErr_Occurred()) return NULL;
+            if (d == -1.0 && PyErr_Occurred()) {             /* (an integer past a double's range: ctypes says so) */
+                PyErr_Clear();
+                return fall_back(entry, args, n, args[0], c->check);
+            }
             f[nf++] = (float)d;
         } else if (PyLong_Check(a)) {
             const unsigned long long x = PyLong_AsUnsignedLongLongMask(a);
             if (x == (unsigned long long)-1 && PyErr_Occurred()) return NULL;
             v[ni++] = (i64)x;
-        } else if (a == Py_None) {
+        } else if (a == Py_None && kinds[k] == 'p') {
             v[ni++] = 0;
         } else {
             return fall_back(entry, args, n, args[0], c->check);

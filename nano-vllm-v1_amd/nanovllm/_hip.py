@@ -196,8 +196,8 @@ def native_caller(handle, signatures, check_fn):
     table = {}
     for name, (res, args) in signatures.items():
         fn = getattr(handle, name)
-        kinds = "".join("f" if a is f32 else "i" for a in args)
-        plain = res is i32 and all(a in (vp, i64, u64, i32, f32) for a in args) and kinds.count("f") <= 8 and kinds.count("i") <= 46
+        kinds = "".join("f" if a is f32 else "p" if a is vp else "i" for a in args)
+        plain = res is i32 and all(a in (vp, i64, u64, i32, f32) for a in args) and kinds.count("f") <= 8 and len(kinds) - kinds.count("f") <= 46
         table[name] = (C.cast(fn, C.c_void_p).value if plain else 0, kinds, fn)
     return Caller(table, check_fn)
 

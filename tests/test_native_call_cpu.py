@@ -70,3 +70,20 @@ def test_errors_and_fallback():
         call("nobody", 1)
     with pytest.raises(TypeError):
         call()
+
+
+def test_what_ctypes_refuses_stays_refused():
+    """None is a null pointer and no integer, and a number has to fit a double: the function is not called."""
+    signatures = {"f": (i32, [vp, i64, i32, u64, f32])}
+    handle, seen = library(signatures, {})
+    call = _hip.native_caller(handle, signatures, _hip.check)
+    good = (None, 1, 2, 3, 4.0)
+    call("f", *good)
+    assert seen.pop() == ("f", good)
+    for at, bad in ((1, None), (2, None), (3, None), (4, None), (4, 10 ** 400)):
+        args = good[:at] + (bad,) + good[at + 1:]
+        with pytest.raises(C.ArgumentError):
+            handle.f(*args)
+        with pytest.raises(C.ArgumentError):
+            call("f", *args)
+    assert not seen
