@@ -1003,6 +1003,7 @@ extern "C" int32_t nvh_gemm_grouped_gated_nt(const void* x, int64_t x_row_stride
     NVH_REQUIRE(x && w && y && tile_expert && tile_row0 && tile_rows, NVH_EINVAL, "nvh_gemm_grouped_gated_nt: null pointer");
     NVH_REQUIRE(max_tiles >= 0 && max_tiles < 65536 && inter > 0 && K > 0 && inter < (1 << 29) && K < (1 << 30) && x_row_stride >= K && y_row_stride >= inter && act >= 0 && act <= 3,
                 NVH_EINVAL, "nvh_gemm_grouped_gated_nt: bad sizes");
+    NVH_REQUIRE(act != 3 || limit > 0.f, NVH_EINVAL, "nvh_gemm_grouped_gated_nt: act 3 needs a limit above 0");
     NVH_REQUIRE(!weights || (act == 3 && gather && pos_of_pair && top > 0 && top < (1 << 20)), NVH_EINVAL, "nvh_gemm_grouped_gated_nt: weights go with act 3 and the rows of the choices");
     NVH_REQUIRE(K % 64 == 0 && inter % 2 == 0 && x_row_stride % 8 == 0 && y_row_stride % 2 == 0 && nvh_aligned16(x) && nvh_aligned16(w) && nvh_aligned16(y), NVH_ENOSYS,
                 "nvh_gemm_grouped_gated_nt: whole k-tiles, pairs of columns and aligned rows only");
