@@ -1057,10 +1057,14 @@ extern "C" int32_t nvh_glu_clamp_pairs(const void* gate_up, int64_t row_stride, 
     if (pairs == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
     const bool vec = pairs * inter >= NVH_PIECES && inter % 8 == 0 && row_stride % 8 == 0 && y_stride % 8 == 0 && nvh_aligned16(gate_up) && nvh_aligned16(y);
-    const dim3 grid((unsigned)nvh_cdiv(pairs * inter, vec ? 2048 : 256));
+    const int64_t most = std::max<int64_t>((1ll << 31) / inter, 1);      // pairs a launch: a grid has fewer than 2^32 threads
     auto launch = [&](auto kernel, auto type) {
         typedef decltype(type) A;
-        kernel<<<grid, 256, 0, st>>>((const A*)gate_up, row_stride, pos_of_pair, weights, (A*)y, y_stride, pairs, (int)inter, limit, alpha);
+        for (int64_t p0 = 0; p0 < pairs; p0 += most) {
+            const int64_t n = std::min(most, pairs - p0);
+            kernel<<<dim3((unsigned)nvh_cdiv(n * inter, vec ? 2048 : 256)), 256, 0, st>>>((const A*)gate_up, row_stride, pos_of_pair + p0, weights ? weights + p0 : nullptr, (A*)y, y_stride, n,
+                                                                                           (int)inter, limit, alpha);
+        }
     };
     if (act_f32) launch(vec ? &glu_clamp_pairs_kernel<float, 8> : &glu_clamp_pairs_kernel<float, 1>, 0.f);
     else launch(vec ? &glu_clamp_pairs_kernel<bf16, 8> : &glu_clamp_pairs_kernel<bf16, 1>, (bf16)0.f);
