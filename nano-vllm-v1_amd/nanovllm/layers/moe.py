@@ -36,6 +36,12 @@ from .activation import Act, ActAndMul
 from .linear import MergedLinear
 
 
+def plain_call(module: nn.Module, forward) -> bool:
+    """Whether calling `module` runs `forward` and nothing else: no hook watches it and its forward is no other one."""
+    return getattr(module.forward, "__func__", None) is forward and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                                                                        or module._backward_pre_hooks or nn.modules.module._has_any_global_hook())
+
+
 class GatedMLP(nn.Module):
     """down(act(gate x) * up x) with gate and up in one product."""
 
@@ -139,6 +145,11 @@ class SparseMoE(nn.Module):
         y, plan, weights, gate = self._experts(x)
         return dict(y=y, plan=plan, weights=None if self.weight_on_input else weights, shared=self.shared(x) if self.shared is not None else None, gate=gate,
                     top=self.top)
+
+    def close_terms(self, x: torch.Tensor, name: str) -> dict:
+        """The result as an argument of a close: its parts, which the close sums (`moe`), or, where something watches or replaces forward(), the
+        rows that the module returns, as argument `name`.  The same bits either way."""
+        return dict(moe=self.parts(x)) if plain_call(self, SparseMoE.forward) else {name: self(x)}
 
     def terms(self, x: torch.Tensor) -> dict:
         """The result as the terms of a sum that a layer's close forms (ops.hyper_norm): the experts' rows under their weights and the

@@ -38,7 +38,7 @@ from ..layers.activation import Act
 from ..layers.attention import WindowedBiasAttention
 from ..layers.layernorm import StreamNorm
 from ..layers.linear import MergedLinear
-from ..layers.moe import SparseMoE
+from ..layers.moe import SparseMoE, plain_call
 from ..layers.recurrent import HGRN2, GatedLinearAttention, Mamba2
 from .lamutar import _get, layer_runs
 
@@ -137,7 +137,10 @@ class DinatarMoE(nn.Module):
                              shared_ff=int(_get(shared, "ff")) if shared else None, act="silu", router_bias=True)
 
     def forward(self, x: torch.Tensor) -> dict:
-        return dict(moe=self.moe.parts(x))
+        return dict(c32=self.moe(x))
+
+    def close_terms(self, x: torch.Tensor) -> dict:
+        return self.moe.close_terms(x, "c32") if plain_call(self, DinatarMoE.forward) else self(x)
 
 
 class DinatarLayer(nn.Module):
@@ -365,7 +368,7 @@ class DinatarForCausalLM(nn.Module):
             layer = self.layers[i]
             terms = layer.mixer(h, positions, p)
             if layer.mlp is not None:
-                terms.update(layer.mlp(h))
+                terms.update(layer.mlp.close_terms(h) if isinstance(layer.mlp, DinatarMoE) else layer.mlp(h))
             nxt = self.layers[self.runs[n + 1][0]].norm1.spec() if n + 1 < len(self.runs) else {}
             h = ops.residual_norm(x, **terms, **nxt)          # the layer's close and the next layer's norm in one launch
             if self.collect is not None:

@@ -41,7 +41,7 @@ from .. import ops
 from ..layers.attention import LatentAttention
 from ..layers.layernorm import PostSumRMSNorm
 from ..layers.linear import MergedLinear
-from ..layers.moe import SparseMoE
+from ..layers.moe import SparseMoE, plain_call
 from ..layers.recurrent import WKV, Retention, TokenShift
 from ..layers.rotary_embedding import rotary_frequencies
 from .lamutar import _get
@@ -111,8 +111,11 @@ class LakatarMoE(nn.Module):
                              groups=int(_get(groups, "count", 1)) if groups else 1, keep_groups=int(_get(groups, "keep", 1)) if groups else 1,
                              route_scale=float(_get(router, "scale", 1.0)), shared_gate=bool(shared))
 
-    def forward(self, x: torch.Tensor) -> dict:
-        return self.moe.parts(x)
+    def forward(self, x: torch.Tensor) -> torch.Tensor:
+        return self.moe(x)
+
+    def close_terms(self, x: torch.Tensor) -> dict:
+        return self.moe.close_terms(x, "y32") if plain_call(self, LakatarMoE.forward) else dict(y32=self(x))
 
 
 class LakatarLayer(nn.Module):
@@ -304,7 +307,7 @@ class LakatarForCausalLM(nn.Module):
         for layer in self.layers:
             h = layer.norm1.close(x, y=layer.mixer(h, positions))
             if layer.mlp is not None:
-                h = layer.norm2.close(x, moe=layer.mlp(h))
+                h = layer.norm2.close(x, **layer.mlp.close_terms(h))
             if self.collect is not None:
                 self.collect.append(x.clone())
         return x

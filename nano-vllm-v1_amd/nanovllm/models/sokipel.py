@@ -287,7 +287,7 @@ class SokipelForCausalLM(nn.Module):
             plain_next = i < last and self.layers[i + 1].canon is None
             h = layer.norm1.close(x, **terms, want_h=layer.mlp is not None or plain_next)
             if layer.mlp is not None:
-                h = layer.norm2.close(x, moe=layer.mlp.parts(h), want_h=plain_next)
+                h = layer.norm2.close(x, **layer.mlp.close_terms(h, "c32"), want_h=plain_next)
             if self.collect is not None:
                 self.collect.append(x.clone())
         return x
