@@ -1247,6 +1247,8 @@ void launch_gemm(const GemmArgs& a) {
 
 // Tile choice: the largest tile whose grid (x split_k) still gives every CU a workgroup.
 enum Tile { T16x32, T32x32, T16x128, T32x128, T64x128, T64x64, T128x64, T128x128, T256x128, T256x256 };
+// Tuning switch: the tile that products over more than 32 rows take whatever their size.
+bool tile_forced() { return nvh_switch(SW_GEMM_FORCE_TILE) >= T16x128 && nvh_switch(SW_GEMM_FORCE_TILE) <= T256x256; }
 Tile pick_tile(int64_t M, int64_t N, int split_k) {
     // decode batches: 128-row weight tiles leave most CUs idle unless the output is very wide; 32-row tiles in
     // two-wave workgroups (three fit a CU) keep the weight stream spread over the chip
@@ -1256,8 +1258,7 @@ Tile pick_tile(int64_t M, int64_t N, int split_k) {
     const bool m32_skinny = nvh_switch_on(SW_GEMM_M32_SKINNY);   // tuning switch
     if (M <= 32) return (narrow && (split_k == 1 || m32_skinny)) ? T32x32 : T32x128;      // with split-K the 128-row tile measured faster
     auto wgs = [&](int bm, int bn) { return nvh_cdiv(M, bm) * nvh_cdiv(N, bn) * split_k; };
-    const int force = (int)nvh_switch(SW_GEMM_FORCE_TILE);   // tuning switch
-    if (force >= T16x128 && force <= T256x256) return (Tile)force;
+    if (tile_forced()) return (Tile)nvh_switch(SW_GEMM_FORCE_TILE);
     if (M <= 64) return nvh_cdiv(N, 128) * split_k >= 384 ? T64x128 : T64x64;   // 33..64 rows: enough workgroups first
     const bool no256 = nvh_switch_on(SW_GEMM_NO_256);
     // big products (prefill of the 14B / 32B shapes, square GEMMs from 4096 up, the LM head from 256 rows): 256 x 256
@@ -1485,7 +1486,7 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
             // 33 .. 64 rows: 64-column tiles leave most CUs without one, and what a workgroup waits for is its stages; 16 columns (32 where 16 would be
             // more than a workgroup a CU) with six stages.  64 rows x N x 1024, us before and now: 1024 7.7 and 6.5, 2048 7.9 and 6.7, 4096 8.0 and 7.1,
             // 6144 8.3 and 7.7, 8192 8.6 and 8.4.  The same sums in the same order.
-            if (a.M <= 64 && a.split_k == 1 && !a.swiglu && !a.qkv && !a.sample && a.N <= 32 * 256) {
+            if (!tile_forced() && a.M <= 64 && a.split_k == 1 && !a.swiglu && !a.qkv && !a.sample && a.N <= 32 * 256) {
                 if (a.N <= 16 * 256) launch_gemm<64, 16, 1, 4, 6>(a);
                 else launch_gemm<64, 32, 2, 2, 6>(a);
                 break;
@@ -1500,7 +1501,7 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
             // One workgroup fits a CU, so a grid a little over 256 takes two rounds: then 128 x 128 tiles, fewer than 200 of them, in one round, eight
             // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 14.9, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
             // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4; one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  The same sums.
-            if (a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
+            if (!tile_forced() && a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
             else launch_gemm<128, 64, 2, 2, 4>(a);
             break;
         case T128x128: {

@@ -52,3 +52,19 @@ def test_switches_are_ignored_without_the_tuning_gate():
     assert subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True).stdout.strip() == "-1"
     env["NVH_TUNING"] = "1"
     assert subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True).stdout.strip() == "1"
+
+
+@pytest.mark.parametrize("flavor", [0, 1])
+@pytest.mark.parametrize("force,tile", [(4, (64, 128)), (5, (64, 64)), (6, (128, 64)), (7, (128, 128)), (8, (256, 128)), (9, (256, 256))])
+def test_a_forced_tile_is_that_tile(force, tile, flavor):
+    """Measurements name the tile they force: no rule behind the choice replaces it (whatever its waves; 128 x 96 and 192 are forms of 128 x 128)."""
+    import ctypes as C
+    from nanovllm import _hip
+    out = C.create_string_buffer(512)
+    for m in (33, 64, 128, 300, 1000):
+        for n in (1024, 4096, 5120, 8192, 18976):
+            for k in (1024, 5120):
+                with _hip.switch("NVH_GEMM_FORCE_TILE", force), _hip.switch("NVH_NO_KWAVES"), _hip.switch("NVH_GEMM_NO_KGROUPS"), _hip.switch("NVH_GEMM_NO_ROUND_CUT"), \
+                        _hip.switch("NVH_SWIGLU_NO_96"), _hip.switch("NVH_SWIGLU_NO_192"):
+                    assert _hip.lib().nvh_gemm_plan(m, n, k, 1, flavor, out, 512) == 0
+                assert out.value.decode().startswith("tile %dx%d " % tile), (m, n, k, out.value)
