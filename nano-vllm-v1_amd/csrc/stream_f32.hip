@@ -863,9 +863,14 @@ extern "C" int32_t nvh_gemm_any_nt(const void* x, int64_t x_row_stride, const vo
         if (vec_ok && K % nvh_any::F32_CHUNK == 0) {
             // The tile whose rounds over the CUs take least.  16 x 16 (two workgroups a CU) and 32 x 32 tiles while they fill at most a round;
             // then 32 x 64 or 64 x 64 ones, a workgroup a CU, a round of which takes 13 and 22 us for K = 1024.
+            // 16 rows or fewer are one row tile, whose time is the weights' way: 16 x 16 at any width, beyond a round with three stages, three workgroups
+            // a CU.  us, without a ring, 32 x 64 and this: 1 x 32000 x 1024 32.1, 33.8, 27.5; 1 x 32000 x 256 12.3, 14.1, 10.8; 1 x 12288 x 5120 49.5,
+            // 56.8, 46.0; 16 x 32000 x 1024 50.4, 34.9, 30.2; 16 x 12288 x 5120 84.5, 58.5, 53.3; two columns blocks a tile 27.5 at one row of
+            // 32000 x 1024, but 51.3 of 12288 x 5120.
             auto tiles = [&](int rows, int cols) { return nvh_cdiv(M, rows) * nvh_cdiv(N, cols); };
 #define NVH_F32_RING(MR, NC, STAGES) launch_f32_ring<MR, NC, STAGES>((const float*)x, x_row_stride, (const float*)w, (const float*)bias, (float*)y, y_row_stride, M, N, K, st)
             if (tiles(16, 16) <= 512) NVH_F32_RING(1, 1, 4);
+            else if (M <= 16) NVH_F32_RING(1, 1, 3);
             else if (tiles(32, 32) <= 256) NVH_F32_RING(2, 2, 2);
             else if (nvh_cdiv(tiles(64, 64), 256) * 22 < nvh_cdiv(tiles(32, 64), 256) * 13) NVH_F32_RING(4, 4, 2);
             else NVH_F32_RING(2, 4, 2);

@@ -23,6 +23,22 @@ def test_plain(m, n, k):
         assert torch.equal(ops.linear_any(x[r:r + 1].contiguous(), w, b)[0], want[r])
 
 
+@pytest.mark.parametrize("k", [32, 96, 160, 1024])
+@pytest.mark.parametrize("m", [1, 4, 15, 16])
+@pytest.mark.parametrize("n", [8192, 8193, 8210, 33000])
+def test_few_rows_of_many_columns(m, n, k):
+    """Around the width from which small tiles take more than a round: the general form's bits, and those of a call of one row."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(m * n + k)
+    x, w, b = torch.randn(m, k, generator=g).cuda(), torch.randn(n, k, generator=g).cuda(), torch.randn(n, generator=g).cuda()
+    want = ops.linear_any(odd_rows(x), w, b)
+    assert torch.equal(ops.linear_any(x, w, b), want)
+    assert torch.equal(ops.linear_any(x[m - 1:].contiguous(), w, b)[0], want[m - 1])
+    exact = x.double() @ w.double().t().contiguous() + b.double()
+    size = x.double().abs() @ w.double().abs().t().contiguous() + b.double().abs()
+    assert ((want.double() - exact).abs() <= size * (k + 4) * 2.0 ** -24).all()
+
+
 @pytest.mark.parametrize("relu2", [False, True])
 @pytest.mark.parametrize("n,k", [(16, 32), (33, 96), (100, 576), (576, 1024)])
 def test_grouped(n, k, relu2):
