@@ -1,6 +1,7 @@
 // Shared device helpers and host-side error plumbing for libnanovllm_hip.so (gfx950 only).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <stdint.h>
 #include <stdio.h>
 #include "../../include/nanovllm_hip.h"
@@ -37,6 +38,19 @@ void nvh_set_error(const char* fmt, ...);
             return NVH_ELAUNCH;                                                  \
         }                                                                        \
     } while (0)
+
+// A kernel with more than 64 KB of dynamic LDS needs an attribute for it, on every device once: `granted` remembers them, a bit a device.  False: refused.
+static inline bool nvh_grant_lds(std::atomic<uint64_t>& granted, const void* kernel, int bytes) {
+    int dev = 0;
+    const bool known = hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64;
+    if (known && (granted.load(std::memory_order_relaxed) >> dev & 1)) return true;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+        (void)hipGetLastError();                             // (the caller reports it; not the next launch)
+        return false;
+    }
+    if (known) granted.fetch_or(1ull << dev, std::memory_order_relaxed);
+    return true;
+}
 
 // Merge per-range attention partials ([row][split][128] fp32 + [row][split][2] (max, sum)) into bf16 rows.
 int32_t nvh_launch_attn_combine(const float* ws_acc, const float* ws_ml, void* out, int64_t rows, int num_splits,

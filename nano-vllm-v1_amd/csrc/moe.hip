@@ -814,11 +814,13 @@ __global__ __launch_bounds__(256, NC == 2 ? 2 : 1) void gemm_grouped_f32_ring_ke
 #undef NVH_RING
 }
 template <int NC>
-void launch_grouped_f32(const GroupedArgs& a, int64_t max_tiles, hipStream_t st) {
+bool launch_grouped_f32(const GroupedArgs& a, int64_t max_tiles, hipStream_t st) {
     constexpr int lds = std::max({nvh_any::f32_ring_bytes<1, NC, 3>(), nvh_any::f32_ring_bytes<2, NC, NC == 4 ? 3 : 2>(), nvh_any::f32_ring_bytes<3, NC, 2>(), NC == 4 ? nvh_any::f32_ring_bytes<4, NC, 2>() : 0});
     static_assert(lds <= (NC == 4 ? 160 : 80) * 1024);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_grouped_f32_ring_kernel<NC>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static std::atomic<uint64_t> granted{0};
+    if (!nvh_grant_lds(granted, reinterpret_cast<const void*>(&gemm_grouped_f32_ring_kernel<NC>), lds)) return false;
     gemm_grouped_f32_ring_kernel<NC><<<dim3((unsigned)nvh_cdiv(a.N, 16 * NC), (unsigned)max_tiles), 256, lds, st>>>(a);
+    return true;
 }
 
 // (a tile of the list is 64 rows: blockIdx.z is its upper or lower half)
@@ -983,8 +985,8 @@ static int32_t grouped_product(const void* x, int64_t x_row_stride, const int32_
         return NVH_OK;
     }
     if (in_f32 && vec_ok && K % nvh_any::F32_CHUNK == 0) {
-        if (tall) launch_grouped_f32<4>(a, max_tiles, st);
-        else launch_grouped_f32<2>(a, max_tiles, st);
+        const bool ok = tall ? launch_grouped_f32<4>(a, max_tiles, st) : launch_grouped_f32<2>(a, max_tiles, st);
+        NVH_REQUIRE(ok, NVH_ENOSYS, "nvh_gemm_grouped_any_nt: more than 64 KB of LDS for a workgroup refused");
     } else if (in_f32) gemm_grouped_f32_kernel<<<dim3((unsigned)nvh_cdiv(N, 32), (unsigned)max_tiles, 2), 256, 0, st>>>(a);
     else if (out_f32) gemm_grouped_bf16_kernel<true><<<grid, 256, 0, st>>>(a);
     else gemm_grouped_bf16_kernel<false><<<grid, 256, 0, st>>>(a);

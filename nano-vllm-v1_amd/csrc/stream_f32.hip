@@ -765,11 +765,13 @@ __global__ __launch_bounds__(256) void gemm_any_f32_ring_kernel(const float* __r
 }
 
 template <int MR, int NC, int STAGES>
-void launch_f32_ring(const float* x, int64_t ldx, const float* w, const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+bool launch_f32_ring(const float* x, int64_t ldx, const float* w, const float* bias, float* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t st) {
     constexpr int lds = nvh_any::f32_ring_bytes<MR, NC, STAGES>();
-    if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_any_f32_ring_kernel<MR, NC, STAGES>), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    static std::atomic<uint64_t> granted{0};
+    if (lds > 64 * 1024 && !nvh_grant_lds(granted, reinterpret_cast<const void*>(&gemm_any_f32_ring_kernel<MR, NC, STAGES>), lds)) return false;
     gemm_any_f32_ring_kernel<MR, NC, STAGES><<<dim3((unsigned)nvh_cdiv(N, 16 * NC), (unsigned)std::min<int64_t>(nvh_cdiv(M, 16 * MR), 65535)), 256, lds, st>>>(
         x, ldx, w, bias, y, ldy, (int)M, (int)N, (int)K);
+    return true;
 }
 
 }  // namespace
@@ -869,12 +871,14 @@ extern "C" int32_t nvh_gemm_any_nt(const void* x, int64_t x_row_stride, const vo
             // 32000 x 1024, but 51.3 of 12288 x 5120.
             auto tiles = [&](int rows, int cols) { return nvh_cdiv(M, rows) * nvh_cdiv(N, cols); };
 #define NVH_F32_RING(MR, NC, STAGES) launch_f32_ring<MR, NC, STAGES>((const float*)x, x_row_stride, (const float*)w, (const float*)bias, (float*)y, y_row_stride, M, N, K, st)
-            if (tiles(16, 16) <= 512) NVH_F32_RING(1, 1, 4);
-            else if (M <= 16) NVH_F32_RING(1, 1, 3);
-            else if (tiles(32, 32) <= 256) NVH_F32_RING(2, 2, 2);
-            else if (nvh_cdiv(tiles(64, 64), 256) * 22 < nvh_cdiv(tiles(32, 64), 256) * 13) NVH_F32_RING(4, 4, 2);
-            else NVH_F32_RING(2, 4, 2);
+            bool ok;
+            if (tiles(16, 16) <= 512) ok = NVH_F32_RING(1, 1, 4);
+            else if (M <= 16) ok = NVH_F32_RING(1, 1, 3);
+            else if (tiles(32, 32) <= 256) ok = NVH_F32_RING(2, 2, 2);
+            else if (nvh_cdiv(tiles(64, 64), 256) * 22 < nvh_cdiv(tiles(32, 64), 256) * 13) ok = NVH_F32_RING(4, 4, 2);
+            else ok = NVH_F32_RING(2, 4, 2);
 #undef NVH_F32_RING
+            NVH_REQUIRE(ok, NVH_ENOSYS, "nvh_gemm_any_nt: more than 64 KB of LDS for a workgroup refused");
             NVH_CHECK_LAUNCH("nvh_gemm_any_nt");
             return NVH_OK;
         }
