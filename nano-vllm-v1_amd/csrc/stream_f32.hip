@@ -5,6 +5,7 @@
 // Every kernel is one workgroup per row (or a flat element grid) with 16-byte accesses where the row allows.
 #include "common.h"
 #include <algorithm>
+#include <type_traits>
 #include "gemm_any.h"
 
 namespace {
@@ -253,32 +254,43 @@ __device__ __forceinline__ void moe_sum(const MoeTerms& m, int64_t t, int c, flo
 // a chain of a load, one or two sums across the workgroup and a store, whose latencies are the launch at any number of rows that a step brings
 // (column by column through LDS every pass over the row waits for its own loads).  R: pieces of 1024 columns.  MOE: with a mixture's terms.
 // us for 64 rows of 1024, column by column and this: residual norm with two terms 9.1 and 4.4; a mixture's launch and a close after it 7.8 + 5.0 and 4.5.
-template <typename A, int R, bool MOE>
-__global__ __launch_bounds__(256) void residual_norm_vec_kernel(CloseArgs p, MoeTerms m) {
+// FORM: what a call can have; terms that it has not cost registers and branches all the same.  us, bf16, one form for everything and so: one branch, 64 x 1024
+// 3.4 and 2.9, 64 x 4096 6.0 and 4.3, 1000 x 5120 35.9 and 14.8; the norm alone, fp32, 1000 x 5120 30.0 and 11.6 (with five pieces instead of eight, and the
+// norm's weights requested when the sums have begun: they come from L2, and what long rows need is more rows a CU).  THREADS: rows of at most 256 columns are
+// one wave's, without a barrier (4000 x 64, two branches 10.6 and 5.3).  None of it changes a sum.
+enum CloseForm { CLOSE_ANY, CLOSE_ONE, CLOSE_BRANCH, CLOSE_SUMS };        // everything; no second branch; a branch alone, no mean and no bias; no branch
+template <typename A, int R, bool MOE, int FORM, int THREADS>
+__global__ __launch_bounds__(THREADS) void residual_norm_vec_kernel(CloseArgs p, MoeTerms m) {
+    constexpr bool HAS_A = FORM != CLOSE_SUMS, HAS_B = FORM == CLOSE_ANY, HAS_C = FORM != CLOSE_BRANCH, CENTRED = FORM != CLOSE_BRANCH;
+    static_assert(!MOE || HAS_C, "a mixture's sum is a term");
+    constexpr bool LATE = R > 4 && FORM != CLOSE_BRANCH;      // the norm's weights after the first sums
     __shared__ float red[16];
     const int64_t row = blockIdx.x;
     const int dim = p.dim;
-    const A* a = p.a ? (const A*)p.a + row * p.a_stride : nullptr;
-    const A* b = p.b ? (const A*)p.b + row * p.b_stride : nullptr;
-    const A* c = p.c ? (const A*)p.c + row * p.c_stride : nullptr;
-    const float* c32 = p.c32 ? p.c32 + row * p.c32_stride : nullptr;
+    const bool has_a = FORM == CLOSE_BRANCH || (HAS_A && p.a);
+    const A* a = (const A*)p.a + (HAS_A ? row * p.a_stride : 0);
+    const A* b = HAS_B && p.b ? (const A*)p.b + row * p.b_stride : nullptr;
+    const A* c = HAS_C && p.c ? (const A*)p.c + row * p.c_stride : nullptr;
+    const float* c32 = HAS_C && p.c32 ? p.c32 + row * p.c32_stride : nullptr;
+    const A *pa = HAS_A ? (const A*)p.wa : nullptr, *pb = HAS_B ? (const A*)p.wb : nullptr, *bias = CENTRED && p.norm ? (const A*)p.nb : nullptr;
     float* xr = p.x + row * dim;
+    auto sum = [](float v, float* at) { return THREADS == 64 ? wave_sum(v) : block_sum4(v, at); };
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 va[R], vb[R], x[R], wa[R], wb[R], vc[R], vc32[R], nw[R], nb[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int col = (threadIdx.x + 256 * j) * 4;
+        const int col = (threadIdx.x + THREADS * j) * 4;
         va[j] = vb[j] = x[j] = wa[j] = wb[j] = vc[j] = vc32[j] = nw[j] = nb[j] = zero;
         if (col < dim) {
-            if (a) va[j] = load4(a + col);
+            if (has_a) va[j] = load4(a + col);
             if (b) vb[j] = load4(b + col);
             if (c) vc[j] = load4(c + col);
             if (c32) vc32[j] = load4(c32 + col);
             x[j] = load4(xr + col);
-            if (p.wa) wa[j] = load4((const A*)p.wa + col);
-            if (p.wb) wb[j] = load4((const A*)p.wb + col);
-            if (p.norm) nw[j] = load4((const A*)p.nw + col);
-            if (p.norm && p.nb) nb[j] = load4((const A*)p.nb + col);
+            if (pa) wa[j] = load4(pa + col);
+            if (pb) wb[j] = load4(pb + col);
+            if (!LATE && p.norm) nw[j] = load4((const A*)p.nw + col);
+            if (!LATE && bias) nb[j] = load4(bias + col);
             if constexpr (MOE) {
                 float s[4];
                 moe_sum<A, 4>(m, row, col, s);
@@ -292,45 +304,55 @@ __global__ __launch_bounds__(256) void residual_norm_vec_kernel(CloseArgs p, Moe
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             sa += va[j][e] * va[j][e];
-            sb += vb[j][e] * vb[j][e];
+            if (HAS_B) sb += vb[j][e] * vb[j][e];
         }
-    if (p.wa) ia = 1.0f / sqrtf(block_sum4(sa, red) / (float)dim + p.branch_eps);
-    if (p.wb) ib = 1.0f / sqrtf(block_sum4(sb, red + 4) / (float)dim + p.branch_eps);
-    float sum = 0.f;
+    if (pa) ia = 1.0f / sqrtf(sum(sa, red) / (float)dim + p.branch_eps);
+    if (pb) ib = 1.0f / sqrtf(sum(sb, red + 4) / (float)dim + p.branch_eps);
+    float total = 0.f;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int col = (threadIdx.x + 256 * j) * 4;
+        const int col = (threadIdx.x + THREADS * j) * 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float s = 0.f;
-            if (a) s += p.wa ? va[j][e] * ia * wa[j][e] : va[j][e];
-            if (b) s += p.wb ? vb[j][e] * ib * wb[j][e] : vb[j][e];
-            s *= p.branch_scale;
+            if (has_a) s += pa ? va[j][e] * ia * wa[j][e] : va[j][e];
+            if (b) s += pb ? vb[j][e] * ib * wb[j][e] : vb[j][e];
+            if (HAS_A) s *= p.branch_scale;
             if (c) s += vc[j][e];
             if (MOE || c32) s += vc32[j][e];
             x[j][e] += s;
-            sum += x[j][e];
+            if (CENTRED) total += x[j][e];
         }
-        if (col < dim && (MOE || a || b || c || c32)) *reinterpret_cast<f32x4*>(xr + col) = x[j];
+        if (col < dim && (MOE || has_a || b || c || c32)) *reinterpret_cast<f32x4*>(xr + col) = x[j];
     }
     if (p.norm == 0) return;
-    const float mean = p.norm == 1 ? block_sum4(sum, red + 8) / (float)dim : 0.f;
+    if constexpr (LATE) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const int col = (threadIdx.x + THREADS * j) * 4;
+            if (col < dim) {
+                nw[j] = load4((const A*)p.nw + col);
+                if (bias) nb[j] = load4(bias + col);
+            }
+        }
+    }
+    const float mean = CENTRED && p.norm == 1 ? sum(total, red + 8) / (float)dim : 0.f;
     float sq = 0.f;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const bool in = (threadIdx.x + 256 * j) * 4 < dim;
+        const bool in = (threadIdx.x + THREADS * j) * 4 < dim;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            x[j][e] = in ? x[j][e] - mean : 0.f;
+            if (CENTRED) x[j][e] = in ? x[j][e] - mean : 0.f;        // (columns past the end are 0 as they are)
             sq += x[j][e] * x[j][e];
         }
     }
-    const float inv = 1.0f / sqrtf(block_sum4(sq, red + 12) / (float)dim + p.eps);
+    const float inv = 1.0f / sqrtf(sum(sq, red + 12) / (float)dim + p.eps);
     A* h = (A*)p.h + row * p.h_stride;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
-        const int col = (threadIdx.x + 256 * j) * 4;
-        if (col < dim) store4(h + col, p.nb ? x[j] * inv * nw[j] + nb[j] : x[j] * inv * nw[j]);
+        const int col = (threadIdx.x + THREADS * j) * 4;
+        if (col < dim) store4(h + col, bias ? x[j] * inv * nw[j] + nb[j] : x[j] * inv * nw[j]);
     }
 }
 
@@ -364,11 +386,29 @@ static bool launch_residual_norm_vec(const CloseArgs& p, const MoeTerms& m, int6
         !rows_of_fours<A>(p.nb, 0) || (p.norm && !rows_of_fours<A>(p.h, p.h_stride)) || !nvh_aligned16(p.x) || !moe_of_fours<A>(m))
         return false;
     const dim3 grid((unsigned)rows);
-    NVH_CLOSE_CASES(residual_norm_vec_kernel, p, m)
+    const bool branch = p.a && !p.b && !p.c && !p.c32 && !m.y && p.norm != 1 && !p.nb;
+    auto launch = [&](auto r, auto threads) {
+        constexpr int R = decltype(r)::value, T = decltype(threads)::value;
+        auto form = [&](auto f, auto moe) { residual_norm_vec_kernel<A, R, decltype(moe)::value, decltype(f)::value, T><<<grid, T, 0, st>>>(p, m); };
+        const std::true_type with{};
+        const std::false_type without{};
+        if (branch) return form(std::integral_constant<int, CLOSE_BRANCH>{}, without);
+        if (!p.a && !p.b) return m.y ? form(std::integral_constant<int, CLOSE_SUMS>{}, with) : form(std::integral_constant<int, CLOSE_SUMS>{}, without);
+        if (!p.b) return m.y ? form(std::integral_constant<int, CLOSE_ONE>{}, with) : form(std::integral_constant<int, CLOSE_ONE>{}, without);
+        return m.y ? form(std::integral_constant<int, CLOSE_ANY>{}, with) : form(std::integral_constant<int, CLOSE_ANY>{}, without);
+    };
+    const std::integral_constant<int, 256> four_waves{};
+    if (p.dim <= 256) launch(std::integral_constant<int, 1>{}, std::integral_constant<int, 64>{});
+    else if (pieces == 1) launch(std::integral_constant<int, 1>{}, four_waves);
+    else if (pieces == 2) launch(std::integral_constant<int, 2>{}, four_waves);
+    else if (pieces == 4) launch(std::integral_constant<int, 4>{}, four_waves);
+    else if (p.dim <= 5120 && !branch) launch(std::integral_constant<int, 5>{}, four_waves);
+    else if (p.dim <= 6144 && !branch) launch(std::integral_constant<int, 6>{}, four_waves);
+    else launch(std::integral_constant<int, 8>{}, four_waves);
     return true;
 }
 
-template <typename A>
+template <typename A, bool MOE>
 __global__ __launch_bounds__(256) void residual_norm_kernel(CloseArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
@@ -404,13 +444,13 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(CloseArgs p, MoeTerm
         s *= p.branch_scale;
         if (c) s += (float)c[i];
         if (c32) s += c32[i];
-        if (m.y) {
+        if constexpr (MOE) {
             float e[1];
             moe_sum<A, 1>(m, row, i, e);
             s += e[0];
         }
         const float v = xr[i] + s;
-        if (a || b || c || c32 || m.y) xr[i] = v;
+        if (MOE || a || b || c || c32) xr[i] = v;
         rowbuf[i] = v;
         sum += v;
     }
@@ -452,7 +492,7 @@ struct PostNormArgs {
     int dim, write_x;
 };
 
-template <typename A>
+template <typename A, bool MOE>
 __global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
@@ -465,10 +505,10 @@ __global__ __launch_bounds__(256) void residual_postnorm_kernel(PostNormArgs p, 
     float sq = 0.f;
     for (int i = threadIdx.x; i < dim; i += 256) {
         float v = p.alpha * xr[i];
-        if (y || y32 || m.y) {
+        if (MOE || y || y32) {
             float s = y ? (float)y[i] : 0.f;
             if (y32) s += y32[i];
-            if (m.y) {
+            if constexpr (MOE) {
                 float e[1];
                 moe_sum<A, 1>(m, row, i, e);
                 s += e[0];
@@ -571,7 +611,7 @@ struct SubNormArgs {
     int dim;
 };
 
-template <typename A>
+template <typename A, bool MOE>
 __global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p, MoeTerms m) {
     extern __shared__ float rowbuf[];
     __shared__ float red[4];
@@ -586,7 +626,7 @@ __global__ __launch_bounds__(256) void residual_subnorm_kernel(SubNormArgs p, Mo
         if (a) y = p.sa * (float)a[i];
         if (b) y = __builtin_fmaf(p.sb, (float)b[i], y);
         if (c32) y += c32[i];
-        if (m.y) {
+        if constexpr (MOE) {
             float e[1];
             moe_sum<A, 1>(m, row, i, e);
             y += e[0];
@@ -910,6 +950,18 @@ extern "C" int32_t nvh_embedding_pos_stream(const int64_t* ids, const int64_t* p
     return NVH_OK;
 }
 
+// The closes column by column, a row in LDS: any size and alignment.
+template <typename Args>
+static int32_t launch_close_columns(void (*kernel)(Args, MoeTerms), const Args& p, const MoeTerms& m, int64_t rows, int64_t dim, hipStream_t st) {
+    const size_t lds = sizeof(float) * (size_t)dim;
+    if (lds > 48 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        NVH_REQUIRE(e == hipSuccess, NVH_ENOSYS, "close of a residual row: %zu bytes of LDS refused", lds);
+    }
+    kernel<<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    return NVH_OK;
+}
+
 static int32_t residual_norm(const void* a, int64_t a_stride, const void* a_weight, const void* b, int64_t b_stride, const void* b_weight,
                              float branch_scale, float branch_eps, const void* c, int64_t c_stride, const float* c32, int64_t c32_stride, float* x,
                              int32_t norm_kind, const void* norm_weight, const void* norm_bias, float eps, void* h, int64_t h_stride, int64_t rows,
@@ -924,14 +976,9 @@ static int32_t residual_norm(const void* a, int64_t a_stride, const void* a_weig
         NVH_CHECK_LAUNCH("nvh_residual_norm");
         return NVH_OK;
     }
-    const size_t lds = sizeof(float) * (size_t)dim;
-    if (lds > 48 * 1024) {
-        const hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_norm_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_norm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_norm: %zu bytes of LDS refused", lds);
-    }
-    if (act_f32) residual_norm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
-    else residual_norm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    const int32_t rc = act_f32 ? (m.y ? launch_close_columns(&residual_norm_kernel<float, true>, p, m, rows, dim, st) : launch_close_columns(&residual_norm_kernel<float, false>, p, m, rows, dim, st))
+                               : (m.y ? launch_close_columns(&residual_norm_kernel<bf16, true>, p, m, rows, dim, st) : launch_close_columns(&residual_norm_kernel<bf16, false>, p, m, rows, dim, st));
+    if (rc != NVH_OK) return rc;
     NVH_CHECK_LAUNCH("nvh_residual_norm");
     return NVH_OK;
 }
@@ -969,14 +1016,9 @@ static int32_t residual_postnorm(const void* y, int64_t y_stride, const float* y
         NVH_CHECK_LAUNCH("nvh_residual_postnorm");
         return NVH_OK;
     }
-    const size_t lds = sizeof(float) * (size_t)dim;
-    if (lds > 48 * 1024) {
-        const hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_postnorm_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_postnorm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_postnorm: %zu bytes of LDS refused", lds);
-    }
-    if (act_f32) residual_postnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
-    else residual_postnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    const int32_t rc = act_f32 ? (m.y ? launch_close_columns(&residual_postnorm_kernel<float, true>, p, m, rows, dim, st) : launch_close_columns(&residual_postnorm_kernel<float, false>, p, m, rows, dim, st))
+                               : (m.y ? launch_close_columns(&residual_postnorm_kernel<bf16, true>, p, m, rows, dim, st) : launch_close_columns(&residual_postnorm_kernel<bf16, false>, p, m, rows, dim, st));
+    if (rc != NVH_OK) return rc;
     NVH_CHECK_LAUNCH("nvh_residual_postnorm");
     return NVH_OK;
 }
@@ -1011,14 +1053,9 @@ static int32_t residual_subnorm(const void* a, int64_t a_stride, float a_scale, 
         NVH_CHECK_LAUNCH("nvh_residual_subnorm");
         return NVH_OK;
     }
-    const size_t lds = sizeof(float) * (size_t)dim;
-    if (lds > 48 * 1024) {
-        const hipError_t e1 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_subnorm_kernel<float>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        const hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(&residual_subnorm_kernel<bf16>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        NVH_REQUIRE(e1 == hipSuccess && e2 == hipSuccess, NVH_ENOSYS, "nvh_residual_subnorm: %zu bytes of LDS refused", lds);
-    }
-    if (act_f32) residual_subnorm_kernel<float><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
-    else residual_subnorm_kernel<bf16><<<dim3((unsigned)rows), 256, lds, st>>>(p, m);
+    const int32_t rc = act_f32 ? (m.y ? launch_close_columns(&residual_subnorm_kernel<float, true>, p, m, rows, dim, st) : launch_close_columns(&residual_subnorm_kernel<float, false>, p, m, rows, dim, st))
+                               : (m.y ? launch_close_columns(&residual_subnorm_kernel<bf16, true>, p, m, rows, dim, st) : launch_close_columns(&residual_subnorm_kernel<bf16, false>, p, m, rows, dim, st));
+    if (rc != NVH_OK) return rc;
     NVH_CHECK_LAUNCH("nvh_residual_subnorm");
     return NVH_OK;
 }

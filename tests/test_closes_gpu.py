@@ -60,3 +60,24 @@ def test_a_mixture_inside_the_close(tokens, dim, top, experts, dtype):
                              (ops.residual_subnorm, dict(weight=wn[:1], eps=1e-5), "c32")):
             one, other = x.clone(), x.clone()
             assert torch.equal(op(one, **kw, moe=moe), op(other, **kw, **{name: summed})) and torch.equal(one, other)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dim", [4, 252, 256, 260, 1024, 2048, 4096, 4100, 5120, 5124, 6144, 6148, 8192])
+def test_every_form_of_the_norm_close(dim, dtype):
+    """Calls with a second branch, with one and further terms, with one alone and without any, at the edges of the columns a lane and a wave hold."""
+    from nanovllm import ops
+    rows = 3
+    g = torch.Generator().manual_seed(dim)
+    def t(*shape):
+        return torch.randn(*shape, generator=g).to(dtype).cuda()
+    a, b, c, w1, w2, w3, w4 = t(rows, dim), t(rows, dim), t(rows, dim), t(dim), t(dim), t(dim), t(dim)
+    c32, x = torch.randn(rows, dim, generator=g).cuda(), torch.randn(rows, dim, generator=g).cuda()
+    branch, second = dict(a=a, a_weight=w1, branch_scale=0.5, branch_eps=1e-6), dict(b=b, b_weight=w2)
+    rms, layer = dict(norm="rms", weight=w3, eps=1e-5), dict(norm="layer", weight=w3, bias=w4, eps=1e-5)
+    for kw in ({**branch, **second, **rms}, {**branch, **second, "c": c, **layer}, {**branch, **rms}, {"a": a, **rms}, branch, {**branch, **layer}, {"a": a, "c32": c32, **rms},
+               {**branch, "c": c, "c32": c32, **layer}, rms, layer, {"c": c, **rms}, {"c32": c32, **layer}, {"c": c, "c32": c32}, second, {"b": b, "c32": c32, **rms}):
+        one, other = x.clone(), x.clone()
+        h = ops.residual_norm(one, **kw)
+        k = ops.residual_norm(other, **{n: odd_rows(v) if torch.is_tensor(v) and v.dim() == 2 else v for n, v in kw.items()})
+        assert close_to(one, other, torch.float32) and (h is None or close_to(h, k, dtype)), kw.keys()
