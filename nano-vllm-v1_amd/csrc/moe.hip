@@ -857,7 +857,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const A* __restrict__ 
 // the gate's value capped above and the other half's value clamped to +-limit,
 //   g = min(w G, limit);  u = clamp(w U, -limit, limit);  y = g sigmoid(alpha g) (u + 1).
 // A pair's row is pos_of_pair[pair] (< 0: the pair has no row).  E: elements a lane, 8 where rows and strides allow 16-byte accesses.
-// us, a workgroup a pair and so: 3024 pairs of 768 5.8 and 5.5, 1024 of 3072 7.4 and 6.3.
 template <typename A, int E>
 __global__ __launch_bounds__(256) void glu_clamp_pairs_kernel(const A* __restrict__ gu, int64_t gu_stride, const int32_t* __restrict__ pos_of_pair,
                                                               const float* __restrict__ weights, A* __restrict__ y, int64_t y_stride, int64_t pairs, int inter, float limit,
@@ -875,6 +874,17 @@ __global__ __launch_bounds__(256) void glu_clamp_pairs_kernel(const A* __restric
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = glu_clamp(v[e], up[e], w, limit, alpha);
     nvh_store_piece<A, E>(y + (int64_t)pos * y_stride + c, v);
+}
+// The same with a workgroup a pair.
+template <typename A>
+__global__ __launch_bounds__(256) void glu_clamp_rows_kernel(const A* __restrict__ gu, int64_t gu_stride, const int32_t* __restrict__ pos_of_pair,
+                                                             const float* __restrict__ weights, A* __restrict__ y, int64_t y_stride, int inter, float limit, float alpha) {
+    const int64_t pair = blockIdx.x;
+    const int pos = pos_of_pair[pair];
+    if (pos < 0) return;
+    const float w = weights ? weights[pair] : 1.0f;
+    const A* row = gu + (int64_t)pos * gu_stride;
+    for (int c = threadIdx.x; c < inter; c += 256) y[(int64_t)pos * y_stride + c] = (A)glu_clamp((float)row[c], (float)row[inter + c], w, limit, alpha);
 }
 
 }  // namespace
@@ -1058,18 +1068,27 @@ extern "C" int32_t nvh_glu_clamp_pairs(const void* gate_up, int64_t row_stride, 
                 "nvh_glu_clamp_pairs: bad argument");
     if (pairs == 0) return NVH_OK;
     hipStream_t st = (hipStream_t)stream;
-    const bool vec = pairs * inter >= NVH_PIECES && inter % 8 == 0 && row_stride % 8 == 0 && y_stride % 8 == 0 && nvh_aligned16(gate_up) && nvh_aligned16(y);
+    // One element a lane spreads few elements over the chip, eight a lane make wide accesses of many; between them, and where rows do not allow wide
+    // accesses, a workgroup a pair.  us, one, eight a lane and a workgroup a pair: 300 x 768 bf16 2.4, 2.7, 2.6; 64 x 3072 2.3, 2.6, 3.7; 900 x 768 3.3,
+    // 3.3, 3.1; 1400 x 768 fp32 4.3, 3.9, 3.6; 4000 x 768 8.2, 5.9, 6.4; 1000 x 3072 8.1, 5.9, 6.6; 3000 x 1001 8.7, none, 6.5.
+    const int64_t total = pairs * inter;
+    const bool wide = inter % 8 == 0 && row_stride % 8 == 0 && y_stride % 8 == 0 && nvh_aligned16(gate_up) && nvh_aligned16(y);
+    const bool few = total < (1 << 19), vec = !few && wide && (inter > 1024 || total >= (act_f32 ? 1 << 21 : 1 << 20));
     const int64_t most = std::max<int64_t>((1ll << 31) / inter, 1);      // pairs a launch: a grid has fewer than 2^32 threads
-    auto launch = [&](auto kernel, auto type) {
+    auto launch = [&](auto kernel, auto rows_kernel, auto type) {
         typedef decltype(type) A;
+        if (!few && !vec) {
+            rows_kernel<<<dim3((unsigned)pairs), 256, 0, st>>>((const A*)gate_up, row_stride, pos_of_pair, weights, (A*)y, y_stride, (int)inter, limit, alpha);
+            return;
+        }
         for (int64_t p0 = 0; p0 < pairs; p0 += most) {
             const int64_t n = std::min(most, pairs - p0);
             kernel<<<dim3((unsigned)nvh_cdiv(n * inter, vec ? 2048 : 256)), 256, 0, st>>>((const A*)gate_up, row_stride, pos_of_pair + p0, weights ? weights + p0 : nullptr, (A*)y, y_stride, n,
                                                                                            (int)inter, limit, alpha);
         }
     };
-    if (act_f32) launch(vec ? &glu_clamp_pairs_kernel<float, 8> : &glu_clamp_pairs_kernel<float, 1>, 0.f);
-    else launch(vec ? &glu_clamp_pairs_kernel<bf16, 8> : &glu_clamp_pairs_kernel<bf16, 1>, (bf16)0.f);
+    if (act_f32) launch(vec ? &glu_clamp_pairs_kernel<float, 8> : &glu_clamp_pairs_kernel<float, 1>, &glu_clamp_rows_kernel<float>, 0.f);
+    else launch(vec ? &glu_clamp_pairs_kernel<bf16, 8> : &glu_clamp_pairs_kernel<bf16, 1>, &glu_clamp_rows_kernel<bf16>, (bf16)0.f);
     NVH_CHECK_LAUNCH("nvh_glu_clamp_pairs");
     return NVH_OK;
 }
