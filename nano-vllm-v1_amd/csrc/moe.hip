@@ -128,7 +128,7 @@ __device__ __forceinline__ int pick_largest(const float (&z)[PL], float& best) {
 // The same with the router's product inside: z[e] = x . w[e] + bias[e] in fp32.  One workgroup per token: its four waves take the experts four at
 // a time in turn, every dot product spread over a wave's lanes and summed across it; the logits meet in LDS and the first wave picks.
 // PL: experts a lane of the picking wave holds: experts <= 64 PL.
-template <typename A, int PL>
+template <typename A, int PL, int PIECES>
 __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restrict__ x, int64_t ldx, const A* __restrict__ w, const A* __restrict__ bias,
                                                                int32_t* __restrict__ ids, float* __restrict__ weights, float* __restrict__ logits_out,
                                                                int experts, int K, int top, int vec, int sigmoid_scores) {
@@ -136,8 +136,7 @@ __global__ __launch_bounds__(256) void moe_route_linear_kernel(const A* __restri
     const int64_t t = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const A* xr = x + t * ldx;
-    // fp32 rows of many experts come at L2's rate: one piece at a time then, for more waves a CU
-    constexpr int EG = 4, PIECES = sizeof(A) == 4 && PL > 1 ? 1 : 2;
+    constexpr int EG = 4;
     for (int e0 = wave * EG; e0 < experts; e0 += 4 * EG) {
         float acc[EG];
         route_dots<EG, PIECES>(xr, [&](int g) { return w + (int64_t)min(e0 + g, experts - 1) * K; }, K, vec, lane, acc);
@@ -910,16 +909,21 @@ extern "C" int32_t nvh_moe_route_linear(const void* x, int64_t x_row_stride, con
     const dim3 grid((unsigned)num_tokens);
     hipStream_t st = (hipStream_t)stream;
     const int vec = K % 8 == 0 && x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w);
-#define NVH_ROUTE_LINEAR(A, PL) moe_route_linear_kernel<A, PL><<<grid, 256, 0, st>>>((const A*)x, x_row_stride, (const A*)w, (const A*)bias, ids, weights, logits_out, (int)experts, (int)K, (int)top, vec, sigmoid_scores)
+#define NVH_ROUTE_LINEAR(A, PL, PIECES) moe_route_linear_kernel<A, PL, PIECES><<<grid, 256, 0, st>>>((const A*)x, x_row_stride, (const A*)w, (const A*)bias, ids, weights, logits_out, (int)experts, (int)K, (int)top, vec, sigmoid_scores)
+    // Many experts: the rows come at L2's rate, and one piece at a time leaves room for more waves a CU, in fp32 always, in bf16 where a row has not two whole
+    // ones (256 rows of 1000, 1100 tokens 72.9 and 44.5 us, 4000 169 and 132).
+    const bool two = K >= 1024;
     if (experts <= 64) {
-        if (act_f32) NVH_ROUTE_LINEAR(float, 1);
-        else NVH_ROUTE_LINEAR(bf16, 1);
+        if (act_f32) NVH_ROUTE_LINEAR(float, 1, 2);
+        else NVH_ROUTE_LINEAR(bf16, 1, 2);
     } else if (experts <= 256) {
-        if (act_f32) NVH_ROUTE_LINEAR(float, 4);
-        else NVH_ROUTE_LINEAR(bf16, 4);
+        if (act_f32) NVH_ROUTE_LINEAR(float, 4, 1);
+        else if (two) NVH_ROUTE_LINEAR(bf16, 4, 2);
+        else NVH_ROUTE_LINEAR(bf16, 4, 1);
     } else {
-        if (act_f32) NVH_ROUTE_LINEAR(float, ROUTE_MAX_PER_LANE);
-        else NVH_ROUTE_LINEAR(bf16, ROUTE_MAX_PER_LANE);
+        if (act_f32) NVH_ROUTE_LINEAR(float, ROUTE_MAX_PER_LANE, 1);
+        else if (two) NVH_ROUTE_LINEAR(bf16, ROUTE_MAX_PER_LANE, 2);
+        else NVH_ROUTE_LINEAR(bf16, ROUTE_MAX_PER_LANE, 1);
     }
 #undef NVH_ROUTE_LINEAR
     NVH_CHECK_LAUNCH("nvh_moe_route_linear");
@@ -943,17 +947,26 @@ extern "C" int32_t nvh_moe_route_scored(const void* x, int64_t x_row_stride, con
     const int64_t rows = experts + num_aux;
     // Rows a wave: four, or three where that is as many passes (17 .. 24 rows), or in fp32; the fp32 rows of many experts come at L2's rate, and more
     // waves a CU are worth more than two pieces at once (128 experts, 1008 tokens: 28.7 us as it was, 31.4 with two rows of two pieces, 26.7 so).
+    // Two pieces at once where a row has two and the tokens are few: they cost registers, which more than four workgroups a CU need more, and without two
+    // whole pieces they are never used.  us, bf16, as it was before either, two at once and one: 17 rows of 1024, 64 tokens 7.4, 4.9, 5.0, 4000 19.0, 14.3, 12.0;
+    // of 1000, 4000 tokens 19.2, 20.8, 14.9; 6 rows of 96, 4000 tokens 12.1, 13.6, 9.6.
+    // More experts than a wave picks from at once: two pieces at any number of tokens (128 experts of 2048, 2000 tokens 55.7 and 58.1).
+    const bool two = K >= 1024 && (num_tokens <= 1024 || experts > 64);
+#define NVH_ROUTE_PIECES(A, PL, EG)                \
+    if (two) NVH_ROUTE_SCORED(A, PL, EG, 2);      \
+    else NVH_ROUTE_SCORED(A, PL, EG, 1)
     if (experts <= 64) {
-        if (act_f32) NVH_ROUTE_SCORED(float, 1, 3, 2);
-        else if (rows > 16 && rows <= 24) NVH_ROUTE_SCORED(bf16, 1, 3, 2);
-        else NVH_ROUTE_SCORED(bf16, 1, 4, 2);
+        if (act_f32) { NVH_ROUTE_PIECES(float, 1, 3); }
+        else if (rows > 16 && rows <= 24) { NVH_ROUTE_PIECES(bf16, 1, 3); }
+        else { NVH_ROUTE_PIECES(bf16, 1, 4); }
     } else if (experts <= 256) {
         if (act_f32) NVH_ROUTE_SCORED(float, 4, 4, 1);
-        else NVH_ROUTE_SCORED(bf16, 4, 4, 2);
+        else { NVH_ROUTE_PIECES(bf16, 4, 4); }
     } else {
         if (act_f32) NVH_ROUTE_SCORED(float, ROUTE_MAX_PER_LANE, 4, 1);
-        else NVH_ROUTE_SCORED(bf16, ROUTE_MAX_PER_LANE, 4, 2);
+        else { NVH_ROUTE_PIECES(bf16, ROUTE_MAX_PER_LANE, 4); }
     }
+#undef NVH_ROUTE_PIECES
 #undef NVH_ROUTE_SCORED
     NVH_CHECK_LAUNCH("nvh_moe_route_scored");
     return NVH_OK;

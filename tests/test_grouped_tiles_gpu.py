@@ -112,3 +112,23 @@ def test_align(experts, top, tokens):
     count = torch.bincount(flat[kept], minlength=experts)
     starts = count.cumsum(0) - count
     assert tiles == [(e, int(starts[e]) + r, min(64, int(count[e]) - r)) for e in range(experts) for r in range(0, int(count[e]), 64)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("experts,k", [(5, 96), (16, 1000), (16, 1024), (30, 1536), (100, 1024), (100, 1000), (300, 2048), (300, 520)])
+def test_routing_does_not_depend_on_the_number_of_tokens(experts, k, dtype):
+    """More tokens than the rows' pieces are taken two at once for, against the same tokens in calls of few: choices, weights, scores and further products."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(experts + k)
+    T, top = 1030, min(experts, 4)
+    x, w, aux = (torch.randn(n, k, generator=g).to(dtype).cuda() for n in (T, experts, 1))
+    many = ops.moe_route_scored(x, w, top, aux=aux, want_scores=True, renorm=True)
+    for lo, hi in ((0, 7), (500, 564), (1020, 1030)):
+        few = ops.moe_route_scored(x[lo:hi], w, top, aux=aux, want_scores=True, renorm=True)
+        assert all(torch.equal(m[lo:hi], f) for m, f in zip(many, few))
+    many_linear, few_linear = ops.moe_route_linear(x, w, None, top, want_logits=True), ops.moe_route_linear(x[:9], w, None, top, want_logits=True)
+    assert all(torch.equal(m[:9], f) for m, f in zip(many_linear, few_linear))
+    size = x.double().abs() @ w.double().abs().t().contiguous()
+    slack = (2 * (k + 8) * 2.0 ** -24 * size).amax(1, keepdim=True) + 2.0 ** -20          # (of the logits; softmax's relative error is at most twice theirs)
+    scores = torch.softmax(x.double() @ w.double().t().contiguous(), 1)
+    assert ((many[3].double() - scores).abs() <= scores * 2 * slack + 1e-30).all()
