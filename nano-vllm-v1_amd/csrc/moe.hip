@@ -339,9 +339,11 @@ __global__ __launch_bounds__(256) void moe_route_scored_kernel(const A* __restri
 // One workgroup: every pair counts itself with its expert, which is its rank there; the sums over the experts before are a scan by one wave; a pair's position is
 // the two together.  What bounds it is the chain of launch, load, barriers and stores.  us, before (counts, starts by one lane, a second count for the
 // positions; 1024 threads always) and so, tokens x choices of experts: 64 x 2 of 16 2.8 and 2.6, 1000 x 4 of 16 4.9 and 3.9, 1000 x 4 of 64 7.4 and 4.0,
-// 301 x 8 of 128 9.6 and 3.8, 1000 x 8 of 256 20.1 and 9.1.
+// 301 x 8 of 128 9.6 and 3.8, 1000 x 8 of 256 20.1 and 8.3, 4000 x 8 of 64 23.6 and 20.0, 8000 x 8 of 64 42.3 and 39.4 (four kept pairs a thread instead of
+// sixteen, and the ranks of the others left in memory meanwhile: 26.7 and 53.4).
 // (Which position a pair gets within its block depends on the order the lanes arrive in; nothing downstream depends on it.)
-constexpr int ALIGN_KEPT = 4;                                // pairs whose expert and place a thread keeps in registers
+// KEPT: pairs whose expert and place a thread keeps in registers; those beyond are counted first and take their places from their run's end.
+template <int KEPT>
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restrict__ ids, int64_t pairs, int experts, int top, int32_t* __restrict__ src_token,
                                                          int32_t* __restrict__ pos_of_pair, int32_t* __restrict__ tile_expert, int32_t* __restrict__ tile_row0,
                                                          int32_t* __restrict__ tile_rows, int max_tiles) {
@@ -350,9 +352,9 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
     int* start = sh + experts;
     int* tile0 = sh + 2 * experts;
     const int tid = threadIdx.x, threads = blockDim.x;
-    int kept_e[ALIGN_KEPT], kept_rank[ALIGN_KEPT];
+    int kept_e[KEPT], kept_rank[KEPT];
 #pragma unroll
-    for (int u = 0; u < ALIGN_KEPT; ++u) {
+    for (int u = 0; u < KEPT; ++u) {
         const int64_t i = tid + (int64_t)u * threads;
         kept_e[u] = i < pairs ? ids[i] : -1;
     }
@@ -360,11 +362,13 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
     __syncthreads();
     // a pair's rank among its expert's is what the count was when it came
 #pragma unroll
-    for (int u = 0; u < ALIGN_KEPT; ++u)
+    for (int u = 0; u < KEPT; ++u)
         if (kept_e[u] >= 0 && kept_e[u] < experts) kept_rank[u] = atomicAdd(&count[kept_e[u]], 1);
-    for (int64_t i = tid + (int64_t)ALIGN_KEPT * threads; i < pairs; i += threads) {
+    const bool more = pairs > (int64_t)KEPT * threads;             // (uniform)
+    if (more) __syncthreads();                               // every rank is taken before a pair without one is counted: the ranks are a run's first places
+    for (int64_t i = tid + (int64_t)KEPT * threads; i < pairs; i += threads) {
         const int e = ids[i];
-        pos_of_pair[i] = e >= 0 && e < experts ? atomicAdd(&count[e], 1) : -1;       // (the rank for now: read back below by this thread)
+        if (e >= 0 && e < experts) atomicAdd(&count[e], 1);  // (no rank: it would have to wait in memory; these places are taken from the run's end, below)
     }
     __syncthreads();
     if (tid < 64) {                                          // sums over the experts before, 64 of them at a time
@@ -398,19 +402,20 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int32_t* __restri
         }
     }
 #pragma unroll
-    for (int u = 0; u < ALIGN_KEPT; ++u) {
+    for (int u = 0; u < KEPT; ++u) {
         const int64_t i = tid + (int64_t)u * threads;
         if (i >= pairs) continue;
         const bool ok = kept_e[u] >= 0 && kept_e[u] < experts;
         const int pos = ok ? start[kept_e[u]] + kept_rank[u] : -1;
-        if (ok) src_token[pos] = (int32_t)(i / top);
+        if (ok) src_token[pos] = (int32_t)((uint32_t)i / (uint32_t)top);
         pos_of_pair[i] = pos;
     }
-    for (int64_t i = tid + (int64_t)ALIGN_KEPT * threads; i < pairs; i += threads) {
-        const int rank = pos_of_pair[i];
-        if (rank < 0) continue;
-        const int pos = start[ids[i]] + rank;
-        src_token[pos] = (int32_t)(i / top);
+    if (more) __syncthreads();                               // the counts have been read; now they go down to what was counted with a rank
+    for (int64_t i = tid + (int64_t)KEPT * threads; i < pairs; i += threads) {
+        const int e = ids[i];
+        const bool ok = e >= 0 && e < experts;
+        const int pos = ok ? start[e] + atomicAdd(&count[e], -1) - 1 : -1;
+        if (ok) src_token[pos] = (int32_t)((uint32_t)i / (uint32_t)top);
         pos_of_pair[i] = pos;
     }
 }
@@ -981,8 +986,11 @@ extern "C" int32_t nvh_moe_align(const int32_t* ids, int64_t num_tokens, int64_t
                 NVH_EINVAL, "nvh_moe_align: bad sizes");
     if (num_tokens == 0) return NVH_OK;
     const size_t lds = sizeof(int) * (size_t)(3 * experts + 1);
-    moe_align_kernel<<<dim3(1), num_tokens * top <= 256 * ALIGN_KEPT ? 256 : 1024, lds, (hipStream_t)stream>>>(ids, num_tokens * top, (int)experts, (int)top, src_token, pos_of_pair, tile_expert, tile_row0,
-                                                                  tile_rows, (int)max_tiles);
+    const int64_t pairs = num_tokens * top;
+    auto launch = [&](auto kernel, int threads) { kernel<<<dim3(1), threads, lds, (hipStream_t)stream>>>(ids, pairs, (int)experts, (int)top, src_token, pos_of_pair, tile_expert, tile_row0, tile_rows, (int)max_tiles); };
+    if (pairs <= 1024) launch(&moe_align_kernel<4>, 256);
+    else if (pairs <= 4096) launch(&moe_align_kernel<4>, 1024);
+    else launch(&moe_align_kernel<16>, 1024);
     NVH_CHECK_LAUNCH("nvh_moe_align");
     return NVH_OK;
 }

@@ -132,3 +132,9 @@ def test_routing_does_not_depend_on_the_number_of_tokens(experts, k, dtype):
     slack = (2 * (k + 8) * 2.0 ** -24 * size).amax(1, keepdim=True) + 2.0 ** -20          # (of the logits; softmax's relative error is at most twice theirs)
     scores = torch.softmax(x.double() @ w.double().t().contiguous(), 1)
     assert ((many[3].double() - scores).abs() <= scores * 2 * slack + 1e-30).all()
+
+
+@pytest.mark.parametrize("experts,top,tokens", [(64, 8, 512), (64, 8, 513), (64, 8, 2048), (64, 8, 2049), (3, 2, 9000)])
+def test_align_of_pairs_beyond_the_kept_ones(experts, top, tokens):
+    """Around the numbers of pairs that the threads keep: those beyond are counted after the others' ranks are taken, and placed from their run's end."""
+    test_align(experts, top, tokens)
