@@ -396,8 +396,7 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(StreamConvArgs p) {
 // The same for TT consecutive tokens a workgroup, four columns a lane: everything a lane reads is on its way at once, an input once instead of once
 // per tap.  STEP (TT 1, one token per sequence): the slot is brought up to date as well - the lane that reads a column's carried inputs is the only
 // one that does.
-// us, four taps over 1024 columns, with the state's update: 1000 tokens 8.2 (one workgroup a token) and 6.2, 2000 13.8 and 6.8; one token of 64 sequences, where
-// the update is inside, 4.7 and 2.5.
+// us, four taps over 1024 columns: one token of 64 sequences, where the update is inside, 4.7 and 2.5.
 template <typename A, int TT, int TAPS, bool STEP>
 __global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, int64_t num_tokens, float* carried_out) {
     static_assert(!STEP || TT == 1, "a step brings one token per sequence");
@@ -451,11 +450,14 @@ __global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, 
 template <typename A>
 static bool launch_stream_conv_run(const StreamConvArgs& p, int64_t num_tokens, int taps, float* carried_out, hipStream_t st) {
     if (taps < 2 || taps > 4 || p.dim % 4 || p.h_stride % 4 || !nvh_aligned16(p.x) || !nvh_aligned16(p.state) || ((uintptr_t)p.h % (4 * sizeof(A)))) return false;
+    // Four tokens a workgroup from about 2 M elements on, where inputs read once instead of once per tap count; below, and for few tokens, more workgroups do.  us, one token a
+    // workgroup (as before, by columns) and four, four taps: 1000 x 64 5.1, 4.7, 6.5; 1000 x 1024 9.2, 5.5, 6.9; 1000 x 2048 18.1, 8.0, 7.4; 2000 x 1024 14.6,
+    // 8.0, 7.2; 4000 x 1024 22.4, 15.0, 10.3.
     constexpr int TT = 4;
     const unsigned cols = (unsigned)nvh_cdiv(p.dim, 1024);
 #define NVH_CONV_RUN(TAPS)                                                                                                                                   \
     if (carried_out) stream_conv_run_kernel<A, 1, TAPS, true><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, carried_out);               \
-    else if (num_tokens >= 256 * TT / 2) stream_conv_run_kernel<A, TT, TAPS, false><<<dim3((unsigned)nvh_cdiv(num_tokens, TT), cols), 256, 0, st>>>(p, num_tokens, nullptr); \
+    else if (num_tokens >= 512 && num_tokens * p.dim >= 15 << 17) stream_conv_run_kernel<A, TT, TAPS, false><<<dim3((unsigned)nvh_cdiv(num_tokens, TT), cols), 256, 0, st>>>(p, num_tokens, nullptr); \
     else stream_conv_run_kernel<A, 1, TAPS, false><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, nullptr)
     if (taps == 2) { NVH_CONV_RUN(2); }
     else if (taps == 3) { NVH_CONV_RUN(3); }

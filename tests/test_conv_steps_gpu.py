@@ -83,3 +83,23 @@ def test_delta_operands(taps, heads, groups, dk, dv, dtype):
         lo = int(cu[i])
         alone = operands(lo, lo + n, slots[i:i + 1].contiguous(), torch.tensor([0, n]).int().cuda(), ctx[i:i + 1].contiguous())
         assert torch.equal(whole[lo:lo + n], alone)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps,dim", [(2, 1024), (3, 2052), (4, 1028)])
+def test_stream_of_many_elements(taps, dim, dtype):
+    """Runs of four tokens a workgroup (from 15 * 2^17 elements on) across the ends of sequences: the bits of a call per sequence, which takes a token each."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(taps * dim)
+    lens, carried = [1, 3, 2, 5, 4, 1900 * 1024 // dim, 1, 62, 9], [0, 4, 7, 0, 3, 2, 9, 0, 1]
+    cu, slots, ctx = portions(g, lens, carried)
+    assert sum(lens) * dim >= 15 << 17
+    x, w = torch.randn(sum(lens), dim, generator=g).cuda(), (torch.randn(dim, taps, generator=g) * 0.3).to(dtype).cuda()
+    state = torch.randn(len(lens) + 1, taps - 1, dim, generator=g).cuda()
+    one, many = state.clone(), state.clone()
+    h = ops.stream_conv(x, w, many, slots, cu, ctx)
+    for b, n in enumerate(lens):
+        lo = int(cu[b])
+        alone = ops.stream_conv(x[lo:lo + n].contiguous(), w, one, slots[b:b + 1].contiguous(), torch.tensor([0, n]).int().cuda(), ctx[b:b + 1].contiguous())
+        assert torch.equal(h[lo:lo + n], alone)
+    assert torch.equal(one, many)
