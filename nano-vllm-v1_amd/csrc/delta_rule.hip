@@ -1129,10 +1129,12 @@ extern "C" int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, con
     GatedDeltaPrepArgs p{qkv, qkv_stride, b, a, b_stride, a_stride, conv_w, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens, out,
                          (int)batch, (int)taps, (int)heads, (int)qk_heads, (int)dk, (int)dv};
     hipStream_t st = (hipStream_t)stream;
-    // Tokens a workgroup: four, or two where four leave the chip fewer than four workgroups a CU; below two a CU one token each, as ever.
+    // Tokens a workgroup: four, or two where four leave the chip fewer than four workgroups a CU; below two and a half a CU (long rows of a sequence's tokens, which
+    // share their inputs: two) one token each, as ever.  us, one and two, 64 tokens of 16 heads of 64 x 64: single tokens 5.8 and 6.3, of a prompt 5.2 and 5.4; 100
+    // of a prompt 6.7 and 6.1; 128 of 8 heads of 128 x 128 6.7 and 6.2.
     const bool run = taps >= 2 && taps <= 4 && (2 * dk + dv + 4) * 4 * (int64_t)sizeof(float) <= 32 * 1024;
     if (run && num_tokens * heads >= 4096) launch_gated_delta_prep_run<4>(p, num_tokens, act_f32, st);
-    else if (run && num_tokens * heads >= 1024) launch_gated_delta_prep_run<2>(p, num_tokens, act_f32, st);
+    else if (run && num_tokens * heads >= (2 * dk + dv >= 256 && batch < num_tokens ? 1024 : 1280)) launch_gated_delta_prep_run<2>(p, num_tokens, act_f32, st);
     else {
         const dim3 grid((unsigned)num_tokens, (unsigned)heads);
         if (act_f32) gated_delta_prep_kernel<float><<<grid, 256, lds, st>>>(p);
