@@ -226,7 +226,6 @@ struct SsdPrepArgs {
     const int32_t *slots, *cu_seqlens_q, *context_lens;
     int batch, taps, H, inner, gn;  // inner = H dv, gn = G N; C = inner + 2 gn
     float *ov, *ok, *oq, *oc, *ow;  // fp32 [T, inner], [T, gn] (B), [T, gn] (C), [T, H] (dt), [T, H] (decay)
-    int step;                  // one token per sequence whose slots are brought up to date on the way (the vector form alone)
 };
 
 template <typename A>
@@ -262,8 +261,9 @@ __global__ __launch_bounds__(256) void ssd_conv_prep_kernel(SsdPrepArgs p) {
 }
 
 // The same with eight consecutive channels per lane and 16-byte accesses (TAPS known at compile time; channel counts of x, B, C
-// multiples of 8, rows 16-byte aligned): a tap is one load of the inputs and one of the weights instead of eight of each.
-template <typename A, int TAPS>
+// multiples of 8, rows 16-byte aligned): a tap is one load of the inputs and one of the weights instead of eight of each.  STEP: one token per sequence,
+// whose slots are brought up to date on the way (a kernel of its own: what it keeps cost steps of many tokens a tenth, 2000 of 1024 + 2 x 128 channels fp32 16.6 -> 18.1 us).
+template <typename A, int TAPS, bool STEP>
 __global__ __launch_bounds__(256) void ssd_conv_prep_vec_kernel(SsdPrepArgs p) {
     const int64_t t = blockIdx.x;
     const int seq = seq_of_token(p.cu_seqlens_q, p.batch, t);
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(256) void ssd_conv_prep_vec_kernel(SsdPrepArgs p) {
     const int C = p.inner + 2 * p.gn;
     const float* st = carried ? p.conv_state + (int64_t)slot * (TAPS - 1) * C : nullptr;
     for (int c = (blockIdx.y * 256 + threadIdx.x) * 8; c < C; c += 256 * 8 * gridDim.y) {
-        float keep[TAPS - 1][8];                             // step: what the slot holds next, this lane's channels being nobody else's
+        float keep[STEP ? TAPS - 1 : 1][8];                  // what the slot holds next, this lane's channels being nobody else's
         float acc[8], wf[8 * TAPS];                          // wf[i * TAPS + k]: channel c + i, tap k (as the weights lie)
         if (p.conv_b) {
             nvh_load8((const A*)p.conv_b, c, 8, true, acc);
@@ -304,10 +304,10 @@ __global__ __launch_bounds__(256) void ssd_conv_prep_vec_kernel(SsdPrepArgs p) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 acc[i] = __builtin_fmaf(wf[i * TAPS + k], in[i], acc[i]);
-                if (k > 0) keep[k - 1][i] = in[i];
+                if (STEP && k > 0) keep[k - 1][i] = in[i];
             }
         }
-        if (p.step && slot >= 0) {                           // (uniform)
+        if (STEP && slot >= 0) {                             // (uniform)
             float* out = p.conv_state + (int64_t)slot * (TAPS - 1) * C + c;
 #pragma unroll
             for (int k = 0; k < TAPS - 1; ++k) {
@@ -1269,7 +1269,7 @@ static int32_t ssd_args(SsdPrepArgs& p, const void* xbc, int64_t xbc_stride, con
     NVH_REQUIRE(xbc && conv_w && slots && context_lens && (taps == 1 || conv_state), NVH_EINVAL, "ssd convolution: null pointer");
     NVH_REQUIRE(batch >= 0 && taps >= 1 && taps <= 64 && heads > 0 && inner > 0 && gn > 0 && xbc_stride >= inner + 2 * gn, NVH_EINVAL, "ssd convolution: bad sizes");
     p = SsdPrepArgs{xbc, xbc_stride, dt, dt_stride, conv_w, conv_b, dt_bias, a_log, conv_state, slots, cu_seqlens_q, context_lens,
-                    (int)batch, (int)taps, (int)heads, (int)inner, (int)gn, nullptr, nullptr, nullptr, nullptr, nullptr, 0};
+                    (int)batch, (int)taps, (int)heads, (int)inner, (int)gn, nullptr, nullptr, nullptr, nullptr, nullptr};
     return NVH_OK;
 }
 
@@ -1291,11 +1291,11 @@ static int32_t ssd_conv_prep(const void* xbc, int64_t xbc_stride, const void* dt
                      (!conv_b || nvh_aligned16(conv_b)) && nvh_aligned16(conv_state) && nvh_aligned16(out_x) && nvh_aligned16(out_b) && nvh_aligned16(out_c);
     const int64_t lanes = vec ? (inner + 2 * gn) / 8 : inner + 2 * gn;
     const dim3 grid((unsigned)num_tokens, (unsigned)(num_tokens >= 512 ? 1 : std::min<int64_t>(nvh_cdiv(lanes, 256), 16)));
-    p.step = step;
     if (vec) {
-#define NVH_CONV_VEC(TAPS)                                                        \
-    if (act_f32) ssd_conv_prep_vec_kernel<float, TAPS><<<grid, 256, 0, st>>>(p); \
-    else ssd_conv_prep_vec_kernel<bf16, TAPS><<<grid, 256, 0, st>>>(p)
+        auto launch = [&](auto step_kernel, auto kernel) { (step ? step_kernel : kernel)<<<grid, 256, 0, st>>>(p); };
+#define NVH_CONV_VEC(TAPS)                                                                                                          \
+    if (act_f32) launch(&ssd_conv_prep_vec_kernel<float, TAPS, true>, &ssd_conv_prep_vec_kernel<float, TAPS, false>); \
+    else launch(&ssd_conv_prep_vec_kernel<bf16, TAPS, true>, &ssd_conv_prep_vec_kernel<bf16, TAPS, false>)
         if (taps == 2) { NVH_CONV_VEC(2); }
         else if (taps == 3) { NVH_CONV_VEC(3); }
         else { NVH_CONV_VEC(4); }
