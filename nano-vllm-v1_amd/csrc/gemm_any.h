@@ -312,7 +312,22 @@ __device__ __forceinline__ void gemm_any_f32_tile_body(const float* __restrict__
             const int f = i * MR + j;
             if (f % 4 != wave) continue;
             const f32x4 sum = (lds[f * 64 + lane] + lds[(F + f) * 64 + lane]) + (lds[(2 * F + f) * 64 + lane] + lds[(3 * F + f) * 64 + lane]);
-            f32_finish(sum, bias, y, ldy, rm, r0 + 16 * j + fr, n0 + 16 * i + 4 * fq, N, gate, ldg, relu2);
+            // (f32_finish, written out: through the function the compiler asks about the gate lane by lane, 16 x 192 x 128 a head 3.9 us instead of 3.7)
+            const int r = r0 + 16 * j + fr;
+            if (r >= rm.rows) continue;
+            const int64_t m = rm.dst(r);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int n = n0 + 16 * i + 4 * fq + e;
+                if (n >= N) continue;
+                float v = sum[e] + (bias ? bias[n] : 0.f);
+                if (gate) v *= sigmoid(gate[m * ldg + n]);
+                if (relu2) {
+                    v = fmaxf(v, 0.f);
+                    v *= v;
+                }
+                y[m * ldy + n] = v;
+            }
         }
 }
 
