@@ -792,6 +792,7 @@ __global__ __launch_bounds__(256) void gemm_heads_short_bf16_kernel(GroupedArgs 
 // columns, two workgroups a CU, 49 rows and more in two halves.  Bit for bit the results of the form below.
 // us, the form below, by 32 and by 64 columns, rows an expert x N x K over 16 experts: 8 x 576 x 1024 19.2, 14.5, 13.8; 38 x 576 x 1024 31.8, 27.8, 21.0;
 // 38 x 1536 x 1024 58.6, 48.1, 40.8; 125 x 1536 x 1024 126, 102, 91; 19 x 576 x 1024 (64 experts) 53.7, 43.0, 45.9; 2.5 x 1536 x 1024 25.9, 22.0, 25.6.
+// By 32 columns, a grid of at most 256 workgroups has two of them share a tile's rows: one of 128 rows x 1024 x 384 7.4 (the form below), 9.2, so 6.9.
 template <int NC>
 __global__ __launch_bounds__(256, NC == 2 ? 2 : 1) void gemm_grouped_f32_ring_kernel(GroupedArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -801,7 +802,15 @@ __global__ __launch_bounds__(256, NC == 2 ? 2 : 1) void gemm_grouped_f32_ring_ke
     const nvh_any::RowMap rm{a.gather, a.tile_row0[blockIdx.y], rows};
     const int n0 = blockIdx.x * 16 * NC;
 #define NVH_RING(MR, STAGES, R0) nvh_any::gemm_any_f32_ring<MR, NC, STAGES>(x, a.ldx, w, a.K, nullptr, (float*)a.y, a.ldy, rm, R0, n0, a.N, a.K, nullptr, 0, a.relu2, smem)
-    if (rows <= 16) {
+    if (NC == 2 && gridDim.z == 2) {                         // (uniform) a half of the tile each
+        const int r0 = blockIdx.z * 32;
+        if (rows <= r0) return;
+        if (rows - r0 <= 16) {
+            NVH_RING(1, 3, r0);
+        } else {
+            NVH_RING(2, 2, r0);
+        }
+    } else if (rows <= 16) {
         NVH_RING(1, 3, 0);
     } else if (NC == 4 && rows <= 32) {
         NVH_RING(2, 3, 0);
@@ -823,7 +832,8 @@ bool launch_grouped_f32(const GroupedArgs& a, int64_t max_tiles, hipStream_t st)
     static_assert(lds <= (NC == 4 ? 160 : 80) * 1024);
     static std::atomic<uint64_t> granted{0};
     if (!nvh_grant_lds(granted, reinterpret_cast<const void*>(&gemm_grouped_f32_ring_kernel<NC>), lds)) return false;
-    gemm_grouped_f32_ring_kernel<NC><<<dim3((unsigned)nvh_cdiv(a.N, 16 * NC), (unsigned)max_tiles), 256, lds, st>>>(a);
+    const int64_t grid = nvh_cdiv(a.N, 16 * NC) * max_tiles;
+    gemm_grouped_f32_ring_kernel<NC><<<dim3((unsigned)nvh_cdiv(a.N, 16 * NC), (unsigned)max_tiles, NC == 2 && grid <= 256 ? 2 : 1), 256, lds, st>>>(a);
     return true;
 }
 

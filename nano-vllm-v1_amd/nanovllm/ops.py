@@ -1294,8 +1294,19 @@ def moe_align(ids: torch.Tensor, experts: int) -> dict:
     return dict(src_token=src, pos_of_pair=pos, tile_expert=te, tile_row0=t0, tile_rows=tr, max_tiles=max_tiles, pairs=pairs)
 
 
-GROUPED_MANY_ROWS = 192     # rows per expert, on average, from which the grouped product takes its tall tiles; fp32: its wide ones
+# The grouped product's tall tiles (128 x 128; fp32: its wide ones, 64 x 64) pay from this many rows per expert on, on average, and only where there are enough
+# of them: us, tiles for few rows and these, bf16 16 experts of 250 rows x 1536 x 1024 (384 tiles) 38.4 and 35.1, 8 of 250 x 768 x 1024 (96) 16.4 and 20.9, one
+# of 192 x 4096 x 2048 (64) 13.8 and 33.0; fp32 16 of 48 x 576 x 1024 (144) 29.4 and 25.7, one of 512 x 1024 x 384 (128) 9.9 and 13.1, but 8
+# of 256 x 256 x 1024 (128, all of them full) 33.4 and 24.6.  (0 rows: always.)
+GROUPED_MANY_ROWS = 192
 GROUPED_MANY_ROWS_F32 = 32
+GROUPED_MANY_TILES = 144
+
+
+def _grouped_many(pairs: int, experts: int, n: int, f32) -> bool:
+    rows, tile = (GROUPED_MANY_ROWS_F32, 64) if f32 else (GROUPED_MANY_ROWS, 128)
+    tiles = experts * -(-pairs // (experts * tile)) * -(-n // tile)
+    return rows == 0 or (pairs >= rows * experts and (tiles >= GROUPED_MANY_TILES or (f32 and experts > 1 and pairs * n >= 128 * tile * tile)))
 
 
 def linear_grouped(x: torch.Tensor, weight: torch.Tensor, plan: dict, gather: bool, out_f32: bool = False, act: str | None = None) -> torch.Tensor:
@@ -1307,7 +1318,7 @@ def linear_grouped(x: torch.Tensor, weight: torch.Tensor, plan: dict, gather: bo
     assert weight.is_contiguous() and x.dim() == 2 and x.shape[1] == k and x.stride(1) == 1 and (gather or x.shape[0] == plan["pairs"])
     out_f32 = bool(out_f32 or f)
     y = torch.empty(plan["pairs"], n, dtype=F32 if out_f32 else BF16, device=x.device)
-    many = plan["pairs"] >= (GROUPED_MANY_ROWS_F32 if f else GROUPED_MANY_ROWS) * e
+    many = _grouped_many(plan["pairs"], e, n, f)
     _hip.call("nvh_gemm_grouped_many_nt" if many else "nvh_gemm_grouped_any_nt", x.data_ptr(), x.stride(0), plan["src_token"].data_ptr() if gather else 0, weight.data_ptr(), y.data_ptr(), n,
               plan["tile_expert"].data_ptr(), plan["tile_row0"].data_ptr(), plan["tile_rows"].data_ptr(), plan["max_tiles"], n, k, int(act == "relu2"), f,
               int(out_f32), _stream())
@@ -1340,7 +1351,7 @@ def linear_grouped_gated(x: torch.Tensor, weight: torch.Tensor, plan: dict, act:
     _hip.call("nvh_gemm_grouped_gated_nt", x.data_ptr(), x.stride(0), plan["src_token"].data_ptr(), weight.data_ptr(), y.data_ptr(), n // 2,
               plan["tile_expert"].data_ptr(), plan["tile_row0"].data_ptr(), plan["tile_rows"].data_ptr(), plan["max_tiles"], n // 2, k,
               3 if act == "glu_clamp" else ACTS[act], plan["pos_of_pair"].data_ptr(), _p(weights), weights.shape[1] if weights is not None else 1,
-              float(limit), float(alpha), int(plan["pairs"] >= GROUPED_MANY_ROWS * e), _stream())
+              float(limit), float(alpha), int(_grouped_many(plan["pairs"], e, n, False)), _stream())
     return y
 
 

@@ -53,3 +53,22 @@ def test_grouped(n, k, relu2):
     want = ops.linear_grouped(odd_rows(x), w, plan, True, act=act)[at]
     assert torch.equal(ops.linear_grouped(x, w, plan, True, act=act)[at], want)
     assert torch.equal(ops.linear_grouped(x[plan["src_token"].long()], w, plan, False, act=act)[at], want)
+
+
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("sizes", [[0, 1, 16, 17, 32, 33, 48, 49, 64, 65, 130], [128], [33, 0, 64], [700, 20]])
+@pytest.mark.parametrize("n,k", [(4, 32), (40, 96), (200, 1024), (1030, 64)])
+def test_grouped_forms(sizes, n, k, many, monkeypatch):
+    """Tiles by 64 columns, by 32, and by 32 with a tile's rows in two workgroups (small grids)."""
+    from nanovllm import ops
+    monkeypatch.setattr(ops, "GROUPED_MANY_ROWS_F32", 0 if many else 1 << 30)
+    g = torch.Generator().manual_seed(n + k)
+    ids = torch.repeat_interleave(torch.arange(len(sizes)), torch.tensor(sizes))[torch.randperm(sum(sizes), generator=g)].int()[:, None].cuda()
+    x, w = torch.randn(ids.shape[0], k, generator=g).cuda(), torch.randn(len(sizes), n, k, generator=g).cuda()
+    plan = ops.moe_align(ids, len(sizes))
+    at = plan["pos_of_pair"].long()
+    want = ops.linear_grouped(odd_rows(x), w, plan, True)[at]
+    assert torch.equal(ops.linear_grouped(x, w, plan, True)[at], want)
+    exact = torch.einsum("tk,tnk->tn", x.double().cpu(), w.double().cpu()[ids[:, 0].long().cpu()])
+    size = torch.einsum("tk,tnk->tn", x.double().abs().cpu(), w.double().abs().cpu()[ids[:, 0].long().cpu()])
+    assert ((want.double().cpu() - exact).abs() <= size * (k + 4) * 2.0 ** -24).all()
