@@ -876,22 +876,37 @@ enum AttnVariant { VAR_PLAIN, VAR_EXT, VAR_BIAS };
 // One query per sequence: which sequence and group of heads a workgroup takes.  All workgroups of a step fit the chip a few to a CU, the ones numbered
 // L and L + 256 beside each other, and as they lie that gives a CU the same long sequence twice.  So the work is dealt out by length: the
 // longest sequences to the first 256 workgroups, the next ones to the next 256 in the opposite order, and so on.  Every workgroup ranks the
-// sequences (at most 256) for itself; a result does not depend on where it is computed.
+// sequences for itself; a result does not depend on where it is computed.
 // us, as they lay and dealt out, 64 sequences of 512 .. 1535 keys, 8 KV heads: 128 x 128 51.2 and 46.3 in one model, 75.3 and 67.7 in another, with a
 // query temperature or pooled blocks 54.5 and 49.2; 128 x 64 58.0 and 52.2; 64 x 128 72.8 and 69.7.
-constexpr int BALANCE_MAX = 256;
-__device__ __forceinline__ void balanced_place(const AttnArgs& a, int* keys, int& seq, int& by) {
-    const int tid = threadIdx.x, total = gridDim.x * gridDim.y, L = blockIdx.x + gridDim.x * blockIdx.y;
+// The ranking costs each workgroup 0.7 us and more as the batch grows, and gives nothing where the sequences are short or alike (dealt out by as they
+// lay, means over five forms of heads: 5 .. 60 keys 1.12 at 64 sequences, 1.24 at 100, 1.48 at 200; 300 keys each 1.05, 1.11, 1.21; 20 .. 275
+// keys 0.97, 1.06, 1.23).  So there are at most 128 sequences, and the longest has to see 512 keys and a quarter more than the shortest (to find out
+// that it does not costs 0.2 us: 6.4 us for 5 .. 60 keys were 6.2).
+constexpr int BALANCE_MAX = 128, BALANCE_KEYS = 512;
+__device__ __forceinline__ int balance_keys(const AttnArgs& a, int b) {      // keys that the sequence's query sees (roughly: what counts is the order)
+    if (b >= a.batch) return -1;
+    int len = a.context_lens[b];
+    if (a.chunk > 0) len = len > 0 ? (len - 1) % a.chunk + 1 : 0;
+    if (a.window > 0) len = min(len, a.window + a.keep_first);
+    return len;
+}
+__device__ __forceinline__ int wave_max_of(int v) {                          // (0 .. 2^23: exact as floats, and in their order as integers)
+    const int m = __float_as_int(row16_max((float)v));
+    return (int)__int_as_float(max(max(__builtin_amdgcn_readlane(m, 0), __builtin_amdgcn_readlane(m, 16)), max(__builtin_amdgcn_readlane(m, 32), __builtin_amdgcn_readlane(m, 48))));
+}
+__device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int& seq, int& by) {
+    const int tid = threadIdx.x, lane = tid & 63, total = gridDim.x * gridDim.y, L = blockIdx.x + gridDim.x * blockIdx.y;
+    const int len0 = balance_keys(a, lane), len1 = balance_keys(a, lane + 64);
+    if (!__any(max(len0, len1) > BALANCE_KEYS)) return false;     // (every wave holds the same lengths: uniform, also over the workgroup)
+    const int longest = wave_max_of(max(max(len0, len1), 0));
+    const int spread = wave_max_of(max(len0 < 0 ? 0 : max(longest - len0, 0), len1 < 0 ? 0 : max(longest - len1, 0)));
+    if (4 * spread < longest) return false;
     const int round = L >> 8, in_round = min(256, total - 256 * round), at = L & 255;
     const int item = 256 * round + (round & 1 ? in_round - 1 - at : at), want = item / (int)gridDim.y;
-    int len = 0;                                             // keys that the sequence's query sees (roughly: what counts is the order)
-    if (tid < a.batch) {
-        len = a.context_lens[tid];
-        if (a.chunk > 0) len = len > 0 ? (len - 1) % a.chunk + 1 : 0;
-        if (a.window > 0) len = min(len, a.window + a.keep_first);
-    }
+    const int len = tid < 64 ? len0 : len1;
     const int key = tid < a.batch ? (len << 8 | (255 - tid)) : -1;
-    keys[tid] = key;
+    if (tid < BALANCE_MAX) keys[tid] = key;
     __syncthreads();
     int rank = 0;
     for (int j = 0; j < a.batch; j += 4) {                   // (four at a time: behind the batch lie the -1 of the lanes without a sequence)
@@ -904,6 +919,7 @@ __device__ __forceinline__ void balanced_place(const AttnArgs& a, int* keys, int
     seq = __builtin_amdgcn_readfirstlane(keys[0]);
     by = item - want * (int)gridDim.y;
     __syncthreads();                                         // (the place is used for other things from here on)
+    return true;
 }
 
 // (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
@@ -916,8 +932,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     constexpr int ROWS_Q = MQ;                               // queries per workgroup
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     int seq = -1, q0 = 0, qlen = 0, qbase = 0, by = blockIdx.y;
-    if (GROUPED && a.balance) {                              // (uniform)
-        balanced_place(a, reinterpret_cast<int*>(smem_raw), seq, by);
+    if (GROUPED && a.balance && balanced_place(a, reinterpret_cast<int*>(smem_raw), seq, by)) {      // (uniform)
         qbase = seq;
         qlen = 1;
     } else if (!a.cu_seqlens_q) {                            // one query per sequence
@@ -1432,8 +1447,12 @@ static void launch_attn_mfma(const AttnArgs& a, int64_t total_q, hipStream_t st)
     if (grouped) {
         b.kv_split = pl.split;
         b.key_parts = pl.key_parts;
-        // (one workgroup a CU or less: nothing to pair; lengths of 2^23 and more do not fit the keys)
-        b.balance = pl.key_parts == 1 && a.batch <= BALANCE_MAX && (int64_t)a.batch * a.G * pl.split > 256 && a.table_stride * a.page < (1 << 23);
+        // (one workgroup a CU or less: nothing to pair; lengths of 2^23 and more do not fit the keys; a query that cannot see many keys: balanced_place)
+        int64_t most = (int64_t)a.table_stride * a.page;
+        b.balance = pl.key_parts == 1 && a.batch <= BALANCE_MAX && (int64_t)a.batch * a.G * pl.split > 256 && most < (1 << 23);
+        if (a.chunk > 0) most = std::min(most, (int64_t)a.chunk);
+        if (a.window > 0) most = std::min(most, (int64_t)a.window + a.keep_first);
+        if (most <= BALANCE_KEYS) b.balance = 0;
         attn_paged_mfma_kernel<NKS, NVT, EXACT, 1, VAR><<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)pl.key_parts), 256, lds, st>>>(b);
         if (pl.key_parts > 1)
             attn_merge_parts_kernel<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)(group / pl.split)), 256, 0, st>>>(a.parts, pl.key_parts, group / pl.split, a.vdim, a.H, a.gate,

@@ -69,6 +69,32 @@ def test_a_step_of_many_sequences(B, window, keep, chunk):
             assert (got[b] == 0).all()
 
 
+@pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (700, 5, 0), (0, 0, 640)])
+@pytest.mark.parametrize("lens", ["longer", "at the line", "alike", "one long"])
+@pytest.mark.parametrize("B", [33, 64, 65, 128, 129])
+def test_dealt_out_or_not(B, lens, window, keep, chunk):
+    """Either side of the lines between which the sequences of a step are dealt out: their number, the longest one and how far they differ."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(B + window + chunk)
+    H, G, dim, vdim = 8, 8, 64, 64
+    lo, hi = {"longer": (1, 1200), "at the line": (300, 512), "alike": (460, 600), "one long": (1, 40)}[lens]
+    ctx = torch.randint(lo, hi + 1, (B,), generator=g).tolist()
+    ctx[5], ctx[B - 1] = {"longer": (0, 1281), "at the line": (513 if B & 1 else 512, 1), "alike": (600, 450 if B & 1 else 451), "one long": (0, 1100)}[lens]
+    k, v, table = caches(g, ctx, G, dim, vdim)
+    q = torch.randn(B, H * dim, generator=g).bfloat16().cuda()
+    k, v, table, dev = k.cuda(), v.cuda(), table.cuda(), torch.tensor(ctx).int().cuda()
+    kw = dict(window=window, keep_first=keep, chunk=chunk)
+    got = ops.attn_paged_any(q, k, v, None, dev, table, dim ** -0.5, H, G, dim, vdim, **kw)
+    for at in range(0, B, 30):                               # (too few workgroups to be dealt out, too many for key parts)
+        n = slice(min(at, B - 30), min(at, B - 30) + 30)
+        assert torch.equal(ops.attn_paged_any(q[n].contiguous(), k, v, None, dev[n].contiguous(), table[n].contiguous(), dim ** -0.5, H, G, dim, vdim, **kw), got[n])
+    for b in (0, 5, B - 1):
+        if ctx[b]:
+            assert close_to(got[b:b + 1], reference(q[b:b + 1].cpu(), k.cpu(), v.cpu(), table[b].cpu(), ctx[b], ctx[b] - 1, H, G, dim, vdim, window, keep, chunk, None))
+        else:
+            assert (got[b] == 0).all()
+
+
 @pytest.mark.parametrize("H,G,dim,vdim", [(2, 1, 128, 128), (2, 2, 64, 128), (1, 1, 256, 192), (2, 2, 48, 80)])
 @pytest.mark.parametrize("window,keep,chunk,sink", [(0, 0, 0, False), (100, 0, 0, True), (200, 70, 0, False), (0, 0, 192, True)])
 def test_tiles_seen_whole(H, G, dim, vdim, window, keep, chunk, sink):
