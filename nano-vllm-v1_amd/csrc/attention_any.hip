@@ -924,7 +924,13 @@ __device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int
 
 // (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
 constexpr int attn_waves(int nks, int nvt, int mode, int var) { return nks + nvt <= 4 ? 4 : nks + nvt <= (mode == 1 && nvt <= 4 && var != VAR_EXT ? 12 : 8) ? 3 : nks + nvt <= 16 ? 2 : 1; }
-template <int NKS, int NVT, bool EXACT, int MODE, int VAR>
+// Wide heads leave one wave per SIMD and use its whole register file: there a second form of the loop's arithmetic costs more in registers than the
+// masking that it leaves out, but for prompts without a window, chunk or slope, of which most tiles are seen whole.  FORMS: whether there are two.
+// us, one form and two: 192 x 192, one query over each of 200 sequences, softcap 1.00 and 1.22 of one form's time; 160 x 128 in the bounded kernel, 64
+// queries 0.99 and 1.11; 192 x 128, windows of 128 keys 0.99 and 1.06; whole prompts 256 x 256 0.99 and 0.92, 192 x 192 1.00 and 0.97, 128 x 256 0.99
+// and 0.96 (all of the time that the masked form took before there were two).
+constexpr bool attn_wide(int nks, int nvt) { return nks + nvt > 16; }
+template <int NKS, int NVT, bool EXACT, int MODE, int VAR, bool FORMS>
 __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_paged_mfma_kernel(AttnArgs a) {
     constexpr bool GROUPED = MODE == 1;                      // rows are the heads of a KV group (one query per sequence)
     constexpr bool EXT = VAR == VAR_EXT, BIAS = VAR == VAR_BIAS;
@@ -1134,7 +1140,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                 if constexpr (!WHOLE) {
                     const bool seen = POOLED ? key < my_blocks : (key <= qpos) & ((key >= lo_window) | (key < a.keep_first)) & (key >= lo_chunk);
                     if (!BIAS && !POOLED) v = __builtin_fmaf(-slope, (float)(qpos - key), v);
-                    v = qok & seen ? v : -INFINITY;
+                    v = (qok & seen) ? v : -INFINITY;
                 }
                 sc[t][r] = v;
                 mx = fmaxf(mx, sc[t][r]);
@@ -1155,7 +1161,8 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         for (int t = 0; t < NKT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float pv = __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * 1.4426950408889634f);
+                // (wide heads: the same value, but without the test the loop is laid out so that it takes up to a tenth longer)
+                const float pv = attn_wide(NKS, NVT) && !WHOLE && sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * 1.4426950408889634f);
                 sum += pv;
                 const bf16 hi = (bf16)pv;
                 const bf16 lo = (bf16)(pv - (float)hi);
@@ -1206,7 +1213,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         }
         __syncthreads();
         fetch(k_after, kpre, vpre);
-        if (k0 >= whole_from && k0 <= whole_to) compute(std::false_type{}, std::true_type{}, k0);
+        if (FORMS && k0 >= whole_from && k0 <= whole_to) compute(std::false_type{}, std::true_type{}, k0);
         else compute(std::false_type{}, std::false_type{}, k0);
     };
     // Two register sets, two tiles ahead: the loads of the tile after next are issued when a tile has been handed to LDS.
@@ -1440,10 +1447,12 @@ static void launch_attn_mfma(const AttnArgs& a, int64_t total_q, hipStream_t st)
     }
     const bool grouped = total_q == a.batch && group / pl.split <= 16 && bias_group_bytes <= BIAS_LDS && !nvh_switch_on(SW_EXP_A);
     const size_t lds = b.bias_offset + (grouped ? bias_group_bytes : bias_bytes);
-    if (lds > 64 * 1024) {                                   // (wide heads or long page tables; a refusal shows as a failed launch)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_paged_mfma_kernel<NKS, NVT, EXACT, 0, VAR>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_paged_mfma_kernel<NKS, NVT, EXACT, 1, VAR>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    }
+    constexpr bool WIDE = attn_wide(NKS, NVT);
+    const auto one_query = &attn_paged_mfma_kernel<NKS, NVT, EXACT, 1, VAR, !WIDE>, prompt = &attn_paged_mfma_kernel<NKS, NVT, EXACT, 0, VAR, !WIDE>;
+    const auto prompt_two = &attn_paged_mfma_kernel<NKS, NVT, EXACT, 0, VAR, !WIDE || (EXACT && VAR == VAR_PLAIN)>;
+    const bool two_forms = !a.window && !a.chunk && !a.slopes;
+    if (lds > 64 * 1024)                                     // (wide heads or long page tables; a refusal shows as a failed launch)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(grouped ? one_query : two_forms ? prompt_two : prompt), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (grouped) {
         b.kv_split = pl.split;
         b.key_parts = pl.key_parts;
@@ -1453,13 +1462,13 @@ static void launch_attn_mfma(const AttnArgs& a, int64_t total_q, hipStream_t st)
         if (a.chunk > 0) most = std::min(most, (int64_t)a.chunk);
         if (a.window > 0) most = std::min(most, (int64_t)a.window + a.keep_first);
         if (most <= BALANCE_KEYS) b.balance = 0;
-        attn_paged_mfma_kernel<NKS, NVT, EXACT, 1, VAR><<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)pl.key_parts), 256, lds, st>>>(b);
+        one_query<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)pl.key_parts), 256, lds, st>>>(b);
         if (pl.key_parts > 1)
             attn_merge_parts_kernel<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)(group / pl.split)), 256, 0, st>>>(a.parts, pl.key_parts, group / pl.split, a.vdim, a.H, a.gate,
                                                                                                         (const bf16*)a.gate_elems, a.ld_elems, (bf16*)a.out);
     } else {
         const dim3 grid((unsigned)(total_q / MQ + a.batch), (unsigned)a.H);
-        attn_paged_mfma_kernel<NKS, NVT, EXACT, 0, VAR><<<grid, 256, lds, st>>>(b);
+        (two_forms ? prompt_two : prompt)<<<grid, 256, lds, st>>>(b);
     }
 }
 

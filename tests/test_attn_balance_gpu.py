@@ -120,3 +120,21 @@ def test_tiles_seen_whole(H, G, dim, vdim, window, keep, chunk, sink):
             if cut < n - 1:                                  # (one query left would be a step of another form)
                 assert torch.equal(run(q[lo + cut:lo + n], [n - cut], [n], tab[b:b + 1]), got[lo + cut:lo + n]), (b, cut)
         lo += n
+
+
+@pytest.mark.parametrize("H,G,dim,vdim", [(2, 1, 128, 128), (4, 2, 64, 64), (1, 1, 128, 256), (2, 1, 192, 128), (1, 1, 192, 192), (2, 1, 256, 192), (1, 1, 256, 256), (2, 1, 160, 128)])
+def test_windows_that_reach_everything(H, G, dim, vdim):
+    """A window, or a chunk, of more than the context leaves out nothing: the bits of the call without one, whichever form of the loop either takes."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(dim + vdim)
+    for lens, ctx in ([1, 63, 64, 65, 130, 450], [1, 63, 64, 65, 130, 450]), ([40, 1, 129], [333, 700, 257]), ([1] * 40, list(range(1, 800, 20))):
+        k, v, table = caches(g, ctx, G, dim, vdim)
+        q = torch.randn(sum(lens), H * dim, generator=g).bfloat16()
+        cu = torch.tensor([0] + lens).cumsum(0).int()
+        args = (k.cuda(), v.cuda(), None if max(lens) == 1 else cu.cuda(), torch.tensor(ctx).int().cuda(), table.cuda(), dim ** -0.5, H, G, dim, vdim)
+        got = ops.attn_paged_any(q.cuda(), *args)
+        for kw in dict(window=5000), dict(chunk=8192), dict(slopes=torch.zeros(H).cuda()):
+            assert torch.equal(ops.attn_paged_any(q.cuda(), *args, **kw), got), kw
+        for b in range(0, len(ctx), 3):
+            lo, n = int(cu[b]), lens[b]
+            assert close_to(got[lo:lo + n], reference(q[lo:lo + n], k, v, table[b], ctx[b], ctx[b] - n, H, G, dim, vdim, 0, 0, 0, None)), (lens, b)
