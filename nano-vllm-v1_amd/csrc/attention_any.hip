@@ -395,7 +395,7 @@ struct AttnArgs {
     int kv_split;              // one-query form: workgroups per (sequence, KV head), each with H / (G kv_split) of the group's heads
     int key_parts;             // one-query form: workgroups that share a sequence's key tiles (tile j goes to part j % key_parts); > 1: the
     float* parts;              // parts leave [batch, G kv_split, key_parts, 16, vdim + 2] (unnormalised rows, then max and sum) here
-    int balance;               // one-query form: sequences are dealt out by their length (balanced_place)
+    int balance;               // one-query form: sequences are dealt out by their length where one sees more keys than this (balanced_place; 0: never)
 };
 
 // The key tiles (of `tile` keys, starting at multiples of it) that a workgroup whose first query sits at position qlo has to
@@ -881,9 +881,10 @@ enum AttnVariant { VAR_PLAIN, VAR_EXT, VAR_BIAS };
 // query temperature or pooled blocks 54.5 and 49.2; 128 x 64 58.0 and 52.2; 64 x 128 72.8 and 69.7.
 // The ranking costs each workgroup 0.7 us and more as the batch grows, and gives nothing where the sequences are short or alike (dealt out by as they
 // lay, means over five forms of heads: 5 .. 60 keys 1.12 at 64 sequences, 1.24 at 100, 1.48 at 200; 300 keys each 1.05, 1.11, 1.21; 20 .. 275
-// keys 0.97, 1.06, 1.23).  So there are at most 128 sequences, and the longest has to see 512 keys and a quarter more than the shortest (to find out
-// that it does not costs 0.2 us: 6.4 us for 5 .. 60 keys were 6.2).
-constexpr int BALANCE_MAX = 128, BALANCE_KEYS = 512;
+// keys 0.97, 1.06, 1.23).  So there are at most 128 sequences, and the longest has to see a quarter more keys than the shortest and more than 192 of them,
+// beyond 64 sequences more than 512 (a.balance; to find out that it does not costs 0.2 us: 6.4 us for 5 .. 60 keys were 6.2).
+constexpr int BALANCE_MAX = 128;
+constexpr int balance_from(int batch) { return batch <= 64 ? 192 : 512; }
 __device__ __forceinline__ int balance_keys(const AttnArgs& a, int b) {      // keys that the sequence's query sees (roughly: what counts is the order)
     if (b >= a.batch) return -1;
     int len = a.context_lens[b];
@@ -898,7 +899,7 @@ __device__ __forceinline__ int wave_max_of(int v) {                          // 
 __device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int& seq, int& by) {
     const int tid = threadIdx.x, lane = tid & 63, total = gridDim.x * gridDim.y, L = blockIdx.x + gridDim.x * blockIdx.y;
     const int len0 = balance_keys(a, lane), len1 = balance_keys(a, lane + 64);
-    if (!__any(max(len0, len1) > BALANCE_KEYS)) return false;     // (every wave holds the same lengths: uniform, also over the workgroup)
+    if (!__any(max(len0, len1) > a.balance)) return false;     // (every wave holds the same lengths: uniform, also over the workgroup)
     const int longest = wave_max_of(max(max(len0, len1), 0));
     const int spread = wave_max_of(max(len0 < 0 ? 0 : max(longest - len0, 0), len1 < 0 ? 0 : max(longest - len1, 0)));
     if (4 * spread < longest) return false;
@@ -1458,10 +1459,10 @@ static void launch_attn_mfma(const AttnArgs& a, int64_t total_q, hipStream_t st)
         b.key_parts = pl.key_parts;
         // (one workgroup a CU or less: nothing to pair; lengths of 2^23 and more do not fit the keys; a query that cannot see many keys: balanced_place)
         int64_t most = (int64_t)a.table_stride * a.page;
-        b.balance = pl.key_parts == 1 && a.batch <= BALANCE_MAX && (int64_t)a.batch * a.G * pl.split > 256 && most < (1 << 23);
+        b.balance = pl.key_parts == 1 && a.batch <= BALANCE_MAX && (int64_t)a.batch * a.G * pl.split > 256 && most < (1 << 23) ? balance_from(a.batch) : 0;
         if (a.chunk > 0) most = std::min(most, (int64_t)a.chunk);
         if (a.window > 0) most = std::min(most, (int64_t)a.window + a.keep_first);
-        if (most <= BALANCE_KEYS) b.balance = 0;
+        if (most <= b.balance) b.balance = 0;
         one_query<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)pl.key_parts), 256, lds, st>>>(b);
         if (pl.key_parts > 1)
             attn_merge_parts_kernel<<<dim3((unsigned)a.batch, (unsigned)(a.G * pl.split), (unsigned)(group / pl.split)), 256, 0, st>>>(a.parts, pl.key_parts, group / pl.split, a.vdim, a.H, a.gate,

@@ -70,16 +70,16 @@ def test_a_step_of_many_sequences(B, window, keep, chunk):
 
 
 @pytest.mark.parametrize("window,keep,chunk", [(0, 0, 0), (700, 5, 0), (0, 0, 640)])
-@pytest.mark.parametrize("lens", ["longer", "at the line", "alike", "one long"])
+@pytest.mark.parametrize("lens", ["longer", "at the line", "alike", "one long", "short"])
 @pytest.mark.parametrize("B", [33, 64, 65, 128, 129])
 def test_dealt_out_or_not(B, lens, window, keep, chunk):
     """Either side of the lines between which the sequences of a step are dealt out: their number, the longest one and how far they differ."""
     from nanovllm import ops
     g = torch.Generator().manual_seed(B + window + chunk)
     H, G, dim, vdim = 8, 8, 64, 64
-    lo, hi = {"longer": (1, 1200), "at the line": (300, 512), "alike": (460, 600), "one long": (1, 40)}[lens]
+    lo, hi = {"longer": (1, 1200), "at the line": (300, 512), "alike": (460, 600), "one long": (1, 40), "short": (1, 192)}[lens]
     ctx = torch.randint(lo, hi + 1, (B,), generator=g).tolist()
-    ctx[5], ctx[B - 1] = {"longer": (0, 1281), "at the line": (513 if B & 1 else 512, 1), "alike": (600, 450 if B & 1 else 451), "one long": (0, 1100)}[lens]
+    ctx[5], ctx[B - 1] = {"longer": (0, 1281), "at the line": (513 if B & 1 else 512, 1), "alike": (600, 450 if B & 1 else 451), "one long": (0, 1100), "short": (193 if B & 1 else 192, 0)}[lens]
     k, v, table = caches(g, ctx, G, dim, vdim)
     q = torch.randn(B, H * dim, generator=g).bfloat16().cuda()
     k, v, table, dev = k.cuda(), v.cuda(), table.cuda(), torch.tensor(ctx).int().cuda()
