@@ -1301,6 +1301,9 @@ int tile_residents(Tile t) {
 // (k-tiles per slab + fixed part) x tile bytes x residents / fill rate, and a grid takes a whole number of rounds:
 // 320 workgroups on 256 slots cost two rounds.  Slabs add their write and the consumer's read.  It ranks the
 // measured split counts of the 14B projections at 256..1024 rows in the measured order.
+// It prices the tiles that pick_tile names, also where an unsplit product is launched with others (T64x64 and T128x64 in the launch below): with
+// those tiles' sizes in the model products of 33 .. 64 rows and K up to 1024 gain 5 .. 15 % (unsplit), but 300 .. 1000 rows lose 4 .. 32 %
+// (600 x 4096 x 5120 with its norm 43.5 -> 57.4 us): the model has no term for what eight waves on one tile hide.
 double splitk_estimate_us(int64_t M, int64_t N, int64_t K, int s) {
     const Tile t = pick_tile(M, N, s);
     const int64_t wgs = nvh_cdiv(M, tile_bm(t)) * nvh_cdiv(N, tile_bn(t)) * s;
@@ -1485,7 +1488,8 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
         case T64x64: {
             // 33 .. 64 rows: 64-column tiles leave most CUs without one, and what a workgroup waits for is its stages; 16 columns (32 where 16 would be
             // more than a workgroup a CU) with six stages.  64 rows x N x 1024, us before and now: 1024 7.7 and 6.5, 2048 7.9 and 6.7, 4096 8.0 and 7.1,
-            // 6144 8.3 and 7.7, 8192 8.6 and 8.4.  The same sums in the same order.
+            // 6144 8.3 and 7.7, 8192 8.5 and 7.5; other K: 64 x 4096 x 25600 127 and 100, 64 x 5120 x 17408 88.3 and 76.1 (142 sizes, K 128 .. 25600, N 128 ..
+            // 8192, 33 .. 64 rows: none slower).  The same sums in the same order.
             if (!tile_forced() && a.M <= 64 && a.split_k == 1 && !a.swiglu && !a.qkv && !a.sample && a.N <= 32 * 256) {
                 if (a.N <= 16 * 256) launch_gemm<64, 16, 1, 4, 6>(a);
                 else launch_gemm<64, 32, 2, 2, 6>(a);
@@ -1500,7 +1504,9 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
         case T128x64:
             // One workgroup fits a CU, so a grid a little over 256 takes two rounds: then 128 x 128 tiles, fewer than 200 of them, in one round, eight
             // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 14.9, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
-            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4; one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  The same sums.
+            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4; one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  Two rounds elsewhere:
+            // 128 x 18992 x 5120 84.5 and 62.9, 1500 x 2048 x 17408 215 and 155, 1024 x 2560 x 5120 69 and 52, gate/up 512 x 6144 x 1024 19.9 and 15.4 (237
+            // sizes, 65 .. 4000 rows, N 560 .. 24000, K 256 .. 17408: 0.70 .. 0.82 of the time).  The same sums.
             if (!tile_forced() && a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
             else launch_gemm<128, 64, 2, 2, 4>(a);
             break;

@@ -336,7 +336,8 @@ __device__ __forceinline__ void gemm_any_f32_tile_body(const float* __restrict__
 // the operands' way to the CUs, which a 64 x 64 tile has half as much of as four 32 x 32 ones.  Chunks, products and sums as above: bit for bit the
 // same results.
 // us, the form above and this, rows x columns x k: 1 x 1024 x 1024 5.9 and 4.7, 64 x 1024 x 1024 11.6 and 5.2, 64 x 4096 x 1024 13.0 and 9.6,
-// 301 x 1024 x 1024 21.2 and 13.9, 301 x 6144 x 1024 74 and 48 (79 TFLOP/s of the 124 that independent products reach), 512 x 6144 x 1024 111 and 70.
+// 301 x 1024 x 1024 21.2 and 13.9, 301 x 6144 x 1024 74 and 48 (79 TFLOP/s of the 124 that independent products reach), 512 x 6144 x 1024 112 and 67,
+// 1 x 32000 x 1024 32.1 and 27.5, 1 x 12288 x 5120 49.5 and 46.0.
 template <int MR, int NC, int STAGES>
 constexpr int f32_ring_bytes() {
     return 4 * STAGES * 16 * (MR + NC) * 128;                // (at least the four waves' partial tiles, 1 KB a fragment: STAGES 2 (MR + NC) >= MR NC)
