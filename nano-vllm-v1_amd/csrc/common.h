@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <atomic>
+#include <utility>
 #include <stdint.h>
 #include <stdio.h>
 #include "../../include/nanovllm_hip.h"
@@ -100,6 +101,12 @@ static inline bool nvh_aligned16(const void* p) { return (reinterpret_cast<uintp
 static inline int64_t nvh_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---- device side ------------------------------------------------------------------
+// f(0), f(1), .. f(N - 1) with constants: a loop whose body chooses by its index, written out whatever its length.
+template <int... I, typename F>
+__device__ __forceinline__ void nvh_static_for_of(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void nvh_static_for(F&& f) { nvh_static_for_of(std::make_integer_sequence<int, N>{}, f); }
+
 // Sum / max over the 16 lanes of a DPP row (lanes 16r..16r+15); every lane of the row
 // receives the result.  quad_perm[1,0,3,2], quad_perm[2,3,0,1], row_half_mirror, row_mirror.
 #define NVH_DPP(x, ctrl) \

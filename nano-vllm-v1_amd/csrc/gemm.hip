@@ -83,11 +83,10 @@ struct RowScale {
     float inv_k, eps;
 };
 
-// Tile of this workgroup.  Workgroups go to the 8 XCDs round-robin by linear id.  With xcd_strip = 8 or 4 (host: gridDim.x a
-// multiple of it) XCD i takes the i-th eighth of the tiles in an order that walks strips of that many column tiles row
-// by row, so the workgroups resident on an XCD at one time share a few column tiles of W and a few row tiles of x in
-// its L2 (Qwen3-14B shapes, 1024 rows: a prefill chunk 27.8 -> 27.15 ms; K = 1024: 2.81 -> 2.78 ms).  K-slabs (gridDim.z)
-// count as further tile rows: slab z of row tile y is row y + gridDim.y * z.
+// Tile of this workgroup.  Workgroups go to the 8 XCDs round-robin by linear id.  With xcd_strip = 8 or 4 XCD i takes the i-th eighth of the tiles in an
+// order that walks strips of that many column tiles (the last one may be narrower) row by row, so the workgroups resident on an XCD at one time share
+// a few column tiles of W and a few row tiles of x in its L2 (Qwen3-14B shapes, 1024 rows: a prefill chunk 27.8 -> 27.15 ms; K = 1024: 2.81 -> 2.78 ms).
+// K-slabs (gridDim.z) count as further tile rows: slab z of row tile y is row y + gridDim.y * z.
 __device__ __forceinline__ void xcd_tile(int xcd_strip, int& bx, int& by, int& bz) {
     bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     if (xcd_strip) {
@@ -95,11 +94,20 @@ __device__ __forceinline__ void xcd_tile(int xcd_strip, int& bx, int& by, int& b
         const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), total = gridDim.x * rows;
         const int xcd = id & 7, nl = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);
         const int sh = xcd_strip == 8 ? 3 : 2, per_strip = rows << sh;
-        const int strip = nl / per_strip, in = nl - strip * per_strip, row = in >> sh;
-        bx = (strip << sh) + (in & (xcd_strip - 1));
+        const int strip = nl / per_strip, in = nl - strip * per_strip, width = min(xcd_strip, (int)gridDim.x - (strip << sh));
+        const int row = width == xcd_strip ? in >> sh : in / width;
+        bx = (strip << sh) + in - row * width;
         bz = row / (int)gridDim.y;
         by = row - bz * (int)gridDim.y;
     }
+}
+// Strips for a grid: from 512 rows on (at 256 rows, a decode batch of 64-row tiles, the same order made a step 0.7 % slower); with a narrower last strip
+// where the grid is at most one workgroup a CU (800 x 5120 x 5120, 27 x 7 tiles: no strips and these 58.4 and 56.6 us; two rounds, 2000 x 5248 x 1024: 35.1 and 36.8).
+static int xcd_strip_of(const dim3& grid, int rows) {
+    if (nvh_switch_on(SW_GEMM_NO_XCD) || grid.y * grid.z == 1 || rows < 512) return 0;             // (the switch is for measurements)
+    if (grid.x % 8 == 0) return 8;
+    if (grid.x % 4 == 0) return 4;
+    return (int64_t)grid.x * grid.y * grid.z <= 256 ? 8 : 0;
 }
 
 template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES, bool NT_W, bool SWIGLU, bool QKV = false, bool SAMPLE = false, bool ROWSCALE = false>
@@ -254,7 +262,81 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
             }
         }
     };
-    if constexpr (NW == 8) {
+    if constexpr (NW == 8 && STAGES > 2) {
+        // Eight waves, two per SIMD, ONE barrier a k-tile, in its middle, and everything else spread between the products: a wave multiplies the first
+        // half of tile t (fragments already in registers) while it reads the second half, meets the barrier, then multiplies the second half while it
+        // reads tile t+1's first.  By the barrier every wave's reads of tile t have returned, so its stage is free for tile t+STAGES, and every wave's
+        // pieces of tile t+1 have landed.  A DMA instruction holds up the wave that issues it while the address unit is busy with others (16 cycles
+        // each), so they go out one by one, half of a tile's behind the barrier and half before the next one.
+        // us with weights from HBM, four barriers a tile (read / multiply in turn) and now, 128 x 128 tiles: 1024 x 4096 x 1024 15.5 and 14.3, 1024 x 3072 x
+        // 1024 15.0 and 13.2, 700 x 4096 x 1024 14.9 and 12.8; 128 x 192: 1024 x 6144 x 1024 19.8 (128 x 128, two workgroups a CU) and 17.9.
+        bf16x8 af[2][TN], bfr[2][TM];
+        constexpr int NF = TN + TM, NM = TN * TM;
+        constexpr int FIRST = PW / 2;                        // pieces of a tile that go out behind the barrier
+        auto stage_piece = [&](int t, auto I) {                  // one instruction of stage(t)
+            constexpr int i = decltype(I)::value;
+            const bf16* src = src_row[i] + kbeg + t * BK;
+            char* dst = smem + (t % STAGES) * STAGE_BYTES + lds_off[i];
+            if (NT_W && piece_is_w[i]) __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)src, (LDS_AS void*)dst, 16, 0, 2);
+            else __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)src, (LDS_AS void*)dst, 16, 0, 0);
+        };
+        auto read_frag = [&](int half, const char* a_base, auto G) {
+            constexpr int g = decltype(G)::value;
+            const int kc = half * 4 + fq;
+            if constexpr (g < TM) {
+                const int r = wm * WM + g * 16 + fr;
+                bfr[half][g] = *reinterpret_cast<const bf16x8*>(a_base + A_BYTES + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+            } else {
+                const int r = wn * WN + (g - TM) * 16 + fr;
+                af[half][g - TM] = *reinterpret_cast<const bf16x8*>(a_base + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+            }
+        };
+        // the products of half `half`, with the fragment reads over their first three quarters and nd pieces of DMA over all of them
+        auto half_tile = [&](auto HALF, const char* read_base, auto ND, auto FROM, int dma_tile) {
+            constexpr int half = decltype(HALF)::value, nd = decltype(ND)::value;
+            nvh_static_for<NM>([&](auto MI) {
+                constexpr int m = decltype(MI)::value;
+                nvh_static_for<nd>([&](auto D) {
+                    if constexpr (decltype(D)::value * NM / (nd > 0 ? nd : 1) == m) stage_piece(dma_tile, std::integral_constant<int, decltype(FROM)::value + decltype(D)::value>{});
+                });
+                nvh_static_for<NF>([&](auto G) {
+                    if constexpr (decltype(G)::value * NM * 3 / 4 / NF == m) read_frag(1 - half, read_base, G);
+                });
+                if constexpr (m % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+                acc[m / TM][m % TM] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[half][m / TM], bfr[half][m % TM], acc[m / TM][m % TM], 0, 0, 0);
+            });
+        };
+        constexpr std::integral_constant<int, 0> H0{};
+        constexpr std::integral_constant<int, 1> H1{};
+        // tile t: the other pieces of tile t - 1 + STAGES go out before the barrier, FIRST ones of tile t + STAGES behind it
+        auto tile = [&](int t, auto BEFORE, auto BEHIND) {
+            constexpr bool before = decltype(BEFORE)::value, behind = decltype(BEHIND)::value;
+            half_tile(H0, smem + (t % STAGES) * STAGE_BYTES, std::integral_constant<int, before ? PW - FIRST : 0>{}, std::integral_constant<int, FIRST>{}, t - 1 + STAGES);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                   // this tile's reads
+            if constexpr (before) wait_vmcnt<(STAGES - 2) * PW>();        // own pieces of tile t+1
+            else wait_tiles_in_flight<PW, STAGES - 2>(max(0, min(STAGES - 2, ntiles - 2 - t)));
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            half_tile(H1, smem + ((t + 1) % STAGES) * STAGE_BYTES, std::integral_constant<int, behind ? FIRST : 0>{}, H0, t + STAGES);
+        };
+        for (int t = 0; t < STAGES && t < ntiles; ++t) stage(t);
+        request_cs();                                            // younger than the stages: the counted waits below only get stricter while these are in flight
+        wait_tiles_in_flight<PW, STAGES - 1>(min(STAGES, ntiles) - 1);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        nvh_static_for<NF>([&](auto G) { read_frag(0, smem, G); });
+        // (past the last tile the reads take what lies in its neighbour's stage: nobody multiplies it)
+        int t = 0;
+        if (STAGES < ntiles) {
+            tile(t++, std::false_type{}, std::true_type{});
+            for (; t + STAGES < ntiles; ++t) tile(t, std::true_type{}, std::true_type{});
+            tile(t++, std::true_type{}, std::false_type{});
+        }
+        for (; t < ntiles; ++t) tile(t, std::false_type{}, std::false_type{});
+    } else if constexpr (NW == 8) {
         // Eight waves, two per SIMD.  Every wave runs the same four phases per k-tile, a barrier before each:
         //   READ k0 (12 fragment reads) | MFMA k0 (32) | READ k1 | MFMA k1
         // and waves 4-7 run ONE barrier behind waves 0-3 (an extra barrier before their loop, one after the others'),
@@ -264,9 +346,8 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
         //    passes its 1st barrier of tile t+1 (the same barrier for the second half) every piece has landed;
         //  * the DMA of tile t+1 (two LDS stages: the buffer of tile t-1) is issued after the 1st barrier of tile t;
         //    the last readers of tile t-1 are the second half's READ k1, drained (lgkmcnt) before that very barrier.
-        // With more than two stages the DMA runs STAGES - 1 tiles ahead and the wait before the fourth barrier leaves
-        // the tiles behind t+1 in flight (measured with 128 x 128 tiles and three stages: 13.8 us against 15.1 us for
-        // 1024 x 4096 x 1024, slower on every grid that is not exactly one workgroup per CU; not dispatched).
+        // (The form above with two stages: 1016 x 34816 x 5120 2 %, 1500 x 12288 x 3072 6 % slower: its DMA has half a tile's time to land, this one's three
+        // quarters.  128 x 128 tiles here, three stages, 1024 x 4096 x 1024: 15.5 us against 14.3 us there.)
         const bool second_half = wave >= 4;              // wave-uniform
         bf16x8 af[TN], bfr[TM];
         auto read_frags = [&](const char* a_base, int ks) {
@@ -355,8 +436,8 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
     // epilogue: lane holds n = n_base + fq*4 .. +3 of row m = m_base + fr
     if constexpr (SAMPLE) {
         static_assert((NW == 8 || NW == 4) && WAVES_N == 2 && !SWIGLU && !QKV, "sampling epilogue: two column halves per workgroup");
-        // the stages are free: in the eight-wave loop every read of them was waited for before its last barrier; the
-        // four-wave loop ends without one
+        // the stages are free: in the eight-wave loop every read whose value is used was waited for before its last barrier;
+        // the four-wave loop ends without one
         if constexpr (NW != 8) __syncthreads();
         ValIdx (*sm_cand)[TM][16] = reinterpret_cast<ValIdx (*)[TM][16]>(smem);
         ValIdx best[TM];
@@ -498,11 +579,11 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
         }
         return;
     }
-    if constexpr (BN == 128 && NW == 4 && BM >= 64) {
-        // full 128-column tiles with a bf16 result: through LDS, so every lane stores 16 contiguous bytes and a row
-        // of the tile leaves as one 256-B line (the fragment layout would store 8 B per lane, 32 B per row piece)
+    if constexpr ((BN == 128 || BN == 192) && (NW == 4 || NW == 8) && BM >= 64) {
+        // full column tiles with a bf16 result: through LDS, so every lane stores 16 contiguous bytes and a row
+        // of the tile leaves as whole lines (the fragment layout would store 8 B per lane, 32 B per row piece)
         if (partials == nullptr && n0 + BN <= N && wide_store) {                 // block-uniform
-            constexpr int TS = 136;
+            constexpr int TS = BN + 8, CPR = BN / 8;
             __syncthreads();                                     // every wave is done with the last stage
             bf16* tile = reinterpret_cast<bf16*>(smem);
 #pragma unroll
@@ -523,10 +604,9 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
                 }
             }
             __syncthreads();
-            const int c = tid & 15, rr = tid >> 4;
 #pragma unroll
-            for (int p = 0; p < BM / 16; ++p) {
-                const int row = p * 16 + rr, m = m0 + row;
+            for (int p = 0; p < BM * CPR / (NW * 64); ++p) {
+                const int at = p * NW * 64 + tid, row = at / CPR, c = at % CPR, m = m0 + row;
                 if (m < M) *reinterpret_cast<bf16x8*>(y + (int64_t)m * y_stride + n0 + c * 8) = *reinterpret_cast<const bf16x8*>(tile + row * TS + c * 8);
             }
             return;
@@ -1190,14 +1270,11 @@ void launch_gemm_nt(const GemmArgs& a) {
     const int ktiles = a.K / BK;
     const bool no_wide = nvh_switch_on(SW_GEMM_NO_WIDE_STORE);   // A/B switch for measurements
     // wide stores need 16-byte aligned output rows and the staging tile inside the kernel's LDS
-    const bool wide = !no_wide && a.ys % 8 == 0 && nvh_aligned16(a.y) && smem >= BM * 136 * 2;
+    const bool wide = !no_wide && a.ys % 8 == 0 && nvh_aligned16(a.y) && smem >= BM * (BN + 8) * 2;
     const int k_per_split = (int)nvh_cdiv(ktiles, a.split_k) * BK;
     dim3 grid((unsigned)nvh_cdiv(a.N, BN), (unsigned)nvh_cdiv(a.M, BM), (unsigned)a.split_k);
-    const bool no_xcd = nvh_switch_on(SW_GEMM_NO_XCD);            // A/B switch for measurements
-    // prefill-sized products only: at 256 rows (a decode batch, 64-row tiles) the same order made a step 0.7 % slower
-    const int xcd_strip = (no_xcd || grid.y * grid.z == 1 || a.M < 512) ? 0 : grid.x % 8 == 0 ? 8 : grid.x % 4 == 0 ? 4 : 0;
     kern<<<grid, 64 * WAVES_N * WAVES_M, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.partials, a.M, a.N, a.K, k_per_split,
-                                                       a.qkv ? *a.qkv : QkvEpilogue{}, wide, a.sample ? *a.sample : SampleEpilogue{}, xcd_strip, a.rowscale);
+                                                       a.qkv ? *a.qkv : QkvEpilogue{}, wide, a.sample ? *a.sample : SampleEpilogue{}, xcd_strip_of(grid, a.M), a.rowscale);
 }
 
 void launch_gemm_kgroups(const GemmArgs& a) {
@@ -1214,9 +1291,7 @@ void launch_gemm_kgroups(const GemmArgs& a) {
         return;
     }
     dim3 grid((unsigned)nvh_cdiv(a.N, 64), (unsigned)nvh_cdiv(a.M, 64), 1);
-    const bool no_xcd = nvh_switch_on(SW_GEMM_NO_XCD);
-    const int xcd_strip = (no_xcd || grid.y == 1 || a.M < 512) ? 0 : grid.x % 8 == 0 ? 8 : grid.x % 4 == 0 ? 4 : 0;   // as launch_gemm_nt
-    kern<<<grid, 512, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.M, a.N, a.K, xcd_strip, a.residual, a.row_sumsq);
+    kern<<<grid, 512, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.M, a.N, a.K, xcd_strip_of(grid, a.M), a.residual, a.row_sumsq);
 }
 
 template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES>
@@ -1503,22 +1578,29 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
         }
         case T128x64:
             // One workgroup fits a CU, so a grid a little over 256 takes two rounds: then 128 x 128 tiles, fewer than 200 of them, in one round, eight
-            // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 14.9, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
-            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4; one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  Two rounds elsewhere:
+            // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 11.7, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
+            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4 (those but the first with four barriers a k-tile); one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  Two rounds elsewhere:
             // 128 x 18992 x 5120 84.5 and 62.9, 1500 x 2048 x 17408 215 and 155, 1024 x 2560 x 5120 69 and 52, gate/up 512 x 6144 x 1024 19.9 and 15.4 (237
             // sizes, 65 .. 4000 rows, N 560 .. 24000, K 256 .. 17408: 0.70 .. 0.82 of the time).  The same sums.
             if (!tile_forced() && a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
             else launch_gemm<128, 64, 2, 2, 4>(a);
             break;
         case T128x128: {
-            // up to one workgroup per CU: nothing shares the CU's LDS, so a third stage (96 KB) keeps two tiles in
-            // flight instead of one (1024 x 4096 x 1024: 19.1 -> 17.2 us); larger grids want two residents of 64 KB
-            // a nearly full round of one workgroup per CU over a short K (the QKV projection of a prefill chunk, epilogue
-            // included): eight waves (two per SIMD, one barrier apart; the QKV epilogue walks 32 rows per pass).  1024 / 896 x
-            // 4096 x 1024: 16.1 / 15.1 -> 14.9 / 14.4 us, a 1024-token chunk 2.89 -> 2.81 ms; K = 2048: 25.5 -> 26.2 us (not taken)
-            const int64_t tiles128 = nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 128) * a.split_k;
-            if (!a.swiglu && !nvh_switch_on(SW_QKV_NO_8WAVE) && tiles128 >= 200 && tiles128 <= 256 && a.K / a.split_k <= 1536) launch_gemm<128, 128, 2, 4, 3>(a);
-            else if (nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 128) * a.split_k <= 256) launch_gemm<128, 128, 2, 2, 3>(a);
+            // up to one workgroup per CU: nothing shares the CU's LDS, so a third stage (96 KB) keeps two tiles in flight instead of one, and eight waves
+            // instead of four, two a SIMD, multiply and read at once (us, four waves and eight: 1024 x 4096 x 2048 27.0 and 23.5, x 4096 46.2 and 40.6;
+            // with the QKV epilogue, which walks 32 rows a pass, 1024 x 4096 x 1024 16.1 and 14.9 when each phase still had a barrier)
+            const int64_t tm = nvh_cdiv(a.M, 128), tiles128 = tm * nvh_cdiv(a.N, 128) * a.split_k;
+            if (tiles128 <= 256) {
+                const bool scaled_long = a.rowscale.sumsq != nullptr && a.K / a.split_k > 1536;     // (row scales over more than one norm's width: refused)
+                if (!a.swiglu && !scaled_long && !nvh_switch_on(SW_QKV_NO_8WAVE)) launch_gemm<128, 128, 2, 4, 3>(a);
+                else launch_gemm<128, 128, 2, 2, 3>(a);
+            }
+            // a little more than a round of them: wider or taller tiles, one a CU, that make it one round (us, 128 x 128, two workgroups a CU, and this:
+            // 128 x 192 1024 x 6144 x 1024 19.8 and 17.9, 1024 x 5248 x 1024 20.7 and 17.8; 256 x 128 1016 x 7168 x 5120 86.2 and 78.8, 1024 x 8192 x 1024
+            // 21.5 and 21.1, but 1000 x 8192 x 512 13.9 and 14.3)
+            else if (!tile_forced() && !a.swiglu && !a.qkv && !a.sample && a.split_k == 1 && tm * nvh_cdiv(a.N, 192) <= 256) launch_gemm<128, 192, 2, 4, 3>(a);
+            else if (!tile_forced() && !a.swiglu && !a.qkv && !a.sample && a.split_k == 1 && a.K >= 1024 && nvh_cdiv(a.M, 256) * nvh_cdiv(a.N, 128) <= 256)
+                launch_gemm<256, 128, 2, 4, 3>(a);
             // gate/up + SwiGLU over a grid whose last round of 128 x 128 tiles is half empty (1024 x 6144: 384 tiles = 1.5
             // rounds of 256 CUs): 128 x 96 tiles make whole rounds (512).  Taken when rounds x tile area, the narrower tile
             // priced 5 % dearer per column, comes out lower: a 1024-token chunk 2.80 -> 2.77 ms.  (128 x 64 tiles, 768 = three
@@ -1534,7 +1616,7 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
             else launch_gemm<128, 128, 2, 2, 2>(a);
             break;
         }
-        case T256x128: launch_gemm<256, 128, 2, 2, 3>(a); break;
+        case T256x128: launch_gemm<256, 128, 2, 4, 3>(a); break;
         case T256x256: launch_gemm<256, 256, 2, 4, 2>(a); break;
     }
     if (!a.plan) NVH_CHECK_LAUNCH("gemm_bf16_nt");
