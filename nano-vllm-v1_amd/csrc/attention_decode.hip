@@ -92,32 +92,68 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     const int start = split * chunk;
     const int end = min(ctx, start + chunk);
 
-    bf16x8 qv[G];
+    // Everything that this token brings is requested before the first keys are, and worked on behind that request.
+    bf16x8 qv[G], qw, kw, k_new, v_new;
+    f32x4 cs[4];
+    const bool has_new = FUSED && start < end && end == ctx;      // (uniform) this range ends with the step's own token
     if (start < end) {
 #pragma unroll
         for (int g = 0; g < G; ++g)
             qv[g] = *reinterpret_cast<const bf16x8*>(q + (int64_t)b * q_stride + (int64_t)(kvh * G + g) * 128 + c * 8);
         if constexpr (FUSED) {
-            const float* cs_row = fz.cos_sin + fz.positions[b] * 128;
-            const bf16x8 qw = *reinterpret_cast<const bf16x8*>(fz.q_norm_w + c * 8);
+            const bf16* row = q + (int64_t)b * q_stride;
+            qw = *reinterpret_cast<const bf16x8*>(fz.q_norm_w + c * 8);
+            kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
+            k_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8);
+            v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
+            const float* cs_row = fz.cos_sin + fz.positions[b] * 128 + 8 * (c & 7);
 #pragma unroll
-            for (int g = 0; g < G; ++g) qv[g] = qknorm_rope_head(qv[g], qw, cs_row, c, fz.eps);
-            if (end == ctx) {                                // (uniform)
-                // the new token's keys and values go to the cache first; its lanes load them from there, in order behind their own stores (others may
-                // see what was there before: settle)
-                const bf16x8 kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
-                const bf16* row = q + (int64_t)b * q_stride;
-                const bf16x8 k_new = qknorm_rope_head(*reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8), kw, cs_row, c, fz.eps);
-                const bf16x8 v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
+            for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4*>(cs_row + (i >> 1) * 64 + (i & 1) * 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // From four query heads a kv head on the scores come from the matrix cores (16x16x32: 16 keys by up to four heads, four instructions) instead of a dot
+    // product and a row sum a key and head: a trip's vector instructions halve.  us a launch, 8 kv heads, before and now: 4 heads each, 30 sequences of
+    // 64..2000 keys 45.6 and 36.2; 5 heads, 8 of 3000..4000 98 and 74; 8 heads, 20 of 64..2000 84 and 54.  With 1 and 2 heads long contexts are bound by
+    // the keys' way to the CU either way (24 of 100..2047 30.9 and 31.2) and many workgroups lose by the registers (256 sequences 208 and 224).
+    constexpr bool MFMA = G >= 4;
+    constexpr int SETS = MFMA ? (G + 3) / 4 : 1;
+    // A wave's own copies in LDS, rows of 256 bytes: the queries (for the matrix cores: row 16 h + i of their operand is query head 4 h + (i & 3), so that every
+    // four lanes' results are the scores of four heads for one key), then the new token's keys and values.
+    __shared__ __attribute__((aligned(16))) bf16 sm_q[MFMA ? 4 : 1][MFMA ? G + (FUSED ? 2 : 0) : 2][128];
+    bf16x8 qa[SETS][4];
+    const int fr = lane & 15, fq = lane >> 4;
+    auto prepare = [&]() {
+        if constexpr (FUSED) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) qv[g] = qknorm_rope_head_cs(qv[g], qw, cs[0], cs[1], cs[2], cs[3], c, fz.eps);
+            if (has_new) {
+                k_new = qknorm_rope_head_cs(k_new, kw, cs[0], cs[1], cs[2], cs[3], c, fz.eps);
                 if (((ctx - 1) & 15) == rowid) {
                     const int64_t off = (((int64_t)tables[(int64_t)b * table_stride + ((ctx - 1) >> 8)] * NVH_KV_PAGE + ((ctx - 1) & 255)) * hkv + kvh) * 128 + c * 8;
                     *reinterpret_cast<bf16x8*>(kc + off) = k_new;
                     *reinterpret_cast<bf16x8*>(vc + off) = v_new;
                 }
+                if (MFMA && lane < 16) {
+                    *reinterpret_cast<bf16x8*>(&sm_q[w][G][c * 8]) = k_new;
+                    *reinterpret_cast<bf16x8*>(&sm_q[w][G + 1][c * 8]) = v_new;
+                }
             }
         }
-    }
+        if constexpr (MFMA) {
+            if (lane < 16) {
+#pragma unroll
+                for (int g = 0; g < G; ++g) *reinterpret_cast<bf16x8*>(&sm_q[w][g][c * 8]) = qv[g];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int h = 0; h < SETS; ++h)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) qa[h][i] = *reinterpret_cast<const bf16x8*>(&sm_q[w][min(4 * h + (fr & 3), G - 1)][(fq + 4 * i) * 8]);
+        }
+    };
 
+    // acc: this row's keys, columns 8 c .. + 7; m and l of the same keys (MFMA: m of the wave's, l of this lane's, key fr of every trip)
     float m[G], l[G], acc[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
@@ -131,12 +167,17 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     // the loads of the next; the page after the one at hand is looked up a trip ahead.  With one workgroup a CU a trip takes 1.0 us (one set,
     // every trip's loads waited for before its work: 1.6 us), about the 64 KB in flight over the memory's latency.  Every trip but the last is
     // worked on behind a request that is made in any case: behind a branch around it the waits would cover the new loads too (a launch of 24
-    // sequences of 100..2047 keys 39.1 us, as it is 31.7; 60 of 64..300 15.7 and 14.5; contexts of one trip 0.2 us longer, for the way past
-    // the loop).  Measured beside it, from 38.0 us: three and four sets 36.1 and 35.7 us, but 100 short sequences 8 and 25 % slower for the registers.
+    // sequences of 100..2047 keys 39.1 us, as it is 30.9; contexts of one trip 0.2 us longer, for the way past the loop).  More in flight gives nothing:
+    // four sets in registers, or four trips in an LDS ring, leave a trip at 1 us (what a CU can have outstanding).
     const int32_t* table = tables + (int64_t)b * table_stride;
     u32x4 ka[4], va[4], kb[4], vb[4];                        // (whole words: as 16-bit elements every one would take a register across the loop)
     const int last_page = (end - 1) >> 8;
     int page = start < end ? table[start >> 8] : 0;
+    // A wave's 16 keys of a trip: key i is token 16 (i >> 2) + 4 w + (i & 3).  Keys and values come a row a token (lane: token 16 u + rowid, 16-byte piece c:
+    // a row's lanes read 256 bytes side by side; with keys loaded as the matrix cores take them, 16 bytes of 16 rows side by side, 24 of 100..2047 took 36 us).
+    // MFMA: keys pass through the wave's own LDS (then lane: key fr, pieces fq + 4 i; piece p of key i lies at place p ^ i, so neither way meets a bank twice).
+    const int ktok = (fr >> 2) * 16 + w * 4 + (fr & 3);
+    __shared__ __attribute__((aligned(16))) char sm_k[MFMA ? 4 : 1][16 * 256];
     auto fetch = [&](int base, u32x4 (&kf)[4], u32x4 (&vf)[4]) {
         // (scalar base of the trip + a 32-bit lane offset: one register per address)
         const int64_t slot0 = (((int64_t)page * NVH_KV_PAGE + (base & 255)) * hkv + kvh) * 128;
@@ -151,48 +192,94 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         page = table[min((base + 64) >> 8, last_page)];
         __builtin_amdgcn_sched_barrier(0);
     };
-    // A last trip that the new token opens: lanes past the end have read its place, which another wave is writing, and a weight of 0 times what a reused
-    // page held there need not be 0.  They take no value at all.  (Any other trip has older keys in its first place.)
-    auto settle = [&](int base, u32x4 (&vf)[4]) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t keep = base + u * 16 + rowid < end ? 0xffffffffu : 0u;
-            vf[u] &= u32x4{keep, keep, keep, keep};
-        }
-    };
-    auto consume = [&](int base, const u32x4 (&kw)[4], const u32x4 (&vw)[4]) {
-        float s[G][4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int tok = base + u * 16 + rowid;
-            const bf16x8 kf = __builtin_bit_cast(bf16x8, kw[u]);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                float d = 0.f;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    bf16x2 a = {qv[g][2 * j], qv[g][2 * j + 1]};
-                    bf16x2 k2 = {kf[2 * j], kf[2 * j + 1]};
-                    d = __builtin_amdgcn_fdot2_f32_bf16(a, k2, d, false);
-                }
-                d = row16_sum(d) * scale_log2;
-                s[g][u] = tok < end ? d : -INFINITY;
-            }
-        }
-        float alpha[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) {                        // s becomes the weights
-            const float mn = fmaxf(fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3])), m[g]);
-            const float mu = (mn == -INFINITY) ? 0.f : mn;
-            alpha[g] = __builtin_amdgcn_exp2f(m[g] - mu);
-            float ps = 0.f;
+    // The trip that the new token is in.  Lanes past the end have read the trip's first place; if that is the new token's own, another wave is writing it, and
+    // a weight of 0 times what a reused page held there need not be 0: they take no value at all.  (Any other trip has older keys in its first place.)  The
+    // token's own keys and values: without MFMA its lanes have loaded them behind their own stores (a trip that holds them is requested after these);
+    // with it they come from the wave's copy.
+    auto settle = [&](int base, u32x4 (&kf)[4], u32x4 (&vf)[4]) {
+        if constexpr (FUSED) {
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                s[g][u] = __builtin_amdgcn_exp2f(s[g][u] - mu);
-                ps += s[g][u];
+                const int tok = base + u * 16 + rowid;
+                if constexpr (MFMA) {
+                    const u32x4 kn = *reinterpret_cast<const u32x4*>(&sm_q[w][G][c * 8]), vn = *reinterpret_cast<const u32x4*>(&sm_q[w][G + 1][c * 8]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        kf[u][e] = tok == ctx - 1 ? kn[e] : kf[u][e];
+                        vf[u][e] = tok < ctx - 1 ? vf[u][e] : tok == ctx - 1 ? vn[e] : 0u;
+                    }
+                } else {
+                    const uint32_t keep = tok < end ? 0xffffffffu : 0u;
+                    vf[u] &= u32x4{keep, keep, keep, keep};
+                }
             }
-            l[g] = l[g] * alpha[g] + ps;
-            m[g] = mn;
+        }
+    };
+    // where a row's weights of a trip are: its token u is key 4 u + row of the wave
+    const int from = fq * 4;
+    auto consume = [&](int base, const u32x4 (&kw)[4], const u32x4 (&vw)[4]) {
+        float s[G][4], alpha[G];
+        if constexpr (MFMA) {
+            u32x4 kt[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int key = 4 * u + fq;
+                *reinterpret_cast<u32x4*>(sm_k[w] + key * 256 + ((c ^ key) << 4)) = kw[u];
+            }
+            asm volatile("" ::: "memory");                       // (a wave's LDS accesses keep their order)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) kt[i] = *reinterpret_cast<const u32x4*>(sm_k[w] + fr * 256 + (((fq + 4 * i) ^ fr) << 4));
+            f32x4 d[SETS];
+#pragma unroll
+            for (int h = 0; h < SETS; ++h) {
+                d[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[h][i], __builtin_bit_cast(bf16x8, kt[i]), d[h], 0, 0, 0);
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float x = base + ktok < end ? d[g >> 2][g & 3] * scale_log2 : -INFINITY;
+                const float mn = fmaxf(row16_max(x), m[g]);
+                const float mu = (mn == -INFINITY) ? 0.f : mn;
+                alpha[g] = __builtin_amdgcn_exp2f(m[g] - mu);
+                const float p = __builtin_amdgcn_exp2f(x - mu);
+                l[g] = l[g] * alpha[g] + p;
+                m[g] = mn;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s[g][u] = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from + 16 * u, __builtin_bit_cast(int, p)));
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int tok = base + u * 16 + rowid;
+                const bf16x8 kf = __builtin_bit_cast(bf16x8, kw[u]);
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    float d = 0.f;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        bf16x2 a = {qv[g][2 * j], qv[g][2 * j + 1]};
+                        bf16x2 k2 = {kf[2 * j], kf[2 * j + 1]};
+                        d = __builtin_amdgcn_fdot2_f32_bf16(a, k2, d, false);
+                    }
+                    d = row16_sum(d) * scale_log2;
+                    s[g][u] = tok < end ? d : -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {                        // s becomes the weights
+                const float mn = fmaxf(fmaxf(fmaxf(s[g][0], s[g][1]), fmaxf(s[g][2], s[g][3])), m[g]);
+                const float mu = (mn == -INFINITY) ? 0.f : mn;
+                alpha[g] = __builtin_amdgcn_exp2f(m[g] - mu);
+                float ps = 0.f;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    s[g][u] = __builtin_amdgcn_exp2f(s[g][u] - mu);
+                    ps += s[g][u];
+                }
+                l[g] = l[g] * alpha[g] + ps;
+                m[g] = mn;
+            }
         }
         // (column by column, so that only four widened values are alive at a time)
 #pragma unroll
@@ -204,7 +291,10 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
             for (int g = 0; g < G; ++g) {
                 float a = acc[g][j] * alpha[g];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) a += s[g][u] * v[u];
+                for (int u = 0; u < 4; ++u) {
+                    if constexpr (MFMA) a = __builtin_fmaf(s[g][u], v[u], a);
+                    else a += s[g][u] * v[u];
+                }
                 acc[g][j] = a;
             }
         }
@@ -214,10 +304,15 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         int base = start;
         if (((end - start - 1) >> 6) & 1) {                  // an even number of trips
             fetch(base, kb, vb);
+            prepare();
             fetch(base + 64, ka, va);
             consume(base, kb, vb);
             base += 64;
+        } else if (MFMA || !has_new || base + 64 < end) {    // (uniform) the first trip waits for no store
+            fetch(base, ka, va);
+            prepare();
         } else {
+            prepare();
             fetch(base, ka, va);
         }
         for (; base + 64 < end; base += 128) {
@@ -226,26 +321,39 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
             fetch(base + 128, ka, va);
             consume(base + 64, kb, vb);
         }
-        if (FUSED && base == ctx - 1) settle(base, va);
+        if (MFMA ? has_new : base == ctx - 1) settle(base, ka, va);
         consume(base, ka, va);
     }
 
-    // merge the 4 rows of the wave (lanes l, l^16, l^32 hold the same output columns)
-#pragma unroll
-    for (int step = 16; step <= 32; step <<= 1) {
+    if constexpr (MFMA) {
+        // the wave's rows hold the same columns of different keys, all by the same maximum
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const float mo = __shfl_xor(m[g], step, 64);
-            const float lo = __shfl_xor(l[g], step, 64);
-            const float mn = fmaxf(m[g], mo);
-            const float mu = (mn == -INFINITY) ? 0.f : mn;
-            const float a = __builtin_amdgcn_exp2f(m[g] - mu), bsc = __builtin_amdgcn_exp2f(mo - mu);
-            l[g] = l[g] * a + lo * bsc;
-            m[g] = mn;
+            l[g] = row16_sum(l[g]);
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const float ao = __shfl_xor(acc[g][j], step, 64);
-                acc[g][j] = acc[g][j] * a + ao * bsc;
+                acc[g][j] += __shfl_xor(acc[g][j], 16, 64);
+                acc[g][j] += __shfl_xor(acc[g][j], 32, 64);
+            }
+        }
+    } else {
+        // merge the 4 rows of the wave (lanes l, l^16, l^32 hold the same output columns)
+#pragma unroll
+        for (int step = 16; step <= 32; step <<= 1) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const float mo = __shfl_xor(m[g], step, 64);
+                const float lo = __shfl_xor(l[g], step, 64);
+                const float mn = fmaxf(m[g], mo);
+                const float mu = (mn == -INFINITY) ? 0.f : mn;
+                const float a = __builtin_amdgcn_exp2f(m[g] - mu), bsc = __builtin_amdgcn_exp2f(mo - mu);
+                l[g] = l[g] * a + lo * bsc;
+                m[g] = mn;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float ao = __shfl_xor(acc[g][j], step, 64);
+                    acc[g][j] = acc[g][j] * a + ao * bsc;
+                }
             }
         }
     }

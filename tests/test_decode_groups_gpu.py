@@ -1,0 +1,57 @@
+"""Decode attention with 1 .. 8 query heads a kv head: trips that the new token opens, ends or lies inside, ranges, pages that hold no numbers behind a
+context's end; against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CTX = [1, 2, 15, 16, 17, 63, 64, 65, 66, 127, 128, 129, 192, 193, 255, 256, 257, 320, 321, 700]
+
+
+def rope_head(x, w, cs, eps):
+    """The q/k epilogue at its rounding points: norm -> bf16, times weight -> bf16, rotated halves -> bf16."""
+    n = (x.float() / torch.sqrt((x.float() ** 2).mean(-1, keepdim=True) + eps)).bfloat16().float()
+    n = (n * w.float()).bfloat16().float()
+    cos, sin = cs[..., :64], cs[..., 64:]
+    a, b = n[..., :64], n[..., 64:]
+    return torch.cat([a * cos - b * sin, b * cos + a * sin], -1).bfloat16()
+
+
+@pytest.mark.parametrize("splits", [1, 5])
+@pytest.mark.parametrize("group", [1, 2, 4, 5, 8])
+def test_new_token_and_edges(group, splits):
+    from nanovllm import ops
+    hkv, hq, eps = 2, 2 * group, 1e-6
+    g = torch.Generator().manual_seed(group * 10 + splits)
+    b, width = len(CTX), 3
+    tables = torch.randperm(b * width, generator=g).int().view(b, width)
+    kc, vc = (torch.randn(b * width, 256, hkv, 128, generator=g).bfloat16() for _ in range(2))
+    for i, n in enumerate(CTX):                              # what a page held before is no number at all, from the new token's own place on
+        for page in range(width):
+            first = max(0, n - 1 - 256 * page)
+            kc[tables[i, page].long(), first:] = vc[tables[i, page].long(), first:] = float("nan")
+    qkv = torch.randn(b, (hq + 2 * hkv) * 128, generator=g).bfloat16()
+    qw, kw = (torch.rand(128, generator=g).bfloat16() + 0.5 for _ in range(2))
+    cs = torch.randn(1024, 128, generator=g)
+    pos = torch.tensor(CTX) - 1
+    kg, vg = kc.cuda(), vc.cuda()
+    got = ops.attn_decode_fused_qkv(qkv.cuda(), hq, hkv, qw.cuda(), kw.cuda(), eps, pos.cuda(), cs.cuda(), kg, vg, torch.tensor(CTX, dtype=torch.int32).cuda(), tables.cuda(),
+                                    128 ** -0.5, splits).cpu().double()
+    heads = qkv.view(b, hq + 2 * hkv, 128)
+    q, k_new = rope_head(heads[:, :hq], qw, cs[pos][:, None], eps), rope_head(heads[:, hq:hq + hkv], kw, cs[pos][:, None], eps)
+    for i, n in enumerate(CTX):
+        t = tables[i].long()
+        k, v = kc[t].reshape(-1, hkv, 128)[:n].clone(), vc[t].reshape(-1, hkv, 128)[:n].clone()
+        k[n - 1], v[n - 1] = k_new[i], heads[i, hq + hkv:]
+        for cache, new in ((kg, k[n - 1]), (vg, v[n - 1])):
+            # (a rounding of the norm apart at most: one unit of bf16)
+            assert ((cache[t[(n - 1) // 256], (n - 1) % 256].cpu().double() - new.double()).abs() <= new.double().abs() * 2.0 ** -7 + 1e-6).all()
+        k, v = (x.double().repeat_interleave(group, 1) for x in (k, v))
+        w = torch.softmax((k * q[i].double()).sum(-1) * 128 ** -0.5, 0)
+        want = (w[:, :, None] * v).sum(0)
+        scale = (w[:, :, None] * v.abs()).sum(0)
+        # the result's own rounding, and scores of fp32 sums over bf16 products with inputs up to a rounding apart
+        assert ((got[i] - want).abs() <= want.abs() * 2.0 ** -8 + scale * 0.03).all(), n
+        assert ((got[i] - want).norm() / want.norm()) < 0.01, n
+    plain = ops.attn_decode(q.cuda(), kg, vg, torch.tensor(CTX, dtype=torch.int32).cuda(), tables.cuda(), 128 ** -0.5, splits).cpu().double()
+    assert ((plain - got).norm() / got.norm()) < 0.01
