@@ -923,6 +923,21 @@ __device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int
     return true;
 }
 
+constexpr float LOG2E_F = 1.4426950408889634f;
+// Over the four lanes fr, fr + 16, fr + 32, fr + 48 (a row of results of the matrix cores): rows and halves of the wave exchanged on the vector ALU.
+__device__ __forceinline__ float rows_max(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+__device__ __forceinline__ float rows_sum(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+
 // (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
 constexpr int attn_waves(int nks, int nvt, int mode, int var) { return nks + nvt <= 4 ? 4 : nks + nvt <= (mode == 1 && nvt <= 4 && var != VAR_EXT ? 12 : 8) ? 3 : nks + nvt <= 16 ? 2 : 1; }
 // Wide heads leave one wave per SIMD and use its whole register file: there a second form of the loop's arithmetic costs more in registers than the
@@ -936,6 +951,14 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     constexpr bool GROUPED = MODE == 1;                      // rows are the heads of a KV group (one query per sequence)
     constexpr bool EXT = VAR == VAR_EXT, BIAS = VAR == VAR_BIAS;
     constexpr bool SPLIT = MODE != 0;                        // the waves share 16 rows and split the keys
+    // The arithmetic around the products.  LEAN: scores, maxima and sinks are kept times log2 e, so that a weight is one subtraction and the hardware's 2^x
+    // (fp32 throughout, about 1 ulp); a row's maximum crosses its four lanes on the vector ALU; each of them adds up its own keys' weights until the end; the
+    // values' rows lie in LDS as the products read them.  us without and with it: 16 heads of 128 x 128 over 8, prompts of 1000 tokens 36.9 and 34.1, 1024 behind
+    // 2000 119.6 and 107.2, 32 of 1000 577 and 530; 32 x 32, 1024 behind 2000 50.3 and 41.0; 64 single tokens behind 1024 (32 x 32) 16.0 and 14.1.  Wide heads,
+    // one wave a SIMD, are bound by how their loop is laid out: 192 x 128 without a window 214 and 171, but with slopes 218 and 236, windows 39 and 40 (and
+    // a row's bits may not depend on a window that it does not reach); 256 x 256 306 and 312.
+    constexpr bool LEAN = !attn_wide(NKS, NVT);
+    constexpr float UNIT = LEAN ? LOG2E_F : 1.0f, BACK = LEAN ? 1.0f : LOG2E_F;
     constexpr int ROWS_Q = MQ;                               // queries per workgroup
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     int seq = -1, q0 = 0, qlen = 0, qbase = 0, by = blockIdx.y;
@@ -972,7 +995,10 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     const int klen = a.context_lens[seq], past = klen - qlen;
     const int nq = GROUPED ? 1 : min(ROWS_Q, qlen - q0);
     const int nrows = GROUPED ? group : nq;                  // real rows of the workgroup's 64
-    const int kld = dim + 8, vld = MK + 8;                   // LDS row strides in elements (8-byte aligned rows)
+    const int kld = dim + 8, vld = MK + 8;                   // LDS row strides in elements (16-byte aligned rows)
+    // Place of key k in a column's row of V: of every 32 keys a lane's eight (four of either 16-key block) lie side by side, a 16-byte read that meets no
+    // bank twice.
+    auto vplace = [](int k) { return !LEAN ? k : (k & ~31) | (k >> 2 & 3) << 3 | (k >> 4 & 1) << 2 | (k & 3); };
     bf16* ks = reinterpret_cast<bf16*>(smem_raw);            // [MK][dim + 8]
     bf16* vt = ks + MK * kld;                                // [vdim][MK + 8]: V transposed
     // GROUPED: every wave holds the same 16 rows (heads) and takes the 16 keys kt = wave of every 64-key tile, with its own
@@ -1030,8 +1056,8 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     for (int i = 0; i < NVT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
     if (a.sinks && (!SPLIT || (wave == 0 && part == 0))) {   // the sink is what a row starts from; where waves or parts share a row, one of them holds it
-        m_run = a.sinks[head];
-        l_run = 1.f;
+        m_run = a.sinks[head] * UNIT;
+        l_run = !LEAN || fq == 0 ? 1.f : 0.f;
     }
     const int32_t* table = a.block_tables + (int64_t)seq * a.table_stride;
     const bool wave_idle = !SPLIT && wave * 16 >= nrows;     // no row of this wave is real
@@ -1054,7 +1080,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         const float* src = a.bias + (int64_t)(GROUPED ? by * group : head) * a.bias_len;
         for (int i = tid; i < heads_here * a.bias_ld; i += 256) {
             const int r = i / a.bias_ld, d = i - r * a.bias_ld - 3;
-            bias_s[i] = src[(int64_t)r * a.bias_len + min(max(d, 0), a.bias_len - 1)];
+            bias_s[i] = src[(int64_t)r * a.bias_len + min(max(d, 0), a.bias_len - 1)] * UNIT;
         }
         bias_row = bias_s + (GROUPED ? min(fr, group - 1) : 0) * a.bias_ld + 3;
     }
@@ -1085,9 +1111,10 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
             }
         }
     };
-    const float slope = a.slopes ? a.slopes[head] : 0.f;
-    const float row_scale = EXT ? a.scale * query_temperature(qpos, a.temp_coef, a.temp_every) : a.scale;
-    const float cap_in = EXT && a.softcap > 0.f ? 2.8853900817779268f / a.softcap : 0.f;     // tanh(s / cap) = 1 - 2 / (2^(cap_in s) + 1)
+    const float slope = a.slopes ? a.slopes[head] * UNIT : 0.f;
+    const float row_scale = (EXT ? a.scale * query_temperature(qpos, a.temp_coef, a.temp_every) : a.scale) * UNIT;
+    const float cap_in = EXT && a.softcap > 0.f ? 2.0f * BACK / a.softcap : 0.f;             // tanh(s / cap) = 1 - 2 / (2^(2 log2 e s / cap) + 1)
+    const float cap = EXT ? a.softcap * UNIT : 0.f;
     const int nblocks = EXT && a.pool > 0 ? blocks_seen(last_key, a.window, a.pool) : 0, my_blocks = EXT && a.pool > 0 ? blocks_seen(qpos, a.window, a.pool) : 0;
     // keys a row sees: lo_window (or one of the first keep_first) and lo_chunk at least, qpos at most
     const int lo_window = a.window > 0 ? qpos - a.window + 1 : 0, lo_chunk = a.chunk > 0 ? qpos / a.chunk * a.chunk : 0;
@@ -1137,7 +1164,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
 #pragma clang fp contract(off)                               // (one rounding in either form: a row's bits do not depend on where its wave begins)
                     v = sc[t][r] * row_scale;
                 }
-                if (EXT && cap_in > 0.f) v = a.softcap - 2.0f * a.softcap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap_in) + 1.0f);
+                if (EXT && cap_in > 0.f) v = cap - 2.0f * cap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap_in) + 1.0f);
                 if constexpr (!WHOLE) {
                     const bool seen = POOLED ? key < my_blocks : (key <= qpos) & ((key >= lo_window) | (key < a.keep_first)) & (key >= lo_chunk);
                     if (!BIAS && !POOLED) v = __builtin_fmaf(-slope, (float)(qpos - key), v);
@@ -1147,11 +1174,14 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                 mx = fmaxf(mx, sc[t][r]);
             }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        if constexpr (LEAN) {
+            mx = rows_max(mx);
+        } else {
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        }
         const float m_new = fmaxf(m_run, mx);
-        // e^x as the hardware's 2^(x log2 e): fp32 throughout, about 1 ulp
-        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * 1.4426950408889634f);
+        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * BACK);
         const float m_ref = m_new == -INFINITY ? 0.f : m_new;                // (a row that has seen nothing: its scores are -inf, their weights 0)
         float sum = 0.f;
         // The weights as the B operand of products over 32 rows: of two 16-key blocks, once with hi and once with lo - or, where a wave
@@ -1162,8 +1192,8 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         for (int t = 0; t < NKT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                // (wide heads: the same value, but without the test the loop is laid out so that it takes up to a tenth longer)
-                const float pv = attn_wide(NKS, NVT) && !WHOLE && sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * 1.4426950408889634f);
+                // (the test: the same value, but without it the form that is not LEAN is laid out so that it takes up to a tenth longer)
+                const float pv = !LEAN && !WHOLE && sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * BACK);
                 sum += pv;
                 const bf16 hi = (bf16)pv;
                 const bf16 lo = (bf16)(pv - (float)hi);
@@ -1175,20 +1205,29 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                     pg[t / 2][t % 2 * 4 + r] = lo;
                 }
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        if constexpr (!LEAN) {
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+        }
         l_run = l_run * alpha + sum;
         m_run = m_new;
 #pragma unroll
         for (int i = 0; i < NVT; ++i)
             if (EXACT || i < nvt) {
                 f32x4 acc = o[i] * alpha;
-                const bf16* vrow = vt + (i * 16 + fr) * vld + fq * 4;
+                const bf16* vrow = vt + (i * 16 + fr) * vld + fq * (LEAN ? 8 : 4);
 #pragma unroll
                 for (int t = 0; t < NP; ++t) {
-                    const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(vrow + (SPLIT ? wave : 2 * t) * 16);
-                    const bf16x4 v1 = SPLIT ? v0 : *reinterpret_cast<const bf16x4*>(vrow + (2 * t + 1) * 16);
-                    const bf16x8 vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    bf16x8 vf;
+                    if constexpr (SPLIT) {
+                        const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(vrow + (LEAN ? (wave >> 1) * 32 + (wave & 1) * 4 : wave * 16));
+                        vf = __builtin_shufflevector(v0, v0, 0, 1, 2, 3, 4, 5, 6, 7);
+                    } else if constexpr (LEAN) {
+                        vf = *reinterpret_cast<const bf16x8*>(vrow + t * 32);
+                    } else {
+                        const bf16x4 v0 = *reinterpret_cast<const bf16x4*>(vrow + 2 * t * 16), v1 = *reinterpret_cast<const bf16x4*>(vrow + (2 * t + 1) * 16);
+                        vf = __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7);
+                    }
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[t], acc, 0, 0, 0);
                     if constexpr (!SPLIT) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pg[t], acc, 0, 0, 0);
                 }
@@ -1209,7 +1248,13 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                     for (int e = 0; e < 8; ++e)
                         if (k0 + piece + e > last_key) v[e] = (bf16)0.f;
                 }
-                *reinterpret_cast<bf16x8*>(vt + c * vld + piece) = v;
+                bf16* dst = vt + c * vld + vplace(piece);
+                if constexpr (LEAN) {
+                    *reinterpret_cast<bf16x4*>(dst) = __builtin_shufflevector(v, v, 0, 1, 2, 3);
+                    *reinterpret_cast<bf16x4*>(dst + 8) = __builtin_shufflevector(v, v, 4, 5, 6, 7);
+                } else {
+                    *reinterpret_cast<bf16x8*>(dst) = v;
+                }
             }
         }
         __syncthreads();
@@ -1264,7 +1309,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                 const int i = tid + 256 * j, r = i & (MK - 1), c = (i / MK) << 3;
                 if (c < vdim) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) vt[(c + e) * vld + r] = r < nblocks - b0 ? vB[j][e] : (bf16)0.f;
+                    for (int e = 0; e < 8; ++e) vt[(c + e) * vld + vplace(r)] = r < nblocks - b0 ? vB[j][e] : (bf16)0.f;
                 }
             }
             __syncthreads();
@@ -1283,6 +1328,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         kb = kb2;
     }
     if (ka <= last_key) tile(ka, ka, kA, vA);
+    if constexpr (LEAN) l_run = rows_sum(l_run);
     // epilogue through LDS: [MQ][vdim] fp32, then turn back by the query's position, gate, store
     __syncthreads();
     float* os = reinterpret_cast<float*>(smem_raw);
@@ -1308,14 +1354,14 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 const float mw = ml[(w * 16 + r) * 2];
-                const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw - big) * 1.4426950408889634f);
+                const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw - big) * BACK);
                 num += os[(w * 16 + r) * vdim + col] * f;
                 den += ml[(w * 16 + r) * 2 + 1] * f;
             }
             if (prow) {                                      // a part's record: the row relative to its maximum, then maximum and sum
                 prow[r * (vdim + 2) + col] = num;
                 if (col == 0) {
-                    prow[r * (vdim + 2) + vdim] = big;
+                    prow[r * (vdim + 2) + vdim] = big * BACK;                // (in units of log2 e, see LEAN)
                     prow[r * (vdim + 2) + vdim + 1] = den;
                 }
             } else {
@@ -1389,7 +1435,7 @@ __global__ __launch_bounds__(256) void attn_merge_parts_kernel(const float* __re
         for (int p = 0; p < nparts; ++p) {
             const float* pr = base + p * pstride;
             if (pr[vdim] == -INFINITY) continue;             // a part without keys (its row is not written)
-            const float f = __builtin_amdgcn_exp2f((pr[vdim] - big) * 1.4426950408889634f);
+            const float f = __builtin_amdgcn_exp2f(pr[vdim] - big);
             num += pr[col] * f;
             den += pr[vdim + 1] * f;
         }
