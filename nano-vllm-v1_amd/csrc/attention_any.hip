@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void attn_rotary_prep_vec_kernel(PrepArgs a, i
             head += NVH_DPP(head, 0x4E);
             head += NVH_DPP(head, 0x141);
             if (per_head >= 16) head += NVH_DPP(head, 0x140);
-            if (per_head >= 32) head += __shfl_xor(head, 16, 64);
+            if (per_head >= 32) head = pair16_sum(head);
         }
         sums[i] = head;
         if (i < pieces) (i << 3 < nq ? sq : sk) += ss[0];
@@ -746,8 +746,7 @@ __global__ __launch_bounds__(256) void attn_paged_f32_kernel(AttnArgs a, int gro
             s[e] = ok ? s[e] - slope * (float)(qpos - (key0 + e)) + biases[e] : -INFINITY;
             top = fmaxf(top, s[e]);
         }
-        top = fmaxf(top, __shfl_xor(top, 16, 64));
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        top = rows_max(top);
         // (a row that sees nothing yet keeps m = -inf)
         const float alpha = top == -INFINITY ? 1.f : expf(m_run - top);
         f32x4 p;
@@ -774,8 +773,7 @@ __global__ __launch_bounds__(256) void attn_paged_f32_kernel(AttnArgs a, int gro
         __builtin_amdgcn_sched_barrier(0);
         k0 = next;
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = rows_sum(l_run);
     float* ml = smem + 4 * 16 * OLD;                         // [4][16][2]
     {
         float* out = smem + (wave * 16 + row) * OLD + 4 * quarter;
@@ -924,20 +922,6 @@ __device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int
 }
 
 constexpr float LOG2E_F = 1.4426950408889634f;
-// Over the four lanes fr, fr + 16, fr + 32, fr + 48 (a row of results of the matrix cores): rows and halves of the wave exchanged on the vector ALU.
-__device__ __forceinline__ float rows_max(float x) {
-    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
-    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
-}
-__device__ __forceinline__ float rows_sum(float x) {
-    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    x = __uint_as_float(p[0]) + __uint_as_float(p[1]);
-    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
-}
-
 // (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
 constexpr int attn_waves(int nks, int nvt, int mode, int var) { return nks + nvt <= 4 ? 4 : nks + nvt <= (mode == 1 && nvt <= 4 && var != VAR_EXT ? 12 : 8) ? 3 : nks + nvt <= 16 ? 2 : 1; }
 // Wide heads leave one wave per SIMD and use its whole register file: there a second form of the loop's arithmetic costs more in registers than the

@@ -331,10 +331,7 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         for (int g = 0; g < G; ++g) {
             l[g] = row16_sum(l[g]);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                acc[g][j] += __shfl_xor(acc[g][j], 16, 64);
-                acc[g][j] += __shfl_xor(acc[g][j], 32, 64);
-            }
+            for (int j = 0; j < 8; ++j) acc[g][j] = rows_sum(acc[g][j]);
         }
     } else {
         // merge the 4 rows of the wave (lanes l, l^16, l^32 hold the same output columns)

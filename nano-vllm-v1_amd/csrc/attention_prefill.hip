@@ -273,7 +273,7 @@ __global__ __launch_bounds__(G * RB * KS * 64, (G * RB * KS <= 4 && STAGES * KS 
                 mx1 = fmaxf(mx1, st[1][r]);
             }
             float mx = fmaxf(mx0, mx1);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * scale_log2;
+            mx = pair32_max(mx) * scale_log2;
             resc = __any(mx > m_run + RESCALE_LOG2);
             alpha = 1.0f;
             if (resc) {
@@ -494,7 +494,7 @@ __global__ __launch_bounds__(G * RB * KS * 64, (G * RB * KS <= 4 && STAGES * KS 
     }
 
     // ---- lane (q, hh) holds O[q][32dt + 8(r>>2) + 4hh + (r&3)]
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = pair32_sum(l_run);
     if (qrow_raw >= lq) return;
     if (num_splits == 1) {
         const float inv = l_run > 0.f ? 1.0f / l_run : 0.f;

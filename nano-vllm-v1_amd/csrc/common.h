@@ -126,19 +126,30 @@ __device__ __forceinline__ float row16_max(float x) {
     x = fmaxf(x, NVH_DPP(x, 0x140));
     return x;
 }
+// With the lane 16 (32) places on, modulo 32 (64): rows (halves) of the wave exchanged on the vector ALU; a shuffle goes through the LDS unit and takes some
+// 100 cycles of a chain.  Both lanes of a pair receive the same bits, those of x op shuffled x.
+__device__ __forceinline__ float pair16_sum(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float pair32_sum(float x) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+}
+__device__ __forceinline__ float pair16_max(float x) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+__device__ __forceinline__ float pair32_max(float x) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+}
+// Over the four lanes l, l + 16, l + 32, l + 48 (a row of results of the matrix cores).
+__device__ __forceinline__ float rows_sum(float x) { return pair32_sum(pair16_sum(x)); }
+__device__ __forceinline__ float rows_max(float x) { return pair32_max(pair16_max(x)); }
 // Full 64-lane reductions (result in every lane).
-__device__ __forceinline__ float wave_sum(float x) {
-    x = row16_sum(x);
-    x += __shfl_xor(x, 16, 64);
-    x += __shfl_xor(x, 32, 64);
-    return x;
-}
-__device__ __forceinline__ float wave_max(float x) {
-    x = row16_max(x);
-    x = fmaxf(x, __shfl_xor(x, 16, 64));
-    x = fmaxf(x, __shfl_xor(x, 32, 64));
-    return x;
-}
+__device__ __forceinline__ float wave_sum(float x) { return rows_sum(row16_sum(x)); }
+__device__ __forceinline__ float wave_max(float x) { return rows_max(row16_max(x)); }
 
 __device__ __forceinline__ float bf2f(bf16 v) { return (float)v; }
 __device__ __forceinline__ bf16 f2bf(float v) { return (bf16)v; }

@@ -245,8 +245,7 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
                                 ss += v[2];
                                 ss += v[3];
                             }
-                        ss += __shfl_xor(ss, 16, 64);
-                        ss += __shfl_xor(ss, 32, 64);
+                        ss = rows_sum(ss);
                     } else {
                         const f32x4* ps = reinterpret_cast<const f32x4*>(rs.sumsq + (int64_t)min(m0 + wm * WM + j * 16 + fr, M - 1) * rs.parts);
                         for (int q = 0; q < (rs.parts >> 2); ++q) {
@@ -778,9 +777,7 @@ __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* _
         const int parts = 2 * (int)gridDim.x;
 #pragma unroll
         for (int j = 0; j < TM; ++j) {
-            float t = sq[j];
-            t += __shfl_xor(t, 16, 64);
-            t += __shfl_xor(t, 32, 64);
+            const float t = rows_sum(sq[j]);
             if (fq == 0) row_sumsq[(int64_t)(m0 + wm * 32 + j * 16 + fr) * parts + 2 * bx + wn] = t;
         }
         return;
