@@ -648,7 +648,7 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
 // where every XCD pulls x and W through its own L2 first: a prefill chunk 2.745 -> 2.736 ms, a decode step of 256
 // sequences 6.251 -> 6.240 ms.  (The same for K-slab grids - the O / down projections of 256 decode rows in four slabs:
 // no change, 6.251 against 6.253 ms; not built in.)
-template <int STAGES, bool RESIDUAL = false>
+template <int STAGES, bool RESIDUAL, bool BEHIND>
 __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* __restrict__ x, int64_t x_stride,
                                                                    const bf16* __restrict__ w, const bf16* __restrict__ bias,
                                                                    bf16* __restrict__ y, int64_t y_stride, int M, int N, int K,
@@ -681,11 +681,11 @@ __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* _
         else src_row[i] = w + (int64_t)min(n0 + r, N - 1) * K + chunk * 8 + half * BK;
         lds_off[i] = half * TILE_BYTES + (is_b ? A_BYTES : 0) + g8 * 1024;
     }
-    auto stage = [&](int t) {
+    auto stage = [&](int t, int from, int to) {
         const int k0 = t * 2 * BK;
         char* base = smem + (t % STAGES) * STAGE_BYTES;
 #pragma unroll
-        for (int i = 0; i < PW; ++i)
+        for (int i = from; i < to; ++i)
             __builtin_amdgcn_global_load_lds((const GLOBAL_AS void*)(src_row[i] + k0), (LDS_AS void*)(base + lds_off[i]), 16, 0, 0);
     };
     f32x4 acc[TN][TM];
@@ -706,13 +706,16 @@ __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* _
                 asm volatile("global_load_dwordx2 %0, %1, off" : "=v"(res_pre[i][j]) : "v"(rp) : "memory");
             }
     }
-    for (int t = 0; t < AHEAD && t < nstages; ++t) stage(t);
+    // BEHIND: a stage's DMA goes out behind the fragment reads, half of it with each k-step: ahead of them a burst of it holds the wave up.  Over a long K, where
+    // what counts is that it starts early, it goes first (chosen at the launch: K up to 3072).  us, ahead and behind: 1024 x 1024 x 1024 7.1 and 6.7, x 2048 10.2 and 9.5, 800 x 1024 x 3072 12.8 and
+    // 12.1, but 960 x 1024 x 4096 19.3 and 19.8.
+    for (int t = 0; t < AHEAD && t < nstages; ++t) stage(t, 0, PW);
     for (int t = 0; t < nstages; ++t) {
         wait_tiles_in_flight<PW, (AHEAD > 0 ? AHEAD - 1 : 0)>(min(AHEAD - 1, nstages - 1 - t));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (t + AHEAD < nstages) stage(t + AHEAD);
+        if (!BEHIND && t + AHEAD < nstages) stage(t + AHEAD, 0, PW);
         const char* a_base = smem + (t % STAGES) * STAGE_BYTES + grp * TILE_BYTES;
         const char* b_base = a_base + A_BYTES;
 #pragma unroll
@@ -728,6 +731,11 @@ __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* _
             for (int j = 0; j < TM; ++j) {
                 const int r = wm * 32 + j * 16 + fr;
                 bfr[j] = *reinterpret_cast<const bf16x8*>(b_base + r * 128 + ((kc ^ ((r >> 1) & 7)) << 4));
+            }
+            if constexpr (BEHIND) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (t + AHEAD < nstages) stage(t + AHEAD, ks * (PW / 2), (ks + 1) * (PW / 2));
+                __builtin_amdgcn_sched_barrier(0);
             }
 #pragma unroll
             for (int i = 0; i < TN; ++i)
@@ -1277,10 +1285,13 @@ void launch_gemm_nt(const GemmArgs& a) {
 void launch_gemm_kgroups(const GemmArgs& a) {
     constexpr int STAGES = 3, smem = STAGES * 2 * (64 + 64) * 128;
     static bool configured = false;
-    auto kern = a.residual ? gemm_kgroups_bf16_nt_kernel<STAGES, true> : gemm_kgroups_bf16_nt_kernel<STAGES, false>;
+    const bool behind = a.K <= 3072;
+    const auto kern = a.residual ? (behind ? &gemm_kgroups_bf16_nt_kernel<STAGES, true, true> : &gemm_kgroups_bf16_nt_kernel<STAGES, true, false>)
+                                 : (behind ? &gemm_kgroups_bf16_nt_kernel<STAGES, false, true> : &gemm_kgroups_bf16_nt_kernel<STAGES, false, false>);
     if (!configured) {
-        (void)hipFuncSetAttribute((const void*)gemm_kgroups_bf16_nt_kernel<STAGES, false>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-        (void)hipFuncSetAttribute((const void*)gemm_kgroups_bf16_nt_kernel<STAGES, true>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        for (const auto k : {&gemm_kgroups_bf16_nt_kernel<STAGES, false, false>, &gemm_kgroups_bf16_nt_kernel<STAGES, false, true>, &gemm_kgroups_bf16_nt_kernel<STAGES, true, false>,
+                             &gemm_kgroups_bf16_nt_kernel<STAGES, true, true>})
+            (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
         configured = true;
     }
     if (a.plan) {

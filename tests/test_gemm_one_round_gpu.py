@@ -54,3 +54,16 @@ def test_slabs(m, n, k, s):
     for p in range(s):
         a, c = x[:, p * per:(p + 1) * per].double(), w[:, p * per:(p + 1) * per].double()
         assert ((got[p].double() - a @ c.t().contiguous()).abs() <= a.abs() @ c.abs().t().contiguous() * per * 2.0 ** -24 + 1e-30).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (833, 1020, 1152), (1000, 964, 3072), (1000, 964, 3200)])
+def test_two_groups(m, n, k):
+    """64 x 64 tiles of two wave groups: stages requested behind the reads (K up to 3072) and ahead of them."""
+    from nanovllm import ops
+    assert plan(m, n, k).startswith("kgroups")
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w, b = ((torch.randn(s, generator=g) * 0.5).bfloat16().cuda() for s in ((m, k), (n, k), (n,)))
+    got = ops.linear(x, w, b).double()
+    want = x.double() @ w.double().t().contiguous() + b.double()
+    slack = (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2.0 ** -24
+    assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + slack).all()
