@@ -935,14 +935,14 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     constexpr bool GROUPED = MODE == 1;                      // rows are the heads of a KV group (one query per sequence)
     constexpr bool EXT = VAR == VAR_EXT, BIAS = VAR == VAR_BIAS;
     constexpr bool SPLIT = MODE != 0;                        // the waves share 16 rows and split the keys
-    // The arithmetic around the products.  LEAN: scores, maxima and sinks are kept times log2 e, so that a weight is one subtraction and the hardware's 2^x
-    // (fp32 throughout, about 1 ulp); a row's maximum crosses its four lanes on the vector ALU; each of them adds up its own keys' weights until the end; the
-    // values' rows lie in LDS as the products read them.  us without and with it: 16 heads of 128 x 128 over 8, prompts of 1000 tokens 36.9 and 34.1, 1024 behind
-    // 2000 119.6 and 107.2, 32 of 1000 577 and 530; 32 x 32, 1024 behind 2000 50.3 and 41.0; 64 single tokens behind 1024 (32 x 32) 16.0 and 14.1.  Wide heads,
-    // one wave a SIMD, are bound by how their loop is laid out: 192 x 128 without a window 214 and 171, but with slopes 218 and 236, windows 39 and 40 (and
-    // a row's bits may not depend on a window that it does not reach); 256 x 256 306 and 312.
+    // LEAN: a row's maximum and its sum cross their four lanes on the vector ALU, and the values' rows lie in LDS as the products read them; the same bits as
+    // the other form's.  us without and with it: 16 heads of 128 x 128 over 8, prompts of 1000 tokens 36.1 and 34.1, 1024 behind 2000 119.8 and 110.3, 32 of
+    // 1000 575 and 536; 32 x 32, 1024 behind 2000 50.4 and 43.1; 64 single tokens behind 1024 (32 x 32) 16.2 and 14.5.  Wide heads, one wave a SIMD, are bound
+    // by how their loop is laid out (with the scores' units of the next lines): 192 x 128 without a window 214 and 171, but with slopes 218 and 236; 256 x 256
+    // 306 and 312.
+    // (Scores kept times log2 e, which saves an instruction a weight, and a lane's sums left to the end, were 1 % faster still.  But such a score is rounded at its
+    // own size instead of a weight at its distance from the maximum, and a bias or sink at the end of fp32's range leaves it.)
     constexpr bool LEAN = !attn_wide(NKS, NVT);
-    constexpr float UNIT = LEAN ? LOG2E_F : 1.0f, BACK = LEAN ? 1.0f : LOG2E_F;
     constexpr int ROWS_Q = MQ;                               // queries per workgroup
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     int seq = -1, q0 = 0, qlen = 0, qbase = 0, by = blockIdx.y;
@@ -1040,8 +1040,8 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     for (int i = 0; i < NVT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
     if (a.sinks && (!SPLIT || (wave == 0 && part == 0))) {   // the sink is what a row starts from; where waves or parts share a row, one of them holds it
-        m_run = a.sinks[head] * UNIT;
-        l_run = !LEAN || fq == 0 ? 1.f : 0.f;
+        m_run = a.sinks[head];
+        l_run = 1.f;
     }
     const int32_t* table = a.block_tables + (int64_t)seq * a.table_stride;
     const bool wave_idle = !SPLIT && wave * 16 >= nrows;     // no row of this wave is real
@@ -1064,7 +1064,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         const float* src = a.bias + (int64_t)(GROUPED ? by * group : head) * a.bias_len;
         for (int i = tid; i < heads_here * a.bias_ld; i += 256) {
             const int r = i / a.bias_ld, d = i - r * a.bias_ld - 3;
-            bias_s[i] = src[(int64_t)r * a.bias_len + min(max(d, 0), a.bias_len - 1)] * UNIT;
+            bias_s[i] = src[(int64_t)r * a.bias_len + min(max(d, 0), a.bias_len - 1)];
         }
         bias_row = bias_s + (GROUPED ? min(fr, group - 1) : 0) * a.bias_ld + 3;
     }
@@ -1095,10 +1095,9 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
             }
         }
     };
-    const float slope = a.slopes ? a.slopes[head] * UNIT : 0.f;
-    const float row_scale = (EXT ? a.scale * query_temperature(qpos, a.temp_coef, a.temp_every) : a.scale) * UNIT;
-    const float cap_in = EXT && a.softcap > 0.f ? 2.0f * BACK / a.softcap : 0.f;             // tanh(s / cap) = 1 - 2 / (2^(2 log2 e s / cap) + 1)
-    const float cap = EXT ? a.softcap * UNIT : 0.f;
+    const float slope = a.slopes ? a.slopes[head] : 0.f;
+    const float row_scale = EXT ? a.scale * query_temperature(qpos, a.temp_coef, a.temp_every) : a.scale;
+    const float cap_in = EXT && a.softcap > 0.f ? 2.0f * LOG2E_F / a.softcap : 0.f;          // tanh(s / cap) = 1 - 2 / (2^(cap_in s) + 1)
     const int nblocks = EXT && a.pool > 0 ? blocks_seen(last_key, a.window, a.pool) : 0, my_blocks = EXT && a.pool > 0 ? blocks_seen(qpos, a.window, a.pool) : 0;
     // keys a row sees: lo_window (or one of the first keep_first) and lo_chunk at least, qpos at most
     const int lo_window = a.window > 0 ? qpos - a.window + 1 : 0, lo_chunk = a.chunk > 0 ? qpos / a.chunk * a.chunk : 0;
@@ -1148,7 +1147,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
 #pragma clang fp contract(off)                               // (one rounding in either form: a row's bits do not depend on where its wave begins)
                     v = sc[t][r] * row_scale;
                 }
-                if (EXT && cap_in > 0.f) v = cap - 2.0f * cap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap_in) + 1.0f);
+                if (EXT && cap_in > 0.f) v = a.softcap - 2.0f * a.softcap * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * cap_in) + 1.0f);
                 if constexpr (!WHOLE) {
                     const bool seen = POOLED ? key < my_blocks : (key <= qpos) & ((key >= lo_window) | (key < a.keep_first)) & (key >= lo_chunk);
                     if (!BIAS && !POOLED) v = __builtin_fmaf(-slope, (float)(qpos - key), v);
@@ -1165,7 +1164,8 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         }
         const float m_new = fmaxf(m_run, mx);
-        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * BACK);
+        // e^x as the hardware's 2^(x log2 e): fp32 throughout, about 1 ulp of the distance from the maximum, wherever the scores lie
+        const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E_F);
         const float m_ref = m_new == -INFINITY ? 0.f : m_new;                // (a row that has seen nothing: its scores are -inf, their weights 0)
         float sum = 0.f;
         // The weights as the B operand of products over 32 rows: of two 16-key blocks, once with hi and once with lo - or, where a wave
@@ -1177,7 +1177,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 // (the test: the same value, but without it the form that is not LEAN is laid out so that it takes up to a tenth longer)
-                const float pv = !LEAN && !WHOLE && sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * BACK);
+                const float pv = !LEAN && !WHOLE && sc[t][r] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((sc[t][r] - m_ref) * LOG2E_F);
                 sum += pv;
                 const bf16 hi = (bf16)pv;
                 const bf16 lo = (bf16)(pv - (float)hi);
@@ -1189,7 +1189,9 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
                     pg[t / 2][t % 2 * 4 + r] = lo;
                 }
             }
-        if constexpr (!LEAN) {
+        if constexpr (LEAN) {
+            sum = rows_sum(sum);
+        } else {
             sum += __shfl_xor(sum, 16, 64);
             sum += __shfl_xor(sum, 32, 64);
         }
@@ -1312,7 +1314,6 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
         kb = kb2;
     }
     if (ka <= last_key) tile(ka, ka, kA, vA);
-    if constexpr (LEAN) l_run = rows_sum(l_run);
     // epilogue through LDS: [MQ][vdim] fp32, then turn back by the query's position, gate, store
     __syncthreads();
     float* os = reinterpret_cast<float*>(smem_raw);
@@ -1338,14 +1339,14 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 const float mw = ml[(w * 16 + r) * 2];
-                const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw - big) * BACK);
+                const float f = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((mw - big) * LOG2E_F);
                 num += os[(w * 16 + r) * vdim + col] * f;
                 den += ml[(w * 16 + r) * 2 + 1] * f;
             }
             if (prow) {                                      // a part's record: the row relative to its maximum, then maximum and sum
                 prow[r * (vdim + 2) + col] = num;
                 if (col == 0) {
-                    prow[r * (vdim + 2) + vdim] = big * BACK;                // (in units of log2 e, see LEAN)
+                    prow[r * (vdim + 2) + vdim] = big;
                     prow[r * (vdim + 2) + vdim + 1] = den;
                 }
             } else {
@@ -1403,7 +1404,7 @@ __global__ __launch_bounds__(256, attn_waves(NKS, NVT, MODE, VAR)) void attn_pag
     }
 }
 
-// The rows of the key parts of a (sequence, group of heads) merged: out = gate * sum_p num_p 2^(m_p - m) / sum_p den_p 2^(m_p - m).
+// The rows of the key parts of a (sequence, group of heads) merged: out = gate * sum_p num_p e^(m_p - m) / sum_p den_p e^(m_p - m).
 __global__ __launch_bounds__(256) void attn_merge_parts_kernel(const float* __restrict__ parts, int nparts, int rows, int vdim, int H, const float* __restrict__ gate,
                                                                const bf16* __restrict__ gate_elems, int64_t ld_elems, bf16* __restrict__ out) {
     // one workgroup per (sequence, group of heads, row): a lane per value column
@@ -1419,7 +1420,7 @@ __global__ __launch_bounds__(256) void attn_merge_parts_kernel(const float* __re
         for (int p = 0; p < nparts; ++p) {
             const float* pr = base + p * pstride;
             if (pr[vdim] == -INFINITY) continue;             // a part without keys (its row is not written)
-            const float f = __builtin_amdgcn_exp2f(pr[vdim] - big);
+            const float f = __builtin_amdgcn_exp2f((pr[vdim] - big) * LOG2E_F);
             num += pr[col] * f;
             den += pr[vdim + 1] * f;
         }
