@@ -93,6 +93,16 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     const int end = min(ctx, start + chunk);
 
     // Everything that this token brings is requested before the first keys are, and worked on behind that request.
+    // The first page and the position together: one behind the other is one more latency in front of the first keys; and the new token's own key and value only
+    // where the range ends with it.  us, mean of four runs each: 8 sequences of 500..1500 keys in 8 ranges 13.66 when the first keys came behind the epilogue,
+    // 13.91 with the page behind the position and every range asking for the new token, 13.79 as it is; 4 in 16 ranges 11.40, 11.27 and 11.19.
+    const int32_t* table = tables + (int64_t)b * table_stride;
+    int page = 0;
+    int64_t pos = 0;
+    if (start < end) {
+        page = table[start >> 8];
+        if constexpr (FUSED) pos = fz.positions[b];
+    }
     bf16x8 qv[G], qw, kw, k_new, v_new;
     f32x4 cs[4];
     const bool has_new = FUSED && start < end && end == ctx;      // (uniform) this range ends with the step's own token
@@ -103,10 +113,12 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         if constexpr (FUSED) {
             const bf16* row = q + (int64_t)b * q_stride;
             qw = *reinterpret_cast<const bf16x8*>(fz.q_norm_w + c * 8);
-            kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
-            k_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8);
-            v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
-            const float* cs_row = fz.cos_sin + fz.positions[b] * 128 + 8 * (c & 7);
+            if (has_new) {
+                kw = *reinterpret_cast<const bf16x8*>(fz.k_norm_w + c * 8);
+                k_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + kvh) * 128 + c * 8);
+                v_new = *reinterpret_cast<const bf16x8*>(row + (int64_t)(hq + hkv + kvh) * 128 + c * 8);
+            }
+            const float* cs_row = fz.cos_sin + pos * 128 + 8 * (c & 7);
 #pragma unroll
             for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4*>(cs_row + (i >> 1) * 64 + (i & 1) * 4);
         }
@@ -169,10 +181,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     // worked on behind a request that is made in any case: behind a branch around it the waits would cover the new loads too (a launch of 24
     // sequences of 100..2047 keys 39.1 us, as it is 30.9; contexts of one trip 0.2 us longer, for the way past the loop).  More in flight gives nothing:
     // four sets in registers, or four trips in an LDS ring, leave a trip at 1 us (what a CU can have outstanding).
-    const int32_t* table = tables + (int64_t)b * table_stride;
     u32x4 ka[4], va[4], kb[4], vb[4];                        // (whole words: as 16-bit elements every one would take a register across the loop)
     const int last_page = (end - 1) >> 8;
-    int page = start < end ? table[start >> 8] : 0;
     // A wave's 16 keys of a trip: key i is token 16 (i >> 2) + 4 w + (i & 3).  Keys and values come a row a token (lane: token 16 u + rowid, 16-byte piece c:
     // a row's lanes read 256 bytes side by side; with keys loaded as the matrix cores take them, 16 bytes of 16 rows side by side, 24 of 100..2047 took 36 us).
     // MFMA: keys pass through the wave's own LDS (then lane: key fr, pieces fq + 4 i; piece p of key i lies at place p ^ i, so neither way meets a bank twice).
