@@ -923,6 +923,8 @@ __device__ __forceinline__ bool balanced_place(const AttnArgs& a, int* keys, int
 
 constexpr float LOG2E_F = 1.4426950408889634f;
 // (two forms of the loop's arithmetic must not cost a wave per SIMD: as many as one form alone leaves room for)
+// (32 x 32 would fit five in 96 registers: us, four and five, 32 heads over 8, 32 prompts of 1000 tokens 376 and 349, but 1024 behind 2000 77 and 80, 4 heads with
+// slopes 64.9 and 68.5; learned bias, 1024 behind 2000, 48 and 56)
 constexpr int attn_waves(int nks, int nvt, int mode, int var) { return nks + nvt <= 4 ? 4 : nks + nvt <= (mode == 1 && nvt <= 4 && var != VAR_EXT ? 12 : 8) ? 3 : nks + nvt <= 16 ? 2 : 1; }
 // Wide heads leave one wave per SIMD and use its whole register file: there a second form of the loop's arithmetic costs more in registers than the
 // masking that it leaves out, but for prompts without a window, chunk or slope, of which most tiles are seen whole.  FORMS: whether there are two.
