@@ -1,16 +1,17 @@
-"""Eight-wave tiles with three stages (128 x 128, 128 x 192, 256 x 128), one a CU: from fewer k-tiles than stages on, ragged edges, widths that end in a
-narrower strip of tiles, K-slabs: the bits of 64 x 64 tiles."""
+"""Eight-wave tiles with three stages (128 x 128, 128 x 192, 256 x 128), one a CU: from fewer k-tiles than stages on, ragged edges with results stored 16 and 8
+bytes at a time, weights read past the caches, widths that end in a narrower strip of tiles, K-slabs: the bits of 64 x 64 tiles.  And two-group tiles: the
+bits of their two sums."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-def plan(m, n, k):
+def plan(m, n, k, slabs=1):
     import ctypes as C
     from nanovllm import _hip
     out = C.create_string_buffer(512)
-    assert _hip.lib().nvh_gemm_plan(m, n, k, 1, 0, out, 512) == 0
+    assert _hip.lib().nvh_gemm_plan(m, n, k, slabs, 0, out, 512) == 0
     return out.value.decode()
 
 
@@ -43,10 +44,32 @@ def test_tall_bits(m, n, k):
     check(lambda: ops.linear(x, w), x, w, None)
 
 
-@pytest.mark.parametrize("m,n,k,s", [(256, 5120, 768, 3), (300, 2560, 832, 4), (128, 5120, 5184, 6)])
-def test_slabs(m, n, k, s):
-    """Slabs of 3 to 14 k-tiles, the last one shorter; each slab is a sum over its part of K alone."""
+@pytest.mark.parametrize("m,n,k,tile", [(1016, 7176, 1024, "256x128 waves 2x4 stages 3 grid"), (1001, 5256, 320, "128x192 waves 2x4 stages 3 grid"),
+                                        (897, 3976, 192, "128x128 waves 2x4 stages 3 grid"), (100, 37984, 1024, "128x192 waves 2x4 stages 3 nt"),
+                                        (128, 37980, 128, "128x192 waves 2x4 stages 3 nt"), (200, 28680, 1024, "256x128 waves 2x4 stages 3 nt"),
+                                        (256, 28676, 1088, "256x128 waves 2x4 stages 3 nt")])
+def test_ragged_and_streamed_bits(m, n, k, tile):
+    """Rows past the last one in tiles whose results leave 16 bytes a lane (N a multiple of 8), and weights of one row of tiles, read non-temporally."""
     from nanovllm import ops
+    assert plan(m, n, k).startswith(f"tile {tile}")
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = ((torch.randn(s, generator=g) * 0.5).bfloat16().cuda() for s in ((m, k), (n, k)))
+    guard = torch.full((m + 8, n), 7.0, dtype=torch.bfloat16, device="cuda")                  # rows behind the result keep what they hold
+
+    def f():
+        from nanovllm import _hip
+        _hip.call("nvh_gemm_bf16_nt", x.data_ptr(), k, w.data_ptr(), 0, guard.data_ptr(), n, m, n, k, 1, 0, torch.cuda.current_stream().cuda_stream)
+        assert bool((guard[m:] == 7.0).all())
+        return guard[:m].clone()
+
+    check(f, x, w, None)
+
+
+@pytest.mark.parametrize("m,n,k,s", [(256, 5120, 768, 3), (300, 2560, 832, 4), (128, 5120, 5184, 6), (128, 4096, 832, 8)])
+def test_slabs(m, n, k, s):
+    """Slabs of 1 to 14 k-tiles, the last one shorter or empty (13 k-tiles by two in 8 slabs); each slab is a sum over its part of K alone."""
+    from nanovllm import ops
+    assert plan(m, n, k, s).replace(" nt", "").startswith("tile 128x128 waves 2x4 stages 3 slabs")
     g = torch.Generator().manual_seed(m + n + k)
     x, w = ((torch.randn(sh, generator=g) * 0.5).bfloat16().cuda() for sh in ((m, k), (n, k)))
     got = ops.linear_splitk(x, w, s)
@@ -63,7 +86,13 @@ def test_two_groups(m, n, k):
     assert plan(m, n, k).startswith("kgroups")
     g = torch.Generator().manual_seed(m + n + k)
     x, w, b = ((torch.randn(s, generator=g) * 0.5).bfloat16().cuda() for s in ((m, k), (n, k), (n,)))
-    got = ops.linear(x, w, b).double()
+    got = ops.linear(x, w, b)
+    # group 0 adds up the even k-tiles, group 1 the odd ones: two K-slabs of the same operands with the even k-tiles in front
+    # (k-tiles of both groups are as many, K is a multiple of 128)
+    even, odd = (torch.cat([torch.arange(c, c + 64) for c in range(first, k, 128)]) for first in (0, 64))
+    order = torch.cat([even, odd]).cuda()
+    parts = ops.linear_splitk(x[:, order].contiguous(), w[:, order].contiguous(), 2)
+    assert torch.equal(got, (parts[0] + parts[1] + b.float()).bfloat16())
     want = x.double() @ w.double().t().contiguous() + b.double()
     slack = (x.double().abs() @ w.double().abs().t().contiguous()) * k * 2.0 ** -24
-    assert ((got - want).abs() <= want.abs() * 2.0 ** -8 + slack).all()
+    assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + slack).all()
