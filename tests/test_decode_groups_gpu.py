@@ -55,3 +55,44 @@ def test_new_token_and_edges(group, splits):
         assert ((got[i] - want).norm() / want.norm()) < 0.01, n
     plain = ops.attn_decode(q.cuda(), kg, vg, torch.tensor(CTX, dtype=torch.int32).cuda(), tables.cuda(), 128 ** -0.5, splits).cpu().double()
     assert ((plain - got).norm() / got.norm()) < 0.01
+
+
+@pytest.mark.parametrize("splits", [1, 5])
+@pytest.mark.parametrize("group", [1, 2, 4, 5, 8])
+def test_weights_in_fp32(group, splits):
+    """Two keys of a context carry its weights and their values nearly cancel, so that the result shows the weights to more than 16 bits."""
+    from nanovllm import ops
+    hkv, hq, scale = 2, 2 * group, 128 ** -0.5
+    g = torch.Generator().manual_seed(100 + group * 10 + splits)
+    ctxs = [2, 17, 64, 65, 130, 257, 700]
+    b, width = len(ctxs), 3
+    tables = torch.randperm(b * width, generator=g).int().view(b, width)
+    u = (torch.randn(b, hkv, 128, generator=g) * 1.2).bfloat16()
+    q = u[:, :, None].expand(b, hkv, group, 128).reshape(b, hq, 128).contiguous()
+    kc = torch.zeros(b * width, 256, hkv, 128, dtype=torch.bfloat16)
+    vc = torch.randn(b * width, 256, hkv, 128, generator=g).bfloat16()
+    wants, seen = [], [0, 0]
+    for i, n in enumerate(ctxs):
+        t = tables[i].long()
+        k, v = (-2.0 * u[i].float()).bfloat16()[None].repeat(n, 1, 1), vc[t].reshape(-1, hkv, 128)[:n].clone()      # (weights of e^-40 and less)
+        one, two = (int(x) for x in torch.randperm(n, generator=g)[:2])
+        k[one] = (u[i].float() * (0.9 + 0.1 * torch.rand(hkv, 1, generator=g))).bfloat16()
+        k[two] = (u[i].float() * (0.9 + 0.1 * torch.rand(hkv, 1, generator=g))).bfloat16()
+        s = (k.double() * u[i].double()).sum(-1) * scale
+        w = torch.softmax(s, 0)
+        v[two] = (-v[one].double() * (w[one] / w[two])[:, None]).bfloat16()
+        for p in range(width):
+            part = slice(256 * p, min(n, 256 * (p + 1)))
+            kc[t[p], :max(0, part.stop - part.start)], vc[t[p], :max(0, part.stop - part.start)] = k[part], v[part]
+        want, mass = (w[:, :, None] * v.double()).sum(0), (w[:, :, None] * v.double().abs()).sum(0)
+        # the result's rounding, and two weights from scores that carry 130 roundings of fp32
+        bound = want.abs() * 2.0 ** -8 + mass * 2 * ((w * s.abs()).sum(0)[:, None] + 4) * 130 * 2.0 ** -24
+        wants.append((want, bound))
+        for kind, coarse in enumerate((w.bfloat16().double(), torch.softmax(s.bfloat16().double(), 0))):     # what the bound is to see: weights, scores of 16 bits
+            coarse = coarse / coarse.sum(0)
+            seen[kind] += bool((((coarse[:, :, None] * v.double()).sum(0) - want).abs() > bound).any())
+    assert min(seen) >= 4, seen
+    got = ops.attn_decode(q.cuda(), kc.cuda(), vc.cuda(), torch.tensor(ctxs, dtype=torch.int32).cuda(), tables.cuda(), scale, splits).cpu().double()
+    for i, (want, bound) in enumerate(wants):
+        err = (got[i].view(hkv, group, 128) - want[:, None]).abs()
+        assert (err <= bound[:, None]).all(), (ctxs[i], (err / bound[:, None]).max().item())
