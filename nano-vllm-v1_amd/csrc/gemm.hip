@@ -1384,9 +1384,12 @@ int tile_residents(Tile t) {
 // (k-tiles per slab + fixed part) x tile bytes x residents / fill rate, and a grid takes a whole number of rounds:
 // 320 workgroups on 256 slots cost two rounds.  Slabs add their write and the consumer's read.  It ranks the
 // measured split counts of the 14B projections at 256..1024 rows in the measured order.
-// It prices the tiles that pick_tile names, also where an unsplit product is launched with others (T64x64 and T128x64 in the launch below): with
-// those tiles' sizes in the model products of 33 .. 64 rows and K up to 1024 gain 5 .. 15 % (unsplit), but 300 .. 1000 rows lose 4 .. 32 %
-// (600 x 4096 x 5120 with its norm 43.5 -> 57.4 us): the model has no term for what eight waves on one tile hide.
+// It prices the tiles that pick_tile names, also where an unsplit product is launched with others (in the launch below T64x64, T128x64 over two rounds, T128x128
+// over a little more than one), and at one fill rate whether four waves share a tile or eight.  Other tiles' sizes in the model: products of 33 .. 64 rows and K
+// up to 1024 gain 5 .. 15 % (unsplit), but 300 .. 1000 rows lose 4 .. 32 % (600 x 4096 x 5120 with its norm 43.5 -> 57.4 us): it has no term for
+// what eight waves on one tile hide.  So it is no longer right everywhere; us with the add + norm behind, unsplit / as it says: 800 x 5120 x 5120 66.9 / 79.7 (3
+// slabs), x 17408 185 / 200 (3), 900 x 5120 x 17408 190 / 203 (3), 1016 x 5120 x 5120 70.4 / 71.8 (3), x 17408 201 / 171 (3), 400 x 5120 x 5120 49.4 / 44.2 (3),
+// 300 x 5120 x 5120 41.5 / 35.1 (2), 512 x 4096 x 4096 36.4 / 32.1 (2).  A count of slabs enters a result's bits, so it stays as it is until all are measured.
 double splitk_estimate_us(int64_t M, int64_t N, int64_t K, int s) {
     const Tile t = pick_tile(M, N, s);
     const int64_t wgs = nvh_cdiv(M, tile_bm(t)) * nvh_cdiv(N, tile_bn(t)) * s;
@@ -1586,20 +1589,23 @@ static int32_t dispatch_gemm(const GemmArgs& a) {
         }
         case T128x64:
             // One workgroup fits a CU, so a grid a little over 256 takes two rounds: then 128 x 128 tiles, fewer than 200 of them, in one round, eight
-            // waves each.  us before and now, 1024 x 3072 x 1024 19.5 and 11.7, 1000 x 2112 x 1024 19.3 and 14.4, 600 x 4096 x 1024 19.3 and 14.9,
-            // 1000 x 3072 x 768 16.7 and 12.7, 1024 x 3072 x 2048 32.3 and 25.4 (those but the first with four barriers a k-tile); one round of 128 x 64: 1024 x 2048 x 1024 11.0 against 13.9.  Two rounds elsewhere:
-            // 128 x 18992 x 5120 84.5 and 62.9, 1500 x 2048 x 17408 215 and 155, 1024 x 2560 x 5120 69 and 52, gate/up 512 x 6144 x 1024 19.9 and 15.4 (237
-            // sizes, 65 .. 4000 rows, N 560 .. 24000, K 256 .. 17408: 0.70 .. 0.82 of the time).  The same sums.
+            // waves each.  us, two rounds and this: 1024 x 3072 x 1024 19.9 and 12.4, 1000 x 2112 x 1024 19.4 and 11.4, 600 x 4096 x 1024 18.7 and 11.5, 1000 x
+            // 3072 x 768 16.3 and 10.2, 1024 x 3072 x 2048 31.5 and 21.4, 128 x 18992 x 5120 84.9 and 60.2, 1500 x 2048 x 17408 217 and 142, 1024 x 2560 x 5120
+            // 68.6 and 49.4, gate/up 512 x 6144 x 1024 19.8 and 14.6 (237 sizes, 65 .. 4000 rows, N 560 .. 24000, K 256 .. 17408, with four barriers a k-tile
+            // 0.70 .. 0.82 of the time).  One round of 128 x 64 against 128 x 128: 1024 x 2048 x 1024 11.3 and 11.8, 1000 x 2048 x 512 7.7 and 8.1, 1024 x 2048 x 5120
+            // 38.5 and 48.9.  The same sums.
             if (!tile_forced() && a.split_k == 1 && !a.qkv && !a.sample && nvh_cdiv(a.M, 128) * nvh_cdiv(a.N, 64) > 256) launch_gemm<128, 128, 2, 4, 3>(a);
             else launch_gemm<128, 64, 2, 2, 4>(a);
             break;
         case T128x128: {
             // up to one workgroup per CU: nothing shares the CU's LDS, so a third stage (96 KB) keeps two tiles in flight instead of one, and eight waves
-            // instead of four, two a SIMD, multiply and read at once (us, four waves and eight: 1024 x 4096 x 2048 27.0 and 23.5, x 4096 46.2 and 40.6;
-            // with the QKV epilogue, which walks 32 rows a pass, 1024 x 4096 x 1024 16.1 and 14.9 when each phase still had a barrier)
+            // instead of four, two a SIMD, multiply and read at once (us, four waves and eight: 1024 x 4096 x 1024 15.8 and 12.9, x 2048 26.4 and 21.2, x 4096 45.4
+            // and 38.9; with the QKV epilogue, which walks 32 rows a pass, 1024 x 4096 x 1024 21.8 and 18.1)
             const int64_t tm = nvh_cdiv(a.M, 128), tiles128 = tm * nvh_cdiv(a.N, 128) * a.split_k;
             if (tiles128 <= 256) {
-                const bool scaled_long = a.rowscale.sumsq != nullptr && a.K / a.split_k > 1536;     // (row scales over more than one norm's width: refused)
+                // (row scales come in pairs, this projection's and gate/up's, and the latter's tile, below, serves K up to 1536: beyond it neither is offered.  What
+                // the epilogue itself holds is 32 partial sums a row, which the entry points check.)
+                const bool scaled_long = a.rowscale.sumsq != nullptr && a.K / a.split_k > 1536;
                 if (!a.swiglu && !scaled_long && !nvh_switch_on(SW_QKV_NO_8WAVE)) launch_gemm<128, 128, 2, 4, 3>(a);
                 else launch_gemm<128, 128, 2, 2, 3>(a);
             }

@@ -503,8 +503,8 @@ __device__ __forceinline__ void wait_steps_in_flight(int ahead) {
 // same order, bit for bit the same results.
 // us at 16 experts, the general 64 x 64 tiles, the tiles for few rows below and this one, rows an expert x N x K: 126 x 1536 x 1024 35.0, 24.2,
 // 25.3; 250 x 1536 x 1024 51.5, 38.4, 35.1 (360 TFLOP/s); 250 x 1024 x 768 32.9, 21.5, 19.0; 500 x 1536 x 1024 85, 65, 49; 126 x 1024 x 384
-// 17.2, 9.4, 12.3.  Tried and slower at these sizes: eight waves and three stages with one workgroup a CU (a grid is seldom whole rounds),
-// stages of 32 k four ahead.
+// 17.2, 9.4, 12.3.  Tried and slower at these sizes: eight waves and three stages with one workgroup a CU (a grid is seldom whole rounds;
+// with four barriers a k-tile, as the dense products' eight waves were then: their loop of one barrier has not been tried here), stages of 32 k four ahead.
 constexpr int TALL = 128;
 
 // Whether tile `t` of the list goes on where tile t - 1, a full one, of the same expert ends.
