@@ -125,8 +125,11 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         __builtin_amdgcn_sched_barrier(0);
     }
     // From four query heads a kv head on the scores come from the matrix cores (16x16x32: 16 keys by up to four heads, four instructions) instead of a dot
-    // product and a row sum a key and head: a trip's vector instructions halve.  us a launch, 8 kv heads, before and now: 4 heads each, 30 sequences of
-    // 64..2000 keys 45.6 and 36.2; 5 heads, 8 of 3000..4000 98 and 74; 8 heads, 20 of 64..2000 84 and 54.  With 1 and 2 heads long contexts are bound by
+    // product and a row sum a key and head: a trip's vector instructions halve.  us of a call with the ranges and the merge that it takes, 8 kv heads, by dot
+    // products and now: 4 heads each, 30 sequences of 64..2000 keys 39.1 and 34.2; 5 heads, 8 of 3000..4000 36.0 and 30.1; 8 heads, 20 of 64..2000 55.4 and
+    // 40.3.  The four instructions' sums meet in pairs: each onto the one before, a score is rounded four times at its full size, and the weights' error (2-norm,
+    // two keys of scores near 16) was 7.2e-7 where dot products give 4.9e-7; in pairs it is 4.9e-7, for up to 3 % of the time with 8 heads (20 of 64..2000 39.5 and
+    // 40.3) and none with 4 (34.1 and 34.2).  With 1 and 2 heads long contexts are bound by
     // the keys' way to the CU either way (24 of 100..2047 30.9 and 31.2) and many workgroups lose by the registers (256 sequences 208 and 224).
     constexpr bool MFMA = G >= 4;
     constexpr int SETS = MFMA ? (G + 3) / 4 : 1;
@@ -242,9 +245,10 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
             f32x4 d[SETS];
 #pragma unroll
             for (int h = 0; h < SETS; ++h) {
-                d[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+                f32x4 part[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) d[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[h][i], __builtin_bit_cast(bf16x8, kt[i]), d[h], 0, 0, 0);
+                for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[h][i], __builtin_bit_cast(bf16x8, kt[i]), f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                d[h] = (part[0] + part[1]) + (part[2] + part[3]);
             }
 #pragma unroll
             for (int g = 0; g < G; ++g) {

@@ -96,3 +96,35 @@ def test_weights_in_fp32(group, splits):
     for i, (want, bound) in enumerate(wants):
         err = (got[i].view(hkv, group, 128) - want[:, None]).abs()
         assert (err <= bound[:, None]).all(), (ctxs[i], (err / bound[:, None]).max().item())
+
+
+def ulp(x):
+    return torch.exp2(torch.floor(torch.log2(x.abs())) - 23)
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 5, 8])
+def test_scores_are_summed_in_pairs(group):
+    """A score's 128 products add up by halves: over many pairs of keys the weights' 2-norm error is what the roundings of such a sum and of the scaled score leave.
+    (A running sum in four steps, each rounded at up to its full size, has 1.5 times that.)"""
+    from nanovllm import ops
+    hkv, hq, scale, b = 2, 2 * group, 128 ** -0.5, 600
+    g = torch.Generator().manual_seed(group)
+    u = (torch.randn(b, hkv, 128, generator=g) * 1.2).bfloat16()
+    k = (u.float()[:, None] * (0.9 + 0.1 * torch.rand(b, 2, hkv, 1, generator=g))).bfloat16()
+    d = (k.double() * u.double()[:, None]).sum(-1)           # [b, 2, hkv], some 175
+    w = torch.softmax(d * scale, 1)
+    v = torch.randn(b, 2, hkv, 128, generator=g).bfloat16()
+    v[:, 1] = (-v[:, 0].double() * (w[:, 0] / w[:, 1])[..., None]).bfloat16()          # the values nearly cancel: what is left shows the weights
+    kc = torch.zeros(b, 256, hkv, 128, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros_like(kc)
+    kc[:, :2], vc[:, :2] = k.cuda(), v.cuda()
+    q = u[:, :, None].expand(b, hkv, group, 128).reshape(b, hq, 128).contiguous()
+    got = ops.attn_decode(q.cuda(), kc, vc, torch.full((b,), 2, dtype=torch.int32).cuda(), torch.arange(b).int().view(b, 1).cuda(), scale, 1).cpu().double().view(b, hkv, group, 128)
+    want, mass = (w[..., None] * v.double()).sum(1), (w[..., None] * v.double().abs()).sum(1)
+    # (where the result itself is rounded at below 2^-23 of the mass)
+    err = ((got - want[:, :, None]) / mass[:, :, None])[(want.abs() < mass * 2.0 ** -14)[:, :, None].expand(-1, -1, group, -1)]
+    # variances in units of log2: the product with the scale, then 1, 2, 4 and 8 sums of halves, quarters ..; the result moves by half of the scores' difference
+    log2e = 1.4426950408889634
+    var = ulp(d * scale * log2e) ** 2 + sum(2.0 ** j * (ulp(d / 2 ** j) * scale * log2e) ** 2 for j in range(4))
+    bound = ((var / 12).sum(1).mean() ** 0.5 / log2e / 2).item()
+    assert err.numel() > 3000 and (err ** 2).mean().item() ** 0.5 < 1.2 * bound, ((err ** 2).mean().item() ** 0.5, bound)
