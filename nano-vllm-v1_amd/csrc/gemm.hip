@@ -132,7 +132,9 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave % WAVES_N, wm = wave / WAVES_N;
     int bx, by, bz;
-    xcd_tile(xcd_strip, bx, by, bz);
+    // (tiles of fewer than 64 rows or columns are never launched in strips: without that code 2 x 3072 x 1024 takes 5.88 us instead of 5.96)
+    if constexpr (BM >= 64 && BN >= 64) xcd_tile(xcd_strip, bx, by, bz);
+    else bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     const int n0 = bx * BN, m0 = by * BM;
     const int kbeg = bz * k_per_split;
     // QKV epilogue: the positions of this thread's tokens, requested before the main loop, so that the epilogue waits for
