@@ -388,7 +388,7 @@ def prefill_kernel_roofline(hf, tokens=1024, iters=3):
         out[name] = dict(us=round(us, 2), tflops=round(flops / us / 1e6, 1), frac=round(flops / us / 1e6 / MFMA_PEAK_TFLOPS, 4))
     dominant = max(out, key=lambda k: out[k]["us"])
     # matrix-pipe busy fraction of the kernels of a chunk as the step launches them (counter pass, tools/evidence_json.py)
-    pmc = ROOT / "profiles" / "r03_prefill_mfma_busy.json"
+    pmc = ROOT / "profiles" / "prefill_mfma_busy.json"
     busy = {k: v["mfma_busy_frac"] for k, v in json.loads(pmc.read_text()).items()} if pmc.exists() else None
     return dict(bound="mfma", kernel=dominant, achieved=out[dominant]["tflops"], peak=MFMA_PEAK_TFLOPS, unit="TFLOP/s",
                 frac=out[dominant]["frac"], per_kernel=out, per_layer_us=round(total_us, 1),
