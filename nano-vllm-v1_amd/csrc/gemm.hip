@@ -84,9 +84,10 @@ struct RowScale {
 };
 
 // Tile of this workgroup.  Workgroups go to the 8 XCDs round-robin by linear id.  With xcd_strip = 8 or 4 XCD i takes the i-th eighth of the tiles in an
-// order that walks strips of that many column tiles (the last one may be narrower) row by row, so the workgroups resident on an XCD at one time share
+// order that walks strips of that many column tiles (NARROW: the last one may be narrower) row by row, so the workgroups resident on an XCD at one time share
 // a few column tiles of W and a few row tiles of x in its L2 (Qwen3-14B shapes, 1024 rows: a prefill chunk 27.8 -> 27.15 ms; K = 1024: 2.81 -> 2.78 ms).
 // K-slabs (gridDim.z) count as further tile rows: slab z of row tile y is row y + gridDim.y * z.
+template <bool NARROW>
 __device__ __forceinline__ void xcd_tile(int xcd_strip, int& bx, int& by, int& bz) {
     bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     if (xcd_strip) {
@@ -94,20 +95,29 @@ __device__ __forceinline__ void xcd_tile(int xcd_strip, int& bx, int& by, int& b
         const int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), total = gridDim.x * rows;
         const int xcd = id & 7, nl = xcd * (total >> 3) + min(xcd, total & 7) + (id >> 3);
         const int sh = xcd_strip == 8 ? 3 : 2, per_strip = rows << sh;
-        const int strip = nl / per_strip, in = nl - strip * per_strip, width = min(xcd_strip, (int)gridDim.x - (strip << sh));
-        const int row = width == xcd_strip ? in >> sh : in / width;
-        bx = (strip << sh) + in - row * width;
+        const int strip = nl / per_strip, in = nl - strip * per_strip, width = (int)gridDim.x - (strip << sh);
+        int row = in >> sh, col = in & (xcd_strip - 1);
+        if (NARROW && width < xcd_strip) {
+            row = in / width;
+            col = in - row * width;
+        }
+        bx = (strip << sh) + col;
         bz = row / (int)gridDim.y;
         by = row - bz * (int)gridDim.y;
     }
 }
-// Strips for a grid: from 512 rows on (at 256 rows, a decode batch of 64-row tiles, the same order made a step 0.7 % slower); with a narrower last strip
-// where the grid is at most one workgroup a CU (800 x 5120 x 5120, 27 x 7 tiles: no strips and these 58.4 and 56.6 us; two rounds, 2000 x 5248 x 1024: 35.1 and 36.8).
-static int xcd_strip_of(const dim3& grid, int rows) {
+// Strips for a grid: from 512 rows on (at 256 rows, a decode batch of 64-row tiles, the same order made a step 0.7 % slower).  A grid whose width is no multiple of 4
+// takes strips with a narrower last one where it is at most one workgroup a CU (two rounds, 2000 x 5248 x 1024: 35.1 us without and 36.8 with) and the tile is
+// one of 128 rows or of two wave groups (64 x 64 of four waves: 512 x 800 x 1024 7.28 and 7.43, 1008 x 64 x 1024 6.58 and 6.90).  Of an odd width every XCD has
+// all columns otherwise: 800 x 5120 x 5120, 27 x 7 tiles, 58.4 and 56.6; two groups 832 x 1216 x 2048 13.1 and 10.0, 960 x 1088 x 1024 7.5 and 7.2.  Of twice an odd one
+// half of them, and only where a tile takes long: eight waves 1024 x 3840 x 1024 14.2 and 13.5, 1280 x 12800 x 5120 155 and 151; two groups 896 x 1152 x 2048 10.6
+// and 10.3, but x 1024 6.7 and 7.1; four waves on 128 x 64, 1024 x 1664 x 1024, 10.6 and 10.7.
+enum NarrowStrips { NONE, ODD_WIDTHS, ANY_WIDTH };
+static int xcd_strip_of(const dim3& grid, int rows, NarrowStrips narrow) {
     if (nvh_switch_on(SW_GEMM_NO_XCD) || grid.y * grid.z == 1 || rows < 512) return 0;             // (the switch is for measurements)
     if (grid.x % 8 == 0) return 8;
     if (grid.x % 4 == 0) return 4;
-    return (int64_t)grid.x * grid.y * grid.z <= 256 ? 8 : 0;
+    return (narrow == ANY_WIDTH || (narrow == ODD_WIDTHS && grid.x % 2 == 1)) && (int64_t)grid.x * grid.y * grid.z <= 256 ? 8 : 0;
 }
 
 template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES, bool NT_W, bool SWIGLU, bool QKV = false, bool SAMPLE = false, bool ROWSCALE = false>
@@ -133,7 +143,7 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
     const int wn = wave % WAVES_N, wm = wave / WAVES_N;
     int bx, by, bz;
     // (tiles of fewer than 64 rows or columns are never launched in strips: without that code 2 x 3072 x 1024 takes 5.88 us instead of 5.96)
-    if constexpr (BM >= 64 && BN >= 64) xcd_tile(xcd_strip, bx, by, bz);
+    if constexpr (BM >= 64 && BN >= 64) xcd_tile<(BM >= 128)>(xcd_strip, bx, by, bz);
     else bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
     const int n0 = bx * BN, m0 = by * BM;
     const int kbeg = bz * k_per_split;
@@ -665,7 +675,7 @@ __global__ __launch_bounds__(512) void gemm_kgroups_bf16_nt_kernel(const bf16* _
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, w4 = wave & 3, wn = w4 & 1, wm = w4 >> 1;
     int bx, by, bz;
-    xcd_tile(xcd_strip, bx, by, bz);
+    xcd_tile<true>(xcd_strip, bx, by, bz);
     const int n0 = bx * BN, m0 = by * BM;
     const int nstages = K / (2 * BK);
     const int dma_r = lane >> 3, dma_pos = lane & 7;
@@ -1281,7 +1291,7 @@ void launch_gemm_nt(const GemmArgs& a) {
     const int k_per_split = (int)nvh_cdiv(ktiles, a.split_k) * BK;
     dim3 grid((unsigned)nvh_cdiv(a.N, BN), (unsigned)nvh_cdiv(a.M, BM), (unsigned)a.split_k);
     kern<<<grid, 64 * WAVES_N * WAVES_M, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.partials, a.M, a.N, a.K, k_per_split,
-                                                       a.qkv ? *a.qkv : QkvEpilogue{}, wide, a.sample ? *a.sample : SampleEpilogue{}, xcd_strip_of(grid, a.M), a.rowscale);
+                                                       a.qkv ? *a.qkv : QkvEpilogue{}, wide, a.sample ? *a.sample : SampleEpilogue{}, xcd_strip_of(grid, a.M, BM < 128 ? NONE : WAVES_N * WAVES_M == 8 ? ANY_WIDTH : ODD_WIDTHS), a.rowscale);
 }
 
 void launch_gemm_kgroups(const GemmArgs& a) {
@@ -1301,7 +1311,7 @@ void launch_gemm_kgroups(const GemmArgs& a) {
         return;
     }
     dim3 grid((unsigned)nvh_cdiv(a.N, 64), (unsigned)nvh_cdiv(a.M, 64), 1);
-    kern<<<grid, 512, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.M, a.N, a.K, xcd_strip_of(grid, a.M), a.residual, a.row_sumsq);
+    kern<<<grid, 512, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, a.M, a.N, a.K, xcd_strip_of(grid, a.M, a.K >= 1536 ? ANY_WIDTH : ODD_WIDTHS), a.residual, a.row_sumsq);
 }
 
 template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES>

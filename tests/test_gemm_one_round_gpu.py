@@ -35,6 +35,17 @@ def test_bits(m, n, tile, k):
     check(lambda: ops.linear(x, w, b), x, w, b)
 
 
+@pytest.mark.parametrize("m,n,k,tile", [(1000, 1852, 192, "128x64 waves 2x2"), (1024, 1664, 192, "128x64 waves 2x2"), (1280, 12800, 192, "256x256 waves 2x4"),
+                                        (1270, 13052, 192, "256x256 waves 2x4"), (700, 604, 192, "64x64 waves 2x2"), (1008, 64, 192, "64x64 waves 2x2")])
+def test_grids_of_odd_and_twice_odd_widths(m, n, k, tile):
+    """Tiles in strips of which the last is narrower (29, 50 and 51 tiles wide) and in the grid's own order (26, 10 and 1): each is computed, once."""
+    from nanovllm import ops
+    assert plan(m, n, k).startswith(f"tile {tile}")
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = ((torch.randn(s, generator=g) * 0.5).bfloat16().cuda() for s in ((m, k), (n, k)))
+    check(lambda: ops.linear(x, w), x, w, None)
+
+
 @pytest.mark.parametrize("m,n,k", [(1024, 8192, 1024), (1016, 7172, 1088), (769, 8188, 1152)])
 def test_tall_bits(m, n, k):
     from nanovllm import ops
@@ -79,7 +90,7 @@ def test_slabs(m, n, k, s):
         assert ((got[p].double() - a @ c.t().contiguous()).abs() <= a.abs() @ c.abs().t().contiguous() * per * 2.0 ** -24 + 1e-30).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (833, 1020, 1152), (1000, 964, 3072), (1000, 964, 3200)])
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 1024), (833, 1020, 1152), (1000, 964, 3072), (1000, 964, 3200), (832, 1216, 1024), (896, 1152, 1024), (896, 1152, 1536)])
 def test_two_groups(m, n, k):
     """64 x 64 tiles of two wave groups: stages requested behind the reads (K up to 3072) and ahead of them."""
     from nanovllm import ops
