@@ -34,9 +34,20 @@ struct DecodeItems {
     const int32_t *item_seq, *item_range, *seq_active, *seq_chunk;
     int batch;
     int max_ranges;
-    const int32_t* order;      // uniform grid: the sequence that blockIdx.z stands for (null: itself)
+    const NvhDecodePiece* pieces;  // pieces (common.h): the list
 };
 
+// PIECES: a decode step of sequences that are otherwise one range each (more than 16 with 8 kv heads).  One workgroup a sequence and head left 256 CUs to wait for
+// the longest context: a CU alone takes in a trip of 64 keys in 0.95 us whatever is asked for, 24 sequences of 100..2047 keys took 30.1 us where their bytes need
+// 16.7, and two workgroups on a CU share its rate, so more and shorter ranges dealt out as they come were slower still (512 keys each: 31).  The step's first
+// launch (elementwise.hip, embedding_pieces_kernel) therefore lays out a list of pieces, the same for every layer: sequences above one and a half times a CU's
+// share of all trips are cut, the pieces lie by length, and where the contexts are long (six trips a CU and more) a workgroup walks a chain of them (the longest,
+// then the shortest, ..), so that 256 workgroups, one a CU, end together.  Short contexts keep a workgroup a piece: on one CU several of them hide each other's
+// way to the first key (33 sequences of 64 keys: 1160 us a step either way, 1255 one at a time).  A cut sequence's last piece to finish merges it.  us a decode
+// step of the 28-layer model, before (the sequences longest first) and now: 18 sequences of 100..2047 keys 1593 and 1345, 24 of them 1625 and 1435, 40 2075 and
+// 1961, 64 2470 and 2283, 128 3945 and 3800, 256 6280 and 6245; 48 of 300..1500 2010 and 1855; 24 of 1040 1367 and 1366; 64 of 64..100 1235 and 1240.
+// Sequences above 1.0 and 1.25 shares cut: 24 of 1040 1517 for 1366.
+//
 // FUSED: `q` is the raw fused qkv row of the step's single new token per sequence.  The kernel applies the
 // q/k epilogue itself (per-head RMSNorm + RoPE, qknorm_rope_head) and writes the new token's K/V to their cache slot
 // (token ctx-1 of the sequence) before it walks the keys, so the separate norm/rope/store launch disappears from a decode step.
@@ -51,8 +62,10 @@ struct FusedQkv {
 __device__ __forceinline__ void merge_row_wave(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml, bf16* __restrict__ out,
                                                int num_splits, int64_t bh, int active, int lane);
 
-template <int G, bool FUSED>
-__global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
+__device__ __forceinline__ void merge_row_pieces(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml, bf16* __restrict__ out, int64_t bh, int active, int lane);
+
+template <int G, bool FUSED, bool PIECES = false>
+__global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decode_kernel(
     const bf16* __restrict__ q, int64_t q_stride, bf16* __restrict__ kc, bf16* __restrict__ vc,
     const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ tables, int64_t table_stride, int hkv,
     float scale_log2, bf16* __restrict__ out, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int min_range, DecodeItems items, FusedQkv fz,
@@ -66,8 +79,26 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15;
     const int rowid = w * 4 + (lane >> 4);
 
-    int split, b, num_splits, ctx, chunk, active;
-    if (items.item_seq) {                                    // work list
+    constexpr bool CHAINS = PIECES && G <= 4;                // (more heads: their registers would spill)
+    int at = blockIdx.z;
+    do {                                                     // (PIECES: a workgroup's pieces; otherwise once)
+    int split, b, num_splits, ctx, chunk, active, piece_start = 0, piece_end = 0, page = 0;
+    int64_t pos = 0;
+    if constexpr (PIECES) {
+        const NvhDecodePiece piece = items.pieces[at];
+        b = piece.seq & 0xffff;
+        if (b >= items.batch || (CHAINS && piece.follows && at == blockIdx.z)) return;   // block-uniform: none, or another workgroup's
+        at = piece.next;
+        split = piece.seq >> 16 & 0xff;
+        active = piece.seq >> 24;
+        num_splits = NVH_PIECE_RANGES;
+        piece_start = piece.start;
+        piece_end = piece.end;
+        ctx = piece.context;
+        page = piece.page;
+        pos = piece.position;
+        chunk = 0;
+    } else if (items.item_seq) {                             // work list
         b = items.item_seq[blockIdx.z];
         if (b < 0 || b >= items.batch) return;               // block-uniform: unused slot
         split = items.item_range[blockIdx.z];
@@ -81,25 +112,23 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         // transposed order - the 8 heads of a sequence side by side on one XCD, whole 2-KB token rows per XCD - measured
         // 6.49 ms against 6.29 ms per step of 256 sequences: not taken)
         split = blockIdx.x;
-        b = items.order ? items.order[blockIdx.z] : blockIdx.z;
+        b = blockIdx.z;
         num_splits = gridDim.x;
         ctx = ctx_lens[b];
         chunk = decode_range_keys(ctx, num_splits, min_range);
         active = ctx > 0 ? (ctx + chunk - 1) / chunk : 0;
     }
-    if (split >= max(active, 1)) return;                     // block-uniform: this range holds no key of the sequence
+    if (!PIECES && split >= max(active, 1)) return;          // block-uniform: this range holds no key of the sequence
     const bool final_here = active <= 1;                     // the whole sequence (or a padded row) is this workgroup's
-    const int start = split * chunk;
-    const int end = min(ctx, start + chunk);
+    const int start = PIECES ? piece_start : split * chunk;
+    const int end = PIECES ? piece_end : min(ctx, start + chunk);
 
     // Everything that this token brings is requested before the first keys are, and worked on behind that request.
     // The first page and the position together: one behind the other is one more latency in front of the first keys; and the new token's own key and value only
     // where the range ends with it.  us, mean of four runs each: 8 sequences of 500..1500 keys in 8 ranges 13.66 when the first keys came behind the epilogue,
     // 13.91 with the page behind the position and every range asking for the new token, 13.79 as it is; 4 in 16 ranges 11.40, 11.27 and 11.19.
     const int32_t* table = tables + (int64_t)b * table_stride;
-    int page = 0;
-    int64_t pos = 0;
-    if (start < end) {
+    if (!PIECES && start < end) {
         page = table[start >> 8];
         if constexpr (FUSED) pos = fz.positions[b];
     }
@@ -404,7 +433,8 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
             }
         }
     }
-    if (final_here || arrivals == nullptr) return;           // block-uniform
+    if (!PIECES && (final_here || arrivals == nullptr)) return;  // block-uniform
+    if (!PIECES || !final_here) {
     // The workgroup that finishes last among the `active` ranges of this (sequence, kv head) merges them - no second
     // launch.  Every storing wave drains its stores, one lane counts the arrival (agent-scope atomic), the last arriver
     // invalidates its CU's L1 (agent-scope acquire) before any wave of it reads the other workgroups' records, and puts
@@ -423,8 +453,15 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 2) void attn_decode_kernel(
         sm_last = last;
     }
     __syncthreads();
-    if (!sm_last) return;
-    for (int g = w; g < G; g += 4) merge_row_wave(ws_acc, ws_ml, out, num_splits, (int64_t)b * hq + kvh * G + g, active, lane);
+    if (sm_last) {
+        for (int g = w; g < G; g += 4) {
+            if constexpr (CHAINS) merge_row_pieces(ws_acc, ws_ml, out, (int64_t)b * hq + kvh * G + g, active, lane);
+            else merge_row_wave(ws_acc, ws_ml, out, num_splits, (int64_t)b * hq + kvh * G + g, active, lane);
+        }
+    }
+    }
+    if (CHAINS && at >= 0) __syncthreads();                  // the LDS is free again
+    } while (CHAINS && at >= 0);
 }
 
 // Merge per-range partials of one output row (sequence/token x query head).  Both kernels below compute the same
@@ -486,6 +523,33 @@ __device__ __forceinline__ void merge_row_wave(const float* __restrict__ ws_acc,
         }
     }
     L = wave_sum(L);
+    const float inv = L > 0.f ? 1.0f / L : 0.f;
+    const float a0 = (A[0][0] + A[1][0]) + (A[2][0] + A[3][0]), a1 = (A[0][1] + A[1][1]) + (A[2][1] + A[3][1]);
+    bf16x2 o = {f2bf(a0 * inv), f2bf(a1 * inv)};
+    *reinterpret_cast<bf16x2*>(out + bh * 128 + lane * 2) = o;
+}
+
+// The same sums for a row of at most NVH_PIECE_RANGES partial results: everything is requested at once (a range past the last repeats the last), one trip to memory.
+__device__ __forceinline__ void merge_row_pieces(const float* __restrict__ ws_acc, const float* __restrict__ ws_ml, bf16* __restrict__ out, int64_t bh, int active, int lane) {
+    const f32x2* ml = reinterpret_cast<const f32x2*>(ws_ml) + bh * NVH_PIECE_RANGES;
+    const f32x2* acc = reinterpret_cast<const f32x2*>(ws_acc + bh * NVH_PIECE_RANGES * 128) + lane;
+    f32x2 v[NVH_PIECE_RANGES];
+#pragma unroll
+    for (int k = 0; k < NVH_PIECE_RANGES; ++k) v[k] = acc[(int64_t)min(k, active - 1) * 64];
+    const f32x2 got = ml[min(lane, active - 1)];
+    const f32x2 rec = lane < active ? got : f32x2{-INFINITY, 0.f};
+    const float M = wave_max(rec[1] > 0.f ? rec[0] : -INFINITY);
+    const float wgt = rec[1] > 0.f ? __builtin_amdgcn_exp2f(rec[0] - (M == -INFINITY ? 0.f : M)) : 0.f;
+    const float L = wave_sum(rec[1] * wgt);
+    f32x2 A[4] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll
+    for (int k = 0; k < NVH_PIECE_RANGES; ++k) {
+        const float wk = __shfl(wgt, k, 64);
+        if (wk != 0.f) {                                         // wave-uniform
+            A[k & 3][0] += v[k][0] * wk;
+            A[k & 3][1] += v[k][1] * wk;
+        }
+    }
     const float inv = L > 0.f ? 1.0f / L : 0.f;
     const float a0 = (A[0][0] + A[1][0]) + (A[2][0] + A[3][0]), a1 = (A[0][1] + A[1][1]) + (A[2][1] + A[3][1]);
     bf16x2 o = {f2bf(a0 * inv), f2bf(a1 * inv)};
@@ -679,8 +743,9 @@ struct DecodeArgs {
     int32_t num_splits, min_range;
     void* workspace;
     hipStream_t st;
-    DecodeItems items;              // item_seq == nullptr: uniform grid
+    DecodeItems items;              // neither item_seq nor pieces: uniform grid
     int64_t num_items;
+    unsigned* arrivals = nullptr;   // pieces: the step's counters
 };
 
 template <bool FUSED>
@@ -707,6 +772,28 @@ int32_t launch_decode(const char* name, const DecodeArgs& a, const FusedQkv& fz)
         grid = dim3(1, (unsigned)a.num_kv_heads, (unsigned)a.num_items);
     }
     const float sl2 = a.softmax_scale * LOG2E;
+    if constexpr (FUSED) {
+        if (a.items.pieces) {
+            grid = dim3(1, (unsigned)a.num_kv_heads, (unsigned)a.num_items);
+#define LAUNCH_DEC(GG)                                                                                                                     \
+    attn_decode_kernel<GG, true, true><<<grid, 256, 0, a.st>>>((const bf16*)a.q, a.q_token_stride, (bf16*)a.k_cache, (bf16*)a.v_cache,     \
+                                                               a.context_lens, a.block_tables, a.table_stride, (int)a.num_kv_heads, sl2,    \
+                                                               (bf16*)a.out, ws_acc, ws_ml, min_range, a.items, fz, a.arrivals)
+            switch (g) {
+                case 1: LAUNCH_DEC(1); break;
+                case 2: LAUNCH_DEC(2); break;
+                case 4: LAUNCH_DEC(4); break;
+                case 5: LAUNCH_DEC(5); break;
+                case 8: LAUNCH_DEC(8); break;
+                default:
+                    nvh_set_error("%s: group size Hq/Hkv = %d unsupported (1,2,4,5,8)", name, g);
+                    return NVH_ENOSYS;
+            }
+#undef LAUNCH_DEC
+            NVH_CHECK_LAUNCH(name);
+            return NVH_OK;
+        }
+    }
     // NVH_DECODE_MERGE_IN_LAUNCH=1: key ranges are merged by the last workgroup to arrive instead of by a second launch
     // (same bits).  Off by default: measured on Qwen3-0.6B decode steps it loses at 1 sequence (1.286 ms against 1.170 ms
     // per step: the drain, the arrival atomic, the acquire and a merge by one workgroup cost more than the 4.7 us launch
@@ -814,21 +901,6 @@ extern "C" int32_t nvh_attn_decode_items(const void* q, int64_t q_token_stride, 
     return launch_decode<false>("nvh_attn_decode_items", a, FusedQkv{});
 }
 
-int32_t nvh_attn_decode_fused_qkv_ordered(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
-                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
-                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
-                                          int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys, void* workspace,
-                                          const int32_t* order, hipStream_t stream) {
-    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
-    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
-                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
-    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
-                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, stream, DecodeItems{}, 0};
-    a.items.order = order;
-    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
-                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
-}
-
 extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stride, const void* q_norm_weight,
                                              const void* k_norm_weight, float eps, const int64_t* positions,
                                              const float* cos_sin, void* k_cache, void* v_cache,
@@ -836,9 +908,30 @@ extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stri
                                              int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
                                              float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys,
                                              void* workspace, nvh_stream_t stream) {
-    return nvh_attn_decode_fused_qkv_ordered(qkv, token_stride, q_norm_weight, k_norm_weight, eps, positions, cos_sin, k_cache, v_cache, context_lens,
-                                             block_tables, table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, num_splits,
-                                             min_range_keys, workspace, nullptr, (hipStream_t)stream);
+    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
+    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
+                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
+    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
+                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, (hipStream_t)stream, DecodeItems{}, 0};
+    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
+                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
+}
+
+int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                         const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
+                                         const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                         int64_t head_dim, float softmax_scale, void* out, void* workspace, const NvhDecodePieces& pieces, hipStream_t stream) {
+    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin && pieces.pieces && pieces.arrivals, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
+    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
+                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
+    NVH_REQUIRE(num_kv_heads > 0 && batch <= NVH_PIECE_ROWS && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
+                "nvh_attn_decode_fused_qkv: %ld sequences in %d pieces", (long)batch, pieces.capacity);
+    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
+                 num_kv_heads, head_dim, softmax_scale, out, NVH_PIECE_RANGES, 0, workspace, stream, DecodeItems{}, pieces.capacity, pieces.arrivals};
+    a.items.batch = (int)batch;
+    a.items.pieces = pieces.pieces;
+    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
+                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }
 
 extern "C" int32_t nvh_attn_decode_fused_qkv_items(const void* qkv, int64_t token_stride, const void* q_norm_weight,

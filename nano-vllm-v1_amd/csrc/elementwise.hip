@@ -570,22 +570,64 @@ extern "C" int32_t nvh_embedding(const int64_t* ids, const void* table, void* ou
     return NVH_OK;
 }
 
-// The same launch with one workgroup more, which leaves the sequences of a decode batch in order of their context lengths, the longest
-// first (ties by index): order[rank] = sequence.  A sequence's rank is the number of sequences in front of it, counted from LDS - about
-// 1 us for 512 sequences, beside the rows' copies.
-__global__ __launch_bounds__(256) void embedding_order_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ table, bf16* __restrict__ out, int dim,
-                                                              int64_t vstart, int64_t vrows, const int32_t* __restrict__ ctx_lens,
-                                                              int32_t* __restrict__ order, int batch) {
-    __shared__ int32_t len[NVH_ORDER_MAX];
+// nvh_embedding with one workgroup more, which lays out the pieces of the step's decode attention (attention_decode.hip, PIECES): how long a piece may be
+// follows from the sum of all contexts and where a sequence is cut from that and its own length, so the order that sequences come in changes no bit of a result.
+// Pieces are put in order of their length by counting (one place a length in trips; equal ones as the counters deal them out, which decides where they run).
+__global__ __launch_bounds__(256) void embedding_pieces_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ table, bf16* __restrict__ out, int dim,
+                                                               int64_t vstart, int64_t vrows, const int32_t* __restrict__ ctx_lens, const int64_t* __restrict__ positions,
+                                                               const int32_t* __restrict__ tables, int64_t table_stride, int batch, int per_head, int hkv, bool may_chain,
+                                                               NvhDecodePieces pl) {
+    __shared__ int count[64], place[64], total, pieces;
     if (blockIdx.x == 0) {
-        for (int i = threadIdx.x; i < batch; i += 256) len[i] = ctx_lens[i];
+        const int tid = threadIdx.x;
+        if (tid < 64) count[tid] = 0;
+        if (tid == 0) total = 0;
         __syncthreads();
-        for (int i = threadIdx.x; i < batch; i += 256) {
-            const int mine = len[i];
-            int rank = 0;
-            for (int j = 0; j < batch; ++j) rank += len[j] > mine || (len[j] == mine && j < i);
-            order[rank] = i;
+        for (int i = tid; i < batch; i += 256) atomicAdd(&total, (max(ctx_lens[i], 0) + 63) >> 6);
+        for (int i = tid; i < batch * hkv; i += 256) pl.arrivals[i] = 0u;
+        __syncthreads();
+        const bool chains = may_chain && pl.capacity > batch && total >= NVH_CHAIN_TRIPS * per_head;
+        int most = max((int)(((int64_t)total * 3 / 2 + per_head - 1) / per_head), NVH_PIECE_TRIPS);   // trips of a piece
+        if (pl.capacity == batch) most = 1 << 26;            // (no context is longer)
+        auto pieces_of = [&](int trips) {
+            const int each = max(most, (trips + NVH_PIECE_RANGES - 1) / NVH_PIECE_RANGES);
+            return max((trips + each - 1) / each, 1);
+        };
+        for (;;) {                                           // (ends: at 2^26 trips nothing is cut)
+            if (tid == 0) pieces = 0;
+            __syncthreads();
+            for (int i = tid; i < batch; i += 256) atomicAdd(&pieces, pieces_of((max(ctx_lens[i], 0) + 63) >> 6));
+            __syncthreads();
+            const int n = pieces;
+            __syncthreads();
+            if (n <= pl.capacity || most >= 1 << 26) break;
+            most += (most + 3) >> 2;
         }
+        for (int pass = 0; pass < 2; ++pass) {
+            for (int i = tid; i < batch; i += 256) {
+                const int ctx = max(ctx_lens[i], 0), trips = (ctx + 63) >> 6, n = pieces_of(trips);
+                for (int k = 0; k < n; ++k) {
+                    const int lo = (int)((int64_t)trips * k / n), hi = (int)((int64_t)trips * (k + 1) / n), bin = min(hi - lo, 63);
+                    if (pass == 0) {
+                        atomicAdd(&count[bin], 1);
+                    } else {
+                        const int at = atomicAdd(&place[bin], 1), next = (at / per_head + 2) * per_head - 1 - at % per_head;
+                        pl.pieces[at] = {i | k << 16 | n << 24, lo * 64, min(hi * 64, ctx), ctx, trips ? tables[i * table_stride + (lo >> 2)] : 0, (int)positions[i],
+                                         chains && next < pieces ? next : -1, chains && at >= per_head};
+                    }
+                }
+            }
+            __syncthreads();
+            if (pass == 0) {
+                int before = 0;
+                if (tid < 64) {
+                    for (int b = tid + 1; b < 64; ++b) before += count[b];
+                    place[tid] = before;
+                }
+                __syncthreads();
+            }
+        }
+        for (int i = pieces + tid; i < pl.capacity; i += 256) pl.pieces[i] = {0xffff, 0, 0, 0, 0, 0, -1, 0};
         return;
     }
     const int64_t t = blockIdx.x - 1;
@@ -599,12 +641,17 @@ __global__ __launch_bounds__(256) void embedding_order_kernel(const int64_t* __r
     }
 }
 
-int32_t nvh_embedding_order(const int64_t* ids, const void* table, void* out, int64_t num_tokens, int64_t dim, int64_t vocab_start, int64_t vocab_rows,
-                            const int32_t* context_lens, int32_t* order, int64_t batch, hipStream_t st) {
-    NVH_REQUIRE(ids && table && out && context_lens && order, NVH_EINVAL, "nvh_embedding: null pointer");
+int32_t nvh_embedding_pieces(const int64_t* ids, const void* table, void* out, int64_t num_tokens, int64_t dim, int64_t vocab_start, int64_t vocab_rows,
+                             const int32_t* context_lens, const int64_t* positions, const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads,
+                             int64_t num_kv_heads, const NvhDecodePieces& pieces, hipStream_t st) {
+    NVH_REQUIRE(ids && table && out && context_lens && positions && block_tables && pieces.pieces && pieces.arrivals, NVH_EINVAL, "nvh_embedding: null pointer");
     NVH_REQUIRE(dim > 0 && dim % 8 == 0 && nvh_aligned16(table) && nvh_aligned16(out), NVH_EINVAL, "nvh_embedding: dim %% 8 and 16-byte alignment required");
-    NVH_REQUIRE(batch >= 0 && batch <= NVH_ORDER_MAX, NVH_EINVAL, "nvh_embedding: %ld sequences to order (at most %d)", (long)batch, NVH_ORDER_MAX);
-    embedding_order_kernel<<<(unsigned)num_tokens + 1, 256, 0, st>>>(ids, (const bf16*)table, (bf16*)out, (int)dim, vocab_start, vocab_rows, context_lens, order, (int)batch);
+    const int per_head = nvh_pieces_per_head(num_kv_heads);
+    NVH_REQUIRE(batch >= 0 && batch <= NVH_PIECE_ROWS && num_kv_heads > 0 && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
+                "nvh_embedding: %ld sequences in %d pieces a head", (long)batch, pieces.capacity);
+    // (chains: up to four query heads a kv head, attn_decode_kernel)
+    embedding_pieces_kernel<<<(unsigned)num_tokens + 1, 256, 0, st>>>(ids, (const bf16*)table, (bf16*)out, (int)dim, vocab_start, vocab_rows, context_lens, positions,
+                                                                      block_tables, table_stride, (int)batch, per_head, (int)num_kv_heads, num_q_heads <= 4 * num_kv_heads, pieces);
     NVH_CHECK_LAUNCH("embedding");
     return NVH_OK;
 }
