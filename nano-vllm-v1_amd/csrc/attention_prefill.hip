@@ -608,11 +608,11 @@ extern "C" int64_t nvh_attn_varlen_workspace_bytes(int64_t total_q, int64_t num_
     return total_q * num_q_heads * num_splits * (head_dim + 2) * (int64_t)sizeof(float);
 }
 
-extern "C" int32_t nvh_attn_varlen(const void* q, int64_t q_token_stride, const void* k, const void* v,
+int32_t nvh_attn_varlen_beside(const void* q, int64_t q_token_stride, const void* k, const void* v,
                                    int64_t kv_token_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                                    const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t max_seqlen_q,
                                    int64_t max_seqlen_k, int64_t total_q, int64_t num_q_heads, int64_t num_kv_heads,
-                                   int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, void* workspace,
+                                   int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, void* workspace, bool beside,
                                    nvh_stream_t stream) {
     NVH_REQUIRE(q && k && v && cu_seqlens_q && cu_seqlens_k && out, NVH_EINVAL, "nvh_attn_varlen: null pointer");
     NVH_REQUIRE(head_dim == 128, NVH_ENOSYS, "nvh_attn_varlen: head_dim %ld unsupported (128 only)", (long)head_dim);
@@ -655,8 +655,11 @@ extern "C" int32_t nvh_attn_varlen(const void* q, int64_t q_token_stride, const 
         // change: the loop is bound by instruction issue, not by the DMA latency)
         case 2: {
             // a grid that leaves half the CUs without a workgroup (one 1024-token chunk: 16 blocks x 8 kv heads): 32-row
-            // blocks put a four-wave workgroup on every CU instead of an eight-wave one on every other
-            const int rb1 = (int)nvh_switch_or(SW_ATTN_RB1, 128);     // A/B switch: 0 = never
+            // blocks put a four-wave workgroup on every CU instead of an eight-wave one on every other (alone: 1024 queries and keys 21.5 us for 24.6,
+            // 924 queries of 1948 keys 36 for 38).  Not in a mixed step with another step in flight: a workgroup takes a CU's LDS whole either way, and
+            // half as many leave the other CUs to that step's decode attention and products (three steps of 924 new tokens and 100 decodes in flight
+            // 3940 -> 3555 us a step; steps of a chunk alone 2112 and 2126, no gain).  A row's bits are the same.
+            const int rb1 = beside ? 0 : (int)nvh_switch_or(SW_ATTN_RB1, 128);     // A/B switch: 0 = never
             if (ks == 2 && wgs <= rb1) LAUNCH_VL(2, 1, 2, 2);
             else if (ks == 2) LAUNCH_VL(2, 2, 2, 2);
             else LAUNCH_VL(2, 2, 1, 2);
@@ -675,4 +678,14 @@ extern "C" int32_t nvh_attn_varlen(const void* q, int64_t q_token_stride, const 
         return nvh_launch_attn_combine(ws_acc, ws_ml, out, total_q * num_q_heads, num_splits, nullptr, 1, 64, nullptr, st);   // same records as decode
     }
     return NVH_OK;
+}
+
+extern "C" int32_t nvh_attn_varlen(const void* q, int64_t q_token_stride, const void* k, const void* v,
+                                   int64_t kv_token_stride, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                   const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t max_seqlen_q,
+                                   int64_t max_seqlen_k, int64_t total_q, int64_t num_q_heads, int64_t num_kv_heads,
+                                   int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, void* workspace,
+                                   nvh_stream_t stream) {
+    return nvh_attn_varlen_beside(q, q_token_stride, k, v, kv_token_stride, cu_seqlens_q, cu_seqlens_k, block_tables, table_stride, batch, max_seqlen_q,
+                                  max_seqlen_k, total_q, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, num_splits, workspace, false, stream);
 }

@@ -98,6 +98,12 @@ int32_t nvh_embedding_pieces(const int64_t* ids, const void* table, void* out, i
                              const int32_t* context_lens, const int64_t* positions, const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads,
                              int64_t num_kv_heads, const NvhDecodePieces& pieces, hipStream_t st);
 
+// nvh_attn_varlen, and whether another step's launches run beside it (attention_prefill.hip).
+int32_t nvh_attn_varlen_beside(const void* q, int64_t q_token_stride, const void* k, const void* v, int64_t kv_token_stride, const int32_t* cu_seqlens_q,
+                               const int32_t* cu_seqlens_k, const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t max_seqlen_q,
+                               int64_t max_seqlen_k, int64_t total_q, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, float softmax_scale,
+                               void* out, int32_t num_splits, void* workspace, bool beside, nvh_stream_t stream);
+
 // Routing and measurement switches.  Every kernel choice in this library is a pure function of the call's shapes; the
 // switches below exist for A/B measurements and for tests that compare two routes.  They are read from the environment
 // (variable NVH_<name>) ONCE per process, and only when NVH_TUNING=1 is set, so that a stray variable in a user's

@@ -295,9 +295,9 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
                 // (the qk-norm / rope / store launch above covered only the tokens past the one-token sequences)
                 FWD(decode_attention(md, st, l, w.qkv, qkv_n, kc, vc, prefix, scale, w.attn, dsplits, w.decode_ws, pieces, stream));
                 if (b > prefix)
-                    FWD(nvh_attn_varlen(w.qkv + prefix * qkv_n, qkv_n, kc, vc, kvsz, st->cu_seqlens_q_tail, st->cu_seqlens_k_tail,
+                    FWD(nvh_attn_varlen_beside(w.qkv + prefix * qkv_n, qkv_n, kc, vc, kvsz, st->cu_seqlens_q_tail, st->cu_seqlens_k_tail,
                                         st->block_tables + prefix * st->table_stride, st->table_stride, b - prefix, st->max_seqlen_q,
-                                        st->max_seqlen_k, t - prefix, hq, hkv, d, scale, w.attn + prefix * qsz, vsplits, w.varlen_ws, stream));
+                                        st->max_seqlen_k, t - prefix, hq, hkv, d, scale, w.attn + prefix * qsz, vsplits, w.varlen_ws, ev_wait != nullptr, stream));
             } else if (st->mode == NVH_MODE_PAGED) {
                 FWD(nvh_attn_varlen(w.qkv, qkv_n, kc, vc, kvsz, st->cu_seqlens_q, st->cu_seqlens_k, st->block_tables,
                                     st->table_stride, b, st->max_seqlen_q, st->max_seqlen_k, t, hq, hkv, d, scale, w.attn, vsplits, w.varlen_ws, stream));
