@@ -128,10 +128,14 @@ class _Staging:
         dev.copy_(self.host[:n], non_blocking=True)
         if self.event is not None:
             self.event.record()
-        out = {}
+        out, typed = {}, {}
         for name, a in arrays.items():
-            view = dev[offs[name]:offs[name] + a.nbytes].view(_TORCH_DTYPE[a.dtype.type])
-            out[name] = view.view(a.shape)
+            kind = a.dtype.type
+            if kind not in typed:
+                typed[kind] = dev.view(_TORCH_DTYPE[kind])           # (n is a multiple of 16, as every offset)
+            at = offs[name] // a.itemsize
+            view = typed[kind][at:at + a.size]
+            out[name] = view if a.ndim == 1 else view.view(a.shape)
         return out
 
 
@@ -191,6 +195,7 @@ class ModelRunner:
         # alternate between the caller's stream and a side stream (Qwen3-0.6B: a 1024-token chunk 2.77 -> 2.18 ms; the
         # Qwen3-14B shape 27.7 -> 26.4 ms).  NANOVLLM_STEP_OVERLAP=0 turns it off.
         self.step_overlap = self.world_size == 1 and os.environ.get("NANOVLLM_STEP_OVERLAP", "1") != "0"
+        self._stream_object = None
         self._side_streams = []                 # created with the first steps that take them
         self._last_step = None                  # lane, completion event and event set of the step launched last
         self._lane_done = {}                    # side lane -> completion event of the last step launched on it
@@ -480,6 +485,10 @@ class ModelRunner:
             arrays["state_slots"] = np.fromiter((s.state_slot for s in seqs), dtype=np.int32, count=len(seqs))
         if fb.get("logit_rows") is not None:
             arrays["logit_rows"] = fb["logit_rows"]
+        elif hasattr(self.model, "gather_rows"):
+            # the last row of every sequence that ends its scheduled tokens here (all sequences when none owns pages)
+            cu = fb["cu_seqlens_q"]
+            arrays["last_rows"] = np.ascontiguousarray((cu[1:][fb["need"]] if fb["need"].size else cu[1:]) - 1, dtype=np.int32)
         if self.rank == 0 or self.shard_sampling:
             temps = np.fromiter((s.temperature for s in seqs), dtype=np.float32, count=len(seqs))
             arrays["temperatures"] = temps[fb["need"]] if fb["need"].size else temps
@@ -518,6 +527,7 @@ class ModelRunner:
         set_context(d["cu_seqlens_q"], d["cu_seqlens_k"], fb["max_seqlen_q"], fb["max_seqlen_k"], d["slot_mapping"],
                     d["context_lens"], d.get("block_tables"), d["need"], d.get("state_slots"))
         fb["logit_rows_dev"] = d.get("logit_rows")
+        fb["last_rows_dev"] = d.get("last_rows")
         return d["input_ids"], d["positions"], d.get("temperatures"), fb
 
     # -------------------------------------------------------------- forward
@@ -609,6 +619,13 @@ class ModelRunner:
             return None
         return graph
 
+    def _current_stream(self):
+        """torch.cuda.current_stream(), whose object is made anew (4 us) only where the stream is another one than last time."""
+        device, last = torch._C._cuda_getDevice(), self._stream_object
+        if last is None or last.device.index != device or last.cuda_stream != torch._C._cuda_getCurrentRawStream(device):
+            last = self._stream_object = torch.cuda.current_stream()
+        return last
+
     OVERLAP_MIN_TOKENS = 256     # steps with fewer new tokens are not worth another stream
     # streams that consecutive prefill-sized steps rotate over (the caller's + side streams).  Measured on Qwen3-0.6B / the 14B
     # shape, 1024-token chunks: 2 lanes 2.19 / 27.1 ms per chunk, 3 lanes 2.11 / 25.2, 4 lanes 2.15 / 25.2, 8 lanes 2.13; an
@@ -663,7 +680,7 @@ class ModelRunner:
             if last is not None and last["record"]:
                 lane, wait, record = (last["lane"] + 1) % self.LANES, last["record"], 3 - last["record"]
         fb["layer_events"] = (wait, record)
-        main = torch.cuda.current_stream()
+        main = self._current_stream()
         while lane > len(self._side_streams):
             self._side_streams.append(torch.cuda.Stream(device=self.device))
         stream = self._side_streams[lane - 1] if lane else main
@@ -674,7 +691,7 @@ class ModelRunner:
             self._lane_done.clear()
         self._step_depth, self._step_fb = 1, fb
         try:
-            with torch.cuda.stream(stream):
+            with torch.cuda.stream(stream) if lane else contextlib.nullcontext():
                 yield fb
                 done = torch.cuda.Event()
                 done.record(stream)
@@ -712,11 +729,7 @@ class ModelRunner:
             elif fb["need"].size == 0 and any(len(s.block_table) for s in seqs):
                 out = (hidden, None, None, 0, temps, need_host)
             elif hasattr(self.model, "gather_rows"):
-                # the last row of every sequence that ends its scheduled tokens here (all sequences when none owns pages)
-                cu = fb["cu_seqlens_q"]
-                last = (cu[1:][fb["need"]] if fb["need"].size else cu[1:]) - 1
-                idx = torch.from_numpy(np.ascontiguousarray(last, dtype=np.int32)).to(self.device, non_blocking=True)
-                rows = self.model.gather_rows(hidden, idx)
+                rows = self.model.gather_rows(hidden, fb["last_rows_dev"])
                 out = (rows, None, None, rows.shape[0], temps, need_host)
             elif self.native is not None:
                 out = (hidden, ctx.cu_seqlens_q, ctx.seq_need_compute_logits if fb["need"].size else None,
