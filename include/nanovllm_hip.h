@@ -685,6 +685,11 @@ int32_t nvh_act_mul(const void* x, int64_t row_stride, void* y, int64_t y_stride
 /* y = xIELU(x) with params = (p, q) of type A, in fp32: z > 0: softplus(p) z^2 + z / 2; else (1/2 + softplus(q)) (e^z - 1 - z) + z / 2. */
 int32_t nvh_xielu(const void* x, int64_t row_stride, void* y, int64_t y_stride, int64_t rows, int64_t inter, const void* params, int32_t act_f32,
                   nvh_stream_t stream);
+/* y = act(bf16(x W^T + bias)) for up to 64 rows in one launch, the bits of nvh_gemm_bf16_nt followed by nvh_act_mul / nvh_xielu; act 2: squared
+ * relu, 3: xIELU with params = (p, q) in bf16.  NVH_ENOSYS where nvh_gemm_act_supported() is 0 (the sizes then take two launches). */
+int32_t nvh_gemm_act_supported(int64_t M, int64_t N, int64_t K);
+int32_t nvh_gemm_act_bf16_nt(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* y, int64_t y_row_stride, int64_t M, int64_t N,
+                             int64_t K, int32_t act, const void* params, nvh_stream_t stream);
 /* out fp32 [rows, vocab] = scale * logits, softcapped when cap > 0. */
 int32_t nvh_logits_scale(const void* logits, int64_t row_stride, float* out, int64_t rows, int64_t vocab, float scale, float cap,
                          int32_t act_f32, nvh_stream_t stream);

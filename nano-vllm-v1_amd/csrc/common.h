@@ -251,6 +251,16 @@ __device__ __forceinline__ float nvh_activation(float g, int act) {
     return g > 0.f ? g * g : 0.f;
 }
 
+// xIELU of bf16 rows (stream_f32.hip and, inside a product, gemm.hip): pos = softplus(p), neg = 1/2 + softplus(q).  The hardware's 2^x and log2: errors of about
+// 1e-7 beside values of at least softplus' own size.
+__device__ __forceinline__ float nvh_softplus_hw(float t) {
+    return fmaxf(t, 0.f) + 0.6931471805599453f * __builtin_amdgcn_logf(1.0f + __builtin_amdgcn_exp2f(-fabsf(t) * 1.4426950408889634f));
+}
+__device__ __forceinline__ float nvh_xielu_hw(float z, float pos, float neg) {
+    const float zn = fminf(z, 0.f);
+    return (z > 0.f ? pos * z * z : neg * ((__builtin_amdgcn_exp2f(zn * 1.4426950408889634f) - 1.0f) - z)) + 0.5f * z;
+}
+
 // Elementwise launches over rows of `cols` columns: a lane (256 a workgroup) takes E consecutive columns, cols a multiple of E.  False: past the end.
 template <int E>
 __device__ __forceinline__ bool nvh_piece(int64_t rows, int cols, int64_t& row, int& c) {

@@ -120,11 +120,18 @@ static int xcd_strip_of(const dim3& grid, int rows, NarrowStrips narrow) {
     return (narrow == ANY_WIDTH || (narrow == ODD_WIDTHS && grid.x % 2 == 1)) && (int64_t)grid.x * grid.y * grid.z <= 256 ? 8 : 0;
 }
 
-template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES, bool NT_W, bool SWIGLU, bool QKV = false, bool SAMPLE = false, bool ROWSCALE = false>
+template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES, bool NT_W, bool SWIGLU, bool QKV = false, bool SAMPLE = false, bool ROWSCALE = false,
+          int ACT = 0>
 __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
     const bf16* __restrict__ x, int64_t x_stride, const bf16* __restrict__ w, const bf16* __restrict__ bias,
     bf16* __restrict__ y, int64_t y_stride, float* __restrict__ partials, int M, int N, int K, int k_per_split,
     QkvEpilogue qe, bool wide_store, SampleEpilogue se, int xcd_strip, RowScale rs) {
+    float act_pos = 0.f, act_neg = 0.f;
+    if constexpr (ACT == 1) {
+        const bf16* numbers = reinterpret_cast<const bf16*>(rs.sumsq);        // (ACT and ROWSCALE never meet)
+        act_pos = nvh_softplus_hw(bf2f(numbers[0]));
+        act_neg = 0.5f + nvh_softplus_hw(bf2f(numbers[1]));
+    }
     constexpr int NW = WAVES_N * WAVES_M;                 // waves per workgroup (4; 2 for the skinny decode tiles)
     static_assert(NW == 8 || NW == 4 || NW == 2, "2, 4 or 8 waves");
     constexpr int WN = BN / WAVES_N, WM = BM / WAVES_M;   // wave tile
@@ -642,7 +649,12 @@ __global__ __launch_bounds__(64 * WAVES_N * WAVES_M) void gemm_bf16_nt_kernel(
             } else {
                 bf16x4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) o[e] = f2bf(acc[i][j][e] + bv[e]);
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = f2bf(acc[i][j][e] + bv[e]);
+                    // (ACT: the activation of the rounded product, as a launch of its own over it gives; xIELU's numbers come with the call)
+                    if constexpr (ACT == 1) o[e] = f2bf(nvh_xielu_hw(bf2f(o[e]), act_pos, act_neg));
+                    if constexpr (ACT == 2) o[e] = f2bf(nvh_activation(bf2f(o[e]), 2));
+                }
                 *reinterpret_cast<bf16x4*>(y + (int64_t)m * y_stride + n) = o;
             }
         }
@@ -1465,6 +1477,61 @@ extern "C" int32_t nvh_gemm_bf16_nt(const void* x, int64_t x_row_stride, const v
     GemmArgs a{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, split_k > 1 ? workspace : nullptr,
                x_row_stride, y_row_stride, (int)M, (int)N, (int)K, split_k, (hipStream_t)stream, false};
     return dispatch_gemm(a);
+}
+
+static bool takes_kwaves(const GemmArgs& a);
+
+// ---- a projection with its ungated activation, up to 64 rows: act(bf16(x W^T + bias)) in the product's epilogue, on the tiles that nvh_gemm_bf16_nt takes
+// there (the same bits as the two launches).  An activation's launch over so few rows is its 4.7 us whatever it does; us of both and of one, 64 rows: 4608 x 1024
+// 11.3 and 6.9 (xIELU).  Larger calls keep two launches: their tiles leave through LDS.
+enum class ActTile { NONE, T16x32, T32x32, T64x16, T64x32 };
+static ActTile act_tile(int64_t M, int64_t N, int64_t K) {
+    GemmArgs a{};
+    a.M = (int)M, a.N = (int)N, a.K = (int)K, a.split_k = 1;
+    if (M < 1 || M > 64 || N <= 0 || N % 4 || N > 32 * 256 || K <= 0 || K % BK || K >= (1 << 30) || tile_forced() || nvh_switch_on(SW_GEMM_NO_NT) || takes_kwaves(a)) return ActTile::NONE;
+    switch (pick_tile(M, N, 1)) {
+        case T16x32: return nvh_cdiv(N, 32) > 768 ? ActTile::NONE : ActTile::T16x32;
+        case T32x32: return ActTile::T32x32;
+        case T64x64: return N <= 16 * 256 ? ActTile::T64x16 : ActTile::T64x32;
+        default: return ActTile::NONE;
+    }
+}
+template <int BM, int BN, int WAVES_N, int WAVES_M, int STAGES, int ACT>
+static void launch_act(const GemmArgs& a, const void* params) {
+    constexpr int smem = STAGES * (BM + BN) * 128;
+    auto kern = gemm_bf16_nt_kernel<BM, BN, WAVES_N, WAVES_M, STAGES, true, false, false, false, false, ACT>;
+    static std::atomic<uint64_t> granted;
+    if (smem > 65536) nvh_grant_lds(granted, (const void*)kern, smem);
+    const dim3 grid((unsigned)nvh_cdiv(a.N, BN), (unsigned)nvh_cdiv(a.M, BM), 1);
+    kern<<<grid, 64 * WAVES_N * WAVES_M, smem, a.st>>>(a.x, a.xs, a.w, a.bias, a.y, a.ys, nullptr, a.M, a.N, a.K, a.K, QkvEpilogue{}, false, SampleEpilogue{}, 0,
+                                                       RowScale{(const float*)params, 0, 0.f, 0.f});
+}
+template <int ACT>
+static void launch_act_tile(ActTile t, const GemmArgs& a, const void* params) {
+    switch (t) {
+        case ActTile::T16x32: return launch_act<16, 32, 2, 1, 8, ACT>(a, params);
+        case ActTile::T32x32: return launch_act<32, 32, 2, 1, 8, ACT>(a, params);
+        case ActTile::T64x16: return launch_act<64, 16, 1, 4, 6, ACT>(a, params);
+        default: return launch_act<64, 32, 2, 2, 6, ACT>(a, params);
+    }
+}
+
+extern "C" int32_t nvh_gemm_act_supported(int64_t M, int64_t N, int64_t K) { return act_tile(M, N, K) != ActTile::NONE; }
+
+extern "C" int32_t nvh_gemm_act_bf16_nt(const void* x, int64_t x_row_stride, const void* w, const void* bias, void* y, int64_t y_row_stride, int64_t M, int64_t N,
+                                        int64_t K, int32_t act, const void* params, nvh_stream_t stream) {
+    const char* name = "nvh_gemm_act_bf16_nt";
+    NVH_REQUIRE(x && w && y, NVH_EINVAL, "%s: null pointer", name);
+    NVH_REQUIRE(act == 2 || (act == 3 && params), NVH_EINVAL, "%s: activation %d (2: squared relu, 3: xIELU with its two numbers)", name, act);
+    const ActTile t = act_tile(M, N, K);
+    NVH_REQUIRE(t != ActTile::NONE, NVH_ENOSYS, "%s: %ld x %ld x %ld takes two launches", name, (long)M, (long)N, (long)K);
+    NVH_REQUIRE(x_row_stride % 8 == 0 && nvh_aligned16(x) && nvh_aligned16(w), NVH_EINVAL, "%s: x/w rows must be 16-byte aligned", name);
+    NVH_REQUIRE(y_row_stride % 4 == 0 && ((uintptr_t)y & 7) == 0 && ((uintptr_t)bias & 7) == 0, NVH_EINVAL, "%s: y rows and bias must be 8-byte aligned", name);
+    const GemmArgs a{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, nullptr, x_row_stride, y_row_stride, (int)M, (int)N, (int)K, 1, (hipStream_t)stream, false};
+    if (act == 3) launch_act_tile<1>(t, a, params);
+    else launch_act_tile<2>(t, a, nullptr);
+    NVH_CHECK_LAUNCH(name);
+    return NVH_OK;
 }
 
 // Decode batches and an output narrow enough that 16-column workgroups (x 16-row tiles of the batch) stay within about

@@ -749,15 +749,9 @@ __global__ __launch_bounds__(256) void xielu_kernel(const A* __restrict__ x, int
     if (i >= rows * inter) return;
     const int64_t row = i / inter;
     const int c = (int)(i - row * inter);
-    // bf16 results: the hardware's 2^x and log2 (errors of about 1e-7 beside values of at least softplus' own size)
-    constexpr float L2E = 1.4426950408889634f, LN2 = 0.6931471805599453f;
     auto softplus = [](float t) {
         if constexpr (sizeof(A) == 4) return fmaxf(t, 0.f) + log1pf(expf(-fabsf(t)));
-        else return fmaxf(t, 0.f) + LN2 * __builtin_amdgcn_logf(1.0f + __builtin_amdgcn_exp2f(-fabsf(t) * L2E));
-    };
-    auto expm1_of = [](float z) {                            // z <= 0
-        if constexpr (sizeof(A) == 4) return expm1f(z);
-        else return __builtin_amdgcn_exp2f(z * L2E) - 1.0f;
+        else return nvh_softplus_hw(t);
     };
     const float pos = softplus((float)params[0]), neg = 0.5f + softplus((float)params[1]);
     const A* src = x + row * x_stride + c;
@@ -768,7 +762,8 @@ __global__ __launch_bounds__(256) void xielu_kernel(const A* __restrict__ x, int
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const float z = (float)in[e];
-        out[e] = (A)((z > 0.f ? pos * z * z : neg * (expm1_of(fminf(z, 0.f)) - z)) + 0.5f * z);
+        if constexpr (sizeof(A) == 4) out[e] = (A)((z > 0.f ? pos * z * z : neg * (expm1f(fminf(z, 0.f)) - z)) + 0.5f * z);
+        else out[e] = (A)nvh_xielu_hw(z, pos, neg);
     }
     if constexpr (VEC) __builtin_memcpy(__builtin_assume_aligned(dst, 16), out, sizeof(out));
     else dst[0] = out[0];

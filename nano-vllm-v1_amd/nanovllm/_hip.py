@@ -118,6 +118,8 @@ SIGNATURES = {
     "nvh_residual_subnorm": (i32, [vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, vp, i64, i64, i64, i32, vp]),
     "nvh_residual_subnorm_moe": (i32, [vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, i64, f32, vp, vp, i64, i64, i64, vp, i64, vp, vp, i64, vp, i64, vp, i64, i32, vp]),
     "nvh_act_mul": (i32, [vp, i64, vp, i64, i64, i64, i32, i32, i32, vp]),
+    "nvh_gemm_act_supported": (i32, [i64, i64, i64]),
+    "nvh_gemm_act_bf16_nt": (i32, [vp, i64, vp, vp, vp, i64, i64, i64, i64, i32, vp, vp]),
     "nvh_xielu": (i32, [vp, i64, vp, i64, i64, i64, vp, i32, vp]),
     "nvh_logits_scale": (i32, [vp, i64, vp, i64, i64, f32, f32, i32, vp]),
     # a residual stream in several copies (csrc/hyper_stream.hip)

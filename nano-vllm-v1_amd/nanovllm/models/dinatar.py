@@ -38,7 +38,7 @@ from ..layers.activation import Act
 from ..layers.attention import WindowedBiasAttention
 from ..layers.layernorm import StreamNorm
 from ..layers.linear import MergedLinear
-from ..layers.moe import SparseMoE, plain_call
+from ..layers.moe import SparseMoE, plain_call, project_act
 from ..layers.recurrent import HGRN2, GatedLinearAttention, Mamba2
 from .lamutar import _get, layer_runs
 
@@ -126,7 +126,7 @@ class DinatarDenseMLP(nn.Module):
         self.down = MergedLinear(ff, [width])
 
     def forward(self, x: torch.Tensor) -> dict:
-        return dict(c=self.down(self.act(self.up(x))))
+        return dict(c=self.down(project_act(self.up, self.act, x)))
 
 
 class DinatarMoE(nn.Module):

@@ -43,6 +43,7 @@ from ..layers.activation import XIELU
 from ..layers.attention import LatentAttention, WindowedBiasAttention
 from ..layers.layernorm import StreamNorm
 from ..layers.linear import MergedLinear
+from ..layers.moe import project_act
 from ..layers.rotary_embedding import rotary_frequencies
 from .lamutar import _get
 
@@ -93,7 +94,7 @@ class MopalornFeedForward(nn.Module):
         self.act = XIELU()
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down(self.act(self.up(x)))
+        return self.down(project_act(self.up, self.act, x))
 
 
 class MopalornLayer(nn.Module):

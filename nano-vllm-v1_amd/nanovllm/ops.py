@@ -1011,6 +1011,22 @@ def xielu(x: torch.Tensor, params: torch.Tensor) -> torch.Tensor:
     return y
 
 
+def linear_act(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, act: str, params: torch.Tensor | None = None) -> torch.Tensor | None:
+    """act(x W^T + bias) in one launch for a few bf16 rows, the bits of linear_any followed by the activation (act: relu2, xielu with its `params`);
+    None where the sizes or types take two."""
+    m = x.shape[0]
+    if m > 64 or m == 0 or x.dim() != 2 or x.dtype != BF16 or weight.dtype != BF16 or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
+        return None
+    n, k = weight.shape
+    if not _hip.lib().nvh_gemm_act_supported(m, n, k):
+        return None
+    _act_flag(x, weight, *(() if params is None else (params,)), *(() if bias is None else (bias,)))
+    assert weight.is_contiguous() and x.shape[1] == k and (act == "relu2" or (act == "xielu" and params.numel() == 2 and params.is_contiguous()))
+    y = torch.empty(m, n, dtype=BF16, device=x.device)
+    _hip.call("nvh_gemm_act_bf16_nt", x.data_ptr(), x.stride(0), weight.data_ptr(), _p(bias), y.data_ptr(), n, m, n, k, 2 if act == "relu2" else 3, _p(params), _stream())
+    return y
+
+
 def logits_scale(logits: torch.Tensor, scale: float, cap: float = 0.0) -> torch.Tensor:
     """fp32 scale * logits (softcapped when cap > 0)."""
     f = _act_flag(logits)
