@@ -564,8 +564,8 @@ int32_t nvh_attn_paged_any(const void* q, int64_t q_row_stride, const void* k_ca
  * y_t = sum_j conv_w[c, j] u_(t - taps + 1 + j) (conv_w [channels, taps] of type A; NULL with taps 1: none; zeros before the sequence's start),
  * continued from conv_state fp32 [slots, taps - 1, channels] unless the sequence starts in this step; unit_qk: q and k are then divided by
  * sqrt(mean(y^2) + eps) per head.  q -> q_out [T, H dim], k and v -> the tokens' slots of the caches above; k_cache = v_cache = NULL: the row
- * opens with q columns only.  update_state (every sequence brings one token): the state is brought up to date in the same launch;
- * otherwise nvh_conv_state_update follows. */
+ * opens with q columns only.  update_state 1 (every sequence brings one token) or 2 (every sequence starts in this step: context_lens[b] is its token
+ * count): the state is brought up to date in the same launch; 0: nvh_conv_state_update follows. */
 int32_t nvh_attn_conv_prep(const void* proj, int64_t proj_row_stride, const void* conv_w, int64_t taps, float* conv_state, const int32_t* slots,
                            const int32_t* cu_seqlens_q, const int32_t* context_lens, const int32_t* slot_mapping, int32_t unit_qk, float eps,
                            void* q_out, void* k_cache, void* v_cache, int64_t page, int64_t batch, int64_t num_tokens, int64_t num_q_heads,
@@ -598,6 +598,11 @@ int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, const void* b,
                              const void* conv_w, const void* dt_bias, const void* a_log, const float* conv_state, const int32_t* slots,
                              const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
                              int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream);
+/* nvh_gated_delta_prep and the nvh_conv_state_update behind it, for steps in which every sequence starts (context_lens[b] is its token count). */
+int32_t nvh_gated_delta_prep_starting(const void* qkv, int64_t qkv_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
+                                      const void* conv_w, const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots,
+                                      const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
+                                      int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream);
 int32_t nvh_delta_prep(const void* r, int64_t r_stride, const void* k, int64_t k_stride, const void* v, int64_t v_stride,
                        const void* a_raw, int64_t a_stride, const void* lowrank, int64_t lowrank_stride,
                        const void* w2, const void* w0, const void* a_bias, float* out, int64_t num_tokens, int64_t heads, int64_t dk,
@@ -768,6 +773,10 @@ int32_t nvh_conv_state_update(const void* xbc, int64_t xbc_stride, float* conv_s
 int32_t nvh_stream_conv(const float* x, const void* w, const float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
                         const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
                         int32_t act_f32, nvh_stream_t stream);
+/* nvh_stream_conv and the nvh_conv_state_update behind it, for steps in which every sequence starts (context_lens[b] is its token count). */
+int32_t nvh_stream_conv_starting(const float* x, const void* w, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                 const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
+                                 int32_t act_f32, nvh_stream_t stream);
 /* One token per sequence (no cu_seqlens_q): nvh_ssd_conv_prep / nvh_stream_conv with the nvh_conv_state_update that follows them. */
 int32_t nvh_ssd_conv_prep_step(const void* xbc, int64_t xbc_stride, const void* dt, int64_t dt_stride, const void* conv_w, const void* conv_b,
                                const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots, const int32_t* context_lens,

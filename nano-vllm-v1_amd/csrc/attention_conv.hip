@@ -6,7 +6,8 @@
 //                        [pages, page, G, dim], values transposed within a page, [pages, G, vdim, page]).  A layer without keys
 //                        of its own has q columns only.  Sums and norms are fp32; a value is rounded once, when it is stored.
 // The carried inputs (state [slots, taps - 1, channels] fp32) are brought up to date in the same launch when every sequence
-// brings one token; in any other step nvh_conv_state_update follows.
+// brings one token, and when every sequence starts in the step (nobody reads a slot then; the launch that follows otherwise takes 3.9 us); in any other step
+// nvh_conv_state_update follows.
 #include "common.h"
 
 namespace {
@@ -19,7 +20,7 @@ struct ConvPrepArgs {
     const int32_t *slots, *cu_seqlens_q, *context_lens, *slot_mapping;
     void *q_out, *k_cache, *v_cache;
     int T, batch, taps, H, G, dim, vdim, page, channels;
-    int unit, update_state, vec, lanes_log2;       // lanes: per row of a head, a power of two, eight channels each
+    int unit, update_state, vec, lanes_log2;       // update_state 1: one token per sequence, 2: every sequence starts in this step;       // lanes: per row of a head, a power of two, eight channels each
     float eps;
 };
 
@@ -28,6 +29,7 @@ struct ConvPrepArgs {
 template <typename A, int TAPS, int KT>
 __global__ __launch_bounds__(256) void attn_conv_prep_kernel(ConvPrepArgs p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    __shared__ int behind_s[KT];                             // the portion's tokens behind this one
     __shared__ int index_s[KT], state_slot_s[KT], cache_slot_s[KT];            // the token's number within its portion; -1: nothing carried; -1: not stored
     const int tid = threadIdx.x, t0 = blockIdx.x * KT, hs = blockIdx.y;
     const int kind = hs < p.H ? 0 : (hs < p.H + p.G ? 1 : 2), head = kind == 0 ? hs : (kind == 1 ? hs - p.H : hs - p.H - p.G);
@@ -35,16 +37,18 @@ __global__ __launch_bounds__(256) void attn_conv_prep_kernel(ConvPrepArgs p) {
     const int col0 = kind == 0 ? head * p.dim : (kind == 1 ? (p.H + head) * p.dim : (p.H + p.G) * p.dim + head * p.vdim);
     if (tid < KT) {
         const int t = t0 + tid;
-        int j = 0, st = -1, cs = -1;
+        int j = 0, st = -1, cs = -1, behind = 0;
         if (t < p.T) {
             const int seq = seq_of_token(p.cu_seqlens_q, p.batch, t);
             const int lo = p.cu_seqlens_q ? p.cu_seqlens_q[seq] : seq, hi = p.cu_seqlens_q ? p.cu_seqlens_q[seq + 1] : seq + 1;
             const int slot = p.slots ? p.slots[seq] : -1;
             j = t - lo;
+            behind = hi - 1 - t;
             if (slot >= 0) st = p.context_lens[seq] != hi - lo ? slot : -2 - slot;       // (-2 - slot: a slot whose sequence starts in this step)
             cs = p.slot_mapping ? p.slot_mapping[t] : -1;
         }
         index_s[tid] = j;
+        behind_s[tid] = behind;
         state_slot_s[tid] = st;
         cache_slot_s[tid] = cs;
     }
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(256) void attn_conv_prep_kernel(ConvPrepArgs p) {
         }
         // One token per sequence: this thread is the only one that reads or writes these channels of the slot.  Ascending
         // entries: an entry is read (as its predecessor's new value) before it is written.
-        if (p.update_state && slot != -1) {
+        if (p.update_state == 1 && slot != -1) {
             const int sl = slot >= 0 ? slot : -2 - slot;
             float* st = p.state + (int64_t)sl * (taps - 1) * p.channels + col0 + c;
             for (int k = 0; k + 1 < taps; ++k) {
@@ -135,6 +139,20 @@ __global__ __launch_bounds__(256) void attn_conv_prep_kernel(ConvPrepArgs p) {
                         if (e < valid) st[(int64_t)k * p.channels + e] = x[e];
                 }
             }
+        }
+        if (p.update_state == 2 && slot <= -2 && (behind_s[r] < taps - 1 || j == 0)) {
+            const int keep = taps - 1, behind = behind_s[r];
+            float* st = p.state + (int64_t)(-2 - slot) * keep * p.channels + col0 + c;
+            float x[8];
+            input(0, x);
+            auto entry = [&](int k, bool zero) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (e < valid) st[(int64_t)k * p.channels + e] = zero ? 0.f : x[e];
+            };
+            if (behind < keep) entry(keep - 1 - behind, false);
+            if (j == 0)
+                for (int k = 0; k < keep - 1 - behind; ++k) entry(k, true);          // (a portion shorter than the taps: zeros in front of its inputs)
         }
         if (kind != 2 && p.unit) {
             float ss = 0.f;
@@ -208,14 +226,15 @@ extern "C" int32_t nvh_attn_conv_prep(const void* proj, int64_t proj_row_stride,
     const int64_t channels = num_q_heads * dim + (own ? num_kv_heads * (dim + vdim) : 0);
     NVH_REQUIRE(proj_row_stride >= channels && channels < (1 << 28), NVH_EINVAL, "nvh_attn_conv_prep: projection row too short");
     NVH_REQUIRE(cu_seqlens_q || num_tokens == batch, NVH_EINVAL, "nvh_attn_conv_prep: one token per sequence without cu_seqlens_q");
-    NVH_REQUIRE(!update_state || num_tokens == batch, NVH_EINVAL, "nvh_attn_conv_prep: the state is updated here only when every sequence brings one token");
+    NVH_REQUIRE(update_state != 1 || num_tokens == batch, NVH_EINVAL, "nvh_attn_conv_prep: the state is updated here only when every sequence brings one token");
+    NVH_REQUIRE(update_state >= 0 && update_state <= 2, NVH_EINVAL, "nvh_attn_conv_prep: update_state %d", update_state);
     if (num_tokens == 0 || batch == 0) return NVH_OK;
     int lanes_log2 = 0;
     while ((8 << lanes_log2) < (own && vdim > dim ? vdim : dim)) ++lanes_log2;
     const bool vec = dim % 8 == 0 && vdim % 8 == 0 && proj_row_stride % 8 == 0 && nvh_aligned16(proj) && nvh_aligned16(conv_w) && nvh_aligned16(conv_state) && nvh_aligned16(q_out) &&
                      nvh_aligned16(k_cache) && nvh_aligned16(v_cache);
     const ConvPrepArgs p{proj, proj_row_stride, conv_w, conv_state, slots, cu_seqlens_q, context_lens, slot_mapping, q_out, k_cache, v_cache, (int)num_tokens, (int)batch, (int)taps,
-                         (int)num_q_heads, (int)num_kv_heads, (int)dim, (int)vdim, (int)page, (int)channels, unit_qk, update_state && taps > 1, vec, lanes_log2, eps};
+                         (int)num_q_heads, (int)num_kv_heads, (int)dim, (int)vdim, (int)page, (int)channels, unit_qk, taps > 1 ? update_state : 0, vec, lanes_log2, eps};
     const int heads = (int)(num_q_heads + (own ? 2 * num_kv_heads : 0));
     hipStream_t st = (hipStream_t)stream;
     // (a token's arithmetic does not depend on the tile it lies in)

@@ -125,9 +125,12 @@ __global__ __launch_bounds__(256) void gated_delta_prep_kernel(GatedDeltaPrepArg
 // once instead of once per tap.  Same sums in the same order.
 // us, one token a workgroup and two or four, heads of 128 x 128: 1000 tokens of 8 heads 33.5 and 17.4 (25 MB written), of 4 15.7 and 11.2, 2000 of 8 61.6 and
 // 28.8, 300 of 8 11.4 and 8.3; eight tokens a workgroup 19.2, 15.7, 30.2, 11.5.
+// carried_out: every sequence starts in this step, so no lane reads a slot and the last TAPS - 1 tokens of each leave their inputs there (a launch of 3.9 us less);
+// a q or k channel that several heads share is the first one's.
 template <typename A, int TT, int TAPS>
-__global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPrepArgs p, int64_t num_tokens, int vec) {
+__global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPrepArgs p, int64_t num_tokens, int vec, float* carried_out) {
     extern __shared__ __attribute__((aligned(16))) float sh[];                            // [TT][n] q (dk) | k (dk) | v (dv) of this head, then the numbers of the tokens
+    __shared__ int slot_of[TT], end_of[TT];
     __shared__ int first_of[TT], state_of[TT];               // the first row of the token's sequence in this step; its slot, or -1: nothing carried
     const int64_t t0 = (int64_t)blockIdx.x * TT;
     const int nt = (int)min((int64_t)TT, num_tokens - t0), tid = threadIdx.x;
@@ -150,6 +153,8 @@ __global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPre
         }
         const int slot = p.slots[seq];
         first_of[tid] = lo;
+        slot_of[tid] = slot;
+        end_of[tid] = hi;
         state_of[tid] = slot >= 0 && p.context_lens[seq] != hi - lo ? slot : -1;
         beta[tid] = sigmoidf_(ldf((const A*)p.b, t * p.b_stride + h));
         dec[tid] = expf(-expf(ldf((const A*)p.a_log, h)) * softplusf_(ldf((const A*)p.a, t * p.a_stride + h) + ldf((const A*)p.dt_bias, h)));
@@ -175,6 +180,13 @@ __global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPre
                 acc = __builtin_fmaf(w[k], x, acc);
             }
             if (tt < nt) sh[tt * n + e] = acc / (1.0f + expf(-acc));
+            if (carried_out && tt < nt && slot_of[tt] >= 0 && (e >= 2 * dk || h % (p.H / p.G) == 0)) {
+                const int len = end_of[tt] - first_of[tt], s = j - (len - (TAPS - 1));
+                float* to = carried_out + (int64_t)slot_of[tt] * (TAPS - 1) * C + c;
+                if (s >= 0) to[(int64_t)s * C] = in[tt + TAPS - 1];
+                if (j == 0)
+                    for (int k = 0; k < TAPS - 1 - len; ++k) to[(int64_t)k * C] = 0.f;
+            }
         }
     }
     __syncthreads();
@@ -224,11 +236,11 @@ __global__ __launch_bounds__(256) void gated_delta_prep_run_kernel(GatedDeltaPre
 }
 
 template <int TT>
-void launch_gated_delta_prep_run(const GatedDeltaPrepArgs& p, int64_t num_tokens, bool act_f32, hipStream_t st) {
+void launch_gated_delta_prep_run(const GatedDeltaPrepArgs& p, int64_t num_tokens, bool act_f32, float* carried_out, hipStream_t st) {
     const dim3 grid((unsigned)nvh_cdiv(num_tokens, TT), (unsigned)p.H);
     const size_t lds = sizeof(float) * (size_t)(TT * (2 * p.dk + p.dv) + 4 * TT);
     const int vec = p.dk % 4 == 0 && p.dv % 4 == 0 && nvh_aligned16(p.out);
-    auto launch = [&](auto kernel) { kernel<<<grid, 256, lds, st>>>(p, num_tokens, vec); };
+    auto launch = [&](auto kernel) { kernel<<<grid, 256, lds, st>>>(p, num_tokens, vec, carried_out); };
     if (act_f32) launch(p.taps == 2 ? &gated_delta_prep_run_kernel<float, TT, 2> : p.taps == 3 ? &gated_delta_prep_run_kernel<float, TT, 3> : &gated_delta_prep_run_kernel<float, TT, 4>);
     else launch(p.taps == 2 ? &gated_delta_prep_run_kernel<bf16, TT, 2> : p.taps == 3 ? &gated_delta_prep_run_kernel<bf16, TT, 3> : &gated_delta_prep_run_kernel<bf16, TT, 4>);
 }
@@ -1112,10 +1124,10 @@ static int32_t launch_delta_scan(const DeltaScanArgs& p, int64_t batch, hipStrea
     return NVH_OK;
 }
 
-extern "C" int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
-                                        const void* conv_w, const void* dt_bias, const void* a_log, const float* conv_state, const int32_t* slots,
-                                        const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
-                                        int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream) {
+static int32_t gated_delta_prep(const void* qkv, int64_t qkv_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
+                                const void* conv_w, const void* dt_bias, const void* a_log, const float* conv_state, float* carried_out, const int32_t* slots,
+                                const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
+                                int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream) {
     NVH_REQUIRE(qkv && b && a && conv_w && dt_bias && a_log && slots && context_lens && out, NVH_EINVAL, "nvh_gated_delta_prep: null pointer");
     NVH_REQUIRE(batch >= 0 && num_tokens >= 0 && taps >= 1 && heads > 0 && qk_heads > 0 && heads % qk_heads == 0 && dk > 0 && dv > 0, NVH_EINVAL,
                 "nvh_gated_delta_prep: bad sizes");
@@ -1133,15 +1145,35 @@ extern "C" int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, con
     // share their inputs: two) one token each, as ever.  us, one and two, 64 tokens of 16 heads of 64 x 64: single tokens 5.8 and 6.3, of a prompt 5.2 and 5.4; 100
     // of a prompt 6.7 and 6.1; 128 of 8 heads of 128 x 128 6.7 and 6.2.
     const bool run = taps >= 2 && taps <= 4 && (2 * dk + dv + 4) * 4 * (int64_t)sizeof(float) <= 32 * 1024;
-    if (run && num_tokens * heads >= 4096) launch_gated_delta_prep_run<4>(p, num_tokens, act_f32, st);
-    else if (run && num_tokens * heads >= (2 * dk + dv >= 256 && batch < num_tokens ? 1024 : 1280)) launch_gated_delta_prep_run<2>(p, num_tokens, act_f32, st);
+    if (run && num_tokens * heads >= 4096) launch_gated_delta_prep_run<4>(p, num_tokens, act_f32, carried_out, st);
+    else if (run && num_tokens * heads >= (2 * dk + dv >= 256 && batch < num_tokens ? 1024 : 1280)) launch_gated_delta_prep_run<2>(p, num_tokens, act_f32, carried_out, st);
     else {
         const dim3 grid((unsigned)num_tokens, (unsigned)heads);
         if (act_f32) gated_delta_prep_kernel<float><<<grid, 256, lds, st>>>(p);
         else gated_delta_prep_kernel<bf16><<<grid, 256, lds, st>>>(p);
+        if (carried_out) {
+            NVH_CHECK_LAUNCH("nvh_gated_delta_prep");
+            return nvh_conv_state_update(qkv, qkv_stride, carried_out, slots, cu_seqlens_q, context_lens, batch, taps, channels, act_f32, stream);
+        }
     }
     NVH_CHECK_LAUNCH("nvh_gated_delta_prep");
     return NVH_OK;
+}
+
+extern "C" int32_t nvh_gated_delta_prep(const void* qkv, int64_t qkv_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
+                                        const void* conv_w, const void* dt_bias, const void* a_log, const float* conv_state, const int32_t* slots,
+                                        const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
+                                        int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream) {
+    return gated_delta_prep(qkv, qkv_stride, b, b_stride, a, a_stride, conv_w, dt_bias, a_log, conv_state, nullptr, slots, cu_seqlens_q, context_lens, out, batch,
+                            num_tokens, taps, heads, qk_heads, dk, dv, act_f32, stream);
+}
+
+extern "C" int32_t nvh_gated_delta_prep_starting(const void* qkv, int64_t qkv_stride, const void* b, int64_t b_stride, const void* a, int64_t a_stride,
+                                                 const void* conv_w, const void* dt_bias, const void* a_log, float* conv_state, const int32_t* slots,
+                                                 const int32_t* cu_seqlens_q, const int32_t* context_lens, float* out, int64_t batch, int64_t num_tokens,
+                                                 int64_t taps, int64_t heads, int64_t qk_heads, int64_t dk, int64_t dv, int32_t act_f32, nvh_stream_t stream) {
+    return gated_delta_prep(qkv, qkv_stride, b, b_stride, a, a_stride, conv_w, dt_bias, a_log, conv_state, taps > 1 ? conv_state : nullptr, slots, cu_seqlens_q,
+                            context_lens, out, batch, num_tokens, taps, heads, qk_heads, dk, dv, act_f32, stream);
 }
 
 extern "C" int32_t nvh_delta_scan(const float* pack, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,

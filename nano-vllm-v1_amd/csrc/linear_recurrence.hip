@@ -397,6 +397,7 @@ __global__ __launch_bounds__(256) void stream_conv_kernel(StreamConvArgs p) {
 // per tap.  STEP (TT 1, one token per sequence): the slot is brought up to date as well - the lane that reads a column's carried inputs is the only
 // one that does.
 // us, four taps over 1024 columns: one token of 64 sequences, where the update is inside, 4.7 and 2.5.
+// carried_out without STEP: every sequence starts in this step, so no lane reads a slot and the last TAPS - 1 tokens of each leave theirs (a launch of 3.9 us less).
 template <typename A, int TT, int TAPS, bool STEP>
 __global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, int64_t num_tokens, float* carried_out) {
     static_assert(!STEP || TT == 1, "a step brings one token per sequence");
@@ -439,6 +440,13 @@ __global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, 
         if (STEP && slot >= 0)
 #pragma unroll
             for (int k = 0; k < TAPS - 1; ++k) *reinterpret_cast<f32x4*>(carried_out + ((int64_t)slot * (TAPS - 1) + k) * dim + col) = kept[k + 1];
+        if (!STEP && carried_out && slot >= 0) {
+            const int n = hi - lo, s = j - (n - (TAPS - 1));
+            float* to = carried_out + (int64_t)slot * (TAPS - 1) * dim + col;
+            if (s >= 0) *reinterpret_cast<f32x4*>(to + (int64_t)s * dim) = in[tt + TAPS - 1];
+            if (j == 0)
+                for (int k = 0; k < TAPS - 1 - n; ++k) *reinterpret_cast<f32x4*>(to + (int64_t)k * dim) = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         const f32x4 h = in[tt + TAPS - 1] + acc;
         A* dst = (A*)p.h + t * p.h_stride + col;
         if constexpr (sizeof(A) == 4) *reinterpret_cast<f32x4*>(dst) = h;
@@ -448,7 +456,7 @@ __global__ __launch_bounds__(256) void stream_conv_run_kernel(StreamConvArgs p, 
 
 // (false: taps, columns or alignment that the form above does not serve)
 template <typename A>
-static bool launch_stream_conv_run(const StreamConvArgs& p, int64_t num_tokens, int taps, float* carried_out, hipStream_t st) {
+static bool launch_stream_conv_run(const StreamConvArgs& p, int64_t num_tokens, int taps, float* carried_out, bool starting, hipStream_t st) {
     if (taps < 2 || taps > 4 || p.dim % 4 || p.h_stride % 4 || !nvh_aligned16(p.x) || !nvh_aligned16(p.state) || ((uintptr_t)p.h % (4 * sizeof(A)))) return false;
     // Four tokens a workgroup from about 2 M elements on, where inputs read once instead of once per tap count; below, and for few tokens, more workgroups do.  us, one token a
     // workgroup (as before, by columns) and four, four taps: 1000 x 64 5.1, 4.7, 6.5; 1000 x 1024 9.2, 5.5, 6.9; 1000 x 2048 18.1, 8.0, 7.4; 2000 x 1024 14.6,
@@ -456,9 +464,9 @@ static bool launch_stream_conv_run(const StreamConvArgs& p, int64_t num_tokens, 
     constexpr int TT = 4;
     const unsigned cols = (unsigned)nvh_cdiv(p.dim, 1024);
 #define NVH_CONV_RUN(TAPS)                                                                                                                                   \
-    if (carried_out) stream_conv_run_kernel<A, 1, TAPS, true><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, carried_out);               \
-    else if (num_tokens >= 512 && num_tokens * p.dim >= 15 << 17) stream_conv_run_kernel<A, TT, TAPS, false><<<dim3((unsigned)nvh_cdiv(num_tokens, TT), cols), 256, 0, st>>>(p, num_tokens, nullptr); \
-    else stream_conv_run_kernel<A, 1, TAPS, false><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, nullptr)
+    if (carried_out && !starting) stream_conv_run_kernel<A, 1, TAPS, true><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, carried_out);               \
+    else if (num_tokens >= 512 && num_tokens * p.dim >= 15 << 17) stream_conv_run_kernel<A, TT, TAPS, false><<<dim3((unsigned)nvh_cdiv(num_tokens, TT), cols), 256, 0, st>>>(p, num_tokens, carried_out); \
+    else stream_conv_run_kernel<A, 1, TAPS, false><<<dim3((unsigned)num_tokens, cols), 256, 0, st>>>(p, num_tokens, carried_out)
     if (taps == 2) { NVH_CONV_RUN(2); }
     else if (taps == 3) { NVH_CONV_RUN(3); }
     else { NVH_CONV_RUN(4); }
@@ -1346,6 +1354,7 @@ extern "C" int32_t nvh_conv_state_update(const void* xbc, int64_t xbc_stride, fl
 static int32_t stream_conv(const float* x, const void* w, const float* state, float* state_out, const int32_t* slots, const int32_t* cu_seqlens_q,
                            const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim, int32_t act_f32,
                            nvh_stream_t stream) {
+    const bool starting = state_out && cu_seqlens_q;         // (otherwise a state that goes out is a step's of one token per sequence)
     NVH_REQUIRE(x && w && slots && context_lens && h && batch >= 0 && num_tokens >= 0 && taps >= 1 && dim > 0 && h_stride >= dim, NVH_EINVAL,
                 "nvh_stream_conv: bad argument");
     NVH_REQUIRE(taps == 1 || state, NVH_EINVAL, "nvh_stream_conv: null state");
@@ -1353,7 +1362,7 @@ static int32_t stream_conv(const float* x, const void* w, const float* state, fl
     if (num_tokens == 0 || batch == 0) return NVH_OK;
     const StreamConvArgs p{x, w, state, slots, cu_seqlens_q, context_lens, h, h_stride, (int)batch, (int)taps, (int)dim};
     hipStream_t st = (hipStream_t)stream;
-    if (act_f32 ? launch_stream_conv_run<float>(p, num_tokens, (int)taps, state_out, st) : launch_stream_conv_run<bf16>(p, num_tokens, (int)taps, state_out, st)) {
+    if (act_f32 ? launch_stream_conv_run<float>(p, num_tokens, (int)taps, state_out, starting, st) : launch_stream_conv_run<bf16>(p, num_tokens, (int)taps, state_out, starting, st)) {
         NVH_CHECK_LAUNCH("nvh_stream_conv");
         return NVH_OK;
     }
@@ -1361,13 +1370,20 @@ static int32_t stream_conv(const float* x, const void* w, const float* state, fl
     if (act_f32) stream_conv_kernel<float><<<grid, 256, 0, st>>>(p);
     else stream_conv_kernel<bf16><<<grid, 256, 0, st>>>(p);
     NVH_CHECK_LAUNCH("nvh_stream_conv");
-    return state_out ? nvh_conv_state_update(x, dim, state_out, slots, nullptr, context_lens, batch, taps, dim, 1, stream) : NVH_OK;
+    return state_out ? nvh_conv_state_update(x, dim, state_out, slots, cu_seqlens_q, context_lens, batch, taps, dim, 1, stream) : NVH_OK;
 }
 
 extern "C" int32_t nvh_stream_conv(const float* x, const void* w, const float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
                                    const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
                                    int32_t act_f32, nvh_stream_t stream) {
     return stream_conv(x, w, state, nullptr, slots, cu_seqlens_q, context_lens, h, h_stride, batch, num_tokens, taps, dim, act_f32, stream);
+}
+
+extern "C" int32_t nvh_stream_conv_starting(const float* x, const void* w, float* state, const int32_t* slots, const int32_t* cu_seqlens_q,
+                                            const int32_t* context_lens, void* h, int64_t h_stride, int64_t batch, int64_t num_tokens, int64_t taps, int64_t dim,
+                                            int32_t act_f32, nvh_stream_t stream) {
+    NVH_REQUIRE(cu_seqlens_q, NVH_EINVAL, "nvh_stream_conv_starting: null cu_seqlens_q");
+    return stream_conv(x, w, state, taps > 1 ? state : nullptr, slots, cu_seqlens_q, context_lens, h, h_stride, batch, num_tokens, taps, dim, act_f32, stream);
 }
 
 extern "C" int32_t nvh_stream_conv_step(const float* x, const void* w, float* state, const int32_t* slots, const int32_t* context_lens, void* h,

@@ -107,6 +107,7 @@ SIGNATURES = {
     "nvh_delta_chunk_workspace_bytes": (i64, [i64, i64, i64, i64, i64]),
     "nvh_delta_scan_chunked": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, vp, vp]),
     "nvh_delta_scan": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, vp]),
+    "nvh_gated_delta_prep_starting": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i32, vp]),
     "nvh_gated_delta_prep": (i32, [vp, i64, vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i64, i32, vp]),
     "nvh_delta_post": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i64, f32, i32, vp]),
     # layer norm / RMS norm around the fp32 stream, plain activations (csrc/stream_f32.hip)
@@ -139,6 +140,7 @@ SIGNATURES = {
     "nvh_ssd_conv_prep_step": (i32, [vp, i64, vp, i64, vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, vp, vp, vp, vp, vp, i32, vp]),
     "nvh_stream_conv_step": (i32, [vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i32, vp]),
     "nvh_conv_state_update": (i32, [vp, i64, vp, vp, vp, vp, i64, i64, i64, i32, vp]),
+    "nvh_stream_conv_starting": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i32, vp]),
     "nvh_stream_conv": (i32, [vp, vp, vp, vp, vp, vp, vp, i64, i64, i64, i64, i64, i32, vp]),
     "nvh_group_rmsnorm_gate": (i32, [vp, vp, i32, vp, i64, i32, i32, vp, i64, i64, i64, i64, f32, i32, vp]),
     # mixture of experts (csrc/moe.hip)

@@ -525,7 +525,8 @@ class ModelRunner:
         fb["items"] = None if plan is None else {k: d[k] for k in ("item_seq", "item_range", "seq_active", "seq_chunk")}
         fb["tails"] = (d.get("cu_seqlens_q_tail"), d.get("cu_seqlens_k_tail"))
         set_context(d["cu_seqlens_q"], d["cu_seqlens_k"], fb["max_seqlen_q"], fb["max_seqlen_k"], d["slot_mapping"],
-                    d["context_lens"], d.get("block_tables"), d["need"], d.get("state_slots"))
+                    d["context_lens"], d.get("block_tables"), d["need"], d.get("state_slots"),
+                    self.config.recurrent_state and bool((fb["context_lens"] == np.diff(fb["cu_seqlens_q"])).all()))
         fb["logit_rows_dev"] = d.get("logit_rows")
         fb["last_rows_dev"] = d.get("last_rows")
         return d["input_ids"], d["positions"], d.get("temperatures"), fb

@@ -260,7 +260,7 @@ class WindowedBiasAttention(nn.Module):
             own = owner is self
             q = ops.attn_conv_prep(proj, None if self.conv_weight is None else self.conv_weight.data, self.conv_inputs.pool(run) if self.conv_inputs is not None else None,
                                    ctx.state_slots, ctx.cu_seqlens_q, ctx.context_lens, ctx.slot_mapping, kc if own else None, vc if own else None, self.num_heads,
-                                   self.num_kv_heads, self.head_dim, self.value_dim, self.unit_qk, ctx.max_seqlen_q == 1)
+                                   self.num_kv_heads, self.head_dim, self.value_dim, self.unit_qk, ctx.max_seqlen_q == 1, ctx.all_start)
             return self._attend(q, kc, vc, run, gate)
         assert self.v_mix is None or v_first is not None, "this attention mixes an earlier layer's values in"
         nq, (nk, nv) = self.num_heads * self.head_dim, self.cache_row_elems()

@@ -104,7 +104,8 @@ class GatedDeltaRule(nn.Module):
         if state is None or ctx.state_slots is None:
             raise RuntimeError("the delta rule needs a bound state pool and a state slot per sequence")
         o = ops.gated_delta_rule(qkv, b, a, self.conv_weight.data, self.dt_bias.data, self.A_log.data, self.conv_inputs.pool(run), state, ctx.state_slots,
-                                 ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.qk_heads, self.key_dim, self.value_dim, max_seqlen_q=ctx.max_seqlen_q or 0)
+                                 ctx.cu_seqlens_q, ctx.context_lens, self.num_heads, self.qk_heads, self.key_dim, self.value_dim, max_seqlen_q=ctx.max_seqlen_q or 0,
+                                 all_start=ctx.all_start)
         return ops.group_rmsnorm_gate(o, self.norm.data, self.value_dim, self.eps, gate, "silu", gate_first=False)
 
 
@@ -295,4 +296,4 @@ class StreamConv(StatePool):
     def forward(self, x: torch.Tensor, run: int = 0) -> torch.Tensor:
         """x fp32 [T, width] (left as it is) -> h in the activation type."""
         ctx = get_context()
-        return ops.stream_conv(x, self.weight.data, self.pool(run), ctx.state_slots, ctx.cu_seqlens_q, ctx.context_lens)
+        return ops.stream_conv(x, self.weight.data, self.pool(run), ctx.state_slots, ctx.cu_seqlens_q, ctx.context_lens, ctx.all_start)

@@ -747,11 +747,11 @@ def attn_paged_any(q, k_cache, v_cache, cu_seqlens_q, context_lens, block_tables
 
 
 def attn_conv_prep(proj, conv_w, conv_state, slots, cu_seqlens_q, context_lens, slot_mapping, k_cache, v_cache, heads: int, kv_heads: int, dim: int,
-                   vdim: int, unit_eps: float | None = None, one_token: bool = False) -> torch.Tensor:
+                   vdim: int, unit_eps: float | None = None, one_token: bool = False, all_start: bool = False) -> torch.Tensor:
     """q [T, H*dim] from the projection rows [q | k | v | ...] (caches None: [q | ...]) after a causal convolution over time per channel with
     `conv_w` [channels, taps] (None: none), continued from `conv_state` [slots, taps - 1, channels] fp32, which is then brought up to date; k and v
     go to their cache slots.  `unit_eps`: q and k are divided by their root mean square per head.  `one_token`: every sequence brings one
-    token (then the state is updated in the same launch)."""
+    token; `all_start`: every sequence starts in this step (either way the state is updated in the same launch)."""
     typed = [x for x in (proj, conv_w, k_cache, v_cache) if x is not None]
     f = _act_flag(*typed)
     own = k_cache is not None
@@ -771,8 +771,8 @@ def attn_conv_prep(proj, conv_w, conv_state, slots, cu_seqlens_q, context_lens, 
     q = torch.empty(t, heads * dim, dtype=proj.dtype, device=proj.device)
     _hip.call("nvh_attn_conv_prep", proj.data_ptr(), proj.stride(0), _p(conv_w), taps, _p(conv_state) if taps > 1 else 0, _p(slots), _p(cu_seqlens_q),
               context_lens.data_ptr(), _p(slot_mapping) if own else 0, int(unit_eps is not None), float(unit_eps or 0.0), q.data_ptr(), _p(k_cache), _p(v_cache), page,
-              batch, t, heads, kv_heads, dim, vdim, int(one_token and taps > 1), f, _stream())
-    if taps > 1 and not one_token:
+              batch, t, heads, kv_heads, dim, vdim, (1 if one_token else 2 if all_start else 0) if taps > 1 else 0, f, _stream())
+    if taps > 1 and not one_token and not all_start:
         _hip.call("nvh_conv_state_update", proj.data_ptr(), proj.stride(0), conv_state.data_ptr(), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch,
                   taps, channels, f, _stream())
     return q
@@ -843,12 +843,12 @@ def delta_rule(r, k, v, a_raw, lowrank, w2, w0, a_bias, state, slots, cu_seqlens
 
 
 def gated_delta_rule(qkv, b, a, conv_w, dt_bias, a_log, conv_state, state, slots, cu_seqlens_q, context_lens, heads: int, qk_heads: int,
-                     dk: int, dv: int, max_seqlen_q: int = 0) -> torch.Tensor:
+                     dk: int, dv: int, max_seqlen_q: int = 0, all_start: bool = False) -> torch.Tensor:
     """One step of the gated delta rule over the packed tokens: fp32 outputs [T, H*dv].  `qkv`: the column view q | k | v of the
     projection rows (qk_heads*dk, qk_heads*dk, heads*dv channels), convolved over time with `conv_w` [C, taps] (continued from
     `conv_state` [slots, taps - 1, C] fp32, then brought up to date) and passed through silu; `b`, `a`: column views [T, H] of the
     write-strength and decay logits.  `state` [slots, H, dk, dv] fp32 is read (unless the sequence starts in this step) and left
-    updated.  `max_seqlen_q` as in delta_rule."""
+    updated.  `max_seqlen_q` as in delta_rule; `all_start`: every sequence starts in this step (the carried inputs are then left in the first launch)."""
     f = _act_flag(qkv, b, a, conv_w, dt_bias, a_log)
     t, c = qkv.shape[0], 2 * qk_heads * dk + heads * dv
     taps = conv_w.shape[1]
@@ -859,11 +859,13 @@ def gated_delta_rule(qkv, b, a, conv_w, dt_bias, a_log, conv_state, state, slots
     assert state.dtype == F32 and state.is_contiguous() and tuple(state.shape[1:]) == (heads, dk, dv) and slots.dtype == torch.int32
     assert context_lens.dtype == torch.int32 and (cu_seqlens_q is None or cu_seqlens_q.dtype == torch.int32)
     pack = torch.empty(t, heads, 5 * dk + dv, dtype=F32, device=qkv.device)
-    _hip.call("nvh_gated_delta_prep", qkv.data_ptr(), qkv.stride(0), b.data_ptr(), b.stride(0), a.data_ptr(), a.stride(0), conv_w.data_ptr(),
+    starting = all_start and taps > 1 and cu_seqlens_q is not None
+    _hip.call("nvh_gated_delta_prep_starting" if starting else "nvh_gated_delta_prep", qkv.data_ptr(), qkv.stride(0), b.data_ptr(), b.stride(0), a.data_ptr(), a.stride(0), conv_w.data_ptr(),
               dt_bias.data_ptr(), a_log.data_ptr(), _p(conv_state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), pack.data_ptr(),
               batch, t, taps, heads, qk_heads, dk, dv, f, _stream())
-    _hip.call("nvh_conv_state_update", qkv.data_ptr(), qkv.stride(0), _p(conv_state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch,
-              taps, c, f, _stream())
+    if not starting:
+        _hip.call("nvh_conv_state_update", qkv.data_ptr(), qkv.stride(0), _p(conv_state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), batch,
+                  taps, c, f, _stream())
     return _delta_scan(pack, state, slots, cu_seqlens_q, context_lens, heads, dk, dv, max_seqlen_q)
 
 
@@ -968,10 +970,10 @@ def residual_subnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, mult: fl
     return h
 
 
-def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor | None, slots, cu_seqlens_q, context_lens) -> torch.Tensor:
+def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor | None, slots, cu_seqlens_q, context_lens, all_start: bool = False) -> torch.Tensor:
     """h_t = x_t + sum_k weight[:, k] x_(t - taps + 1 + k) over the fp32 stream x [T, dim] (the last tap on the token itself), in weight's
     type.  Rows before this step come from `state` [slots, taps - 1, dim] fp32 (zeros at a sequence's start), which is then brought up
-    to date with this step's rows."""
+    to date with this step's rows (in one launch where every sequence starts in this step, `all_start`)."""
     f = _act_flag(weight)
     t, dim = x.shape
     taps = weight.shape[1]
@@ -984,6 +986,10 @@ def stream_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor | Non
         assert t == batch
         _hip.call("nvh_stream_conv_step", x.data_ptr(), weight.data_ptr(), _p(state), slots.data_ptr(), context_lens.data_ptr(), h.data_ptr(), dim, batch, taps,
                   dim, f, _stream())
+        return h
+    if all_start and taps > 1:
+        _hip.call("nvh_stream_conv_starting", x.data_ptr(), weight.data_ptr(), _p(state), slots.data_ptr(), cu_seqlens_q.data_ptr(), context_lens.data_ptr(),
+                  h.data_ptr(), dim, batch, t, taps, dim, f, _stream())
         return h
     _hip.call("nvh_stream_conv", x.data_ptr(), weight.data_ptr(), _p(state), slots.data_ptr(), _p(cu_seqlens_q), context_lens.data_ptr(), h.data_ptr(), dim,
               batch, t, taps, dim, f, _stream())

@@ -11,7 +11,7 @@ from dataclasses import dataclass
 import torch
 
 FIELDS = ("cu_seqlens_q", "cu_seqlens_k", "max_seqlen_q", "max_seqlen_k", "slot_mapping", "context_lens",
-          "block_tables", "seq_need_compute_logits", "state_slots")
+          "block_tables", "seq_need_compute_logits", "state_slots", "all_start")
 
 
 @dataclass
@@ -25,6 +25,7 @@ class Context:
     block_tables: torch.Tensor | None = None      # int32 [B, W], -1 padded (0 padded in graph buffers)
     seq_need_compute_logits: torch.Tensor | None = None   # int32 [B']
     state_slots: torch.Tensor | None = None       # int32 [B]: recurrent-state slot of every sequence (-1: a padded row); not in the reference
+    all_start: bool = False                       # every sequence's first tokens are in this step: no recurrent state or carried input is read; not in the reference
 
 
 _current = Context()
@@ -36,7 +37,7 @@ def get_context() -> Context:
 
 def set_context(*args, **kwargs) -> None:
     """set_context(cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, slot_mapping,
-    context_lens, block_tables, seq_need_compute_logits[, state_slots]); every argument optional."""
+    context_lens, block_tables, seq_need_compute_logits[, state_slots, all_start]); every argument optional."""
     global _current
     if len(args) > len(FIELDS):
         raise TypeError(f"set_context takes at most {len(FIELDS)} positional arguments")
