@@ -34,19 +34,21 @@ struct DecodeItems {
     const int32_t *item_seq, *item_range, *seq_active, *seq_chunk;
     int batch;
     int max_ranges;
+    const int32_t* order;      // uniform grid: the sequence that blockIdx.z stands for (null: itself)
     const NvhDecodePiece* pieces;  // pieces (common.h): the list
 };
 
-// PIECES: a decode step of sequences that are otherwise one range each (more than 16 with 8 kv heads).  One workgroup a sequence and head left 256 CUs to wait for
+// PIECES: a decode step of 17 .. 64 sequences (with 8 kv heads), which are one range each otherwise.  One workgroup a sequence and head left 256 CUs to wait for
 // the longest context: a CU alone takes in a trip of 64 keys in 0.95 us whatever is asked for, 24 sequences of 100..2047 keys took 30.1 us where their bytes need
 // 16.7, and two workgroups on a CU share its rate, so more and shorter ranges dealt out as they come were slower still (512 keys each: 31).  The step's first
 // launch (elementwise.hip, embedding_pieces_kernel) therefore lays out a list of pieces, the same for every layer: sequences above one and a half times a CU's
 // share of all trips are cut, the pieces lie by length, and where the contexts are long (six trips a CU and more) a workgroup walks a chain of them (the longest,
 // then the shortest, ..), so that 256 workgroups, one a CU, end together.  Short contexts keep a workgroup a piece: on one CU several of them hide each other's
 // way to the first key (33 sequences of 64 keys: 1160 us a step either way, 1255 one at a time).  A cut sequence's last piece to finish merges it.  us a decode
-// step of the 28-layer model, before (the sequences longest first) and now: 18 sequences of 100..2047 keys 1593 and 1345, 24 of them 1625 and 1435, 40 2075 and
-// 1961, 64 2470 and 2283, 128 3945 and 3800, 256 6280 and 6245; 48 of 300..1500 2010 and 1855; 24 of 1040 1367 and 1366; 64 of 64..100 1235 and 1240.
-// Sequences above 1.0 and 1.25 shares cut: 24 of 1040 1517 for 1366.
+// step of the 28-layer model, before and now: 18 sequences of 100..2047 keys 1593 and 1345, 24 of them 1625 and 1437, 40 2075 and 1961, 64 2470 and 2283; 48 of
+// 300..1500 2010 and 1855; 24 of 1040 1367 and 1366; 64 of 64..100 1235 and 1240.  Sequences above 1.0 and 1.25 shares cut: 24 of 1040 1517 for 1366.  More
+// sequences keep a workgroup each, the longest first: the chains' registers leave a CU three workgroups instead of four (128 of 100..2047 3945 and 3800, but 220 of
+// 60 1798 and 1853), and a list without chains gains nothing on an order (256 of 100..2047 6251 and 6432).
 //
 // FUSED: `q` is the raw fused qkv row of the step's single new token per sequence.  The kernel applies the
 // q/k epilogue itself (per-head RMSNorm + RoPE, qknorm_rope_head) and writes the new token's K/V to their cache slot
@@ -85,18 +87,20 @@ __global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decod
     int split, b, num_splits, ctx, chunk, active, piece_start = 0, piece_end = 0, page = 0;
     int64_t pos = 0;
     if constexpr (PIECES) {
+        // (one entry for all lanes: into scalar registers, as every address below is built on it)
         const NvhDecodePiece piece = items.pieces[at];
-        b = piece.seq & 0xffff;
-        if (b >= items.batch || (CHAINS && piece.follows && at == blockIdx.z)) return;   // block-uniform: none, or another workgroup's
-        at = piece.next;
-        split = piece.seq >> 16 & 0xff;
-        active = piece.seq >> 24;
+        const int entry = __builtin_amdgcn_readfirstlane(piece.seq);
+        b = entry & 0xffff;
+        if (b >= items.batch || (CHAINS && at == (int)blockIdx.z && __builtin_amdgcn_readfirstlane(piece.follows))) return;   // block-uniform: none, or another workgroup's
+        at = __builtin_amdgcn_readfirstlane(piece.next);
+        split = entry >> 16 & 0xff;
+        active = entry >> 24;
         num_splits = NVH_PIECE_RANGES;
-        piece_start = piece.start;
-        piece_end = piece.end;
-        ctx = piece.context;
-        page = piece.page;
-        pos = piece.position;
+        piece_start = __builtin_amdgcn_readfirstlane(piece.start);
+        piece_end = __builtin_amdgcn_readfirstlane(piece.end);
+        ctx = __builtin_amdgcn_readfirstlane(piece.context);
+        page = __builtin_amdgcn_readfirstlane(piece.page);
+        pos = __builtin_amdgcn_readfirstlane(piece.position);
         chunk = 0;
     } else if (items.item_seq) {                             // work list
         b = items.item_seq[blockIdx.z];
@@ -112,7 +116,7 @@ __global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decod
         // transposed order - the 8 heads of a sequence side by side on one XCD, whole 2-KB token rows per XCD - measured
         // 6.49 ms against 6.29 ms per step of 256 sequences: not taken)
         split = blockIdx.x;
-        b = blockIdx.z;
+        b = items.order ? items.order[blockIdx.z] : blockIdx.z;
         num_splits = gridDim.x;
         ctx = ctx_lens[b];
         chunk = decode_range_keys(ctx, num_splits, min_range);
@@ -897,8 +901,23 @@ extern "C" int32_t nvh_attn_decode_items(const void* q, int64_t q_token_stride, 
     NVH_REQUIRE(item_seq, NVH_EINVAL, "nvh_attn_decode_items: null work list");
     DecodeArgs a{q, q_token_stride, const_cast<void*>(k_cache), const_cast<void*>(v_cache), context_lens, block_tables,
                  table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace,
-                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
+                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr, nullptr}, num_items};
     return launch_decode<false>("nvh_attn_decode_items", a, FusedQkv{});
+}
+
+int32_t nvh_attn_decode_fused_qkv_ordered(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
+                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                          int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys, void* workspace,
+                                          const int32_t* order, hipStream_t stream) {
+    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
+    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
+                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
+    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
+                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, stream, DecodeItems{}, 0};
+    a.items.order = order;
+    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
+                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }
 
 extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stride, const void* q_norm_weight,
@@ -908,13 +927,9 @@ extern "C" int32_t nvh_attn_decode_fused_qkv(const void* qkv, int64_t token_stri
                                              int64_t batch, int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim,
                                              float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys,
                                              void* workspace, nvh_stream_t stream) {
-    NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
-    NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
-                "nvh_attn_decode_fused_qkv: 16-byte alignment required");
-    DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
-                 num_kv_heads, head_dim, softmax_scale, out, num_splits, min_range_keys, workspace, (hipStream_t)stream, DecodeItems{}, 0};
-    return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
-                               FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
+    return nvh_attn_decode_fused_qkv_ordered(qkv, token_stride, q_norm_weight, k_norm_weight, eps, positions, cos_sin, k_cache, v_cache, context_lens,
+                                             block_tables, table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, num_splits,
+                                             min_range_keys, workspace, nullptr, (hipStream_t)stream);
 }
 
 int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
@@ -924,7 +939,7 @@ int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, 
     NVH_REQUIRE(q_norm_weight && k_norm_weight && positions && cos_sin && pieces.pieces && pieces.arrivals, NVH_EINVAL, "nvh_attn_decode_fused_qkv: null pointer");
     NVH_REQUIRE(nvh_aligned16(q_norm_weight) && nvh_aligned16(k_norm_weight) && nvh_aligned16(cos_sin), NVH_EINVAL,
                 "nvh_attn_decode_fused_qkv: 16-byte alignment required");
-    NVH_REQUIRE(num_kv_heads > 0 && batch <= NVH_PIECE_ROWS && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
+    NVH_REQUIRE(nvh_takes_pieces(batch, num_kv_heads) && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
                 "nvh_attn_decode_fused_qkv: %ld sequences in %d pieces", (long)batch, pieces.capacity);
     DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
                  num_kv_heads, head_dim, softmax_scale, out, NVH_PIECE_RANGES, 0, workspace, stream, DecodeItems{}, pieces.capacity, pieces.arrivals};
@@ -947,7 +962,7 @@ extern "C" int32_t nvh_attn_decode_fused_qkv_items(const void* qkv, int64_t toke
                 "nvh_attn_decode_fused_qkv_items: 16-byte alignment required");
     DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
                  num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace, (hipStream_t)stream,
-                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
+                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr, nullptr}, num_items};
     return launch_decode<true>("nvh_attn_decode_fused_qkv_items", a,
                                FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }

@@ -63,6 +63,17 @@ int32_t nvh_noalloc_scratch(float** out);
 // Device address, on the current GPU, of the arrival counters the decode attention uses to merge key ranges in its own
 // launch (resolved on first use, or by nvh_device_check before a graph capture).
 int32_t nvh_decode_arrivals(unsigned** out);
+// nvh_attn_decode_fused_qkv whose sequences are dispatched in the given order (attention_decode.hip; null: as they lie), and nvh_embedding with
+// one workgroup more that leaves that order, the longest context first (elementwise.hip).
+#define NVH_ORDER_MAX 1024
+int32_t nvh_attn_decode_fused_qkv_ordered(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
+                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
+                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,
+                                          int64_t head_dim, float softmax_scale, void* out, int32_t num_splits, int32_t min_range_keys, void* workspace,
+                                          const int32_t* order, hipStream_t stream);
+int32_t nvh_embedding_order(const int64_t* ids, const void* table, void* out, int64_t num_tokens, int64_t dim, int64_t vocab_start, int64_t vocab_rows,
+                            const int32_t* context_lens, int32_t* order, int64_t batch, hipStream_t st);
+
 // Decode attention over pieces that the step itself lays out (attention_decode.hip, "Pieces"): written by nvh_embedding_pieces (elementwise.hip), read by the
 // attention of every layer.
 struct NvhDecodePiece {
@@ -78,17 +89,17 @@ struct NvhDecodePieces {
     unsigned* arrivals;        // [rows * kv heads], zero: ranges of a sequence that have left their partial result
     int capacity;              // nvh_piece_capacity()
 };
-#define NVH_PIECE_ROWS 1024    // most sequences of a step with pieces
 #define NVH_PIECE_RANGES 8     // most pieces of a sequence
 #define NVH_PIECE_TRIPS 8      // sequences of up to so many trips of 64 keys are not cut
 #define NVH_CHAIN_TRIPS 6      // trips a workgroup from which on pieces are chained
 static inline int nvh_pieces_per_head(int64_t num_kv_heads) { return num_kv_heads < 256 ? (int)(256 / num_kv_heads) : 1; }
-// Places in the list: one a sequence, and for up to two sequences a workgroup some that cutting fills (pieces are made longer until they are enough); above
-// that nothing is cut.  Every place is a workgroup, and an empty one costs about 10 ns: up to one sequence a workgroup as many as cutting by one and a half
-// shares can fill, above that a quarter (64 of 64..100 keys 1246 us a step with two thirds and 1240, 1235 without any).
+static inline bool nvh_takes_pieces(int64_t rows, int64_t num_kv_heads) { return num_kv_heads > 0 && rows > 0 && rows <= 2 * nvh_pieces_per_head(num_kv_heads); }
+// Places in the list: one a sequence and some that cutting fills (pieces are made longer until they are enough).  Every place is a workgroup, and an empty one
+// costs about 10 ns: up to one sequence a workgroup as many as cutting by one and a half shares can fill, above that a quarter (64 of 64..100 keys 1246 us a step
+// with two thirds and 1240, 1235 without any).
 static inline int nvh_piece_capacity(int64_t rows, int64_t num_kv_heads) {
     const int per_head = nvh_pieces_per_head(num_kv_heads);
-    return (int)rows + (rows <= per_head ? (2 * per_head + 2) / 3 : rows <= 2 * per_head ? (per_head + 3) / 4 : 0);
+    return (int)rows + (rows <= per_head ? (2 * per_head + 2) / 3 : (per_head + 3) / 4);
 }
 int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,

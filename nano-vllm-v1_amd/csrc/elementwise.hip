@@ -570,6 +570,45 @@ extern "C" int32_t nvh_embedding(const int64_t* ids, const void* table, void* ou
     return NVH_OK;
 }
 
+// The same launch with one workgroup more, which leaves the sequences of a decode batch in order of their context lengths, the longest
+// first (ties by index): order[rank] = sequence.  A sequence's rank is the number of sequences in front of it, counted from LDS - about
+// 1 us for 512 sequences, beside the rows' copies.
+__global__ __launch_bounds__(256) void embedding_order_kernel(const int64_t* __restrict__ ids, const bf16* __restrict__ table, bf16* __restrict__ out, int dim,
+                                                              int64_t vstart, int64_t vrows, const int32_t* __restrict__ ctx_lens,
+                                                              int32_t* __restrict__ order, int batch) {
+    __shared__ int32_t len[NVH_ORDER_MAX];
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < batch; i += 256) len[i] = ctx_lens[i];
+        __syncthreads();
+        for (int i = threadIdx.x; i < batch; i += 256) {
+            const int mine = len[i];
+            int rank = 0;
+            for (int j = 0; j < batch; ++j) rank += len[j] > mine || (len[j] == mine && j < i);
+            order[rank] = i;
+        }
+        return;
+    }
+    const int64_t t = blockIdx.x - 1;
+    const int64_t id = ids[t] - vstart;
+    const bool hit = id >= 0 && id < vrows;
+    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int c = threadIdx.x; c < (dim >> 3); c += 256) {
+        bf16x8 v = zero;
+        if (hit) v = *reinterpret_cast<const bf16x8*>(table + id * dim + c * 8);
+        *reinterpret_cast<bf16x8*>(out + t * dim + c * 8) = v;
+    }
+}
+
+int32_t nvh_embedding_order(const int64_t* ids, const void* table, void* out, int64_t num_tokens, int64_t dim, int64_t vocab_start, int64_t vocab_rows,
+                            const int32_t* context_lens, int32_t* order, int64_t batch, hipStream_t st) {
+    NVH_REQUIRE(ids && table && out && context_lens && order, NVH_EINVAL, "nvh_embedding: null pointer");
+    NVH_REQUIRE(dim > 0 && dim % 8 == 0 && nvh_aligned16(table) && nvh_aligned16(out), NVH_EINVAL, "nvh_embedding: dim %% 8 and 16-byte alignment required");
+    NVH_REQUIRE(batch >= 0 && batch <= NVH_ORDER_MAX, NVH_EINVAL, "nvh_embedding: %ld sequences to order (at most %d)", (long)batch, NVH_ORDER_MAX);
+    embedding_order_kernel<<<(unsigned)num_tokens + 1, 256, 0, st>>>(ids, (const bf16*)table, (bf16*)out, (int)dim, vocab_start, vocab_rows, context_lens, order, (int)batch);
+    NVH_CHECK_LAUNCH("embedding");
+    return NVH_OK;
+}
+
 // nvh_embedding with one workgroup more, which lays out the pieces of the step's decode attention (attention_decode.hip, PIECES): how long a piece may be
 // follows from the sum of all contexts and where a sequence is cut from that and its own length, so the order that sequences come in changes no bit of a result.
 // Pieces are put in order of their length by counting (one place a length in trips; equal ones as the counters deal them out, which decides where they run).
@@ -586,14 +625,13 @@ __global__ __launch_bounds__(256) void embedding_pieces_kernel(const int64_t* __
         for (int i = tid; i < batch; i += 256) atomicAdd(&total, (max(ctx_lens[i], 0) + 63) >> 6);
         for (int i = tid; i < batch * hkv; i += 256) pl.arrivals[i] = 0u;
         __syncthreads();
-        const bool chains = may_chain && pl.capacity > batch && total >= NVH_CHAIN_TRIPS * per_head;
+        const bool chains = may_chain && total >= NVH_CHAIN_TRIPS * per_head;
         int most = max((int)(((int64_t)total * 3 / 2 + per_head - 1) / per_head), NVH_PIECE_TRIPS);   // trips of a piece
-        if (pl.capacity == batch) most = 1 << 26;            // (no context is longer)
         auto pieces_of = [&](int trips) {
             const int each = max(most, (trips + NVH_PIECE_RANGES - 1) / NVH_PIECE_RANGES);
             return max((trips + each - 1) / each, 1);
         };
-        for (;;) {                                           // (ends: at 2^26 trips nothing is cut)
+        for (;;) {                                           // (ends: no context has 2^26 trips, so there nothing is cut)
             if (tid == 0) pieces = 0;
             __syncthreads();
             for (int i = tid; i < batch; i += 256) atomicAdd(&pieces, pieces_of((max(ctx_lens[i], 0) + 63) >> 6));
@@ -647,7 +685,7 @@ int32_t nvh_embedding_pieces(const int64_t* ids, const void* table, void* out, i
     NVH_REQUIRE(ids && table && out && context_lens && positions && block_tables && pieces.pieces && pieces.arrivals, NVH_EINVAL, "nvh_embedding: null pointer");
     NVH_REQUIRE(dim > 0 && dim % 8 == 0 && nvh_aligned16(table) && nvh_aligned16(out), NVH_EINVAL, "nvh_embedding: dim %% 8 and 16-byte alignment required");
     const int per_head = nvh_pieces_per_head(num_kv_heads);
-    NVH_REQUIRE(batch >= 0 && batch <= NVH_PIECE_ROWS && num_kv_heads > 0 && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
+    NVH_REQUIRE(nvh_takes_pieces(batch, num_kv_heads) && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
                 "nvh_embedding: %ld sequences in %d pieces a head", (long)batch, pieces.capacity);
     // (chains: up to four query heads a kv head, attn_decode_kernel)
     embedding_pieces_kernel<<<(unsigned)num_tokens + 1, 256, 0, st>>>(ids, (const bf16*)table, (bf16*)out, (int)dim, vocab_start, vocab_rows, context_lens, positions,

@@ -13,6 +13,7 @@ struct Workspace {
     float* slabs;
     void* decode_ws;
     void* varlen_ws;
+    int32_t* order;
     NvhDecodePieces pieces;
     int64_t total;
 };
@@ -50,10 +51,11 @@ Workspace carve(const nvh_qwen3_model* md, int64_t t, int64_t b, int32_t decode_
                                     ? (smax > 1 ? smax * t * h : 0) : (sq > 1 ? sq * t * (qsz + 2 * kvsz) : 0);
     w.slabs = (float*)take(slab_floats * 4);
     // (pieces of the decode attention: only where a sequence is otherwise one range)
-    const int64_t rows = decode_splits == 1 && b <= NVH_PIECE_ROWS ? b : 0;
-    w.decode_ws = take(nvh_attn_decode_workspace_bytes(b, md->num_q_heads, d, rows ? NVH_PIECE_RANGES : decode_splits));
+    const int64_t most = 2 * nvh_pieces_per_head(md->num_kv_heads), rows = decode_splits == 1 ? (b < most ? b : most) : 0;
+    w.decode_ws = take(rows ? nvh_attn_decode_workspace_bytes(rows, md->num_q_heads, d, NVH_PIECE_RANGES) : nvh_attn_decode_workspace_bytes(b, md->num_q_heads, d, decode_splits));
     w.varlen_ws = take(nvh_attn_varlen_workspace_bytes(t, md->num_q_heads, d, varlen_splits));
-    w.pieces.capacity = nvh_piece_capacity(rows, md->num_kv_heads);
+    w.order = (int32_t*)take(b * 4);
+    w.pieces.capacity = nvh_piece_capacity(rows, md->num_kv_heads) + (int)most;      // (of fewer rows may be more)
     w.pieces.pieces = (NvhDecodePiece*)take(rows ? w.pieces.capacity * (int64_t)sizeof(NvhDecodePiece) : 0);
     w.pieces.arrivals = (unsigned*)take(rows * md->num_kv_heads * 4);
     w.total = off;
@@ -70,7 +72,7 @@ extern "C" int64_t nvh_qwen3_workspace_bytes(const nvh_qwen3_model* model, int64
 
 // The fused decode attention of layer l over the first `rows` sequences of the step: uniform grid or work list.
 static int32_t decode_attention(const nvh_qwen3_model* md, const nvh_step* st, int l, const bf16* qkv, int64_t qkv_n, void* kc, void* vc,
-                                int64_t rows, float scale, bf16* attn, int32_t dsplits, void* ws, const NvhDecodePieces* pieces, nvh_stream_t stream) {
+                                int64_t rows, float scale, bf16* attn, int32_t dsplits, void* ws, const NvhDecodePieces* pieces, const int32_t* order, nvh_stream_t stream) {
     if (st->decode_items > 0)
         return nvh_attn_decode_fused_qkv_items(qkv, qkv_n, md->q_norm[l], md->k_norm[l], md->eps, st->positions, md->cos_sin, kc, vc,
                                                st->context_lens, st->block_tables, st->table_stride, rows, md->num_q_heads,
@@ -80,9 +82,9 @@ static int32_t decode_attention(const nvh_qwen3_model* md, const nvh_step* st, i
         return nvh_attn_decode_fused_qkv_pieces(qkv, qkv_n, md->q_norm[l], md->k_norm[l], md->eps, st->positions, md->cos_sin, kc, vc, st->context_lens,
                                                 st->block_tables, st->table_stride, rows, md->num_q_heads, md->num_kv_heads, md->head_dim, scale, attn, ws,
                                                 *pieces, (hipStream_t)stream);
-    return nvh_attn_decode_fused_qkv(qkv, qkv_n, md->q_norm[l], md->k_norm[l], md->eps, st->positions, md->cos_sin, kc, vc, st->context_lens,
-                                     st->block_tables, st->table_stride, rows, md->num_q_heads, md->num_kv_heads, md->head_dim, scale, attn, dsplits,
-                                     st->decode_min_range, ws, stream);
+    return nvh_attn_decode_fused_qkv_ordered(qkv, qkv_n, md->q_norm[l], md->k_norm[l], md->eps, st->positions, md->cos_sin, kc, vc,
+                                             st->context_lens, st->block_tables, st->table_stride, rows, md->num_q_heads, md->num_kv_heads,
+                                             md->head_dim, scale, attn, dsplits, st->decode_min_range, ws, order, (hipStream_t)stream);
 }
 
 #define FWD(call)                 \
@@ -198,10 +200,16 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
     const int64_t decode_rows = st->mode == NVH_MODE_DECODE ? b : prefix;
     NvhDecodePieces own = w.pieces;
     own.capacity = nvh_piece_capacity(decode_rows, md->num_kv_heads);
-    const NvhDecodePieces* const pieces = runs(0) && last_part > 0 && decode_rows > 0 && decode_rows <= NVH_PIECE_ROWS && dsplits == 1 && b <= NVH_PIECE_ROWS &&
-                                          st->decode_items == 0 && !nvh_switch_on(SW_NO_DECODE_PIECES) ? &own : nullptr;
+    const NvhDecodePieces* const pieces = runs(0) && last_part > 0 && dsplits == 1 && nvh_takes_pieces(decode_rows, hkv) && st->decode_items == 0 &&
+                                          !nvh_switch_on(SW_NO_DECODE_PIECES) ? &own : nullptr;
+    // Decode attention without a work list or pieces: the sequences are dispatched longest first.  More workgroups than fit at once are started as others
+    // end, and a long context among the last ones runs on alone (256 sequences of 100..2047 keys, a layer's launch: 201 us as they come, 177 us
+    // in order; 100 of 128..1151 keys: 57 -> 52 us).  Only where there are more workgroups than CUs, and in calls that run the embedding, which
+    // leaves the order, themselves.
+    const int32_t* const order = runs(0) && last_part > 0 && !pieces && decode_rows * hkv * dsplits > 256 && decode_rows <= NVH_ORDER_MAX && st->decode_items == 0 ? w.order : nullptr;
     if (runs(0)) {
         if (pieces) FWD(nvh_embedding_pieces(st->input_ids, md->embed, w.residual, t, h, md->vocab_start, md->vocab_rows, st->context_lens, st->positions, st->block_tables, st->table_stride, decode_rows, hq, hkv, *pieces, (hipStream_t)stream));
+        else if (order) FWD(nvh_embedding_order(st->input_ids, md->embed, w.residual, t, h, md->vocab_start, md->vocab_rows, st->context_lens, w.order, decode_rows, (hipStream_t)stream));
         else FWD(nvh_embedding(st->input_ids, md->embed, w.residual, t, h, md->vocab_start, md->vocab_rows, stream));
         if (comm) FWD(nvh_allreduce_bf16(comm, w.residual, w.residual, t * h, stream));
     }
@@ -282,7 +290,7 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
         }
         if (decode_fused) {
             // one launch: q/k norm + RoPE + KV store of the new token + attention
-            FWD(decode_attention(md, st, l, w.qkv, qkv_n, kc, vc, b, scale, w.attn, dsplits, w.decode_ws, pieces, stream));
+            FWD(decode_attention(md, st, l, w.qkv, qkv_n, kc, vc, b, scale, w.attn, dsplits, w.decode_ws, pieces, order, stream));
         } else {
             if (t > prefix && !qk_done)
                 FWD(nvh_qknorm_rope_store(w.qkv + prefix * qkv_n, qkv_n, hq, hkv, md->q_norm[l], md->k_norm[l], md->eps,
@@ -293,7 +301,7 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
                                     d, scale, w.attn, dsplits, st->decode_min_range, w.decode_ws, stream));
             } else if (prefix > 0) {
                 // (the qk-norm / rope / store launch above covered only the tokens past the one-token sequences)
-                FWD(decode_attention(md, st, l, w.qkv, qkv_n, kc, vc, prefix, scale, w.attn, dsplits, w.decode_ws, pieces, stream));
+                FWD(decode_attention(md, st, l, w.qkv, qkv_n, kc, vc, prefix, scale, w.attn, dsplits, w.decode_ws, pieces, order, stream));
                 if (b > prefix)
                     FWD(nvh_attn_varlen_beside(w.qkv + prefix * qkv_n, qkv_n, kc, vc, kvsz, st->cu_seqlens_q_tail, st->cu_seqlens_k_tail,
                                         st->block_tables + prefix * st->table_stride, st->table_stride, b - prefix, st->max_seqlen_q,
