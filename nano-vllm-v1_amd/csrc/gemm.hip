@@ -1482,8 +1482,8 @@ extern "C" int32_t nvh_gemm_bf16_nt(const void* x, int64_t x_row_stride, const v
 static bool takes_kwaves(const GemmArgs& a);
 
 // ---- a projection with its ungated activation, up to 64 rows: act(bf16(x W^T + bias)) in the product's epilogue, on the tiles that nvh_gemm_bf16_nt takes
-// there (the same bits as the two launches).  An activation's launch over so few rows is its 4.7 us whatever it does; us of both and of one, 64 rows: 4608 x 1024
-// 11.3 and 6.9 (xIELU).  Larger calls keep two launches: their tiles leave through LDS.
+// there (the same bits as the two launches).  us in a step's trace, 64 x 4608 x 1024 and its xIELU: 6.9 and 4.5, together 7.9;
+// a step of 8 such layers 754 -> 740.  Larger calls keep two launches: their tiles leave through LDS.
 enum class ActTile { NONE, T16x32, T32x32, T64x16, T64x32 };
 static ActTile act_tile(int64_t M, int64_t N, int64_t K) {
     GemmArgs a{};

@@ -82,3 +82,20 @@ def test_pieces_give_what_one_range_a_sequence_gives(tmp_path, hq, hkv, rows, ki
         assert torch.equal(got["pieces"], one)
     a, b = got["pieces"].float(), one.float()
     assert (a - b).norm() <= 2.0 ** -7 * b.norm() and (a - b).abs().max() <= 2.0 ** -4 * b.abs().max()
+
+
+@pytest.mark.parametrize("lq,lk", [(1, 700), (33, 600), (257, 513), (512, 512), (900, 1900), (1000, 1000)])
+def test_prompt_attention_rows_do_not_depend_on_the_block(lq, lk, switches):
+    """Query blocks of 32 and of 64 rows (taken where another step runs beside a mixed one): the same bits for every row."""
+    from nanovllm import ops
+    g = torch.Generator().manual_seed(lq + lk)
+    q = torch.randn(lq, 16, 128, generator=g).bfloat16().cuda()
+    pages = -(-lk // 256)
+    kc, vc = (torch.randn(pages, 256, 8, 128, generator=g).bfloat16().cuda() for _ in range(2))
+    table = torch.randperm(pages, generator=g).int()[None].cuda()
+    cu = lambda n: torch.tensor([0, n], dtype=torch.int32).cuda()
+    got = []
+    for blocks in (-1, 0):
+        switches("NVH_ATTN_RB1", blocks)
+        got.append(ops.attn_varlen(q, kc, vc, cu(lq), cu(lk), lq, 128 ** -0.5, block_tables=table, max_seqlen_k=lk, num_splits=1))
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)
