@@ -93,13 +93,17 @@ struct NvhDecodePieces {
 #define NVH_PIECE_TRIPS 8      // sequences of up to so many trips of 64 keys are not cut
 #define NVH_CHAIN_TRIPS 6      // trips a workgroup from which on pieces are chained
 static inline int nvh_pieces_per_head(int64_t num_kv_heads) { return num_kv_heads < 256 ? (int)(256 / num_kv_heads) : 1; }
-static inline bool nvh_takes_pieces(int64_t rows, int64_t num_kv_heads) { return num_kv_heads > 0 && rows > 0 && rows <= 2 * nvh_pieces_per_head(num_kv_heads); }
+// The captured step that a batch of so many rows runs in (ModelRunner.decode_buckets).  Whether there are pieces, and how many places for them beside one a
+// sequence, decides where sequences are cut and so the last bits: both follow from this, not from the rows, so that a batch run eagerly is cut like the captured
+// one (a padded row takes a place of its own and nothing else).
+static inline int64_t nvh_captured_rows(int64_t rows) { return rows > 8 ? (rows + 15) / 16 * 16 : rows > 4 ? 8 : rows > 2 ? 4 : rows; }
+static inline bool nvh_takes_pieces(int64_t rows, int64_t num_kv_heads) { return num_kv_heads > 0 && rows > 0 && nvh_captured_rows(rows) <= 2 * nvh_pieces_per_head(num_kv_heads); }
 // Places in the list: one a sequence and some that cutting fills (pieces are made longer until they are enough).  Every place is a workgroup, and an empty one
 // costs about 10 ns: up to one sequence a workgroup as many as cutting by one and a half shares can fill, above that a quarter (64 of 64..100 keys 1246 us a step
 // with two thirds and 1240, 1235 without any).
 static inline int nvh_piece_capacity(int64_t rows, int64_t num_kv_heads) {
     const int per_head = nvh_pieces_per_head(num_kv_heads);
-    return (int)rows + (rows <= per_head ? (2 * per_head + 2) / 3 : (per_head + 3) / 4);
+    return (int)rows + (nvh_captured_rows(rows) <= per_head ? (2 * per_head + 2) / 3 : (per_head + 3) / 4);
 }
 int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,

@@ -36,16 +36,20 @@ def _sequences(runner, lens, g):
 
 
 def _lens(kind, rows, g):
+    if kind in ("long third", "long tenth"):                 # a third or a tenth of them cut in three
+        return [2047 if i % (3 if kind == "long third" else 10) == 0 else 64 for i in range(rows)]
     if kind == "short":                                      # nothing is cut, a workgroup a piece
         return torch.randint(1, 130, (rows,), generator=g).tolist()
-    if kind == "one long":                                   # one sequence cut as often as it can be
+    if kind == "one long":                                   # one sequence cut in four: the most that the engine's contexts without a work list give
         return [2047] + [1 + i % 64 for i in range(rows - 1)]
     return [64 + (2047 - 64) * i // (rows - 1) for i in range(rows)]          # chains; ends on and around the edges of trips and pages
 
 
 @pytest.mark.parametrize("hq,hkv,rows,kind", [(16, 8, 17, "spread"), (16, 8, 32, "one long"), (16, 8, 33, "spread"), (16, 8, 64, "spread"), (16, 8, 64, "one long"),
                                               (16, 8, 65, "spread"), (16, 8, 40, "short"), (8, 8, 20, "spread"), (32, 8, 33, "spread"), (40, 8, 20, "spread"),
-                                              (40, 8, 33, "one long"), (64, 8, 33, "spread"), (16, 4, 66, "spread")])
+                                              (40, 8, 33, "one long"), (64, 8, 33, "spread"), (16, 4, 66, "spread"),
+                                              # (6 kv heads: 40 rows have places for another number of cuts than the captured step's 48; 82 have a list, its 96 have none)
+                                              (12, 6, 40, "long third"), (12, 6, 82, "long tenth")])
 def test_pieces_give_what_one_range_a_sequence_gives(tmp_path, hq, hkv, rows, kind):
     """A decode step over pieces against the same step with a workgroup a sequence, which other tests hold against the oracle.  Attention outputs are sums in
     another order in fp32, rounded to bf16: through two layers and the head, logits within a few of bf16's 2^-8; uncut ones (short) to the bit.
