@@ -105,6 +105,9 @@ static inline int nvh_piece_capacity(int64_t rows, int64_t num_kv_heads) {
     const int per_head = nvh_pieces_per_head(num_kv_heads);
     return (int)rows + (nvh_captured_rows(rows) <= per_head ? (2 * per_head + 2) / 3 : (per_head + 3) / 4);
 }
+// Room for the list of any up to `rows` sequences: fewer may take more places (with 8 kv heads 32 take 54 and 33 take 41), and a mixed step of `rows` lays one
+// out for those of them that decode.
+static inline int nvh_piece_room(int64_t rows, int64_t num_kv_heads) { return (int)rows + (2 * nvh_pieces_per_head(num_kv_heads) + 2) / 3; }
 int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, const void* q_norm_weight, const void* k_norm_weight, float eps,
                                          const int64_t* positions, const float* cos_sin, void* k_cache, void* v_cache, const int32_t* context_lens,
                                          const int32_t* block_tables, int64_t table_stride, int64_t batch, int64_t num_q_heads, int64_t num_kv_heads,

@@ -55,8 +55,8 @@ Workspace carve(const nvh_qwen3_model* md, int64_t t, int64_t b, int32_t decode_
     w.decode_ws = take(rows ? nvh_attn_decode_workspace_bytes(rows, md->num_q_heads, d, NVH_PIECE_RANGES) : nvh_attn_decode_workspace_bytes(b, md->num_q_heads, d, decode_splits));
     w.varlen_ws = take(nvh_attn_varlen_workspace_bytes(t, md->num_q_heads, d, varlen_splits));
     w.order = (int32_t*)take(b * 4);
-    w.pieces.capacity = nvh_piece_capacity(rows, md->num_kv_heads) + (int)most;      // (of fewer rows may be more)
-    w.pieces.pieces = (NvhDecodePiece*)take(rows ? w.pieces.capacity * (int64_t)sizeof(NvhDecodePiece) : 0);
+    w.pieces.capacity = rows ? nvh_piece_room(rows, md->num_kv_heads) : 0;
+    w.pieces.pieces = (NvhDecodePiece*)take(w.pieces.capacity * (int64_t)sizeof(NvhDecodePiece));
     w.pieces.arrivals = (unsigned*)take(rows * md->num_kv_heads * 4);
     w.total = off;
     return w;
@@ -202,6 +202,7 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
     own.capacity = nvh_piece_capacity(decode_rows, md->num_kv_heads);
     const NvhDecodePieces* const pieces = runs(0) && last_part > 0 && dsplits == 1 && nvh_takes_pieces(decode_rows, hkv) && st->decode_items == 0 &&
                                           !nvh_switch_on(SW_NO_DECODE_PIECES) ? &own : nullptr;
+    NVH_REQUIRE(!pieces || own.capacity <= w.pieces.capacity, NVH_EINVAL, "nvh_qwen3_forward: %d pieces in room for %d", own.capacity, w.pieces.capacity);
     // Decode attention without a work list or pieces: the sequences are dispatched longest first.  More workgroups than fit at once are started as others
     // end, and a long context among the last ones runs on alone (256 sequences of 100..2047 keys, a layer's launch: 201 us as they come, 177 us
     // in order; 100 of 128..1151 keys: 57 -> 52 us).  Only where there are more workgroups than CUs, and in calls that run the embedding, which
