@@ -656,9 +656,10 @@ int32_t nvh_attn_varlen_beside(const void* q, int64_t q_token_stride, const void
         case 2: {
             // a grid that leaves half the CUs without a workgroup (one 1024-token chunk: 16 blocks x 8 kv heads): 32-row
             // blocks put a four-wave workgroup on every CU instead of an eight-wave one on every other (alone: 1024 queries and keys 21.5 us for 24.6,
-            // 924 queries of 1948 keys 36 for 38).  Not in a mixed step with another step in flight: a workgroup takes a CU's LDS whole either way, and
-            // half as many leave the other CUs to that step's decode attention and products (three steps of 924 new tokens and 100 decodes in flight
-            // 3940 -> 3555 us a step; steps of a chunk alone 2112 and 2126, no gain).  A row's bits are the same.
+            // 924 queries of 1948 keys 36 for 38).  Not in a mixed step while the step before it runs: a workgroup takes a CU's LDS whole either way, and half as
+            // many leave the other CUs to that step's decode attention and products (mixed steps of 924 new tokens and 100 decodes whose ids nobody reads
+            // 3690 -> 3480 us; with the ids read back, where nothing runs beside them, 4935 - 4960 in 32-row blocks and 4995 - 5000 in 64; chunks 2112 and
+            // 2126, no gain).  A row's bits are the same.
             const int rb1 = beside ? 0 : (int)nvh_switch_or(SW_ATTN_RB1, 128);     // A/B switch: 0 = never
             if (ks == 2 && wgs <= rb1) LAUNCH_VL(2, 1, 2, 2);
             else if (ks == 2) LAUNCH_VL(2, 2, 2, 2);

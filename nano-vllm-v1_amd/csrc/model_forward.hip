@@ -240,6 +240,15 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
                           so == 1 && sd == 1 && sq == 1 && d == 128 && st->mode != NVH_MODE_DECODE && t > prefix && parts_o > 0 && parts_d > 0 && parts_o <= 32 && parts_d <= 32 &&
                           nvh_gemm_rowscaled_supported(t, qkv_n, h, 2) && nvh_gemm_rowscaled_supported(t, 2 * md->inter, h, 1) && (int64_t)(parts_o > parts_d ? parts_o : parts_d) * 4 <= h * 2;
     float* const rowsq = reinterpret_cast<float*>(w.y);
+    // Prompt attention of a mixed step: is the step before this one still running?  That it left events does not say so: a loop that reads a mixed step's ids back
+    // before it goes on finds it ended (an event's query costs the host under 1 us).
+    bool beside = false;
+    if (ev_wait && prefix > 0 && b > prefix) {
+        const hipError_t e = hipEventQuery(ev_wait[md->layers - 1]);
+        if (e == hipErrorNotReady) (void)hipGetLastError();              // (no error: the answer)
+        NVH_REQUIRE(e == hipSuccess || e == hipErrorNotReady, NVH_ELAUNCH, "nvh_qwen3_forward: layer event query: %s", hipGetErrorString(e));
+        beside = e == hipErrorNotReady;
+    }
     for (int l = 0; l < md->layers; ++l) {
       if (runs(2 * l + 1)) {
         // the step before this one (on another stream) is done with the attention of this layer: its keys are in the
@@ -306,7 +315,7 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
                 if (b > prefix)
                     FWD(nvh_attn_varlen_beside(w.qkv + prefix * qkv_n, qkv_n, kc, vc, kvsz, st->cu_seqlens_q_tail, st->cu_seqlens_k_tail,
                                         st->block_tables + prefix * st->table_stride, st->table_stride, b - prefix, st->max_seqlen_q,
-                                        st->max_seqlen_k, t - prefix, hq, hkv, d, scale, w.attn + prefix * qsz, vsplits, w.varlen_ws, ev_wait != nullptr, stream));
+                                        st->max_seqlen_k, t - prefix, hq, hkv, d, scale, w.attn + prefix * qsz, vsplits, w.varlen_ws, beside, stream));
             } else if (st->mode == NVH_MODE_PAGED) {
                 FWD(nvh_attn_varlen(w.qkv, qkv_n, kc, vc, kvsz, st->cu_seqlens_q, st->cu_seqlens_k, st->block_tables,
                                     st->table_stride, b, st->max_seqlen_q, st->max_seqlen_k, t, hq, hkv, d, scale, w.attn, vsplits, w.varlen_ws, stream));

@@ -91,8 +91,9 @@ def test_pieces_give_what_one_range_a_sequence_gives(tmp_path, hq, hkv, rows, ki
 
 
 @pytest.mark.parametrize("lq,lk", [(1, 700), (33, 600), (257, 513), (512, 512), (900, 1900), (1000, 1000)])
-def test_prompt_attention_rows_do_not_depend_on_the_block(lq, lk, switches):
-    """Query blocks of 32 and of 64 rows (taken where another step runs beside a mixed one): the same bits for every row."""
+@pytest.mark.parametrize("splits", [1, 3])
+def test_prompt_attention_rows_do_not_depend_on_the_block(lq, lk, splits, switches):
+    """Query blocks of 32 rows (small grids) and of 64: the same bits for every row, in one key range and in several."""
     from nanovllm import ops
     g = torch.Generator().manual_seed(lq + lk)
     q = torch.randn(lq, 16, 128, generator=g).bfloat16().cuda()
@@ -103,8 +104,51 @@ def test_prompt_attention_rows_do_not_depend_on_the_block(lq, lk, switches):
     got = []
     for blocks in (-1, 0):
         switches("NVH_ATTN_RB1", blocks)
-        got.append(ops.attn_varlen(q, kc, vc, cu(lq), cu(lk), lq, 128 ** -0.5, block_tables=table, max_seqlen_k=lk, num_splits=1))
+        got.append(ops.attn_varlen(q, kc, vc, cu(lq), cu(lk), lq, 128 ** -0.5, block_tables=table, max_seqlen_k=lk, num_splits=splits))
     assert torch.isfinite(got[0]).all() and torch.equal(*got)
+
+
+def test_mixed_steps_in_flight_give_the_bits_of_one_stream(tmp_path):
+    """Three mixed steps in a row that read nothing back - decodes over pieces and portions of one prompt, each reading the keys of the one before, the last with
+    its keys in ranges - with steps in flight and without: the same logits and caches."""
+    from nanovllm.engine.sequence import Sequence
+    rows, portions = 33, [(1500, 300), (1800, 270), (2070, 300)]
+    g = torch.Generator().manual_seed(5)
+    lens = torch.randint(1, 900, (rows,), generator=g).tolist()
+    pages = [-(-(n + 3) // 256) for n in lens] + [10]
+    runner = _runner(tmp_path, 16, 8, 48, sum(pages), True)
+    runner.config.max_model_len = 4096
+    tokens = [torch.randint(0, 1024, (n + 3,), generator=g).tolist() for n in lens + [2367]]
+    tables, at = [], 0
+    for p in pages:
+        tables.append(list(range(at, at + p)))
+        at += p
+    cache = torch.randn(runner.kv_cache.shape, generator=g).bfloat16()
+    events, forward = [], runner.native.forward
+
+    def step(i):
+        seqs = []
+        for j, (tok, table) in enumerate(zip(tokens, tables)):
+            cached, new = portions[i] if j == rows else (lens[j] - 1 + i, 1)
+            s = Sequence(tok[:cached + new])
+            s.block_table, s.num_cached_tokens, s.num_new_tokens = table[:-(-(cached + new) // 256)], cached, new
+            seqs.append(s)
+        return runner.forward_logits(seqs)[0].clone()
+
+    got = []
+    try:
+        runner.native.forward = lambda *x, **k: (events.append((k["layer_events"], k["decode_prefix"])), forward(*x, **k))[1]
+        for overlap in (False, True):
+            runner.step_overlap, runner._last_step = overlap, None
+            runner.kv_cache.copy_(cache)
+            torch.cuda.synchronize()
+            logits = [step(i) for i in range(3)]
+            torch.cuda.synchronize()
+            got.append(logits + [runner.kv_cache.clone()])
+    finally:
+        runner.exit()
+    assert events == [((0, 0), rows)] * 3 + [((0, 1), rows), ((1, 2), rows), ((2, 1), rows)]
+    assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(*got))
 
 
 def _attention_runner(tmp_path, hq, hkv, slots, pages, max_len):
