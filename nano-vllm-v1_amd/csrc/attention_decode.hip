@@ -35,7 +35,6 @@ struct DecodeItems {
     int batch;
     int max_ranges;
     const int32_t* order;      // uniform grid: the sequence that blockIdx.z stands for (null: itself)
-    const NvhDecodePiece* pieces;  // pieces (common.h): the list
 };
 
 // PIECES: a decode step of 17 .. 64 sequences (with 8 kv heads), which are one range each otherwise.  One workgroup a sequence and head left 256 CUs to wait for
@@ -71,7 +70,7 @@ __global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decod
     const bf16* __restrict__ q, int64_t q_stride, bf16* __restrict__ kc, bf16* __restrict__ vc,
     const int32_t* __restrict__ ctx_lens, const int32_t* __restrict__ tables, int64_t table_stride, int hkv,
     float scale_log2, bf16* __restrict__ out, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int min_range, DecodeItems items, FusedQkv fz,
-    unsigned* __restrict__ arrivals) {
+    unsigned* __restrict__ arrivals, const NvhDecodePiece* __restrict__ pieces) {
     __shared__ float sm_acc[4][G][128];
     __shared__ float sm_ml[4][G][2];
     __shared__ int sm_last;
@@ -81,9 +80,6 @@ __global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decod
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15;
     const int rowid = w * 4 + (lane >> 4);
 
-    // (never taken: it brings every line of the arguments in with one wait, where the compiler fetches two of them behind the branches below; one sequence 818 us a
-    // step of 28 layers without it, 814 with it)
-    if (!PIECES && ((fz.q_norm_w == nullptr && FUSED) | (gridDim.x == 0) | (ctx_lens == nullptr) | (items.batch < 0) | (items.item_seq == reinterpret_cast<const int32_t*>(1)))) return;
     constexpr bool CHAINS = PIECES && G <= 4;                // (more heads: their registers would spill)
     int at = blockIdx.z;
     do {                                                     // (PIECES: a workgroup's pieces; otherwise once)
@@ -91,7 +87,7 @@ __global__ __launch_bounds__(256, G <= 2 ? (PIECES ? 3 : 4) : 2) void attn_decod
     int64_t pos = 0;
     if constexpr (PIECES) {
         // (one entry for all lanes: into scalar registers, as every address below is built on it)
-        const NvhDecodePiece piece = items.pieces[at];
+        const NvhDecodePiece piece = pieces[at];
         const int entry = __builtin_amdgcn_readfirstlane(piece.seq);
         b = entry & 0xffff;
         if (b >= items.batch || (CHAINS && at == (int)blockIdx.z && __builtin_amdgcn_readfirstlane(piece.follows))) return;   // block-uniform: none, or another workgroup's
@@ -753,6 +749,7 @@ struct DecodeArgs {
     DecodeItems items;              // neither item_seq nor pieces: uniform grid
     int64_t num_items;
     unsigned* arrivals = nullptr;   // pieces: the step's counters
+    const NvhDecodePiece* pieces = nullptr;
 };
 
 template <bool FUSED>
@@ -780,12 +777,12 @@ int32_t launch_decode(const char* name, const DecodeArgs& a, const FusedQkv& fz)
     }
     const float sl2 = a.softmax_scale * LOG2E;
     if constexpr (FUSED) {
-        if (a.items.pieces) {
+        if (a.pieces) {
             grid = dim3(1, (unsigned)a.num_kv_heads, (unsigned)a.num_items);
 #define LAUNCH_DEC(GG)                                                                                                                     \
     attn_decode_kernel<GG, true, true><<<grid, 256, 0, a.st>>>((const bf16*)a.q, a.q_token_stride, (bf16*)a.k_cache, (bf16*)a.v_cache,     \
                                                                a.context_lens, a.block_tables, a.table_stride, (int)a.num_kv_heads, sl2,    \
-                                                               (bf16*)a.out, ws_acc, ws_ml, min_range, a.items, fz, a.arrivals)
+                                                               (bf16*)a.out, ws_acc, ws_ml, min_range, a.items, fz, a.arrivals, a.pieces)
             switch (g) {
                 case 1: LAUNCH_DEC(1); break;
                 case 2: LAUNCH_DEC(2); break;
@@ -813,7 +810,7 @@ int32_t launch_decode(const char* name, const DecodeArgs& a, const FusedQkv& fz)
 #define LAUNCH_DEC(GG)                                                                                                  \
     attn_decode_kernel<GG, FUSED><<<grid, 256, 0, a.st>>>((const bf16*)a.q, a.q_token_stride, (bf16*)a.k_cache, (bf16*)a.v_cache, \
                                                           a.context_lens, a.block_tables, a.table_stride, (int)a.num_kv_heads, \
-                                                          sl2, (bf16*)a.out, ws_acc, ws_ml, min_range, a.items, fz, arrivals)
+                                                          sl2, (bf16*)a.out, ws_acc, ws_ml, min_range, a.items, fz, arrivals, nullptr)
     switch (g) {
         case 1: LAUNCH_DEC(1); break;
         case 2: LAUNCH_DEC(2); break;
@@ -904,7 +901,7 @@ extern "C" int32_t nvh_attn_decode_items(const void* q, int64_t q_token_stride, 
     NVH_REQUIRE(item_seq, NVH_EINVAL, "nvh_attn_decode_items: null work list");
     DecodeArgs a{q, q_token_stride, const_cast<void*>(k_cache), const_cast<void*>(v_cache), context_lens, block_tables,
                  table_stride, batch, num_q_heads, num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace,
-                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr, nullptr}, num_items};
+                 (hipStream_t)stream, DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
     return launch_decode<false>("nvh_attn_decode_items", a, FusedQkv{});
 }
 
@@ -945,9 +942,8 @@ int32_t nvh_attn_decode_fused_qkv_pieces(const void* qkv, int64_t token_stride, 
     NVH_REQUIRE(nvh_takes_pieces(batch, num_kv_heads) && pieces.capacity == nvh_piece_capacity(batch, num_kv_heads), NVH_EINVAL,
                 "nvh_attn_decode_fused_qkv: %ld sequences in %d pieces", (long)batch, pieces.capacity);
     DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
-                 num_kv_heads, head_dim, softmax_scale, out, NVH_PIECE_RANGES, 0, workspace, stream, DecodeItems{}, pieces.capacity, pieces.arrivals};
+                 num_kv_heads, head_dim, softmax_scale, out, NVH_PIECE_RANGES, 0, workspace, stream, DecodeItems{}, pieces.capacity, pieces.arrivals, pieces.pieces};
     a.items.batch = (int)batch;
-    a.items.pieces = pieces.pieces;
     return launch_decode<true>("nvh_attn_decode_fused_qkv", a,
                                FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }
@@ -965,7 +961,7 @@ extern "C" int32_t nvh_attn_decode_fused_qkv_items(const void* qkv, int64_t toke
                 "nvh_attn_decode_fused_qkv_items: 16-byte alignment required");
     DecodeArgs a{qkv, token_stride, k_cache, v_cache, context_lens, block_tables, table_stride, batch, num_q_heads,
                  num_kv_heads, head_dim, softmax_scale, out, max_ranges, 0, workspace, (hipStream_t)stream,
-                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr, nullptr}, num_items};
+                 DecodeItems{item_seq, item_range, seq_active, seq_chunk, (int)batch, max_ranges, nullptr}, num_items};
     return launch_decode<true>("nvh_attn_decode_fused_qkv_items", a,
                                FusedQkv{(const bf16*)q_norm_weight, (const bf16*)k_norm_weight, positions, cos_sin, eps});
 }
