@@ -44,8 +44,8 @@ struct DecodeItems {
 // share of all trips are cut, the pieces lie by length, and where the contexts are long (six trips a CU and more) a workgroup walks a chain of them (the longest,
 // then the shortest, ..), so that 256 workgroups, one a CU, end together.  Short contexts keep a workgroup a piece: on one CU several of them hide each other's
 // way to the first key (33 sequences of 64 keys: 1160 us a step either way, 1255 one at a time).  A cut sequence's last piece to finish merges it.  us a decode
-// step of the 28-layer model, before and now: 18 sequences of 100..2047 keys 1593 and 1345, 24 of them 1625 and 1437, 40 2075 and 1961, 64 2470 and 2283; 48 of
-// 300..1500 2010 and 1855; 24 of 1040 1367 and 1366; 64 of 64..100 1235 and 1240.  Sequences above 1.0 and 1.25 shares cut: 24 of 1040 1517 for 1366.  More
+// step of the 28-layer model, before and now: 18 sequences of 100..2047 keys 1596 and 1343, 24 of them 1623 and 1429, 40 2065 and 1947, 64 2459 and 2267; 48 of
+// 300..1500 2001 and 1842; 24 of 1040 1357 and 1360; 64 of 64..100 1234 and 1229; 48 of 100..200 1280 and 1285 (the list's own time and its empty places).  Sequences above 1.0 and 1.25 shares cut: 24 of 1040 1517 for 1366.  More
 // sequences keep a workgroup each, the longest first: the chains' registers leave a CU three workgroups instead of four (128 of 100..2047 3945 and 3800, but 220 of
 // 60 1798 and 1853), and a list without chains gains nothing on an order (256 of 100..2047 6251 and 6432).
 //

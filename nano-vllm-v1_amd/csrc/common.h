@@ -99,8 +99,8 @@ static inline int nvh_pieces_per_head(int64_t num_kv_heads) { return num_kv_head
 static inline int64_t nvh_captured_rows(int64_t rows) { return rows > 8 ? (rows + 15) / 16 * 16 : rows > 4 ? 8 : rows > 2 ? 4 : rows; }
 static inline bool nvh_takes_pieces(int64_t rows, int64_t num_kv_heads) { return num_kv_heads > 0 && rows > 0 && nvh_captured_rows(rows) <= 2 * nvh_pieces_per_head(num_kv_heads); }
 // Places in the list: one a sequence and some that cutting fills (pieces are made longer until they are enough).  Every place is a workgroup, and an empty one
-// costs about 10 ns: up to one sequence a workgroup as many as cutting by one and a half shares can fill, above that a quarter (64 of 64..100 keys 1246 us a step
-// with two thirds and 1240, 1235 without any).
+// costs about 10 ns: up to one sequence a workgroup as many as cutting by one and a half shares can fill, above that a quarter (64 of 64..100 keys: 6 us a step more
+// with two thirds).
 static inline int nvh_piece_capacity(int64_t rows, int64_t num_kv_heads) {
     const int per_head = nvh_pieces_per_head(num_kv_heads);
     return (int)rows + (nvh_captured_rows(rows) <= per_head ? (2 * per_head + 2) / 3 : (per_head + 3) / 4);
