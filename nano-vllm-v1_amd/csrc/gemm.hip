@@ -1490,7 +1490,7 @@ static ActTile act_tile(int64_t M, int64_t N, int64_t K) {
     a.M = (int)M, a.N = (int)N, a.K = (int)K, a.split_k = 1;
     if (M < 1 || M > 64 || N <= 0 || N % 4 || N > 32 * 256 || K <= 0 || K % BK || K >= (1 << 30) || tile_forced() || nvh_switch_on(SW_GEMM_NO_NT) || takes_kwaves(a)) return ActTile::NONE;
     switch (pick_tile(M, N, 1)) {
-        case T16x32: return nvh_cdiv(N, 32) > 768 ? ActTile::NONE : ActTile::T16x32;
+        case T16x32: return ActTile::T16x32;
         case T32x32: return ActTile::T32x32;
         case T64x64: return N <= 16 * 256 ? ActTile::T64x16 : ActTile::T64x32;
         default: return ActTile::NONE;
