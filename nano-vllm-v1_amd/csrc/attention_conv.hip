@@ -20,7 +20,9 @@ struct ConvPrepArgs {
     const int32_t *slots, *cu_seqlens_q, *context_lens, *slot_mapping;
     void *q_out, *k_cache, *v_cache;
     int T, batch, taps, H, G, dim, vdim, page, channels;
-    int unit, update_state, vec, lanes_log2;       // update_state 1: one token per sequence, 2: every sequence starts in this step;       // lanes: per row of a head, a power of two, eight channels each
+    int unit;
+    int update_state;              // 1: one token per sequence, 2: every sequence starts in this step, 0: left to nvh_conv_state_update
+    int vec, lanes_log2;           // lanes: per row of a head, a power of two, eight channels each
     float eps;
 };
 
