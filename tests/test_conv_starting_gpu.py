@@ -4,13 +4,16 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-LENS = [[1], [2], [3, 1, 2, 5], [4, 64, 1, 15, 17, 2], [300, 3, 700]]      # shorter than the taps, ends on and around the edges of tiles of 4, 16 and 64 tokens
+LENS = [[1], [2], [3, 1, 2, 5], [4, 64, 1, 15, 17, 2], [300, 3, 700],      # shorter than the taps, ends on and around the edges of tiles of 4, 16 and 64 tokens
+        [1, 300, 2, 1, 700, 3, 1]]      # short portions among enough tokens for tiles of 2 and 4 of them (below 1024 tokens x heads there is one a workgroup)
 
 
 def _step(lens, g):
     cu = torch.tensor([0] + lens).cumsum(0).int().cuda()
     slots = torch.randperm(len(lens) + 3, generator=g)[:len(lens)].int()
     slots[0] = -1 if len(lens) > 4 else slots[0]             # (a row without a slot)
+    if len(lens) > 6:
+        slots[2] = -1                                        # (and one of those that begin inside a tile)
     return cu, slots.cuda(), torch.tensor(lens).int().cuda()
 
 
