@@ -34,11 +34,12 @@ def test_trips_and_pages(hq, hkv, splits):
     assert (got - ref).abs().max() < 1.5e-2 + 2e-2 * ref.abs().max()
 
 
-@pytest.mark.parametrize("count", [129, 150, 160])
+@pytest.mark.parametrize("count", [129, 150, 160, 257, 270])
 @pytest.mark.parametrize("eager", [False, True])
 def test_order_of_dispatch_changes_no_bit(count, eager):
-    """A decode step of more workgroups than CUs (2 kv heads x 129 sequences and up; 150: with padded rows in the captured graph), the same
-    sequences handed over in two orders: every sequence gets the same logits bit for bit."""
+    """A decode step of more workgroups than CUs (2 kv heads x 129 sequences and up; 150, 257, 270: with padded rows in the captured graph), the same
+    sequences handed over in two orders: every sequence gets the same logits bit for bit.  Up to 256 of them are in a list of pieces, more in order of their
+    lengths."""
     from nanovllm.config import Config
     from nanovllm.engine.model_runner import ModelRunner
     from nanovllm.engine.sequence import Sequence
@@ -46,7 +47,7 @@ def test_order_of_dispatch_changes_no_bit(count, eager):
     lens = torch.randint(1, 520, (count,), generator=g).tolist()
     lens[0], lens[-1] = 1, 519
     pages = [-(-n // 256) for n in lens]
-    runner = ModelRunner(Config(TINY, max_num_batched_tokens=1024, max_num_seqs=160, max_model_len=1024, num_kvcache_blocks=sum(pages), chunked_prefill=True,
+    runner = ModelRunner(Config(TINY, max_num_batched_tokens=1024, max_num_seqs=max(160, -(-count // 16) * 16), max_model_len=1024, num_kvcache_blocks=sum(pages), chunked_prefill=True,
                                 enforce_eager=eager), 0, [])
     try:
         seqs, at = [], 0
@@ -67,10 +68,10 @@ def test_order_of_dispatch_changes_no_bit(count, eager):
         runner.exit()
 
 
-@pytest.mark.parametrize("count", [129, 140])
+@pytest.mark.parametrize("count", [129, 140, 257])
 def test_order_in_a_mixed_step(count):
-    """Decoding sequences in front of a portion of a prompt, enough for the dispatch by length: handed over in two orders every sequence, the portion's
-    last token too, gets the same logits bit for bit."""
+    """Decoding sequences in front of a portion of a prompt, enough for a list of pieces (up to 256) or the dispatch by length: handed over in two orders every
+    sequence, the portion's last token too, gets the same logits bit for bit."""
     from nanovllm.config import Config
     from nanovllm.engine.model_runner import ModelRunner
     from nanovllm.engine.sequence import Sequence
@@ -78,7 +79,7 @@ def test_order_in_a_mixed_step(count):
     lens = torch.randint(1, 520, (count,), generator=g).tolist() + [300]
     lens[0], lens[count - 1] = 1, 519
     pages = [-(-n // 256) for n in lens]
-    runner = ModelRunner(Config(TINY, max_num_batched_tokens=1024, max_num_seqs=160, max_model_len=1024, num_kvcache_blocks=sum(pages), chunked_prefill=True), 0, [])
+    runner = ModelRunner(Config(TINY, max_num_batched_tokens=1024, max_num_seqs=max(160, count + 1), max_model_len=1024, num_kvcache_blocks=sum(pages), chunked_prefill=True), 0, [])
     try:
         seqs, at = [], 0
         for i, (n, p) in enumerate(zip(lens, pages)):
