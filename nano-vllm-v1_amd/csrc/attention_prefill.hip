@@ -658,7 +658,7 @@ int32_t nvh_attn_varlen_beside(const void* q, int64_t q_token_stride, const void
             // blocks put a four-wave workgroup on every CU instead of an eight-wave one on every other (alone: 1024 queries and keys 21.5 us for 24.6,
             // 924 queries of 1948 keys 36 for 38).  Not in a mixed step while the step before it runs: a workgroup takes a CU's LDS whole either way, and half as
             // many leave the other CUs to that step's decode attention and products (mixed steps of 924 new tokens and 100 decodes whose ids nobody reads
-            // 3690 -> 3480 us; with the ids read back, where nothing runs beside them, 4935 - 4960 in 32-row blocks and 4995 - 5000 in 64; chunks 2112 and
+            // 3690 -> 3480 us; with the ids read back, where nothing runs beside them, 4822 - 4862 in 32-row blocks and 4894 - 4913 in 64; chunks 2112 and
             // 2126, no gain).  A row's bits are the same.
             const int rb1 = beside ? 0 : (int)nvh_switch_or(SW_ATTN_RB1, 128);     // A/B switch: 0 = never
             if (ks == 2 && wgs <= rb1) LAUNCH_VL(2, 1, 2, 2);
