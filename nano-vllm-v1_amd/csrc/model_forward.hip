@@ -241,7 +241,7 @@ static int32_t forward_impl(const nvh_qwen3_model* md, const nvh_step* st, void*
                           nvh_gemm_rowscaled_supported(t, qkv_n, h, 2) && nvh_gemm_rowscaled_supported(t, 2 * md->inter, h, 1) && (int64_t)(parts_o > parts_d ? parts_o : parts_d) * 4 <= h * 2;
     float* const rowsq = reinterpret_cast<float*>(w.y);
     // Prompt attention of a mixed step: is the step before this one still running?  That it left events does not say so: a loop that reads a mixed step's ids back
-    // before it goes on finds it ended (an event's query costs the host under 1 us).
+    // before it goes on finds it ended.
     bool beside = false;
     if (ev_wait && prefix > 0 && b > prefix) {
         const hipError_t e = hipEventQuery(ev_wait[md->layers - 1]);
